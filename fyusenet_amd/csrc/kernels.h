@@ -37,13 +37,15 @@ struct Act {
 // well: there the L2's write-back of whole lines serves HBM better than 64-byte pieces (measured on 90 and 180 MB
 // outputs: 10 to 19 % slower written through).
 //
-// (The compiler does not look inside the asm statement: a vector instruction that writes a register of a store of more
-// than eight bytes must be two wait states ahead of it on this part, which the s_nop provides whatever came before.)
+// (The compiler does not look inside the asm statement.  A store of more than eight bytes reads its data registers
+// after it has been issued: on this part no vector instruction may write one of them in the two wait states BEHIND the
+// store, which the s_nop keeps free whatever comes next.  Without it the first register of a lane's four -- two fp16
+// channels out of eight -- held the next fragment's values now and then, on layers whose workgroups walk several tiles.)
 template <class V>
 __device__ __forceinline__ void store_through(V* dst, const V v) {
     static_assert(sizeof(V) == 16, "store_through: 16-byte values");
     typedef int wt_i4 __attribute__((ext_vector_type(4)));
-    asm volatile("s_nop 1\n\tglobal_store_dwordx4 %0, %1, off sc1" ::"v"(dst), "v"(__builtin_bit_cast(wt_i4, v)) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst), "v"(__builtin_bit_cast(wt_i4, v)) : "memory");
 }
 template <class V>
 __device__ __forceinline__ void store_out(bool through, V* dst, const V v) {

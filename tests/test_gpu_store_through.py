@@ -96,3 +96,18 @@ def test_written_through_outputs_with_several_networks_in_flight(monkeypatch):
     pool.close()
     for i in range(len(frames)):
         assert np.array_equal(outs[i], want[i]), i
+
+
+@pytest.mark.parametrize("size", [(892, 864), (640, 960)], ids=["892x864", "640x960"])
+def test_written_through_outputs_of_many_tiles_per_workgroup(size, monkeypatch):
+    """fp16 stride-2 layers whose workgroups walk six and more tiles: the registers of a store are written again for the
+    next fragment as soon as it has been issued."""
+    w, h = size
+    x = prng.uniform(7100, (3, h, w), 0.0, 1.0)
+    monkeypatch.delenv("FYNHIP_PLAIN_STORES", raising=False)
+    got, infos = _passes(networks.StyleNet(fa.STORAGE_F16, w, h), [x] * 4, False)
+    assert any("stores=through" in i for i in infos.values()), infos
+    monkeypatch.setenv("FYNHIP_PLAIN_STORES", "1")
+    want, _ = _passes(networks.StyleNet(fa.STORAGE_F16, w, h), [x], False)
+    for i, a in enumerate(got):
+        assert np.array_equal(a, want[0]), "pass %d: %d values differ" % (i, int((a != want[0]).sum()))
