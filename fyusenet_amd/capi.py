@@ -128,6 +128,8 @@ SYMBOLS = {
     "fyn_net_async_wait": (ctypes.c_int, [_P, ctypes.c_uint64]),
     "fyn_net_async_end": (ctypes.c_int, [_P]),
     "fyn_layer_kernel_info": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_char_p, ctypes.c_size_t]),
+    "fyn_host_acquire": (ctypes.c_int, [ctypes.c_size_t, ctypes.POINTER(_P)]),
+    "fyn_host_release": (ctypes.c_int, [_P]),
     "fyn_net_device_allocations": (ctypes.c_int, [_P, ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]),
 }
 
@@ -160,6 +162,38 @@ def check(status):
 def fptr(arr):
     assert arr.dtype == np.float32 and arr.flags["C_CONTIGUOUS"]
     return arr.ctypes.data_as(_F)
+
+
+class _ResultBlock:
+    """A block of the library's page-locked memory under an array; goes back when the array is gone."""
+
+    __slots__ = ("__array_interface__", "_ptr")
+
+    def __init__(self, ptr, shape, typestr):
+        self._ptr = ptr
+        self.__array_interface__ = {"shape": shape, "typestr": typestr, "data": (ptr, False), "version": 3}
+
+    def __del__(self):
+        if _lib is not None:
+            _lib.fyn_host_release(self._ptr)
+
+
+#: Results of this size and more are written by the GPU into memory taken from the library (smaller ones are copied
+#: faster than the array is set up).
+RESULT_BLOCK_BYTES = 64 << 10
+
+
+def result_array(shape, dtype=np.float32):
+    """An uninitialised array for a result, in memory that the GPU writes in place where there is any."""
+    nbytes = 4
+    for n in shape:
+        nbytes *= n
+    if nbytes >= RESULT_BLOCK_BYTES:
+        ptr = _P()
+        check(lib().fyn_host_acquire(nbytes, ctypes.byref(ptr)))
+        if ptr.value:
+            return np.asarray(_ResultBlock(ptr.value, tuple(shape), "<f4" if dtype == np.float32 else "<i4"))
+    return np.empty(shape, dtype)
 
 
 def device_info(device=0):

@@ -284,6 +284,19 @@ int fyn_net_async_end(fyn_net* net) {
     FYN_API_END
 }
 
+int fyn_host_acquire(size_t bytes, void** ptr) {
+    FYN_API_BEGIN
+    if (!ptr) fynhip::fail(FYN_ERR_INVALID, "null pointer");
+    *ptr = fynhip::HostPool::acquire(bytes, true);
+    FYN_API_END
+}
+
+int fyn_host_release(void* ptr) {
+    FYN_API_BEGIN
+    fynhip::HostPool::release(ptr);
+    FYN_API_END
+}
+
 int fyn_net_device_allocations(fyn_net* net, size_t* calls, size_t* bytes) {
     FYN_API_BEGIN
     if (calls) *calls = N(net)->alloc_calls_;

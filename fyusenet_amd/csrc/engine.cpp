@@ -171,8 +171,25 @@ Net::Net(int dev, int stor) : device(dev), storage(stor) {
     if (dev < 0 || dev >= count) fail(FYN_ERR_DEVICE, "device %d not present (%d devices)", dev, count);
     FYN_HIP(hipSetDevice(dev));
     stream = lease_stream(dev, false);
-    // resolved here, where the caller may still allocate: looking the symbol up loads the code object on this device
-    static_scratch_ = static_scratch(dev);
+    HostPool::network_created();
+    try {
+        // resolved here, where the caller may still allocate: looking the symbol up loads the code object on this device
+        static_scratch_ = static_scratch(dev);
+        signal_.create(static_cast<unsigned*>(dev_alloc(64)));
+    } catch (...) {
+        release_all();
+        throw;
+    }
+}
+
+void Net::release_all() {
+    if (stream) (void)hipStreamSynchronize(stream);
+    for (void* p : allocs_) (void)hipFree(p);
+    allocs_.clear();
+    signal_.destroy();
+    HostPool::release(in_pin_);
+    return_stream(device, stream);
+    HostPool::network_gone();
 }
 
 Net::~Net() {
@@ -189,8 +206,7 @@ Net::~Net() {
         if (kv.second->ev1) (void)hipEventDestroy(kv.second->ev1);
     }
     layers.clear();
-    for (void* p : allocs_) (void)hipFree(p);
-    return_stream(device, stream);
+    release_all();
 }
 
 void* Net::dev_alloc(size_t bytes, bool zero) {
@@ -524,8 +540,60 @@ void Net::forward(uint64_t* seq_out) {
 
 void Net::finish() {
     FYN_HIP(hipSetDevice(device));
-    FYN_HIP(hipStreamSynchronize(stream));
-    collect_timings();
+    if (events_pending_) {
+        FYN_HIP(hipStreamSynchronize(stream));
+        settled();
+        collect_timings();
+        return;
+    }
+    const HostDone done = signal_.next();
+    launch_tell_host(done, stream);
+    FYN_HIP(hipGetLastError());
+    wait_signal(done.value);
+}
+
+// Everything queued on the stream ahead of the launch with this value has been carried out then.
+void Net::wait_signal(unsigned value) {
+    signal_.wait(value, stream);
+    if (value == signal_.last()) settled();
+}
+
+// The stream is idle: nothing reads the input area any more.
+void Net::settled() {
+    in_off_ = 0;
+    HostPool::release(in_pin_);
+    in_pin_ = nullptr;
+    in_bytes_ = 0;
+}
+
+void Net::count_area(size_t bytes, size_t& most) {
+    if (bytes <= most) return;
+    most = bytes;
+    alloc_calls_++;
+    alloc_bytes_ += bytes;
+}
+
+// `floats` of page-locked memory that no queued launch reads, on loan until the stream has been waited for.
+float* Net::in_area(size_t floats) {
+    const size_t bytes = (floats * sizeof(float) + 255) & ~size_t(255);
+    if (in_off_ + bytes > in_bytes_) {
+        if (in_off_) FYN_HIP(hipStreamSynchronize(stream));
+        settled();
+        in_pin_ = static_cast<char*>(HostPool::acquire(bytes, false));
+        in_bytes_ = bytes;
+        count_area(bytes, in_most_);
+    }
+    float* p = reinterpret_cast<float*>(in_pin_ + in_off_);
+    in_off_ += bytes;
+    return p;
+}
+
+// Page-locked memory for a result on its way to the caller's, on loan for one call.
+HostLoan Net::out_area(size_t floats) {
+    const size_t bytes = floats * sizeof(float);
+    HostLoan l(bytes);
+    count_area(bytes, out_most_);
+    return l;
 }
 
 void Net::use_graph(bool enable) {
@@ -560,22 +628,53 @@ void Net::async_sizes(size_t* in_floats, size_t* out_floats) const {
     *out_floats = async_out_floats_;
 }
 
+// A host transfer in pieces: while the link moves one, the host copies the next.  Pieces below a megabyte are not worth
+// their launches (4 us each).
+static size_t piece_pixels(size_t npix, size_t bytes) {
+    const size_t pieces = std::min<size_t>(12, std::max<size_t>(1, bytes / (1280u << 10)));
+    return std::max<size_t>(4, ((npix + pieces - 1) / pieces + 3) & ~size_t(3));
+}
+
+void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
+    const size_t npix = (size_t)v.h * v.w, plane = (npix + 3) & ~size_t(3);
+    const bool host = host_memory(data);
+    float* st = host ? in_area(plane * v.c) : staging(plane * v.c);
+    if (amax) launch_fill_zero(amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
+    const size_t step = piece_pixels(npix, npix * v.c * sizeof(float));
+    const bool planes = order == FYN_ORDER_CHANNELWISE;
+    HostCopy copies;
+    std::vector<size_t> marks;
+    for (size_t p0 = 0; p0 < npix; p0 += step) {
+        const size_t p1 = std::min(npix, p0 + step);
+        for (int c = 0; c < (planes ? v.c : 1); c++) {
+            float* dst = st + (planes ? c * plane + p0 : p0 * v.c);
+            const float* src = data + (planes ? c * npix + p0 : p0 * v.c);
+            const size_t bytes = (p1 - p0) * (planes ? 1 : v.c) * sizeof(float);
+            if (host) copies.add(dst, src, bytes);
+            else FYN_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, stream));
+        }
+        marks.push_back(copies.mark());
+    }
+    copies.start();
+    size_t piece = 0;
+    for (size_t p0 = 0; p0 < npix; p0 += step) {
+        const size_t p1 = std::min(npix, p0 + step);
+        copies.upto(marks[piece++]);
+        if (planes) launch_chw_to_tensor(st, plane, v, p0, p1, stream, amax);
+        else launch_hwc_to_tensor(st, v, p0, p1, stream, amax);
+    }
+    FYN_HIP(hipGetLastError());
+    // the caller's buffer is borrowed for this call only
+    if (!host) FYN_HIP(hipStreamSynchronize(stream));
+}
+
 void Net::set_input(int layer_no, int port, const float* data, int order) {
     if (!is_setup) fail(FYN_ERR_STATE, "set_input() before setup()");
     if (!data) fail(FYN_ERR_INVALID, "null input buffer");
     FYN_HIP(hipSetDevice(device));
-    const TView& v = input_tensor(layer_no, port).v;
-    const size_t n = (size_t)v.c * v.h * v.w;
-    float* st = staging(n);
-    FYN_HIP(hipMemcpyAsync(st, data, n * sizeof(float), hipMemcpyHostToDevice, stream));
-    unsigned* amax = input_tensor(layer_no, port).amax;
-    if (amax) launch_fill_zero(amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
-    if (order == FYN_ORDER_CHANNELWISE) launch_chw_to_tensor(st, v, stream, amax);
-    else if (order == FYN_ORDER_GPU_SHALLOW) launch_hwc_to_tensor(st, v.c, v, stream, amax);
-    else fail(FYN_ERR_UNSUPPORTED, "input order %d not supported for upload", order);
-    FYN_HIP(hipGetLastError());
-    // the host buffer is borrowed for this call only
-    FYN_HIP(hipStreamSynchronize(stream));
+    const Tensor& t = input_tensor(layer_no, port);
+    if (order != FYN_ORDER_CHANNELWISE && order != FYN_ORDER_GPU_SHALLOW) fail(FYN_ERR_UNSUPPORTED, "input order %d not supported for upload", order);
+    upload(data, order, t.v, t.amax);
 }
 
 // What a layer hands out: its output tensor; a layer that only passes its input on (download) may name up to three
@@ -586,17 +685,87 @@ static TView result_view(Layer* l) {
     return v;
 }
 
+// CHW planes of a tensor into the caller's memory.  Memory that the GPU reaches (HostPool) is written by the converting
+// launch itself; anything else is filled from the staging area piece by piece, behind the launches that fill that.
+void Net::download_planes(const TView& v, int include_padding, float* out) {
+    const size_t npix = include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, bytes = npix * v.c * sizeof(float);
+    if (!host_memory(out)) {
+        float* st = staging(npix * v.c);
+        launch_tensor_to_chw(v, st, npix, include_padding, 0, npix, HostDone{}, stream);
+        FYN_HIP(hipGetLastError());
+        FYN_HIP(hipMemcpyAsync(out, st, bytes, hipMemcpyDefault, stream));
+        FYN_HIP(hipStreamSynchronize(stream));
+        settled();
+        return;
+    }
+    if (HostPool::contains(out, bytes)) {
+        const HostDone done = signal_.next();
+        launch_tensor_to_chw(v, out, npix, include_padding, 0, npix, done, stream);
+        FYN_HIP(hipGetLastError());
+        wait_signal(done.value);
+        return;
+    }
+    const size_t plane = npix < 64 ? npix : (npix + 3) & ~size_t(3);
+    const HostLoan loan = out_area(plane * v.c);
+    float* st = loan.floats();
+    const size_t step = piece_pixels(npix, bytes);
+    const unsigned first = signal_.last() + 1;
+    for (size_t p0 = 0; p0 < npix; p0 += step) launch_tensor_to_chw(v, st, plane, include_padding, p0, std::min(npix, p0 + step), signal_.next(), stream);
+    FYN_HIP(hipGetLastError());
+    unsigned value = first;
+    for (size_t p0 = 0; p0 < npix; p0 += step) {
+        const size_t p1 = std::min(npix, p0 + step);
+        wait_signal(value++);
+        HostCopy copies;
+        for (int c = 0; c < v.c; c++) copies.add(out + c * npix + p0, st + c * plane + p0, (p1 - p0) * sizeof(float));
+        copies.start();
+    }
+}
+
+// The same for interleaved pixels of pc floats.
+void Net::download_pixels(const TView& v, int pc, float* out) {
+    const size_t npix = (size_t)v.h * v.w, bytes = npix * pc * sizeof(float);
+    const bool host = host_memory(out), direct = host && HostPool::contains(out, bytes);
+    const HostLoan loan = host && !direct ? out_area(npix * pc) : HostLoan();
+    float* st = direct ? out : host ? loan.floats() : staging(npix * pc);
+    const size_t step = host && !direct ? piece_pixels(npix, bytes) : npix;
+    const unsigned first = signal_.last() + 1;
+    for (size_t p0 = 0; p0 < npix; p0 += step) launch_tensor_to_hwc(v, st, pc, p0, std::min(npix, p0 + step), signal_.next(), stream);
+    FYN_HIP(hipGetLastError());
+    unsigned value = first;
+    for (size_t p0 = 0; p0 < npix; p0 += step) {
+        wait_signal(value++);
+        if (host && !direct) memcpy(out + p0 * pc, st + p0 * pc, (std::min(npix, p0 + step) - p0) * pc * sizeof(float));
+    }
+    if (!host) {
+        FYN_HIP(hipMemcpyAsync(out, st, bytes, hipMemcpyDefault, stream));
+        FYN_HIP(hipStreamSynchronize(stream));
+    }
+}
+
+// Indices and values of an arg-max layer, either of them where it is wanted.
+void Net::download_argmax(const int* idx_dev, const TView& v, int32_t* idx, float* val) {
+    const size_t n = (size_t)v.h * v.w, area = (n + 63) & ~size_t(63);
+    if (!idx && !val) return finish();
+    const bool direct = (!idx || (host_memory(idx) && HostPool::contains(idx, n * 4))) && (!val || (host_memory(val) && HostPool::contains(val, n * 4)));
+    const bool host = (!idx || host_memory(idx)) && (!val || host_memory(val));
+    const HostLoan loan = host && !direct ? out_area(2 * area) : HostLoan();
+    float* st = direct ? nullptr : host ? loan.floats() : staging(2 * area);
+    int* di = !idx ? nullptr : direct ? idx : reinterpret_cast<int*>(st);
+    float* dv = !val ? nullptr : direct ? val : st + area;
+    const HostDone done = signal_.next();
+    launch_argmax_to_host(idx_dev, v, di, dv, 0, n, done, stream);
+    FYN_HIP(hipGetLastError());
+    wait_signal(done.value);
+    if (direct) return;
+    if (idx) FYN_HIP(host ? (memcpy(idx, di, n * 4), hipSuccess) : hipMemcpy(idx, di, n * 4, hipMemcpyDefault));
+    if (val) FYN_HIP(host ? (memcpy(val, dv, n * 4), hipSuccess) : hipMemcpy(val, dv, n * 4, hipMemcpyDefault));
+}
+
 void Net::copy_result(int layer_no, float* chw, int include_padding) {
     if (!is_setup) fail(FYN_ERR_STATE, "copy_result() before setup()");
     FYN_HIP(hipSetDevice(device));
-    Layer* l = layer(layer_no);
-    const TView v = result_view(l);
-    const size_t n = include_padding ? (size_t)v.c * v.hp() * v.wp() : (size_t)v.c * v.h * v.w;
-    float* st = staging(n);
-    launch_tensor_to_chw(v, st, include_padding, stream);
-    FYN_HIP(hipGetLastError());
-    FYN_HIP(hipMemcpyAsync(chw, st, n * sizeof(float), hipMemcpyDeviceToHost, stream));
-    FYN_HIP(hipStreamSynchronize(stream));
+    download_planes(result_view(layer(layer_no)), include_padding, chw);
 }
 
 void Net::copy_result_static(int layer_no, float* chw, int include_padding) {
@@ -610,7 +779,8 @@ void Net::copy_result_static(int layer_no, float* chw, int include_padding) {
         fail(FYN_ERR_INVALID, "result of layer %s (%d) has %zu floats, the fixed staging area holds %zu: use fyn_layer_copy_result",
              l->d.name, l->d.number, n, (size_t)FYN_STATIC_SCRATCH_FLOATS);
     // every element of [0, n) is written by the conversion kernel: nothing of an earlier call is read
-    launch_tensor_to_chw(v, static_scratch_, include_padding, stream);
+    launch_tensor_to_chw(v, static_scratch_, include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, include_padding, 0,
+                         include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, HostDone{}, stream);
     FYN_HIP(hipGetLastError());
     FYN_HIP(hipMemcpyAsync(chw, static_scratch_, n * sizeof(float), hipMemcpyDefault, stream));
     FYN_HIP(hipStreamSynchronize(stream));
@@ -643,13 +813,7 @@ void Net::get_output(int layer_no, float* data, int order) {
         copy_result(layer_no, data, 0);
     } else if (order == FYN_ORDER_GPU_SHALLOW) {
         if (v.c > 4) fail(FYN_ERR_UNSUPPORTED, "GPU_SHALLOW download holds at most 4 channels per texel (layer has %d)", v.c);
-        const int pc = v.c == 3 ? 4 : v.c;  // rendered textures are RGBA (base/buffermanager.cpp:478-483)
-        const size_t n = (size_t)v.h * v.w * pc;
-        float* st = staging(n);
-        launch_tensor_to_hwc(v, st, pc, stream);
-        FYN_HIP(hipGetLastError());
-        FYN_HIP(hipMemcpyAsync(data, st, n * sizeof(float), hipMemcpyDeviceToHost, stream));
-        FYN_HIP(hipStreamSynchronize(stream));
+        download_pixels(v, v.c == 3 ? 4 : v.c, data);  // rendered textures are RGBA (base/buffermanager.cpp:478-483)
     } else if (order == FYN_ORDER_GPU_DEEP) {
         // tiled RGBA buffer, tile t at grid (t % tx, t / tx), padding shared between tiles
         // (gpu/deep/deeptiler.cpp:63-110)
@@ -796,6 +960,7 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
         fail(FYN_ERR_UNSUPPORTED, "output order %d not supported by the frame pipeline", out_order);
     }
     async_in_floats_ = (size_t)vi.c * vi.h * vi.w;
+    async_in_plane_ = ((size_t)vi.h * vi.w + 3) & ~size_t(3);
     async_in_order_ = in_order;
     async_out_order_ = out_order;
     async_own_streams_ = copy_streams;
@@ -807,9 +972,9 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
     }
     slots_.resize(depth);
     for (AsyncSlot& s : slots_) {
-        FYN_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.pin_in), async_in_floats_ * sizeof(float), hipHostMallocDefault));
+        FYN_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.pin_in), async_in_plane_ * vi.c * sizeof(float), hipHostMallocDefault));
         FYN_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.pin_out), async_out_floats_ * sizeof(float), hipHostMallocDefault));
-        FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), async_in_floats_ * sizeof(float)));
+        FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), async_in_plane_ * vi.c * sizeof(float)));
         FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_out), async_out_floats_ * sizeof(float)));
         FYN_HIP(hipEventCreateWithFlags(&s.up, hipEventDisableTiming));
         FYN_HIP(hipEventCreateWithFlags(&s.comp, hipEventDisableTiming));
@@ -830,17 +995,21 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
     FYN_HIP(hipSetDevice(device));
     AsyncSlot& s = slots_[async_seq_ % slots_.size()];
     async_complete(s);  // oldest frame: its output is delivered before the slot is reused
-    memcpy(s.pin_in, in, async_in_floats_ * sizeof(float));
-    FYN_HIP(hipMemcpyAsync(s.dev_in, s.pin_in, async_in_floats_ * sizeof(float), hipMemcpyHostToDevice, up_stream_));
+    const TView& vi = async_in_->v;
+    const size_t npix = (size_t)vi.h * vi.w;
+    if (async_in_order_ == FYN_ORDER_CHANNELWISE)
+        for (int c = 0; c < vi.c; c++) memcpy(s.pin_in + c * async_in_plane_, in + c * npix, npix * sizeof(float));
+    else memcpy(s.pin_in, in, async_in_floats_ * sizeof(float));
+    FYN_HIP(hipMemcpyAsync(s.dev_in, s.pin_in, async_in_plane_ * vi.c * sizeof(float), hipMemcpyHostToDevice, up_stream_));
     FYN_HIP(hipEventRecord(s.up, up_stream_));
     FYN_HIP(hipStreamWaitEvent(stream, s.up, 0));
     if (async_in_->amax) launch_fill_zero(async_in_->amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
-    if (async_in_order_ == FYN_ORDER_CHANNELWISE) launch_chw_to_tensor(s.dev_in, async_in_->v, stream, async_in_->amax);
-    else launch_hwc_to_tensor(s.dev_in, async_in_->v.c, async_in_->v, stream, async_in_->amax);
+    if (async_in_order_ == FYN_ORDER_CHANNELWISE) launch_chw_to_tensor(s.dev_in, async_in_plane_, vi, 0, npix, stream, async_in_->amax);
+    else launch_hwc_to_tensor(s.dev_in, vi, 0, npix, stream, async_in_->amax);
     forward(nullptr);
     const TView& vo = async_out_view_;
-    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, s.dev_out, 0, stream);
-    else launch_tensor_to_hwc(vo, s.dev_out, vo.c == 3 ? 4 : vo.c, stream);
+    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, s.dev_out, (size_t)vo.h * vo.w, 0, 0, (size_t)vo.h * vo.w, HostDone{}, stream);
+    else launch_tensor_to_hwc(vo, s.dev_out, vo.c == 3 ? 4 : vo.c, 0, (size_t)vo.h * vo.w, HostDone{}, stream);
     FYN_HIP(hipGetLastError());
     FYN_HIP(hipEventRecord(s.comp, stream));
     FYN_HIP(hipStreamWaitEvent(down_stream_, s.comp, 0));

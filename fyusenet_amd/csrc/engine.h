@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/fynhip.h"
+#include "host_io.h"
 #include "kernels.h"
 
 namespace fynhip {
@@ -151,7 +152,7 @@ class Net {
     void* dev_alloc(size_t bytes, bool zero = true);
     void dev_free(void* p);   // setup-time only (waits for the stream)
     void dev_free_many(const std::vector<void*>& ptrs);   // the same for several areas, one wait
-    float* staging(size_t floats);  // fp32 staging area for layout conversion
+    float* staging(size_t floats);  // fp32 staging area in device memory, for callers whose buffers lie there
 
   private:
     struct AsyncSlot {
@@ -168,10 +169,11 @@ class Net {
     bool async_own_streams_ = true;
     TView async_out_view_{};   // what the output layer hands out (a download layer may name other channel counts)
     int async_in_order_ = 0, async_out_order_ = 0;
-    size_t async_in_floats_ = 0, async_out_floats_ = 0;
+    size_t async_in_floats_ = 0, async_out_floats_ = 0, async_in_plane_ = 0;   // (planes lie on multiples of four floats)
     uint64_t async_seq_ = 0;
     void async_complete(AsyncSlot& s);
     void run_layers(bool with_events);
+    void release_all();
     void collect_timings();
     void dump_layer(Layer* l);
     std::vector<void*> allocs_;
@@ -181,6 +183,20 @@ class Net {
   private:
     float* staging_ = nullptr;
     size_t staging_floats_ = 0;
+    // Page-locked staging of the synchronous calls.  Inputs are put in one behind the other and converted by launches that
+    // read them in place; the area goes back once the stream has been waited for.
+    char* in_pin_ = nullptr;
+    size_t in_bytes_ = 0, in_off_ = 0, in_most_ = 0, out_most_ = 0;
+    HostSignal signal_;
+    float* in_area(size_t floats);
+    HostLoan out_area(size_t floats);
+    void count_area(size_t bytes, size_t& most);   // staging areas count as allocations when they are larger than any before
+    void wait_signal(unsigned value);
+    void settled();
+    void upload(const float* data, int order, const TView& v, unsigned* amax);
+    void download_planes(const TView& v, int include_padding, float* out);
+    void download_pixels(const TView& v, int pc, float* out);
+    void download_argmax(const int* idx_dev, const TView& v, int32_t* idx, float* val);
     float* static_scratch_ = nullptr;   // this device's address of the fixed staging area
     unsigned* amax_dev_ = nullptr;      // one value-range word per tensor
     void assign_range_words();

@@ -1,0 +1,217 @@
+// Page-locked host memory pool and host-polled completion words.
+#include "host_io.h"
+
+#include <immintrin.h>
+
+#include <algorithm>
+#include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <cstring>
+#include <deque>
+#include <map>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "engine.h"
+
+namespace fynhip {
+
+namespace {
+struct Block {
+    size_t bytes;
+    bool lent;
+};
+std::mutex g_pool_mu;
+std::map<char*, Block> g_blocks;   // by address
+size_t g_pool_bytes = 0;
+int g_networks = 0;
+
+size_t size_class(size_t bytes) {   // sizes in steps of an eighth of the next power of two, so that like sizes share blocks
+    size_t step = 4096;
+    while (step * 16 <= bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+void give_back_idle() {   // (the lock is held)
+    for (auto it = g_blocks.begin(); it != g_blocks.end();) {
+        if (it->second.lent) {
+            ++it;
+            continue;
+        }
+        g_pool_bytes -= it->second.bytes;
+        (void)hipHostFree(it->first);
+        it = g_blocks.erase(it);
+    }
+}
+}  // namespace
+
+void* HostPool::acquire(size_t bytes, bool bounded) {
+    const size_t want = size_class(bytes ? bytes : 1);
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    for (auto& kv : g_blocks)
+        if (!kv.second.lent && kv.second.bytes == want) {
+            kv.second.lent = true;
+            return kv.first;
+        }
+    if (bounded && g_networks == 0) return nullptr;
+    if (g_pool_bytes + want > kBytes) {
+        give_back_idle();
+        if (bounded && g_pool_bytes + want > kBytes) return nullptr;
+    }
+    void* p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, want, hipHostMallocPortable);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        if (bounded) return nullptr;
+        fail(FYN_ERR_DEVICE, "no page-locked memory (%zu bytes): %s", want, hipGetErrorString(e));
+    }
+    g_blocks[static_cast<char*>(p)] = Block{want, true};
+    g_pool_bytes += want;
+    return p;
+}
+
+void HostPool::release(void* p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    auto it = g_blocks.find(static_cast<char*>(p));
+    if (it == g_blocks.end() || !it->second.lent) return;
+    it->second.lent = false;
+    if (g_networks == 0 || g_pool_bytes > kBytes) give_back_idle();
+}
+
+bool HostPool::contains(const void* p, size_t bytes) {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    char* c = const_cast<char*>(static_cast<const char*>(p));
+    auto it = g_blocks.upper_bound(c);
+    if (it == g_blocks.begin()) return false;
+    --it;
+    return it->second.lent && c + bytes <= it->first + it->second.bytes;
+}
+
+void HostPool::network_created() {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    g_networks++;
+}
+void HostPool::network_gone() {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    if (--g_networks == 0) give_back_idle();
+}
+
+void HostSignal::create(unsigned* counter) {
+    counter_ = counter;
+    flag_ = static_cast<unsigned*>(HostPool::acquire(64, false));
+    *flag_ = value_ = 0;
+}
+void HostSignal::destroy() {
+    HostPool::release(flag_);
+    flag_ = nullptr;
+}
+HostDone HostSignal::next() { return HostDone{counter_, flag_, ++value_}; }
+
+void HostSignal::wait(unsigned value, hipStream_t s) {
+    // (values pass in rising order; the difference survives the wrap-around)
+    auto done = [&] { return (int)(__atomic_load_n(flag_, __ATOMIC_ACQUIRE) - value) >= 0; };
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 1; !done(); i++) {
+        _mm_pause();
+        if (i % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+            FYN_HIP(hipStreamSynchronize(s));
+            if (!done()) fail(FYN_ERR_DEVICE, "a launch ended without telling so");
+            return;
+        }
+    }
+}
+
+// ---- copies ----
+struct HostCopy::Job {
+    struct Slice {
+        char* dst;
+        const char* src;
+        size_t bytes;
+    };
+    std::vector<Slice> slices;
+    size_t bytes = 0;
+    std::unique_ptr<std::atomic<char>[]> made;
+    std::atomic<size_t> next{0};
+    bool one() {   // makes the next copy; false: all have been taken
+        const size_t i = next.fetch_add(1, std::memory_order_relaxed);
+        if (i >= slices.size()) return false;
+        memcpy(slices[i].dst, slices[i].src, slices[i].bytes);
+        made[i].store(1, std::memory_order_release);
+        return true;
+    }
+};
+
+// The helper threads.  They sleep while there is nothing to copy; the object is never destroyed, so that they may be
+// asleep in it when the process ends.
+struct HostCopyHelpers {
+    static constexpr size_t kSlice = 256u << 10, kAlone = 8u << 20;   // (waking a thread takes 20 to 50 us, and smaller buffers tend to lie in this core's caches: those jobs are done alone)
+    std::mutex mu;
+    std::condition_variable cv;
+    std::deque<std::shared_ptr<HostCopy::Job>> jobs;
+    HostCopyHelpers() {
+        const unsigned cpus = std::thread::hardware_concurrency();
+        for (unsigned i = 0; i < std::min(3u, cpus / 4); i++) std::thread([this] { work(); }).detach();
+    }
+    static HostCopyHelpers& get() {
+        static HostCopyHelpers* h = new HostCopyHelpers;
+        return *h;
+    }
+    void offer(const std::shared_ptr<HostCopy::Job>& job) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            jobs.push_back(job);
+        }
+        cv.notify_all();
+    }
+    void work() {
+        for (;;) {
+            std::shared_ptr<HostCopy::Job> job;
+            {
+                std::unique_lock<std::mutex> lk(mu);
+                cv.wait(lk, [this] { return !jobs.empty(); });
+                job = jobs.front();
+                if (job->next.load(std::memory_order_relaxed) >= job->slices.size()) {
+                    jobs.pop_front();
+                    continue;
+                }
+            }
+            while (job->one()) {
+            }
+        }
+    }
+};
+
+HostCopy::HostCopy() : job_(std::make_shared<Job>()) {}
+HostCopy::~HostCopy() {
+    if (job_->made) upto(mark());
+}
+void HostCopy::add(void* dst, const void* src, size_t bytes) {
+    for (size_t o = 0; o < bytes; o += HostCopyHelpers::kSlice)
+        job_->slices.push_back({static_cast<char*>(dst) + o, static_cast<const char*>(src) + o, std::min(HostCopyHelpers::kSlice, bytes - o)});
+    job_->bytes += bytes;
+}
+size_t HostCopy::mark() const { return job_->slices.size(); }
+void HostCopy::start() {
+    job_->made.reset(new std::atomic<char>[job_->slices.size()]());
+    if (job_->bytes >= HostCopyHelpers::kAlone) HostCopyHelpers::get().offer(job_);
+}
+void HostCopy::upto(size_t mark) {
+    for (;;) {
+        while (seen_ < mark && job_->made[seen_].load(std::memory_order_acquire)) seen_++;
+        if (seen_ >= mark) return;
+        if (!job_->one()) _mm_pause();
+    }
+}
+
+bool host_memory(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {   // memory that HIP knows nothing of
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type != hipMemoryTypeDevice;
+}
+
+}  // namespace fynhip

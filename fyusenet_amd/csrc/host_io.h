@@ -1,0 +1,81 @@
+// Page-locked host memory and the words in it through which launches tell the host that they are done.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <memory>
+
+#include "kernels.h"
+
+namespace fynhip {
+
+// Blocks of page-locked memory, kept for the next user instead of being locked and released every time (locking 25 MB
+// takes milliseconds, a transfer of them half of one).  Shared by all networks and threads of the process.  Results are
+// put into it only while less than kBytes are locked (networks' own staging areas are not refused), and what nobody has
+// on loan goes back to the system when room is needed and with the last network.
+class HostPool {
+  public:
+    static constexpr size_t kBytes = size_t(512) << 20;
+    static void* acquire(size_t bytes, bool bounded);   // bounded: null when the pool is full or there is no GPU; else throws when memory cannot be had
+    static void release(void* p);                       // null is nothing
+    static bool contains(const void* p, size_t bytes);  // whether the range lies inside a block on loan
+    static void network_created();
+    static void network_gone();
+};
+
+// A block on loan for a scope.
+class HostLoan {
+  public:
+    HostLoan() = default;
+    explicit HostLoan(size_t bytes) : p_(HostPool::acquire(bytes, false)) {}
+    HostLoan(HostLoan&& o) noexcept : p_(o.p_) { o.p_ = nullptr; }
+    HostLoan(const HostLoan&) = delete;
+    HostLoan& operator=(const HostLoan&) = delete;
+    ~HostLoan() { HostPool::release(p_); }
+    float* floats() const { return static_cast<float*>(p_); }
+
+  private:
+    void* p_ = nullptr;
+};
+
+// Copies between host buffers, shared with a few helper threads of the process when they are large: one core moves 20 to
+// 40 GB/s of memory that no cache holds, less than the link to the GPU takes (55 GB/s); four move 100.  The copies are
+// done in the order in which they were added, so that what depends on the first ones can start early.
+class HostCopy {
+  public:
+    HostCopy();
+    ~HostCopy();   // (all copies have been made then)
+    void add(void* dst, const void* src, size_t bytes);
+    size_t mark() const;       // for upto(): the copies added so far
+    void start();              // all copies have been added
+    void upto(size_t mark);    // returns when these copies have been made, having done its share
+
+  private:
+    struct Job;
+    std::shared_ptr<Job> job_;
+    size_t seen_ = 0;
+    friend struct HostCopyHelpers;
+};
+
+// One stream's word.
+class HostSignal {
+  public:
+    void create(unsigned* counter);   // a word of device memory that is zero
+    void destroy();
+    HostDone next();                           // for the next launch on the stream
+    // Returns when the launch that was given `value`, and so everything in front of it on the stream, has been carried
+    // out.  Polls for a while, then leaves the waiting to the runtime, which also reports a failed launch.
+    void wait(unsigned value, hipStream_t s);
+    unsigned last() const { return value_; }
+
+  private:
+    unsigned* flag_ = nullptr;
+    unsigned* counter_ = nullptr;
+    unsigned value_ = 0;
+};
+
+// Whether the host can read and write the memory itself (false: device memory).
+bool host_memory(const void* p);
+
+}  // namespace fynhip

@@ -454,12 +454,22 @@ void launch_gemv(const GemvParams& p, hipStream_t s);
 bool fc_mfma_supported(const GemvParams& p);
 int launch_fc_mfma(const GemvParams& p, hipStream_t s);
 
-// Layout conversion between the engine layout and CHW fp32 staging buffers.
-// (amax: value-range word of the tensor, raised by what is written, or null; range.h)
-void launch_chw_to_tensor(const float* chw, const TView& t, hipStream_t s, unsigned* amax = nullptr);   // net area only
-void launch_tensor_to_chw(const TView& t, float* chw, int include_padding, hipStream_t s);
-void launch_hwc_to_tensor(const float* hwc, int pc, const TView& t, hipStream_t s, unsigned* amax = nullptr);   // GPU_SHALLOW in
-void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, hipStream_t s);             // GPU_SHALLOW out
+// What the last workgroup of a launch tells the host when the whole launch has been carried out (layout.hip): `value` in
+// the page-locked word `flag` (null: nothing); `counter`, a word of device memory that is zero between launches, belongs
+// to one stream.
+struct HostDone {
+    unsigned* counter;
+    unsigned* flag;
+    unsigned value;
+};
+// Layout conversion between tensors and fp32 buffers in page-locked host memory or device memory (layout.hip); pixels
+// [p0, p1) of the area.  (amax: value-range word of the tensor, raised by what is written, or null; range.h)
+void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax);   // net area only; plane, p0: multiples of 4
+void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s);
+void launch_hwc_to_tensor(const float* hwc, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax);   // GPU_SHALLOW in; p0: a multiple of 4
+void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s);   // GPU_SHALLOW out, pc = 1, 2 or 4
+void launch_argmax_to_host(const int* idx, const TView& t, int* idx_out, float* val_out, size_t p0, size_t p1, const HostDone& done, hipStream_t s);
+void launch_tell_host(const HostDone& done, hipStream_t s);
 void launch_fill_zero(void* ptr, size_t bytes, hipStream_t s);
 int launch_poison_lds(hipStream_t s);   // debugging aid: all-ones words into every CU's LDS
 

@@ -765,14 +765,7 @@ void Net::copy_argmax(int layer_no, int32_t* idx, float* val) {
     FYN_HIP(hipSetDevice(device));
     ArgMaxLayer* l = dynamic_cast<ArgMaxLayer*>(layer(layer_no));
     if (!l) fail(FYN_ERR_INVALID, "layer %d is not an arg-max layer", layer_no);
-    const size_t n = (size_t)l->oh * l->ow;
-    FYN_HIP(hipStreamSynchronize(stream));
-    if (idx) FYN_HIP(hipMemcpy(idx, l->idx_dev, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (val) {
-        std::vector<float> chw(2 * n);
-        copy_result(layer_no, chw.data(), 0);
-        memcpy(val, chw.data() + n, n * sizeof(float));
-    }
+    download_argmax(l->idx_dev, l->tout().v, idx, val);
 }
 
 }  // namespace fynhip

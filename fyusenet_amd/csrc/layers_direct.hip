@@ -1,7 +1,6 @@
 // Bandwidth-bound layer kernels for gfx950 (no matrix cores): depthwise 3x3 convolution, pooling,
 // global pooling, explicit batch-norm, add/sub, concat, exact arg-max, the fully connected
-// matrix-vector product, a direct (fallback) convolution and the layout converters at the
-// upload/download boundary.  All operate on the channel-packed NHWC layout described in kernels.h;
+// matrix-vector product and a direct (fallback) convolution (the layout converters of the upload/download boundary are in layout.hip).  All operate on the channel-packed NHWC layout described in kernels.h;
 // one thread moves 4 consecutive channels of one pixel (16 B in fp32 storage, 8 B in fp16 storage),
 // consecutive threads touch consecutive channels, so every wavefront access is one contiguous run.
 // The activation of the producing layer is applied on input fetch (shaders/activation.inc:3-18).
@@ -1473,105 +1472,6 @@ void launch_shift_reduce(const ShiftReduceParams& p, hipStream_t s) {
     const size_t lds = (size_t)(256 + p.k - 1) * (p.q.cp + 1) * sizeof(float);
     if (p.out.f16) hipLaunchKernelGGL((shift_reduce_kernel<_Float16>), dim3(tiles_x * p.out.h), dim3(256), lds, s, p);
     else hipLaunchKernelGGL((shift_reduce_kernel<float>), dim3(tiles_x * p.out.h), dim3(256), lds, s, p);
-}
-
-// ---------------------------------------------------------------------------------------------
-// layout converters (UploadLayer / DownloadLayer / GPULayerBase::copyResult formats)
-// ---------------------------------------------------------------------------------------------
-// One thread converts four channels of one pixel; pixels are the fastest index, so that plane accesses are
-// contiguous across a wavefront (image-like tensors of up to 4 channels are contiguous on the packed side too).
-template <typename T>
-__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, const TView t, unsigned* amax) {
-    const size_t npix = (size_t)t.h * t.w;
-    const size_t n = npix * (t.cp >> 2);
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    float vmax = 0.f;
-    if (idx < n) {
-        const size_t pix = idx % npix;
-        const int c = (int)(idx / npix) * 4;
-        const int x = (int)(pix % t.w), y = (int)(pix / t.w);
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[i] = c + i < t.c ? chw[(size_t)(c + i) * npix + pix] : 0.f;
-            vmax = fmaxf(vmax, fabsf(v[i]));
-        }
-        st4<T>(reinterpret_cast<T*>(t.ptr) + tv_off(t, y, x) + c, make_float4(v[0], v[1], v[2], v[3]));
-    }
-    if (amax) range_publish_block256(amax, vmax);   // (every thread takes part)
-}
-void launch_chw_to_tensor(const float* chw, const TView& t, hipStream_t s, unsigned* amax) {
-    FYN_DISPATCH_T(t.f16, chw_to_tensor_kernel, grid1d((size_t)t.h * t.w * (t.cp >> 2), 256), dim3(256), s, chw, t, amax);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void tensor_to_chw_kernel(const TView t, float* chw, int keep_pad) {
-    const int oh = keep_pad ? t.hp() : t.h, ow = keep_pad ? t.wp() : t.w;
-    const size_t npix = (size_t)oh * ow;
-    const size_t n = npix * ((t.c + 3) >> 2);
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= n) return;
-    const size_t pix = idx % npix;
-    const int c = (int)(idx / npix) * 4;
-    const int x = (int)(pix % ow), y = (int)(pix / ow);
-    const int sy = keep_pad ? y : y + t.pad, sx = keep_pad ? x : x + t.pad;
-    const float4 v = ld4<T>(reinterpret_cast<const T*>(t.ptr) + ((size_t)sy * t.wp() + sx) * t.cp + c);
-    const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (c + i < t.c) chw[(size_t)(c + i) * npix + pix] = vv[i];
-}
-void launch_tensor_to_chw(const TView& t, float* chw, int include_padding, hipStream_t s) {
-    const int oh = include_padding ? t.hp() : t.h, ow = include_padding ? t.wp() : t.w;
-    FYN_DISPATCH_T(t.f16, tensor_to_chw_kernel, grid1d((size_t)oh * ow * ((t.c + 3) >> 2), 256), dim3(256), s, t, chw, include_padding);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, int pc, const TView t, unsigned* amax) {
-    const size_t n = (size_t)t.h * t.w * t.cp;
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    float vmax = 0.f;
-    if (idx < n) {
-        const int c = (int)(idx % t.cp);
-        const size_t pix = idx / t.cp;
-        const int x = (int)(pix % t.w), y = (int)(pix / t.w);
-        const float v = (c < t.c && c < pc) ? hwc[pix * pc + c] : 0.f;
-        reinterpret_cast<T*>(t.ptr)[tv_off(t, y, x) + c] = (T)v;
-        vmax = fabsf(v);
-    }
-    if (amax) range_publish_block256(amax, vmax);   // (every thread takes part)
-}
-void launch_hwc_to_tensor(const float* hwc, int pc, const TView& t, hipStream_t s, unsigned* amax) {
-    FYN_DISPATCH_T(t.f16, hwc_to_tensor_kernel, grid1d((size_t)t.h * t.w * t.cp, 256), dim3(256), s, hwc, pc, t, amax);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void tensor_to_hwc_kernel(const TView t, float* hwc, int pc) {
-    const size_t n = (size_t)t.h * t.w * pc;
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= n) return;
-    const int c = (int)(idx % pc);
-    const size_t pix = idx / pc;
-    const int x = (int)(pix % t.w), y = (int)(pix / t.w);
-    hwc[idx] = c < t.c ? (float)reinterpret_cast<const T*>(t.ptr)[tv_off(t, y, x) + c] : 0.f;
-}
-void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, hipStream_t s) {
-    FYN_DISPATCH_T(t.f16, tensor_to_hwc_kernel, grid1d((size_t)t.h * t.w * pc, 256), dim3(256), s, t, hwc, pc);
-}
-
-__global__ __launch_bounds__(256) void fill_zero_kernel(uint4* p, size_t n16, unsigned char* tail, size_t ntail) {
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * 256;
-    for (size_t i = idx; i < n16; i += stride) p[i] = make_uint4(0, 0, 0, 0);
-    if (idx < ntail) tail[idx] = 0;
-}
-void launch_fill_zero(void* ptr, size_t bytes, hipStream_t s) {
-    const size_t n16 = bytes / 16;
-    size_t blocks = (n16 + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<uint4*>(ptr), n16,
-                       reinterpret_cast<unsigned char*>(ptr) + n16 * 16, bytes - n16 * 16);
 }
 
 // Debugging aid: fills the LDS of every CU with all-ones words (a NaN as fp16 and as fp32, -1 as an integer).  The LDS

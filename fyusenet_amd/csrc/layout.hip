@@ -1,0 +1,247 @@
+// Layout converters between host buffers and device tensors.
+//
+// The host side of a transfer is page-locked memory that the kernels read and write in place, over PCIe: conversion and
+// transfer are one launch, where a copy into a device buffer followed by a conversion kernel (or the reverse) costs a
+// second launch and a round trip through the runtime's copy queue -- 10 us on a small frame.  What bounds them is the
+// link (about 55 GB/s each way), so a thread moves sixteen bytes per access and 128 workgroups are enough: measured on
+// 25 MB, 64 to 256 workgroups of such loads 448 us = 55 GB/s, 1024 workgroups 488 us, the copy engine alone 439 us.
+// The same kernels serve buffers in device memory.
+#include <hip/hip_fp16.h>
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "kernels.h"
+#include "range.h"
+
+namespace fynhip {
+
+namespace {
+constexpr unsigned kMaxBlocks = 128;
+
+// Stores of the workgroup's threads, then -- by the workgroup that arrives last -- the host's word: when the host reads
+// `value` there, everything the launch has written lies in memory.  A host that polls the word sees the result 5 us
+// earlier than one that waits for the stream (10.8 against 5.9 us around an empty kernel), because the stream's
+// completion signal is a packet of its own behind the kernel.
+__device__ __forceinline__ void tell_host(const HostDone& d) {
+    if (!d.flag) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence_system();
+        if (__hip_atomic_fetch_add(d.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+            __hip_atomic_store(d.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch on this stream
+            __threadfence_system();
+            __hip_atomic_store(d.flag, d.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ float4 load4(const T* p) {
+    if constexpr (sizeof(T) == 2) {
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        const h4 h = *reinterpret_cast<const h4*>(p);
+        return make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
+    } else {
+        return *reinterpret_cast<const float4*>(p);
+    }
+}
+template <typename T>
+__device__ __forceinline__ void store4(T* p, float a, float b, float c, float d) {
+    if constexpr (sizeof(T) == 2) {
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        h4 h;
+        h[0] = (_Float16)a; h[1] = (_Float16)b; h[2] = (_Float16)c; h[3] = (_Float16)d;
+        *reinterpret_cast<h4*>(p) = h;
+    } else {
+        *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
+    }
+}
+}  // namespace
+
+// Pixels [p0, p1) of planes `plane` floats apart (both multiples of four, as is the planes' address in units of four
+// floats): a thread takes four pixels of four channels.  Channels beyond the tensor's read as zero.
+template <typename T>
+__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, unsigned p0, unsigned p1, unsigned* amax) {
+    const unsigned quads = (p1 - p0 + 3) >> 2;
+    const size_t n = (size_t)quads * (t.cp >> 2);
+    float vmax = 0.f;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const unsigned pix = p0 + (unsigned)(i % quads) * 4;
+        const int c = (int)(i / quads) * 4;
+        float4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = c + k < t.c ? *reinterpret_cast<const float4*>(chw + (size_t)(c + k) * plane + pix) : make_float4(0.f, 0.f, 0.f, 0.f);
+        unsigned y = pix / (unsigned)t.w, x = pix - y * (unsigned)t.w;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (pix + j < p1) {
+                float e[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    e[k] = j == 0 ? v[k].x : j == 1 ? v[k].y : j == 2 ? v[k].z : v[k].w;
+                    vmax = fmaxf(vmax, fabsf(e[k]));
+                }
+                store4<T>(reinterpret_cast<T*>(t.ptr) + ((size_t)(y + t.pad) * t.wp() + x + t.pad) * t.cp + c, e[0], e[1], e[2], e[3]);
+            }
+            if (++x == (unsigned)t.w) {
+                x = 0;
+                y++;
+            }
+        }
+    }
+    if (amax) range_publish_block256(amax, vmax);   // (every thread takes part)
+}
+void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax) {
+    const size_t items = (p1 - p0 + 3) / 4 * (t.cp >> 2);
+    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
+    if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, (unsigned)p0, (unsigned)p1, amax);
+    else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, (unsigned)p0, (unsigned)p1, amax);
+}
+
+// Interleaved pixels of t.c floats: the buffer is read as one run of sixteen-byte pieces (an element's pixel and channel
+// follow from its index), the tensor's pad channels keep the zeros they were allocated with.  p0 * t.c is a multiple of
+// four; the last piece may reach up to three floats behind the buffer's end.
+template <typename T>
+__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, const TView t, size_t p0, size_t p1, unsigned* amax) {
+    const size_t e1 = p1 * t.c, q1 = (e1 + 3) >> 2;
+    float vmax = 0.f;
+    for (size_t q = p0 * t.c / 4 + (size_t)blockIdx.x * 256 + threadIdx.x; q < q1; q += (size_t)gridDim.x * 256) {
+        const float4 v = *reinterpret_cast<const float4*>(hwc + q * 4);
+        const float e[4] = {v.x, v.y, v.z, v.w};
+        unsigned pix = (unsigned)(q * 4 / t.c), c = (unsigned)(q * 4 - (size_t)pix * t.c);
+        unsigned y = pix / (unsigned)t.w, x = pix - y * (unsigned)t.w;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (q * 4 + k < e1) {
+                reinterpret_cast<T*>(t.ptr)[((size_t)(y + t.pad) * t.wp() + x + t.pad) * t.cp + c] = (T)e[k];
+                vmax = fmaxf(vmax, fabsf(e[k]));
+            }
+            if (++c == (unsigned)t.c) {
+                c = 0;
+                if (++x == (unsigned)t.w) {
+                    x = 0;
+                    y++;
+                }
+            }
+        }
+    }
+    if (amax) range_publish_block256(amax, vmax);
+}
+void launch_hwc_to_tensor(const float* hwc, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax) {
+    const size_t items = ((p1 - p0) * t.c + 3) / 4;
+    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
+    if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, p0, p1, amax);
+    else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, p0, p1, amax);
+}
+
+// Pixels [p0, p1) of the net area (keep_pad: of the area with its halo) to planes `plane` floats apart.  Q = 4: a thread
+// takes four pixels of four channels, planes on sixteen-byte boundaries (p0 a multiple of four, the last piece may
+// reach up to three floats behind a plane); Q = 1: one pixel of four channels, any planes.
+template <typename T, int Q>
+__global__ __launch_bounds__(256) void tensor_to_chw_kernel(const TView t, float* chw, size_t plane, int keep_pad, unsigned p0, unsigned p1, const HostDone done) {
+    const unsigned ow = (unsigned)(keep_pad ? t.wp() : t.w);
+    const int off = keep_pad ? 0 : t.pad;
+    const unsigned groups = (p1 - p0 + Q - 1) / Q;
+    const size_t n = (size_t)groups * ((t.c + 3) >> 2);
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const unsigned pix = p0 + (unsigned)(i % groups) * Q;
+        const int c = (int)(i / groups) * 4;
+        unsigned y = pix / ow, x = pix - y * ow;
+        float4 v[Q];
+#pragma unroll
+        for (int j = 0; j < Q; j++) {
+            v[j] = pix + j < p1 ? load4<T>(reinterpret_cast<const T*>(t.ptr) + ((size_t)(y + off) * t.wp() + x + off) * t.cp + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+            if (++x == ow) {
+                x = 0;
+                y++;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            float e[Q];
+#pragma unroll
+            for (int j = 0; j < Q; j++) e[j] = k == 0 ? v[j].x : k == 1 ? v[j].y : k == 2 ? v[j].z : v[j].w;
+            if (c + k < t.c) {
+                float* dst = chw + (size_t)(c + k) * plane + pix;
+                if constexpr (Q == 4) *reinterpret_cast<float4*>(dst) = make_float4(e[0], e[1], e[2], e[3]);
+                else *dst = e[0];
+            }
+        }
+    }
+    tell_host(done);
+}
+void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
+    const bool quad = plane % 4 == 0 && (reinterpret_cast<size_t>(chw) & 15) == 0 && p0 % 4 == 0;
+    const size_t items = (p1 - p0 + (quad ? 3 : 0)) / (quad ? 4 : 1) * ((t.c + 3) >> 2);
+    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
+    const unsigned a = (unsigned)p0, b = (unsigned)p1;
+    if (t.f16) {
+        if (quad) hipLaunchKernelGGL((tensor_to_chw_kernel<_Float16, 4>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
+        else hipLaunchKernelGGL((tensor_to_chw_kernel<_Float16, 1>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
+    } else {
+        if (quad) hipLaunchKernelGGL((tensor_to_chw_kernel<float, 4>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
+        else hipLaunchKernelGGL((tensor_to_chw_kernel<float, 1>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
+    }
+}
+
+// Interleaved pixels of PC = 1, 2 or 4 floats: a pixel per thread, one store each.
+template <typename T, int PC>
+__global__ __launch_bounds__(256) void tensor_to_hwc_kernel(const TView t, float* hwc, size_t p0, size_t p1, const HostDone done) {
+    for (size_t pix = p0 + (size_t)blockIdx.x * 256 + threadIdx.x; pix < p1; pix += (size_t)gridDim.x * 256) {
+        const unsigned y = (unsigned)pix / (unsigned)t.w, x = (unsigned)pix - y * (unsigned)t.w;
+        const float4 v = load4<T>(reinterpret_cast<const T*>(t.ptr) + ((size_t)(y + t.pad) * t.wp() + x + t.pad) * t.cp);
+        if constexpr (PC == 4) *reinterpret_cast<float4*>(hwc + pix * 4) = make_float4(v.x, v.y, v.z, t.c > 3 ? v.w : 0.f);
+        else if constexpr (PC == 2) *reinterpret_cast<float2*>(hwc + pix * 2) = make_float2(v.x, v.y);
+        else hwc[pix] = v.x;
+    }
+    tell_host(done);
+}
+template <typename T>
+static void launch_hwc_out(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
+    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (p1 - p0 + 255) / 256));
+    if (pc == 4) hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 4>), grid, dim3(256), 0, s, t, hwc, p0, p1, done);
+    else if (pc == 2) hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 2>), grid, dim3(256), 0, s, t, hwc, p0, p1, done);
+    else hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 1>), grid, dim3(256), 0, s, t, hwc, p0, p1, done);
+}
+void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
+    if (t.f16) launch_hwc_out<_Float16>(t, hwc, pc, p0, p1, done, s);
+    else launch_hwc_out<float>(t, hwc, pc, p0, p1, done, s);
+}
+
+// An arg-max layer's two results: the exact indices it keeps beside its tensor, and the tensor's second channel.
+template <typename T>
+__global__ __launch_bounds__(256) void argmax_to_host_kernel(const int* idx, const TView t, int* idx_out, float* val_out, size_t p0, size_t p1, const HostDone done) {
+    for (size_t pix = p0 + (size_t)blockIdx.x * 256 + threadIdx.x; pix < p1; pix += (size_t)gridDim.x * 256) {
+        const unsigned y = (unsigned)pix / (unsigned)t.w, x = (unsigned)pix - y * (unsigned)t.w;
+        if (idx_out) idx_out[pix] = idx[pix];
+        if (val_out) val_out[pix] = (float)reinterpret_cast<const T*>(t.ptr)[((size_t)(y + t.pad) * t.wp() + x + t.pad) * t.cp + 1];
+    }
+    tell_host(done);
+}
+void launch_argmax_to_host(const int* idx, const TView& t, int* idx_out, float* val_out, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
+    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (p1 - p0 + 255) / 256));
+    if (t.f16) hipLaunchKernelGGL(argmax_to_host_kernel<_Float16>, grid, dim3(256), 0, s, idx, t, idx_out, val_out, p0, p1, done);
+    else hipLaunchKernelGGL(argmax_to_host_kernel<float>, grid, dim3(256), 0, s, idx, t, idx_out, val_out, p0, p1, done);
+}
+
+__global__ void tell_host_kernel(const HostDone done) { tell_host(done); }
+void launch_tell_host(const HostDone& done, hipStream_t s) { hipLaunchKernelGGL(tell_host_kernel, dim3(1), dim3(64), 0, s, done); }
+
+__global__ __launch_bounds__(256) void fill_zero_kernel(uint4* p, size_t n16, unsigned char* tail, size_t ntail) {
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t stride = (size_t)gridDim.x * 256;
+    for (size_t i = idx; i < n16; i += stride) p[i] = make_uint4(0, 0, 0, 0);
+    if (idx < ntail) tail[idx] = 0;
+}
+void launch_fill_zero(void* ptr, size_t bytes, hipStream_t s) {
+    const size_t n16 = bytes / 16;
+    size_t blocks = (n16 + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    if (blocks == 0) blocks = 1;
+    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<uint4*>(ptr), n16,
+                       reinterpret_cast<unsigned char*>(ptr) + n16 * 16, bytes - n16 * 16);
+}
+
+}  // namespace fynhip

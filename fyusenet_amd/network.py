@@ -64,7 +64,7 @@ class Layer:
         c, h, w, p = self.outputShape()
         if includePadding:
             h, w = h + 2 * p, w + 2 * p
-        out = np.empty((c, h, w), dtype=np.float32)
+        out = capi.result_array((c, h, w))
         capi.check(capi.lib().fyn_layer_copy_result(self._net._h, self.number, capi.fptr(out), 1 if includePadding else 0))
         return out
 
@@ -253,9 +253,9 @@ class NeuralNetwork:
         lyr = self.layers[layer] if not isinstance(layer, Layer) else layer
         c, h, w, p = lyr.outputShape()
         if order == capi.ORDER_CHANNELWISE:
-            out = np.empty((c, h, w), dtype=np.float32)
+            out = capi.result_array((c, h, w))
         elif order == capi.ORDER_GPU_SHALLOW:
-            out = np.empty((h, w, 4 if c == 3 else c), dtype=np.float32)
+            out = capi.result_array((h, w, 4 if c == 3 else c))
         else:
             from .formats import deep_tiling
             tx, ty = deep_tiling(c)
@@ -266,8 +266,8 @@ class NeuralNetwork:
     def getArgMax(self, layer):
         lyr = self.layers[layer] if not isinstance(layer, Layer) else layer
         c, h, w, p = lyr.outputShape()
-        idx = np.empty((h, w), dtype=np.int32)
-        val = np.empty((h, w), dtype=np.float32)
+        idx = capi.result_array((h, w), np.int32)
+        val = capi.result_array((h, w))
         capi.check(capi.lib().fyn_layer_copy_argmax(self._h, lyr.number, idx.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), capi.fptr(val)))
         return idx, val
 

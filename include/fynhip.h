@@ -282,8 +282,15 @@ int fyn_net_async_wait(fyn_net* net, uint64_t ticket);
 /* Floats per frame that submit reads from `in` and writes to `out` (between begin and end). */
 int fyn_net_async_sizes(fyn_net* net, size_t* in_floats, size_t* out_floats);
 int fyn_net_async_end(fyn_net* net);
-/* Device allocations this network has made since fyn_net_create: number of hipMalloc calls and the bytes asked for
- * (both only ever grow).  A diagnostic without a counterpart in the reference, whose textures belong to the GL driver;
+/* Memory for results that the GPU writes in place, over PCIe: fyn_net_get_output, fyn_layer_copy_result and
+ * fyn_layer_copy_argmax into such memory skip the copy from the library's own page-locked area and the first touch of
+ * fresh pages.  *ptr is NULL (and the call succeeds) where none is to be had: no network exists, or 512 MiB are taken
+ * already; use ordinary memory then.  Blocks may be released from any thread and outlive the network; they are kept for
+ * the next caller and go back to the system with the last network.  No counterpart in the reference. */
+int fyn_host_acquire(size_t bytes, void** ptr);
+int fyn_host_release(void* ptr);
+/* Device allocations this network has made since fyn_net_create: number of hipMalloc calls (and of page-locked staging
+ * areas taken) and the bytes asked for (both only ever grow).  A diagnostic without a counterpart in the reference, whose textures belong to the GL driver;
  * it lets a caller check that a call sequence of its serving loop allocates nothing. */
 int fyn_net_device_allocations(fyn_net* net, size_t* calls, size_t* bytes);
 /* Text description of the kernel variant chosen for a layer (for profiles / reports). */
