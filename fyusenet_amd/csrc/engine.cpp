@@ -71,17 +71,64 @@ const Tensor& Layer::tout() const { return net->tensors[out]; }
 // overlap each other badly (four ResNet-50 instances side by side: 3000 frames/s instead of 4700), whereas streams
 // that exist by then are unaffected by later graph launches.  Leasing also keeps the stream count of a process that
 // builds and destroys many networks constant.  Streams are never destroyed; a network that finds none free gets a
-// new one.  The first kMainStreams entries serve networks' own streams (consecutive ones land on different hardware
-// queues), the rest their copy streams.
+// new one.  The first kMainStreams entries serve networks' own streams, the rest their copy streams.
+//
+// The process has a few hardware queues (4 by default) and a stream is tied to one of them when it is created; kernels
+// of two streams that share a queue never overlap, whatever else is idle.  Which streams share one is up to the runtime
+// (and to the streams that the application made before), so it is found out once, when the streams are created: a stream
+// whose kernel never ran at the same time as a busy one's shares its queue.  A lease then takes a stream of the queue
+// that has the fewest leases.  Four ResNet-50 instances side by side with one other network alive: 154 us per frame where
+// two of them shared a queue, 108 us where each had its own.
 // ---------------------------------------------------------------------------------------------
 namespace {
 struct DeviceStreams {
     std::vector<hipStream_t> streams;
     std::vector<char> leased;
+    std::vector<int> queue;   // streams with equal numbers share a hardware queue
+    std::map<int, uint64_t> last;   // queue -> when a stream of it was leased last
+    uint64_t leases = 0;
 };
 constexpr size_t kMainStreams = 8, kCopyStreams = 8;
 std::mutex g_streams_mu;
 std::map<int, DeviceStreams> g_streams;
+
+__global__ void occupy_kernel(unsigned long long ticks, unsigned long long* span) {
+    const unsigned long long t0 = wall_clock64();
+    unsigned long long t = t0;
+    while (t - t0 < ticks) t = wall_clock64();
+    span[0] = t0;
+    span[1] = t;
+}
+
+// Fills ds.queue: every stream's kernel is run beside one of each queue known so far.
+void find_queues(DeviceStreams& ds) {
+    const size_t n = ds.streams.size();
+    ds.queue.assign(n, 0);
+    unsigned long long* span = nullptr;   // [stream][start, end]
+    if (hipHostMalloc(reinterpret_cast<void**>(&span), n * 2 * sizeof(*span), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    const unsigned long long ticks = 5000;   // 50 us of the 100 MHz clock: longer than it takes to launch two kernels
+    auto run = [&](size_t i, unsigned long long t) { hipLaunchKernelGGL(occupy_kernel, dim3(1), dim3(1), 0, ds.streams[i], t, span + 2 * i); };
+    for (size_t i = 0; i < n; i++) run(i, 1);   // (a stream's first launch takes longer)
+    for (size_t i = 0; i < n; i++) (void)hipStreamSynchronize(ds.streams[i]);
+    std::vector<size_t> first;   // one stream of each queue
+    for (size_t j = 0; j < n; j++) {
+        size_t q = 0;
+        for (; q < first.size(); q++) {
+            run(first[q], ticks);
+            run(j, ticks);
+            (void)hipStreamSynchronize(ds.streams[first[q]]);
+            (void)hipStreamSynchronize(ds.streams[j]);
+            if (span[2 * j] >= span[2 * first[q] + 1]) break;   // one behind the other
+        }
+        if (q == first.size()) first.push_back(j);
+        ds.queue[j] = (int)q;
+    }
+    (void)hipHostFree(span);
+    FYN_HIP(hipGetLastError());
+}
 
 hipStream_t lease_stream(int device, bool copy) {
     std::lock_guard<std::mutex> lk(g_streams_mu);
@@ -94,13 +141,21 @@ hipStream_t lease_stream(int device, bool copy) {
             ds.streams.push_back(st);
             ds.leased.push_back(0);
         }
+        find_queues(ds);
     }
+    std::map<int, int> count;
+    for (size_t i = 0; i < ds.streams.size(); i++) count[ds.queue[i]] += ds.leased[i];
+    // (equal counts: the queue whose last lease is longest ago, so that networks made together get queues of their own)
+    auto better = [&](int a, int b) { return count[a] != count[b] ? count[a] < count[b] : ds.last[a] < ds.last[b]; };
     const size_t lo = copy ? kMainStreams : 0, hi = copy ? kMainStreams + kCopyStreams : kMainStreams;
+    size_t best = hi;
     for (size_t i = lo; i < hi; i++)
-        if (!ds.leased[i]) {
-            ds.leased[i] = 1;
-            return ds.streams[i];
-        }
+        if (!ds.leased[i] && (best == hi || better(ds.queue[i], ds.queue[best]))) best = i;
+    if (best < hi) {
+        ds.leased[best] = 1;
+        ds.last[ds.queue[best]] = ++ds.leases;
+        return ds.streams[best];
+    }
     hipStream_t st = nullptr;   // all taken: one more, destroyed again when it comes back
     if (copy) FYN_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     else FYN_HIP(hipStreamCreate(&st));
@@ -927,12 +982,21 @@ void Net::time_layer(int layer_no, int iters, float* ms) {
 
 // ---------------------------------------------------------------------------------------------
 // Frame pipeline (the counterpart of the reference engine's asynchronous mode, base/engine.cpp:386-683, with
-// its two upload/download buffer sets, gpu/uploadlayer.h:74): three streams of equal priority joined by events.
-// Frame i:   up stream    pinned host slot -> device staging slot
-//            main stream  staging -> input tensor, all layers, output tensor -> device staging slot
-//            down stream  device staging slot -> pinned host slot
-// A slot is reused only after its download has completed, which also orders the staging buffers.
+// its two upload/download buffer sets, gpu/uploadlayer.h:74).  Two forms:
+//   overlapped   three streams of equal priority joined by events, for one network with large frames:
+//                up stream    page-locked slot -> device staging slot (copy engine)
+//                main stream  staging -> input tensor, all layers, output tensor -> device staging slot
+//                down stream  device staging slot -> page-locked slot (copy engine).  The copy is made as one of rows with
+//                gaps between them: some versions of the runtime carry out plain copies to the host with a kernel, and
+//                every workgroup of such a kernel keeps a CU for the 90 us of a frame from layers that need it whole.
+//   in place     everything on the network's stream, the layout kernels reading and writing the page-locked slots over
+//                the link: networks that run side by side overlap each other's transfers, and where the transfers of a
+//                frame take less than the two hand-overs between streams (about 20 us = 1 MB) nothing is gained by them.
+// There is one slot more than frames that may be in flight between two calls: submit() queues its frame first and
+// delivers the one that has to leave afterwards, so that the GPU has the next frame in its queue while the host copies.
 // ---------------------------------------------------------------------------------------------
+static constexpr size_t kRowGap = 256;   // bytes between the rows of an overlapped download
+
 void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, int out_order, int depth, bool copy_streams) {
     if (!is_setup) fail(FYN_ERR_STATE, "async_begin() before setup()");
     if (!slots_.empty()) fail(FYN_ERR_STATE, "frame pipeline is already active");
@@ -963,29 +1027,42 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
     async_in_plane_ = ((size_t)vi.h * vi.w + 3) & ~size_t(3);
     async_in_order_ = in_order;
     async_out_order_ = out_order;
-    async_own_streams_ = copy_streams;
+    async_own_streams_ = copy_streams && (async_in_floats_ + async_out_floats_) * sizeof(float) > (1u << 20);
+    async_depth_ = depth;
+    const size_t in_bytes = async_in_plane_ * vi.c * sizeof(float), out_bytes = async_out_floats_ * sizeof(float);
     if (async_own_streams_) {
         up_stream_ = lease_stream(device, true);
         down_stream_ = lease_stream(device, true);
-    } else {
-        up_stream_ = down_stream_ = stream;
+        const size_t rows = std::max<size_t>(4, (out_bytes + (1u << 20) - 1) >> 20);
+        async_row_ = (out_bytes / rows + 255 + 1) & ~size_t(255);
+        async_rows_ = (out_bytes + async_row_ - 1) / async_row_;
     }
-    slots_.resize(depth);
+    slots_.resize(depth + 1);
     for (AsyncSlot& s : slots_) {
-        FYN_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.pin_in), async_in_plane_ * vi.c * sizeof(float), hipHostMallocDefault));
-        FYN_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.pin_out), async_out_floats_ * sizeof(float), hipHostMallocDefault));
-        FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), async_in_plane_ * vi.c * sizeof(float)));
-        FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_out), async_out_floats_ * sizeof(float)));
+        s.pin_in = static_cast<float*>(HostPool::acquire(in_bytes, false));
+        s.pin_out = static_cast<float*>(HostPool::acquire(async_own_streams_ ? async_rows_ * (async_row_ + kRowGap) : out_bytes, false));
+        if (!async_own_streams_) continue;
+        FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), in_bytes));
+        FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_out), async_rows_ * async_row_));
         FYN_HIP(hipEventCreateWithFlags(&s.up, hipEventDisableTiming));
         FYN_HIP(hipEventCreateWithFlags(&s.comp, hipEventDisableTiming));
         FYN_HIP(hipEventCreateWithFlags(&s.down, hipEventDisableTiming));
     }
 }
 
+constexpr size_t kPipelineShared = 1u << 20;   // copies of a pipeline from this size on are shared with the helper threads
+
 void Net::async_complete(AsyncSlot& s) {
     if (!s.busy) return;
-    FYN_HIP(hipEventSynchronize(s.down));
-    if (s.user_out) memcpy(s.user_out, s.pin_out, async_out_floats_ * sizeof(float));
+    if (async_own_streams_) FYN_HIP(hipEventSynchronize(s.down));
+    else signal_.wait(s.value, stream);
+    if (s.user_out) {
+        HostCopy out;
+        const size_t bytes = async_out_floats_ * sizeof(float), row = async_own_streams_ ? async_row_ : bytes;
+        for (size_t o = 0, r = 0; o < bytes; o += row, r++)
+            out.add(reinterpret_cast<char*>(s.user_out) + o, reinterpret_cast<char*>(s.pin_out) + r * (row + kRowGap), std::min(row, bytes - o));
+        out.start(kPipelineShared);
+    }
     s.busy = false;
 }
 
@@ -994,31 +1071,47 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
     if (!in || !out) fail(FYN_ERR_INVALID, "null frame buffer");
     FYN_HIP(hipSetDevice(device));
     AsyncSlot& s = slots_[async_seq_ % slots_.size()];
-    async_complete(s);  // oldest frame: its output is delivered before the slot is reused
+    async_complete(s);
     const TView& vi = async_in_->v;
-    const size_t npix = (size_t)vi.h * vi.w;
-    if (async_in_order_ == FYN_ORDER_CHANNELWISE)
-        for (int c = 0; c < vi.c; c++) memcpy(s.pin_in + c * async_in_plane_, in + c * npix, npix * sizeof(float));
-    else memcpy(s.pin_in, in, async_in_floats_ * sizeof(float));
-    FYN_HIP(hipMemcpyAsync(s.dev_in, s.pin_in, async_in_plane_ * vi.c * sizeof(float), hipMemcpyHostToDevice, up_stream_));
-    FYN_HIP(hipEventRecord(s.up, up_stream_));
-    FYN_HIP(hipStreamWaitEvent(stream, s.up, 0));
-    if (async_in_->amax) launch_fill_zero(async_in_->amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
-    if (async_in_order_ == FYN_ORDER_CHANNELWISE) launch_chw_to_tensor(s.dev_in, async_in_plane_, vi, 0, npix, stream, async_in_->amax);
-    else launch_hwc_to_tensor(s.dev_in, vi, 0, npix, stream, async_in_->amax);
-    forward(nullptr);
     const TView& vo = async_out_view_;
-    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, s.dev_out, (size_t)vo.h * vo.w, 0, 0, (size_t)vo.h * vo.w, HostDone{}, stream);
-    else launch_tensor_to_hwc(vo, s.dev_out, vo.c == 3 ? 4 : vo.c, 0, (size_t)vo.h * vo.w, HostDone{}, stream);
+    const size_t npix = (size_t)vi.h * vi.w, opix = (size_t)vo.h * vo.w;
+    const bool planes = async_in_order_ == FYN_ORDER_CHANNELWISE;
+    {
+        HostCopy copies;
+        if (planes)
+            for (int c = 0; c < vi.c; c++) copies.add(s.pin_in + c * async_in_plane_, in + c * npix, npix * sizeof(float));
+        else copies.add(s.pin_in, in, async_in_floats_ * sizeof(float));
+        copies.start(kPipelineShared);
+    }
+    const float* src = s.pin_in;
+    if (async_own_streams_) {
+        FYN_HIP(hipMemcpyAsync(s.dev_in, s.pin_in, async_in_plane_ * vi.c * sizeof(float), hipMemcpyHostToDevice, up_stream_));
+        FYN_HIP(hipEventRecord(s.up, up_stream_));
+        FYN_HIP(hipStreamWaitEvent(stream, s.up, 0));
+        src = s.dev_in;
+    }
+    if (async_in_->amax) launch_fill_zero(async_in_->amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
+    if (planes) launch_chw_to_tensor(src, async_in_plane_, vi, 0, npix, stream, async_in_->amax);
+    else launch_hwc_to_tensor(src, vi, 0, npix, stream, async_in_->amax);
+    forward(nullptr);
+    float* dst = async_own_streams_ ? s.dev_out : s.pin_out;
+    const HostDone done = async_own_streams_ ? HostDone{} : signal_.next();
+    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, dst, opix, 0, 0, opix, done, stream);
+    else launch_tensor_to_hwc(vo, dst, vo.c == 3 ? 4 : vo.c, 0, opix, done, stream);
+    s.value = done.value;
+    if (async_own_streams_) {
+        FYN_HIP(hipGetLastError());
+        FYN_HIP(hipEventRecord(s.comp, stream));
+        FYN_HIP(hipStreamWaitEvent(down_stream_, s.comp, 0));
+        FYN_HIP(hipMemcpy2DAsync(s.pin_out, async_row_ + kRowGap, s.dev_out, async_row_, async_row_, async_rows_, hipMemcpyDeviceToHost, down_stream_));
+        FYN_HIP(hipEventRecord(s.down, down_stream_));
+    }
     FYN_HIP(hipGetLastError());
-    FYN_HIP(hipEventRecord(s.comp, stream));
-    FYN_HIP(hipStreamWaitEvent(down_stream_, s.comp, 0));
-    FYN_HIP(hipMemcpyAsync(s.pin_out, s.dev_out, async_out_floats_ * sizeof(float), hipMemcpyDeviceToHost, down_stream_));
-    FYN_HIP(hipEventRecord(s.down, down_stream_));
     s.user_out = out;
     s.busy = true;
     s.ticket = ++async_seq_;
     if (ticket) *ticket = s.ticket;
+    if (async_seq_ > (uint64_t)async_depth_) async_complete(slots_[(async_seq_ - async_depth_ - 1) % slots_.size()]);
 }
 
 void Net::async_wait(uint64_t ticket) {
@@ -1041,8 +1134,8 @@ void Net::async_end() {
     }
     if (stream) (void)hipStreamSynchronize(stream);
     for (AsyncSlot& s : slots_) {
-        if (s.pin_in) (void)hipHostFree(s.pin_in);
-        if (s.pin_out) (void)hipHostFree(s.pin_out);
+        HostPool::release(s.pin_in);
+        HostPool::release(s.pin_out);
         if (s.dev_in) (void)hipFree(s.dev_in);
         if (s.dev_out) (void)hipFree(s.dev_out);
         if (s.up) (void)hipEventDestroy(s.up);

@@ -158,6 +158,7 @@ class Net {
     struct AsyncSlot {
         float *pin_in = nullptr, *pin_out = nullptr, *dev_in = nullptr, *dev_out = nullptr;
         hipEvent_t up = nullptr, comp = nullptr, down = nullptr;
+        unsigned value = 0;   // in place: what the stream's word reads when pin_out is filled
         float* user_out = nullptr;
         uint64_t ticket = 0;
         bool busy = false;
@@ -167,6 +168,8 @@ class Net {
     const Tensor* async_in_ = nullptr;
     const Tensor* async_out_ = nullptr;
     bool async_own_streams_ = true;
+    int async_depth_ = 0;
+    size_t async_row_ = 0, async_rows_ = 0;   // bytes of a row and rows of an overlapped download
     TView async_out_view_{};   // what the output layer hands out (a download layer may name other channel counts)
     int async_in_order_ = 0, async_out_order_ = 0;
     size_t async_in_floats_ = 0, async_out_floats_ = 0, async_in_plane_ = 0;   // (planes lie on multiples of four floats)

@@ -146,7 +146,7 @@ struct HostCopy::Job {
 // The helper threads.  They sleep while there is nothing to copy; the object is never destroyed, so that they may be
 // asleep in it when the process ends.
 struct HostCopyHelpers {
-    static constexpr size_t kSlice = 256u << 10, kAlone = 8u << 20;   // (waking a thread takes 20 to 50 us, and smaller buffers tend to lie in this core's caches: those jobs are done alone)
+    static constexpr size_t kSlice = 256u << 10;
     std::mutex mu;
     std::condition_variable cv;
     std::deque<std::shared_ptr<HostCopy::Job>> jobs;
@@ -193,9 +193,9 @@ void HostCopy::add(void* dst, const void* src, size_t bytes) {
     job_->bytes += bytes;
 }
 size_t HostCopy::mark() const { return job_->slices.size(); }
-void HostCopy::start() {
+void HostCopy::start(size_t alone) {
     job_->made.reset(new std::atomic<char>[job_->slices.size()]());
-    if (job_->bytes >= HostCopyHelpers::kAlone) HostCopyHelpers::get().offer(job_);
+    if (job_->bytes >= alone) HostCopyHelpers::get().offer(job_);
 }
 void HostCopy::upto(size_t mark) {
     for (;;) {

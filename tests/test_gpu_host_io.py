@@ -1,0 +1,111 @@
+"""Host frames and results at the edges of the layout kernels and of the transfers' pieces (fyusenet/gpu/uploadlayer.cpp:92-186,
+gpulayerbase.cpp:525-564): a copy layer hands back what was put in, through every host layout, into memory of the
+library's and of the caller's own."""
+import numpy as np
+import pytest
+
+import fyusenet_amd as fa
+from fyusenet_amd import capi, prng, samples
+
+STORAGES = pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+
+
+def _copy_net(c, h, w, storage, pad=0):
+    class Net(fa.NeuralNetwork):
+        def buildLayers(self, f):
+            b = fa.ConcatLayerBuilder("copy").number(1).deep().input(c, 0).outputPadding(pad)
+            b.size(w, h)
+            b.outputChannels_ = c
+            b.push(f)
+
+        def connectLayers(self, layers, bm):
+            pass
+
+    net = Net(storage)
+    net.setup()
+    return net
+
+
+@pytest.mark.gpu
+@STORAGES
+@pytest.mark.parametrize("c,h,w", [(1, 1, 1), (3, 1, 2), (3, 5, 7), (4, 1, 3), (2, 9, 4), (8, 33, 41), (70, 50, 61), (3, 701, 433), (4, 1201, 640), (260, 63, 65)])
+def test_frames_come_back_as_they_went_in(c, h, w, storage):
+    pad = 2
+    net = _copy_net(c, h, w, storage, pad)
+    lyr = net.layers[1]
+    x = prng.uniform(500 + c * h, (c, h, w), -2.0, 2.0)
+    want = x if storage == fa.STORAGE_F32 else x.astype(np.float16).astype(np.float32)
+    orders = [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW]
+    for order in orders:
+        lyr.setInput(np.zeros_like(x), 0)
+        lyr.setInput(x if order == fa.ORDER_CHANNELWISE else np.ascontiguousarray(x.transpose(1, 2, 0)), 0, order)
+        net.forward()
+        assert np.array_equal(net.getOutput(1), want), order
+        own = np.full(x.shape, np.nan, np.float32)
+        capi.check(capi.lib().fyn_net_get_output(net._h, 1, capi.fptr(own), fa.ORDER_CHANNELWISE))
+        assert np.array_equal(own, want), order
+    halo = lyr.copyResult(includePadding=True)
+    assert np.array_equal(halo[:, pad:-pad, pad:-pad], want) and np.count_nonzero(halo) == np.count_nonzero(want)
+    if c <= 4:
+        pc = 4 if c == 3 else c
+        own = np.full((h, w, pc), np.nan, np.float32)
+        capi.check(capi.lib().fyn_net_get_output(net._h, 1, capi.fptr(own), fa.ORDER_GPU_SHALLOW))
+        for got in (net.getOutput(1, fa.ORDER_GPU_SHALLOW), own):
+            assert np.array_equal(got[..., :c].transpose(2, 0, 1), want) and not got[..., c:].any()
+    net.cleanup()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order", [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW], ids=["chw", "hwc"])
+@pytest.mark.parametrize("width,height,depth", [(404, 300, 1), (404, 300, 2), (660, 500, 3)])
+def test_overlapped_pipeline_matches_the_synchronous_path(width, height, depth, order):
+    """Frames large enough for streams of their own: the upload of a frame runs beside the layers of the one before it,
+    and its result leaves while the next is computed."""
+    net = samples.StyleNetSample(3, width, height)
+    net.setup()
+    hwc = order == fa.ORDER_GPU_SHALLOW
+    frames = [prng.uniform(3300 + i, (height, width, 3) if hwc else (3, height, width), 0.0, 1.0) for i in range(2 * depth + 3)]
+    want = []
+    for f in frames:
+        net.layers[net.UPLOAD].setInput(f, 0, order)
+        net.forward()
+        want.append(net.getOutput(net.output_layer, order))
+    assert not np.array_equal(want[0], want[1])
+    net.asyncBegin(net.UPLOAD, net.output_layer, inOrder=order, outOrder=order, depth=depth)
+    outs = [np.full_like(want[0], np.nan) for _ in frames]
+    for i, (f, o) in enumerate(zip(frames, outs)):
+        ticket = net.asyncSubmit(f, o)
+        for k in range(i - depth + 1):
+            assert np.array_equal(outs[k], want[k]), (i, k)
+    net.asyncWait(ticket)
+    for i in range(len(frames)):
+        assert np.array_equal(outs[i], want[i]), i
+    net.asyncEnd()
+    net.cleanup()
+
+
+@pytest.mark.gpu
+def test_results_belong_to_the_caller():
+    """A result handed out stays what it was while later frames pass and after the network has gone; memory of results
+    that nobody holds is used again."""
+    net = _copy_net(4, 120, 160, fa.STORAGE_F32)
+    kept = []
+    for i in range(6):
+        net.layers[1].setInput(np.full((4, 120, 160), i, np.float32), 0)
+        net.forward()
+        kept.append(net.getOutput(1))
+    assert len({k.ctypes.data for k in kept}) == 6
+    address = kept.pop(2).ctypes.data
+    again = net.getOutput(1)
+    assert again.ctypes.data == address and (again == 5).all()
+    net.cleanup()
+    for value, k in zip((0, 1, 3, 4, 5), kept):
+        assert (k == value).all()
+
+
+
+def test_results_without_any_network_lie_in_ordinary_memory():
+    capi.check(capi.lib().fyn_host_release(None))
+    a = capi.result_array((64, 1024))
+    a[:] = 1
+    assert a.shape == (64, 1024) and a.dtype == np.float32
