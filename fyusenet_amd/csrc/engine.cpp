@@ -2,7 +2,10 @@
 #include "engine.h"
 #include "range.h"
 
+#include <immintrin.h>
+
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <limits>
 #include <map>
@@ -231,6 +234,12 @@ Net::Net(int dev, int stor) : device(dev), storage(stor) {
         // resolved here, where the caller may still allocate: looking the symbol up loads the code object on this device
         static_scratch_ = static_scratch(dev);
         signal_.create(static_cast<unsigned*>(dev_alloc(64)));
+        upload_words_ = static_cast<unsigned*>(dev_alloc(64));
+        feed_ = static_cast<FeedWord*>(HostPool::acquire(sizeof(FeedWord), false));
+        *feed_ = FeedWord{};
+        // (where the runtime is told to finish a launch before the call returns, the frame is copied first)
+        for (const char* e : {"HIP_LAUNCH_BLOCKING", "CUDA_LAUNCH_BLOCKING", "AMD_SERIALIZE_KERNEL"})
+            if (const char* v = getenv(e)) feed_ahead_ = feed_ahead_ && (!*v || *v == '0');
     } catch (...) {
         release_all();
         throw;
@@ -242,6 +251,7 @@ void Net::release_all() {
     for (void* p : allocs_) (void)hipFree(p);
     allocs_.clear();
     signal_.destroy();
+    HostPool::release(feed_);
     HostPool::release(in_pin_);
     return_stream(device, stream);
     HostPool::network_gone();
@@ -611,6 +621,10 @@ void Net::finish() {
 void Net::wait_signal(unsigned value) {
     signal_.wait(value, stream);
     if (value == signal_.last()) settled();
+    if (__atomic_load_n(&feed_->late, __ATOMIC_RELAXED)) {
+        feed_->late = 0;
+        fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
+    }
 }
 
 // The stream is idle: nothing reads the input area any more.
@@ -683,44 +697,62 @@ void Net::async_sizes(size_t* in_floats, size_t* out_floats) const {
     *out_floats = async_out_floats_;
 }
 
-// A host transfer in pieces: while the link moves one, the host copies the next.  Pieces below a megabyte are not worth
+// A result in pieces: while the link moves one, the host copies the one before.  Pieces below a megabyte are not worth
 // their launches (4 us each).
 static size_t piece_pixels(size_t npix, size_t bytes) {
     const size_t pieces = std::min<size_t>(12, std::max<size_t>(1, bytes / (1280u << 10)));
     return std::max<size_t>(4, ((npix + pieces - 1) / pieces + 3) & ~size_t(3));
 }
 
+// A frame into its tensor.  Host memory: the converting launch is queued first and takes the pixels as the host puts them
+// into page-locked memory (HostFeed), so that launch latency, copy and transfer overlap: 3.8 MB in 90 us instead of 135 for
+// two copies with a launch behind each.
 void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
-    const size_t npix = (size_t)v.h * v.w, plane = (npix + 3) & ~size_t(3);
-    const bool host = host_memory(data);
-    float* st = host ? in_area(plane * v.c) : staging(plane * v.c);
-    if (amax) launch_fill_zero(amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
-    const size_t step = piece_pixels(npix, npix * v.c * sizeof(float));
-    const bool planes = order == FYN_ORDER_CHANNELWISE;
+    const size_t npix = (size_t)v.h * v.w, plane = (npix + 31) & ~size_t(31);
+    const bool host = host_memory(data), planes = order == FYN_ORDER_CHANNELWISE;
+    const UploadRange range{amax, upload_words_};
+    if (!host) {
+        float* st = staging(plane * v.c);
+        for (int c = 0; c < (planes ? v.c : 1); c++)
+            FYN_HIP(hipMemcpyAsync(st + c * plane, data + c * npix, npix * (planes ? 1 : v.c) * sizeof(float), hipMemcpyDefault, stream));
+        if (planes) launch_chw_to_tensor(st, plane, v, range, HostFeed{}, true, stream);
+        else launch_hwc_to_tensor(st, v, range, HostFeed{}, true, stream);
+        FYN_HIP(hipGetLastError());
+        FYN_HIP(hipStreamSynchronize(stream));   // the caller's buffer is borrowed for this call only
+        return;
+    }
+    float* st = in_area(plane * v.c);
+    // pieces: a small one first, so that the launch has something to do when it starts; multiples of 32 pixels (whole lines)
     HostCopy copies;
-    std::vector<size_t> marks;
-    for (size_t p0 = 0; p0 < npix; p0 += step) {
+    std::vector<std::pair<size_t, size_t>> pieces;   // copies made, pixels complete
+    const size_t most = std::max<size_t>(32, (256u << 10) / (v.c * sizeof(float)) & ~size_t(31));
+    size_t step = std::max<size_t>(32, most / 8 & ~size_t(31));
+    for (size_t p0 = 0; p0 < npix;) {
         const size_t p1 = std::min(npix, p0 + step);
-        for (int c = 0; c < (planes ? v.c : 1); c++) {
-            float* dst = st + (planes ? c * plane + p0 : p0 * v.c);
-            const float* src = data + (planes ? c * npix + p0 : p0 * v.c);
-            const size_t bytes = (p1 - p0) * (planes ? 1 : v.c) * sizeof(float);
-            if (host) copies.add(dst, src, bytes);
-            else FYN_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, stream));
-        }
-        marks.push_back(copies.mark());
+        for (int c = 0; c < (planes ? v.c : 1); c++)
+            copies.add(st + (planes ? c * plane + p0 : p0 * v.c), data + (planes ? c * npix + p0 : p0 * v.c), (p1 - p0) * (planes ? 1 : v.c) * sizeof(float));
+        pieces.push_back({copies.mark(), p1});
+        p0 = p1;
+        step = std::min(most, step * 2);
     }
+    auto launch = [&](const HostFeed& feed) {
+        if (planes) launch_chw_to_tensor(st, plane, v, range, feed, false, stream);
+        else launch_hwc_to_tensor(st, v, range, feed, false, stream);
+        FYN_HIP(hipGetLastError());
+    };
     copies.start();
-    size_t piece = 0;
-    for (size_t p0 = 0; p0 < npix; p0 += step) {
-        const size_t p1 = std::min(npix, p0 + step);
-        copies.upto(marks[piece++]);
-        if (planes) launch_chw_to_tensor(st, plane, v, p0, p1, stream, amax);
-        else launch_hwc_to_tensor(st, v, p0, p1, stream, amax);
+    if (!feed_ahead_) {
+        copies.upto(copies.mark());
+        launch(HostFeed{});
+        return;
     }
-    FYN_HIP(hipGetLastError());
-    // the caller's buffer is borrowed for this call only
-    if (!host) FYN_HIP(hipStreamSynchronize(stream));
+    const HostFeed feed{feed_, feed_base_};
+    launch(feed);
+    feed_base_ += (unsigned)npix;
+    for (const auto& piece : pieces) {
+        copies.upto(piece.first);
+        __atomic_store_n(&feed_->ready, feed.base + (unsigned)piece.second, __ATOMIC_RELEASE);
+    }
 }
 
 void Net::set_input(int layer_no, int port, const float* data, int order) {
@@ -983,17 +1015,22 @@ void Net::time_layer(int layer_no, int iters, float* ms) {
 // ---------------------------------------------------------------------------------------------
 // Frame pipeline (the counterpart of the reference engine's asynchronous mode, base/engine.cpp:386-683, with
 // its two upload/download buffer sets, gpu/uploadlayer.h:74).  Two forms:
-//   overlapped   three streams of equal priority joined by events, for one network with large frames:
-//                up stream    page-locked slot -> device staging slot (copy engine)
+//   overlapped   for one network with large frames:
+//                up stream    page-locked slot -> device staging slot (copy engine), piece by piece behind the host's copy
 //                main stream  staging -> input tensor, all layers, output tensor -> device staging slot
 //                down stream  device staging slot -> page-locked slot (copy engine).  The copy is made as one of rows with
 //                gaps between them: some versions of the runtime carry out plain copies to the host with a kernel, and
 //                every workgroup of such a kernel keeps a CU for the 90 us of a frame from layers that need it whole.
+//                The streams are not joined by events: while a queue of the GPU waits for another one's signal, every
+//                launch on the main stream starts about a microsecond later (18 launches beside a copy each way: 173 us
+//                without events, 219 with them).  A thread of the pipeline's own joins them: it lets the launch that
+//                converts the frame go on when the upload has ended (HostFeed; in a running pipeline that is long before
+//                the launch's turn), sends the result on its way when the last launch has told so, and delivers it.
 //   in place     everything on the network's stream, the layout kernels reading and writing the page-locked slots over
 //                the link: networks that run side by side overlap each other's transfers, and where the transfers of a
-//                frame take less than the two hand-overs between streams (about 20 us = 1 MB) nothing is gained by them.
+//                frame are short (1 MB) nothing is gained by streams of their own.
 // There is one slot more than frames that may be in flight between two calls: submit() queues its frame first and
-// delivers the one that has to leave afterwards, so that the GPU has the next frame in its queue while the host copies.
+// sees to the delivery of the one that has to leave afterwards, so that the GPU has the next frame in its queue.
 // ---------------------------------------------------------------------------------------------
 static constexpr size_t kRowGap = 256;   // bytes between the rows of an overlapped download
 
@@ -1037,33 +1074,132 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
         async_row_ = (out_bytes / rows + 255 + 1) & ~size_t(255);
         async_rows_ = (out_bytes + async_row_ - 1) / async_row_;
     }
-    slots_.resize(depth + 1);
+    slots_ = std::vector<AsyncSlot>(depth + 1);
     for (AsyncSlot& s : slots_) {
         s.pin_in = static_cast<float*>(HostPool::acquire(in_bytes, false));
         s.pin_out = static_cast<float*>(HostPool::acquire(async_own_streams_ ? async_rows_ * (async_row_ + kRowGap) : out_bytes, false));
         if (!async_own_streams_) continue;
         FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), in_bytes));
         FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_out), async_rows_ * async_row_));
-        FYN_HIP(hipEventCreateWithFlags(&s.up, hipEventDisableTiming));
-        FYN_HIP(hipEventCreateWithFlags(&s.comp, hipEventDisableTiming));
-        FYN_HIP(hipEventCreateWithFlags(&s.down, hipEventDisableTiming));
+    }
+    if (async_own_streams_) {
+        carry_end_ = false;
+        carry_error_ = nullptr;
+        uploads_ = 0;
+        async_pixels_ = (size_t)vi.h * vi.w;
+        async_feed_ = static_cast<FeedWord*>(HostPool::acquire(sizeof(FeedWord), false));
+        *async_feed_ = FeedWord{};
+        carrier_ = std::thread([this] { carry(); });
     }
 }
 
 constexpr size_t kPipelineShared = 1u << 20;   // copies of a pipeline from this size on are shared with the helper threads
 
+// The caller's memory takes what a slot's download left in page-locked memory.
+static void add_rows(HostCopy& copies, float* to, const float* from, size_t bytes, size_t row, size_t gap) {
+    for (size_t o = 0, r = 0; o < bytes; o += row, r++)
+        copies.add(reinterpret_cast<char*>(to) + o, reinterpret_cast<const char*>(from) + r * (row + gap), std::min(row, bytes - o));
+}
+
 void Net::async_complete(AsyncSlot& s) {
+    if (async_own_streams_) {
+        for (int i = 0; i < 4096 && s.busy.load(std::memory_order_acquire); i++) _mm_pause();
+        std::unique_lock<std::mutex> lk(carry_mu_);
+        carry_done_.wait(lk, [&] { return !s.busy.load(std::memory_order_acquire) || carry_error_; });
+        if (carry_error_) std::rethrow_exception(carry_error_);
+        if (__atomic_load_n(&async_feed_->late, __ATOMIC_RELAXED)) fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
+        return;
+    }
     if (!s.busy) return;
-    if (async_own_streams_) FYN_HIP(hipEventSynchronize(s.down));
-    else signal_.wait(s.value, stream);
+    signal_.wait(s.value, stream);
     if (s.user_out) {
         HostCopy out;
-        const size_t bytes = async_out_floats_ * sizeof(float), row = async_own_streams_ ? async_row_ : bytes;
-        for (size_t o = 0, r = 0; o < bytes; o += row, r++)
-            out.add(reinterpret_cast<char*>(s.user_out) + o, reinterpret_cast<char*>(s.pin_out) + r * (row + kRowGap), std::min(row, bytes - o));
+        const size_t bytes = async_out_floats_ * sizeof(float);
+        add_rows(out, s.user_out, s.pin_out, bytes, bytes, 0);
         out.start(kPipelineShared);
     }
     s.busy = false;
+}
+
+// Whether the copies on a stream of the pipeline's are through (asked: an event would occupy a queue of the GPU).
+static bool copies_made(hipStream_t st) {
+    const hipError_t e = hipStreamQuery(st);
+    if (e != hipErrorNotReady) FYN_HIP(e);
+    return e == hipSuccess;
+}
+
+// The pipeline's thread.  Results leave in the order of submission; while one is being copied to the caller, the next is
+// sent on its way and uploads are reported.
+void Net::carry() {
+    try {
+        FYN_HIP(hipSetDevice(device));
+        unsigned uploaded = 0;       // uploads reported
+        AsyncSlot* sent = nullptr;   // its download is under way
+        auto front = [&]() -> AsyncSlot* {
+            std::lock_guard<std::mutex> lk(carry_mu_);
+            return carried_.empty() ? nullptr : carried_.front();
+        };
+        auto turn = [&](bool idle) {
+            const unsigned n = uploads_.load(std::memory_order_acquire);
+            if (n != uploaded && copies_made(up_stream_)) {   // (all of the n frames' copies: they had been queued)
+                __atomic_store_n(&async_feed_->ready, n * (unsigned)async_pixels_, __ATOMIC_RELEASE);
+                uploaded = n;
+            }
+            if (!idle) return;
+            AsyncSlot* s = front();
+            if (s && signal_.reached(s->value)) {
+                FYN_HIP(hipMemcpy2DAsync(s->pin_out, async_row_ + kRowGap, s->dev_out, async_row_, async_row_, async_rows_, hipMemcpyDeviceToHost, down_stream_));
+                sent = s;
+            }
+        };
+        auto since = std::chrono::steady_clock::now();
+        for (;;) {
+            {
+                std::unique_lock<std::mutex> lk(carry_mu_);
+                if (carried_.empty() && uploaded == uploads_.load(std::memory_order_acquire)) {
+                    carry_more_.wait(lk, [&] { return carry_end_ || !carried_.empty() || uploaded != uploads_.load(std::memory_order_acquire); });
+                    if (carry_end_ && carried_.empty()) return;
+                    since = std::chrono::steady_clock::now();
+                }
+            }
+            turn(!sent);
+            if (!sent || !copies_made(down_stream_)) {
+                for (int i = 0; i < 48; i++) _mm_pause();
+                if (sent) continue;
+                const auto waited = std::chrono::steady_clock::now() - since;
+                if (waited > std::chrono::milliseconds(5)) std::this_thread::sleep_for(std::chrono::microseconds(20));   // (long frames)
+                if (waited > std::chrono::seconds(1)) {   // something may have failed
+                    AsyncSlot* s = front();
+                    if (s && copies_made(stream) && !signal_.reached(s->value)) fail(FYN_ERR_DEVICE, "a launch ended without telling so");
+                    since = std::chrono::steady_clock::now();
+                }
+                continue;
+            }
+            AsyncSlot* s = sent;
+            sent = nullptr;
+            {
+                std::lock_guard<std::mutex> lk(carry_mu_);
+                carried_.pop_front();
+            }
+            {
+                HostCopy out;
+                add_rows(out, s->user_out, s->pin_out, async_out_floats_ * sizeof(float), async_row_, kRowGap);
+                out.start(kPipelineShared);
+                for (size_t m = 1; m <= out.mark(); m++) {
+                    turn(!sent);
+                    out.upto(m);
+                }
+            }
+            since = std::chrono::steady_clock::now();
+            std::lock_guard<std::mutex> lk(carry_mu_);
+            s->busy.store(false, std::memory_order_release);
+            carry_done_.notify_all();
+        }
+    } catch (...) {
+        std::lock_guard<std::mutex> lk(carry_mu_);
+        carry_error_ = std::current_exception();
+        carry_done_.notify_all();
+    }
 }
 
 void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
@@ -1082,34 +1218,49 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
             for (int c = 0; c < vi.c; c++) copies.add(s.pin_in + c * async_in_plane_, in + c * npix, npix * sizeof(float));
         else copies.add(s.pin_in, in, async_in_floats_ * sizeof(float));
         copies.start(kPipelineShared);
+        if (async_own_streams_) {
+            // (the copy engine follows in pieces of two megabytes and more)
+            const size_t all = (planes ? async_in_plane_ * vi.c : async_in_floats_) * sizeof(float);
+            const size_t pieces = std::max<size_t>(1, std::min<size_t>(8, all >> 21)), marks = copies.mark();
+            size_t sent = 0;
+            for (size_t m = 1; m <= pieces; m++) {
+                copies.upto(marks * m / pieces);
+                const size_t to = m == pieces ? all : copies.end_of(marks * m / pieces) - reinterpret_cast<char*>(s.pin_in);
+                FYN_HIP(hipMemcpyAsync(reinterpret_cast<char*>(s.dev_in) + sent, reinterpret_cast<char*>(s.pin_in) + sent, to - sent, hipMemcpyHostToDevice, up_stream_));
+                sent = to;
+            }
+        }
     }
     const float* src = s.pin_in;
     if (async_own_streams_) {
-        FYN_HIP(hipMemcpyAsync(s.dev_in, s.pin_in, async_in_plane_ * vi.c * sizeof(float), hipMemcpyHostToDevice, up_stream_));
-        FYN_HIP(hipEventRecord(s.up, up_stream_));
-        FYN_HIP(hipStreamWaitEvent(stream, s.up, 0));
         src = s.dev_in;
+        const HostFeed feed{async_feed_, uploads_.load() * (unsigned)npix};
+        {
+            std::lock_guard<std::mutex> lk(carry_mu_);
+            uploads_++;
+            carry_more_.notify_one();
+        }
+        if (feed_ahead_) launch_await_feed(feed, npix, stream);
+        else FYN_HIP(hipStreamSynchronize(up_stream_));
     }
-    if (async_in_->amax) launch_fill_zero(async_in_->amax, RANGE_WORDS * sizeof(unsigned), stream);   // the tensor's value-range record starts over
-    if (planes) launch_chw_to_tensor(src, async_in_plane_, vi, 0, npix, stream, async_in_->amax);
-    else launch_hwc_to_tensor(src, vi, 0, npix, stream, async_in_->amax);
+    const UploadRange range{async_in_->amax, upload_words_};
+    if (planes) launch_chw_to_tensor(src, async_in_plane_, vi, range, HostFeed{}, async_own_streams_, stream);
+    else launch_hwc_to_tensor(src, vi, range, HostFeed{}, async_own_streams_, stream);
     forward(nullptr);
     float* dst = async_own_streams_ ? s.dev_out : s.pin_out;
-    const HostDone done = async_own_streams_ ? HostDone{} : signal_.next();
+    const HostDone done = signal_.next();
     if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, dst, opix, 0, 0, opix, done, stream);
     else launch_tensor_to_hwc(vo, dst, vo.c == 3 ? 4 : vo.c, 0, opix, done, stream);
-    s.value = done.value;
-    if (async_own_streams_) {
-        FYN_HIP(hipGetLastError());
-        FYN_HIP(hipEventRecord(s.comp, stream));
-        FYN_HIP(hipStreamWaitEvent(down_stream_, s.comp, 0));
-        FYN_HIP(hipMemcpy2DAsync(s.pin_out, async_row_ + kRowGap, s.dev_out, async_row_, async_row_, async_rows_, hipMemcpyDeviceToHost, down_stream_));
-        FYN_HIP(hipEventRecord(s.down, down_stream_));
-    }
     FYN_HIP(hipGetLastError());
+    s.value = done.value;
     s.user_out = out;
     s.busy = true;
     s.ticket = ++async_seq_;
+    if (async_own_streams_) {
+        std::lock_guard<std::mutex> lk(carry_mu_);
+        carried_.push_back(&s);
+        carry_more_.notify_one();
+    }
     if (ticket) *ticket = s.ticket;
     if (async_seq_ > (uint64_t)async_depth_) async_complete(slots_[(async_seq_ - async_depth_ - 1) % slots_.size()]);
 }
@@ -1128,29 +1279,44 @@ void Net::async_wait(uint64_t ticket) {
 void Net::async_end() {
     if (slots_.empty()) return;
     (void)hipSetDevice(device);
-    for (uint64_t t = (async_seq_ > slots_.size() ? async_seq_ - slots_.size() + 1 : 1); t <= async_seq_; t++) {
-        AsyncSlot& s = slots_[(t - 1) % slots_.size()];
-        if (s.busy && s.ticket == t) async_complete(s);
+    std::exception_ptr error;
+    try {
+        for (uint64_t t = (async_seq_ > slots_.size() ? async_seq_ - slots_.size() + 1 : 1); t <= async_seq_; t++) {
+            AsyncSlot& s = slots_[(t - 1) % slots_.size()];
+            if (s.busy && s.ticket == t) async_complete(s);
+        }
+    } catch (...) {
+        error = std::current_exception();
+    }
+    if (carrier_.joinable()) {
+        {
+            std::lock_guard<std::mutex> lk(carry_mu_);
+            carry_end_ = true;
+            carry_more_.notify_one();
+        }
+        carrier_.join();
+        carried_.clear();
+        carry_error_ = nullptr;
     }
     if (stream) (void)hipStreamSynchronize(stream);
+    if (up_stream_) (void)hipStreamSynchronize(up_stream_);
+    if (down_stream_) (void)hipStreamSynchronize(down_stream_);
     for (AsyncSlot& s : slots_) {
         HostPool::release(s.pin_in);
         HostPool::release(s.pin_out);
         if (s.dev_in) (void)hipFree(s.dev_in);
         if (s.dev_out) (void)hipFree(s.dev_out);
-        if (s.up) (void)hipEventDestroy(s.up);
-        if (s.comp) (void)hipEventDestroy(s.comp);
-        if (s.down) (void)hipEventDestroy(s.down);
     }
+    const bool late = async_feed_ && async_feed_->late;
+    HostPool::release(async_feed_);
+    async_feed_ = nullptr;
     slots_.clear();
-    if (async_own_streams_) {
-        if (up_stream_) (void)hipStreamSynchronize(up_stream_);
-        if (down_stream_) (void)hipStreamSynchronize(down_stream_);
-        return_stream(device, up_stream_);
-        return_stream(device, down_stream_);
-    }
+    return_stream(device, up_stream_);
+    return_stream(device, down_stream_);
     up_stream_ = down_stream_ = nullptr;
     async_seq_ = 0;
+    if (error) std::rethrow_exception(error);
+    if (late) fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
 }
 
 }  // namespace fynhip

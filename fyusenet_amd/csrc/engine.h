@@ -7,12 +7,18 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
+#include <deque>
+#include <exception>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/fynhip.h"
@@ -157,11 +163,10 @@ class Net {
   private:
     struct AsyncSlot {
         float *pin_in = nullptr, *pin_out = nullptr, *dev_in = nullptr, *dev_out = nullptr;
-        hipEvent_t up = nullptr, comp = nullptr, down = nullptr;
-        unsigned value = 0;   // in place: what the stream's word reads when pin_out is filled
+        unsigned value = 0;   // what the stream's word reads when the frame's launches are through (in place: pin_out is filled then)
         float* user_out = nullptr;
         uint64_t ticket = 0;
-        bool busy = false;
+        std::atomic<bool> busy{false};
     };
     std::vector<AsyncSlot> slots_;
     hipStream_t up_stream_ = nullptr, down_stream_ = nullptr;
@@ -175,6 +180,17 @@ class Net {
     size_t async_in_floats_ = 0, async_out_floats_ = 0, async_in_plane_ = 0;   // (planes lie on multiples of four floats)
     uint64_t async_seq_ = 0;
     void async_complete(AsyncSlot& s);
+    // overlapped pipelines: the thread that delivers results, and the frames handed to it
+    std::thread carrier_;
+    std::mutex carry_mu_;
+    std::condition_variable carry_more_, carry_done_;
+    std::deque<AsyncSlot*> carried_;
+    std::exception_ptr carry_error_;
+    std::atomic<unsigned> uploads_{0};     // frames whose upload has been queued
+    FeedWord* async_feed_ = nullptr;       // pixels of them that have arrived in device memory
+    size_t async_pixels_ = 0;              // of a frame
+    bool carry_end_ = false;
+    void carry();
     void run_layers(bool with_events);
     void release_all();
     void collect_timings();
@@ -191,6 +207,10 @@ class Net {
     char* in_pin_ = nullptr;
     size_t in_bytes_ = 0, in_off_ = 0, in_most_ = 0, out_most_ = 0;
     HostSignal signal_;
+    FeedWord* feed_ = nullptr;          // progress of the host's copies into the input area
+    unsigned feed_base_ = 0;            // ... when all frames so far have been copied
+    bool feed_ahead_ = true;            // uploads are launched ahead of the copy
+    unsigned* upload_words_ = nullptr;  // UploadRange::words of the network's stream
     float* in_area(size_t floats);
     HostLoan out_area(size_t floats);
     void count_area(size_t bytes, size_t& most);   // staging areas count as allocations when they are larger than any before

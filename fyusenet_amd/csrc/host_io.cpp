@@ -109,9 +109,13 @@ void HostSignal::destroy() {
 }
 HostDone HostSignal::next() { return HostDone{counter_, flag_, ++value_}; }
 
-void HostSignal::wait(unsigned value, hipStream_t s) {
+bool HostSignal::reached(unsigned value) const {
     // (values pass in rising order; the difference survives the wrap-around)
-    auto done = [&] { return (int)(__atomic_load_n(flag_, __ATOMIC_ACQUIRE) - value) >= 0; };
+    return (int)(__atomic_load_n(flag_, __ATOMIC_ACQUIRE) - value) >= 0;
+}
+
+void HostSignal::wait(unsigned value, hipStream_t s) const {
+    auto done = [&] { return reached(value); };
     const auto t0 = std::chrono::steady_clock::now();
     for (int i = 1; !done(); i++) {
         _mm_pause();
@@ -193,6 +197,7 @@ void HostCopy::add(void* dst, const void* src, size_t bytes) {
     job_->bytes += bytes;
 }
 size_t HostCopy::mark() const { return job_->slices.size(); }
+char* HostCopy::end_of(size_t mark) const { return job_->slices[mark - 1].dst + job_->slices[mark - 1].bytes; }
 void HostCopy::start(size_t alone) {
     job_->made.reset(new std::atomic<char>[job_->slices.size()]());
     if (job_->bytes >= alone) HostCopyHelpers::get().offer(job_);

@@ -50,6 +50,7 @@ class HostCopy {
     ~HostCopy();   // (all copies have been made then)
     void add(void* dst, const void* src, size_t bytes);
     size_t mark() const;       // for upto(): the copies added so far
+    char* end_of(size_t mark) const;   // where the last of these copies ends in its target
     void start(size_t alone = 8u << 20);   // all copies have been added; fewer bytes than `alone` are not shared
     void upto(size_t mark);    // returns when these copies have been made, having done its share
 
@@ -68,7 +69,8 @@ class HostSignal {
     HostDone next();                           // for the next launch on the stream
     // Returns when the launch that was given `value`, and so everything in front of it on the stream, has been carried
     // out.  Polls for a while, then leaves the waiting to the runtime, which also reports a failed launch.
-    void wait(unsigned value, hipStream_t s);
+    void wait(unsigned value, hipStream_t s) const;
+    bool reached(unsigned value) const;   // whether that is so already (any thread)
     unsigned last() const { return value_; }
 
   private:

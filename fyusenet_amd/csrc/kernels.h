@@ -462,13 +462,31 @@ struct HostDone {
     unsigned* flag;
     unsigned value;
 };
-// Layout conversion between tensors and fp32 buffers in page-locked host memory or device memory (layout.hip); pixels
-// [p0, p1) of the area.  (amax: value-range word of the tensor, raised by what is written, or null; range.h)
-void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax);   // net area only; plane, p0: multiples of 4
+// How far the host has come with the frame that a launch converts.  `ready`: pixels copied, counted on from one frame to
+// the next (a launch starts at `base`, modulo 2^32); the launch reads a pixel when ready - base exceeds it.  `late`: set by
+// a launch that gave up waiting.
+struct FeedWord {
+    unsigned ready, late;
+};
+struct HostFeed {
+    FeedWord* word;   // page-locked; null: the frame is there
+    unsigned base;
+};
+// The value-range record (range.h) of an uploaded tensor, which the launch writes, and two zero words of device memory in
+// which its workgroups meet (they belong to one stream).  record null: none is kept.
+struct UploadRange {
+    unsigned* record;
+    unsigned* words;
+};
+// Layout conversion between tensors and fp32 buffers in page-locked host memory or (device: more workgroups pay) device
+// memory (layout.hip); downloads: pixels [p0, p1) of the area.
+// (planes: multiples of four floats; with a feed word of 32, the buffer on a 128-byte boundary: no line is read before all of it is there)
+void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, bool device, hipStream_t s);   // net area only
+void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, bool device, hipStream_t s);   // GPU_SHALLOW in
 void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s);
-void launch_hwc_to_tensor(const float* hwc, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax);   // GPU_SHALLOW in; p0: a multiple of 4
 void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s);   // GPU_SHALLOW out, pc = 1, 2 or 4
 void launch_argmax_to_host(const int* idx, const TView& t, int* idx_out, float* val_out, size_t p0, size_t p1, const HostDone& done, hipStream_t s);
+void launch_await_feed(const HostFeed& feed, size_t npix, hipStream_t s);   // holds the stream until the frame is there (one workgroup looks, not those of a whole conversion)
 void launch_tell_host(const HostDone& done, hipStream_t s);
 void launch_fill_zero(void* ptr, size_t bytes, hipStream_t s);
 int launch_poison_lds(hipStream_t s);   // debugging aid: all-ones words into every CU's LDS

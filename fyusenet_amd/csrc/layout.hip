@@ -17,7 +17,60 @@
 namespace fynhip {
 
 namespace {
-constexpr unsigned kMaxBlocks = 128;
+constexpr unsigned kMaxBlocks = 128;          // buffers behind the link
+constexpr unsigned kMaxDeviceBlocks = 1024;   // buffers in device memory: 3.8 MB of pixels in 4 us instead of 11
+unsigned blocks_for(size_t items, bool device) { return (unsigned)std::min<size_t>(device ? kMaxDeviceBlocks : kMaxBlocks, (items + 255) / 256); }
+
+// The host may still be copying the frame when the launch runs (HostFeed): before a workgroup reads pixels it looks, where
+// it has to, whether they are there.  The launch's own latency (8 us) and the host's copy then overlap the transfer
+// instead of preceding it.  Every thread of the workgroup calls this with the workgroup's largest pixel; `seen` holds what
+// the last look said.  The wait ends after kFeedTicks in any case, and the host is told (FeedWord::late).
+constexpr unsigned long long kFeedTicks = 400000000ull;   // 4 s of the 100 MHz clock
+__device__ __forceinline__ void await_feed(const HostFeed& f, unsigned need, unsigned& seen) {
+    if (!f.word || seen >= need) return;   // (the same for all threads)
+    __shared__ unsigned box;
+    if (threadIdx.x == 0) {
+        const unsigned long long t0 = wall_clock64();
+        unsigned r;
+        while ((int)((r = __hip_atomic_load(&f.word->ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) - f.base) - need) < 0) {
+            __builtin_amdgcn_s_sleep(48);   // (1.3 us: more looks would take the link from the copy that is waited for)
+            if (wall_clock64() - t0 > kFeedTicks) {
+                __hip_atomic_store(&f.word->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                r = 0x7fffffffu;
+                break;
+            }
+        }
+        box = r;
+    }
+    __syncthreads();
+    seen = box;
+    __syncthreads();
+}
+
+// The value range of an uploaded tensor.  Its record is written, not raised, so that no launch has to clear it first: the
+// workgroups meet in a word of the network's (device scope: they sit on different XCDs), and the one that arrives last
+// moves the maximum into the record and leaves the words as they were found.
+__device__ __forceinline__ void publish_range(const UploadRange& u, float m) {
+    if (!u.record) return;
+    __shared__ float wave_max[4];
+    __shared__ unsigned last;
+    m = range_wave_max(m);
+    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        (void)__hip_atomic_fetch_max(&u.words[0], __float_as_uint(fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]))), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the maximum has been taken before the arrival counts)
+        unsigned all = 0u;
+        if (__hip_atomic_fetch_add(&u.words[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+            all = __hip_atomic_exchange(&u.words[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | 0x80000000u;   // (the sign bit marks the last workgroup)
+            __hip_atomic_store(&u.words[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        last = all;
+    }
+    __syncthreads();
+    if (last && threadIdx.x < RANGE_SLOTS) u.record[threadIdx.x * RANGE_STRIDE] = threadIdx.x == 0 ? last & 0x7fffffffu : 0u;
+}
 
 // Stores of the workgroup's threads, then -- by the workgroup that arrives last -- the host's word: when the host reads
 // `value` there, everything the launch has written lies in memory.  A host that polls the word sees the result 5 us
@@ -60,15 +113,20 @@ __device__ __forceinline__ void store4(T* p, float a, float b, float c, float d)
 }
 }  // namespace
 
-// Pixels [p0, p1) of planes `plane` floats apart (both multiples of four, as is the planes' address in units of four
-// floats): a thread takes four pixels of four channels.  Channels beyond the tensor's read as zero.
+// Planes `plane` floats apart (a multiple of four, as is the planes' address in units of four floats): a thread takes four
+// pixels of four channels.  Channels beyond the tensor's read as zero.
 template <typename T>
-__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, unsigned p0, unsigned p1, unsigned* amax) {
-    const unsigned quads = (p1 - p0 + 3) >> 2;
+__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, const UploadRange range, const HostFeed feed) {
+    const unsigned npix = (unsigned)t.h * t.w, quads = (npix + 3) >> 2;
     const size_t n = (size_t)quads * (t.cp >> 2);
     float vmax = 0.f;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        const unsigned pix = p0 + (unsigned)(i % quads) * 4;
+    unsigned seen = 0;
+    for (size_t i0 = (size_t)blockIdx.x * 256; i0 < n; i0 += (size_t)gridDim.x * 256) {
+        const unsigned q0 = (unsigned)(i0 % quads);
+        await_feed(feed, q0 + 256 >= quads ? npix : (q0 + 256) * 4, seen);
+        const size_t i = i0 + threadIdx.x;
+        if (i >= n) break;
+        const unsigned pix = (unsigned)(i % quads) * 4;
         const int c = (int)(i / quads) * 4;
         float4 v[4];
 #pragma unroll
@@ -76,7 +134,7 @@ __global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, si
         unsigned y = pix / (unsigned)t.w, x = pix - y * (unsigned)t.w;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            if (pix + j < p1) {
+            if (pix + j < npix) {
                 float e[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
@@ -91,23 +149,26 @@ __global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, si
             }
         }
     }
-    if (amax) range_publish_block256(amax, vmax);   // (every thread takes part)
+    publish_range(range, vmax);
 }
-void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax) {
-    const size_t items = (p1 - p0 + 3) / 4 * (t.cp >> 2);
-    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
-    if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, (unsigned)p0, (unsigned)p1, amax);
-    else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, (unsigned)p0, (unsigned)p1, amax);
+void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, bool device, hipStream_t s) {
+    const dim3 grid(blocks_for(((size_t)t.h * t.w + 3) / 4 * (t.cp >> 2), device));
+    if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, range, feed);
+    else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, range, feed);
 }
 
 // Interleaved pixels of t.c floats: the buffer is read as one run of sixteen-byte pieces (an element's pixel and channel
-// follow from its index), the tensor's pad channels keep the zeros they were allocated with.  p0 * t.c is a multiple of
-// four; the last piece may reach up to three floats behind the buffer's end.
+// follow from its index), the tensor's pad channels keep the zeros they were allocated with.  The last piece may reach
+// up to three floats behind the buffer's end.
 template <typename T>
-__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, const TView t, size_t p0, size_t p1, unsigned* amax) {
-    const size_t e1 = p1 * t.c, q1 = (e1 + 3) >> 2;
+__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, const TView t, const UploadRange range, const HostFeed feed) {
+    const size_t npix = (size_t)t.h * t.w, e1 = npix * t.c, q1 = (e1 + 3) >> 2;
     float vmax = 0.f;
-    for (size_t q = p0 * t.c / 4 + (size_t)blockIdx.x * 256 + threadIdx.x; q < q1; q += (size_t)gridDim.x * 256) {
+    unsigned seen = 0;
+    for (size_t q0 = (size_t)blockIdx.x * 256; q0 < q1; q0 += (size_t)gridDim.x * 256) {
+        await_feed(feed, q0 + 256 >= q1 ? (unsigned)npix : (unsigned)((q0 + 256) * 4 / t.c + 1), seen);
+        const size_t q = q0 + threadIdx.x;
+        if (q >= q1) break;
         const float4 v = *reinterpret_cast<const float4*>(hwc + q * 4);
         const float e[4] = {v.x, v.y, v.z, v.w};
         unsigned pix = (unsigned)(q * 4 / t.c), c = (unsigned)(q * 4 - (size_t)pix * t.c);
@@ -127,13 +188,12 @@ __global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, co
             }
         }
     }
-    if (amax) range_publish_block256(amax, vmax);
+    publish_range(range, vmax);
 }
-void launch_hwc_to_tensor(const float* hwc, const TView& t, size_t p0, size_t p1, hipStream_t s, unsigned* amax) {
-    const size_t items = ((p1 - p0) * t.c + 3) / 4;
-    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
-    if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, p0, p1, amax);
-    else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, p0, p1, amax);
+void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, bool device, hipStream_t s) {
+    const dim3 grid(blocks_for(((size_t)t.h * t.w * t.c + 3) / 4, device));
+    if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, range, feed);
+    else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, range, feed);
 }
 
 // Pixels [p0, p1) of the net area (keep_pad: of the area with its halo) to planes `plane` floats apart.  Q = 4: a thread
@@ -172,7 +232,43 @@ __global__ __launch_bounds__(256) void tensor_to_chw_kernel(const TView t, float
     }
     tell_host(done);
 }
+// All planes of a small or odd area, one behind the other without gaps: the buffer is written as one run of sixteen-byte
+// pieces, whatever planes they fall into (46 KB in planes of 36 floats, one float per store: 14 us; this way 4).
+template <typename T>
+__global__ __launch_bounds__(256) void tensor_to_run_kernel(const TView t, float* chw, unsigned npix, int keep_pad, const HostDone done) {
+    const unsigned ow = (unsigned)(keep_pad ? t.wp() : t.w);
+    const int off = keep_pad ? 0 : t.pad;
+    const size_t n = (size_t)npix * t.c;
+    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
+        unsigned c = (unsigned)(i / npix), pix = (unsigned)(i - (size_t)c * npix);
+        unsigned y = pix / ow, x = pix - y * ow;
+        float e[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (i + k < n) e[k] = (float)reinterpret_cast<const T*>(t.ptr)[((size_t)(y + off) * t.wp() + x + off) * t.cp + c];
+            if (++x == ow) {
+                x = 0;
+                y++;
+            }
+            if (++pix == npix) {
+                pix = x = y = 0;
+                c++;
+            }
+        }
+        if (i + 4 <= n) *reinterpret_cast<float4*>(chw + i) = make_float4(e[0], e[1], e[2], e[3]);
+        else
+            for (int k = 0; i + k < n; k++) chw[i + k] = e[k];
+    }
+    tell_host(done);
+}
 void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
+    const size_t npix = include_padding ? (size_t)t.hp() * t.wp() : (size_t)t.h * t.w;
+    if (plane == npix && p0 == 0 && p1 == npix && (plane % 4 != 0 || plane < 256) && (reinterpret_cast<size_t>(chw) & 15) == 0 && t.c > 1) {
+        const dim3 grid(blocks_for((npix * t.c + 3) / 4, false));
+        if (t.f16) hipLaunchKernelGGL(tensor_to_run_kernel<_Float16>, grid, dim3(256), 0, s, t, chw, (unsigned)npix, include_padding, done);
+        else hipLaunchKernelGGL(tensor_to_run_kernel<float>, grid, dim3(256), 0, s, t, chw, (unsigned)npix, include_padding, done);
+        return;
+    }
     const bool quad = plane % 4 == 0 && (reinterpret_cast<size_t>(chw) & 15) == 0 && p0 % 4 == 0;
     const size_t items = (p1 - p0 + (quad ? 3 : 0)) / (quad ? 4 : 1) * ((t.c + 3) >> 2);
     const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
@@ -225,6 +321,12 @@ void launch_argmax_to_host(const int* idx, const TView& t, int* idx_out, float* 
     if (t.f16) hipLaunchKernelGGL(argmax_to_host_kernel<_Float16>, grid, dim3(256), 0, s, idx, t, idx_out, val_out, p0, p1, done);
     else hipLaunchKernelGGL(argmax_to_host_kernel<float>, grid, dim3(256), 0, s, idx, t, idx_out, val_out, p0, p1, done);
 }
+
+__global__ void await_feed_kernel(const HostFeed feed, unsigned npix) {
+    unsigned seen = 0;
+    await_feed(feed, npix, seen);
+}
+void launch_await_feed(const HostFeed& feed, size_t npix, hipStream_t s) { hipLaunchKernelGGL(await_feed_kernel, dim3(1), dim3(64), 0, s, feed, (unsigned)npix); }
 
 __global__ void tell_host_kernel(const HostDone done) { tell_host(done); }
 void launch_tell_host(const HostDone& done, hipStream_t s) { hipLaunchKernelGGL(tell_host_kernel, dim3(1), dim3(64), 0, s, done); }
