@@ -235,8 +235,7 @@ Net::Net(int dev, int stor) : device(dev), storage(stor) {
         static_scratch_ = static_scratch(dev);
         signal_.create(static_cast<unsigned*>(dev_alloc(64)));
         upload_words_ = static_cast<unsigned*>(dev_alloc(64));
-        feed_ = static_cast<FeedWord*>(HostPool::acquire(sizeof(FeedWord), false));
-        *feed_ = FeedWord{};
+        feed_ = signal_.feed();
         // (where the runtime is told to finish a launch before the call returns, the frame is copied first)
         for (const char* e : {"HIP_LAUNCH_BLOCKING", "CUDA_LAUNCH_BLOCKING", "AMD_SERIALIZE_KERNEL"})
             if (const char* v = getenv(e)) feed_ahead_ = feed_ahead_ && (!*v || *v == '0');
@@ -250,9 +249,7 @@ void Net::release_all() {
     if (stream) (void)hipStreamSynchronize(stream);
     for (void* p : allocs_) (void)hipFree(p);
     allocs_.clear();
-    signal_.destroy();
-    HostPool::release(feed_);
-    HostPool::release(in_pin_);
+    signal_.destroy();   // (the stream is idle: the areas that waited for the word are free)
     return_stream(device, stream);
     HostPool::network_gone();
 }
@@ -607,7 +604,6 @@ void Net::finish() {
     FYN_HIP(hipSetDevice(device));
     if (events_pending_) {
         FYN_HIP(hipStreamSynchronize(stream));
-        settled();
         collect_timings();
         return;
     }
@@ -620,19 +616,10 @@ void Net::finish() {
 // Everything queued on the stream ahead of the launch with this value has been carried out then.
 void Net::wait_signal(unsigned value) {
     signal_.wait(value, stream);
-    if (value == signal_.last()) settled();
     if (__atomic_load_n(&feed_->late, __ATOMIC_RELAXED)) {
         feed_->late = 0;
         fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
     }
-}
-
-// The stream is idle: nothing reads the input area any more.
-void Net::settled() {
-    in_off_ = 0;
-    HostPool::release(in_pin_);
-    in_pin_ = nullptr;
-    in_bytes_ = 0;
 }
 
 void Net::count_area(size_t bytes, size_t& most) {
@@ -640,21 +627,6 @@ void Net::count_area(size_t bytes, size_t& most) {
     most = bytes;
     alloc_calls_++;
     alloc_bytes_ += bytes;
-}
-
-// `floats` of page-locked memory that no queued launch reads, on loan until the stream has been waited for.
-float* Net::in_area(size_t floats) {
-    const size_t bytes = (floats * sizeof(float) + 255) & ~size_t(255);
-    if (in_off_ + bytes > in_bytes_) {
-        if (in_off_) FYN_HIP(hipStreamSynchronize(stream));
-        settled();
-        in_pin_ = static_cast<char*>(HostPool::acquire(bytes, false));
-        in_bytes_ = bytes;
-        count_area(bytes, in_most_);
-    }
-    float* p = reinterpret_cast<float*>(in_pin_ + in_off_);
-    in_off_ += bytes;
-    return p;
 }
 
 // Page-locked memory for a result on its way to the caller's, on loan for one call.
@@ -715,18 +687,24 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         float* st = staging(plane * v.c);
         for (int c = 0; c < (planes ? v.c : 1); c++)
             FYN_HIP(hipMemcpyAsync(st + c * plane, data + c * npix, npix * (planes ? 1 : v.c) * sizeof(float), hipMemcpyDefault, stream));
-        if (planes) launch_chw_to_tensor(st, plane, v, range, HostFeed{}, true, stream);
-        else launch_hwc_to_tensor(st, v, range, HostFeed{}, true, stream);
+        if (planes) launch_chw_to_tensor(st, plane, v, range, HostFeed{}, HostDone{}, true, stream);
+        else launch_hwc_to_tensor(st, v, range, HostFeed{}, HostDone{}, true, stream);
         FYN_HIP(hipGetLastError());
         FYN_HIP(hipStreamSynchronize(stream));   // the caller's buffer is borrowed for this call only
         return;
     }
-    float* st = in_area(plane * v.c);
+    // (page-locked memory, the pool's again when the launch has told that it is through; a caller that never waits is
+    // held at a few frames)
+    const size_t bytes = plane * v.c * sizeof(float);
+    unsigned& before = uploads_told_[upload_no_++ % kUploads];
+    if (before) signal_.wait(before, stream);
+    float* st = static_cast<float*>(HostPool::acquire(bytes, false));
+    count_area(bytes, in_most_);
     // pieces: a small one first, so that the launch has something to do when it starts; multiples of 32 pixels (whole lines)
     HostCopy copies;
     std::vector<std::pair<size_t, size_t>> pieces;   // copies made, pixels complete
-    const size_t most = std::max<size_t>(32, (256u << 10) / (v.c * sizeof(float)) & ~size_t(31));
-    size_t step = std::max<size_t>(32, most / 8 & ~size_t(31));
+    const size_t most = std::max<size_t>(4096, (256u << 10) / (v.c * sizeof(float)) & ~size_t(31));
+    size_t step = most / 8 & ~size_t(31);
     for (size_t p0 = 0; p0 < npix;) {
         const size_t p1 = std::min(npix, p0 + step);
         for (int c = 0; c < (planes ? v.c : 1); c++)
@@ -735,10 +713,13 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         p0 = p1;
         step = std::min(most, step * 2);
     }
+    const HostDone done = signal_.next();
+    before = done.value;
     auto launch = [&](const HostFeed& feed) {
-        if (planes) launch_chw_to_tensor(st, plane, v, range, feed, false, stream);
-        else launch_hwc_to_tensor(st, v, range, feed, false, stream);
+        if (planes) launch_chw_to_tensor(st, plane, v, range, feed, done, false, stream);
+        else launch_hwc_to_tensor(st, v, range, feed, done, false, stream);
         FYN_HIP(hipGetLastError());
+        signal_.release_then(st, done.value);
     };
     copies.start();
     if (!feed_ahead_) {
@@ -782,7 +763,6 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
         FYN_HIP(hipGetLastError());
         FYN_HIP(hipMemcpyAsync(out, st, bytes, hipMemcpyDefault, stream));
         FYN_HIP(hipStreamSynchronize(stream));
-        settled();
         return;
     }
     if (HostPool::contains(out, bytes)) {
@@ -1244,8 +1224,8 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
         else FYN_HIP(hipStreamSynchronize(up_stream_));
     }
     const UploadRange range{async_in_->amax, upload_words_};
-    if (planes) launch_chw_to_tensor(src, async_in_plane_, vi, range, HostFeed{}, async_own_streams_, stream);
-    else launch_hwc_to_tensor(src, vi, range, HostFeed{}, async_own_streams_, stream);
+    if (planes) launch_chw_to_tensor(src, async_in_plane_, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
+    else launch_hwc_to_tensor(src, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
     forward(nullptr);
     float* dst = async_own_streams_ ? s.dev_out : s.pin_out;
     const HostDone done = signal_.next();

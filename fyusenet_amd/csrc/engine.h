@@ -202,20 +202,17 @@ class Net {
   private:
     float* staging_ = nullptr;
     size_t staging_floats_ = 0;
-    // Page-locked staging of the synchronous calls.  Inputs are put in one behind the other and converted by launches that
-    // read them in place; the area goes back once the stream has been waited for.
-    char* in_pin_ = nullptr;
-    size_t in_bytes_ = 0, in_off_ = 0, in_most_ = 0, out_most_ = 0;
+    size_t in_most_ = 0, out_most_ = 0;   // largest page-locked areas of the synchronous calls so far
+    static constexpr unsigned kUploads = 4;   // areas of uploads that may be waiting for their launch
+    unsigned uploads_told_[kUploads] = {}, upload_no_ = 0;
     HostSignal signal_;
     FeedWord* feed_ = nullptr;          // progress of the host's copies into the input area
     unsigned feed_base_ = 0;            // ... when all frames so far have been copied
     bool feed_ahead_ = true;            // uploads are launched ahead of the copy
     unsigned* upload_words_ = nullptr;  // UploadRange::words of the network's stream
-    float* in_area(size_t floats);
     HostLoan out_area(size_t floats);
     void count_area(size_t bytes, size_t& most);   // staging areas count as allocations when they are larger than any before
     void wait_signal(unsigned value);
-    void settled();
     void upload(const float* data, int order, const TView& v, unsigned* amax);
     void download_planes(const TView& v, int include_padding, float* out);
     void download_pixels(const TView& v, int pc, float* out);

@@ -22,7 +22,19 @@ namespace {
 struct Block {
     size_t bytes;
     bool lent;
+    const unsigned* flag;   // lent until this word reads `value`, null: until it is given back
+    unsigned value;
 };
+bool told(const unsigned* flag, unsigned value) {   // (values pass in rising order; the difference survives the wrap-around)
+    return (int)(__atomic_load_n(flag, __ATOMIC_ACQUIRE) - value) >= 0;
+}
+bool idle(Block& b) {
+    if (b.flag && told(b.flag, b.value)) {
+        b.flag = nullptr;
+        b.lent = false;
+    }
+    return !b.lent;
+}
 std::mutex g_pool_mu;
 std::map<char*, Block> g_blocks;   // by address
 size_t g_pool_bytes = 0;
@@ -35,7 +47,7 @@ size_t size_class(size_t bytes) {   // sizes in steps of an eighth of the next p
 }
 void give_back_idle() {   // (the lock is held)
     for (auto it = g_blocks.begin(); it != g_blocks.end();) {
-        if (it->second.lent) {
+        if (!idle(it->second)) {
             ++it;
             continue;
         }
@@ -50,7 +62,7 @@ void* HostPool::acquire(size_t bytes, bool bounded) {
     const size_t want = size_class(bytes ? bytes : 1);
     std::lock_guard<std::mutex> lk(g_pool_mu);
     for (auto& kv : g_blocks)
-        if (!kv.second.lent && kv.second.bytes == want) {
+        if (kv.second.bytes == want && idle(kv.second)) {
             kv.second.lent = true;
             return kv.first;
         }
@@ -66,7 +78,7 @@ void* HostPool::acquire(size_t bytes, bool bounded) {
         if (bounded) return nullptr;
         fail(FYN_ERR_DEVICE, "no page-locked memory (%zu bytes): %s", want, hipGetErrorString(e));
     }
-    g_blocks[static_cast<char*>(p)] = Block{want, true};
+    g_blocks[static_cast<char*>(p)] = Block{want, true, nullptr, 0};
     g_pool_bytes += want;
     return p;
 }
@@ -78,6 +90,23 @@ void HostPool::release(void* p) {
     if (it == g_blocks.end() || !it->second.lent) return;
     it->second.lent = false;
     if (g_networks == 0 || g_pool_bytes > kBytes) give_back_idle();
+}
+
+void HostPool::release_then(void* p, const unsigned* flag, unsigned value) {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    auto it = g_blocks.find(static_cast<char*>(p));
+    if (it == g_blocks.end()) return;
+    it->second.flag = flag;
+    it->second.value = value;
+}
+
+void HostPool::forget(const unsigned* flag) {
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    for (auto& kv : g_blocks)
+        if (kv.second.flag == flag) {
+            kv.second.flag = nullptr;
+            kv.second.lent = false;
+        }
 }
 
 bool HostPool::contains(const void* p, size_t bytes) {
@@ -100,18 +129,19 @@ void HostPool::network_gone() {
 
 void HostSignal::create(unsigned* counter) {
     counter_ = counter;
-    flag_ = static_cast<unsigned*>(HostPool::acquire(64, false));
+    flag_ = static_cast<unsigned*>(HostPool::acquire(kFeed + sizeof(FeedWord), false));
     *flag_ = value_ = 0;
+    *feed() = FeedWord{};
 }
 void HostSignal::destroy() {
+    if (flag_) HostPool::forget(flag_);
     HostPool::release(flag_);
     flag_ = nullptr;
 }
 HostDone HostSignal::next() { return HostDone{counter_, flag_, ++value_}; }
 
 bool HostSignal::reached(unsigned value) const {
-    // (values pass in rising order; the difference survives the wrap-around)
-    return (int)(__atomic_load_n(flag_, __ATOMIC_ACQUIRE) - value) >= 0;
+    return told(flag_, value);
 }
 
 void HostSignal::wait(unsigned value, hipStream_t s) const {

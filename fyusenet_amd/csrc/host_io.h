@@ -19,6 +19,8 @@ class HostPool {
     static constexpr size_t kBytes = size_t(512) << 20;
     static void* acquire(size_t bytes, bool bounded);   // bounded: null when the pool is full or there is no GPU; else throws when memory cannot be had
     static void release(void* p);                       // null is nothing
+    static void release_then(void* p, const unsigned* flag, unsigned value);   // when the word `flag` reads `value` (HostSignal)
+    static void forget(const unsigned* flag);           // the word goes away: blocks that wait for it are free
     static bool contains(const void* p, size_t bytes);  // whether the range lies inside a block on loan
     static void network_created();
     static void network_gone();
@@ -72,8 +74,11 @@ class HostSignal {
     void wait(unsigned value, hipStream_t s) const;
     bool reached(unsigned value) const;   // whether that is so already (any thread)
     unsigned last() const { return value_; }
+    FeedWord* feed() const { return reinterpret_cast<FeedWord*>(reinterpret_cast<char*>(flag_) + kFeed); }   // another word beside it, zero at first
+    void release_then(void* block, unsigned value) const { HostPool::release_then(block, flag_, value); }
 
   private:
+    static constexpr size_t kFeed = 128;   // (words that the GPU and the host write lie in lines of their own)
     unsigned* flag_ = nullptr;
     unsigned* counter_ = nullptr;
     unsigned value_ = 0;

@@ -116,7 +116,7 @@ __device__ __forceinline__ void store4(T* p, float a, float b, float c, float d)
 // Planes `plane` floats apart (a multiple of four, as is the planes' address in units of four floats): a thread takes four
 // pixels of four channels.  Channels beyond the tensor's read as zero.
 template <typename T>
-__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, const UploadRange range, const HostFeed feed) {
+__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, const UploadRange range, const HostFeed feed, const HostDone done) {
     const unsigned npix = (unsigned)t.h * t.w, quads = (npix + 3) >> 2;
     const size_t n = (size_t)quads * (t.cp >> 2);
     float vmax = 0.f;
@@ -150,18 +150,19 @@ __global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, si
         }
     }
     publish_range(range, vmax);
+    tell_host(done);
 }
-void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, bool device, hipStream_t s) {
+void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s) {
     const dim3 grid(blocks_for(((size_t)t.h * t.w + 3) / 4 * (t.cp >> 2), device));
-    if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, range, feed);
-    else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, range, feed);
+    if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, range, feed, done);
+    else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, range, feed, done);
 }
 
 // Interleaved pixels of t.c floats: the buffer is read as one run of sixteen-byte pieces (an element's pixel and channel
 // follow from its index), the tensor's pad channels keep the zeros they were allocated with.  The last piece may reach
 // up to three floats behind the buffer's end.
 template <typename T>
-__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, const TView t, const UploadRange range, const HostFeed feed) {
+__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, const TView t, const UploadRange range, const HostFeed feed, const HostDone done) {
     const size_t npix = (size_t)t.h * t.w, e1 = npix * t.c, q1 = (e1 + 3) >> 2;
     float vmax = 0.f;
     unsigned seen = 0;
@@ -189,11 +190,12 @@ __global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, co
         }
     }
     publish_range(range, vmax);
+    tell_host(done);
 }
-void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, bool device, hipStream_t s) {
+void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s) {
     const dim3 grid(blocks_for(((size_t)t.h * t.w * t.c + 3) / 4, device));
-    if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, range, feed);
-    else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, range, feed);
+    if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, range, feed, done);
+    else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, range, feed, done);
 }
 
 // Pixels [p0, p1) of the net area (keep_pad: of the area with its halo) to planes `plane` floats apart.  Q = 4: a thread
