@@ -698,7 +698,7 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
     const size_t bytes = plane * v.c * sizeof(float);
     unsigned& before = uploads_told_[upload_no_++ % kUploads];
     if (before) signal_.wait(before, stream);
-    float* st = static_cast<float*>(HostPool::acquire(bytes, false));
+    float* st = static_cast<float*>(HostPool::acquire(bytes, false, true));
     count_area(bytes, in_most_);
     // pieces: a small one first, so that the launch has something to do when it starts; multiples of 32 pixels (whole lines)
     HostCopy copies;
@@ -1056,7 +1056,7 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
     }
     slots_ = std::vector<AsyncSlot>(depth + 1);
     for (AsyncSlot& s : slots_) {
-        s.pin_in = static_cast<float*>(HostPool::acquire(in_bytes, false));
+        s.pin_in = static_cast<float*>(HostPool::acquire(in_bytes, false, true));
         s.pin_out = static_cast<float*>(HostPool::acquire(async_own_streams_ ? async_rows_ * (async_row_ + kRowGap) : out_bytes, false));
         if (!async_own_streams_) continue;
         FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), in_bytes));

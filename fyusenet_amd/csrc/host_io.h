@@ -17,7 +17,7 @@ namespace fynhip {
 class HostPool {
   public:
     static constexpr size_t kBytes = size_t(512) << 20;
-    static void* acquire(size_t bytes, bool bounded);   // bounded: null when the pool is full or there is no GPU; else throws when memory cannot be had
+    static void* acquire(size_t bytes, bool bounded, bool filled_by_host = false);   // bounded: null when the pool is full or there is no GPU; else throws when memory cannot be had
     static void release(void* p);                       // null is nothing
     static void release_then(void* p, const unsigned* flag, unsigned value);   // when the word `flag` reads `value` (HostSignal)
     static void forget(const unsigned* flag);           // the word goes away: blocks that wait for it are free
