@@ -411,6 +411,15 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
                         v[o] = o < p.cout ? ((a[o] * acc_mul) * sc4[o] + bi4[o]) + r : 0.f;
                         vmax = fmaxf(vmax, fabsf(v[o]));
                     }
+                    if (p.post_fn != FFN_COPY) {   // (what the layer behind would have read, and its own arithmetic)
+#pragma unroll
+                        for (int o = 0; o < 4; o++) {
+                            float x = sizeof(TOut) == 4 ? v[o] : (float)(_Float16)v[o];
+                            if (p.post_act.kind != ACT_NONE) x = fminf(p.post_act.hi, fmaxf(p.post_act.lo, x)) + p.post_act.leak * fminf(x, 0.f);
+                            x = p.post_fn == FFN_SIGMOID ? sigmoid1(x) : tanh1(x);
+                            v[o] = o < p.cout ? x : 0.f;
+                        }
+                    }
                     const size_t oidx = ((size_t)(p.out_off_y + y) * p.out_wp + p.out_off_x + gx) * p.out_cp;
                     if (sizeof(TOut) == 4) {
                         *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + oidx) = v;

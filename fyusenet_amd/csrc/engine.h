@@ -95,6 +95,9 @@ class Layer {
     virtual bool tracks_range() const { return false; }
     virtual bool add_range_reset(unsigned*) { return false; }
     virtual void setup_ranges() {}   // (re)reads the words of the layer's tensors into its kernel arguments
+    // a sigmoid or tanh layer: its arguments, for the layer in front that computes it as well (computed_by), else null
+    virtual const FuncParams* pointwise() const { return nullptr; }
+    virtual void computed_by(int) {}
     Act act() const;
     const Tensor& tin(int port) const;
     const Tensor& tout() const;
@@ -233,6 +236,7 @@ void fuse_batchnorm_layers(Net* net);   // after every layer's setup(): batch-no
 void keep_projection_inputs(Net* net);    // before buffers are assigned: inputs of such projections live until the layer that may compute them has run
 void fuse_projection_layers(Net* net);   // after every layer's setup(): 1x1 shortcut projections that the 1x1 layer adding them can compute in its own launch
 void fuse_depthwise_layers(Net* net);   // after every layer's setup(): depthwise 3x3 layers that their 1x1 reader can compute itself
+void fuse_function_layers(Net* net);   // after every layer's setup(): sigmoid / tanh layers that the row-rolling convolution in front of them can apply to what it stores
 Layer* create_custom_layer(Net* net, const fyn_layer_desc& d, const fyn_custom_layer& impl);
 
 }  // namespace fynhip

@@ -357,5 +357,34 @@ void fuse_batchnorm_layers(Net* net) {
     }
 }
 
+// A sigmoid or tanh layer whose input comes from a convolution in the row-rolling form and goes nowhere else (the end of
+// the style-net samples): the convolution applies it to what it stores, into the layer's own tensor.  The launch writes
+// that tensor in the convolution's place in the order, earlier than its buffer was handed over for: every other tenant
+// of the buffer must be through by then.
+void fuse_function_layers(Net* net) {
+    if (net->sw.get("FYNHIP_NO_FUNCTION_FUSION") || !net->reuse_buffers) return;
+    std::map<int, int> readers;
+    for (auto& kv : net->layers)
+        for (int t : kv.second->in)
+            if (t >= 0) readers[t]++;
+    for (auto& kv : net->layers) {
+        Layer* f = kv.second.get();
+        const FuncParams* p = f->pointwise();
+        if (!p) continue;
+        const Tensor& t = net->tensors[f->in[0]];
+        const Tensor& o = net->tensors[f->out];
+        if (t.producer < 0 || t.locked || readers[f->in[0]] != 1) continue;
+        ConvLayer* c = dynamic_cast<ConvLayer*>(net->layer(t.producer));
+        if (!c || !c->rows || o.v.f16 != t.v.f16 || o.v.cp != 4 || t.v.cp != 4 || o.v.h != t.v.h || o.v.w != t.v.w) continue;
+        bool early_ok = true;
+        for (const Tensor& other : net->tensors)
+            if (&other != &o && other.buffer == o.buffer && other.producer < f->d.number && std::max(other.last_reader, other.producer) >= c->d.number) early_ok = false;
+        if (!early_ok) continue;
+        c->fn_layer_no = f->d.number;
+        c->fn_params = *p;
+        f->computed_by(c->d.number);
+    }
+}
+
 
 }  // namespace fynhip

@@ -17,6 +17,11 @@ struct Act {
     float leak, lo, hi;
 };
 
+// functions of function-type layers
+enum FuncFn { FFN_COPY = 0, FFN_SIGMOID = 1, FFN_TANH = 2, FFN_ARITH = 3, FFN_CAST = 4, FFN_BGR = 5 };
+__device__ __forceinline__ float sigmoid1(float x) { return __frcp_rn(1.0f + __expf(-x)); }
+__device__ __forceinline__ float tanh1(float x) { return 1.0f - 2.0f * __frcp_rn(1.0f + __expf(2.0f * x)); }   // = 2 e^{2x}/(1+e^{2x}) - 1 without the inf/inf of large x
+
 // Output stores that are written through the XCD's L2 as they are issued (sc1: visible at device scope) instead of
 // staying dirty there until the write-back at the kernel's end.  A kernel's stores then overlap the work of the
 // workgroups that are still computing, and the next launch does not wait behind the write-back of a whole output
@@ -202,6 +207,10 @@ struct ConvRowsParams {
     unsigned* reset[4];
     int nreset;
     Act act;
+    // A sigmoid or tanh layer behind the convolution applied to the values as they are stored (FFN_COPY: none); `out` is
+    // that layer's tensor then, post_act the activation it applies on fetch.
+    int post_fn;
+    Act post_act;
 };
 int ensure_lds(const void* fn, size_t lds_bytes);   // 0, or -2 when the device refuses the size (conv_mfma.hip)
 bool conv_rows_supported(int k, int cin_pitch, int cout, bool f16);
@@ -311,6 +320,12 @@ int launch_conv_d16(const ConvP16Params& p, hipStream_t s);   // (p.dw_in set: w
 bool conv_d16_dw_supported(int chunks, int dw_stride);
 // (p.tile_h = 3, 5 or 7: a K x K convolution on an input of at most four channels instead, cin_chunks = steps of eight taps)
 bool conv_d16_small_supported(int k, int dil, int in_cp, int cout, int out_cp);
+// 3x3 convolutions between tensors of few channels, any stride, edge rule and source step (conv_g16.hip)
+bool conv_g16_supported(int k, int dil, int in_cp, int cout, int out_cp);
+int conv_g16_steps(int in_cp);                       // matrix steps of the window
+bool conv_g16_exists(const ConvP16Params& p);        // whether p.wm fragments per wave have been compiled
+size_t conv_g16_lds_bytes(const ConvP16Params& p);   // of a workgroup: its weights
+int launch_conv_g16(const ConvP16Params& p, hipStream_t s);
 // a 1x1 layer and the depthwise 3x3 layer behind it as one launch (conv_d16.hip: conv_e16dw_kernel)
 bool conv_e16dw_supported(int in_cp, int chunks, int dw_stride);
 int launch_conv_e16dw(const ConvP16Params& p, hipStream_t s);
@@ -385,7 +400,6 @@ void launch_addsub(const TView& a, const TView& b, const TView& out, int sub, co
 // texel picked by `map` and passed through `fn`; the stencil modes (linear scaling, non-maximum suppression,
 // blur) have kernels of their own.  Source coordinates beyond the stored input repeat its edge.
 enum FuncMap { FMAP_SCALE = 0, FMAP_TRANSPOSE = 1, FMAP_IMGEXTRACT = 2 };
-enum FuncFn { FFN_COPY = 0, FFN_SIGMOID = 1, FFN_TANH = 2, FFN_ARITH = 3, FFN_CAST = 4, FFN_BGR = 5 };
 struct FuncParams {
     TView in, out;
     Act act;

@@ -628,6 +628,119 @@ class ConvLayer : public Layer {
             net->dev_free(wp);
         }
     }
+    // The LDS-staged weights, gathered windows form for few channels (conv_g16.hip) against what has been chosen so far.
+    void setup_g16(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
+        ConvP16Params q{};
+        q.in = in_v.ptr; q.out = out_v.ptr; q.res = res_v ? res_v->ptr : nullptr;
+        q.in_hp = in_v.hp(); q.in_wp = in_v.wp(); q.in_cp = in_v.cp;
+        q.stride = stride;
+        q.in_y0 = q.in_x0 = in_v.pad - 1;
+        if (frac_shift) {   // (the frame of repeated pixels, as in setup_p16)
+            q.in_shift = frac_shift - 1;
+            q.in_y0 = (in_v.pad << q.in_shift) - 1;
+            q.in_x0 = (in_v.pad << q.in_shift) - 2;
+        }
+        q.in_clamp = clamp ? 1 : 0;
+        q.npos_y = oh; q.npos_x = ow;
+        q.out_wp = out_v.wp(); q.out_cp = out_v.cp; q.out_off_y = q.out_off_x = out_v.pad;
+        if (res_v) { q.res_wp = res_v->wp(); q.res_cp = res_v->cp; q.res_off_y = q.res_off_x = res_v->pad; }
+        q.res_relu = res_relu; q.res_scale = res_scale;
+        q.cin_chunks = conv_g16_steps(in_v.cp);
+        q.f16 = out_v.f16 ? 1 : 0;
+        q.scale = scale_dev; q.bias = bias_dev;
+        q.acc_mul = 1.f;
+        q.act = act();
+        q.in_amax = tin(0).amax;
+        const int frags = (oc + 15) / 16, tiles = (oh * ow + 15) / 16;
+        if ((long long)in_v.elems() * (q.f16 ? 2 : 4) > (1ll << 31)) return;
+        int want = 0;   // FYNHIP_G16_FRAGS=fragments per wave (tests)
+        if (const char* e = net->sw.get("FYNHIP_G16_FRAGS")) want = atoi(e);
+        // all fragments in every wave (a window is fetched and converted once), or, where the positions alone do not fill
+        // the chip, a wave per fragment
+        std::vector<ConvP16Params> cands;
+        for (int fr = frags; fr >= 1; fr--) {
+            if (frags % fr != 0 || (want ? fr != want : (fr == 1 && frags > 1 && tiles > 4096))) continue;
+            ConvP16Params c = q;
+            c.wm = fr;
+            c.cout_blocks = frags / fr;
+            c.mfrags = frags;
+            if (!conv_g16_exists(c)) continue;
+            const size_t lds = conv_g16_lds_bytes(c);
+            if (lds > 150 * 1024) continue;
+            // as many workgroups per CU as registers and weights allow (512 against 768 workgroups on 16 -> 20 channels at
+            // 312x256: fp16 8.1 and 7.6 us, 1248: 8.7), each wave the same number of tiles
+            const int most = std::max(8, (lds <= 48 * 1024 ? 768 : lds <= 80 * 1024 ? 512 : 256) / c.cout_blocks), per = (tiles + 4 * most - 1) / (4 * most);
+            c.pos_groups = (tiles + 4 * per - 1) / (4 * per);
+            if (c.pos_groups > 8) c.pos_groups = (c.pos_groups + 7) / 8 * 8;
+            cands.push_back(c);
+        }
+        if (cands.empty()) return;
+        const size_t halves = (size_t)frags * q.cin_chunks * (q.f16 ? 1 : 2) * 64 * 8;
+        void* const wp = net->dev_alloc(halves * 2, true);
+        for (ConvP16Params& c : cands) c.wpack = wp;
+        const bool always = net->sw.get("FYNHIP_FORCE_G16_CONV") != nullptr;
+        const char* at = net->sw.get("FYNHIP_AUTOTUNE");
+        int pick = 0;
+        char key[160];
+        snprintf(key, sizeof(key), "g16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
+        int cached[3] = {0, 0, 0};
+        if (want || always) {
+        } else if (tune_cache_triple(net, key, cached)) {
+            pick = -1;
+            for (size_t i = 0; cached[0] && i < cands.size(); i++)
+                if (cands[i].wm == cached[1]) pick = (int)i;
+        } else if (!(at && at[0] == '0')) {
+            float best = 1e30f, t_other = 1e30f;
+            for (int rep = 0; rep < 3; rep++) {
+                for (size_t i = 0; i < cands.size(); i++) {
+                    const float t = time_calls(net, [&]() {
+                        if (launch_conv_g16(cands[i], net->stream) != 0) fail(FYN_ERR_DEVICE, "gathering convolution launch failed while tuning");
+                    }, 10);
+                    if (t < best) { best = t; pick = (int)i; }
+                }
+                t_other = std::min(t_other, time_calls(net, [&]() { run(net->stream); }, 10));
+            }
+            if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
+                fprintf(stderr, "[tune] 3x3 on %d channels, %dx%d positions, to %d: gathered windows (%d fragment(s) per wave, %d workgroups) %.1f us, %s %.1f us\n", in_v.cp, oh, ow, oc,
+                        cands[pick].wm, cands[pick].pos_groups * cands[pick].cout_blocks, best * 1e3f, own_info().c_str(), t_other * 1e3f);
+            tune_cache_store_triple(net, key, best < t_other ? 1 : 0, cands[pick].wm, 0);
+            if (best >= t_other) pick = -1;
+        } else {
+            pick = -1;
+        }
+        if (pick >= 0) {
+            if (p16) net->dev_free(p16_wpack_dev);
+            p16_wpack_dev = wp;
+            p16 = g16 = true;
+            kr16 = false;
+            pp = cands[pick];
+        } else {
+            net->dev_free(wp);
+        }
+    }
+    // weights of that form: [cout fragment][step][plane][lane][8 halves]; lane group kq of step s is group g = 4s + kq of
+    // eight channels, tap g / G and channels 8 * (g % G) of it (G groups per pixel)
+    void pack_g16(const float* w, float wmul) {
+        const int cin = d.in_channels, npl = pp.f16 ? 1 : 2, groups = pp.in_cp / 8, steps = pp.cin_chunks, frags = (oc + 15) / 16;
+        std::vector<uint16_t> pack((size_t)frags * steps * npl * 64 * 8, 0);
+        for (int mf = 0; mf < frags; mf++)
+            for (int s = 0; s < steps; s++) {
+                uint16_t* base = pack.data() + (size_t)(mf * steps + s) * npl * 64 * 8;
+                for (int lane = 0; lane < 64; lane++) {
+                    const int o = mf * 16 + (lane & 15), g = 4 * s + (lane >> 4), tap = g / groups;
+                    if (o >= oc || tap >= 9) continue;
+                    for (int j = 0; j < 8; j++) {
+                        const int ci = (g % groups) * 8 + j;
+                        if (ci >= cin) continue;
+                        const float v = w[((size_t)o * 9 + tap) * cin + ci] * wmul;
+                        const uint16_t hi = f2h_bits(v);
+                        base[(size_t)lane * 8 + j] = hi;
+                        if (npl == 2) base[(size_t)(64 + lane) * 8 + j] = f2h_bits(v - h2f(hi));
+                    }
+                }
+            }
+        reupload(net, static_cast<uint16_t*>(p16_wpack_dev), pack);
+    }
     // weights of that form: [cout fragment][chunk][plane][lane][8 halves]
     void pack_d16(const float* w, float wmul) {
         if (pp.tile_h) pack_taps16(w, wmul);
@@ -1013,6 +1126,10 @@ class ConvLayer : public Layer {
                 (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 8 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_D16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") &&
                 !net->sw.get("FYNHIP_FORCE_KSPLIT") && !net->sw.get("FYNHIP_CONV_TILE") && !net->sw.get("FYNHIP_CONV_KC") && !net->sw.get("FYNHIP_CONV_KC_MAX") && !net->sw.get("FYNHIP_CONV_PD"))
                 setup_d16(in_v, out_v, res_v, res_relu, res_scale);
+            // few channels on both sides, 3x3: windows gathered from the tensor
+            if (!h16 && !c4 && !d16 && same_storage && conv_g16_supported(k, dil, in_v.cp, oc, out_v.cp) && d.in_channels <= in_v.cp &&
+                (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_G16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") && !only_kr)
+                setup_g16(in_v, out_v, res_v, res_relu, res_scale);
         }
         if (direct) {
             scale_dev = static_cast<float*>(net->dev_alloc(padded * sizeof(float)));
@@ -1043,7 +1160,8 @@ class ConvLayer : public Layer {
         } else if (p16) {
             const float wmul = weight_prescale(w, (size_t)oc * k * k * d.in_channels);
             pp.acc_mul = pp2.acc_mul = 1.0f / wmul;
-            if (c4) pack_c4(w, wmul);
+            if (g16) pack_g16(w, wmul);
+            else if (c4) pack_c4(w, wmul);
             else if (d16) pack_d16(w, wmul);
             else if (kr16) pack_kr16(w, wmul);
             else if (h16) pack_h16(w, wmul);
@@ -1120,6 +1238,15 @@ class ConvLayer : public Layer {
         run(s);
     }
     void run(hipStream_t s) {
+        if (rows && fn_layer_no >= 0 && net->fusion_on()) {
+            ConvRowsParams q = rp;
+            q.out = fn_params.out.ptr;
+            q.out_wp = fn_params.out.wp(); q.out_cp = fn_params.out.cp; q.out_off_y = q.out_off_x = fn_params.out.pad;
+            q.out_amax = nullptr;   // (the function layer keeps no value-range word)
+            q.post_fn = fn_params.fn; q.post_act = fn_params.act;
+            if (launch_conv_rows(q, fn_params.out.f16 != 0, s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
+            return;
+        }
         if (rows) {
             if (launch_conv_rows(rp, tout().v.f16 != 0, s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
@@ -1133,7 +1260,7 @@ class ConvLayer : public Layer {
             return;
         }
         if (p16) {
-            if ((c4 ? launch_conv_p16c4(pp, k, s) : (d16 ? launch_conv_d16(pp, s) : (kr16 ? launch_conv_kr16(pp, k, s) : (h16 ? launch_conv_h16(pp, k, s) : launch_conv_p16(pp, s))))) != 0 ||
+            if ((g16 ? launch_conv_g16(pp, s) : c4 ? launch_conv_p16c4(pp, k, s) : (d16 ? launch_conv_d16(pp, s) : (kr16 ? launch_conv_kr16(pp, k, s) : (h16 ? launch_conv_h16(pp, k, s) : launch_conv_p16(pp, s))))) != 0 ||
                 (h16 && h16_two && launch_conv_h16(pp2, k, s) != 0))
                 fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
@@ -1144,6 +1271,7 @@ class ConvLayer : public Layer {
         if (wide && !fused) launch_shift_reduce(sr, s);
     }
     std::string info() const override {
+        if (fn_layer_no >= 0) return own_info() + "; the function layer " + std::to_string(fn_layer_no) + " behind it is applied to what is stored";
         if (pj_into >= 0 && static_cast<ConvLayer*>(net->layer(pj_into))->pj_spread_ok)
             return "conv 1x1 projection (runs inside the launch of layer " + std::to_string(pj_into) + "; no launch of its own); apart: " + own_info();
         if (pj_fused && pj_spread_ok) {
@@ -1173,6 +1301,12 @@ class ConvLayer : public Layer {
                      pp.f16 ? "f16" : (conv_p16c4_uses_fp8(pp, k) ? "f16+fp8-split" : "f16x2-split"), pp.tile_h * pp.tile_w * 4, pp.tile_h, pp.tile_w, pp.pos_groups * pp.cout_blocks, pp.tiles_x * pp.tiles_y * pp.cout_blocks,
                      conv_p16c4_lds_bytes(pp, k), c4_steps);
             return mode + buf + (conv_p16_stores_through(pp, 1) ? " stores=through" : "");
+        }
+        if (p16 && g16) {
+            char buf[220];
+            snprintf(buf, sizeof(buf), "conv_g16 %s windows gathered from the tensor: %d steps of four 8-channel groups, %d fragment(s) of 16 output channels per wave, blocks=%d lds=%zu",
+                     pp.f16 ? "f16" : "f16x2-split", pp.cin_chunks, pp.wm, pp.pos_groups * pp.cout_blocks, conv_g16_lds_bytes(pp));
+            return mode + buf;
         }
         if (p16 && d16) {
             char buf[360];
@@ -1223,11 +1357,14 @@ class ConvLayer : public Layer {
     MfmaLaunch launch;
     ConvRowsParams rp{};          // row-rolling form of the folded convolution (conv_rows.hip)
     void* rows_wpack_dev = nullptr;
+    int fn_layer_no = -1;         // the sigmoid or tanh layer behind that this form applies to what it stores (fuse_function_layers)
+    FuncParams fn_params{};
     bool p16 = false;             // 16-position-fragment form of a 3x3 convolution (conv_p16.hip)
     bool c4 = false;              // ... its variant for inputs of at most four channels
     int c4_steps = 0;
     bool h16 = false;             // ... its fp16-storage form for wide layers (conv_h16.hip)
     bool kr16 = false;            // ... the K-resident form for layers with few positions (conv_p16.hip, conv_kr16_kernel)
+    bool g16 = false;             // ... the form that gathers 3x3 windows of few channels (conv_g16.hip)
     bool d16 = false;             // ... the LDS-free 1x1 form for many positions and few input channels (conv_d16.hip)
     // A depthwise 3x3 layer whose only reader is this 1x1 layer in the K-resident form can be computed inside this
     // layer's staging (fuse_depthwise_layers below): the fields of ConvP16Params that describe it

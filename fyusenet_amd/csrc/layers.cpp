@@ -549,6 +549,7 @@ class FuncLayer : public Layer {
         }
     }
     void forward(hipStream_t s) override {
+        if (fused_into >= 0 && net->fusion_on()) return;   // computed by the convolution in front
         if (d.type == FYN_LAYER_NONMAX2D) launch_nonmax(p.in, p.out, s);
         else if (d.type == FYN_LAYER_BLUR2D) {
             // shaders/generickernel.frag:83-107: 3x3 visits (-1..1)^2; larger kernels stop one short of the last
@@ -558,7 +559,10 @@ class FuncLayer : public Layer {
         } else if (linear) launch_scale_linear(p, s);
         else launch_func(p, s);
     }
-    std::string info() const override { return kind; }
+    std::string info() const override { return fused_into >= 0 ? std::string(kind) + " (runs inside the launch of layer " + std::to_string(fused_into) + "; no launch of its own)" : kind; }
+    const FuncParams* pointwise() const override { return (p.fn == FFN_SIGMOID || p.fn == FFN_TANH) && p.map == FMAP_SCALE ? &p : nullptr; }
+    void computed_by(int layer) override { fused_into = layer; }
+    int fused_into = -1;
     FuncParams p{};
     bool linear = false;
     const char* kind = "function";

@@ -681,8 +681,8 @@ __device__ __forceinline__ float4 mask_channels(float4 v, int c, int nc) {
 
 __device__ __forceinline__ float func1(float x, int fn, int op, float operand) {
     switch (fn) {
-        case FFN_SIGMOID: return __frcp_rn(1.0f + __expf(-x));
-        case FFN_TANH: return 1.0f - 2.0f * __frcp_rn(1.0f + __expf(2.0f * x));   // = 2 e^{2x}/(1+e^{2x}) - 1 without the inf/inf of large x
+        case FFN_SIGMOID: return sigmoid1(x);
+        case FFN_TANH: return tanh1(x);
         case FFN_ARITH: return op == 0 ? x + operand : op == 1 ? x - operand : op == 2 ? x * operand : x / operand;
         case FFN_CAST: {
             if (op == 7) return x;
