@@ -1243,15 +1243,23 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
     static_assert(R >= 1 && (R == 1 || DWS == 0), "rounds: without a depthwise layer in the staging");
     constexpr int RPD = G::RPD, BD = G::BD, STEPS = G::STEPS;
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ unsigned range_box[2];
     if ((blockIdx.x | blockIdx.y | blockIdx.z) == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // (a grid of output-channel blocks x tile columns x tile rows: no division stands between the kernel's start and its
-    // first request; consecutive workgroups are the channel blocks of one tile)
-    const int cb = blockIdx.x, txi = blockIdx.y, tyi = blockIdx.z;
-    if (tid < 2) range_box[tid] = 0u;
+    // Which workgroup computes what.  A grid of output-channel blocks x tile columns x tile rows: no division stands between
+    // the kernel's start and its first request, and as consecutive workgroups go to consecutive XCDs, a block's weights
+    // come into few L2s and every tile's pixels into all.  Where pixels are the larger part (p.tile_major), the grid is
+    // XCDs x blocks x tiles of an XCD's band instead: a band's pixels come into one L2 -- where the layer in front, banded
+    // the same way, has just left most of them -- and the weights into all.
+    int cb = blockIdx.x, txi = blockIdx.y, tyi = blockIdx.z;
+    if (p.tile_major) {
+        const unsigned n = (unsigned)(p.tiles_x * p.tiles_y), t = ((n * blockIdx.x) >> 3) + blockIdx.z;
+        if (t >= (n * (blockIdx.x + 1)) >> 3) return;
+        cb = blockIdx.y;
+        tyi = (int)(((float)t + 0.5f) * p.rcp_tiles_x);
+        txi = (int)t - tyi * p.tiles_x;
+    }
     // (two source tensors: the larger of their value ranges scales both, or nothing is scaled when one keeps no word)
     const bool ranged = p.in_amax && (SRC != 2 || p.in2_amax);
     // (both loads are issued here and met where the scale is computed: nothing waits for them in between)
@@ -1539,7 +1547,7 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
                 }
             }
             lds_barrier();   // the tile is staged
-            lds_barrier();   // the MFMA waves have left their accumulators for wave 0
+            lds_barrier();   // the MFMA waves have left their accumulators for each other
             return;
         }
         if (stid < 16 * FM) {
@@ -1551,7 +1559,7 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
             stage_tile(SW == 8 ? tid : stid, r, r > 0);
             lds_barrier();   // the round is staged
         }
-        lds_barrier();   // the MFMA waves have left their accumulators for wave 0
+        lds_barrier();   // the MFMA waves have left their accumulators for each other
         return;
     }
 
@@ -1588,18 +1596,19 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
     float inv_in_scale = 1.f;
     if (ranged) (void)range_scale(range_after_act(range_reduce(range_word()), p.act), &inv_in_scale);
     const float acc_mul = p.acc_mul * inv_in_scale;
-    // The residual values of the epilogue (wave 0) are requested here, so that their memory round trip passes under the
+    // The residual values of the epilogue are requested here, so that their memory round trip passes under the
     // staging and the step stream instead of behind them (small tiles: the registers are there).
     constexpr bool RES_EARLY = FM * FN <= 4;
     typedef typename std::conditional<HSTORE, half4_t, f32x4_t>::type res_t;
     res_t res_early[RES_EARLY ? FM : 1][RES_EARLY ? FN : 1];
     if constexpr (RES_EARLY) {
-        if (w == 0 && p.res) {
+        if (w < FM * FN && p.res) {
             const store_t* res = reinterpret_cast<const store_t*>(p.res);
 #pragma unroll
             for (int fn = 0; fn < FN; fn++)
 #pragma unroll
                 for (int fm = 0; fm < FM; fm++) {
+                    if (((fm * FN + fn) & 3) != w) continue;
                     const int m = fn * 16 + mq;
                     const int py = tyi * G::TH + m / G::TW, px = txi * G::TW + m % G::TW;
                     const int ch = cb * 16 * FM + fm * 16 + kq * 4;
@@ -1656,16 +1665,16 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
             lds_barrier();   // every MFMA wave is through with the round: the staging waves may write the next
         }
     }
-    // the four partial sums meet in wave 0
-    if (w > 0) {
+    // the four partial sums of a fragment meet in one of the waves, the fragments dealt to them in turn
+    auto owner = [](int fm, int fn) { return (fm * FN + fn) & 3; };
 #pragma unroll
-        for (int fm = 0; fm < FM; fm++)
+    for (int fm = 0; fm < FM; fm++)
 #pragma unroll
-            for (int fn = 0; fn < FN; fn++)
-                *reinterpret_cast<f32x4_t*>(lds + red_off + (((w - 1) * FM + fm) * FN + fn) * 1024 + lane * 16) = acc[fm][fn];
-    }
+        for (int fn = 0; fn < FN; fn++)
+            if (owner(fm, fn) != w)
+                *reinterpret_cast<f32x4_t*>(lds + red_off + (((w < owner(fm, fn) ? w : w - 1) * FM + fm) * FN + fn) * 1024 + lane * 16) = acc[fm][fn];
     lds_barrier();
-    if (w > 0) return;
+    if (w >= FM * FN) return;
     float vmax = 0.f;
     {
         const float* sb = reinterpret_cast<const float*>(lds + sb_off);
@@ -1675,6 +1684,7 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
         for (int fn = 0; fn < FN; fn++)
 #pragma unroll
         for (int fm = 0; fm < FM; fm++) {
+            if (owner(fm, fn) != w) continue;
             const int m = fn * 16 + mq;
             const int py = tyi * G::TH + m / G::TW, px = txi * G::TW + m % G::TW;
             const bool okp = py < p.npos_y && px < p.npos_x;
@@ -1721,7 +1731,10 @@ __global__ __launch_bounds__(512) void conv_kr16_kernel(const ConvP16Params p) {
             }
         }
     }
-    if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 1);
+    if (p.out_amax) {
+        vmax = range_wave_max(vmax);
+        if (lane == 0) range_raise(p.out_amax, vmax);
+    }
 }
 
 typedef void (*p16_fn)(const ConvP16Params);
@@ -1928,7 +1941,15 @@ int P16_NAME(launch_conv_kr16)(const ConvP16Params& p, int k, hipStream_t s) {
         return -5;
     if (e->lds > 160 * 1024) return -2;
     if (ensure_lds(reinterpret_cast<const void*>(e->fn), e->lds) != 0) return -2;
-    hipLaunchKernelGGL(e->fn, dim3(p.cout_blocks, p.tiles_x, p.tiles_y), dim3(512), e->lds, s, p);
+    // (a tile's place in its XCD's band counts in the grid's last dimension; fewer tiles than XCDs, or a block's weights
+    // larger than the pixels of all tiles: blocks first.  The waits for a tile's pixels in ResNet-50's 56x56 and 28x28
+    // layers go from 3250 to 2600 and from 2780 to 2200 clocks, its frame in fp32 from 319 to 314 us)
+    const long long n = (long long)p.tiles_x * p.tiles_y, pixels = (long long)p.npos_y * p.stride * p.npos_x * p.stride * p.in_cp;
+    ConvP16Params q = p;
+    q.tile_major = n >= 8 && n < (1 << 22) && pixels > (long long)k * k * p.cin_chunks * KC * 16 * p.mfrags && p.cout_blocks <= 65535;
+    q.rcp_tiles_x = 1.0f / (float)p.tiles_x;
+    const dim3 grid = q.tile_major ? dim3(8, p.cout_blocks, (unsigned)((n + 7) / 8)) : dim3(p.cout_blocks, p.tiles_x, p.tiles_y);
+    hipLaunchKernelGGL(e->fn, grid, dim3(512), e->lds, s, q);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

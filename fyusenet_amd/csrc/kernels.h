@@ -240,6 +240,7 @@ struct ConvP16Params {
     int tile_h, tile_w, wm;    // tiles_x counts workgroup tiles of (4/wm)*tile_w columns
     int tiles_x, tiles_y;
     float rcp_tiles_x;    // 1.0f / tiles_x
+    int tile_major;       // launch_conv_kr16 sets it: workgroups are dealt to the XCDs by bands of tiles
     int pos_groups;       // workgroups per block of output channels; workgroup g walks tiles g, g + pos_groups, ...
     int cin_chunks;
     int exact_split;      // launch_conv_p16 on fp32 tensors: three fp16 passes even where the fp8 form of the correction terms would run
