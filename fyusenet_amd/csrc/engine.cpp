@@ -468,6 +468,7 @@ void Net::setup() {
     fuse_projection_layers(this);
     fuse_batchnorm_layers(this);
     fuse_function_layers(this);
+    fuse_concat_layers(this);
     assign_range_resets();
     poison_lds_ = sw.get("FYNHIP_POISON_LDS") != nullptr;
     FYN_HIP(hipStreamSynchronize(stream));

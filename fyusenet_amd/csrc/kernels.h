@@ -395,6 +395,28 @@ struct BnParams {
     Act act;
 };
 void launch_batchnorm(const BnParams& p, hipStream_t s);
+// A concatenation in one launch, with what may stand around it: bilinear scale layers in front of inputs, a plain
+// batch-norm layer behind (scale null: none).  Every input's channels are whole vectors (launch_cat_supported) and `out`
+// has no channels behind them.
+struct CatPart {
+    TView in;        // the input, or the scale layer's input
+    int c_off;       // first channel of the output
+    int linear;      // bilinear scaling as in FuncParams, with the activation `act` behind it
+    int ux, uy, dx, dy, ox, oy;
+    Act act;
+};
+struct CatParams {
+    static constexpr int kMost = 4;
+    CatPart part[kMost];
+    int n;
+    TView out;
+    Act act;         // the concatenation's own
+    const float* scale;
+    const float* bias;
+    Act bn_act;
+};
+bool launch_cat_supported(const CatParams& p);
+void launch_cat(const CatParams& p, hipStream_t s);
 void launch_addsub(const TView& a, const TView& b, const TView& out, int sub, const Act& act, hipStream_t s);
 
 // Function-type layers with one input and no weights.  Every output texel (4 channels) is produced from ONE source

@@ -1596,15 +1596,17 @@ class BatchNormLayer : public Layer {
     void forward(hipStream_t s) override {
         if (!have_weights) fail(FYN_ERR_STATE, "layer %s (%d): forward() without scale/bias", d.name, d.number);
         if (fused_into >= 0 && net->fusion_on()) return;   // applied by the convolution layers that read it
-        launch_batchnorm(p, s);
+        if (cat.n && net->fusion_on()) launch_cat(cat, s);
+        else launch_batchnorm(p, s);
     }
     std::string info() const override {
-        return fused_into >= 0 ? "batchnorm (runs inside the launch of layer " + std::to_string(fused_into) + "; no launch of its own)" : "batchnorm";
+        return fused_into >= 0 ? "batchnorm (runs inside the launch of layer " + std::to_string(fused_into) + "; no launch of its own)" : cat.n ? "batchnorm with the concatenation in front of it" : "batchnorm";
     }
     int fused_into = -1;
     bool have_weights = false;
     std::vector<float> block;
     BnParams p{};
+    CatParams cat{};   // the concatenation in front, when this layer makes its launch (fuse_concat_layers)
     float *scale_dev = nullptr, *bias_dev = nullptr;
 };
 

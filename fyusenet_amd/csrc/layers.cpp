@@ -589,20 +589,43 @@ class ConcatLayer : public Layer {
     void port_shape(int port, int& c, int& h, int& w, int& pad) const override {
         c = d.inputs[port].channels; h = d.height; w = d.width; pad = d.inputs[port].padding;
     }
+    // the layer in one launch; one launch per input where its channels are no whole vectors
+    void setup() override {
+        whole = CatParams{};
+        whole.n = d.num_inputs;
+        whole.out = tout().v;
+        whole.act = act();
+        if (relu && whole.act.kind == ACT_NONE) {
+            whole.act.kind = ACT_RELU;
+            whole.act.lo = 0.f;
+        }
+        int off = 0;
+        for (int i = 0; i < std::min<int>(d.num_inputs, CatParams::kMost); i++) {
+            whole.part[i].in = tin(i).v;
+            whole.part[i].in.c = d.inputs[i].channels;
+            whole.part[i].c_off = off;
+            off += d.inputs[i].channels;
+        }
+        one_launch = launch_cat_supported(whole);
+        joined = whole;
+    }
     void forward(hipStream_t s) override {
-        Act a = act();
-        if (relu && a.kind == ACT_NONE) {
-            a.kind = ACT_RELU;
-            a.lo = 0.f;
+        if (fused_into >= 0 && net->fusion_on()) return;   // written by the batch-norm layer behind
+        if (one_launch) {
+            launch_cat(net->fusion_on() ? joined : whole, s);
+            return;
         }
         int off = 0;
         for (int i = 0; i < d.num_inputs; i++) {
-            launch_concat_part(tin(i).v, tout().v, off, a, s, i == d.num_inputs - 1);
+            launch_concat_part(tin(i).v, tout().v, off, whole.act, s, i == d.num_inputs - 1);
             off += d.inputs[i].channels;
         }
     }
-    std::string info() const override { return "concat"; }
+    std::string info() const override { return fused_into >= 0 ? "concat (runs inside the launch of layer " + std::to_string(fused_into) + "; no launch of its own)" : "concat"; }
     bool relu;
+    bool one_launch = false;
+    CatParams whole{}, joined{};   // the layer alone; with the scale layers in front of it
+    int fused_into = -1;
 };
 
 class ArgMaxLayer : public Layer {
@@ -770,6 +793,59 @@ void Net::copy_argmax(int layer_no, int32_t* idx, float* val) {
     ArgMaxLayer* l = dynamic_cast<ArgMaxLayer*>(layer(layer_no));
     if (!l) fail(FYN_ERR_INVALID, "layer %d is not an arg-max layer", layer_no);
     download_argmax(l->idx_dev, l->tout().v, idx, val);
+}
+
+// What stands around a concatenation becomes part of its launch: bilinear scale layers that only it reads, and a batch-norm
+// layer that is its only reader (which then makes the launch, in its own place in the order).  Neither the scaled nor the
+// concatenated tensor is written.  What is read in place of them must still be there when the launch runs: no tensor
+// produced in between may live in the same buffer.
+void fuse_concat_layers(Net* net) {
+    if (net->sw.get("FYNHIP_NO_CONCAT_FUSION") || !net->reuse_buffers) return;
+    std::map<int, int> readers;
+    for (auto& kv : net->layers)
+        for (int t : kv.second->in)
+            if (t >= 0) readers[t]++;
+    auto survives = [&](int tensor, int from, int to) {   // from the end of layer `from` through layer `to`
+        for (size_t i = 0; i < net->tensors.size(); i++) {
+            const Tensor& o = net->tensors[i];
+            if ((int)i != tensor && o.buffer == net->tensors[tensor].buffer && o.producer > from && o.producer <= to) return false;
+        }
+        return true;
+    };
+    for (auto& kv : net->layers) {
+        ConcatLayer* cat = dynamic_cast<ConcatLayer*>(kv.second.get());
+        if (!cat || !cat->one_launch) continue;
+        const Tensor& t = net->tensors[cat->out];
+        BatchNormLayer* bn = nullptr;
+        if (!t.locked && readers[cat->out] == 1)
+            for (auto& kr : net->layers)
+                if (!kr.second->in.empty() && kr.second->in[0] == cat->out) bn = dynamic_cast<BatchNormLayer*>(kr.second.get());
+        if (bn && (bn->p.res.ptr || bn->fused_into >= 0 || bn->d.number < cat->d.number || bn->p.out.cp != t.v.cp || bn->p.out.f16 != t.v.f16)) bn = nullptr;
+        for (int i = 0; bn && i < cat->d.num_inputs; i++)
+            if (!survives(cat->in[i], cat->d.number, bn->d.number)) bn = nullptr;
+        const int at = bn ? bn->d.number : cat->d.number;
+        for (int i = 0; i < cat->d.num_inputs; i++) {
+            const Tensor& x = net->tensors[cat->in[i]];
+            FuncLayer* f = x.producer >= 0 ? dynamic_cast<FuncLayer*>(net->layer(x.producer)) : nullptr;
+            if (!f || !f->linear || x.locked || readers[cat->in[i]] != 1 || f->p.in.c != cat->whole.part[i].in.c || !survives(f->in[0], f->d.number, at)) continue;
+            CatParams with = cat->joined;
+            CatPart& q = with.part[i];
+            q.in = f->p.in;
+            q.linear = 1;
+            q.ux = f->p.ux; q.uy = f->p.uy; q.dx = f->p.dx; q.dy = f->p.dy; q.ox = f->p.ox; q.oy = f->p.oy;
+            q.act = f->p.act;
+            if (!launch_cat_supported(with)) continue;
+            cat->joined = with;
+            f->computed_by(at);
+        }
+        if (bn) {
+            bn->cat = cat->joined;
+            bn->cat.out = bn->p.out;
+            bn->cat.scale = bn->scale_dev; bn->cat.bias = bn->bias_dev;
+            bn->cat.bn_act = bn->p.act;
+            cat->fused_into = bn->d.number;
+        }
+    }
 }
 
 }  // namespace fynhip
