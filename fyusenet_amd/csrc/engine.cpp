@@ -469,6 +469,7 @@ void Net::setup() {
     fuse_batchnorm_layers(this);
     fuse_function_layers(this);
     fuse_concat_layers(this);
+    fuse_argmax_layers(this);
     assign_range_resets();
     poison_lds_ = sw.get("FYNHIP_POISON_LDS") != nullptr;
     FYN_HIP(hipStreamSynchronize(stream));

@@ -238,6 +238,7 @@ void fuse_projection_layers(Net* net);   // after every layer's setup(): 1x1 sho
 void fuse_depthwise_layers(Net* net);   // after every layer's setup(): depthwise 3x3 layers that their 1x1 reader can compute itself
 void fuse_function_layers(Net* net);   // after every layer's setup(): sigmoid / tanh layers that the row-rolling convolution in front of them can apply to what it stores
 void fuse_concat_layers(Net* net);   // after every layer's setup(): bilinear scale layers in front of concatenations and batch-norm layers behind them
+void fuse_argmax_layers(Net* net);   // after every layer's setup(): arg-max layers that the streaming 1x1 convolution in front of them can compute
 Layer* create_custom_layer(Net* net, const fyn_layer_desc& d, const fyn_custom_layer& impl);
 
 }  // namespace fynhip

@@ -321,6 +321,15 @@ int launch_conv_d16(const ConvP16Params& p, hipStream_t s);   // (p.dw_in set: w
 bool conv_d16_dw_supported(int chunks, int dw_stride);
 // (p.tile_h = 3, 5 or 7: a K x K convolution on an input of at most four channels instead, cin_chunks = steps of eight taps)
 bool conv_d16_small_supported(int k, int dil, int in_cp, int cout, int out_cp);
+// 1x1 convolutions on many positions with few channels, and the arg-max over the result's channels (conv_s16.hip)
+struct ArgMaxTail {
+    TView out;      // the arg-max layer's tensor: index, value
+    int* idx;       // exact indices; null: no arg-max
+    int channels;
+    Act act;        // the layer's activation on fetch
+};
+bool conv_s16_supported(int k, int dil, int in_cp, int cout, int out_cp, bool f16);
+int launch_conv_s16(const ConvP16Params& p, const ArgMaxTail& tail, hipStream_t s);
 // 3x3 convolutions between tensors of few channels, any stride, edge rule and source step (conv_g16.hip)
 bool conv_g16_supported(int k, int dil, int in_cp, int cout, int out_cp);
 int conv_g16_steps(int in_cp);                       // matrix steps of the window

@@ -628,6 +628,54 @@ class ConvLayer : public Layer {
             net->dev_free(wp);
         }
     }
+    // The streaming 1x1 form for many positions and few channels (conv_s16.hip) against what has been chosen so far.
+    void setup_s16(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
+        ConvP16Params q{};
+        q.in = in_v.ptr; q.out = out_v.ptr; q.res = res_v ? res_v->ptr : nullptr;
+        q.in_hp = in_v.hp(); q.in_wp = in_v.wp(); q.in_cp = in_v.cp;
+        q.stride = stride;
+        q.in_y0 = q.in_x0 = in_v.pad;
+        q.npos_y = oh; q.npos_x = ow;
+        q.out_wp = out_v.wp(); q.out_cp = out_v.cp; q.out_off_y = q.out_off_x = out_v.pad;
+        if (res_v) { q.res_wp = res_v->wp(); q.res_cp = res_v->cp; q.res_off_y = q.res_off_x = res_v->pad; }
+        q.res_relu = res_relu; q.res_scale = res_scale;
+        q.cin_chunks = (in_v.cp + 31) / 32;
+        q.mfrags = (oc + 15) / 16;
+        q.wm = q.cout_blocks = 1;
+        q.f16 = out_v.f16 ? 1 : 0;
+        q.scale = scale_dev; q.bias = bias_dev;
+        q.acc_mul = 1.f;
+        q.act = act();
+        q.in_amax = tin(0).amax;
+        void* const wp = net->dev_alloc((size_t)q.mfrags * q.cin_chunks * (q.f16 ? 1 : 2) * 1024, true);
+        q.wpack = wp;
+        const char* at = net->sw.get("FYNHIP_AUTOTUNE");
+        bool pick = net->sw.get("FYNHIP_FORCE_S16_CONV") != nullptr;
+        char key[160];
+        snprintf(key, sizeof(key), "s16:%dx%d:%dx%d:s%d:cp%d:r%d:h%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, q.f16);
+        if (!pick && !tune_cache_flag(net, key, &pick) && !(at && at[0] == '0')) {
+            float t_new = 1e30f, t_other = 1e30f;
+            for (int rep = 0; rep < 3; rep++) {
+                t_new = std::min(t_new, time_calls(net, [&]() {
+                    if (launch_conv_s16(q, ArgMaxTail{}, net->stream) != 0) fail(FYN_ERR_DEVICE, "streaming 1x1 convolution launch failed while tuning");
+                }, 10));
+                t_other = std::min(t_other, time_calls(net, [&]() { run(net->stream); }, 10));
+            }
+            if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
+                fprintf(stderr, "[tune] 1x1 on %d channels, %dx%d positions, to %d: streaming form %.1f us, %s %.1f us\n", in_v.cp, oh, ow, oc, t_new * 1e3f, own_info().c_str(), t_other * 1e3f);
+            pick = t_new < t_other;
+            tune_cache_store_flag(net, key, pick);
+        }
+        if (pick) {
+            if (p16) net->dev_free(p16_wpack_dev);
+            p16_wpack_dev = wp;
+            p16 = s16 = true;
+            kr16 = d16 = false;
+            pp = q;
+        } else {
+            net->dev_free(wp);
+        }
+    }
     // The LDS-staged weights, gathered windows form for few channels (conv_g16.hip) against what has been chosen so far.
     void setup_g16(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
         ConvP16Params q{};
@@ -1126,6 +1174,12 @@ class ConvLayer : public Layer {
                 (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 8 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_D16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") &&
                 !net->sw.get("FYNHIP_FORCE_KSPLIT") && !net->sw.get("FYNHIP_CONV_TILE") && !net->sw.get("FYNHIP_CONV_KC") && !net->sw.get("FYNHIP_CONV_KC_MAX") && !net->sw.get("FYNHIP_CONV_PD"))
                 setup_d16(in_v, out_v, res_v, res_relu, res_scale);
+            // few channels on both sides, 1x1, images of 128x128 and more (below, the forms that take neighbouring
+            // depthwise and batch-norm layers into their launch are as fast): streaming
+            if (!frac_shift && same_storage && conv_s16_supported(k, dil, in_v.cp, oc, out_v.cp, out_v.f16 != 0) && d.in_channels <= in_v.cp &&
+                (oh * ow >= 16384 || net->sw.get("FYNHIP_FORCE_S16_CONV")) && (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") &&
+                !net->sw.get("FYNHIP_NO_S16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") && !net->sw.get("FYNHIP_FORCE_D16_CONV") && !net->sw.get("FYNHIP_D16_BLOCKS") && !only_kr)
+                setup_s16(in_v, out_v, res_v, res_relu, res_scale);
             // few channels on both sides, 3x3: windows gathered from the tensor
             if (!h16 && !c4 && !d16 && same_storage && conv_g16_supported(k, dil, in_v.cp, oc, out_v.cp) && d.in_channels <= in_v.cp &&
                 (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_G16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") && !only_kr)
@@ -1161,6 +1215,7 @@ class ConvLayer : public Layer {
             const float wmul = weight_prescale(w, (size_t)oc * k * k * d.in_channels);
             pp.acc_mul = pp2.acc_mul = 1.0f / wmul;
             if (g16) pack_g16(w, wmul);
+            else if (s16) pack_frag16(pp, p16_wpack_dev, w, wmul);
             else if (c4) pack_c4(w, wmul);
             else if (d16) pack_d16(w, wmul);
             else if (kr16) pack_kr16(w, wmul);
@@ -1260,7 +1315,7 @@ class ConvLayer : public Layer {
             return;
         }
         if (p16) {
-            if ((g16 ? launch_conv_g16(pp, s) : c4 ? launch_conv_p16c4(pp, k, s) : (d16 ? launch_conv_d16(pp, s) : (kr16 ? launch_conv_kr16(pp, k, s) : (h16 ? launch_conv_h16(pp, k, s) : launch_conv_p16(pp, s))))) != 0 ||
+            if ((s16 ? launch_conv_s16(pp, net->fusion_on() ? argmax_tail : ArgMaxTail{}, s) : g16 ? launch_conv_g16(pp, s) : c4 ? launch_conv_p16c4(pp, k, s) : (d16 ? launch_conv_d16(pp, s) : (kr16 ? launch_conv_kr16(pp, k, s) : (h16 ? launch_conv_h16(pp, k, s) : launch_conv_p16(pp, s))))) != 0 ||
                 (h16 && h16_two && launch_conv_h16(pp2, k, s) != 0))
                 fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
@@ -1301,6 +1356,11 @@ class ConvLayer : public Layer {
                      pp.f16 ? "f16" : (conv_p16c4_uses_fp8(pp, k) ? "f16+fp8-split" : "f16x2-split"), pp.tile_h * pp.tile_w * 4, pp.tile_h, pp.tile_w, pp.pos_groups * pp.cout_blocks, pp.tiles_x * pp.tiles_y * pp.cout_blocks,
                      conv_p16c4_lds_bytes(pp, k), c4_steps);
             return mode + buf + (conv_p16_stores_through(pp, 1) ? " stores=through" : "");
+        }
+        if (p16 && s16) {
+            char buf[220];
+            snprintf(buf, sizeof(buf), "conv_s16 %s streaming: %d chunks and %d fragments of 16 output channels in registers", pp.f16 ? "f16" : "f16x2-split", pp.cin_chunks, pp.mfrags);
+            return mode + buf + (argmax_tail.idx ? "; the arg-max layer behind it is computed from what is stored" : "");
         }
         if (p16 && g16) {
             char buf[220];
@@ -1364,6 +1424,8 @@ class ConvLayer : public Layer {
     int c4_steps = 0;
     bool h16 = false;             // ... its fp16-storage form for wide layers (conv_h16.hip)
     bool kr16 = false;            // ... the K-resident form for layers with few positions (conv_p16.hip, conv_kr16_kernel)
+    bool s16 = false;             // ... the streaming 1x1 form (conv_s16.hip)
+    ArgMaxTail argmax_tail{};     // ... with the arg-max layer behind it (fuse_argmax_layers)
     bool g16 = false;             // ... the form that gathers 3x3 windows of few channels (conv_g16.hip)
     bool d16 = false;             // ... the LDS-free 1x1 form for many positions and few input channels (conv_d16.hip)
     // A depthwise 3x3 layer whose only reader is this 1x1 layer in the K-resident form can be computed inside this

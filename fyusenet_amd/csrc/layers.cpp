@@ -636,9 +636,13 @@ class ArgMaxLayer : public Layer {
         ow = d.width;
     }
     void setup() override { idx_dev = static_cast<int32_t*>(net->dev_alloc((size_t)oh * ow * sizeof(int32_t))); }
-    void forward(hipStream_t s) override { launch_argmax(tin(0).v, tout().v, idx_dev, act(), s); }
-    std::string info() const override { return "argmax"; }
+    void forward(hipStream_t s) override {
+        if (fused_into >= 0 && net->fusion_on()) return;   // computed by the convolution in front
+        launch_argmax(tin(0).v, tout().v, idx_dev, act(), s);
+    }
+    std::string info() const override { return fused_into >= 0 ? "argmax (runs inside the launch of layer " + std::to_string(fused_into) + "; no launch of its own)" : "argmax"; }
     int32_t* idx_dev = nullptr;
+    int fused_into = -1;
 };
 
 class UploadLayer : public Layer {
@@ -793,6 +797,27 @@ void Net::copy_argmax(int layer_no, int32_t* idx, float* val) {
     ArgMaxLayer* l = dynamic_cast<ArgMaxLayer*>(layer(layer_no));
     if (!l) fail(FYN_ERR_INVALID, "layer %d is not an arg-max layer", layer_no);
     download_argmax(l->idx_dev, l->tout().v, idx, val);
+}
+
+// An arg-max layer behind a 1x1 convolution in the streaming form: the convolution computes it from the values it stores
+// (whoever else reads them).  The launch writes the arg-max layer's tensor earlier than its buffer was handed over for:
+// every other tenant of the buffer must be through by then.
+void fuse_argmax_layers(Net* net) {
+    if (net->sw.get("FYNHIP_NO_ARGMAX_FUSION") || !net->reuse_buffers) return;
+    for (auto& kv : net->layers) {
+        ArgMaxLayer* am = dynamic_cast<ArgMaxLayer*>(kv.second.get());
+        if (!am) continue;
+        const Tensor& t = net->tensors[am->in[0]];
+        const Tensor& o = net->tensors[am->out];
+        ConvLayer* c = t.producer >= 0 ? dynamic_cast<ConvLayer*>(net->layer(t.producer)) : nullptr;
+        if (!c || !c->s16 || c->argmax_tail.idx || o.v.f16 != t.v.f16 || o.v.cp != 4 || o.v.h != t.v.h || o.v.w != t.v.w || t.v.c > 16 * c->pp.mfrags) continue;
+        bool early_ok = true;
+        for (const Tensor& other : net->tensors)
+            if (&other != &o && other.buffer == o.buffer && other.producer < am->d.number && std::max(other.last_reader, other.producer) >= c->d.number) early_ok = false;
+        if (!early_ok) continue;
+        c->argmax_tail = ArgMaxTail{o.v, am->idx_dev, t.v.c, am->act()};
+        am->fused_into = c->d.number;
+    }
 }
 
 // What stands around a concatenation becomes part of its launch: bilinear scale layers that only it reads, and a batch-norm

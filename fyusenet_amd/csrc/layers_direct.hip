@@ -902,9 +902,20 @@ __global__ __launch_bounds__(256) void cat_kernel(const CatParams p) {
     const int y = blockIdx.y, x = (int)(i / cg), c = (int)(i - (unsigned)x * cg) * V;
     FV<V> v;
     if (q.linear) {
-        const int ny = (2 * y + 1) * q.dy - q.oy - q.uy, nx = (2 * x + 1) * q.dx - q.ox - q.ux;
-        const int y0 = floordiv_pos(ny, 2 * q.uy), x0 = floordiv_pos(nx, 2 * q.ux);
-        const float fy = (float)(ny - y0 * 2 * q.uy) / (float)(2 * q.uy), fx = (float)(nx - x0 * 2 * q.ux) / (float)(2 * q.ux);
+        // (factors that are powers of two, as scale factors are: shifts instead of divisions, the same values)
+        auto split = [](int n, int d, float& f) {
+            int q0;
+            if ((d & (d - 1)) == 0) {
+                q0 = n >> __builtin_ctz(d);
+                f = (float)(n & (d - 1)) * __frcp_rn((float)d);
+            } else {
+                q0 = floordiv_pos(n, d);
+                f = (float)(n - q0 * d) / (float)d;
+            }
+            return q0;
+        };
+        float fy, fx;
+        const int y0 = split((2 * y + 1) * q.dy - q.oy - q.uy, 2 * q.uy, fy), x0 = split((2 * x + 1) * q.dx - q.ox - q.ux, 2 * q.ux, fx);
         const int sy = y0 + q.in.pad, sx = x0 + q.in.pad;
         const FV<V> t00 = fetch_clamped_v<T, V>(q.in, sy, sx, c), t01 = fetch_clamped_v<T, V>(q.in, sy, sx + 1, c);
         const FV<V> t10 = fetch_clamped_v<T, V>(q.in, sy + 1, sx, c), t11 = fetch_clamped_v<T, V>(q.in, sy + 1, sx + 1, c);

@@ -1,11 +1,13 @@
 """Convolutions between tensors of few channels: the form that gathers 3x3 windows from the tensor (conv_g16), at the
 edges of its 16-position tiles, channel groups and fragments, for every edge rule, step and source step; and a sigmoid or
-tanh layer that the convolution in front of it applies to what it stores.  Tolerances: rel-L2 <= 1e-4 (fp32 storage),
+tanh layer that the convolution in front of it applies to what it stores.  The streaming 1x1 form (conv_s16) at the edges of
+its trips, chunks and fragments, with the arg-max layer behind it.  Tolerances: rel-L2 <= 1e-4 (fp32 storage),
 <= 2e-3 (fp16 storage)."""
+import numpy as np
 import pytest
 
 import fyusenet_amd as fa
-from fyusenet_amd import prng, samples
+from fyusenet_amd import networks, prng, samples
 from fyusenet_amd.builders import ActType, ConvLayerBuilder, LayerType
 from oracle import oracle as O
 from util import conv_block, oracle_single, rel_l2, run_single
@@ -88,3 +90,79 @@ def test_function_layer_applied_by_the_convolution_in_front(monkeypatch, storage
         net.cleanup()
     assert rel_l2(outs[0], outs[1]) <= (1e-6 if storage == fa.STORAGE_F32 else 1e-4)
     assert rel_l2(outs[0], want) <= TOL[storage]
+
+
+# cin, cout, h, w, stride, pads (in, out), act, residual
+STREAMED = [
+    (8, 8, 3, 5, 1, (0, 0), ActType.NONE, None),                 # fewer positions than a trip, a quarter of a chunk
+    (32, 21, 37, 29, 1, (0, 1), ActType.RELU, None),             # ragged fragment, halo behind
+    (40, 16, 20, 66, 1, (1, 0), ActType.LEAKY_RELU, None),       # ragged second chunk, halo in front, a leak
+    (96, 32, 31, 33, 1, (0, 0), ActType.RELU, ActType.RELU),
+    (16, 64, 50, 130, 2, (0, 0), ActType.CLIP, None),            # steps over the input
+    (128, 20, 16, 17, 1, (0, 0), ActType.NONE, ActType.NONE),
+]
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("case", STREAMED, ids=lambda c: "%dto%d_%dx%d_s%d" % c[:5])
+def test_streamed_pointwise(monkeypatch, case, storage):
+    cin, cout, h, w, stride, (pad_in, pad_out), act, residual = case
+    monkeypatch.setenv("FYNHIP_FORCE_S16_CONV", "1")
+    b = ConvLayerBuilder(1, "conv").type(LayerType.CONVOLUTION2D).number(1).shape(cout, h, w, cin).prefixAct(act).downsample(stride)
+    b.deep().inputPadding(pad_in).outputPadding(pad_out)
+    if act == ActType.LEAKY_RELU:
+        b.leakyReLU(0.2)
+    if act == ActType.CLIP:
+        b.clip(-0.5, 0.75)
+    inputs = [prng.normal(71 + cin, (cin, h, w))]
+    if residual is not None:
+        b.residual(residual).residualPadding(pad_out)
+        inputs.append(prng.normal(73 + cin, (cout, h // stride, w // stride)))
+    weights = conv_block(79 + cin, cout, 1, cin)
+    got, info = run_single(b, storage, inputs, weights)
+    assert "conv_s16" in info, info
+    assert rel_l2(got, oracle_single(b, storage, inputs, weights)) <= TOL[storage]
+
+
+class Labels(networks._StreamNet):
+    """upload -> 3x3 conv -> 1x1 conv to the classes -> arg-max."""
+    config_id = 7
+    input_key = (0, 0)
+
+    def __init__(self, storage, w, h, classes, act):
+        super().__init__(storage)
+        self.w, self.h, self.classes, self.act = w, h, classes, act
+        self.output_layer, self.argmax_layer = 2, 3
+
+    def define(self):
+        w, h = self.w, self.h
+        self._add(fa.UpDownLayerBuilder(fa.UpDownLayerBuilder.UPLOAD, "upload").number(0).shape(3, h, w, 3).outputPadding(1))
+        self.conv(1, "front", 3, 3, 32, h, w, 0)
+        self.conv(2, "scores", 1, 32, self.classes, h, w, 1, act=ActType.RELU, bn=False)
+        self._add(fa.ArgMaxLayerBuilder("labels").number(3).shape(2, h, w, self.classes).prefixAct(self.act).deep())
+        self._edges.append((2, 3, 0))
+
+    def setInput(self, x):
+        self.layers[0].setInput(x, 0)
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("w,h,classes,act", [(150, 130, 21, ActType.NONE), (129, 129, 5, ActType.RELU), (131, 140, 64, ActType.NONE)])
+def test_argmax_computed_by_the_convolution_in_front(monkeypatch, storage, w, h, classes, act):
+    """Labels and best values are those of the stored scores: with ReLU on fetch many positions tie at zero."""
+    monkeypatch.setenv("FYNHIP_FORCE_S16_CONV", "1")
+    if storage == fa.STORAGE_F32 and classes > 32:
+        classes = 32
+    x = prng.uniform(9, (3, h, w), -1.0, 1.0)
+    net = Labels(storage, w, h, classes, act)
+    net.setup()
+    for _ in range(2):
+        net.setInput(x)
+        net.forward()
+        labels, best = net.getArgMax(3)
+    assert "no launch of its own" in net.layers[3].kernelInfo()
+    scores = net.getOutput(2)
+    net.cleanup()
+    fetched = np.maximum(scores, 0) if act == ActType.RELU else scores
+    assert np.array_equal(labels, fetched.argmax(axis=0))
+    assert np.array_equal(best, fetched.max(axis=0))
