@@ -517,6 +517,7 @@ struct FeedWord {
 struct HostFeed {
     FeedWord* word;   // page-locked; null: the frame is there
     unsigned base;
+    float ticks_per_pixel;   // of the 100 MHz clock, at the rate of a fast copy
 };
 // The value-range record (range.h) of an uploaded tensor, which the launch writes, and two zero words of device memory in
 // which its workgroups meet (they belong to one stream).  record null: none is kept.

@@ -33,7 +33,10 @@ __device__ __forceinline__ void await_feed(const HostFeed& f, unsigned need, uns
         const unsigned long long t0 = wall_clock64();
         unsigned r;
         while ((int)((r = __hip_atomic_load(&f.word->ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) - f.base) - need) < 0) {
-            __builtin_amdgcn_s_sleep(48);   // (1.3 us: more looks would take the link from the copy that is waited for)
+            // (not before the host can have come so far: a look takes the word's line from the core that is copying, and
+            // the link from the copy; 1.3 us at least)
+            const unsigned long long t1 = wall_clock64(), ticks = min(10000u, 130u + (unsigned)((float)(need - r) * f.ticks_per_pixel));
+            while (wall_clock64() - t1 < ticks) __builtin_amdgcn_s_sleep(8);
             if (wall_clock64() - t0 > kFeedTicks) {
                 __hip_atomic_store(&f.word->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 r = 0x7fffffffu;
