@@ -679,11 +679,11 @@ static size_t piece_pixels(size_t npix, size_t bytes) {
     return std::max<size_t>(4, ((npix + pieces - 1) / pieces + 3) & ~size_t(3));
 }
 
+static constexpr float kTicksPerByte = 1.f / 800.f;   // 80 GB/s, 10 ns a tick
+
 // A frame into its tensor.  Host memory: the converting launch is queued first and takes the pixels as the host puts them
 // into page-locked memory (HostFeed), so that launch latency, copy and transfer overlap: 3.8 MB in 90 us instead of 135 for
 // two copies with a launch behind each.
-static constexpr float kTicksPerByte = 1.f / 800.f;   // 80 GB/s, 10 ns a tick
-
 void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
     const size_t npix = (size_t)v.h * v.w, plane = (npix + 31) & ~size_t(31);
     const bool host = host_memory(data), planes = order == FYN_ORDER_CHANNELWISE;

@@ -3,8 +3,9 @@
 // The host side of a transfer is page-locked memory that the kernels read and write in place, over PCIe: conversion and
 // transfer are one launch, where a copy into a device buffer followed by a conversion kernel (or the reverse) costs a
 // second launch and a round trip through the runtime's copy queue -- 10 us on a small frame.  What bounds them is the
-// link (about 55 GB/s each way), so a thread moves sixteen bytes per access and 128 workgroups are enough: measured on
+// link (about 55 GB/s each way), so a thread moves sixteen bytes per access and few workgroups are enough: measured on
 // 25 MB, 64 to 256 workgroups of such loads 448 us = 55 GB/s, 1024 workgroups 488 us, the copy engine alone 439 us.
+// From the host 48 take a frame (below), to the host 128.
 // The same kernels serve buffers in device memory.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -19,7 +20,12 @@ namespace fynhip {
 namespace {
 constexpr unsigned kMaxBlocks = 128;          // buffers behind the link
 constexpr unsigned kMaxDeviceBlocks = 1024;   // buffers in device memory: 3.8 MB of pixels in 4 us instead of 11
-unsigned blocks_for(size_t items, bool device) { return (unsigned)std::min<size_t>(device ? kMaxDeviceBlocks : kMaxBlocks, (items + 255) / 256); }
+// Frames from the host: the workgroups keep pace with the host's copy, and each one's looks at its progress (HostFeed) and
+// its arrival at the end cost the others time.  A segmentation frame (3.7 MB) from call to launch complete, with 24, 32,
+// 40, 48, 64 and 80 workgroups: 106, 98, 92, 93, 96, 97 us (111 with 128 that ended with a fence each); 25 MB: 566, 492,
+// 489, 490, 497, 534.
+constexpr unsigned kMaxUploadBlocks = 48;
+unsigned upload_blocks(size_t items, bool device) { return (unsigned)std::min<size_t>(device ? kMaxDeviceBlocks : kMaxUploadBlocks, (items + 255) / 256); }
 
 // The host may still be copying the frame when the launch runs (HostFeed): before a workgroup reads pixels it looks, where
 // it has to, whether they are there.  The launch's own latency (8 us) and the host's copy then overlap the transfer
@@ -39,6 +45,7 @@ __device__ __forceinline__ void await_feed(const HostFeed& f, unsigned need, uns
             while (wall_clock64() - t1 < ticks) __builtin_amdgcn_s_sleep(8);
             if (wall_clock64() - t0 > kFeedTicks) {
                 __hip_atomic_store(&f.word->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (before the workgroup counts as arrived, below)
                 r = 0x7fffffffu;
                 break;
             }
@@ -90,6 +97,18 @@ __device__ __forceinline__ void tell_host(const HostDone& d) {
             __threadfence_system();
             __hip_atomic_store(d.flag, d.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
+    }
+}
+
+// The same for a launch that has read the host's memory.  What it tells is that nothing reads it any more, so nothing has to
+// be made visible first: the fence above is a write-back, 0.2 us for every workgroup and one after the other.
+__device__ __forceinline__ void tell_host_read(const HostDone& d) {
+    if (!d.flag) return;
+    __syncthreads();   // (the values read have all been used)
+    if (threadIdx.x == 0 && __hip_atomic_fetch_add(d.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+        __hip_atomic_store(d.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __hip_atomic_store(d.flag, d.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -153,10 +172,10 @@ __global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, si
         }
     }
     publish_range(range, vmax);
-    tell_host(done);
+    tell_host_read(done);
 }
 void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s) {
-    const dim3 grid(blocks_for(((size_t)t.h * t.w + 3) / 4 * (t.cp >> 2), device));
+    const dim3 grid(upload_blocks(((size_t)t.h * t.w + 3) / 4 * (t.cp >> 2), device));
     if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, range, feed, done);
     else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, range, feed, done);
 }
@@ -193,10 +212,10 @@ __global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, co
         }
     }
     publish_range(range, vmax);
-    tell_host(done);
+    tell_host_read(done);
 }
 void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s) {
-    const dim3 grid(blocks_for(((size_t)t.h * t.w * t.c + 3) / 4, device));
+    const dim3 grid(upload_blocks(((size_t)t.h * t.w * t.c + 3) / 4, device));
     if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, range, feed, done);
     else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, range, feed, done);
 }
@@ -269,7 +288,7 @@ __global__ __launch_bounds__(256) void tensor_to_run_kernel(const TView t, float
 void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
     const size_t npix = include_padding ? (size_t)t.hp() * t.wp() : (size_t)t.h * t.w;
     if (plane == npix && p0 == 0 && p1 == npix && (plane % 4 != 0 || plane < 256) && (reinterpret_cast<size_t>(chw) & 15) == 0 && t.c > 1) {
-        const dim3 grid(blocks_for((npix * t.c + 3) / 4, false));
+        const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, ((npix * t.c + 3) / 4 + 255) / 256));
         if (t.f16) hipLaunchKernelGGL(tensor_to_run_kernel<_Float16>, grid, dim3(256), 0, s, t, chw, (unsigned)npix, include_padding, done);
         else hipLaunchKernelGGL(tensor_to_run_kernel<float>, grid, dim3(256), 0, s, t, chw, (unsigned)npix, include_padding, done);
         return;
