@@ -456,6 +456,7 @@ void Net::setup() {
         b.free_after = std::max(t.last_reader, l->d.number);
         t.buffer = found;
         t.v.ptr = b.ptr;
+        t.written = t.producer;
     }
     // pass-through layers were given the tensor id only; nothing else to do for them
     assign_range_words();
@@ -474,6 +475,13 @@ void Net::setup() {
     poison_lds_ = sw.get("FYNHIP_POISON_LDS") != nullptr;
     FYN_HIP(hipStreamSynchronize(stream));
     is_setup = true;
+}
+
+bool Net::alone(int tensor, int from, int to) const {
+    const Tensor& t = tensors[tensor];
+    for (const Tensor& o : tensors)
+        if (&o != &t && o.buffer == t.buffer && o.written <= to && std::max(o.last_reader, o.producer) >= from) return false;
+    return true;
 }
 
 // Value ranges (range.h), fp32 storage only.  A tensor gets a word when whoever writes it keeps the word up to date:
@@ -511,10 +519,10 @@ void Net::assign_range_resets() {
         // layers behind the last reader, in execution order ...
         for (int no : order)
             if (no > last && layer(no)->add_range_reset(t.amax)) { done = true; break; }
-        // ... then the layers in front of the producer (they run in the next pass, before it)
+        // ... then the layers in front of the launch that writes it (they run in the next pass, before it)
         if (!done)
             for (int no : order)
-                if (no < t.producer && layer(no)->add_range_reset(t.amax)) { done = true; break; }
+                if (no < t.written && layer(no)->add_range_reset(t.amax)) { done = true; break; }
         if (!done) {
             t.amax = nullptr;
             lost = true;

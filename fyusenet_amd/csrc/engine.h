@@ -7,6 +7,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstdarg>
@@ -44,7 +45,8 @@ struct Error : public std::runtime_error {
 struct Tensor {
     TView v{};
     int producer = -1;     // layer number writing it (-1: external input)
-    int last_reader = -1;  // highest layer number reading it
+    int written = -1;      // layer in whose launch that happens: the producer, or a layer in front that computes it as well
+    int last_reader = -1;  // highest layer number in whose launch it is read
     bool locked = false;   // never reused (network outputs, external inputs)
     int buffer = -1;       // index into Net::buffers_
     unsigned* amax = nullptr;   // value-range word (range.h) when a producer keeps it, else null
@@ -156,6 +158,13 @@ class Net {
     std::vector<Tensor> tensors;
     std::vector<DevBuffer> buffers;
     uint64_t seq = 0;
+
+    // Whether a tensor's buffer is the tensor's alone from layer `from` through layer `to`: no other tensor in it is
+    // written by the launch of one of them, nor read by it.  Asked before a launch is made to write the tensor earlier
+    // than its producer, or to read it later than its last reader; whoever does so enters it in `written` or
+    // `last_reader`, which is what the next one to ask finds.
+    bool alone(int tensor, int from, int to) const;
+    void read_until(int tensor, int layer_no) { tensors[tensor].last_reader = std::max(tensors[tensor].last_reader, layer_no); }
 
     // device allocations owned by the net
     void* dev_alloc(size_t bytes, bool zero = true);

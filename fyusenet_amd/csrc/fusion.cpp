@@ -36,15 +36,8 @@ void fuse_depthwise_layers(Net* net) {
         ConvLayer* ex = dynamic_cast<ConvLayer*>(net->layer(t.producer));
         if (!ex || ex->k != 1 || ex->stride != 1 || ex->dil != 1 || ex->clamp || ex->frac_shift || ex->direct || (ex->d.flags & FYN_FLAG_RESIDUAL_INPUT)) continue;
         const TView& in_v = ex->tin(0).v;
-        // The launch writes the depthwise layer's output in the 1x1 layer's place in the order, i.e. earlier than the
-        // buffer was handed over for: every other tenant of that buffer must be through by then -- neither read at or
-        // behind the 1x1 layer (its own input included: the launch reads it while it writes) nor produced between the two.
-        bool early_ok = true;
-        for (const Tensor& o : net->tensors)
-            if (&o != &net->tensors[dw->out] && o.buffer == net->tensors[dw->out].buffer && o.producer < dw->d.number &&
-                std::max(o.last_reader, o.producer) >= ex->d.number)
-                early_ok = false;
-        if (!early_ok) continue;
+        // (the launch writes the depthwise layer's output in the 1x1 layer's place in the order, while it reads its own input)
+        if (!net->alone(dw->out, ex->d.number, dw->d.number)) continue;
         if (in_v.f16 != dw->p.out.f16 || ex->d.in_channels != in_v.cp || ex->tout().v.cp != dw->p.in.cp || ex->oc % 4 != 0 ||
             !conv_e16dw_supported(in_v.cp, (in_v.cp + 31) / 32, dw->stride))
             continue;
@@ -112,6 +105,7 @@ void fuse_depthwise_layers(Net* net) {
         ex->edw_fused = true;
         ex->edw_dw_no = dw->d.number;
         dw->fused_into = ex->d.number;
+        net->tensors[dw->out].written = ex->d.number;
         ex->pack_edw();
     }
     for (auto& kv : net->layers) {
@@ -124,15 +118,8 @@ void fuse_depthwise_layers(Net* net) {
         if (!dw || dw->dil != 1 || (dw->stride != 1 && dw->stride != 2) || dw->p.res.ptr || dw->p.in.cp % 8 != 0 || dw->p.in.cp != dw->p.out.cp ||
             dw->p.in.f16 != dw->p.out.f16 || dw->p.out.f16 != pw->pp.f16 || dw->p.out.cp != pw->pp.in_cp)
             continue;
-        // The launch reads the depthwise layer's input in the 1x1 layer's place in the order, i.e. later than the buffer
-        // was kept for: no tensor produced behind the depthwise layer up to and including the 1x1 layer (whose output
-        // the launch writes while it reads) may live in that buffer.
-        bool late_ok = true;
-        for (const Tensor& o : net->tensors)
-            if (&o != &net->tensors[dw->in[0]] && o.buffer == net->tensors[dw->in[0]].buffer && o.producer > dw->d.number &&
-                o.producer <= pw->d.number)
-                late_ok = false;
-        if (!late_ok) continue;
+        // (the launch reads the depthwise layer's input in the 1x1 layer's place in the order, while it writes that layer's output)
+        if (!net->alone(dw->in[0], dw->d.number, pw->d.number)) continue;
         ConvP16Params& f = pw->dw_fields;
         f.dw_in = dw->p.in.ptr; f.dw_w = dw->w_dev; f.dw_scale = dw->scale_dev; f.dw_bias = dw->bias_dev;
         f.dw_hp = dw->p.in.hp(); f.dw_wp = dw->p.in.wp(); f.dw_cp = dw->p.in.cp;
@@ -166,6 +153,7 @@ void fuse_depthwise_layers(Net* net) {
         pw->dw_fused = true;
         pw->dw_layer_no = dw->d.number;
         dw->fused_into = pw->d.number;
+        net->read_until(dw->in[0], pw->d.number);
     }
 }
 
@@ -195,8 +183,7 @@ void keep_projection_inputs(Net* net) {
         ConvLayer* c = dynamic_cast<ConvLayer*>(kv.second.get());
         ConvLayer* pr = projection_of(net, c);
         if (!pr) continue;
-        Tensor& x2 = net->tensors[pr->in[0]];
-        x2.last_reader = std::max(x2.last_reader, c->d.number);
+        net->read_until(pr->in[0], c->d.number);
     }
 }
 // A 1x1 projection (a residual block's shortcut convolution) whose only reader adds it to its own 1x1 convolution: both
@@ -218,14 +205,10 @@ void fuse_projection_layers(Net* net) {
         const TView& v1 = c->tin(0).v;
         const TView& v2 = pr->tin(0).v;
         const TView& ov = c->tout().v;
-        Tensor& x2 = net->tensors[pr->in[0]];
         if (v1.f16 != ov.f16 || v2.f16 != ov.f16 || rt.v.f16 != ov.f16 || c->d.in_channels != v1.cp || pr->d.in_channels != v2.cp || v1.cp % 8 != 0 || v2.cp % 8 != 0 ||
             v1.cp < 8 || v2.cp < 8 || c->oc % 4 != 0 || c->oc < 8 || ov.cp < c->oc || c->oh * c->ow > 4096)
             continue;
-        bool live = true;   // (the projection's input must still hold its values when the reader runs)
-        for (const Tensor& o : net->tensors)
-            if (&o != &x2 && o.buffer == x2.buffer && o.producer > pr->d.number && o.producer <= c->d.number) live = false;
-        if (!live) continue;
+        if (!net->alone(pr->in[0], pr->d.number, c->d.number)) continue;   // (the projection's input must still hold its values when the reader runs)
         const int n1 = (v1.cp + 31) / 32, n2 = (v2.cp + 31) / 32;
         ConvP16Params q{};
         q.in = v1.ptr; q.out = ov.ptr;
@@ -309,7 +292,7 @@ void fuse_projection_layers(Net* net) {
         c->pj_fused = true;
         c->pj_layer_no = pr->d.number;
         pr->pj_into = c->d.number;
-        x2.last_reader = std::max(x2.last_reader, c->d.number);   // (its value-range word is cleared behind its last reader)
+        net->read_until(pr->in[0], c->d.number);   // (its value-range word is cleared behind its last reader)
         c->pack_two_sources();
     }
 }
@@ -325,7 +308,7 @@ void fuse_batchnorm_layers(Net* net) {
     for (auto& kv : net->layers) {
         BatchNormLayer* bn = dynamic_cast<BatchNormLayer*>(kv.second.get());
         if (!bn || bn->p.res.ptr || bn->p.act.kind != ACT_NONE) continue;
-        Tensor& x = net->tensors[bn->in[0]];
+        const Tensor& x = net->tensors[bn->in[0]];
         const Tensor& y = net->tensors[bn->out];
         // (no halo: around the layer's output it holds zeros, which scale and bias applied to the input's halo would not give)
         if (y.locked || x.v.pad != 0 || y.v.pad != 0 || x.v.h != y.v.h || x.v.w != y.v.w || x.v.cp != y.v.cp || x.v.f16 != y.v.f16 || x.v.c != y.v.c) continue;
@@ -343,24 +326,20 @@ void fuse_batchnorm_layers(Net* net) {
             }
         }
         if (!all || readers.empty()) continue;
-        bool live = true;
-        for (const Tensor& o : net->tensors)
-            if (&o != &x && o.buffer == x.buffer && o.producer > bn->d.number && o.producer <= last) live = false;
-        if (!live) continue;
+        if (!net->alone(bn->in[0], bn->d.number, last)) continue;
         for (ConvLayer* c : readers) {
             c->bn_fused = true;
             c->bn_layer_no = bn->d.number;
             c->bn_in = x.v.ptr; c->bn_mul = bn->scale_dev; c->bn_add = bn->bias_dev;
         }
         bn->fused_into = readers.front()->d.number;
-        x.last_reader = std::max(x.last_reader, last);   // (its value-range word is cleared behind its last reader)
+        net->read_until(bn->in[0], last);   // (its value-range word is cleared behind its last reader)
     }
 }
 
 // A sigmoid or tanh layer whose input comes from a convolution in the row-rolling form and goes nowhere else (the end of
 // the style-net samples): the convolution applies it to what it stores, into the layer's own tensor.  The launch writes
-// that tensor in the convolution's place in the order, earlier than its buffer was handed over for: every other tenant
-// of the buffer must be through by then.
+// that tensor in the convolution's place in the order, earlier than its buffer was handed over for.
 void fuse_function_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_FUNCTION_FUSION") || !net->reuse_buffers) return;
     std::map<int, int> readers;
@@ -376,13 +355,11 @@ void fuse_function_layers(Net* net) {
         if (t.producer < 0 || t.locked || readers[f->in[0]] != 1) continue;
         ConvLayer* c = dynamic_cast<ConvLayer*>(net->layer(t.producer));
         if (!c || !c->rows || o.v.f16 != t.v.f16 || o.v.cp != 4 || t.v.cp != 4 || o.v.h != t.v.h || o.v.w != t.v.w) continue;
-        bool early_ok = true;
-        for (const Tensor& other : net->tensors)
-            if (&other != &o && other.buffer == o.buffer && other.producer < f->d.number && std::max(other.last_reader, other.producer) >= c->d.number) early_ok = false;
-        if (!early_ok) continue;
+        if (!net->alone(f->out, c->d.number, f->d.number)) continue;
         c->fn_layer_no = f->d.number;
         c->fn_params = *p;
         f->computed_by(c->d.number);
+        net->tensors[f->out].written = c->d.number;
     }
 }
 

@@ -800,8 +800,7 @@ void Net::copy_argmax(int layer_no, int32_t* idx, float* val) {
 }
 
 // An arg-max layer behind a 1x1 convolution in the streaming form: the convolution computes it from the values it stores
-// (whoever else reads them).  The launch writes the arg-max layer's tensor earlier than its buffer was handed over for:
-// every other tenant of the buffer must be through by then.
+// (whoever else reads them).  The launch writes the arg-max layer's tensor earlier than its buffer was handed over for.
 void fuse_argmax_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_ARGMAX_FUSION") || !net->reuse_buffers) return;
     for (auto& kv : net->layers) {
@@ -811,32 +810,22 @@ void fuse_argmax_layers(Net* net) {
         const Tensor& o = net->tensors[am->out];
         ConvLayer* c = t.producer >= 0 ? dynamic_cast<ConvLayer*>(net->layer(t.producer)) : nullptr;
         if (!c || !c->s16 || c->argmax_tail.idx || o.v.f16 != t.v.f16 || o.v.cp != 4 || o.v.h != t.v.h || o.v.w != t.v.w || t.v.c > 16 * c->pp.mfrags) continue;
-        bool early_ok = true;
-        for (const Tensor& other : net->tensors)
-            if (&other != &o && other.buffer == o.buffer && other.producer < am->d.number && std::max(other.last_reader, other.producer) >= c->d.number) early_ok = false;
-        if (!early_ok) continue;
+        if (!net->alone(am->out, c->d.number, am->d.number)) continue;
         c->argmax_tail = ArgMaxTail{o.v, am->idx_dev, t.v.c, am->act()};
         am->fused_into = c->d.number;
+        net->tensors[am->out].written = c->d.number;
     }
 }
 
 // What stands around a concatenation becomes part of its launch: bilinear scale layers that only it reads, and a batch-norm
 // layer that is its only reader (which then makes the launch, in its own place in the order).  Neither the scaled nor the
-// concatenated tensor is written.  What is read in place of them must still be there when the launch runs: no tensor
-// produced in between may live in the same buffer.
+// concatenated tensor is written.  What is read in place of them must still be there when the launch runs.
 void fuse_concat_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_CONCAT_FUSION") || !net->reuse_buffers) return;
     std::map<int, int> readers;
     for (auto& kv : net->layers)
         for (int t : kv.second->in)
             if (t >= 0) readers[t]++;
-    auto survives = [&](int tensor, int from, int to) {   // from the end of layer `from` through layer `to`
-        for (size_t i = 0; i < net->tensors.size(); i++) {
-            const Tensor& o = net->tensors[i];
-            if ((int)i != tensor && o.buffer == net->tensors[tensor].buffer && o.producer > from && o.producer <= to) return false;
-        }
-        return true;
-    };
     for (auto& kv : net->layers) {
         ConcatLayer* cat = dynamic_cast<ConcatLayer*>(kv.second.get());
         if (!cat || !cat->one_launch) continue;
@@ -847,12 +836,12 @@ void fuse_concat_layers(Net* net) {
                 if (!kr.second->in.empty() && kr.second->in[0] == cat->out) bn = dynamic_cast<BatchNormLayer*>(kr.second.get());
         if (bn && (bn->p.res.ptr || bn->fused_into >= 0 || bn->d.number < cat->d.number || bn->p.out.cp != t.v.cp || bn->p.out.f16 != t.v.f16)) bn = nullptr;
         for (int i = 0; bn && i < cat->d.num_inputs; i++)
-            if (!survives(cat->in[i], cat->d.number, bn->d.number)) bn = nullptr;
+            if (!net->alone(cat->in[i], cat->d.number, bn->d.number)) bn = nullptr;
         const int at = bn ? bn->d.number : cat->d.number;
         for (int i = 0; i < cat->d.num_inputs; i++) {
             const Tensor& x = net->tensors[cat->in[i]];
             FuncLayer* f = x.producer >= 0 ? dynamic_cast<FuncLayer*>(net->layer(x.producer)) : nullptr;
-            if (!f || !f->linear || x.locked || readers[cat->in[i]] != 1 || f->p.in.c != cat->whole.part[i].in.c || !survives(f->in[0], f->d.number, at)) continue;
+            if (!f || !f->linear || x.locked || readers[cat->in[i]] != 1 || f->p.in.c != cat->whole.part[i].in.c || !net->alone(f->in[0], f->d.number, at)) continue;
             CatParams with = cat->joined;
             CatPart& q = with.part[i];
             q.in = f->p.in;
@@ -862,7 +851,9 @@ void fuse_concat_layers(Net* net) {
             if (!launch_cat_supported(with)) continue;
             cat->joined = with;
             f->computed_by(at);
+            net->read_until(f->in[0], at);
         }
+        for (int i = 0; i < cat->d.num_inputs; i++) net->read_until(cat->in[i], at);
         if (bn) {
             bn->cat = cat->joined;
             bn->cat.out = bn->p.out;
