@@ -706,15 +706,15 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         FYN_HIP(hipStreamSynchronize(stream));   // the caller's buffer is borrowed for this call only
         return;
     }
-    // (page-locked memory, the pool's again when the launch has told that it is through; a caller that never waits is
-    // held at a few frames)
+    // (a caller that never waits is held at a few frames)
     const size_t bytes = plane * v.c * sizeof(float);
     unsigned& before = uploads_told_[upload_no_++ % kUploads];
     if (before) signal_.wait(before, stream);
-    float* st = static_cast<float*>(HostPool::acquire(bytes, false, true));
+    HostLoan area(bytes, true);
     count_area(bytes, in_most_);
+    float* st = area.floats();
     // pieces: a small one first, so that the launch has something to do when it starts; multiples of 32 pixels (whole lines)
-    HostCopy copies;
+    HostCopy copies;   // (made before the loan ends, whatever happens)
     std::vector<std::pair<size_t, size_t>> pieces;   // copies made, pixels complete
     const size_t most = std::max<size_t>(4096, (256u << 10) / (v.c * sizeof(float)) & ~size_t(31));
     size_t step = most / 8 & ~size_t(31);
@@ -726,13 +726,20 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         p0 = p1;
         step = std::min(most, step * 2);
     }
-    const HostDone done = signal_.next();
-    before = done.value;
     auto launch = [&](const HostFeed& feed) {
+        const HostDone done = signal_.next();
         if (planes) launch_chw_to_tensor(st, plane, v, range, feed, done, false, stream);
         else launch_hwc_to_tensor(st, v, range, feed, done, false, stream);
-        FYN_HIP(hipGetLastError());
-        signal_.release_then(st, done.value);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            // (one that is not running will not tell, and one that is runs to its end once the frame is there)
+            copies.upto(copies.mark());
+            if (feed.word) __atomic_store_n(&feed.word->ready, feed.base + (unsigned)npix, __ATOMIC_RELEASE);
+            (void)hipStreamSynchronize(stream);
+            fail(FYN_ERR_DEVICE, "converting a frame failed: %s", hipGetErrorString(e));
+        }
+        before = done.value;
+        area.used_until(signal_, done.value);
     };
     copies.start();
     if (!feed_ahead_) {
@@ -741,8 +748,8 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         return;
     }
     const HostFeed feed{feed_, feed_base_, (float)v.c * (float)sizeof(float) * kTicksPerByte};
-    launch(feed);
     feed_base_ += (unsigned)npix;
+    launch(feed);
     for (const auto& piece : pieces) {
         copies.upto(piece.first);
         __atomic_store_n(&feed_->ready, feed.base + (unsigned)piece.second, __ATOMIC_RELEASE);

@@ -19,27 +19,13 @@ class HostPool {
     static constexpr size_t kBytes = size_t(512) << 20;
     static void* acquire(size_t bytes, bool bounded, bool filled_by_host = false);   // bounded: null when the pool is full or there is no GPU; else throws when memory cannot be had
     static void release(void* p);                       // null is nothing
-    static void release_then(void* p, const unsigned* flag, unsigned value);   // when the word `flag` reads `value` (HostSignal)
+    static void release_then(void* p, const unsigned* flag, unsigned value);   // when the word `flag` reads `value` (HostSignal); nothing else may use the block any more by now
     static void forget(const unsigned* flag);           // the word goes away: blocks that wait for it are free
     static bool contains(const void* p, size_t bytes);  // whether the range lies inside a block on loan
     static void network_created();
     static void network_gone();
 };
 
-// A block on loan for a scope.
-class HostLoan {
-  public:
-    HostLoan() = default;
-    explicit HostLoan(size_t bytes) : p_(HostPool::acquire(bytes, false)) {}
-    HostLoan(HostLoan&& o) noexcept : p_(o.p_) { o.p_ = nullptr; }
-    HostLoan(const HostLoan&) = delete;
-    HostLoan& operator=(const HostLoan&) = delete;
-    ~HostLoan() { HostPool::release(p_); }
-    float* floats() const { return static_cast<float*>(p_); }
-
-  private:
-    void* p_ = nullptr;
-};
 
 // Copies between host buffers, shared with a few helper threads of the process when they are large: one core moves 20 to
 // 40 GB/s of memory that no cache holds, less than the link to the GPU takes (55 GB/s); four move 100.  The copies are
@@ -81,6 +67,28 @@ class HostSignal {
     static constexpr size_t kFeed = 128;   // (words that the GPU and the host write lie in lines of their own)
     unsigned* flag_ = nullptr;
     unsigned* counter_ = nullptr;
+    unsigned value_ = 0;
+};
+
+// A block on loan for a scope.  Where launches read or write it, the scope ends the host's use of it and the last of them
+// the GPU's: the block is the pool's again when both have.
+class HostLoan {
+  public:
+    HostLoan() = default;
+    explicit HostLoan(size_t bytes, bool filled_by_host = false) : p_(HostPool::acquire(bytes, false, filled_by_host)) {}
+    HostLoan(HostLoan&& o) noexcept : p_(o.p_), signal_(o.signal_), value_(o.value_) { o.p_ = nullptr; }
+    HostLoan(const HostLoan&) = delete;
+    HostLoan& operator=(const HostLoan&) = delete;
+    ~HostLoan() {
+        if (signal_ && !signal_->reached(value_)) signal_->release_then(p_, value_);
+        else HostPool::release(p_);
+    }
+    void used_until(const HostSignal& s, unsigned value) { signal_ = &s; value_ = value; }   // by the launch that was given `value`
+    float* floats() const { return static_cast<float*>(p_); }
+
+  private:
+    void* p_ = nullptr;
+    const HostSignal* signal_ = nullptr;
     unsigned value_ = 0;
 };
 

@@ -1,0 +1,83 @@
+// The pool of page-locked host memory and the shared host copies (csrc/host_io.h) without a GPU: the two runtime calls
+// behind the pool are this program's own.  One check per call, named by the argument; exit status 0: it holds.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <set>
+
+#include "../../fyusenet_amd/csrc/host_io.h"
+
+using namespace fynhip;
+
+extern "C" hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+    *p = aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+extern "C" hipError_t hipHostFree(void* p) {
+    free(p);
+    return hipSuccess;
+}
+
+#define CHECK(x)                                              \
+    do {                                                      \
+        if (!(x)) {                                           \
+            fprintf(stderr, "line %d: %s\n", __LINE__, #x);   \
+            return 1;                                         \
+        }                                                     \
+    } while (0)
+
+static constexpr size_t kArea = 1 << 20;
+
+// A block that a launch uses is handed out again when the scope of the loan has ended and the launch has told so.
+static int loans() {
+    HostSignal signal;
+    signal.create(nullptr);
+    float* first;
+    {
+        HostLoan none(kArea);   // (no launch: back at once)
+        first = none.floats();
+    }
+    HostDone done = signal.next();
+    {
+        HostLoan area(kArea);
+        CHECK(area.floats() == first);
+        area.used_until(signal, done.value);
+        HostLoan other(kArea);
+        CHECK(other.floats() != first);
+        *done.flag = done.value;   // the launch has told, the scope has not ended
+        HostLoan third(kArea);
+        CHECK(third.floats() != first && third.floats() != other.floats());
+    }
+    done = signal.next();
+    float* held;
+    {
+        HostLoan area(kArea);
+        held = area.floats();
+        area.used_until(signal, done.value);
+    }
+    {
+        std::set<float*> seen;   // the scope has ended, the launch has not told
+        HostLoan a(kArea), b(kArea), c(kArea), d(kArea);
+        for (const HostLoan* l : {&a, &b, &c, &d}) seen.insert(l->floats());
+        CHECK(seen.size() == 4 && !seen.count(held));
+        CHECK(HostPool::contains(held, kArea));
+    }
+    *done.flag = done.value;
+    bool again = false;
+    HostLoan a(kArea), b(kArea), c(kArea), d(kArea), e(kArea);
+    for (const HostLoan* l : {&a, &b, &c, &d, &e}) again = again || l->floats() == held;
+    CHECK(again);
+    signal.destroy();
+    return 0;
+}
+
+int main(int argc, char** argv) {
+    const struct {
+        const char* name;
+        int (*run)();
+    } checks[] = {{"loans", loans}};
+    for (const auto& c : checks)
+        if (argc == 2 && !strcmp(argv[1], c.name)) return c.run();
+    fprintf(stderr, "no such check\n");
+    return 2;
+}
