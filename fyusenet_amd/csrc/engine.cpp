@@ -633,6 +633,14 @@ void Net::wait_signal(unsigned value) {
     }
 }
 
+// Behind launches that use the caller's memory or an area on loan: a failure is reported when none of them runs any more.
+void Net::check_queued() {
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return;
+    (void)hipStreamSynchronize(stream);
+    fail(FYN_ERR_DEVICE, "launch failed: %s", hipGetErrorString(e));
+}
+
 void Net::count_area(size_t bytes, size_t& most) {
     if (bytes <= most) return;
     most = bytes;
@@ -780,7 +788,7 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
     if (!host_memory(out)) {
         float* st = staging(npix * v.c);
         launch_tensor_to_chw(v, st, npix, include_padding, 0, npix, HostDone{}, stream);
-        FYN_HIP(hipGetLastError());
+        check_queued();
         FYN_HIP(hipMemcpyAsync(out, st, bytes, hipMemcpyDefault, stream));
         FYN_HIP(hipStreamSynchronize(stream));
         return;
@@ -788,17 +796,21 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
     if (HostPool::contains(out, bytes)) {
         const HostDone done = signal_.next();
         launch_tensor_to_chw(v, out, npix, include_padding, 0, npix, done, stream);
-        FYN_HIP(hipGetLastError());
+        check_queued();
         wait_signal(done.value);
         return;
     }
     const size_t plane = npix < 64 ? npix : (npix + 3) & ~size_t(3);
-    const HostLoan loan = out_area(plane * v.c);
+    HostLoan loan = out_area(plane * v.c);
     float* st = loan.floats();
     const size_t step = piece_pixels(npix, bytes);
     const unsigned first = signal_.last() + 1;
-    for (size_t p0 = 0; p0 < npix; p0 += step) launch_tensor_to_chw(v, st, plane, include_padding, p0, std::min(npix, p0 + step), signal_.next(), stream);
-    FYN_HIP(hipGetLastError());
+    for (size_t p0 = 0; p0 < npix; p0 += step) {
+        const HostDone done = signal_.next();
+        launch_tensor_to_chw(v, st, plane, include_padding, p0, std::min(npix, p0 + step), done, stream);
+        loan.used_until(signal_, done.value);
+    }
+    check_queued();
     unsigned value = first;
     for (size_t p0 = 0; p0 < npix; p0 += step) {
         const size_t p1 = std::min(npix, p0 + step);
@@ -813,12 +825,16 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
 void Net::download_pixels(const TView& v, int pc, float* out) {
     const size_t npix = (size_t)v.h * v.w, bytes = npix * pc * sizeof(float);
     const bool host = host_memory(out), direct = host && HostPool::contains(out, bytes);
-    const HostLoan loan = host && !direct ? out_area(npix * pc) : HostLoan();
+    HostLoan loan = host && !direct ? out_area(npix * pc) : HostLoan();
     float* st = direct ? out : host ? loan.floats() : staging(npix * pc);
     const size_t step = host && !direct ? piece_pixels(npix, bytes) : npix;
     const unsigned first = signal_.last() + 1;
-    for (size_t p0 = 0; p0 < npix; p0 += step) launch_tensor_to_hwc(v, st, pc, p0, std::min(npix, p0 + step), signal_.next(), stream);
-    FYN_HIP(hipGetLastError());
+    for (size_t p0 = 0; p0 < npix; p0 += step) {
+        const HostDone done = signal_.next();
+        launch_tensor_to_hwc(v, st, pc, p0, std::min(npix, p0 + step), done, stream);
+        loan.used_until(signal_, done.value);
+    }
+    check_queued();
     unsigned value = first;
     for (size_t p0 = 0; p0 < npix; p0 += step) {
         wait_signal(value++);
@@ -836,13 +852,14 @@ void Net::download_argmax(const int* idx_dev, const TView& v, int32_t* idx, floa
     if (!idx && !val) return finish();
     const bool direct = (!idx || (host_memory(idx) && HostPool::contains(idx, n * 4))) && (!val || (host_memory(val) && HostPool::contains(val, n * 4)));
     const bool host = (!idx || host_memory(idx)) && (!val || host_memory(val));
-    const HostLoan loan = host && !direct ? out_area(2 * area) : HostLoan();
+    HostLoan loan = host && !direct ? out_area(2 * area) : HostLoan();
     float* st = direct ? nullptr : host ? loan.floats() : staging(2 * area);
     int* di = !idx ? nullptr : direct ? idx : reinterpret_cast<int*>(st);
     float* dv = !val ? nullptr : direct ? val : st + area;
     const HostDone done = signal_.next();
     launch_argmax_to_host(idx_dev, v, di, dv, 0, n, done, stream);
-    FYN_HIP(hipGetLastError());
+    loan.used_until(signal_, done.value);
+    check_queued();
     wait_signal(done.value);
     if (direct) return;
     if (idx) FYN_HIP(host ? (memcpy(idx, di, n * 4), hipSuccess) : hipMemcpy(idx, di, n * 4, hipMemcpyDefault));

@@ -225,6 +225,7 @@ class Net {
     HostLoan out_area(size_t floats);
     void count_area(size_t bytes, size_t& most);   // staging areas count as allocations when they are larger than any before
     void wait_signal(unsigned value);
+    void check_queued();
     void upload(const float* data, int order, const TView& v, unsigned* amax);
     void download_planes(const TView& v, int include_padding, float* out);
     void download_pixels(const TView& v, int pc, float* out);
