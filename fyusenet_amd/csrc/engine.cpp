@@ -239,6 +239,7 @@ Net::Net(int dev, int stor) : device(dev), storage(stor) {
         // (where the runtime is told to finish a launch before the call returns, the frame is copied first)
         for (const char* e : {"HIP_LAUNCH_BLOCKING", "CUDA_LAUNCH_BLOCKING", "AMD_SERIALIZE_KERNEL"})
             if (const char* v = getenv(e)) feed_ahead_ = feed_ahead_ && (!*v || *v == '0');
+        if (const char* v = sw.get("FYNHIP_FEED_GIVE_UP")) feed_give_up_ = (unsigned)atoi(v);   // (tests)
     } catch (...) {
         release_all();
         throw;
@@ -621,16 +622,7 @@ void Net::finish() {
     const HostDone done = signal_.next();
     launch_tell_host(done, stream);
     FYN_HIP(hipGetLastError());
-    wait_signal(done.value);
-}
-
-// Everything queued on the stream ahead of the launch with this value has been carried out then.
-void Net::wait_signal(unsigned value) {
-    signal_.wait(value, stream);
-    if (__atomic_load_n(&feed_->late, __ATOMIC_RELAXED)) {
-        feed_->late = 0;
-        fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
-    }
+    signal_.wait(done.value, stream);
 }
 
 // Behind launches that use the caller's memory or an area on loan: a failure is reported when none of them runs any more.
@@ -755,12 +747,18 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         launch(HostFeed{});
         return;
     }
-    const HostFeed feed{feed_, feed_base_, (float)v.c * (float)sizeof(float) * kTicksPerByte};
+    const HostFeed feed{feed_, feed_base_, (float)v.c * (float)sizeof(float) * kTicksPerByte, feed_give_up_};
     feed_base_ += (unsigned)npix;
     launch(feed);
     for (const auto& piece : pieces) {
         copies.upto(piece.first);
         __atomic_store_n(&feed_->ready, feed.base + (unsigned)piece.second, __ATOMIC_RELEASE);
+    }
+    __atomic_thread_fence(__ATOMIC_SEQ_CST);   // (the progress has been told before the look)
+    if (__atomic_load_n(&feed_->late, __ATOMIC_RELAXED)) {   // a slow source, a stopped process: the frame is complete now
+        signal_.wait(before, stream);
+        feed_->late = 0;
+        launch(HostFeed{});
     }
 }
 
@@ -797,7 +795,7 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
         const HostDone done = signal_.next();
         launch_tensor_to_chw(v, out, npix, include_padding, 0, npix, done, stream);
         check_queued();
-        wait_signal(done.value);
+        signal_.wait(done.value, stream);
         return;
     }
     const size_t plane = npix < 64 ? npix : (npix + 3) & ~size_t(3);
@@ -814,7 +812,7 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
     unsigned value = first;
     for (size_t p0 = 0; p0 < npix; p0 += step) {
         const size_t p1 = std::min(npix, p0 + step);
-        wait_signal(value++);
+        signal_.wait(value++, stream);
         HostCopy copies;
         for (int c = 0; c < v.c; c++) copies.add(out + c * npix + p0, st + c * plane + p0, (p1 - p0) * sizeof(float));
         copies.start();
@@ -837,7 +835,7 @@ void Net::download_pixels(const TView& v, int pc, float* out) {
     check_queued();
     unsigned value = first;
     for (size_t p0 = 0; p0 < npix; p0 += step) {
-        wait_signal(value++);
+        signal_.wait(value++, stream);
         if (host && !direct) memcpy(out + p0 * pc, st + p0 * pc, (std::min(npix, p0 + step) - p0) * pc * sizeof(float));
     }
     if (!host) {
@@ -860,7 +858,7 @@ void Net::download_argmax(const int* idx_dev, const TView& v, int32_t* idx, floa
     launch_argmax_to_host(idx_dev, v, di, dv, 0, n, done, stream);
     loan.used_until(signal_, done.value);
     check_queued();
-    wait_signal(done.value);
+    signal_.wait(done.value, stream);
     if (direct) return;
     if (idx) FYN_HIP(host ? (memcpy(idx, di, n * 4), hipSuccess) : hipMemcpy(idx, di, n * 4, hipMemcpyDefault));
     if (val) FYN_HIP(host ? (memcpy(val, dv, n * 4), hipSuccess) : hipMemcpy(val, dv, n * 4, hipMemcpyDefault));
@@ -1251,7 +1249,7 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
     const float* src = s.pin_in;
     if (async_own_streams_) {
         src = s.dev_in;
-        const HostFeed feed{async_feed_, uploads_.load() * (unsigned)npix, 0.f};
+        const HostFeed feed{async_feed_, uploads_.load() * (unsigned)npix, 0.f, kFeedGiveUp};
         {
             std::lock_guard<std::mutex> lk(carry_mu_);
             uploads_++;

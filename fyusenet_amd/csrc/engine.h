@@ -221,10 +221,10 @@ class Net {
     FeedWord* feed_ = nullptr;          // progress of the host's copies into the input area
     unsigned feed_base_ = 0;            // ... when all frames so far have been copied
     bool feed_ahead_ = true;            // uploads are launched ahead of the copy
+    unsigned feed_give_up_ = kFeedGiveUp;
     unsigned* upload_words_ = nullptr;  // UploadRange::words of the network's stream
     HostLoan out_area(size_t floats);
     void count_area(size_t bytes, size_t& most);   // staging areas count as allocations when they are larger than any before
-    void wait_signal(unsigned value);
     void check_queued();
     void upload(const float* data, int order, const TView& v, unsigned* amax);
     void download_planes(const TView& v, int include_padding, float* out);

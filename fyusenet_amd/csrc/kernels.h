@@ -510,7 +510,7 @@ struct HostDone {
 };
 // How far the host has come with the frame that a launch converts.  `ready`: pixels copied, counted on from one frame to
 // the next (a launch starts at `base`, modulo 2^32); the launch reads a pixel when ready - base exceeds it.  `late`: set by
-// a launch that gave up waiting.
+// a launch that gave up waiting after `give_up` ticks: what it has converted may be stale.
 struct FeedWord {
     unsigned ready, late;
 };
@@ -518,7 +518,9 @@ struct HostFeed {
     FeedWord* word;   // page-locked; null: the frame is there
     unsigned base;
     float ticks_per_pixel;   // of the 100 MHz clock, at the rate of a fast copy
+    unsigned give_up;
 };
+constexpr unsigned kFeedGiveUp = 400000000u;   // 4 s
 // The value-range record (range.h) of an uploaded tensor, which the launch writes, and two zero words of device memory in
 // which its workgroups meet (they belong to one stream).  record null: none is kept.
 struct UploadRange {

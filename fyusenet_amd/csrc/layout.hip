@@ -30,8 +30,9 @@ unsigned upload_blocks(size_t items, bool device) { return (unsigned)std::min<si
 // The host may still be copying the frame when the launch runs (HostFeed): before a workgroup reads pixels it looks, where
 // it has to, whether they are there.  The launch's own latency (8 us) and the host's copy then overlap the transfer
 // instead of preceding it.  Every thread of the workgroup calls this with the workgroup's largest pixel; `seen` holds what
-// the last look said.  The wait ends after kFeedTicks in any case, and the host is told (FeedWord::late).
-constexpr unsigned long long kFeedTicks = 400000000ull;   // 4 s of the 100 MHz clock
+// the last look said.  The wait ends after HostFeed::give_up ticks in any case, and the host is told (FeedWord::late): it
+// looks at that word when the frame is complete and has the frame converted again.  It cannot miss it: the word is set
+// before the last look at the progress, and looked at behind the last progress.
 __device__ __forceinline__ void await_feed(const HostFeed& f, unsigned need, unsigned& seen) {
     if (!f.word || seen >= need) return;   // (the same for all threads)
     __shared__ unsigned box;
@@ -39,16 +40,18 @@ __device__ __forceinline__ void await_feed(const HostFeed& f, unsigned need, uns
         const unsigned long long t0 = wall_clock64();
         unsigned r;
         while ((int)((r = __hip_atomic_load(&f.word->ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) - f.base) - need) < 0) {
+            if (wall_clock64() - t0 >= f.give_up) {
+                __hip_atomic_store(&f.word->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (also before the workgroup counts as arrived, below)
+                __threadfence_system();
+                r = __hip_atomic_load(&f.word->ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) - f.base;
+                if ((int)(r - need) < 0) r = 0x7fffffffu;
+                break;
+            }
             // (not before the host can have come so far: a look takes the word's line from the core that is copying, and
             // the link from the copy; 1.3 us at least)
             const unsigned long long t1 = wall_clock64(), ticks = min(10000u, 130u + (unsigned)((float)(need - r) * f.ticks_per_pixel));
             while (wall_clock64() - t1 < ticks) __builtin_amdgcn_s_sleep(8);
-            if (wall_clock64() - t0 > kFeedTicks) {
-                __hip_atomic_store(&f.word->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (before the workgroup counts as arrived, below)
-                r = 0x7fffffffu;
-                break;
-            }
         }
         box = r;
     }

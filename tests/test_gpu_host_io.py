@@ -103,6 +103,43 @@ def test_results_belong_to_the_caller():
         assert (k == value).all()
 
 
+@pytest.mark.gpu
+@STORAGES
+@pytest.mark.parametrize("order", [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW], ids=["chw", "hwc"])
+@pytest.mark.parametrize("c,h,w", [(3, 5, 7), (3, 701, 433), (4, 1080, 1920)])
+def test_a_frame_that_is_late_is_converted_again(monkeypatch, c, h, w, order, storage):
+    """Launches that give up at the first pixel that is not there yet (FYNHIP_FEED_GIVE_UP, ticks; 4 s as a rule): the frame
+    arrives all the same, every time."""
+    monkeypatch.setenv("FYNHIP_FEED_GIVE_UP", "0")
+    net = _copy_net(c, h, w, storage, 1)
+    for i in range(6):
+        x = prng.uniform(900 + i, (c, h, w), -2.0, 2.0)
+        net.layers[1].setInput(x if order == fa.ORDER_CHANNELWISE else np.ascontiguousarray(x.transpose(1, 2, 0)), 0, order)
+        net.forward()
+        assert np.array_equal(net.getOutput(1), x if storage == fa.STORAGE_F32 else x.astype(np.float16).astype(np.float32)), i
+    net.cleanup()
+
+
+@pytest.mark.gpu
+def test_a_late_frame_leaves_its_own_value_range(monkeypatch):
+    """The value range that the first convolution scales by is the frame's, not that of what lay in the area before."""
+    frames = [prng.uniform(40 + i, (3, 500, 660), 0.0, top) for i, top in enumerate((1.0, 1000.0, 1e-3, 1.0))]
+    results = []
+    for give_up in (None, "0"):
+        if give_up is not None:
+            monkeypatch.setenv("FYNHIP_FEED_GIVE_UP", give_up)
+        net = samples.StyleNetSample(3, 660, 500)
+        net.setup()
+        got = []
+        for f in frames:
+            net.layers[net.UPLOAD].setInput(f, 0)
+            net.forward()
+            got.append(np.array(net.getOutput(net.output_layer)))
+        net.cleanup()
+        results.append(got)
+    for i, (a, b) in enumerate(zip(*results)):
+        assert np.array_equal(a, b), i
+
 
 def test_results_without_any_network_lie_in_ordinary_memory():
     capi.check(capi.lib().fyn_host_release(None))
