@@ -46,22 +46,40 @@ size_t size_class(size_t bytes) {   // sizes in steps of an eighth of the next p
     while (step * 16 <= bytes) step *= 2;
     return (bytes + step - 1) / step * step;
 }
-void give_back_idle() {   // (the lock is held)
-    for (auto it = g_blocks.begin(); it != g_blocks.end();) {
-        if (!idle(it->second)) {
-            ++it;
-            continue;
+// The pool's lock.  The runtime is not called under it: locking and releasing memory may wait for the GPU, and what the
+// GPU waits for (a frame that another thread is copying) may need the lock.
+class PoolLock {
+  public:
+    PoolLock() { g_pool_mu.lock(); }
+    ~PoolLock() { unlock(); }
+    PoolLock(const PoolLock&) = delete;
+    PoolLock& operator=(const PoolLock&) = delete;
+    void give_back_idle() {   // (when the lock is left)
+        for (auto it = g_blocks.begin(); it != g_blocks.end();) {
+            if (!idle(it->second)) {
+                ++it;
+                continue;
+            }
+            g_pool_bytes -= it->second.bytes;
+            freed_.push_back(it->first);
+            it = g_blocks.erase(it);
         }
-        g_pool_bytes -= it->second.bytes;
-        (void)hipHostFree(it->first);
-        it = g_blocks.erase(it);
     }
-}
+    void lock() { g_pool_mu.lock(); }
+    void unlock() {
+        g_pool_mu.unlock();
+        for (char* p : freed_) (void)hipHostFree(p);
+        freed_.clear();
+    }
+
+  private:
+    std::vector<char*> freed_;
+};
 }  // namespace
 
 void* HostPool::acquire(size_t bytes, bool bounded, bool filled_by_host) {
     const size_t want = size_class(bytes ? bytes : 1);
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    PoolLock lk;
     // (a block that served the same purpose before: the host's copy into one that the host has written lately finds its
     // lines in the caches -- 3.8 MB in 60 us, against 90 into one that the GPU has written)
     std::pair<char* const, Block>* pick = nullptr;
@@ -74,32 +92,35 @@ void* HostPool::acquire(size_t bytes, bool bounded, bool filled_by_host) {
     }
     if (bounded && g_networks == 0) return nullptr;
     if (g_pool_bytes + want > kBytes) {
-        give_back_idle();
+        lk.give_back_idle();
         if (bounded && g_pool_bytes + want > kBytes) return nullptr;
     }
+    g_pool_bytes += want;   // (taken before the lock is left)
+    lk.unlock();
     void* p = nullptr;
     const hipError_t e = hipHostMalloc(&p, want, hipHostMallocPortable);
+    lk.lock();
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        g_pool_bytes -= want;
         if (bounded) return nullptr;
         fail(FYN_ERR_DEVICE, "no page-locked memory (%zu bytes): %s", want, hipGetErrorString(e));
     }
     g_blocks[static_cast<char*>(p)] = Block{want, true, nullptr, 0, filled_by_host};
-    g_pool_bytes += want;
     return p;
 }
 
 void HostPool::release(void* p) {
     if (!p) return;
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    PoolLock lk;
     auto it = g_blocks.find(static_cast<char*>(p));
     if (it == g_blocks.end() || !it->second.lent) return;
     it->second.lent = false;
-    if (g_networks == 0 || g_pool_bytes > kBytes) give_back_idle();
+    if (g_networks == 0 || g_pool_bytes > kBytes) lk.give_back_idle();
 }
 
 void HostPool::release_then(void* p, const unsigned* flag, unsigned value) {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    PoolLock lk;
     auto it = g_blocks.find(static_cast<char*>(p));
     if (it == g_blocks.end()) return;
     it->second.flag = flag;
@@ -107,7 +128,7 @@ void HostPool::release_then(void* p, const unsigned* flag, unsigned value) {
 }
 
 void HostPool::forget(const unsigned* flag) {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    PoolLock lk;
     for (auto& kv : g_blocks)
         if (kv.second.flag == flag) {
             kv.second.flag = nullptr;
@@ -116,7 +137,7 @@ void HostPool::forget(const unsigned* flag) {
 }
 
 bool HostPool::contains(const void* p, size_t bytes) {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    PoolLock lk;
     char* c = const_cast<char*>(static_cast<const char*>(p));
     auto it = g_blocks.upper_bound(c);
     if (it == g_blocks.begin()) return false;
@@ -125,12 +146,12 @@ bool HostPool::contains(const void* p, size_t bytes) {
 }
 
 void HostPool::network_created() {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
+    PoolLock lk;
     g_networks++;
 }
 void HostPool::network_gone() {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    if (--g_networks == 0) give_back_idle();
+    PoolLock lk;
+    if (--g_networks == 0) lk.give_back_idle();
 }
 
 void HostSignal::create(unsigned* counter) {

@@ -1,19 +1,27 @@
 // The pool of page-locked host memory and the shared host copies (csrc/host_io.h) without a GPU: the two runtime calls
 // behind the pool are this program's own.  One check per call, named by the argument; exit status 0: it holds.
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <set>
+#include <thread>
 
 #include "../../fyusenet_amd/csrc/host_io.h"
 
 using namespace fynhip;
 
+// Called in the place where the runtime may wait for the GPU.
+static void (*g_runtime_waits)() = [] {};
+
 extern "C" hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+    g_runtime_waits();
     *p = aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 extern "C" hipError_t hipHostFree(void* p) {
+    g_runtime_waits();
     free(p);
     return hipSuccess;
 }
@@ -71,11 +79,48 @@ static int loans() {
     return 0;
 }
 
+// A thread inside one of the runtime's two calls, which may have to wait for the GPU, does not keep another one from
+// the pool: what the GPU waits for may be that thread.
+static std::atomic<int> g_inside{0}, g_other{0}, g_stuck{0};
+static int runtime_calls_outside_the_lock() {
+    HostPool::network_created();
+    void* const idle = HostPool::acquire(kArea, false);
+    void* const mine = HostPool::acquire(2 * kArea, false);
+    HostPool::release(idle);
+    g_runtime_waits = [] {
+        g_inside++;
+        const auto t0 = std::chrono::steady_clock::now();
+        while (g_other.load() < g_inside.load())
+            if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(5)) {
+                g_stuck++;
+                return;
+            }
+    };
+    std::thread other([&] {
+        for (int call = 1; call <= 2; call++) {
+            while (g_inside.load() < call) {
+            }
+            (void)HostPool::contains(mine, kArea);
+            g_other = call;
+        }
+    });
+    void* const fresh = HostPool::acquire(4 * kArea, false);   // locks memory
+    HostPool::network_gone();                                  // releases the idle block
+    other.join();
+    CHECK(g_inside.load() == 2 && g_stuck.load() == 0);
+    g_runtime_waits = [] {};
+    CHECK(HostPool::contains(mine, 2 * kArea) && HostPool::contains(fresh, 4 * kArea) && !HostPool::contains(idle, kArea));
+    HostPool::release(mine);
+    HostPool::release(fresh);
+    CHECK(!HostPool::contains(mine, 1) && !HostPool::contains(fresh, 1));
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const struct {
         const char* name;
         int (*run)();
-    } checks[] = {{"loans", loans}};
+    } checks[] = {{"loans", loans}, {"runtime_calls_outside_the_lock", runtime_calls_outside_the_lock}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) return c.run();
     fprintf(stderr, "no such check\n");
