@@ -211,15 +211,16 @@ struct HostCopyHelpers {
     std::mutex mu;
     std::condition_variable cv;
     std::deque<std::shared_ptr<HostCopy::Job>> jobs;
+    const unsigned count = std::min(3u, std::thread::hardware_concurrency() / 4);
     HostCopyHelpers() {
-        const unsigned cpus = std::thread::hardware_concurrency();
-        for (unsigned i = 0; i < std::min(3u, cpus / 4); i++) std::thread([this] { work(); }).detach();
+        for (unsigned i = 0; i < count; i++) std::thread([this] { work(); }).detach();
     }
     static HostCopyHelpers& get() {
         static HostCopyHelpers* h = new HostCopyHelpers;
         return *h;
     }
     void offer(const std::shared_ptr<HostCopy::Job>& job) {
+        if (!count) return;   // (few CPUs: nobody would take it from the queue)
         {
             std::lock_guard<std::mutex> lk(mu);
             jobs.push_back(job);

@@ -1,5 +1,8 @@
 // The pool of page-locked host memory and the shared host copies (csrc/host_io.h) without a GPU: the two runtime calls
-// behind the pool are this program's own.  One check per call, named by the argument; exit status 0: it holds.
+// behind the pool and the number of CPUs are this program's own.  One check per call, named by the argument; exit status 0: it holds.
+#include <malloc.h>
+#include <sys/sysinfo.h>
+
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -25,6 +28,10 @@ extern "C" hipError_t hipHostFree(void* p) {
     free(p);
     return hipSuccess;
 }
+
+// What std::thread::hardware_concurrency asks.
+static int g_cpus = 8;
+extern "C" int get_nprocs() noexcept { return g_cpus; }
 
 #define CHECK(x)                                              \
     do {                                                      \
@@ -116,11 +123,34 @@ static int runtime_calls_outside_the_lock() {
     return 0;
 }
 
+// Copies on offer to helpers where the process has too few CPUs for any: they are made, and nothing is kept of them.
+static int copies_without_helpers() {
+    g_cpus = 3;
+    CHECK(std::thread::hardware_concurrency() == 3);
+    const int n = 20000;
+    char from[256], to[256];
+    for (size_t i = 0; i < sizeof(from); i++) from[i] = (char)(7 * i);
+    auto in_use = [] { return mallinfo2().uordblks; };
+    const size_t before = in_use();
+    for (int i = 0; i < n; i++) {
+        memset(to, 0, sizeof(to));
+        {
+            HostCopy copies;
+            copies.add(to, from, sizeof(to));
+            copies.start(0);   // (shared from no bytes on)
+        }
+        CHECK(!memcmp(to, from, sizeof(to)));
+    }
+    CHECK(in_use() < before + (64u << 10));
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const struct {
         const char* name;
         int (*run)();
-    } checks[] = {{"loans", loans}, {"runtime_calls_outside_the_lock", runtime_calls_outside_the_lock}};
+    } checks[] = {{"loans", loans}, {"runtime_calls_outside_the_lock", runtime_calls_outside_the_lock},
+                  {"copies_without_helpers", copies_without_helpers}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) return c.run();
     fprintf(stderr, "no such check\n");

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["loans", "runtime_calls_outside_the_lock"])
+@pytest.mark.parametrize("check", ["loans", "runtime_calls_outside_the_lock", "copies_without_helpers"])
 def test_host_io(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
