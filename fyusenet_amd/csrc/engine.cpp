@@ -710,8 +710,10 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
     const size_t bytes = plane * v.c * sizeof(float);
     unsigned& before = uploads_told_[upload_no_++ % kUploads];
     if (before) signal_.wait(before, stream);
+    size_t under_way = 0;   // (areas of earlier frames that their launches still read)
+    for (unsigned told : uploads_told_) under_way += told && !signal_.reached(told);
     HostLoan area(bytes, true);
-    count_area(bytes, in_most_);
+    count_area(bytes, in_most_[under_way]);
     float* st = area.floats();
     // pieces: a small one first, so that the launch has something to do when it starts; multiples of 32 pixels (whole lines)
     HostCopy copies;   // (made before the loan ends, whatever happens)
@@ -1052,7 +1054,7 @@ static constexpr size_t kRowGap = 256;   // bytes between the rows of an overlap
 void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, int out_order, int depth, bool copy_streams) {
     if (!is_setup) fail(FYN_ERR_STATE, "async_begin() before setup()");
     if (!slots_.empty()) fail(FYN_ERR_STATE, "frame pipeline is already active");
-    if (depth < 1 || depth > 8) fail(FYN_ERR_INVALID, "pipeline depth %d out of range (1..8)", depth);
+    if (depth < 1 || depth > kMaxDepth) fail(FYN_ERR_INVALID, "pipeline depth %d out of range (1..%d)", depth, kMaxDepth);
     FYN_HIP(hipSetDevice(device));
     Layer* li = layer(in_layer);
     if (li->d.type == FYN_LAYER_UPLOAD) {
@@ -1090,12 +1092,18 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
         async_rows_ = (out_bytes + async_row_ - 1) / async_row_;
     }
     slots_ = std::vector<AsyncSlot>(depth + 1);
-    for (AsyncSlot& s : slots_) {
+    const size_t pin_out_bytes = async_own_streams_ ? async_rows_ * (async_row_ + kRowGap) : out_bytes;
+    for (size_t i = 0; i < slots_.size(); i++) {
+        AsyncSlot& s = slots_[i];
         s.pin_in = static_cast<float*>(HostPool::acquire(in_bytes, false, true));
-        s.pin_out = static_cast<float*>(HostPool::acquire(async_own_streams_ ? async_rows_ * (async_row_ + kRowGap) : out_bytes, false));
+        s.pin_out = static_cast<float*>(HostPool::acquire(pin_out_bytes, false));
+        count_area(in_bytes, slot_in_most_[i]);
+        count_area(pin_out_bytes, slot_out_most_[i]);
         if (!async_own_streams_) continue;
         FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_in), in_bytes));
         FYN_HIP(hipMalloc(reinterpret_cast<void**>(&s.dev_out), async_rows_ * async_row_));
+        alloc_calls_ += 2;
+        alloc_bytes_ += in_bytes + async_rows_ * async_row_;
     }
     if (async_own_streams_) {
         carry_end_ = false;

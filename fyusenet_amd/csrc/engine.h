@@ -209,13 +209,16 @@ class Net {
     void dump_layer(Layer* l);
     std::vector<void*> allocs_;
   public:
-    // device allocations made for this network since it was created (calls of hipMalloc, bytes asked for)
+    // allocations made for this network since it was created: calls of hipMalloc, and page-locked areas in use beyond
+    // what was in use at once before (the pool may have had them); bytes asked for
     size_t alloc_calls_ = 0, alloc_bytes_ = 0;
   private:
     float* staging_ = nullptr;
     size_t staging_floats_ = 0;
-    size_t in_most_ = 0, out_most_ = 0;   // largest page-locked areas of the synchronous calls so far
     static constexpr unsigned kUploads = 4;   // areas of uploads that may be waiting for their launch
+    static constexpr int kMaxDepth = 8;       // of a frame pipeline
+    // largest page-locked areas so far: of an upload with so many others under way, of a read-back, of a pipeline's slots
+    size_t in_most_[kUploads] = {}, out_most_ = 0, slot_in_most_[kMaxDepth + 1] = {}, slot_out_most_[kMaxDepth + 1] = {};
     unsigned uploads_told_[kUploads] = {}, upload_no_ = 0;
     HostSignal signal_;
     FeedWord* feed_ = nullptr;          // progress of the host's copies into the input area
@@ -224,7 +227,7 @@ class Net {
     unsigned feed_give_up_ = kFeedGiveUp;
     unsigned* upload_words_ = nullptr;  // UploadRange::words of the network's stream
     HostLoan out_area(size_t floats);
-    void count_area(size_t bytes, size_t& most);   // staging areas count as allocations when they are larger than any before
+    void count_area(size_t bytes, size_t& most);   // an area counts as an allocation when it is larger than any before in its place
     void check_queued();
     void upload(const float* data, int order, const TView& v, unsigned* amax);
     void download_planes(const TView& v, int include_padding, float* out);

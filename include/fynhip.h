@@ -291,9 +291,12 @@ int fyn_net_async_end(fyn_net* net);
  * the next caller and go back to the system with the last network.  No counterpart in the reference. */
 int fyn_host_acquire(size_t bytes, void** ptr);
 int fyn_host_release(void* ptr);
-/* Device allocations this network has made since fyn_net_create: number of hipMalloc calls (and of page-locked staging
- * areas taken) and the bytes asked for (both only ever grow).  A diagnostic without a counterpart in the reference, whose textures belong to the GL driver;
- * it lets a caller check that a call sequence of its serving loop allocates nothing. */
+/* Allocations this network has made since fyn_net_create: calls of hipMalloc, plus the page-locked areas it has in use
+ * beyond what it ever had in use at once (frames on their way in: up to four; a result on its way out; the slots of a
+ * frame pipeline), whether they had to be locked anew or another network had left them; and the bytes asked for.  Both
+ * only ever grow.  A diagnostic without a counterpart in the reference, whose textures belong to the GL driver; it lets a
+ * caller check that a call sequence of its serving loop allocates nothing.  Memory taken with fyn_host_acquire is the
+ * caller's and does not count. */
 int fyn_net_device_allocations(fyn_net* net, size_t* calls, size_t* bytes);
 /* Text description of the kernel variant chosen for a layer (for profiles / reports). */
 int fyn_layer_kernel_info(fyn_net* net, int layer, char* buf, size_t buflen);

@@ -1,6 +1,8 @@
 """Host frames and results at the edges of the layout kernels and of the transfers' pieces (fyusenet/gpu/uploadlayer.cpp:92-186,
 gpulayerbase.cpp:525-564): a copy layer hands back what was put in, through every host layout, into memory of the
 library's and of the caller's own."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -139,6 +141,46 @@ def test_a_late_frame_leaves_its_own_value_range(monkeypatch):
         results.append(got)
     for i, (a, b) in enumerate(zip(*results)):
         assert np.array_equal(a, b), i
+
+def _allocations(net):
+    calls, nbytes = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    capi.check(capi.lib().fyn_net_device_allocations(net._h, ctypes.byref(calls), ctypes.byref(nbytes)))
+    return calls.value, nbytes.value
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,height,device_slots", [(64, 48, 0), (660, 500, 2)])
+def test_allocations_count_every_area_in_use(width, height, device_slots):
+    """The slots of a pipeline count when it is made, its frames do not; frames handed over one behind the other without
+    waiting count up to four areas, frames one after the other a single one."""
+    net = samples.StyleNetSample(3, width, height)
+    net.setup()
+    frame = prng.uniform(1, (3, height, width), 0.0, 1.0)
+    result = np.empty((3, height, width), np.float32)
+    begin = _allocations(net)
+    for _ in range(5):
+        net.layers[net.UPLOAD].setInput(frame, 0)
+        net.forward()
+        capi.check(capi.lib().fyn_net_get_output(net._h, net.output_layer, capi.fptr(result), fa.ORDER_CHANNELWISE))
+    one = _allocations(net)
+    assert one[0] - begin[0] == 2 and one[1] - begin[1] >= 2 * frame.nbytes   # (a frame in, a result out)
+    for _ in range(12):
+        net.layers[net.UPLOAD].setInput(frame, 0)
+    net.finish()
+    four = _allocations(net)
+    assert four[0] - one[0] <= 3
+    for again in range(2):
+        before = _allocations(net)
+        net.asyncBegin(net.UPLOAD, net.output_layer, depth=2)
+        made = _allocations(net)
+        assert made[0] - before[0] == 3 * ((0 if again else 2) + device_slots), again
+        assert again or made[1] - before[1] >= 3 * 2 * frame.nbytes
+        for _ in range(7):
+            ticket = net.asyncSubmit(frame, result)
+        net.asyncWait(ticket)
+        assert _allocations(net) == made
+        net.asyncEnd()
+    net.cleanup()
 
 
 def test_results_without_any_network_lie_in_ordinary_memory():
