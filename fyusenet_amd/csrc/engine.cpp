@@ -694,9 +694,10 @@ static constexpr float kTicksPerByte = 1.f / 800.f;   // 80 GB/s, 10 ns a tick
 // two copies with a launch behind each.
 void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
     const size_t npix = (size_t)v.h * v.w, plane = (npix + 31) & ~size_t(31);
-    const bool host = host_memory(data), planes = order == FYN_ORDER_CHANNELWISE;
+    const bool planes = order == FYN_ORDER_CHANNELWISE;
+    const Memory kind = memory_of(data);
     const UploadRange range{amax, upload_words_};
-    if (!host) {
+    if (kind == Memory::Device) {
         float* st = staging(plane * v.c);
         for (int c = 0; c < (planes ? v.c : 1); c++)
             FYN_HIP(hipMemcpyAsync(st + c * plane, data + c * npix, npix * (planes ? 1 : v.c) * sizeof(float), hipMemcpyDefault, stream));
@@ -705,6 +706,14 @@ void Net::upload(const float* data, int order, const TView& v, unsigned* amax) {
         FYN_HIP(hipGetLastError());
         FYN_HIP(hipStreamSynchronize(stream));   // the caller's buffer is borrowed for this call only
         return;
+    }
+    // Page-locked memory may be the target of the application's work on the default stream, which the network's stream runs
+    // behind: the host reads when that has ended.  (The pool's blocks hold results that have been waited for.)
+    if (kind == Memory::PageLocked && !HostPool::contains(data, npix * v.c * sizeof(float))) {
+        const HostDone done = signal_.next();
+        launch_tell_host(done, stream);
+        check_queued();
+        signal_.wait(done.value, stream);
     }
     // (a caller that never waits is held at a few frames)
     const size_t bytes = plane * v.c * sizeof(float);

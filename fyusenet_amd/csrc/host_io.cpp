@@ -268,13 +268,14 @@ void HostCopy::upto(size_t mark) {
     }
 }
 
-bool host_memory(const void* p) {
+Memory memory_of(const void* p) {
     hipPointerAttribute_t a{};
-    if (hipPointerGetAttributes(&a, p) != hipSuccess) {   // memory that HIP knows nothing of
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
-        return true;
+        return Memory::Pageable;
     }
-    return a.type != hipMemoryTypeDevice;
+    if (a.type == hipMemoryTypeDevice) return Memory::Device;
+    return a.type == hipMemoryTypeUnregistered ? Memory::Pageable : Memory::PageLocked;
 }
 
 }  // namespace fynhip

@@ -92,7 +92,10 @@ class HostLoan {
     unsigned value_ = 0;
 };
 
-// Whether the host can read and write the memory itself (false: device memory).
-bool host_memory(const void* p);
+// What HIP knows of a buffer of the caller's: memory of the host's that it knows nothing of, page-locked or managed memory
+// (which work on a stream may be using), device memory.
+enum class Memory { Pageable, PageLocked, Device };
+Memory memory_of(const void* p);
+inline bool host_memory(const void* p) { return memory_of(p) != Memory::Device; }   // the host can read and write it itself
 
 }  // namespace fynhip

@@ -141,6 +141,40 @@ def test_a_late_frame_leaves_its_own_value_range(monkeypatch):
         results.append(got)
     for i, (a, b) in enumerate(zip(*results)):
         assert np.array_equal(a, b), i
+@pytest.mark.gpu
+@pytest.mark.parametrize("order", [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW], ids=["chw", "hwc"])
+def test_page_locked_input_is_read_behind_the_default_stream(order):
+    """A frame that the application's default stream is still writing into page-locked memory when it is handed over."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def call(name, *args):
+        assert getattr(hip, name)(*args) == 0, name
+
+    c, h, w = 3, 301, 500
+    net = _copy_net(c, h, w, fa.STORAGE_F32)
+    shape = (c, h, w) if order == fa.ORDER_CHANNELWISE else (h, w, c)
+    nbytes, large = 4 * c * h * w, 1 << 30
+    pinned, frame, a, b = (ctypes.c_void_p() for _ in range(4))
+    call("hipHostMalloc", ctypes.byref(pinned), ctypes.c_size_t(nbytes), ctypes.c_uint(0))
+    for p, n in ((frame, nbytes), (a, large), (b, large)):
+        call("hipMalloc", ctypes.byref(p), ctypes.c_size_t(n))
+    view = np.ctypeslib.as_array((ctypes.c_float * (c * h * w)).from_address(pinned.value)).reshape(shape)
+    view[:] = 0
+    for i in range(3):
+        x = np.ascontiguousarray(prng.uniform(60 + i, shape, -2.0, 2.0))
+        call("hipMemcpy", frame, x.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(nbytes), ctypes.c_int(1))
+        for _ in range(16):     # (milliseconds of work in front of the copy)
+            call("hipMemcpyAsync", b, a, ctypes.c_size_t(large), ctypes.c_int(3), None)
+        call("hipMemcpyAsync", pinned, frame, ctypes.c_size_t(nbytes), ctypes.c_int(2), None)
+        net.layers[1].setInput(view, 0, order)
+        net.forward()
+        got = net.getOutput(1)
+        assert np.array_equal(got, x if order == fa.ORDER_CHANNELWISE else x.transpose(2, 0, 1)), i
+    net.cleanup()
+    for p in (frame, a, b):
+        call("hipFree", p)
+    call("hipHostFree", pinned)
+
 
 def _allocations(net):
     calls, nbytes = ctypes.c_size_t(0), ctypes.c_size_t(0)
