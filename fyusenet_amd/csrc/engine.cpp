@@ -233,8 +233,9 @@ Net::Net(int dev, int stor) : device(dev), storage(stor) {
     try {
         // resolved here, where the caller may still allocate: looking the symbol up loads the code object on this device
         static_scratch_ = static_scratch(dev);
-        signal_.create(static_cast<unsigned*>(dev_alloc(64)));
-        upload_words_ = static_cast<unsigned*>(dev_alloc(64));
+        unsigned* const words = static_cast<unsigned*>(dev_alloc(256));
+        signal_.create(words);
+        upload_words_ = words + 32;   // (a line of their own)
         feed_ = signal_.feed();
         // (where the runtime is told to finish a launch before the call returns, the frame is copied first)
         for (const char* e : {"HIP_LAUNCH_BLOCKING", "CUDA_LAUNCH_BLOCKING", "AMD_SERIALIZE_KERNEL"})

@@ -647,13 +647,15 @@ class ConvLayer : public Layer {
         q.acc_mul = 1.f;
         q.act = act();
         q.in_amax = tin(0).amax;
-        void* const wp = net->dev_alloc((size_t)q.mfrags * q.cin_chunks * (q.f16 ? 1 : 2) * 1024, true);
-        q.wpack = wp;
         const char* at = net->sw.get("FYNHIP_AUTOTUNE");
         bool pick = net->sw.get("FYNHIP_FORCE_S16_CONV") != nullptr;
         char key[160];
         snprintf(key, sizeof(key), "s16:%dx%d:%dx%d:s%d:cp%d:r%d:h%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, q.f16);
-        if (!pick && !tune_cache_flag(net, key, &pick) && !(at && at[0] == '0')) {
+        const bool timed = !pick && !tune_cache_flag(net, key, &pick) && !(at && at[0] == '0');
+        if (!pick && !timed) return;
+        void* const wp = net->dev_alloc((size_t)q.mfrags * q.cin_chunks * (q.f16 ? 1 : 2) * 1024, true);
+        q.wpack = wp;
+        if (timed) {
             float t_new = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
                 t_new = std::min(t_new, time_calls(net, [&]() {
@@ -723,21 +725,32 @@ class ConvLayer : public Layer {
             cands.push_back(c);
         }
         if (cands.empty()) return;
-        const size_t halves = (size_t)frags * q.cin_chunks * (q.f16 ? 1 : 2) * 64 * 8;
-        void* const wp = net->dev_alloc(halves * 2, true);
-        for (ConvP16Params& c : cands) c.wpack = wp;
-        const bool always = net->sw.get("FYNHIP_FORCE_G16_CONV") != nullptr;
+        const bool always = want || net->sw.get("FYNHIP_FORCE_G16_CONV") != nullptr;
+        // Timed where it can win.  Measured against what had been chosen before, 13 pairs of channels on 20x20 to 960x540
+        // positions, both storages: never ahead below 128x128 positions (0.3 to 0.97 of the other form's speed) nor beside
+        // the K-resident form (0.3 to 0.75), nor with more than 40 channels on either side (0.15 to 0.83; 0.97 on one of
+        // 95 us); ahead by up to 1.26x elsewhere.
+        if (!always && (kr16 || oh * ow < 16384 || in_v.cp > 40 || oc > 40)) return;
         const char* at = net->sw.get("FYNHIP_AUTOTUNE");
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "g16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
         int cached[3] = {0, 0, 0};
-        if (want || always) {
+        bool timed = false;
+        if (always) {
         } else if (tune_cache_triple(net, key, cached)) {
             pick = -1;
             for (size_t i = 0; cached[0] && i < cands.size(); i++)
                 if (cands[i].wm == cached[1]) pick = (int)i;
-        } else if (!(at && at[0] == '0')) {
+        } else {
+            timed = !(at && at[0] == '0');
+            if (!timed) pick = -1;
+        }
+        if (pick < 0) return;
+        const size_t halves = (size_t)frags * q.cin_chunks * (q.f16 ? 1 : 2) * 64 * 8;
+        void* const wp = net->dev_alloc(halves * 2, true);
+        for (ConvP16Params& c : cands) c.wpack = wp;
+        if (timed) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
                 for (size_t i = 0; i < cands.size(); i++) {
@@ -753,8 +766,6 @@ class ConvLayer : public Layer {
                         cands[pick].wm, cands[pick].pos_groups * cands[pick].cout_blocks, best * 1e3f, own_info().c_str(), t_other * 1e3f);
             tune_cache_store_triple(net, key, best < t_other ? 1 : 0, cands[pick].wm, 0);
             if (best >= t_other) pick = -1;
-        } else {
-            pick = -1;
         }
         if (pick >= 0) {
             if (p16) net->dev_free(p16_wpack_dev);
