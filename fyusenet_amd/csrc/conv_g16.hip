@@ -1,17 +1,21 @@
 // 3x3 convolutions between tensors of few channels (16 to 64 in, up to 64 out), any stride, edge rule and source step:
-// the layers of the small style nets (12 / 20 / 40 channels) and layers like them (reference:
+// layers at image size like those of small style nets and decoders (reference:
 // gpu/vanilla/convlayerNxN_vanilla.cpp, gpu/vanilla/fractionalconvlayerNxN_vanilla.cpp, gpu/deep/deepconvlayerNxN.cpp:129-211).
 //
 // The forms that stage pixels in LDS (conv_p16.hip) work on chunks of 32 input channels and blocks of 64 output
-// channels: 12 -> 20 channels fill a seventh of that, 40 -> 40 two fifths, and a launch pays some 5 us of staging,
-// barriers and start-up whatever its size.  Here a step of the matrix instruction (v_mfma_f32_16x16x32_f16, 16 positions
+// channels: 12 -> 20 channels fill a seventh of that, 40 -> 40 two fifths.  Here a step of the matrix instruction
+// (v_mfma_f32_16x16x32_f16, 16 positions
 // x 32 values of the reduction) is four groups of eight channels wherever they lie: the window's 9 * G groups (G = groups
 // per pixel) are numbered tap by tap, lane group kq of step s takes group 4s + kq straight from the tensor, and only the
 // last step is padded (40 channels: 12 steps instead of 18, 16 channels: 5 instead of 9).  The window's nine-fold
 // overlap is left to the L1.  A wave owns 16 positions at a time and all its fragments of output channels; the weights
 // lie in LDS, staged once per workgroup; the registers a step has emptied take the next tile's values at once, so a
 // whole tile of loads is always in flight and no barrier stands in the loop.  Workgroups walk bands of positions per XCD.
-// Bound: the tensors' own traffic on large layers, memory latency on small ones.
+// Bound: the L1's rate at the nine-fold window on large layers, memory latency on small ones.  24 -> 12 channels at step
+// 1/4, 312x256 positions, fp32 tensors: 11.4 us where the general forms take 14.4 (7.4 MB: 0.6 TB/s, matrix pipes 7 %
+// busy).  960x540 positions, fp16: 16 -> 16 channels 18.2 us against 22.2, 24 -> 24 25.3 against 27.8.  Behind from 40
+// channels on (each output fragment's waves fetch the window again where registers do not hold all fragments): 64 -> 64 at
+// 256x256, fp32, 79.8 us against 11.8.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

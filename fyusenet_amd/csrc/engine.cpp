@@ -688,7 +688,10 @@ static size_t piece_pixels(size_t npix, size_t bytes) {
     return std::max<size_t>(4, ((npix + pieces - 1) / pieces + 3) & ~size_t(3));
 }
 
-static constexpr float kTicksPerByte = 1.f / 800.f;   // 80 GB/s, 10 ns a tick
+// How soon a workgroup looks again for pixels that are not there: not before a copy at 80 GB/s (10 ns a tick; four cores of
+// the host this was measured on reach 100) could have brought them.  Behind a slower copy it looks again after the time
+// that the rest would take at that rate, so the rate decides how many looks there are and not how long a frame takes.
+static constexpr float kTicksPerByte = 1.f / 800.f;
 
 // A frame into its tensor.  Host memory: the converting launch is queued first and takes the pixels as the host puts them
 // into page-locked memory (HostFeed), so that launch latency, copy and transfer overlap: 3.8 MB in 90 us instead of 135 for

@@ -23,7 +23,8 @@ constexpr unsigned kMaxDeviceBlocks = 1024;   // buffers in device memory: 3.8 M
 // Frames from the host: the workgroups keep pace with the host's copy, and each one's looks at its progress (HostFeed) and
 // its arrival at the end cost the others time.  A segmentation frame (3.7 MB) from call to launch complete, with 24, 32,
 // 40, 48, 64 and 80 workgroups: 106, 98, 92, 93, 96, 97 us (111 with 128 that ended with a fence each); 25 MB: 566, 492,
-// 489, 490, 497, 534.
+// 489, 490, 497, 534.  (Two sizes, one host with a 55 GB/s link: elsewhere the number is a guess; what depends on it is how
+// close to the link's rate an upload runs, not what arrives.)
 constexpr unsigned kMaxUploadBlocks = 48;
 unsigned upload_blocks(size_t items, bool device) { return (unsigned)std::min<size_t>(device ? kMaxDeviceBlocks : kMaxUploadBlocks, (items + 255) / 256); }
 

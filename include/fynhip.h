@@ -204,7 +204,10 @@ int fyn_net_setup(fyn_net* net);
 
 /* UploadLayer::setInputBuffer + upload (gpu/uploadlayer.cpp:92-186): host fp32 buffer in `order`
  * for the UPLOAD layer `layer`; for any other layer: writes the tensor on input port `port`
- * directly (what LayerTestBase::generateTextures does, unit_tests/layertestbase.cpp:208-417). */
+ * directly (what LayerTestBase::generateTextures does, unit_tests/layertestbase.cpp:208-417).
+ * `data` is borrowed for the call: host memory has been read when it returns (the conversion may still run on the
+ * network's stream).  Page-locked memory is read when the work queued on the default stream before the call has ended, as
+ * device memory is. */
 int fyn_net_set_input(fyn_net* net, int layer, int port, const float* data, int order);
 /* Number of floats fyn_net_set_input reads from `data` for that layer and port (channels x height x width; the size
  * the CPUBuffer handed to UploadLayer::setInputBuffer must have). */
@@ -213,7 +216,7 @@ int fyn_net_input_floats(fyn_net* net, int layer, int port, size_t* count);
 /* NeuralNetwork::forward (base/neuralnetwork.cpp:173-187): runs all layers in ascending number on
  * the network's stream; returns the sequence number used.  Asynchronous w.r.t. the host. */
 int fyn_net_forward(fyn_net* net, uint64_t* seq_out);
-/* NeuralNetwork::finish (base/neuralnetwork.cpp:196-206): waits for the stream. */
+/* NeuralNetwork::finish (base/neuralnetwork.cpp:196-206): waits for the stream (polling for up to 2 ms, then asleep). */
 int fyn_net_finish(fyn_net* net);
 
 /* GPULayerBase::copyResult(float*, bool) (gpu/gpulayerbase.cpp:525-564): output of `layer` as CHW
@@ -252,7 +255,7 @@ int fyn_net_enable_intermediate_output(fyn_net* net, const char* dir);
  * convolution next to it can run as one launch when nothing else reads the tensor between them, a
  * plain batch-norm layer is applied on fetch by the convolutions that read it, a 1x1 shortcut
  * projection is computed by the 1x1 layer that adds it, a sigmoid or tanh layer by the convolution in
- * front of it, and bilinear scale layers in front of a concatenation and a batch-norm layer behind it
+ * front of it, an arg-max layer by the 1x1 convolution in front of it (which still writes the scores), and bilinear scale layers in front of a concatenation and a batch-norm layer behind it
  * run in its launch. */
 int fyn_net_set_buffer_reuse(fyn_net* net, int enable);
 
@@ -267,17 +270,22 @@ int fyn_layer_time(fyn_net* net, int layer, int iters, float* ms_total);
  * events around pass i (for medians and percentiles). */
 int fyn_net_time_steps(fyn_net* net, int iters, float* ms_each);
 /* Frame pipeline for streams of frames handed over in host memory -- the reference engine's asynchronous mode
- * (fyusenet/base/engine.cpp:386-683, two upload/download buffer sets: gpu/uploadlayer.h:74).  The upload of frame
- * i+1 and the download of frame i-1 overlap the layers of frame i (pinned staging buffers, three streams).
- *   begin : input = an upload layer (or an unconnected input port), output = any layer; `depth` frames in flight.
- *   submit: copies `in` (borrowed for the call) and queues the frame; `out` must stay valid until the frame's
- *           ticket has been waited for (it is filled then, or when its slot is reused `depth` submits later).
+ * (fyusenet/base/engine.cpp:386-683, two upload/download buffer sets: gpu/uploadlayer.h:74).  The transfers of a frame
+ * overlap the layers of its neighbours.
+ *   begin : input = an upload layer (or an unconnected input port), output = any layer; `depth` frames in flight
+ *           (page-locked memory for depth + 1).
+ *   submit: copies `in` (borrowed for the call) and queues the frame; delivers, or waits for, the frame that was
+ *           submitted `depth` calls earlier.  `out` belongs to the pipeline from then on: it may be written at any time,
+ *           by a thread of the library's, until the frame's ticket has been waited for.
  *   wait  : blocks until the frame (and all earlier ones) has been delivered.   end: drains and frees the pipeline.
  * Orders: input CHANNELWISE or GPU_SHALLOW, output CHANNELWISE or GPU_SHALLOW.
- * copy_streams != 0: uploads and downloads run on two streams of the pipeline's own (overlap inside this network).
- * copy_streams == 0: they are queued on the network's stream, between the frames' layers; for several networks that
- * run side by side, whose frames overlap each other, and whose streams would otherwise outnumber the hardware queues
- * of the process (streams that share a queue wait for each other's events). */
+ * copy_streams != 0, and more than 1 MB per frame (input and result together): uploads and downloads run on two streams
+ * of the pipeline's own (overlap inside this network).  A thread of the pipeline's joins them to the network's stream and
+ * delivers the results; it polls while frames are under way and sleeps otherwise.
+ * copy_streams == 0, or smaller frames: transfers run on the network's stream, between the frames' layers; for several
+ * networks that run side by side, whose frames overlap each other.
+ * A frame whose upload has not arrived four seconds after its turn (the process was stopped, say) is lost: submit, wait
+ * and end report FYN_ERR_DEVICE, and the pipeline has to be begun anew. */
 int fyn_net_async_begin(fyn_net* net, int in_layer, int in_port, int in_order, int out_layer, int out_order, int depth, int copy_streams);
 int fyn_net_async_submit(fyn_net* net, const float* in, float* out, uint64_t* ticket);
 int fyn_net_async_wait(fyn_net* net, uint64_t ticket);
