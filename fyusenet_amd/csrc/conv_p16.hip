@@ -1943,8 +1943,8 @@ int P16_NAME(launch_conv_kr16)(const ConvP16Params& p, int k, hipStream_t s) {
     if (ensure_lds(reinterpret_cast<const void*>(e->fn), e->lds) != 0) return -2;
     // (a tile's place in its XCD's band counts in the grid's last dimension; fewer tiles than XCDs, or a block's weights
     // larger than the pixels of all tiles: blocks first.  The waits for a tile's pixels in ResNet-50's 56x56 and 28x28
-    // layers go from 3250 to 2600 and from 2780 to 2200 clocks; what that gives the frame, 1 to 2 %, is no more than boxes
-    // and runs differ by)
+    // layers go from 3250 to 2600 and from 2780 to 2200 clocks; what that gives the frame, 1 to 2 %, is no more than runs
+    // differ by)
     const long long n = (long long)p.tiles_x * p.tiles_y, pixels = (long long)p.npos_y * p.stride * p.npos_x * p.stride * p.in_cp;
     ConvP16Params q = p;
     q.tile_major = n >= 8 && n < (1 << 22) && pixels > (long long)k * k * p.cin_chunks * KC * 16 * p.mfrags && p.cout_blocks <= 65535;

@@ -837,7 +837,8 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
 // The same for interleaved pixels of pc floats.
 void Net::download_pixels(const TView& v, int pc, float* out) {
     const size_t npix = (size_t)v.h * v.w, bytes = npix * pc * sizeof(float);
-    const bool host = host_memory(out), direct = host && HostPool::contains(out, bytes);
+    // (a pixel is one store of up to sixteen bytes)
+    const bool host = host_memory(out), direct = host && (reinterpret_cast<size_t>(out) & 15) == 0 && HostPool::contains(out, bytes);
     HostLoan loan = host && !direct ? out_area(npix * pc) : HostLoan();
     float* st = direct ? out : host ? loan.floats() : staging(npix * pc);
     const size_t step = host && !direct ? piece_pixels(npix, bytes) : npix;

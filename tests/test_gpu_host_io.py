@@ -104,6 +104,30 @@ def test_results_belong_to_the_caller():
     for value, k in zip((0, 1, 3, 4, 5), kept):
         assert (k == value).all()
 
+@pytest.mark.gpu
+@STORAGES
+@pytest.mark.parametrize("order", [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW], ids=["chw", "hwc"])
+@pytest.mark.parametrize("c,h,w", [(1, 64, 300), (2, 63, 301), (3, 65, 302), (4, 66, 299)])
+def test_results_at_any_place_of_a_block(c, h, w, order, storage):
+    """A result that begins one, two or three floats into memory of the library's (fyn_host_acquire), with guards around it."""
+    net = _copy_net(c, h, w, storage)
+    x = prng.uniform(70 + c, (c, h, w), -2.0, 2.0)
+    net.layers[1].setInput(x, 0)
+    net.forward()
+    want = x if storage == fa.STORAGE_F32 else x.astype(np.float16).astype(np.float32)
+    pc = 4 if c == 3 else c
+    n = h * w * (c if order == fa.ORDER_CHANNELWISE else pc)
+    for offset in range(4):
+        block = capi.result_array((n + 8,))
+        assert type(block.base).__name__ == "_ResultBlock"
+        block[:] = 77.0
+        out = block[offset:offset + n]
+        capi.check(capi.lib().fyn_net_get_output(net._h, 1, capi.fptr(out), order))
+        got = out.reshape(c, h, w) if order == fa.ORDER_CHANNELWISE else out.reshape(h, w, pc)[..., :c].transpose(2, 0, 1)
+        assert np.array_equal(got, want), offset
+        assert (block[:offset] == 77.0).all() and (block[offset + n:] == 77.0).all(), offset
+    net.cleanup()
+
 
 @pytest.mark.gpu
 @STORAGES
