@@ -75,12 +75,13 @@ class HostSignal {
 class HostLoan {
   public:
     HostLoan() = default;
-    explicit HostLoan(size_t bytes, bool filled_by_host = false) : p_(HostPool::acquire(bytes, false, filled_by_host)) {}
-    HostLoan(HostLoan&& o) noexcept : p_(o.p_), signal_(o.signal_), value_(o.value_) { o.p_ = nullptr; }
+    explicit HostLoan(size_t bytes, bool filled_by_host = false) : p_(HostPool::acquire(bytes, false, filled_by_host)), frame_(filled_by_host) {}
+    HostLoan(HostLoan&& o) noexcept : p_(o.p_), frame_(o.frame_), signal_(o.signal_), value_(o.value_) { o.p_ = nullptr; }
     HostLoan(const HostLoan&) = delete;
     HostLoan& operator=(const HostLoan&) = delete;
     ~HostLoan() {
-        if (signal_ && !signal_->reached(value_)) signal_->release_then(p_, value_);
+        // (the area of a frame waits for the next one: it does not go back to the system here, however full the pool is)
+        if (signal_ && (frame_ || !signal_->reached(value_))) signal_->release_then(p_, value_);
         else HostPool::release(p_);
     }
     void used_until(const HostSignal& s, unsigned value) { signal_ = &s; value_ = value; }   // by the launch that was given `value`
@@ -88,6 +89,7 @@ class HostLoan {
 
   private:
     void* p_ = nullptr;
+    bool frame_ = false;
     const HostSignal* signal_ = nullptr;
     unsigned value_ = 0;
 };
