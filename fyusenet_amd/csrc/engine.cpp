@@ -1120,7 +1120,7 @@ void Net::async_begin(int in_layer, int in_port, int in_order, int out_layer, in
         alloc_bytes_ += in_bytes + async_rows_ * async_row_;
     }
     if (async_own_streams_) {
-        carry_end_ = false;
+        carry_end_ = carry_stale_ = false;
         carry_error_ = nullptr;
         uploads_ = 0;
         async_pixels_ = (size_t)vi.h * vi.w;
@@ -1141,11 +1141,15 @@ static void add_rows(HostCopy& copies, float* to, const float* from, size_t byte
 void Net::async_complete(AsyncSlot& s) {
     if (async_own_streams_) {
         for (int i = 0; i < 4096 && s.busy.load(std::memory_order_acquire); i++) _mm_pause();
-        std::unique_lock<std::mutex> lk(carry_mu_);
-        carry_done_.wait(lk, [&] { return !s.busy.load(std::memory_order_acquire) || carry_error_; });
-        if (carry_error_) std::rethrow_exception(carry_error_);
-        if (__atomic_load_n(&async_feed_->late, __ATOMIC_RELAXED)) fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
-        return;
+        for (;;) {
+            {
+                std::unique_lock<std::mutex> lk(carry_mu_);
+                carry_done_.wait(lk, [&] { return !s.busy.load(std::memory_order_acquire) || carry_error_ || carry_stale_; });
+                if (carry_error_) std::rethrow_exception(carry_error_);
+                if (!carry_stale_) return;
+            }
+            async_again();
+        }
     }
     if (!s.busy) return;
     signal_.wait(s.value, stream);
@@ -1156,6 +1160,35 @@ void Net::async_complete(AsyncSlot& s) {
         out.start(kPipelineShared);
     }
     s.busy = false;
+}
+
+// A frame's conversion, layers and result, on the network's stream.
+void Net::queue_frame(AsyncSlot& s) {
+    const TView &vi = async_in_->v, &vo = async_out_view_;
+    const size_t opix = (size_t)vo.h * vo.w;
+    const float* src = async_own_streams_ ? s.dev_in : s.pin_in;
+    float* dst = async_own_streams_ ? s.dev_out : s.pin_out;
+    const UploadRange range{async_in_->amax, upload_words_};
+    if (async_in_order_ == FYN_ORDER_CHANNELWISE) launch_chw_to_tensor(src, async_in_plane_, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
+    else launch_hwc_to_tensor(src, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
+    forward(nullptr);
+    const HostDone done = signal_.next();
+    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, dst, opix, 0, 0, opix, done, stream);
+    else launch_tensor_to_hwc(vo, dst, vo.c == 3 ? 4 : vo.c, 0, opix, done, stream);
+    FYN_HIP(hipGetLastError());
+    s.value = done.value;
+}
+
+// A frame was computed before its upload had arrived (the process was stopped while the frame's launches waited): it and
+// the ones behind it are computed again.  The pipeline's thread leaves them alone until then; a frame keeps its slot, and
+// so its place in device memory, until its result has been delivered.
+void Net::async_again() {
+    FYN_HIP(hipStreamSynchronize(up_stream_));
+    FYN_HIP(hipStreamSynchronize(stream));
+    async_feed_->late = 0;   // (no launch waits any more)
+    for (AsyncSlot* s : carried_) queue_frame(*s);
+    std::lock_guard<std::mutex> lk(carry_mu_);
+    carry_stale_ = false;
 }
 
 // Whether the copies on a stream of the pipeline's are through (asked: an event would occupy a queue of the GPU).
@@ -1182,9 +1215,15 @@ void Net::carry() {
                 __atomic_store_n(&async_feed_->ready, n * (unsigned)async_pixels_, __ATOMIC_RELEASE);
                 uploaded = n;
             }
-            if (!idle) return;
+            if (!idle || carry_stale_) return;
             AsyncSlot* s = front();
             if (s && signal_.reached(s->value)) {
+                if (__atomic_load_n(&async_feed_->late, __ATOMIC_ACQUIRE)) {
+                    std::lock_guard<std::mutex> lk(carry_mu_);
+                    carry_stale_ = true;
+                    carry_done_.notify_all();
+                    return;
+                }
                 FYN_HIP(hipMemcpy2DAsync(s->pin_out, async_row_ + kRowGap, s->dev_out, async_row_, async_row_, async_rows_, hipMemcpyDeviceToHost, down_stream_));
                 sent = s;
             }
@@ -1193,6 +1232,7 @@ void Net::carry() {
         for (;;) {
             {
                 std::unique_lock<std::mutex> lk(carry_mu_);
+                if (carry_end_ && carry_stale_) return;   // (computing them again has failed)
                 if (carried_.empty() && uploaded == uploads_.load(std::memory_order_acquire)) {
                     carry_more_.wait(lk, [&] { return carry_end_ || !carried_.empty() || uploaded != uploads_.load(std::memory_order_acquire); });
                     if (carry_end_ && carried_.empty()) return;
@@ -1205,7 +1245,7 @@ void Net::carry() {
                 if (sent) continue;
                 const auto waited = std::chrono::steady_clock::now() - since;
                 if (waited > std::chrono::milliseconds(5)) std::this_thread::sleep_for(std::chrono::microseconds(20));   // (long frames)
-                if (waited > std::chrono::seconds(1)) {   // something may have failed
+                if (waited > std::chrono::seconds(1) && !carry_stale_) {   // something may have failed
                     AsyncSlot* s = front();
                     if (s && copies_made(stream) && !signal_.reached(s->value)) fail(FYN_ERR_DEVICE, "a launch ended without telling so");
                     since = std::chrono::steady_clock::now();
@@ -1246,8 +1286,7 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
     AsyncSlot& s = slots_[async_seq_ % slots_.size()];
     async_complete(s);
     const TView& vi = async_in_->v;
-    const TView& vo = async_out_view_;
-    const size_t npix = (size_t)vi.h * vi.w, opix = (size_t)vo.h * vo.w;
+    const size_t npix = (size_t)vi.h * vi.w;
     const bool planes = async_in_order_ == FYN_ORDER_CHANNELWISE;
     {
         HostCopy copies;
@@ -1268,10 +1307,8 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
             }
         }
     }
-    const float* src = s.pin_in;
     if (async_own_streams_) {
-        src = s.dev_in;
-        const HostFeed feed{async_feed_, uploads_.load() * (unsigned)npix, 0.f, kFeedGiveUp};
+        const HostFeed feed{async_feed_, uploads_.load() * (unsigned)npix, 0.f, feed_give_up_};
         {
             std::lock_guard<std::mutex> lk(carry_mu_);
             uploads_++;
@@ -1280,16 +1317,7 @@ void Net::async_submit(const float* in, float* out, uint64_t* ticket) {
         if (feed_ahead_) launch_await_feed(feed, npix, stream);
         else FYN_HIP(hipStreamSynchronize(up_stream_));
     }
-    const UploadRange range{async_in_->amax, upload_words_};
-    if (planes) launch_chw_to_tensor(src, async_in_plane_, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
-    else launch_hwc_to_tensor(src, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
-    forward(nullptr);
-    float* dst = async_own_streams_ ? s.dev_out : s.pin_out;
-    const HostDone done = signal_.next();
-    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, dst, opix, 0, 0, opix, done, stream);
-    else launch_tensor_to_hwc(vo, dst, vo.c == 3 ? 4 : vo.c, 0, opix, done, stream);
-    FYN_HIP(hipGetLastError());
-    s.value = done.value;
+    queue_frame(s);
     s.user_out = out;
     s.busy = true;
     s.ticket = ++async_seq_;
@@ -1344,7 +1372,6 @@ void Net::async_end() {
         if (s.dev_in) (void)hipFree(s.dev_in);
         if (s.dev_out) (void)hipFree(s.dev_out);
     }
-    const bool late = async_feed_ && async_feed_->late;
     HostPool::release(async_feed_);
     async_feed_ = nullptr;
     slots_.clear();
@@ -1353,7 +1380,6 @@ void Net::async_end() {
     up_stream_ = down_stream_ = nullptr;
     async_seq_ = 0;
     if (error) std::rethrow_exception(error);
-    if (late) fail(FYN_ERR_DEVICE, "a launch waited too long for its frame");
 }
 
 }  // namespace fynhip

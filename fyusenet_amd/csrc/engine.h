@@ -202,7 +202,10 @@ class Net {
     FeedWord* async_feed_ = nullptr;       // pixels of them that have arrived in device memory
     size_t async_pixels_ = 0;              // of a frame
     bool carry_end_ = false;
+    std::atomic<bool> carry_stale_{false};   // the result at the front was computed before its frame had arrived
     void carry();
+    void async_again();
+    void queue_frame(AsyncSlot& s);
     void run_layers(bool with_events);
     void release_all();
     void collect_timings();

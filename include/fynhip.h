@@ -283,9 +283,7 @@ int fyn_net_time_steps(fyn_net* net, int iters, float* ms_each);
  * of the pipeline's own (overlap inside this network).  A thread of the pipeline's joins them to the network's stream and
  * delivers the results; it polls while frames are under way and sleeps otherwise.
  * copy_streams == 0, or smaller frames: transfers run on the network's stream, between the frames' layers; for several
- * networks that run side by side, whose frames overlap each other.
- * A frame whose upload has not arrived four seconds after its turn (the process was stopped, say) is lost: submit, wait
- * and end report FYN_ERR_DEVICE, and the pipeline has to be begun anew. */
+ * networks that run side by side, whose frames overlap each other. */
 int fyn_net_async_begin(fyn_net* net, int in_layer, int in_port, int in_order, int out_layer, int out_order, int depth, int copy_streams);
 int fyn_net_async_submit(fyn_net* net, const float* in, float* out, uint64_t* ticket);
 int fyn_net_async_wait(fyn_net* net, uint64_t ticket);

@@ -87,6 +87,40 @@ def test_overlapped_pipeline_matches_the_synchronous_path(width, height, depth, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("graph", [False, True], ids=["eager", "graph"])
+@pytest.mark.parametrize("order", [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW], ids=["chw", "hwc"])
+@pytest.mark.parametrize("depth", [1, 2, 4])
+def test_overlapped_pipeline_computes_late_frames_again(monkeypatch, depth, order, graph):
+    """Launches that give up at once on a frame that has not arrived (FYNHIP_FEED_GIVE_UP): every result is the frame's own."""
+    monkeypatch.setenv("FYNHIP_FEED_GIVE_UP", "0")
+    width, height = 660, 500
+    net = samples.StyleNetSample(3, width, height)
+    net.setup()
+    net.useGraph(graph)
+    hwc = order == fa.ORDER_GPU_SHALLOW
+    frames = [prng.uniform(4100 + i, (height, width, 3) if hwc else (3, height, width), 0.0, 1.0) for i in range(3 * depth + 4)]
+    want = []
+    for f in frames:
+        net.layers[net.UPLOAD].setInput(f, 0, order)
+        net.forward()
+        want.append(np.array(net.getOutput(net.output_layer, order)))
+    for again in range(2):
+        net.asyncBegin(net.UPLOAD, net.output_layer, inOrder=order, outOrder=order, depth=depth)
+        outs = [np.full_like(want[0], np.nan) for _ in frames]
+        tickets = [net.asyncSubmit(f, o) for f, o in zip(frames, outs)]
+        if again:
+            net.asyncEnd()
+        else:
+            for t, (got, w) in enumerate(zip(outs, want)):
+                net.asyncWait(tickets[t])
+                assert np.array_equal(got, w), t
+            net.asyncEnd()
+        for i, (got, w) in enumerate(zip(outs, want)):
+            assert np.array_equal(got, w), (again, i)
+    net.cleanup()
+
+
+@pytest.mark.gpu
 def test_results_belong_to_the_caller():
     """A result handed out stays what it was while later frames pass and after the network has gone; memory of results
     that nobody holds is used again."""
