@@ -5,22 +5,28 @@
 // Replaces, for such layers, the render passes of DeepConvLayerNxN::forward (fyusenet/gpu/deep/deepconvlayerNxN.cpp:
 // 129-211); epilogue order of shaders/deep/deepconv3x3_tiled.frag:36-45 (acc*scale + bias, then the residual).
 //
-// Why another MFMA kernel: these layers run for hundreds of microseconds, and what bounds the general kernel on them is
-// operand traffic and the rounds of a launch.  Its waves hold 32 output channels x 96 positions, so every wave reads the
-// whole position tile from LDS for each k16 step (128 bytes per CU and MFMA cycle, about what the LDS delivers), and
-// its 1872 workgroups, two per CU, make 3.7 rounds with a prologue and an epilogue per tile in the open.  Here a wave
-// holds 64 channels x 96 positions (4 x 6 fragments, 96 accumulator registers): 64 bytes per cycle from LDS and 43 from
-// the L1 (weights), and a workgroup walks its tiles with four staging waves running a stage ahead, as in conv_p16.hip.
+// Why another MFMA kernel: these layers run for hundreds of microseconds, and what bounds them is how the operands reach
+// the matrix cores.  A fragment here is one row of sixteen positions, so the fragment that output row r needs at tap row
+// ky is the one row r + 1 needed at ky - 1: the taps are walked column by column (kx outside, ky inside), a wave keeps
+// the TH fragments of its tile's rows in registers and every step replaces one of them.  A kernel column of K steps
+// reads TH + K - 1 fragments from LDS instead of TH * K (20 instead of 108 for K = 9, TH = 12).  That makes the position
+// side so cheap that the four MFMA waves can each take 32 output channels of the workgroup's 128 and ALL of its
+// positions: no two waves load the same weights, 21 bytes per MFMA cycle and CU through the L1 (which delivers 64) and 23
+// from LDS (128), where two groups of 64 channels x two tiles of positions took 43 and 64.
+// Measured, fp16: 9x9 128 -> 128 at 464x381 positions (469 GFLOP) 338 -> 280 us a layer = 1.67 PFLOP/s, what the library
+// reaches on a 16384^3 product here (1.63); 352x225 206 -> 146 us; 3x3 128 -> 128 at 156x128 (5.9 GFLOP) 9.4 -> 6.1 us.
+// Bound: the matrix pipes at the clock the part holds under them (79 % busy at 1.95-2.0 GHz in the launch of 12-row
+// tiles; without any operand traffic the same loop is 90 % busy at 2.2).  Weights requested 2, 3, 4 or 8 steps ahead,
+// results stored by the staging waves, and the weights brought into the L2 ahead of use: no difference.
 //
-// GEMM view: M = output channels (A = weights, packed per lane, streamed through L2/L1 into a register ring of three
-// steps), N = positions (B = activations, a halo tile of one 32-channel chunk in LDS), K = taps x channels, one tap of one
-// chunk per step.  A stage is one chunk of one tile: K kernel rows of K steps; the code of one kernel row is unrolled
-// (the tap's column is an immediate offset of the LDS reads), the rows are a loop that moves the fragments' base
-// registers by a row pitch.
+// GEMM view: M = output channels (A = weights, packed per lane, streamed through L2/L1 into a register ring), N = positions (B = activations, a halo tile of one 32-channel chunk in LDS), K = taps x channels, one tap of one
+// chunk per step.  The code of nine steps is unrolled: one kernel column of the 9x9 kernel (the columns are a loop that
+// moves one base register by a pixel), the whole chunk of a 3x3 kernel.
 //
-// Workgroup = 4 staging waves + 4 MFMA waves (2 groups of 64 output channels x 2 tiles of TH x 8 positions side by
-// side).  A lane's accumulators of one fragment are 4 consecutive output channels of one position: no transposition in
-// the epilogue; residual (staged to LDS by the staging waves during a tile's last chunk) and scale/bias from LDS.
+// Workgroup = 4 staging waves + 4 MFMA waves (32 output channels each x TH rows of 16 positions).  The weights are packed
+// so that a lane's eight accumulators of a row are eight consecutive output channels of one position: no transposition in
+// the epilogue, one 16-byte store per lane and row; residual (staged to LDS by the staging waves during a tile's last
+// chunk) and scale/bias from LDS.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -33,59 +39,71 @@
 namespace fynhip {
 
 namespace {
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-constexpr int HPD = 3;    // depth of the weight-fragment ring (steps); a kernel row is a whole number of turns
-constexpr int HFM = 4;    // fragments of 16 output channels per wave
+constexpr int HNS = 9;    // unrolled steps, and slots of the weight-fragment ring
+constexpr int HFM = 2;    // fragments of 16 output channels per wave
 
+// (TW_: the workgroup's tile is two times TW_ = 8 columns wide, the sixteen positions of a fragment)
 template <int K_, int TH_, int TW_>
 struct GeoH {
     static constexpr int K = K_, TH = TH_, TW = TW_;
-    static constexpr int WM = 2, WN = 2, TWG = WN * TW;
+    static constexpr int WM = 4, TWG = 2 * TW;
     static constexpr int HW = TWG + K - 1, HH = TH + K - 1;
-    static constexpr int ROW_PITCH = HW * PITCH + p16_row_pad(TH, TW, 1, WN, HW);
+    static constexpr int ROW_PITCH = HW * PITCH + p16_row_pad(TH, TWG, 1, 1, HW);
     static constexpr int BUF = HH * ROW_PITCH;            // one staging buffer (fp16 storage: one plane)
-    static constexpr int NPOS = TH * TW, FN = NPOS / 16;  // per wave
+    static constexpr int FN = TH;                         // position fragments: rows of the tile
+    // steps from the request of a weight fragment to its use (so many slots of the ring are registers; eight are no faster)
+    static constexpr int LEAD = (K == 3 && TH > 10) ? 2 : 3;
     static constexpr int NITEMS = HH * HW * (KC / 8);     // staging items: (pixel, 8 channels)
     static constexpr int NB = (NITEMS + 255) / 256;
     static constexpr int CPB = 16 * HFM * WM;             // output channels per workgroup
     static constexpr int RES_PITCH = CPB * 2 + 16;        // bytes per position of the residual tile
     static constexpr int RPIECES = TH * TWG * (CPB / 8);  // residual 16-byte pieces
-    static constexpr int RNB = (RPIECES + 255) / 256;
-    static_assert(NPOS % 16 == 0, "whole position fragments");
-    static_assert(K % HPD == 0, "a kernel row is whole turns of the weight ring");
-    static_assert(K * PITCH < 65536, "the tap column fits the LDS instructions' immediate field");
+    static constexpr int RNB = RPIECES / 256;
+    static_assert(RPIECES % 256 == 0, "whole turns of the staging threads");
+    static_assert(TWG == 16, "a fragment is a row of the tile");
+    static_assert(HNS % K == 0 && (K * K) % HNS == 0, "the unrolled steps are whole kernel columns");
+    static_assert(HH * ROW_PITCH + K * PITCH < 65536, "offsets inside a staging buffer fit the LDS instructions' immediate field");
 };
 
-// The K steps of one kernel row of a stage.  `brow`: per-lane LDS offsets of the row's fragments at tap column 0;
-// `nxt`: offsets of the fragments of the step that follows the row (the next kernel row, or the first step of the next
-// stage in the other staging buffer -- LAST: the stage's barrier sits in front of the first such read; the staging waves
-// have filled that buffer by then, and all reads of this stage's buffer were issued a step earlier).  One slot per
-// MFMA: the MFMA, then a share of the step's memory instructions, fenced so that the compiler keeps the order.
-// Position fragment fn is used by four consecutive MFMAs, after which its registers take the fragment of the next
-// step; the ring slot of the previous step takes the weights of the step after the next.
+// Nine steps of a stage: HNS / K kernel columns of K taps each.  `col`: per-lane LDS offset of (row 0, first of these
+// columns); `next_col`: the same for the column behind the last one (LAST: the first column of the next stage, in the
+// other staging buffer -- the stage's barrier sits in front of the first such read; the staging waves have filled that
+// buffer by then, and all reads of this stage's buffer were issued a step earlier).  The fragment of input row r lives in
+// slot r % TH: at tap row ky the live rows are ky .. ky + TH - 1, the slots are used in their order, and the one that held
+// row ky takes row ky + TH behind its last MFMA; a column's last step refills every slot with the next column's rows 0 ..
+// TH - 1.  A refilled slot is used a whole step later.  One slot of the schedule per MFMA: the MFMA, then a share of the
+// step's memory instructions, fenced so that the compiler keeps the order.  A step also
+// requests the weights of the step LEAD further on.
 template <class G, bool LAST>
-__device__ __forceinline__ void h16_row(f32x4_t (&acc)[HFM][G::FN], half8_t (&a_q)[HPD][HFM], half8_t (&b)[G::FN], const int (&brow)[G::FN],
-                                        const int (&nxt)[G::FN], const unsigned char* lds, const unsigned char*& wnext,
-                                        const unsigned char* wbase, const unsigned char* wend, unsigned wstep, unsigned wlane) {
+__device__ __forceinline__ void h16_steps(f32x4_t (&acc)[HFM][G::FN], half8_t (&a_q)[HNS][HFM], half8_t (&b)[G::FN], int col, int next_col,
+                                          const unsigned char* lds, const __amdgpu_buffer_rsrc_t weights, unsigned& wnext, unsigned wend, unsigned wstep,
+                                          unsigned wlane) {
     constexpr int FN = G::FN, K = G::K;
+    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int dd = 0; dd < K; dd++) {
-        const int d = dd % HPD, dprev = (d + HPD - 1) % HPD;
-        const unsigned char* w_ = wnext;
+    for (int d = 0; d < HNS; d++) {
+        const int kx = d / K, ky = d % K;
+        const unsigned w_ = wnext;
         wnext += wstep;
-        if (wnext == wend) wnext = wbase;
+        if (wnext == wend) wnext = 0;
 #pragma unroll
         for (int i = 0; i < HFM * FN; i++) {
-            const int fn = i / HFM, fm = i % HFM;
-            acc[fm][fn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_q[d][fm], b[fn], acc[fm][fn], 0, 0, 0);
-            if (LAST && dd == K - 1 && i == 1) lds_barrier();
+            const int slot = i / HFM, fm = i % HFM;
+            const int row = ((slot - ky) % FN + FN) % FN;   // the output row whose fragment this slot holds
+            acc[fm][row] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_q[d][fm], b[slot], acc[fm][row], 0, 0, 0);
+            if (LAST && d == HNS - 1 && i == 0) lds_barrier();
             if (fm == HFM - 1) {
-                if (dd + 1 < K) b[fn] = *reinterpret_cast<const half8_t*>(lds + brow[fn] + (dd + 1) * PITCH);
-                else b[fn] = *reinterpret_cast<const half8_t*>(lds + nxt[fn]);
+                if (ky + 1 < K) {
+                    if (row == 0) b[slot] = *reinterpret_cast<const half8_t*>(lds + col + kx * PITCH + (ky + FN) * G::ROW_PITCH);
+                } else if (d + 1 < HNS) {
+                    b[slot] = *reinterpret_cast<const half8_t*>(lds + col + (kx + 1) * PITCH + slot * G::ROW_PITCH);
+                } else {
+                    b[slot] = *reinterpret_cast<const half8_t*>(lds + next_col + slot * G::ROW_PITCH);
+                }
             }
 #pragma unroll
-            for (int j = 0; j < HFM; j++)   // the weight fragments of the step after the next, spread over this step's slots
-                if (i == j * FN + 1) a_q[dprev][j] = *reinterpret_cast<const half8_t*>(w_ + j * 1024 + wlane);
+            for (int j = 0; j < HFM; j++)   // the weight fragments, spread over the step's slots
+                if (i == j * FN + 1) a_q[(d + G::LEAD) % HNS][j] = __builtin_bit_cast(half8_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights, wlane + j * 1024, w_, 0));
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -159,13 +177,13 @@ __device__ __forceinline__ void h16_stager(const ConvP16Params& p, unsigned char
             const int m = idx / (CPB / 8), c8 = idx % (CPB / 8);
             const int ty = m / G::TWG, tx = m - ty * G::TWG;
             const int py = tyi * G::TH + ty, px = txi * G::TWG + tx;
-            const bool ok = idx < G::RPIECES && py < p.npos_y && px < p.npos_x;
+            const bool ok = py < p.npos_y && px < p.npos_x;
             rv[i] = *reinterpret_cast<const half8_t*>(res + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + cb * CPB + c8 * 8 : 0));
         }
 #pragma unroll
         for (int i = 0; i < G::RNB; i++) {
             const int idx = stid + i * 256;
-            if (idx < G::RPIECES) *reinterpret_cast<half8_t*>(lds + res_off + (idx / (CPB / 8)) * G::RES_PITCH + (idx % (CPB / 8)) * 16) = rv[i];
+            *reinterpret_cast<half8_t*>(lds + res_off + (idx / (CPB / 8)) * G::RES_PITCH + (idx % (CPB / 8)) * 16) = rv[i];
         }
     };
     auto advance = [&](int& tile, int& c) {
@@ -225,27 +243,20 @@ __global__ __launch_bounds__(512) void conv_h16_kernel(const ConvP16Params p) {
 
     // ---------------------------------------------------------------------- MFMA waves
     const int mq = lane & 15, kq = lane >> 4;
-    const int mw = (wave - 4) % G::WM;   // this wave's 64 output channels of the workgroup's 128
-    const int wn = (wave - 4) / G::WM;   // ... and its tile of positions
-    int base[FN];    // per-lane LDS offset of the B fragments at tap (0, 0) in staging buffer 0
-#pragma unroll
-    for (int fn = 0; fn < FN; fn++) {
-        const int m = fn * 16 + mq;
-        const int ty = m / TW, tx = m - ty * TW;
-        base[fn] = ty * G::ROW_PITCH + (wn * TW + tx) * PITCH + kq * 16;
-    }
-    // A fragments: [(chunk*K + ky)*K + kx][cout fragment of 16][lane] x 8 halves
+    const int mw = wave - 4;   // this wave's 32 output channels of the workgroup's 128
+    const int base = mq * PITCH + kq * 16;   // per-lane LDS offset of the fragments at row 0, tap column 0 in staging buffer 0
+    // A fragments: [(chunk*K + kx)*K + ky][cout fragment of 16][lane] x 8 halves
     const unsigned wstep = (unsigned)p.mfrags * 1024;
     const unsigned char* wbase = reinterpret_cast<const unsigned char*>(p.wpack) + (size_t)(cb * (CPB / 16) + mw * HFM) * 1024;   // (uniform)
     const unsigned wlane = lane * 16;
-    const unsigned char* wend = wbase + (size_t)nchunks * K * K * wstep;
-    half8_t a_q[HPD][HFM];
+    const unsigned wend = (unsigned)(nchunks * K * K) * wstep;
+    // (as a buffer: the step's offset is a scalar operand of the load, no address arithmetic per lane)
+    const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(wbase), 0, (int)wend, 0x00020000);
+    half8_t a_q[HNS][HFM];
 #pragma unroll
-    for (int d = 0; d < HPD - 1; d++)
+    for (int d = 0; d < G::LEAD; d++)
 #pragma unroll
         for (int fm = 0; fm < HFM; fm++) a_q[d][fm] = *reinterpret_cast<const half8_t*>(wbase + (size_t)d * wstep + fm * 1024 + wlane);
-#pragma unroll
-    for (int fm = 0; fm < HFM; fm++) a_q[HPD - 1][fm] = a_q[0][fm];   // (defined; overwritten by the first step's loads)
     f32x4_t acc[HFM][FN];
     auto zero_acc = [&]() {
 #pragma unroll
@@ -254,71 +265,61 @@ __global__ __launch_bounds__(512) void conv_h16_kernel(const ConvP16Params p) {
             for (int fn = 0; fn < FN; fn++) acc[fm][fn] = (f32x4_t)(0.f);
     };
     zero_acc();
-    _Float16* out = reinterpret_cast<_Float16*>(p.out);
-    const bool have_res = p.res != nullptr;
     const bool res_scale = p.res_scale != 0;
     const float res_floor = p.res_relu ? 0.f : -__builtin_inff();
 
     auto finish_tile = [&](int tile) {
-        const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
         const float* sb = reinterpret_cast<const float*>(lds + sb_off);
         f32x4_t rs[HFM], bi[HFM], scm[HFM];
 #pragma unroll
         for (int fm = 0; fm < HFM; fm++) {
-            const f32x4_t sc = *reinterpret_cast<const f32x4_t*>(sb + mw * 64 + fm * 16 + kq * 4);
-            bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + CPB + mw * 64 + fm * 16 + kq * 4);
+            const f32x4_t sc = *reinterpret_cast<const f32x4_t*>(sb + mw * 32 + kq * 8 + fm * 4);
+            bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + CPB + mw * 32 + kq * 8 + fm * 4);
             scm[fm] = sc * p.acc_mul;
             rs[fm] = res_scale ? sc : (f32x4_t)(1.f);
         }
+        // a lane's eight channels of each row
+        const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
+        const int px = txi * G::TWG + mq;
+        _Float16* out = reinterpret_cast<_Float16*>(p.out) + ((size_t)(p.out_off_y + tyi * TH) * p.out_wp + p.out_off_x + px) * p.out_cp + cb * CPB + mw * 32 + kq * 8;
+        const int row_pitch = p.out_wp * p.out_cp;
+        const int nrows = px < p.npos_x ? p.npos_y - tyi * TH : 0;
+        auto rows = [&](auto residual) {
 #pragma unroll
-        for (int fn = 0; fn < FN; fn++) {
-            const int m = fn * 16 + mq;
-            const int ty = m / TW, tx = wn * TW + (m - ty * TW);
-            const int py = tyi * TH + ty, px = txi * G::TWG + tx;
-            const bool ok = py < p.npos_y && px < p.npos_x;
-            const size_t obase = ((size_t)(p.out_off_y + py) * p.out_wp + p.out_off_x + px) * p.out_cp + cb * CPB + mw * 64 + kq * 4;
+            for (int ty = 0; ty < FN; ty++) {
+                half8_t rv, hv;
+                if constexpr (decltype(residual)::value)
+                    rv = *reinterpret_cast<const half8_t*>(lds + res_off + (ty * G::TWG + mq) * G::RES_PITCH + (mw * 32 + kq * 8) * 2);
 #pragma unroll
-            for (int fm = 0; fm < HFM; fm++) {
-                f32x4_t v;
+                for (int fm = 0; fm < HFM; fm++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = acc[fm][fn][e] * scm[fm][e] + bi[fm][e];
-                if (have_res) {
-                    const half4_t rv = *reinterpret_cast<const half4_t*>(lds + res_off + (ty * G::TWG + tx) * G::RES_PITCH + (mw * 64 + fm * 16 + kq * 4) * 2);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = fmaf(fmaxf((float)rv[e], res_floor), rs[fm][e], v[e]);
-                }
-                half4_t hv;
-#pragma unroll
-                for (int e = 0; e < 4; e++) hv[e] = (_Float16)v[e];
-                if (ok) *reinterpret_cast<half4_t*>(out + obase + fm * 16) = hv;
+                    for (int e = 0; e < 4; e++) {
+                        float v = acc[fm][ty][e] * scm[fm][e] + bi[fm][e];
+                        if constexpr (decltype(residual)::value) v = fmaf(fmaxf((float)rv[fm * 4 + e], res_floor), rs[fm][e], v);
+                        hv[fm * 4 + e] = (_Float16)v;
+                    }
+                if (ty < nrows) *reinterpret_cast<half8_t*>(out + (size_t)ty * row_pitch) = hv;
+                if (ty % 3 == 2) __builtin_amdgcn_sched_barrier(0);   // (no more than three rows' residuals at a time in registers)
             }
-        }
+        };
+        if (p.res) rows(std::true_type());
+        else rows(std::false_type());
     };
 
     lds_barrier();   // the first stage is staged
     half8_t b[FN];
-    int brow[FN], nxt[FN];
 #pragma unroll
-    for (int fn = 0; fn < FN; fn++) {
-        brow[fn] = base[fn];
-        b[fn] = *reinterpret_cast<const half8_t*>(lds + brow[fn]);
-    }
-    const unsigned char* wnext = wbase + (size_t)((HPD - 1) % (nchunks * K * K)) * wstep;
+    for (int r = 0; r < FN; r++) b[r] = *reinterpret_cast<const half8_t*>(lds + base + r * G::ROW_PITCH);
+    unsigned wnext = G::LEAD * wstep;
     int tile = group, c = 0, buf = 0;
     for (;;) {
-        for (int ky = 0; ky < K - 1; ky++) {
-#pragma unroll
-            for (int fn = 0; fn < FN; fn++) nxt[fn] = brow[fn] + G::ROW_PITCH;
-            h16_row<G, false>(acc, a_q, b, brow, nxt, lds, wnext, wbase, wend, wstep, wlane);
-#pragma unroll
-            for (int fn = 0; fn < FN; fn++) brow[fn] = nxt[fn];
+        int col = base + buf * G::BUF;
+        for (int kx = HNS / K; kx < K; kx += HNS / K) {
+            h16_steps<G, false>(acc, a_q, b, col, col + HNS / K * PITCH, lds, weights, wnext, wend, wstep, wlane);
+            col += HNS / K * PITCH;
         }
         buf = 1 - buf;
-#pragma unroll
-        for (int fn = 0; fn < FN; fn++) nxt[fn] = base[fn] + buf * G::BUF;
-        h16_row<G, true>(acc, a_q, b, brow, nxt, lds, wnext, wbase, wend, wstep, wlane);
-#pragma unroll
-        for (int fn = 0; fn < FN; fn++) brow[fn] = nxt[fn];
+        h16_steps<G, true>(acc, a_q, b, col, base + buf * G::BUF, lds, weights, wnext, wend, wstep, wlane);
         if (++c == nchunks) {
             finish_tile(tile);
             c = 0; tile += p.pos_groups;
@@ -339,8 +340,8 @@ constexpr H16Entry h16_entry() {
     return H16Entry{K, TH, TW, conv_h16_kernel<K, TH, TW>, (size_t)(2 * G::BUF + 2 * G::CPB * 4), (size_t)(TH * G::TWG * G::RES_PITCH)};
 }
 const H16Entry H16_TABLE[] = {
-    h16_entry<9, 12, 8>(), h16_entry<9, 8, 8>(), h16_entry<9, 4, 8>(),
-    h16_entry<3, 12, 8>(), h16_entry<3, 8, 8>(), h16_entry<3, 4, 8>(),
+    h16_entry<9, 12, 8>(), h16_entry<9, 10, 8>(), h16_entry<9, 8, 8>(), h16_entry<9, 6, 8>(), h16_entry<9, 5, 8>(), h16_entry<9, 4, 8>(),
+    h16_entry<3, 12, 8>(), h16_entry<3, 10, 8>(), h16_entry<3, 8, 8>(), h16_entry<3, 6, 8>(), h16_entry<3, 5, 8>(), h16_entry<3, 4, 8>(),
 };
 constexpr int H16_COUNT = sizeof(H16_TABLE) / sizeof(H16_TABLE[0]);
 const H16Entry* h16_find(const ConvP16Params& p, int k) {
@@ -371,8 +372,9 @@ int launch_conv_h16(const ConvP16Params& p, int k, hipStream_t s) {
     if (p.cin_chunks < 1 || p.in_cp < p.cin_chunks * KC || p.mfrags % 8 != 0 || p.cout_blocks * 8 != p.mfrags || p.out_cp < p.cout_blocks * 128 ||
         (p.res && p.res_cp < p.cout_blocks * 128) || (p.res && p.cin_chunks < 2 && p.pos_groups != p.tiles_x * p.tiles_y) ||
         p.pos_groups < 1 || p.pos_groups > p.tiles_x * p.tiles_y || p.tiles_x < 1 || p.tiles_y < 1 || !p.f16 ||
-        p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.tiles_x * p.tiles_y > 4000000 || p.in_cp % 8 != 0 || p.out_cp % 4 != 0 || (p.res && p.res_cp % 8 != 0) ||
-        p.tiles_x * 2 * e->tw < p.npos_x || p.tiles_y * e->th < p.npos_y || !p.in || !p.out || !p.wpack || !p.scale || !p.bias)
+        p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.tiles_x * p.tiles_y > 4000000 || p.in_cp % 8 != 0 || p.out_cp % 8 != 0 || (p.res && p.res_cp % 8 != 0) ||
+        p.tiles_x * 2 * e->tw < p.npos_x || p.tiles_y * e->th < p.npos_y || !p.in || !p.out || !p.wpack || !p.scale || !p.bias ||
+        (size_t)p.cin_chunks * k * k * p.mfrags * 1024 >= (size_t)1 << 31)   // (offsets into the weights are 32 bits wide)
         return -1;
     const size_t lds = conv_h16_lds_bytes(p, k);
     if (ensure_lds(reinterpret_cast<const void*>(e->fn), lds) != 0) return -2;

@@ -329,7 +329,9 @@ class ConvLayer : public Layer {
         int want_h = 0, want_w = 0, want_rows1 = 0, want_h2 = 0;   // FYNHIP_P16_TILE=h,w and FYNHIP_H16_SPLIT=rows of the first band,h of the second (tests)
         if (const char* e = net->sw.get("FYNHIP_P16_TILE")) sscanf(e, "%d,%d", &want_h, &want_w);
         if (const char* e = net->sw.get("FYNHIP_H16_SPLIT")) sscanf(e, "%d,%d", &want_rows1, &want_h2);
-        // a band of `rows` output rows from row `row0` on, in tiles of th x tw; cost in MFMA cycles per wave (0: cannot be built)
+        // a band of `rows` output rows from row `row0` on, in tiles of th rows x two times tw columns; cost in cycles per wave:
+        // 32 MFMA cycles a step and row, and what a step, a tile and a launch cost beside them (fitted to 464x381 positions:
+        // tiles of 5, 8 and 12 rows within 5 %)
         auto band = [&](int th, int tw, int row0, int rows, ConvP16Params* c, double* cost) {
             *c = q;
             c->tile_h = th; c->tile_w = tw;
@@ -342,7 +344,7 @@ class ConvLayer : public Layer {
             const size_t lds = conv_h16_lds_bytes(*c, k);
             if (lds == 0 || lds > 160 * 1024) return false;
             const int rounds = (c->tiles_x * c->tiles_y * c->cout_blocks + 255) / 256;
-            *cost = (double)rounds * ((double)c->cin_chunks * k * k * (th * tw / 16) * 64 + 5000) + 10000;
+            *cost = (double)rounds * ((double)c->cin_chunks * k * k * (32 * th + 80) + 5000) + 10000;
             return true;
         };
         struct Cand { double cost; ConvP16Params a, b; bool two; };
@@ -430,24 +432,23 @@ class ConvLayer : public Layer {
             p16_wpack_dev = nullptr;
         }
     }
-    // weights of that form: [(chunk*K + ky)*K + kx][cout fragment of 16][lane][8 halves], zero steps behind the last
+    // weights of that form: [(chunk*K + kx)*K + ky][cout fragment of 16][lane][8 halves], zero steps behind the last; a
+    // fragment's rows are dealt so that a lane ends up with eight consecutive channels of a wave's 32 (p16_row_channel)
     void pack_h16(const float* w, float wmul) {
         const int cin = d.in_channels;
         std::vector<uint16_t> pack(((size_t)pp.cin_chunks * k * k + 8) * pp.mfrags * 64 * 8, 0);
         for (int chunk = 0; chunk < pp.cin_chunks; chunk++)
-            for (int tap = 0; tap < k * k; tap++)
-                for (int mf = 0; mf < pp.mfrags; mf++) {
-                    uint16_t* base = pack.data() + ((size_t)(chunk * k * k + tap) * pp.mfrags + mf) * 64 * 8;
-                    for (int lane = 0; lane < 64; lane++) {
-                        const int o = mf * 16 + (lane & 15);
-                        if (o >= oc) continue;
-                        for (int j = 0; j < 8; j++) {
-                            const int ci = chunk * 32 + 8 * (lane >> 4) + j;
-                            if (ci >= cin) continue;
-                            base[(size_t)lane * 8 + j] = f2h_bits(w[((size_t)o * k * k + tap) * cin + ci] * wmul);
+            for (int kx = 0; kx < k; kx++)
+                for (int ky = 0; ky < k; ky++)
+                    for (int mf = 0; mf < pp.mfrags; mf++) {
+                        uint16_t* base = pack.data() + (((size_t)(chunk * k + kx) * k + ky) * pp.mfrags + mf) * 64 * 8;
+                        for (int lane = 0; lane < 64; lane++) {
+                            const int o = p16_row_channel(mf, lane & 15, 2), ci = chunk * 32 + 8 * (lane >> 4);
+                            if (o >= oc) continue;
+                            const float* from = w + (((size_t)o * k + ky) * k + kx) * cin + ci;
+                            for (int j = 0; j < 8 && ci + j < cin; j++) base[(size_t)lane * 8 + j] = f2h_bits(from[j] * wmul);
                         }
                     }
-                }
         FYN_HIP(hipStreamSynchronize(net->stream));
         FYN_HIP(hipMemcpyAsync(p16_wpack_dev, pack.data(), pack.size() * 2, hipMemcpyHostToDevice, net->stream));
         FYN_HIP(hipStreamSynchronize(net->stream));
@@ -1398,7 +1399,7 @@ class ConvLayer : public Layer {
         }
         if (p16 && h16) {
             char buf[220];
-            snprintf(buf, sizeof(buf), "conv_h16 f16 tile=128x%d(cout x pos) waves=2x2 th=%d tw=%d blocks=%d tiles=%d lds=%zu steps=%d chunks=%d",
+            snprintf(buf, sizeof(buf), "conv_h16 f16 tile=128x%d(cout x pos) waves=4x1 th=%d tw=%d blocks=%d tiles=%d lds=%zu steps=%d chunks=%d",
                      pp.tile_h * pp.tile_w * 2, pp.tile_h, pp.tile_w, pp.pos_groups * pp.cout_blocks, pp.tiles_x * pp.tiles_y * pp.cout_blocks,
                      conv_h16_lds_bytes(pp, k), k * k, pp.cin_chunks);
             std::string info = mode + buf;

@@ -411,6 +411,33 @@ def test_fp16_sixteen_position_fragment_form(case, act, shallow, monkeypatch):
     assert err <= TOL[fa.STORAGE_F16], info
 
 
+@pytest.mark.parametrize("k,tile,h,w,residual", [
+    (9, "10,8", 31, 33, True),      # a row and a column behind the last whole tile
+    (9, "6,8", 18, 16, False),      # whole tiles
+    (9, "5,8", 4, 15, True),        # fewer rows than a tile has: the fragments' slots turn round more than once per column
+    (3, "10,8", 9, 49, False),
+    (3, "6,8", 50, 700, True),      # 396 tiles: workgroups walk two
+    (3, "5,8", 11, 17, True),
+    (3, "12,8", 13, 31, True),      # (weights requested two steps ahead instead of three)
+])
+def test_fp16_row_fragment_tiles(k, tile, h, w, residual, monkeypatch):
+    """Heights of the tile that are no multiple of the kernel's size, or smaller: a wave's fragments move through its
+    registers one row per tap, and a column's last step refills all of them."""
+    monkeypatch.setenv("FYNHIP_FORCE_P16_CONV", "1")
+    monkeypatch.setenv("FYNHIP_P16_TILE", tile)
+    kw = {"bn": True, "residual": (A.RELU, True)} if residual else {"pad_out": 1}
+    b = conv_builder(k, 128, h, w, 64, 1, 1, A.RELU, **kw)
+    wts = conv_block(2300 + k + h, 128, k, 64, bn=residual)
+    inputs = [prng.uniform(47 * h + w, (64, h, w), -1, 1)]
+    if residual:
+        inputs.append(prng.uniform(61, (128, h, w), -1, 1))
+    got, info = run_single(b, fa.STORAGE_F16, inputs, wts)
+    ref = oracle_single(b, fa.STORAGE_F16, inputs, wts)
+    print("  ", info, "rel_l2=%.3e" % rel_l2(got, ref), flush=True)
+    assert "conv_h16" in info and "th=%s tw=%s" % tuple(tile.split(",")) in info
+    assert rel_l2(got, ref) <= TOL[fa.STORAGE_F16], info   # (operands and result rounded to 11 bits, as in the test above)
+
+
 KR16_CASES = [
     # (k, cin, cout, h, w, fragments per block, kw)
     (1, 1024, 256, 14, 14, 1, {}),                                              # a ResNet stage-3 reduction layer
