@@ -25,6 +25,7 @@
 
 #include <cstdlib>
 #include <type_traits>
+#include <utility>
 
 #include "kernels.h"
 #include "p16_common.h"
@@ -84,7 +85,9 @@ struct Geo {
     static constexpr int RPIECES = TH * TWG * RPP;       // residual 16-byte pieces
     static constexpr int RNB = (RPIECES + 255) / 256;    // ... per staging thread
     static constexpr int slot_off(int c) { return (S == 1) ? c * PITCH : ((c & 1) * HWH + (c >> 1)) * PITCH; }
-    static constexpr int tap_off(int t) { return (t / 3) * ROW_PITCH + slot_off(t % 3); }
+    // tiles whose fragments are rows of sixteen positions take the taps column by column (p16_rows_c8), the others row by row
+    static constexpr bool ROWS = TW == 16;
+    static constexpr int tap_off(int t) { return ROWS ? (t % 3) * ROW_PITCH + slot_off(t / 3) : (t / 3) * ROW_PITCH + slot_off(t % 3); }
     static_assert(S == 1 || S == 2, "input step 1 or 2");
     static_assert(NPOS % 16 == 0, "whole position fragments");
     static_assert(PLANE + 2 * ROW_PITCH + 2 * PITCH + HWH * PITCH + 64 < 65536, "B fragment offsets inside a staging buffer fit the LDS instructions' immediate field");
@@ -222,6 +225,138 @@ __device__ __forceinline__ void p16_stage_c8(f32x4_t (&acc)[2][G::FN], half8_t (
     }
 }
 
+// The fp8 form on tiles whose fragments are rows of sixteen positions: two stages (chunks) as nine pairs of steps.  The
+// taps are walked column by column (kx outside, ky inside), so the fp16 fragment that output row r needs at tap row ky is
+// the one row r + 1 needed at ky - 1: a column reads TH + 2 fragments from LDS instead of 3 * TH, and with the fp8
+// operands (two reads per pair of steps and row) two chunks take 18 * TH + 6 * (TH + 2) reads instead of 36 * TH.
+// A pair's work on one output row is six MFMAs -- fp16 of its first step, fp8 of both, fp16 of its second, two channel
+// fragments each: 128 matrix-pipe cycles, a slot of the schedule.  A slot requests what the slot two further on takes
+// (a row's fp8 operands; the fp16 fragments that are new there) and its share of the weights LW pairs ahead.  Pair 4 has
+// a step in either chunk: all rows' fp16 MFMAs of its first step run first, behind the barrier that hands over the second
+// chunk (everything the pair takes of the first one has been read by then), the rest after them.  All indices are
+// compile-time constants once the loop is unrolled: the arrays are registers for as long as a value is needed.
+template <class G>
+struct RowsRing {
+    static constexpr int LA = 2;                       // slots from an LDS read to its use
+    static constexpr int LW = G::FN > 5 ? 1 : 2;       // pairs of steps from the request of weights to their use
+    half8_t a0[LW][2][2];                              // [pair][step][channel fragment]: fp16 weights
+    i32x8_t a2[LW][2];                                 // [pair][channel fragment]: fp8 weights of both steps
+    half8_t b0[LA];                                    // fp16 fragments of rows 0 .. of the first column
+    i32x8_t b8[LA];                                    // fp8 operands of rows 0 .. of the first pair
+};
+// The chunk a workgroup begins its tiles with: every second one begins two further on.  Workgroups start together and stay
+// in step, and a chunk is a quarter of a 512-byte pixel or less: all of them asking for the same quarter at the same time
+// is served slower than two (3x3 128 -> 128 at 480x270 with a residual: 72.7 -> 66.8 us; the two channel groups of the
+// sums are added in another order then).
+__device__ __forceinline__ int rows_first_chunk(int group, int nchunks) { return nchunks >= 4 && (group & 1) ? 2 : 0; }
+// f(0), f(1), ... f(N - 1) with the index as a type (the loops of a stage are expanded ahead of the optimiser, which takes
+// arrays indexed in loops this long to memory)
+template <class F, int... I>
+__device__ __forceinline__ void expand(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>()), ...);
+}
+template <class G>
+__device__ __forceinline__ void rows_load_b8(i32x8_t& dst, int half, const unsigned char* at) {
+    const i32x4_t v = *reinterpret_cast<const i32x4_t*>(at);
+    if (half == 0) { dst[0] = v[0]; dst[1] = v[1]; dst[2] = v[2]; dst[3] = v[3]; }
+    else { dst[4] = v[0]; dst[5] = v[1]; dst[6] = v[2]; dst[7] = v[3]; }
+}
+// weight k of a pair at offset w: 0..3 the fp16 fragments [step][channel fragment], 4..7 the fp8 halves
+__device__ __forceinline__ i32x4_t rows_load_w(const __amdgpu_buffer_rsrc_t weights, unsigned w, int k, unsigned wstep, unsigned wlane) {
+    const int step = (k / 2) % 2, fm = k % 2, plane = k < 4 ? 0 : 2;
+    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(i32x4_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights, wlane + (fm * NPLW + plane) * 1024, w + step * wstep, 0));
+}
+__device__ __forceinline__ void rows_put_w(half8_t (&a0)[2][2], i32x8_t (&a2)[2], int k, const i32x4_t v) {
+    const int step = (k / 2) % 2, fm = k % 2;
+    if (k < 4) a0[step][fm] = __builtin_bit_cast(half8_t, v);
+    else if (step == 0) { a2[fm][0] = v[0]; a2[fm][1] = v[1]; a2[fm][2] = v[2]; a2[fm][3] = v[3]; }
+    else { a2[fm][4] = v[0]; a2[fm][5] = v[1]; a2[fm][6] = v[2]; a2[fm][7] = v[3]; }
+}
+template <class G>
+__device__ __forceinline__ void p16_rows_c8(f32x4_t (&acc)[2][G::FN], RowsRing<G>& ring, const int (&base)[2], const unsigned char* lds,
+                                            const __amdgpu_buffer_rsrc_t weights, unsigned& wnext, unsigned wend, unsigned wstep, unsigned wlane) {
+    constexpr int TH = G::FN, LA = RowsRing<G>::LA, LW = RowsRing<G>::LW, NP = NT;   // (two chunks: nine pairs of steps)
+    constexpr int LB = 3;   // rows of pair 4 whose operands in the second chunk are read while its first step runs
+    static_assert(TH >= 4, "a slot has room for its share of the requests");
+    half8_t a0[NP + LW][2][2], b0[7][TH + 2];
+    i32x8_t a2[NP + LW][2], b8[NP + 1][TH];
+#pragma unroll
+    for (int d = 0; d < LW; d++)
+#pragma unroll
+        for (int fm = 0; fm < 2; fm++) {
+            a0[d][0][fm] = ring.a0[d][0][fm]; a0[d][1][fm] = ring.a0[d][1][fm];
+            a2[d][fm] = ring.a2[d][fm];
+        }
+#pragma unroll
+    for (int r = 0; r < LA; r++) { b0[0][r] = ring.b0[r]; b8[0][r] = ring.b8[r]; }
+    // column col (0 .. 5, three per chunk; 6: the first of the chunk that follows), row `row` of the staged tile
+    auto at = [&](int col, int row) { return lds + base[(col / 3) % 2] + (col % 3) * PITCH + row * G::ROW_PITCH; };
+    auto read_b0 = [&](int col, int row) { b0[col][row] = *reinterpret_cast<const half8_t*>(at(col, row)); };
+    auto read_b8 = [&](int p, int r, int half) {
+        const int s = 2 * p + half;
+        rows_load_b8<G>(b8[p][r], half, at(s / 3, r + s % 3) + G::PLANE);
+    };
+    // the n-th read for pair p, row r (not pair 4): both fp8 halves, then the fp16 fragments that no earlier row or step had
+    auto request = [&](int p, int r, int n) {
+        if (n < 2) { read_b8(p, r, n); return; }
+        const int s = 2 * p + n - 2;
+        if (n < 4) {
+            if (s % 3 == 0) read_b0(s / 3, r);
+            else if (r == TH - 1) read_b0(s / 3, TH - 1 + s % 3);
+        }
+    };
+    unsigned w_ = wnext;   // offset of the weights that the pair requests
+    auto slot = [&](auto index) __attribute__((always_inline)) {
+        constexpr int g = decltype(index)::value;
+        constexpr int blk = g / TH, r = g % TH, p = blk < 5 ? blk : blk - 1;   // (blocks 4 and 5: the two parts of pair 4)
+        constexpr int sa = 2 * p, sb = 2 * p + 1;
+        constexpr int u = g + LA, ublk = u / TH, ur = u % TH, up = ublk < 5 ? ublk : ublk - 1;   // the slot whose operands this one requests
+        if constexpr (r == 0 && blk != 5) {
+            w_ = wnext;
+            wnext += 2 * wstep;
+            if (wnext == wend) wnext = 0;
+        }
+        if constexpr (g == 4 * TH || g == (NP + 1) * TH - LA) lds_barrier();
+        constexpr int m0 = blk == 5 ? 2 : 0, m1 = blk == 4 ? 2 : 6;
+        auto issue = [&](auto index_m) __attribute__((always_inline)) {
+            constexpr int m = decltype(index_m)::value, fm = m % 2, n = m - m0;
+            if constexpr (m >= m0 && m < m1) {
+                if constexpr (m < 2) acc[fm][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[p][0][fm], b0[sa / 3][r + sa % 3], acc[fm][r], 0, 0, 0);
+                else if constexpr (m < 4) acc[fm][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a2[p][fm], b8[p][r], acc[fm][r], 0, 0, 0, 0, 0, 0);
+                else acc[fm][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[p][1][fm], b0[sb / 3][r + sb % 3], acc[fm][r], 0, 0, 0);
+                if constexpr (blk == 4) {
+                    if constexpr (r < LB && n == 0) read_b8(4, r, 1);
+                    if constexpr (r < LB && n == 1) read_b0(3, r);
+                } else if constexpr (ublk != 4 && ublk != 5) {
+                    request(up, ur, n);
+                }
+                if constexpr (blk == 5 && r + LB < TH && n == 0) read_b8(4, r + LB, 1);
+                if constexpr (blk == 5 && r + LB < TH && n == 1) read_b0(3, r + LB);
+                // (what pair 4 takes of the first chunk, ahead of the barrier by a slot)
+                if constexpr (g >= 3 * TH - 1 && g < 4 * TH - 1 && n == 4) read_b8(4, g - (3 * TH - 1), 0);
+                if constexpr (g == 4 * TH - 2 && n == 5) read_b0(2, TH + 1);
+                // a share of the eight weight loads of pair p + LW
+                constexpr int k = (r * 8 + TH - 1) / TH + (blk == 4 ? n : n - 2);
+                if constexpr (blk != 5 && (blk == 4 || n >= 2) && k < 8 && k * TH / 8 == r)
+                    rows_put_w(a0[p + LW], a2[p + LW], k, rows_load_w(weights, w_, k, wstep, wlane));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        expand(issue, std::make_integer_sequence<int, 6>());
+    };
+    expand(slot, std::make_integer_sequence<int, (NP + 1) * TH>());
+#pragma unroll
+    for (int d = 0; d < LW; d++)
+#pragma unroll
+        for (int fm = 0; fm < 2; fm++) {
+            ring.a0[d][0][fm] = a0[NP + d][0][fm]; ring.a0[d][1][fm] = a0[NP + d][1][fm];
+            ring.a2[d][fm] = a2[NP + d][fm];
+        }
+#pragma unroll
+    for (int r = 0; r < LA; r++) { ring.b0[r] = b0[6][r]; ring.b8[r] = b8[NP][r]; }
+}
+
 // The staging waves of a workgroup (threads 0..255): stage after stage -- a 32-channel chunk of a tile's halo: global
 // loads, activation, hi/lo conversion, LDS writes -- one stage ahead of the MFMA waves, across tile boundaries; scale and
 // bias at the start and, during a tile's last chunk, its residual tile.  One barrier per stage, after the one that hands
@@ -256,8 +391,10 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
     raw_t raw[2][G::NB];
     float in_scale = 1.f, inv_unused;
     // (unconditional loads: items outside the tensor read its first element and are zeroed when stored)
-    auto fetch = [&](auto set_, int tile, int chunk) {
+    const int first_chunk = (C8 && G::ROWS) ? rows_first_chunk(group, nchunks) : 0;
+    auto fetch = [&](auto set_, int tile, int stage) {
         constexpr int SET = decltype(set_)::value;
+        const int chunk = stage + first_chunk < nchunks ? stage + first_chunk : stage + first_chunk - nchunks;
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
         const int y0 = tyi * G::TH * G::STEP + p.in_y0, x0 = txi * G::TWG * G::STEP + p.in_x0;
 #pragma unroll
@@ -320,23 +457,39 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
             else split_all(std::integral_constant<int, ACT_LEAKY>());
         }
     };
-    auto residual_in = [&](int tile) {   // the residual tile of a tile: [position][CPB channels] as stored, in 16-byte pieces
+    // The residual tile of a tile: [position][CPB channels] as stored, in 16-byte pieces.  They are spread over the tile's
+    // chunks but the first (the MFMA waves may still be reading the tile before until that is through), and a chunk's share
+    // is requested before the next stage is converted and written behind it: all of it in the last chunk is a burst that all
+    // workgroups ask for at the same time (3x3 128 -> 128 at 480x270, 8x16 tiles: 69 -> 65 us; 57 without a residual)
+    constexpr int RSH = 4, RSHARES = (G::RNB + RSH - 1) / RSH;   // pieces of a share, shares
+    f32x4_t rv[RSHARES * RSH];
+    auto residual_due = [&](int share, int c) { return nchunks < 2 || share * (nchunks - 1) / RSHARES == c - 1; };
+    auto residual_request = [&](int tile, int c) {
         const store_t* res = reinterpret_cast<const store_t*>(p.res);
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
-        f32x4_t rv[G::RNB];
 #pragma unroll
-        for (int i = 0; i < G::RNB; i++) {
-            const int idx = stid + i * 256;
-            const int m = idx / G::RPP, piece = idx % G::RPP;
-            const int ty = m / G::TWG, tx = m - ty * G::TWG;
-            const int py = tyi * G::TH + ty, px = txi * G::TWG + tx;
-            const bool ok = idx < G::RPIECES && py < p.npos_y && px < p.npos_x && cb * CPB + piece * (16 / ESZ) < p.res_cp;
-            rv[i] = *reinterpret_cast<const f32x4_t*>(res + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + cb * CPB + piece * (16 / ESZ) : 0));
+        for (int share = 0; share < RSHARES; share++) {
+            if (!residual_due(share, c)) continue;
+#pragma unroll
+            for (int i = share * RSH; i < (share + 1) * RSH; i++) {
+                const int idx = stid + i * 256;
+                const int m = idx / G::RPP, piece = idx % G::RPP;
+                const int ty = m / G::TWG, tx = m - ty * G::TWG;
+                const int py = tyi * G::TH + ty, px = txi * G::TWG + tx;
+                const bool ok = idx < G::RPIECES && py < p.npos_y && px < p.npos_x && cb * CPB + piece * (16 / ESZ) < p.res_cp;
+                rv[i] = *reinterpret_cast<const f32x4_t*>(res + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + cb * CPB + piece * (16 / ESZ) : 0));
+            }
         }
+    };
+    auto residual_store = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < G::RNB; i++) {
-            const int idx = stid + i * 256;
-            if (idx < G::RPIECES) *reinterpret_cast<f32x4_t*>(lds + res_off + (idx / G::RPP) * G::RES_PITCH + (idx % G::RPP) * 16) = rv[i];
+        for (int share = 0; share < RSHARES; share++) {
+            if (!residual_due(share, c)) continue;
+#pragma unroll
+            for (int i = share * RSH; i < (share + 1) * RSH; i++) {
+                const int idx = stid + i * 256;
+                if (idx < G::RPIECES) *reinterpret_cast<f32x4_t*>(lds + res_off + (idx / G::RPP) * G::RES_PITCH + (idx % G::RPP) * 16) = rv[i];
+            }
         }
     };
     // the stage after (tile, c); false: there is none
@@ -366,8 +519,9 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
     // One iteration per stage n of the MFMA waves: stage n+1 (fetched an iteration ago) is written to the other
     // buffer, then stage n+2 is fetched into the registers that stage n left.  Unrolled by two: set = parity of the stage.
     auto iteration = [&](auto next_set, auto free_set, unsigned char* next_buf) {
-        if (c + 1 == nchunks && p.res) residual_in(tile);
+        if (p.res) residual_request(tile, c);
         if (have1) store(next_set, next_buf);
+        if (p.res) residual_store(c);
         if (have2) fetch(free_set, t2, c2);
         lds_barrier();
         const bool go_on = have1;
@@ -436,10 +590,18 @@ __global__ __launch_bounds__(512) void conv_p16_kernel(const ConvP16Params p) {
     const unsigned char* wbase = reinterpret_cast<const unsigned char*>(p.wpack) + (size_t)((cb * 2 * WM + mw * 2) * NPLW) * 1024;   // (uniform: the loads take it as their scalar base)
     const unsigned wlane = lane * 16;
     const unsigned char* wend = wbase + (size_t)nchunks * NT * wstep;
+    constexpr bool RC8 = C8 && G::ROWS;
     half8_t a_q[C8 ? 1 : PD][2][NPL];   // exact form: hi and lo weights of a step
     half8_t a0[C8 ? PD : 1][2];         // fp8 form: hi weights of a step ...
     i32x8_t a2[C8 ? PD / 2 : 1][2];     // ... and the fp8 weights of a pair of steps
-    if constexpr (C8) {
+    typename std::conditional<RC8, RowsRing<G>, int>::type ring;   // (fp8 form on rows)
+    const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(wbase), 0, (int)((unsigned)(nchunks * NT) * wstep), 0x00020000);
+    if constexpr (RC8) {
+#pragma unroll
+        for (int d = 0; d < RowsRing<G>::LW; d++)
+#pragma unroll
+            for (int k = 0; k < 8; k++) rows_put_w(ring.a0[d], ring.a2[d], k, rows_load_w(weights, (rows_first_chunk(group, nchunks) * NT + 2 * d) * wstep, k, wstep, wlane));
+    } else if constexpr (C8) {
 #pragma unroll
         for (int d = 0; d < PD; d++)
 #pragma unroll
@@ -542,7 +704,14 @@ __global__ __launch_bounds__(512) void conv_p16_kernel(const ConvP16Params p) {
     half8_t b[C8 ? 1 : FN][NPL];
     half8_t b0[C8 ? FN : 1];
     i32x8_t b1[C8 ? FN : 1];
-    if constexpr (C8) {
+    if constexpr (RC8) {
+#pragma unroll
+        for (int r = 0; r < RowsRing<G>::LA; r++) {
+            ring.b0[r] = *reinterpret_cast<const half8_t*>(lds + bbase[0][r]);
+            rows_load_b8<G>(ring.b8[r], 0, lds + bbase[0][r] + G::PLANE);
+            rows_load_b8<G>(ring.b8[r], 1, lds + bbase[0][r] + G::ROW_PITCH + G::PLANE);
+        }
+    } else if constexpr (C8) {
 #pragma unroll
         for (int fn = 0; fn < FN; fn++) {
             b0[fn] = *reinterpret_cast<const half8_t*>(lds + bbase[0][fn]);
@@ -559,7 +728,20 @@ __global__ __launch_bounds__(512) void conv_p16_kernel(const ConvP16Params p) {
 
     const unsigned char* wnext = wbase + (size_t)((PD - 1) % (nchunks * NT)) * wstep;
     int tile = group, c = 0;
-    if constexpr (C8) {
+    if constexpr (RC8) {
+        const int base[2] = {bbase[0][0], bbase[1][0]};
+        unsigned wend = (unsigned)(nchunks * NT) * wstep, wnext8 = (rows_first_chunk(group, nchunks) * NT + 2 * RowsRing<G>::LW) * wstep;
+        for (;;) {
+            p16_rows_c8<G>(acc, ring, base, lds, weights, wnext8, wend, wstep, wlane);
+            c += 2;
+            if (c == nchunks) {
+                finish_tile(tile);
+                c = 0; tile += p.pos_groups;
+                if (tile >= ntiles) break;
+                zero_acc();
+            }
+        }
+    } else if constexpr (C8) {
         // (an even number of chunks: a tile is whole pairs of stages)
         for (;;) {
             p16_stage_c8<G, 0>(acc, a0, a2, b0, b1, bbase, lds, wnext, wbase, wend, wstep, wlane);
@@ -1754,6 +1936,7 @@ constexpr P16Entry entry() {
 const P16Entry kEntries[] = {
     entry<8, 10, 1, 4>(), entry<10, 8, 1, 4>(), entry<8, 8, 1, 4>(), entry<8, 6, 1, 4>(), entry<4, 8, 1, 4>(), entry<4, 4, 1, 4>(),
     entry<8, 8, 1, 2>(), entry<8, 6, 1, 2>(), entry<4, 8, 1, 2>(),
+    entry<8, 16, 1, 4>(), entry<6, 16, 1, 4>(), entry<5, 16, 1, 4>(), entry<4, 16, 1, 4>(), entry<6, 16, 1, 2>(), entry<4, 16, 1, 2>(),
     entry<10, 8, 2, 4>(), entry<8, 10, 2, 4>(), entry<8, 8, 2, 4>(),
     entry<8, 6, 2, 2>(), entry<4, 8, 2, 2>(), entry<8, 4, 2, 2>(),
 };

@@ -172,13 +172,14 @@ class ConvLayer : public Layer {
             if (res_v && c.cin_chunks < 2) c.pos_groups = c.tiles_x * c.tiles_y;   // (residual tile: one stage per tile is too few to walk)
             const size_t lds = conv_p16_lds_bytes(c);
             if (lds == 0 || lds > 160 * 1024) continue;
+            if (tw == 16 && !conv_p16_uses_fp8(c) && !want_h) continue;   // (rows of sixteen positions pay in the fp8 form's schedule)
             // (a workgroup's eight waves take 140-240 registers each: one workgroup per CU whatever its LDS share)
             const int rounds = (c.tiles_x * c.tiles_y * c.cout_blocks + 255) / 256;
             cands.push_back(Cand{(double)rounds * (th * tw + 8) + 16, c});   // (+8: a tile's fixed part, +16: the launch's, in positions)
         }
         if (cands.empty()) return;
         std::sort(cands.begin(), cands.end(), [](const Cand& a, const Cand& b) { return a.cost < b.cost; });
-        if (cands.size() > 3) cands.resize(3);
+        if (cands.size() > 4) cands.resize(4);
         const size_t halves = ((size_t)q.cin_chunks * 9 + 8) * q.mfrags * (q.f16 ? 1 : 3) * 64 * 8;
         p16_wpack_dev = net->dev_alloc(halves * 2, true);
         for (Cand& c : cands) c.q.wpack = p16_wpack_dev;
@@ -916,7 +917,8 @@ class ConvLayer : public Layer {
             }
         upload_p16_pack(net, p16_wpack_dev, pack, c8, frags);
     }
-    // weights of that form: [(chunk*9 + tap)][cout fragment of 16][plane][lane][8 halves], zero steps behind the last
+    // weights of that form: [(chunk*9 + tap)][cout fragment of 16][plane][lane][8 halves], zero steps behind the last; taps
+    // row by row, or column by column for tiles whose fragments are rows of sixteen positions
     void pack_p16(const float* w, float wmul) {
         const int cin = d.in_channels;
         const int npl = pp.f16 ? 1 : 3;   // fp32 tensors: hi, lo, and the fp8 operands of the correction terms
@@ -927,6 +929,7 @@ class ConvLayer : public Layer {
             for (int tap = 0; tap < 9; tap++)
                 for (int mf = 0; mf < pp.mfrags; mf++) {
                     const size_t frag = (size_t)(chunk * 9 + tap) * pp.mfrags + mf;
+                    const int at = pp.tile_w == 16 ? tap % 3 * 3 + tap / 3 : tap;
                     uint16_t* base = pack.data() + frag * npl * 64 * 8;
                     for (int lane = 0; lane < 64; lane++) {
                         const int o = p16_row_channel(mf, lane & 15, pp.f16 ? 2 : 1);
@@ -934,7 +937,7 @@ class ConvLayer : public Layer {
                         for (int j = 0; j < 8; j++) {
                             const int ci = chunk * 32 + 8 * (lane >> 4) + j;
                             if (ci >= cin) continue;
-                            const float v = w[(((size_t)o * 3 + tap / 3) * 3 + tap % 3) * cin + ci] * wmul;
+                            const float v = w[((size_t)o * 9 + at) * cin + ci] * wmul;
                             const uint16_t hi = f2h_bits(v);
                             base[(size_t)lane * 8 + j] = hi;
                             if (npl == 3) p16_lo_planes(base, c8.data() + (frag * 64 + lane) * 16, lane, j, v, hi);

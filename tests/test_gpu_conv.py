@@ -348,6 +348,51 @@ def test_sixteen_position_fragment_form(case, act, shallow, storage, monkeypatch
         assert rel_l2(got, exact) <= 3e-5
 
 
+P16_ROW_CASES = [
+    # (cin, cout, h, w, tile "rows,16,channel groups", kw): tiles whose fragments are rows of sixteen positions
+    (64, 128, 5, 16, "5,16,4", {}),                                              # one whole tile, one pair of chunks
+    (128, 128, 37, 50, "5,16,4", {"bn": True, "residual": (A.RELU, True)}),      # ragged in both directions
+    (128, 128, 9, 17, "8,16,4", {"residual": (A.NONE, False)}),                  # a row and a column behind the last whole tile
+    (64, 128, 130, 300, "8,16,4", {"bn": True}),                                 # 323 tiles: workgroups walk two
+    (40, 40, 23, 41, "4,16,2", {"residual": (A.RELU, False)}),                   # a ragged second chunk, a ragged block of output channels
+    (64, 64, 19, 65, "4,16,2", {"pad_out": 1}),
+    (64, 72, 13, 31, "6,16,2", {"bn": True}),                                    # two blocks of output channels, the second holds 8
+    (256, 128, 7, 20, "6,16,4", {"residual": (A.RELU, False)}),                  # eight chunks; every second workgroup begins with the third
+    (192, 128, 40, 33, "4,16,4", {"bn": True}),                                  # six
+    (128, 256, 3, 15, "4,16,4", {"residual": (A.NONE, True)}),                   # fewer rows and columns than a tile has
+]
+
+
+@pytest.mark.parametrize("case", P16_ROW_CASES, ids=lambda c: "%dx%dx%d_to%d_%s" % (c[0], c[2], c[3], c[1], c[4].replace(",", "x")))
+@pytest.mark.parametrize("shallow", [False, True], ids=["deep", "shallow"])
+def test_fp8_form_on_rows_of_sixteen_positions(case, shallow, monkeypatch):
+    """The fp8 form of the correction terms on tiles whose fragments are rows: every compiled tile, edges, tile walking, ragged
+    channels; against the oracle, and against three fp16 passes over the same tiles."""
+    cin, cout, h, w, tile, kw = case
+    if shallow:
+        if "residual" in kw or "pad_out" in kw:
+            pytest.skip("the shallow variant is run on the plain cases")
+        kw = dict(kw, deep=False, pad_in=0)
+    monkeypatch.setenv("FYNHIP_FORCE_P16_CONV", "1")
+    monkeypatch.setenv("FYNHIP_P16_TILE", tile)
+    wts = conv_block(1700 + cin + h, cout, 3, cin, bn=kw.get("bn", False))
+    inputs = [prng.uniform(31 * cin + w, (cin, h, w), -1, 1)]
+    if "residual" in kw:
+        inputs.append(prng.uniform(67, (cout, h, w), -1, 1))
+    b = conv_builder(3, cout, h, w, cin, 1, 1, A.RELU, **kw)
+    got, info = run_single(b, fa.STORAGE_F32, inputs, wts)
+    ref = oracle_single(b, fa.STORAGE_F32, inputs, wts)
+    print("  ", info, "rel_l2=%.3e" % rel_l2(got, ref), flush=True)
+    th, tw, wm = tile.split(",")
+    assert "conv_p16 f16+fp8-split" in info and "waves=%sx" % wm in info and "th=%s tw=%s" % (th, tw) in info
+    monkeypatch.setenv("FYNHIP_EXACT_SPLIT", "1")
+    exact, info = run_single(conv_builder(3, cout, h, w, cin, 1, 1, A.RELU, **kw), fa.STORAGE_F32, inputs, wts)
+    assert "conv_p16 f16x2-split" in info and "th=%s tw=%s" % (th, tw) in info
+    # (three passes over 22-bit operands; the correction terms, 2^-11 of the result, carry four bits: the bounds of the other tiles)
+    assert rel_l2(exact, ref) <= 2e-6
+    assert rel_l2(got, exact) <= 3e-5
+
+
 H16_CASES = [
     # (k, cin, cout, h, w, tile "h,w", kw)
     (9, 64, 128, 30, 40, "12,8", {}),                                              # two chunks, ragged in both directions
