@@ -800,7 +800,7 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
     const size_t npix = include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, bytes = npix * v.c * sizeof(float);
     if (!host_memory(out)) {
         float* st = staging(npix * v.c);
-        launch_tensor_to_chw(v, st, npix, include_padding, 0, npix, HostDone{}, stream);
+        launch_tensor_to_chw(v, st, npix, include_padding, 0, npix, HostDone{}, true, stream);
         check_queued();
         FYN_HIP(hipMemcpyAsync(out, st, bytes, hipMemcpyDefault, stream));
         FYN_HIP(hipStreamSynchronize(stream));
@@ -808,7 +808,7 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
     }
     if (HostPool::contains(out, bytes)) {
         const HostDone done = signal_.next();
-        launch_tensor_to_chw(v, out, npix, include_padding, 0, npix, done, stream);
+        launch_tensor_to_chw(v, out, npix, include_padding, 0, npix, done, false, stream);
         check_queued();
         signal_.wait(done.value, stream);
         return;
@@ -820,7 +820,7 @@ void Net::download_planes(const TView& v, int include_padding, float* out) {
     const unsigned first = signal_.last() + 1;
     for (size_t p0 = 0; p0 < npix; p0 += step) {
         const HostDone done = signal_.next();
-        launch_tensor_to_chw(v, st, plane, include_padding, p0, std::min(npix, p0 + step), done, stream);
+        launch_tensor_to_chw(v, st, plane, include_padding, p0, std::min(npix, p0 + step), done, false, stream);
         loan.used_until(signal_, done.value);
     }
     check_queued();
@@ -845,7 +845,7 @@ void Net::download_pixels(const TView& v, int pc, float* out) {
     const unsigned first = signal_.last() + 1;
     for (size_t p0 = 0; p0 < npix; p0 += step) {
         const HostDone done = signal_.next();
-        launch_tensor_to_hwc(v, st, pc, p0, std::min(npix, p0 + step), done, stream);
+        launch_tensor_to_hwc(v, st, pc, p0, std::min(npix, p0 + step), done, false, stream);
         loan.used_until(signal_, done.value);
     }
     check_queued();
@@ -898,7 +898,7 @@ void Net::copy_result_static(int layer_no, float* chw, int include_padding) {
              l->d.name, l->d.number, n, (size_t)FYN_STATIC_SCRATCH_FLOATS);
     // every element of [0, n) is written by the conversion kernel: nothing of an earlier call is read
     launch_tensor_to_chw(v, static_scratch_, include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, include_padding, 0,
-                         include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, HostDone{}, stream);
+                         include_padding ? (size_t)v.hp() * v.wp() : (size_t)v.h * v.w, HostDone{}, true, stream);
     FYN_HIP(hipGetLastError());
     FYN_HIP(hipMemcpyAsync(chw, static_scratch_, n * sizeof(float), hipMemcpyDefault, stream));
     FYN_HIP(hipStreamSynchronize(stream));
@@ -1173,8 +1173,8 @@ void Net::queue_frame(AsyncSlot& s) {
     else launch_hwc_to_tensor(src, vi, range, HostFeed{}, HostDone{}, async_own_streams_, stream);
     forward(nullptr);
     const HostDone done = signal_.next();
-    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, dst, opix, 0, 0, opix, done, stream);
-    else launch_tensor_to_hwc(vo, dst, vo.c == 3 ? 4 : vo.c, 0, opix, done, stream);
+    if (async_out_order_ == FYN_ORDER_CHANNELWISE) launch_tensor_to_chw(vo, dst, opix, 0, 0, opix, done, async_own_streams_, stream);
+    else launch_tensor_to_hwc(vo, dst, vo.c == 3 ? 4 : vo.c, 0, opix, done, async_own_streams_, stream);
     FYN_HIP(hipGetLastError());
     s.value = done.value;
 }

@@ -527,13 +527,13 @@ struct UploadRange {
     unsigned* record;
     unsigned* words;
 };
-// Layout conversion between tensors and fp32 buffers in page-locked host memory or (device: more workgroups pay) device
+// Layout conversion between tensors and fp32 buffers in page-locked host memory or (device: other workgroups pay) device
 // memory (layout.hip); downloads: pixels [p0, p1) of the area.
 // (planes: multiples of four floats; with a feed word of 32, the buffer on a 128-byte boundary: no line is read before all of it is there)
 void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s);   // net area only
 void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s);   // GPU_SHALLOW in
-void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s);
-void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s);   // GPU_SHALLOW out, pc = 1, 2 or 4
+void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, bool device, hipStream_t s);
+void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, bool device, hipStream_t s);   // GPU_SHALLOW out, pc = 1, 2 or 4
 void launch_argmax_to_host(const int* idx, const TView& t, int* idx_out, float* val_out, size_t p0, size_t p1, const HostDone& done, hipStream_t s);
 void launch_await_feed(const HostFeed& feed, size_t npix, hipStream_t s);   // holds the stream until the frame is there (one workgroup looks, not those of a whole conversion)
 void launch_tell_host(const HostDone& done, hipStream_t s);

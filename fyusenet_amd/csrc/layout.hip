@@ -19,14 +19,19 @@ namespace fynhip {
 
 namespace {
 constexpr unsigned kMaxBlocks = 128;          // buffers behind the link
-constexpr unsigned kMaxDeviceBlocks = 1024;   // buffers in device memory: 3.8 MB of pixels in 4 us instead of 11
+// Buffers in device memory: few workgroups of 1024 threads.  At a launch's end its workgroups meet in one word (the value range
+// of what was uploaded, the host's word), one after the other (15 ns each, twice): 936 workgroups of 256 threads took 26.5
+// us for 3.8 MB of interleaved pixels, 78 of 1024 take 8; the result's 5 MB 10 -> 8.6.  A stream of 512x624 frames through
+// the sample's style net 2897 -> 2663 us for twelve.
+constexpr unsigned kMaxDeviceBlocks = 128;
+constexpr int kDeviceThreads = 1024;
 // Frames from the host: the workgroups keep pace with the host's copy, and each one's looks at its progress (HostFeed) and
 // its arrival at the end cost the others time.  A segmentation frame (3.7 MB) from call to launch complete, with 24, 32,
 // 40, 48, 64 and 80 workgroups: 106, 98, 92, 93, 96, 97 us (111 with 128 that ended with a fence each); 25 MB: 566, 492,
 // 489, 490, 497, 534.  (Two sizes, one host with a 55 GB/s link: elsewhere the number is a guess; what depends on it is how
 // close to the link's rate an upload runs, not what arrives.)
 constexpr unsigned kMaxUploadBlocks = 48;
-unsigned upload_blocks(size_t items, bool device) { return (unsigned)std::min<size_t>(device ? kMaxDeviceBlocks : kMaxUploadBlocks, (items + 255) / 256); }
+unsigned blocks_for(size_t items, unsigned most, int threads) { return (unsigned)std::min<size_t>(most, (items + threads - 1) / threads); }
 
 // The host may still be copying the frame when the launch runs (HostFeed): before a workgroup reads pixels it looks, where
 // it has to, whether they are there.  The launch's own latency (8 us) and the host's copy then overlap the transfer
@@ -64,16 +69,18 @@ __device__ __forceinline__ void await_feed(const HostFeed& f, unsigned need, uns
 // The value range of an uploaded tensor.  Its record is written, not raised, so that no launch has to clear it first: the
 // workgroups meet in a word of the network's (device scope: they sit on different XCDs), and the one that arrives last
 // moves the maximum into the record and leaves the words as they were found.
+template <int NT>
 __device__ __forceinline__ void publish_range(const UploadRange& u, float m) {
     if (!u.record) return;
-    __shared__ float wave_max[4];
+    __shared__ float wave_max[NT / 64];
     __shared__ unsigned last;
     m = range_wave_max(m);
     if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        (void)__hip_atomic_fetch_max(&u.words[0], __float_as_uint(fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]))), __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int w = 0; w < NT / 64; w++) m = fmaxf(m, wave_max[w]);
+        (void)__hip_atomic_fetch_max(&u.words[0], __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the maximum has been taken before the arrival counts)
         unsigned all = 0u;
         if (__hip_atomic_fetch_add(&u.words[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
@@ -141,15 +148,15 @@ __device__ __forceinline__ void store4(T* p, float a, float b, float c, float d)
 
 // Planes `plane` floats apart (a multiple of four, as is the planes' address in units of four floats): a thread takes four
 // pixels of four channels.  Channels beyond the tensor's read as zero.
-template <typename T>
-__global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, const UploadRange range, const HostFeed feed, const HostDone done) {
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void chw_to_tensor_kernel(const float* chw, size_t plane, const TView t, const UploadRange range, const HostFeed feed, const HostDone done) {
     const unsigned npix = (unsigned)t.h * t.w, quads = (npix + 3) >> 2;
     const size_t n = (size_t)quads * (t.cp >> 2);
     float vmax = 0.f;
     unsigned seen = 0;
-    for (size_t i0 = (size_t)blockIdx.x * 256; i0 < n; i0 += (size_t)gridDim.x * 256) {
+    for (size_t i0 = (size_t)blockIdx.x * NT; i0 < n; i0 += (size_t)gridDim.x * NT) {
         const unsigned q0 = (unsigned)(i0 % quads);
-        await_feed(feed, q0 + 256 >= quads ? npix : (q0 + 256) * 4, seen);
+        await_feed(feed, q0 + NT >= quads ? npix : (q0 + NT) * 4, seen);
         const size_t i = i0 + threadIdx.x;
         if (i >= n) break;
         const unsigned pix = (unsigned)(i % quads) * 4;
@@ -175,25 +182,30 @@ __global__ __launch_bounds__(256) void chw_to_tensor_kernel(const float* chw, si
             }
         }
     }
-    publish_range(range, vmax);
+    publish_range<NT>(range, vmax);
     tell_host_read(done);
 }
 void launch_chw_to_tensor(const float* chw, size_t plane, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s) {
-    const dim3 grid(upload_blocks(((size_t)t.h * t.w + 3) / 4 * (t.cp >> 2), device));
-    if (t.f16) hipLaunchKernelGGL(chw_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, chw, plane, t, range, feed, done);
-    else hipLaunchKernelGGL(chw_to_tensor_kernel<float>, grid, dim3(256), 0, s, chw, plane, t, range, feed, done);
+    const size_t items = ((size_t)t.h * t.w + 3) / 4 * (t.cp >> 2);
+    auto go = [&](auto kernel, unsigned most, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(blocks_for(items, most, threads)), dim3(threads), 0, s, chw, plane, t, range, feed, done);
+    };
+    if (device && t.f16) go(chw_to_tensor_kernel<_Float16, kDeviceThreads>, kMaxDeviceBlocks, kDeviceThreads);
+    else if (device) go(chw_to_tensor_kernel<float, kDeviceThreads>, kMaxDeviceBlocks, kDeviceThreads);
+    else if (t.f16) go(chw_to_tensor_kernel<_Float16, 256>, kMaxUploadBlocks, 256);
+    else go(chw_to_tensor_kernel<float, 256>, kMaxUploadBlocks, 256);
 }
 
 // Interleaved pixels of t.c floats: the buffer is read as one run of sixteen-byte pieces (an element's pixel and channel
 // follow from its index), the tensor's pad channels keep the zeros they were allocated with.  The last piece may reach
 // up to three floats behind the buffer's end.
-template <typename T>
-__global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, const TView t, const UploadRange range, const HostFeed feed, const HostDone done) {
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void hwc_to_tensor_kernel(const float* hwc, const TView t, const UploadRange range, const HostFeed feed, const HostDone done) {
     const size_t npix = (size_t)t.h * t.w, e1 = npix * t.c, q1 = (e1 + 3) >> 2;
     float vmax = 0.f;
     unsigned seen = 0;
-    for (size_t q0 = (size_t)blockIdx.x * 256; q0 < q1; q0 += (size_t)gridDim.x * 256) {
-        await_feed(feed, q0 + 256 >= q1 ? (unsigned)npix : (unsigned)((q0 + 256) * 4 / t.c + 1), seen);
+    for (size_t q0 = (size_t)blockIdx.x * NT; q0 < q1; q0 += (size_t)gridDim.x * NT) {
+        await_feed(feed, q0 + NT >= q1 ? (unsigned)npix : (unsigned)((q0 + NT) * 4 / t.c + 1), seen);
         const size_t q = q0 + threadIdx.x;
         if (q >= q1) break;
         const float4 v = *reinterpret_cast<const float4*>(hwc + q * 4);
@@ -215,25 +227,65 @@ __global__ __launch_bounds__(256) void hwc_to_tensor_kernel(const float* hwc, co
             }
         }
     }
-    publish_range(range, vmax);
+    publish_range<NT>(range, vmax);
+    tell_host_read(done);
+}
+// The same for images of three channels in device memory: a thread takes four pixels, three loads and four whole-pixel
+// stores of sixteen bytes (fp32 tensors), instead of one load and four stores of a channel each.
+template <typename T>
+__global__ __launch_bounds__(kDeviceThreads) void hwc3_to_tensor_kernel(const float* hwc, const TView t, const UploadRange range, const HostDone done) {
+    const unsigned npix = (unsigned)t.h * t.w, quads = (npix + 3) >> 2;
+    float vmax = 0.f;
+    for (unsigned q = blockIdx.x * kDeviceThreads + threadIdx.x; q < quads; q += gridDim.x * kDeviceThreads) {
+        float e[12];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            // (the last pixels' piece: no further behind the buffer's end than the kernel above reads)
+            const bool there = (size_t)q * 12 + k * 4 < (size_t)npix * 3;
+            const float4 v = there ? *reinterpret_cast<const float4*>(hwc + (size_t)q * 12 + k * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+            e[4 * k] = v.x; e[4 * k + 1] = v.y; e[4 * k + 2] = v.z; e[4 * k + 3] = v.w;
+        }
+        unsigned y = q * 4 / (unsigned)t.w, x = q * 4 - y * (unsigned)t.w;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (q * 4 + j < npix) {
+                store4<T>(reinterpret_cast<T*>(t.ptr) + ((size_t)(y + t.pad) * t.wp() + x + t.pad) * 4, e[3 * j], e[3 * j + 1], e[3 * j + 2], 0.f);
+                vmax = fmaxf(fmaxf(vmax, fabsf(e[3 * j])), fmaxf(fabsf(e[3 * j + 1]), fabsf(e[3 * j + 2])));
+            }
+            if (++x == (unsigned)t.w) {
+                x = 0;
+                y++;
+            }
+        }
+    }
+    publish_range<kDeviceThreads>(range, vmax);
     tell_host_read(done);
 }
 void launch_hwc_to_tensor(const float* hwc, const TView& t, const UploadRange& range, const HostFeed& feed, const HostDone& done, bool device, hipStream_t s) {
-    const dim3 grid(upload_blocks(((size_t)t.h * t.w * t.c + 3) / 4, device));
-    if (t.f16) hipLaunchKernelGGL(hwc_to_tensor_kernel<_Float16>, grid, dim3(256), 0, s, hwc, t, range, feed, done);
-    else hipLaunchKernelGGL(hwc_to_tensor_kernel<float>, grid, dim3(256), 0, s, hwc, t, range, feed, done);
+    const size_t items = ((size_t)t.h * t.w * t.c + 3) / 4;
+    auto go = [&](auto kernel, unsigned most, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(blocks_for(items, most, threads)), dim3(threads), 0, s, hwc, t, range, feed, done);
+    };
+    if (device && t.c == 3 && t.cp == 4) {
+        const dim3 grid(blocks_for(((size_t)t.h * t.w + 3) / 4, kMaxDeviceBlocks, kDeviceThreads));
+        if (t.f16) hipLaunchKernelGGL(hwc3_to_tensor_kernel<_Float16>, grid, dim3(kDeviceThreads), 0, s, hwc, t, range, done);
+        else hipLaunchKernelGGL(hwc3_to_tensor_kernel<float>, grid, dim3(kDeviceThreads), 0, s, hwc, t, range, done);
+    } else if (device && t.f16) go(hwc_to_tensor_kernel<_Float16, kDeviceThreads>, kMaxDeviceBlocks, kDeviceThreads);
+    else if (device) go(hwc_to_tensor_kernel<float, kDeviceThreads>, kMaxDeviceBlocks, kDeviceThreads);
+    else if (t.f16) go(hwc_to_tensor_kernel<_Float16, 256>, kMaxUploadBlocks, 256);
+    else go(hwc_to_tensor_kernel<float, 256>, kMaxUploadBlocks, 256);
 }
 
 // Pixels [p0, p1) of the net area (keep_pad: of the area with its halo) to planes `plane` floats apart.  Q = 4: a thread
 // takes four pixels of four channels, planes on sixteen-byte boundaries (p0 a multiple of four, the last piece may
 // reach up to three floats behind a plane); Q = 1: one pixel of four channels, any planes.
 template <typename T, int Q>
-__global__ __launch_bounds__(256) void tensor_to_chw_kernel(const TView t, float* chw, size_t plane, int keep_pad, unsigned p0, unsigned p1, const HostDone done) {
+__global__ __launch_bounds__(kDeviceThreads) void tensor_to_chw_kernel(const TView t, float* chw, size_t plane, int keep_pad, unsigned p0, unsigned p1, const HostDone done) {
     const unsigned ow = (unsigned)(keep_pad ? t.wp() : t.w);
     const int off = keep_pad ? 0 : t.pad;
     const unsigned groups = (p1 - p0 + Q - 1) / Q;
     const size_t n = (size_t)groups * ((t.c + 3) >> 2);
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         const unsigned pix = p0 + (unsigned)(i % groups) * Q;
         const int c = (int)(i / groups) * 4;
         unsigned y = pix / ow, x = pix - y * ow;
@@ -289,7 +341,7 @@ __global__ __launch_bounds__(256) void tensor_to_run_kernel(const TView t, float
     }
     tell_host(done);
 }
-void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
+void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_padding, size_t p0, size_t p1, const HostDone& done, bool device, hipStream_t s) {
     const size_t npix = include_padding ? (size_t)t.hp() * t.wp() : (size_t)t.h * t.w;
     if (plane == npix && p0 == 0 && p1 == npix && (plane % 4 != 0 || plane < 256) && (reinterpret_cast<size_t>(chw) & 15) == 0 && t.c > 1) {
         const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, ((npix * t.c + 3) / 4 + 255) / 256));
@@ -299,21 +351,22 @@ void launch_tensor_to_chw(const TView& t, float* chw, size_t plane, int include_
     }
     const bool quad = plane % 4 == 0 && (reinterpret_cast<size_t>(chw) & 15) == 0 && p0 % 4 == 0;
     const size_t items = (p1 - p0 + (quad ? 3 : 0)) / (quad ? 4 : 1) * ((t.c + 3) >> 2);
-    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (items + 255) / 256));
+    const int threads = device ? kDeviceThreads : 256;
+    const dim3 grid(blocks_for(items, device ? kMaxDeviceBlocks : kMaxBlocks, threads));
     const unsigned a = (unsigned)p0, b = (unsigned)p1;
     if (t.f16) {
-        if (quad) hipLaunchKernelGGL((tensor_to_chw_kernel<_Float16, 4>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
-        else hipLaunchKernelGGL((tensor_to_chw_kernel<_Float16, 1>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
+        if (quad) hipLaunchKernelGGL((tensor_to_chw_kernel<_Float16, 4>), grid, dim3(threads), 0, s, t, chw, plane, include_padding, a, b, done);
+        else hipLaunchKernelGGL((tensor_to_chw_kernel<_Float16, 1>), grid, dim3(threads), 0, s, t, chw, plane, include_padding, a, b, done);
     } else {
-        if (quad) hipLaunchKernelGGL((tensor_to_chw_kernel<float, 4>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
-        else hipLaunchKernelGGL((tensor_to_chw_kernel<float, 1>), grid, dim3(256), 0, s, t, chw, plane, include_padding, a, b, done);
+        if (quad) hipLaunchKernelGGL((tensor_to_chw_kernel<float, 4>), grid, dim3(threads), 0, s, t, chw, plane, include_padding, a, b, done);
+        else hipLaunchKernelGGL((tensor_to_chw_kernel<float, 1>), grid, dim3(threads), 0, s, t, chw, plane, include_padding, a, b, done);
     }
 }
 
 // Interleaved pixels of PC = 1, 2 or 4 floats: a pixel per thread, one store each.
 template <typename T, int PC>
-__global__ __launch_bounds__(256) void tensor_to_hwc_kernel(const TView t, float* hwc, size_t p0, size_t p1, const HostDone done) {
-    for (size_t pix = p0 + (size_t)blockIdx.x * 256 + threadIdx.x; pix < p1; pix += (size_t)gridDim.x * 256) {
+__global__ __launch_bounds__(kDeviceThreads) void tensor_to_hwc_kernel(const TView t, float* hwc, size_t p0, size_t p1, const HostDone done) {
+    for (size_t pix = p0 + (size_t)blockIdx.x * blockDim.x + threadIdx.x; pix < p1; pix += (size_t)gridDim.x * blockDim.x) {
         const unsigned y = (unsigned)pix / (unsigned)t.w, x = (unsigned)pix - y * (unsigned)t.w;
         const float4 v = load4<T>(reinterpret_cast<const T*>(t.ptr) + ((size_t)(y + t.pad) * t.wp() + x + t.pad) * t.cp);
         if constexpr (PC == 4) *reinterpret_cast<float4*>(hwc + pix * 4) = make_float4(v.x, v.y, v.z, t.c > 3 ? v.w : 0.f);
@@ -323,15 +376,16 @@ __global__ __launch_bounds__(256) void tensor_to_hwc_kernel(const TView t, float
     tell_host(done);
 }
 template <typename T>
-static void launch_hwc_out(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
-    const dim3 grid((unsigned)std::min<size_t>(kMaxBlocks, (p1 - p0 + 255) / 256));
-    if (pc == 4) hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 4>), grid, dim3(256), 0, s, t, hwc, p0, p1, done);
-    else if (pc == 2) hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 2>), grid, dim3(256), 0, s, t, hwc, p0, p1, done);
-    else hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 1>), grid, dim3(256), 0, s, t, hwc, p0, p1, done);
+static void launch_hwc_out(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, bool device, hipStream_t s) {
+    const int threads = device ? kDeviceThreads : 256;
+    const dim3 grid(blocks_for(p1 - p0, device ? kMaxDeviceBlocks : kMaxBlocks, threads));
+    if (pc == 4) hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 4>), grid, dim3(threads), 0, s, t, hwc, p0, p1, done);
+    else if (pc == 2) hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 2>), grid, dim3(threads), 0, s, t, hwc, p0, p1, done);
+    else hipLaunchKernelGGL((tensor_to_hwc_kernel<T, 1>), grid, dim3(threads), 0, s, t, hwc, p0, p1, done);
 }
-void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, hipStream_t s) {
-    if (t.f16) launch_hwc_out<_Float16>(t, hwc, pc, p0, p1, done, s);
-    else launch_hwc_out<float>(t, hwc, pc, p0, p1, done, s);
+void launch_tensor_to_hwc(const TView& t, float* hwc, int pc, size_t p0, size_t p1, const HostDone& done, bool device, hipStream_t s) {
+    if (t.f16) launch_hwc_out<_Float16>(t, hwc, pc, p0, p1, done, device, s);
+    else launch_hwc_out<float>(t, hwc, pc, p0, p1, done, device, s);
 }
 
 // An arg-max layer's two results: the exact indices it keeps beside its tensor, and the tensor's second channel.

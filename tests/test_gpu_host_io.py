@@ -200,6 +200,32 @@ def test_a_late_frame_leaves_its_own_value_range(monkeypatch):
     for i, (a, b) in enumerate(zip(*results)):
         assert np.array_equal(a, b), i
 @pytest.mark.gpu
+@STORAGES
+@pytest.mark.parametrize("c,h,w", [(3, 303, 401), (3, 401, 302), (3, 16, 8191), (4, 257, 515), (2, 401, 501), (1, 701, 389)])
+def test_overlapped_pipeline_on_odd_frames(c, h, w, storage):
+    """The conversions between buffers in device memory: pixel counts that are no multiple of four, rows that end inside a
+    thread's four pixels, every channel count of interleaved pixels; from both host layouts to both."""
+    net = _copy_net(c, h, w, storage, pad=1)
+    x = [prng.uniform(700 + i + c * w, (c, h, w), -2.0, 2.0) for i in range(3)]
+    for in_order in (fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW):
+        for out_order in (fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW):
+            net.asyncBegin(1, 1, inOrder=in_order, outOrder=out_order, depth=2)
+            pc = 4 if c == 3 else c
+            outs = [np.full((c, h, w) if out_order == fa.ORDER_CHANNELWISE else (h, w, pc), np.nan, np.float32) for _ in x]
+            for f, o in zip(x, outs):
+                ticket = net.asyncSubmit(f if in_order == fa.ORDER_CHANNELWISE else np.ascontiguousarray(f.transpose(1, 2, 0)), o)
+            net.asyncWait(ticket)
+            net.asyncEnd()
+            for f, o in zip(x, outs):
+                want = f if storage == fa.STORAGE_F32 else f.astype(np.float16).astype(np.float32)
+                if out_order == fa.ORDER_GPU_SHALLOW:
+                    assert not o[..., c:].any()
+                    o = o[..., :c].transpose(2, 0, 1)
+                assert np.array_equal(o, want), (in_order, out_order)
+    net.cleanup()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("order", [fa.ORDER_CHANNELWISE, fa.ORDER_GPU_SHALLOW], ids=["chw", "hwc"])
 def test_page_locked_input_is_read_behind_the_default_stream(order):
     """A frame that the application's default stream is still writing into page-locked memory when it is handed over."""
