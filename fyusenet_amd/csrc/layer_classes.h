@@ -680,8 +680,8 @@ class ConvLayer : public Layer {
             net->dev_free(wp);
         }
     }
-    // The LDS-staged weights, gathered windows form for few channels (conv_g16.hip) against what has been chosen so far.
-    void setup_g16(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
+    // what the two forms for few channels share
+    ConvP16Params small_channel_params(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
         ConvP16Params q{};
         q.in = in_v.ptr; q.out = out_v.ptr; q.res = res_v ? res_v->ptr : nullptr;
         q.in_hp = in_v.hp(); q.in_wp = in_v.wp(); q.in_cp = in_v.cp;
@@ -703,6 +703,11 @@ class ConvLayer : public Layer {
         q.acc_mul = 1.f;
         q.act = act();
         q.in_amax = tin(0).amax;
+        return q;
+    }
+    // The LDS-staged weights, gathered windows form for few channels (conv_g16.hip) against what has been chosen so far.
+    void setup_g16(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
+        const ConvP16Params q = small_channel_params(in_v, out_v, res_v, res_relu, res_scale);
         const int frags = (oc + 15) / 16, tiles = (oh * ow + 15) / 16;
         if ((long long)in_v.elems() * (q.f16 ? 2 : 4) > (1ll << 31)) return;
         int want = 0;   // FYNHIP_G16_FRAGS=fragments per wave (tests)
@@ -774,6 +779,75 @@ class ConvLayer : public Layer {
             p16_wpack_dev = wp;
             p16 = g16 = true;
             kr16 = false;
+            pp = cands[pick];
+        } else {
+            net->dev_free(wp);
+        }
+    }
+    // The form with a tile's window in LDS (conv_p16n.hip) against what has been chosen so far, in the heights of tile that
+    // have been compiled.
+    void setup_p16n(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
+        ConvP16Params q = small_channel_params(in_v, out_v, res_v, res_relu, res_scale);
+        q.wm = q.mfrags = (oc + 15) / 16;
+        q.cout_blocks = 1;
+        if ((long long)in_v.elems() > (1ll << 30)) return;
+        int want = 0;   // FYNHIP_P16N_ROWS=rows of a tile (tests)
+        if (const char* e = net->sw.get("FYNHIP_P16N_ROWS")) want = atoi(e);
+        std::vector<ConvP16Params> cands;
+        for (int th : {5, 4, 2}) {
+            if (want && th != want) continue;
+            ConvP16Params c = q;
+            c.tile_h = th; c.tile_w = 16;
+            c.tiles_x = (ow + 15) / 16; c.tiles_y = (oh + th - 1) / th;
+            c.rcp_tiles_x = 1.0f / (float)c.tiles_x;
+            const size_t lds = conv_p16n_lds_bytes(c);
+            if (lds == 0 || lds > 160 * 1024 || (long long)c.tiles_x * c.tiles_y > 4000000) continue;
+            c.pos_groups = std::min(c.tiles_x * c.tiles_y, lds <= 80 * 1024 ? 512 : 256);
+            cands.push_back(c);
+        }
+        if (cands.empty()) return;
+        const bool always = want || net->sw.get("FYNHIP_FORCE_P16N_CONV") != nullptr;
+        const char* at = net->sw.get("FYNHIP_AUTOTUNE");
+        int pick = 0;
+        char key[160];
+        snprintf(key, sizeof(key), "p16n:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
+        int cached[3] = {0, 0, 0};
+        bool timed = false;
+        if (always) {
+        } else if (tune_cache_triple(net, key, cached)) {
+            pick = -1;
+            for (size_t i = 0; cached[0] && i < cands.size(); i++)
+                if (cands[i].tile_h == cached[1]) pick = (int)i;
+        } else {
+            timed = !(at && at[0] == '0');
+            if (!timed) pick = -1;
+        }
+        if (pick < 0) return;
+        const size_t halves = (size_t)q.wm * q.cin_chunks * (q.f16 ? 1 : 2) * 64 * 8;
+        void* const wp = net->dev_alloc(halves * 2, true);
+        for (ConvP16Params& c : cands) c.wpack = wp;
+        if (timed) {
+            float best = 1e30f, t_other = 1e30f;
+            for (int rep = 0; rep < 3; rep++) {
+                for (size_t i = 0; i < cands.size(); i++) {
+                    const float t = time_calls(net, [&]() {
+                        if (launch_conv_p16n(cands[i], net->stream) != 0) fail(FYN_ERR_DEVICE, "few-channel convolution launch failed while tuning");
+                    }, 10);
+                    if (t < best) { best = t; pick = (int)i; }
+                }
+                t_other = std::min(t_other, time_calls(net, [&]() { run(net->stream); }, 10));
+            }
+            if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
+                fprintf(stderr, "[tune] 3x3 on %d channels, %dx%d positions, to %d: window in LDS (%d rows, %d workgroups) %.1f us, %s %.1f us\n", in_v.cp, oh, ow, oc,
+                        cands[pick].tile_h, cands[pick].pos_groups, best * 1e3f, own_info().c_str(), t_other * 1e3f);
+            tune_cache_store_triple(net, key, best < t_other ? 1 : 0, cands[pick].tile_h, 0);
+            if (best >= t_other) pick = -1;
+        }
+        if (pick >= 0) {
+            if (p16) net->dev_free(p16_wpack_dev);
+            p16_wpack_dev = wp;
+            p16 = p16n = true;
+            kr16 = g16 = false;
             pp = cands[pick];
         } else {
             net->dev_free(wp);
@@ -1199,6 +1273,11 @@ class ConvLayer : public Layer {
             if (!h16 && !c4 && !d16 && same_storage && conv_g16_supported(k, dil, in_v.cp, oc, out_v.cp) && d.in_channels <= in_v.cp &&
                 (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_G16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") && !only_kr)
                 setup_g16(in_v, out_v, res_v, res_relu, res_scale);
+            // ... and windows staged in LDS (a test that forces another form, or a tile of one, wants that form)
+            if (!h16 && !c4 && !d16 && !s16 && same_storage && k == 3 && dil == 1 && in_v.cp % 8 == 0 && oc <= 48 && out_v.cp % 4 == 0 && out_v.cp >= oc && d.in_channels <= in_v.cp &&
+                (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_P16N_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") &&
+                !net->sw.get("FYNHIP_P16_TILE") && !net->sw.get("FYNHIP_FORCE_G16_CONV") && !net->sw.get("FYNHIP_G16_FRAGS") && !only_kr)
+                setup_p16n(in_v, out_v, res_v, res_relu, res_scale);
         }
         if (direct) {
             scale_dev = static_cast<float*>(net->dev_alloc(padded * sizeof(float)));
@@ -1229,7 +1308,7 @@ class ConvLayer : public Layer {
         } else if (p16) {
             const float wmul = weight_prescale(w, (size_t)oc * k * k * d.in_channels);
             pp.acc_mul = pp2.acc_mul = 1.0f / wmul;
-            if (g16) pack_g16(w, wmul);
+            if (g16 || p16n) pack_g16(w, wmul);
             else if (s16) pack_frag16(pp, p16_wpack_dev, w, wmul);
             else if (c4) pack_c4(w, wmul);
             else if (d16) pack_d16(w, wmul);
@@ -1330,7 +1409,7 @@ class ConvLayer : public Layer {
             return;
         }
         if (p16) {
-            if ((s16 ? launch_conv_s16(pp, net->fusion_on() ? argmax_tail : ArgMaxTail{}, s) : g16 ? launch_conv_g16(pp, s) : c4 ? launch_conv_p16c4(pp, k, s) : (d16 ? launch_conv_d16(pp, s) : (kr16 ? launch_conv_kr16(pp, k, s) : (h16 ? launch_conv_h16(pp, k, s) : launch_conv_p16(pp, s))))) != 0 ||
+            if ((s16 ? launch_conv_s16(pp, net->fusion_on() ? argmax_tail : ArgMaxTail{}, s) : p16n ? launch_conv_p16n(pp, s) : g16 ? launch_conv_g16(pp, s) : c4 ? launch_conv_p16c4(pp, k, s) : (d16 ? launch_conv_d16(pp, s) : (kr16 ? launch_conv_kr16(pp, k, s) : (h16 ? launch_conv_h16(pp, k, s) : launch_conv_p16(pp, s))))) != 0 ||
                 (h16 && h16_two && launch_conv_h16(pp2, k, s) != 0))
                 fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
@@ -1376,6 +1455,12 @@ class ConvLayer : public Layer {
             char buf[220];
             snprintf(buf, sizeof(buf), "conv_s16 %s streaming: %d chunks and %d fragments of 16 output channels in registers", pp.f16 ? "f16" : "f16x2-split", pp.cin_chunks, pp.mfrags);
             return mode + buf + (argmax_tail.idx ? "; the arg-max layer behind it is computed from what is stored" : "");
+        }
+        if (p16 && p16n) {
+            char buf[240];
+            snprintf(buf, sizeof(buf), "conv_p16n %s window of %dx16 positions in LDS: %d steps of four 8-channel groups over 4 waves, %d fragment(s) of 16 output channels, blocks=%d tiles=%d lds=%zu",
+                     pp.f16 ? "f16" : "f16x2-split", pp.tile_h, pp.cin_chunks, pp.wm, pp.pos_groups, pp.tiles_x * pp.tiles_y, conv_p16n_lds_bytes(pp));
+            return mode + buf;
         }
         if (p16 && g16) {
             char buf[220];
@@ -1441,6 +1526,7 @@ class ConvLayer : public Layer {
     bool kr16 = false;            // ... the K-resident form for layers with few positions (conv_p16.hip, conv_kr16_kernel)
     bool s16 = false;             // ... the streaming 1x1 form (conv_s16.hip)
     ArgMaxTail argmax_tail{};     // ... with the arg-max layer behind it (fuse_argmax_layers)
+    bool p16n = false;             // ... the form for few channels with a tile's window in LDS (conv_p16n.hip)
     bool g16 = false;             // ... the form that gathers 3x3 windows of few channels (conv_g16.hip)
     bool d16 = false;             // ... the LDS-free 1x1 form for many positions and few input channels (conv_d16.hip)
     // A depthwise 3x3 layer whose only reader is this 1x1 layer in the K-resident form can be computed inside this

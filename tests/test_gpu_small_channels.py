@@ -68,6 +68,65 @@ def test_gathered_windows_of_repeated_pixels(monkeypatch, storage, cin, cout, h,
     assert rel_l2(got, oracle_single(b, storage, [x], weights)) <= TOL[storage]
 
 
+# cin, cout, h, w, stride, deep, act, residual, rows of a tile
+WINDOWED = [
+    (16, 16, 2, 3, 1, False, ActType.NONE, None, 2),             # fewer positions than a row
+    (12, 20, 24, 34, 2, False, ActType.RELU, None, 4),           # steps over the input, a ragged fragment, a window's even and odd columns
+    (16, 20, 25, 33, 2, True, ActType.LEAKY_RELU, None, 2),      # zero padding, a leak
+    (20, 40, 31, 65, 2, False, ActType.RELU, None, 2),
+    (24, 48, 16, 18, 2, True, ActType.CLIP, None, 4),
+    (40, 40, 11, 17, 1, False, ActType.RELU, ActType.NONE, 5),   # a row and a column behind the last whole tile
+    (40, 36, 20, 20, 1, True, ActType.NONE, ActType.RELU, 2),
+    (40, 12, 30, 47, 2, True, ActType.RELU, None, 4),
+    (48, 33, 40, 23, 1, True, ActType.RELU, None, 5),            # channels behind the output's count
+    (24, 8, 90, 1000, 1, False, ActType.RELU, None, 2),          # 2835 tiles: workgroups walk six
+    (40, 40, 130, 400, 1, False, ActType.RELU, ActType.RELU, 5), # 650 tiles, the residual of a second tile
+]
+
+
+def _windowed(case):
+    cin, cout, h, w, stride, deep, act, residual, _ = case
+    b = ConvLayerBuilder(3, "conv").type(LayerType.CONVOLUTION2D).number(1).shape(cout, h, w, cin).prefixAct(act).downsample(stride)
+    if act == ActType.LEAKY_RELU:
+        b.leakyReLU(0.2)
+    if act == ActType.CLIP:
+        b.clip(-0.5, 0.75)
+    if deep:
+        b.deep().inputPadding(1).outputPadding(1)
+    if residual is not None:
+        b.residual(residual)
+        if deep:
+            b.residualPadding(1)
+    return b
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("case", WINDOWED, ids=lambda c: "%dto%d_%dx%d_s%d_%s_th%d" % (c[0], c[1], c[2], c[3], c[4], "deep" if c[5] else "shallow", c[8]))
+def test_windows_in_lds(monkeypatch, case, storage):
+    cin, cout, h, w, stride, deep, act, residual, rows = case
+    monkeypatch.setenv("FYNHIP_P16N_ROWS", str(rows))
+    b = _windowed(case)
+    inputs = [prng.normal(141 + cin, (cin, h, w))]
+    if residual is not None:
+        inputs.append(prng.normal(143 + cin, (cout, h // stride, w // stride)))
+    weights = conv_block(147 + cin, cout, 3, cin)
+    got, info = run_single(b, storage, inputs, weights)
+    assert "conv_p16n" in info and "of %dx16" % rows in info, info
+    # (fp32 tensors: three passes over 22-bit operands, as in the other exact forms)
+    assert rel_l2(got, oracle_single(b, storage, inputs, weights)) <= (2e-6 if storage == fa.STORAGE_F32 else TOL[storage])
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("cin,cout,h,w,step,stride", [(40, 20, 13, 16, 0.5, 2), (20, 12, 12, 19, 0.25, 2), (16, 16, 7, 9, 0.5, 1)])
+def test_windows_in_lds_of_repeated_pixels(monkeypatch, storage, cin, cout, h, w, step, stride):
+    monkeypatch.setenv("FYNHIP_FORCE_P16N_CONV", "1")
+    b = ConvLayerBuilder(3, "conv").type(LayerType.FRACCONVOLUTION2D).number(1).shape(cout, h, w, cin).prefixAct(ActType.RELU).downsample(stride).sourceStep(step)
+    x, weights = prng.normal(161, (cin, h, w)), conv_block(167, cout, 3, cin)
+    got, info = run_single(b, storage, [x], weights)
+    assert "conv_p16n" in info, info
+    assert rel_l2(got, oracle_single(b, storage, [x], weights)) <= (2e-6 if storage == fa.STORAGE_F32 else TOL[storage])
+
+
 @pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
 @pytest.mark.parametrize("kernel,width,height", [(3, 64, 48), (9, 100, 76)])
 def test_function_layer_applied_by_the_convolution_in_front(monkeypatch, storage, kernel, width, height):
