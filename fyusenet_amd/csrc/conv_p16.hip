@@ -263,7 +263,7 @@ __device__ __forceinline__ void rows_load_b8(i32x8_t& dst, int half, const unsig
 }
 // weight k of a pair at offset w: 0..3 the fp16 fragments [step][channel fragment], 4..7 the fp8 halves
 __device__ __forceinline__ i32x4_t rows_load_w(const __amdgpu_buffer_rsrc_t weights, unsigned w, int k, unsigned wstep, unsigned wlane) {
-    const int step = (k / 2) % 2, fm = k % 2, plane = k < 4 ? 0 : 2;
+    const int step = (k / 2) % 2, fm = k % 2, plane = k < 4 ? 0 : 2;   // (fp16 tensors: k < 4)
     typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
     return __builtin_bit_cast(i32x4_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights, wlane + (fm * NPLW + plane) * 1024, w + step * wstep, 0));
 }
@@ -998,8 +998,11 @@ struct GeoC4 {
     static constexpr int NITEMS = HH * HW;                            // staging items: pixels
     static constexpr int NB = (NITEMS + 255) / 256;
     static constexpr int CPB = 32;
+    // tiles whose fragments are rows of sixteen positions take the tap pairs in another order: c4_rows
+    static constexpr bool ROWS = TW == 16;
+    static_assert(!ROWS || K == 9, "rows: eight taps of a kernel row and one more");
     static_assert(NPOS % 16 == 0 && (2 * NS) % PD == 0, "whole position fragments; whole ring turns");
-    static_assert(2 * BUF + PLANE < 65536, "offsets fit the LDS instructions' immediate field");
+    static_assert((ROWS ? BUF : 2 * BUF + PLANE) < 65536, "offsets fit the LDS instructions' immediate field");
 };
 
 template <class G, bool C8>
@@ -1205,6 +1208,119 @@ __device__ __forceinline__ void c4_stage_c8(f32x4_t (&acc)[2][G::FN], half8_t (&
     }
 }
 
+// The stage on tiles whose fragments are rows of sixteen positions (9x9; fp16 tensors, or fp32 with the fp8 form).  Steps
+// 0 .. 8 take the first eight taps of kernel row ky (a lane group's pair: taps 2 kq and 2 kq + 1), steps 9 .. 11 the ninth
+// tap of four rows each (a pair with an empty partner).  In the first nine the fragment of output row r at ky is that of
+// row r + 1 at ky - 1, and so are the fp8 operands of a pair of steps (ky, ky + 1) -- rows r + ky and r + ky + 1 -- for row
+// r + 2 at the pair before: both move through registers, and a tile of TH rows reads 4 TH + 8 + 6 TH + 12 fragments from
+// LDS instead of 24 TH (TH = 5: 70 against 120).  That leaves room for the weights there (48 KB, or 24 with fp16 tensors):
+// the MFMA waves then load nothing from memory, and what they store need not have arrived before they go on -- loads and
+// stores of a wave are counted in one order, so weights requested behind a tile's stores waited for the burst that all
+// workgroups store at the same time.  Schedule
+// and lifetimes as in p16_rows_c8: a slot is one output row of a pair of steps, what it takes is requested LA slots ahead,
+// the weights of a pair one pair ahead; the barrier that hands over the next tile lies in front of the first request for it.
+// 9x9 3 -> 32: 512x624 fp32 18.8 -> 17.3 us (19.2 with the weights from memory), 1920x1080 fp32 112 -> 102 (104), 1524x1856
+// fp16 78 -> 65 (68).  Bound there: the stores (265 MB in 102 us beside 33 read).
+template <class G>
+struct C4Ring {
+    static constexpr int LA = HSTORE ? 4 : 2;          // slots (64 or 128 matrix-pipe cycles) from an LDS read to its use
+    static constexpr int LW = 1;                       // pairs of steps from the request of weights to their use
+    half8_t a0[LW][2][2];
+    i32x8_t a2[LW][2];
+    half8_t b0[LA + 1];                                // rows 0 ..
+    i32x8_t b8[LA];                                    // pairs of rows 0 ..
+};
+template <class G>
+__device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& ring, const unsigned char* at_rows, const unsigned char* at_ninth,
+                                        const unsigned char* at_last, const unsigned char* next_rows, const unsigned char* weights) {
+    constexpr int TH = G::FN, LA = C4Ring<G>::LA, LW = C4Ring<G>::LW, NP = 6, RP = G::ROW_PITCH;
+    constexpr bool C8 = !HSTORE;
+    static_assert(TH >= 4 && TH > LA - 1 && G::NS == 2 * NP, "a slot has room for its share of the requests");
+    half8_t a0[NP + LW][2][2], b0[TH + 8], n0[LA + 1], l0[3][TH];
+    i32x8_t a2[NP + LW][2], b8[TH + 6], n8[LA], u8[2][TH];   // (b8[s]: rows s and s + 1; u8: the pairs that hold a step of the ninth tap; n0, n8: the next tile's)
+#pragma unroll
+    for (int d = 0; d < LW; d++)
+#pragma unroll
+        for (int fm = 0; fm < 2; fm++) {
+            a0[d][0][fm] = ring.a0[d][0][fm]; a0[d][1][fm] = ring.a0[d][1][fm];
+            if constexpr (C8) a2[d][fm] = ring.a2[d][fm];
+        }
+#pragma unroll
+    for (int r = 0; r <= LA; r++) b0[r] = ring.b0[r];
+    if constexpr (C8) {
+#pragma unroll
+        for (int r = 0; r < LA; r++) b8[r] = ring.b8[r];
+    }
+    auto half_of = [](const unsigned char* at) { return *reinterpret_cast<const half8_t*>(at); };
+    // the ninth tap of rows 4 j + kq and output row r (the last step: only row 8 of the first lane group counts)
+    auto ninth = [&](int j, int r) { return j < 2 ? at_ninth + (4 * j + r) * RP : at_last + r * RP; };
+    // the n-th read for row r of pair p (p = NP: the next tile's first pair)
+    auto request = [&](auto p_, auto r_, auto n_) __attribute__((always_inline)) {
+        constexpr int p = decltype(p_)::value, r = decltype(r_)::value, n = decltype(n_)::value;
+        if constexpr (p == 0) {
+            if constexpr (C8 && n < 2) rows_load_b8<G>(b8[r], n, at_rows + (r + n) * RP + G::PLANE);
+            if constexpr (n == 2) b0[r + 1] = half_of(at_rows + (r + 1) * RP);
+        } else if constexpr (p < 4) {
+            if constexpr (C8 && n < 2 && r >= TH - 2) rows_load_b8<G>(b8[r + 2 * p], n, at_rows + (r + 2 * p + n) * RP + G::PLANE);
+            if constexpr (n >= 2 && n < 4 && r == TH - 1) b0[TH + 2 * p + n - 3] = half_of(at_rows + (TH + 2 * p + n - 3) * RP);
+        } else if constexpr (p == 4) {
+            if constexpr (C8 && n == 0) rows_load_b8<G>(u8[0][r], 0, at_rows + (r + 8) * RP + G::PLANE);
+            if constexpr (C8 && n == 1) rows_load_b8<G>(u8[0][r], 1, ninth(0, r) + G::PLANE);
+            if constexpr (n == 2) l0[0][r] = half_of(ninth(0, r));
+            if constexpr (n == 3 && r == TH - 1) b0[TH + 7] = half_of(at_rows + (TH + 7) * RP);
+        } else if constexpr (p == 5) {
+            if constexpr (C8 && n < 2) rows_load_b8<G>(u8[1][r], n, ninth(1 + n, r) + G::PLANE);
+            if constexpr (n == 2) l0[1][r] = half_of(ninth(1, r));
+            if constexpr (n == 3) l0[2][r] = half_of(ninth(2, r));
+        } else {
+            if constexpr (C8 && n < 2) rows_load_b8<G>(n8[r], n, next_rows + (r + n) * RP + G::PLANE);
+            if constexpr (n == 2) n0[r + 1] = half_of(next_rows + (r + 1) * RP);
+            if constexpr (n == 3 && r == 0) n0[0] = half_of(next_rows);
+        }
+    };
+    auto slot = [&](auto index) __attribute__((always_inline)) {
+        constexpr int g = decltype(index)::value, p = g / TH, r = g % TH, u = g + LA;
+        if constexpr (g == NP * TH - LA) lds_barrier();
+        auto issue = [&](auto index_m) __attribute__((always_inline)) {
+            constexpr int m = decltype(index_m)::value, fm = m % 2;
+            if constexpr (!(HSTORE && (m == 2 || m == 3))) {
+                if constexpr (m < 2) {
+                    const half8_t b = p < 4 ? b0[r + 2 * p] : p == 4 ? b0[r + 8] : l0[1][r];
+                    acc[fm][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[p][0][fm], b, acc[fm][r], 0, 0, 0);
+                } else if constexpr (m < 4) {
+                    acc[fm][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a2[p][fm], p < 4 ? b8[p < 4 ? r + 2 * p : 0] : u8[p < 4 ? 0 : p - 4][r], acc[fm][r], 0, 0, 0, 0, 0, 0);
+                } else {
+                    const half8_t b = p < 4 ? b0[p < 4 ? r + 2 * p + 1 : 0] : p == 4 ? l0[0][r] : l0[2][r];
+                    acc[fm][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[p][1][fm], b, acc[fm][r], 0, 0, 0);
+                }
+                // (fp16 tensors issue four matrix instructions a slot: their reads are the last two kinds)
+                constexpr int n = HSTORE ? (m < 2 ? m + 2 : -1) : m;
+                if constexpr (n >= 0 && n < 4) request(std::integral_constant<int, u / TH>(), std::integral_constant<int, u % TH>(), std::integral_constant<int, n>());
+                // a share of the weights of pair p + LW
+                constexpr int NW = HSTORE ? 4 : 8, k = (r * NW + TH - 1) / TH + m - (HSTORE ? 4 : 2);
+                if constexpr (m >= (HSTORE ? 4 : 2) && k < NW && k * TH / NW == r)
+                    rows_put_w(a0[p + LW], a2[p + LW], k, *reinterpret_cast<const i32x4_t*>(weights + ((p + LW) % NP * NW + k) * 1024));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        expand(issue, std::make_integer_sequence<int, 6>());
+    };
+    expand(slot, std::make_integer_sequence<int, NP * TH>());
+#pragma unroll
+    for (int d = 0; d < LW; d++)
+#pragma unroll
+        for (int fm = 0; fm < 2; fm++) {
+            ring.a0[d][0][fm] = a0[NP + d][0][fm]; ring.a0[d][1][fm] = a0[NP + d][1][fm];
+            if constexpr (C8) ring.a2[d][fm] = a2[NP + d][fm];
+        }
+#pragma unroll
+    for (int r = 0; r <= LA; r++) ring.b0[r] = n0[r];
+    if constexpr (C8) {
+#pragma unroll
+        for (int r = 0; r < LA; r++) ring.b8[r] = n8[r];
+    }
+}
+
 template <int K, int TH, int TW, bool C8>
 __global__ __launch_bounds__(512) void conv_p16c4_kernel(const ConvP16Params p) {
     using G = GeoC4<K, TH, TW>;
@@ -1247,15 +1363,34 @@ __global__ __launch_bounds__(512) void conv_p16c4_kernel(const ConvP16Params p) 
         const int pi = 4 * st + kq;
         const int row = pi / G::PPR, col = 2 * (pi - row * G::PPR);
         off[st] = pi < G::NPAIR ? row * G::ROW_PITCH + col * G::PIX : 0;
+        if constexpr (G::ROWS) off[st] = st < K ? st * G::ROW_PITCH + 2 * kq * G::PIX : min(4 * (st - K) + kq, K - 1) * G::ROW_PITCH + (K - 1) * G::PIX;
     }
     const unsigned wstep = (unsigned)p.mfrags * NPLW * 1024;
     const unsigned char* wbase = reinterpret_cast<const unsigned char*>(p.wpack) + (size_t)(cb * 2 * NPLW) * 1024;   // (uniform: the loads take it as their scalar base)
     const unsigned wlane = lane * 16;
     const unsigned char* wend = wbase + (size_t)NS * wstep;
     // weight ring: fp16 planes (hi, lo), or with the fp8 form the hi plane and the fp8 plane in pairs of steps
+    constexpr bool RWS = G::ROWS && (C8 || HSTORE);
     half8_t a_q[PD][2][C8 ? 1 : NPL];
     half8_t a0[C8 ? PD : 1][2];
     i32x8_t a2[C8 ? PD / 2 : 1][2];
+    typename std::conditional<RWS, C4Ring<G>, int>::type ring;
+    constexpr int NW = HSTORE ? 4 : 8;   // weight fragments of a pair of steps (rows_load_w)
+    constexpr int w_off = sb_off + 2 * 32 * 4;
+    if constexpr (RWS) {
+        // the block's weights into LDS, as the MFMA waves take them: [pair of steps][fragment][lane]
+        const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(wbase), 0, (int)((unsigned)NS * wstep), 0x00020000);
+        constexpr int SHARE = NS / 2 * NW / 4;
+        i32x4_t w[SHARE];
+#pragma unroll
+        for (int i = 0; i < SHARE; i++) {
+            const int c = wn * SHARE + i, k = c % NW, step = (k / 2) % 2, fm = k % 2, plane = k < 4 ? 0 : 2;
+            typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+            w[i] = __builtin_bit_cast(i32x4_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights, wlane, (unsigned)((fm * NPLW + plane) * 1024) + (unsigned)(c / NW * 2 + step) * wstep, 0));
+        }
+#pragma unroll
+        for (int i = 0; i < SHARE; i++) *reinterpret_cast<i32x4_t*>(lds + w_off + (wn * SHARE + i) * 1024 + wlane) = w[i];
+    } else
 #pragma unroll
     for (int d = 0; d < PD; d++)
 #pragma unroll
@@ -1330,6 +1465,36 @@ __global__ __launch_bounds__(512) void conv_p16c4_kernel(const ConvP16Params p) 
         }
     };
     lds_barrier();   // the first stage is staged
+    if constexpr (RWS) {
+        const unsigned char* const rows_at = lds + bbase[0] + 2 * kq * G::PIX;                             // row 0, this lane's pair of the first eight taps
+        const unsigned char* const ninth_at = lds + bbase[0] + kq * G::ROW_PITCH + (K - 1) * G::PIX;       // row kq, the ninth tap
+        const unsigned char* const last_at = lds + bbase[0] + (K - 1) * G::ROW_PITCH + (K - 1) * G::PIX;   // the last row's
+        constexpr int LA = C4Ring<G>::LA;
+#pragma unroll
+        for (int r = 0; r <= LA; r++) ring.b0[r] = *reinterpret_cast<const half8_t*>(rows_at + r * G::ROW_PITCH);
+        if constexpr (C8) {
+#pragma unroll
+            for (int r = 0; r < LA; r++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) rows_load_b8<G>(ring.b8[r], h, rows_at + (r + h) * G::ROW_PITCH + G::PLANE);
+        }
+#pragma unroll
+        for (int d = 0; d < C4Ring<G>::LW; d++)
+#pragma unroll
+            for (int k = 0; k < NW; k++) rows_put_w(ring.a0[d], ring.a2[d], k, *reinterpret_cast<const i32x4_t*>(lds + w_off + (d * NW + k) * 1024 + wlane));
+        int buf = 0;
+        for (int t = group;;) {
+            const int here = buf * G::BUF, there = G::BUF - here;
+            c4_rows<G>(acc, ring, rows_at + here, ninth_at + here, last_at + here, rows_at + there, lds + w_off + wlane);
+            finish_tile(t);
+            t += p.pos_groups;
+            if (t >= ntiles) break;
+            zero_acc();
+            buf = 1 - buf;
+        }
+        if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 4);
+        return;
+    }
     half8_t b[C8 ? 1 : FN][NPL];   // exact form: hi and lo fragments of a step
     half8_t b0[C8 ? FN : 1];       // fp8 form: hi fragments ...
     i32x8_t b1[C8 ? FN : 1];       // ... and the fp8 fragments of a pair of steps
@@ -1961,14 +2126,15 @@ struct C4Entry {
     p16_fn fn, fn8;   // three fp16 passes; fp8 correction terms (fp32 tensors, an even number of steps) or null
     size_t buf;
     int steps;
+    size_t weights;   // the block's weights in LDS (rows of sixteen positions)
 };
 template <int K, int TH, int TW>
 constexpr C4Entry c4entry() {
     using G = GeoC4<K, TH, TW>;
-    if constexpr (!HSTORE && G::NS % 2 == 0) return C4Entry{K, TH, TW, conv_p16c4_kernel<K, TH, TW, false>, conv_p16c4_kernel<K, TH, TW, true>, (size_t)G::BUF, G::NS};
-    else return C4Entry{K, TH, TW, conv_p16c4_kernel<K, TH, TW, false>, nullptr, (size_t)G::BUF, G::NS};
+    if constexpr (!HSTORE && G::NS % 2 == 0) return C4Entry{K, TH, TW, conv_p16c4_kernel<K, TH, TW, false>, conv_p16c4_kernel<K, TH, TW, true>, (size_t)G::BUF, G::NS, G::ROWS ? (size_t)G::NS * 2 * (HSTORE ? 1024 : 2048) : 0};
+    else return C4Entry{K, TH, TW, conv_p16c4_kernel<K, TH, TW, false>, nullptr, (size_t)G::BUF, G::NS, G::ROWS ? (size_t)G::NS * 2 * (HSTORE ? 1024 : 2048) : 0};
 }
-const C4Entry kC4Entries[] = {c4entry<9, 8, 8>(), c4entry<9, 4, 8>(), c4entry<9, 8, 4>(), c4entry<3, 8, 8>(), c4entry<3, 4, 8>()};
+const C4Entry kC4Entries[] = {c4entry<9, 8, 16>(), c4entry<9, 5, 16>(), c4entry<9, 4, 16>(), c4entry<9, 8, 8>(), c4entry<9, 4, 8>(), c4entry<9, 8, 4>(), c4entry<3, 8, 8>(), c4entry<3, 4, 8>()};
 struct KREntry {
     int taps, cpw, fm, nfrag, th, tw, stride, dws, rounds, src;   // (cpw: chunks per wave and round)
     p16_fn fn;
@@ -2230,7 +2396,7 @@ size_t P16_NAME(conv_p16c4_lds_bytes)(const ConvP16Params& p, int k) {
     if (p.f16) return conv_p16c4_lds_bytes_half(p, k);
 #endif
     const C4Entry* e = find_c4entry(p, k);
-    return e ? 2 * e->buf + 2 * 32 * 4 : 0;
+    return e ? 2 * e->buf + 2 * 32 * 4 + e->weights : 0;
 }
 
 // k x k convolution on a four-channel input: wpack = [step][cout fragment of 16][plane][lane][8 halves], lane = (output

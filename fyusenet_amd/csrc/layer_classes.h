@@ -971,7 +971,11 @@ class ConvLayer : public Layer {
                 uint16_t* base = pack.data() + (((size_t)st * pp.mfrags + mf) * npl) * 64 * 8;
                 for (int lane = 0; lane < 64; lane++) {
                     const int o = p16_row_channel(mf, lane & 15, pp.f16 ? 2 : 1), pi = 4 * st + (lane >> 4);
-                    const int ky = pi / ppr, kx0 = 2 * (pi % ppr);
+                    int ky = pi / ppr, kx0 = 2 * (pi % ppr);
+                    if (pp.tile_w == 16) {   // (rows of sixteen positions: eight taps of a row a step, then the ninth tap of four rows)
+                        ky = st < k ? st : 4 * (st - k) + (lane >> 4);
+                        kx0 = st < k ? 2 * (lane >> 4) : k - 1;
+                    }
                     if (o >= oc || ky >= k) continue;
                     for (int j = 0; j < 8; j++) {
                         const int kx = kx0 + j / 4, ci = j % 4;

@@ -814,6 +814,46 @@ def test_small_input_sixteen_position_fragment_form(case, shallow, storage, monk
         assert rel_l2(got, exact) <= 3e-5
 
 
+C4_ROW_CASES = [
+    # cin, cout, h, w, tile "rows,16", kw: fragments that are rows of sixteen positions
+    (3, 32, 5, 64, "5,16", {}),                       # one whole tile
+    (3, 32, 41, 67, "5,16", {"bn": True}),            # a row and three columns behind the last whole tile
+    (4, 64, 17, 130, "8,16", {"pad_out": 1}),         # four channels, two blocks of output channels
+    (3, 12, 3, 15, "4,16", {}),                       # fewer rows and columns than a tile has, a ragged block
+    (1, 32, 100, 600, "4,16", {"bn": True}),          # 250 tiles
+    (3, 32, 150, 640, "5,16", {}),                    # 300 tiles: workgroups walk two
+    (3, 40, 200, 700, "8,16", {}),                    # 275 tiles, a second block that holds 8 channels
+]
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("shallow", [False, True], ids=["deep", "shallow"])
+@pytest.mark.parametrize("case", C4_ROW_CASES, ids=lambda c: "%dx%dx%d_to%d_%s" % (c[0], c[2], c[3], c[1], c[4].replace(",", "x")))
+def test_small_input_form_on_rows_of_sixteen_positions(case, shallow, storage, monkeypatch):
+    """The 9x9 first layer on tiles whose fragments are rows: against the oracle, and fp32 tensors against three fp16 passes
+    over the same tiles."""
+    cin, cout, h, w, tile, kw = case
+    if shallow:
+        kw = dict({k: v for k, v in kw.items() if k != "pad_out"}, deep=False, pad_in=0)
+    monkeypatch.setenv("FYNHIP_FORCE_P16_CONV", "1")
+    monkeypatch.setenv("FYNHIP_NO_D16_CONV", "1")
+    monkeypatch.setenv("FYNHIP_P16_TILE", tile)
+    wts = conv_block(1250 + cin + h, cout, 9, cin, bn=kw.get("bn", False))
+    x = prng.uniform(71 * cin + w, (cin, h, w), 0, 1)
+    got, info = run_single(conv_builder(9, cout, h, w, cin, 1, 1, A.NONE, **kw), storage, [x], wts)
+    ref = oracle_single(conv_builder(9, cout, h, w, cin, 1, 1, A.NONE, **kw), storage, [x], wts)
+    print("  ", info, "rel_l2=%.3e" % rel_l2(got, ref), flush=True)
+    assert ("conv_p16c4 f16+fp8-split" if storage == fa.STORAGE_F32 else "conv_p16c4 f16 ") in info and "th=%s tw=%s" % tuple(tile.split(",")) in info
+    assert rel_l2(got, ref) <= TOL[storage], info
+    if storage == fa.STORAGE_F32:
+        monkeypatch.setenv("FYNHIP_EXACT_SPLIT", "1")
+        exact, info = run_single(conv_builder(9, cout, h, w, cin, 1, 1, A.NONE, **kw), storage, [x], wts)
+        assert "conv_p16c4 f16x2-split" in info
+        # (the bounds of the other tiles: 22-bit operands, four-bit correction terms)
+        assert rel_l2(exact, ref) <= 2e-6
+        assert rel_l2(got, exact) <= 3e-5
+
+
 TP16_CASES = [
     # cin, cout, h, w, tile "h,w,channel groups", batch-norm
     (64, 32, 20, 26, "4,8,1", True),        # four tiles of positions side by side, ragged on both sides
