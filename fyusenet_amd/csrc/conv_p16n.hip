@@ -1,4 +1,4 @@
-// 3x3 convolutions between tensors of few channels (16 to 48 in, up to 48 out) with the window of a tile in LDS: the layers
+// 3x3 convolutions between tensors of few channels (16 to 64 in, up to 128 out) with the window of a tile in LDS: the layers
 // of small style nets and decoders (reference: gpu/vanilla/convlayerNxN_vanilla.cpp,
 // gpu/vanilla/fractionalconvlayerNxN_vanilla.cpp, gpu/deep/deepconvlayerNxN.cpp:129-211).
 //
@@ -10,13 +10,14 @@
 //
 // Such a layer is a launch's start, one memory round trip and about a microsecond of work, so everything is requested at
 // once and nothing runs twice: a workgroup of four waves takes tiles of TH rows of sixteen positions and all output
-// channels; its waves all stage, then each takes every fourth step (its weights stay in registers from tile to tile: no
+// channels (a block of them where there are too few tiles for the chip); its waves all stage, then each takes every fourth step (its weights stay in registers from tile to tile: no
 // two waves read the same ones, which is what a split by positions would cost), and the partial sums meet in LDS, where the
 // fragments are dealt to the waves for the epilogue.  The next tile's window is requested before this one's matrix
 // instructions.
 // Measured (fp32 tensors, one launch): 12 -> 20 channels, step 2, at 312x256 positions 13.2 -> 11.0 us (conv_g16), at 24x32
 // 6.4 -> 4.0 (conv_p16); 20 -> 40, step 2, at 12x16 6.0 -> 4.7 (conv_mfma); 40 -> 20 at step 1/2, 156x128 9.1 -> 7.6, 12x16
-// 7.4 -> 5.0; 20 -> 12 at step 1/4, 24x32 5.8 -> 3.8; 40 -> 40 at 156x128 with a residual 8.2 -> 8.0.  The samples' 3x3 style
+// 7.4 -> 5.0; 20 -> 12 at step 1/4, 24x32 5.8 -> 3.8; 40 -> 40 at 156x128 with a residual 8.2 -> 8.0; 64 -> 64 at
+// 56x56 5.7 -> 5.2 (conv_kr16, whose waves split whole chunks of 32 channels: two of four had none).  The samples' 3x3 style
 // net on a 64x48 frame 77.7 -> 69.7 us.  Bound: a launch's start and its memory round trip (a microsecond of matrix
 // instructions in 40 -> 40 at 156x128), on large images the conversion and the partial sums beside them.
 #include <hip/hip_runtime.h>
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(256, 2) void conv_p16n_kernel(const ConvP16Params p
     typedef float f32x8_t __attribute__((ext_vector_type(8)));
     typedef typename std::conditional<HS, half8_t, f32x8_t>::type raw_t;
     extern __shared__ __align__(16) unsigned char lds[];
-    if (blockIdx.x == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
+    if ((blockIdx.x | blockIdx.y) == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int mq = lane & 15, kq = lane >> 4;
@@ -76,6 +77,7 @@ __global__ __launch_bounds__(256, 2) void conv_p16n_kernel(const ConvP16Params p
         if (group < (per << 3)) group = (group & 7) * per + (group >> 3);
     }
     const int ntiles = p.tiles_x * p.tiles_y;
+    const int ch0 = (int)blockIdx.y * FR * 16;   // this grid row's block of output channels
 
     // ---- staging
     int i_yx[N::NB], l_off[N::NB];   // an item's pixel inside the window (row << 16 | column << 3 | group), its place in LDS
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void conv_p16n_kernel(const ConvP16Params p
         for (int f = 0; f < FR; f++)
 #pragma unroll
             for (int pl = 0; pl < NPL; pl++)
-                a[s][f][pl] = *reinterpret_cast<const half8_t*>(reinterpret_cast<const unsigned char*>(p.wpack) + ((f * NS + step) * NPL + pl) * 1024 + lane * 16);
+                a[s][f][pl] = *reinterpret_cast<const half8_t*>(reinterpret_cast<const unsigned char*>(p.wpack) + (((int)blockIdx.y * FR + f) * NS + step) * NPL * 1024 + pl * 1024 + lane * 16);
     }
     const bool last_step = wave + 4 * (SPW - 1) < NS;                  // whether the wave has one (the same for all lanes)
     const bool pad_lane = 4 * (wave + 4 * (SPW - 1)) + kq >= 9 * G;    // its group is padding: zeros, whatever lies there
@@ -130,8 +132,8 @@ __global__ __launch_bounds__(256, 2) void conv_p16n_kernel(const ConvP16Params p
     if (p.in_amax) in_scale = range_scale(range_after_act(range_reduce(range_bits), p.act), &inv_in_scale);
     const float acc_mul = p.acc_mul * inv_in_scale;
     if (tid < FR * 16) {
-        reinterpret_cast<float*>(lds + N::SB)[tid] = p.scale[tid];
-        reinterpret_cast<float*>(lds + N::SB)[FR * 16 + tid] = p.bias[tid];
+        reinterpret_cast<float*>(lds + N::SB)[tid] = p.scale[ch0 + tid];
+        reinterpret_cast<float*>(lds + N::SB)[FR * 16 + tid] = p.bias[ch0 + tid];
     }
     const float res_floor = p.res_relu ? 0.f : -__builtin_inff();
     float vmax = 0.f;
@@ -181,14 +183,14 @@ __global__ __launch_bounds__(256, 2) void conv_p16n_kernel(const ConvP16Params p
             const int q = wave + 4 * i;
             f = q / TH;
             py = tyi * TH + q - f * TH;
-            return q < N::NQ && py < p.npos_y && px < p.npos_x && f * 16 + kq * 4 + 4 <= p.out_cp;   // (the last fragment may reach beyond the channel pitch)
+            return q < N::NQ && py < p.npos_y && px < p.npos_x && ch0 + f * 16 + kq * 4 + 4 <= p.out_cp;   // (the last fragment may reach beyond the channel pitch)
         };
         if (p.res) {
 #pragma unroll
             for (int i = 0; i < N::NO; i++) {
                 int f, py;
                 const bool ok = mine(i, f, py);
-                const store_t* r = reinterpret_cast<const store_t*>(p.res) + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + f * 16 + kq * 4 : 0);
+                const store_t* r = reinterpret_cast<const store_t*>(p.res) + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + ch0 + f * 16 + kq * 4 : 0);
                 if constexpr (HS) *reinterpret_cast<half4_t*>(rv[i]) = *reinterpret_cast<const half4_t*>(r);
                 else *reinterpret_cast<f32x4_t*>(rv[i]) = *reinterpret_cast<const f32x4_t*>(r);
             }
@@ -247,7 +249,7 @@ __global__ __launch_bounds__(256, 2) void conv_p16n_kernel(const ConvP16Params p
                 if (p.res) v[e] = fmaf(fmaxf((float)rv[i][e], res_floor), p.res_scale ? sc[e] : 1.f, v[e]);
                 if constexpr (!HS) vmax = fmaxf(vmax, ok ? fabsf(v[e]) : 0.f);
             }
-            store_t* o = reinterpret_cast<store_t*>(p.out) + ((size_t)(p.out_off_y + py) * p.out_wp + p.out_off_x + px) * p.out_cp + f * 16 + kq * 4;
+            store_t* o = reinterpret_cast<store_t*>(p.out) + ((size_t)(p.out_off_y + py) * p.out_wp + p.out_off_x + px) * p.out_cp + ch0 + f * 16 + kq * 4;
             if constexpr (HS) {
                 half4_t hv;
 #pragma unroll
@@ -278,9 +280,11 @@ constexpr P16NEntry p16n_entry() {
 #define P16N_ROWS(HS, G, FR, S) p16n_entry<HS, G, FR, S, 2>(), p16n_entry<HS, G, FR, S, S == 1 ? 5 : 4>()
 #define P16N_FRAGS(HS, G, S) P16N_ROWS(HS, G, 1, S), P16N_ROWS(HS, G, 2, S), P16N_ROWS(HS, G, 3, S)
 #define P16N_STEPS(HS, G) P16N_FRAGS(HS, G, 1), P16N_FRAGS(HS, G, 2)
+// (64 input channels: a wave's weights for two fragments fill the registers that three take elsewhere)
+#define P16N_WIDE(HS) p16n_entry<HS, 8, 1, 1, 2>(), p16n_entry<HS, 8, 2, 1, 2>(), p16n_entry<HS, 8, 1, 1, 5>(), p16n_entry<HS, 8, 2, 1, 5>(), p16n_entry<HS, 8, 1, 2, 2>(), p16n_entry<HS, 8, 2, 2, 2>()
 const P16NEntry P16N_TABLE[] = {
-    P16N_STEPS(false, 2), P16N_STEPS(false, 3), P16N_STEPS(false, 5), P16N_FRAGS(false, 6, 1),
-    P16N_STEPS(true, 2), P16N_STEPS(true, 3), P16N_STEPS(true, 5), P16N_FRAGS(true, 6, 1),
+    P16N_STEPS(false, 2), P16N_STEPS(false, 3), P16N_STEPS(false, 5), P16N_FRAGS(false, 6, 1), P16N_WIDE(false),
+    P16N_STEPS(true, 2), P16N_STEPS(true, 3), P16N_STEPS(true, 5), P16N_FRAGS(true, 6, 1), P16N_WIDE(true),
 };
 const P16NEntry* p16n_find(const ConvP16Params& p) {
     for (const P16NEntry& e : P16N_TABLE)
@@ -294,20 +298,20 @@ size_t conv_p16n_lds_bytes(const ConvP16Params& p) {
     return e ? e->lds : 0;
 }
 
-// p.tile_h = rows of a tile (2, or 5 with a step of one and 4 with a step of two), p.wm = p.mfrags = fragments of 16 output channels (scale, bias and wpack hold 16 * wm
-// rows; rows beyond out_cp are not stored), tiles of tile_h x 16 positions, p.pos_groups = workgroups; weights, in_y0, in_x0,
+// p.tile_h = rows of a tile (2, or 5 with a step of one and 4 with a step of two), p.wm = fragments of 16 output channels per grid row, p.cout_blocks = grid rows, p.mfrags =
+// wm * cout_blocks (scale, bias and wpack hold 16 * mfrags rows; rows beyond out_cp are not stored), tiles of tile_h x 16 positions, p.pos_groups = workgroups; weights, in_y0, in_x0,
 // in_shift, in_clamp and stride as for launch_conv_g16.
 int launch_conv_p16n(const ConvP16Params& p, hipStream_t s) {
     const P16NEntry* e = p16n_find(p);
     if (!e) return -1;
     const long long in_elems = (long long)p.in_hp * p.in_wp * p.in_cp;
-    if (in_elems > (1ll << 30) || p.mfrags != p.wm || p.tiles_x < 1 || p.tiles_y < 1 || p.tiles_x * 16 < p.npos_x || p.tiles_y * p.tile_h < p.npos_y || p.pos_groups < 1 ||
+    if (in_elems > (1ll << 30) || p.mfrags != p.wm * p.cout_blocks || p.cout_blocks < 1 || p.cout_blocks > 16 || p.tiles_x < 1 || p.tiles_y < 1 || p.tiles_x * 16 < p.npos_x || p.tiles_y * p.tile_h < p.npos_y || p.pos_groups < 1 ||
         p.pos_groups > p.tiles_x * p.tiles_y || p.tiles_x * p.tiles_y > 4000000 || p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.out_cp % 4 != 0 || p.out_cp < 4 ||
         (p.res && (p.res_cp < p.out_cp || p.res_cp % 4 != 0)) || p.nreset < 0 || p.nreset > 4 || p.dw_in || p.in_mul || p.in2 || !p.in || !p.out || !p.wpack || !p.scale || !p.bias ||
         p.in_shift < 0 || p.in_shift > 8 || ((long long)p.in_hp << p.in_shift) > (1 << 28) || ((long long)p.in_wp << p.in_shift) > (1 << 28))
         return -5;
     if (e->lds > 160 * 1024 || ensure_lds(reinterpret_cast<const void*>(e->fn), e->lds) != 0) return -2;
-    hipLaunchKernelGGL(e->fn, dim3((unsigned)p.pos_groups), dim3(256), e->lds, s, p);
+    hipLaunchKernelGGL(e->fn, dim3((unsigned)p.pos_groups, (unsigned)p.cout_blocks), dim3(256), e->lds, s, p);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -788,23 +788,29 @@ class ConvLayer : public Layer {
     // have been compiled.
     void setup_p16n(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
         ConvP16Params q = small_channel_params(in_v, out_v, res_v, res_relu, res_scale);
-        q.wm = q.mfrags = (oc + 15) / 16;
-        q.cout_blocks = 1;
+        q.mfrags = (oc + 15) / 16;
         if ((long long)in_v.elems() > (1ll << 30)) return;
+        // (64 channels at image size belong to the forms on whole chunks: 23 against 13 us at 256x256, ahead up to 64x64)
+        if (in_v.cp > 48 && oh * ow > 8192 && !net->sw.get("FYNHIP_P16N_ROWS") && !net->sw.get("FYNHIP_FORCE_P16N_CONV")) return;
         int want = 0;   // FYNHIP_P16N_ROWS=rows of a tile (tests)
         if (const char* e = net->sw.get("FYNHIP_P16N_ROWS")) want = atoi(e);
         std::vector<ConvP16Params> cands;
-        for (int th : {5, 4, 2}) {
-            if (want && th != want) continue;
-            ConvP16Params c = q;
-            c.tile_h = th; c.tile_w = 16;
-            c.tiles_x = (ow + 15) / 16; c.tiles_y = (oh + th - 1) / th;
-            c.rcp_tiles_x = 1.0f / (float)c.tiles_x;
-            const size_t lds = conv_p16n_lds_bytes(c);
-            if (lds == 0 || lds > 160 * 1024 || (long long)c.tiles_x * c.tiles_y > 4000000) continue;
-            c.pos_groups = std::min(c.tiles_x * c.tiles_y, lds <= 80 * 1024 ? 512 : 256);
-            cands.push_back(c);
-        }
+        // as many fragments per workgroup as there are and fit, or fewer where that makes more workgroups than the chip holds otherwise
+        for (int fr = std::min(3, q.mfrags); fr >= 1; fr--)
+            for (int th : {5, 4, 2}) {
+                if (q.mfrags % fr != 0 || (want && th != want)) continue;
+                ConvP16Params c = q;
+                c.wm = fr;
+                c.cout_blocks = q.mfrags / fr;
+                c.tile_h = th; c.tile_w = 16;
+                c.tiles_x = (ow + 15) / 16; c.tiles_y = (oh + th - 1) / th;
+                c.rcp_tiles_x = 1.0f / (float)c.tiles_x;
+                const size_t lds = conv_p16n_lds_bytes(c);
+                if (lds == 0 || lds > 160 * 1024 || (long long)c.tiles_x * c.tiles_y > 4000000) continue;
+                if (!cands.empty() && cands[0].wm != fr && c.tiles_x * c.tiles_y * c.cout_blocks > 512) continue;
+                c.pos_groups = std::max(1, std::min(c.tiles_x * c.tiles_y, (lds <= 80 * 1024 ? 512 : 256) / c.cout_blocks));
+                cands.push_back(c);
+            }
         if (cands.empty()) return;
         const bool always = want || net->sw.get("FYNHIP_FORCE_P16N_CONV") != nullptr;
         const char* at = net->sw.get("FYNHIP_AUTOTUNE");
@@ -817,13 +823,13 @@ class ConvLayer : public Layer {
         } else if (tune_cache_triple(net, key, cached)) {
             pick = -1;
             for (size_t i = 0; cached[0] && i < cands.size(); i++)
-                if (cands[i].tile_h == cached[1]) pick = (int)i;
+                if (cands[i].tile_h == cached[1] && cands[i].wm == cached[2]) pick = (int)i;
         } else {
             timed = !(at && at[0] == '0');
             if (!timed) pick = -1;
         }
         if (pick < 0) return;
-        const size_t halves = (size_t)q.wm * q.cin_chunks * (q.f16 ? 1 : 2) * 64 * 8;
+        const size_t halves = (size_t)q.mfrags * q.cin_chunks * (q.f16 ? 1 : 2) * 64 * 8;
         void* const wp = net->dev_alloc(halves * 2, true);
         for (ConvP16Params& c : cands) c.wpack = wp;
         if (timed) {
@@ -838,9 +844,9 @@ class ConvLayer : public Layer {
                 t_other = std::min(t_other, time_calls(net, [&]() { run(net->stream); }, 10));
             }
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
-                fprintf(stderr, "[tune] 3x3 on %d channels, %dx%d positions, to %d: window in LDS (%d rows, %d workgroups) %.1f us, %s %.1f us\n", in_v.cp, oh, ow, oc,
-                        cands[pick].tile_h, cands[pick].pos_groups, best * 1e3f, own_info().c_str(), t_other * 1e3f);
-            tune_cache_store_triple(net, key, best < t_other ? 1 : 0, cands[pick].tile_h, 0);
+                fprintf(stderr, "[tune] 3x3 on %d channels, %dx%d positions, to %d: window in LDS (%d rows, %d fragment(s), %d workgroups) %.1f us, %s %.1f us\n", in_v.cp, oh, ow, oc,
+                        cands[pick].tile_h, cands[pick].wm, cands[pick].pos_groups * cands[pick].cout_blocks, best * 1e3f, own_info().c_str(), t_other * 1e3f);
+            tune_cache_store_triple(net, key, best < t_other ? 1 : 0, cands[pick].tile_h, cands[pick].wm);
             if (best >= t_other) pick = -1;
         }
         if (pick >= 0) {
@@ -1278,7 +1284,7 @@ class ConvLayer : public Layer {
                 (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_G16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") && !only_kr)
                 setup_g16(in_v, out_v, res_v, res_relu, res_scale);
             // ... and windows staged in LDS (a test that forces another form, or a tile of one, wants that form)
-            if (!h16 && !c4 && !d16 && !s16 && same_storage && k == 3 && dil == 1 && in_v.cp % 8 == 0 && oc <= 48 && out_v.cp % 4 == 0 && out_v.cp >= oc && d.in_channels <= in_v.cp &&
+            if (!h16 && !c4 && !d16 && !s16 && same_storage && k == 3 && dil == 1 && in_v.cp % 8 == 0 && oc <= 128 && out_v.cp % 4 == 0 && out_v.cp >= oc && d.in_channels <= in_v.cp &&
                 (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 4 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_P16N_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") &&
                 !net->sw.get("FYNHIP_P16_TILE") && !net->sw.get("FYNHIP_FORCE_G16_CONV") && !net->sw.get("FYNHIP_G16_FRAGS") && !only_kr)
                 setup_p16n(in_v, out_v, res_v, res_relu, res_scale);
@@ -1463,7 +1469,7 @@ class ConvLayer : public Layer {
         if (p16 && p16n) {
             char buf[240];
             snprintf(buf, sizeof(buf), "conv_p16n %s window of %dx16 positions in LDS: %d steps of four 8-channel groups over 4 waves, %d fragment(s) of 16 output channels, blocks=%d tiles=%d lds=%zu",
-                     pp.f16 ? "f16" : "f16x2-split", pp.tile_h, pp.cin_chunks, pp.wm, pp.pos_groups, pp.tiles_x * pp.tiles_y, conv_p16n_lds_bytes(pp));
+                     pp.f16 ? "f16" : "f16x2-split", pp.tile_h, pp.cin_chunks, pp.wm, pp.pos_groups * pp.cout_blocks, pp.tiles_x * pp.tiles_y, conv_p16n_lds_bytes(pp));
             return mode + buf;
         }
         if (p16 && g16) {

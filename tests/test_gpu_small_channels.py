@@ -79,6 +79,10 @@ WINDOWED = [
     (40, 36, 20, 20, 1, True, ActType.NONE, ActType.RELU, 2),
     (40, 12, 30, 47, 2, True, ActType.RELU, None, 4),
     (48, 33, 40, 23, 1, True, ActType.RELU, None, 5),            # channels behind the output's count
+    (64, 64, 9, 33, 1, True, ActType.RELU, ActType.RELU, 2),     # two blocks of output channels
+    (64, 88, 14, 20, 1, False, ActType.NONE, ActType.NONE, 5),   # three, the last with 24 channels (six fragments)
+    (64, 20, 22, 30, 2, True, ActType.RELU, None, 2),
+    (40, 64, 7, 18, 1, True, ActType.RELU, None, 5),             # four fragments, two a block
     (24, 8, 90, 1000, 1, False, ActType.RELU, None, 2),          # 2835 tiles: workgroups walk six
     (40, 40, 130, 400, 1, False, ActType.RELU, ActType.RELU, 5), # 650 tiles, the residual of a second tile
 ]
