@@ -501,12 +501,12 @@ class ConvLayer : public Layer {
         const size_t halves = (size_t)((oc + 31) / 32 * 2) * 4 * (q.cin_chunks / 4) * k * k * (q.f16 ? 1 : 2) * 64 * 8;
         void* const kr_wpack = net->dev_alloc(halves * 2, true);
         for (ConvP16Params& c : cands) c.wpack = kr_wpack;
-        const bool had_p16 = p16;   // the 3x3 16-position form was chosen over the general kernel: this form has to beat it instead
+        const bool had_p16 = p16;   // the 3x3 16-position form (h16: the wide one) was chosen over the general kernel: this form has to beat it instead
         const bool always = net->sw.get("FYNHIP_FORCE_KR16_CONV") != nullptr;
         const char* at = net->sw.get("FYNHIP_AUTOTUNE");
         int pick = 0;
         char key[160];
-        snprintf(key, sizeof(key), "kr16:k%d:%dx%d:%dx%d:s%d:r%d:e%d:h%d:p%d", k, d.in_channels, oc, oh, ow, stride, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, had_p16 ? 1 : 0);
+        snprintf(key, sizeof(key), "kr16:k%d:%dx%d:%dx%d:s%d:r%d:e%d:h%d:p%d", k, d.in_channels, oc, oh, ow, stride, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, h16 ? 2 : had_p16 ? 1 : 0);
         int cached[3] = {0, 0, 0};
         if (!want_fm && tune_cache_triple(net, key, cached)) {
             pick = -1;
@@ -525,7 +525,8 @@ class ConvLayer : public Layer {
                 }
                 if (had_p16)
                     t_other = std::min(t_other, time_calls(net, [&]() {
-                        if (launch_conv_p16(pp, net->stream) != 0) fail(FYN_ERR_DEVICE, "16-position convolution launch failed while tuning");
+                        if (h16 ? launch_conv_h16(pp, k, net->stream) != 0 || (h16_two && launch_conv_h16(pp2, k, net->stream) != 0) : launch_conv_p16(pp, net->stream) != 0)
+                            fail(FYN_ERR_DEVICE, "16-position convolution launch failed while tuning");
                     }, 10));
                 else
                     t_other = std::min(t_other, time_launch(net, launch, 10));
@@ -542,6 +543,7 @@ class ConvLayer : public Layer {
             if (had_p16) net->dev_free(p16_wpack_dev);
             p16_wpack_dev = kr_wpack;
             p16 = true; kr16 = true;
+            h16 = h16_two = false;
             pp = cands[pick];
         } else {
             net->dev_free(kr_wpack);
@@ -1256,7 +1258,9 @@ class ConvLayer : public Layer {
                 !net->sw.get("FYNHIP_NO_P16_CONV"))
                 setup_c4(in_v, out_v);
             // few positions, many input channels: the whole reduction of a 4x4 tile resident in LDS instead of K-split launches
-            if ((!p16 || (!h16 && !c4)) && !frac_shift && same_storage && (k == 1 || (k == 3 && (stride == 1 || stride == 2))) && dil == 1 && in_v.cp % 8 == 0 &&
+            // (against the wide fp16 form too: it has one workgroup per tile and 128 channels, 14 for 28x28 positions and 128
+            // channels, 6.0 us where this one takes 3.5)
+            if (!c4 && (!h16 || (!net->sw.get("FYNHIP_P16_TILE") && !net->sw.get("FYNHIP_H16_SPLIT"))) && !frac_shift && same_storage && (k == 1 || (k == 3 && (stride == 1 || stride == 2))) && dil == 1 && in_v.cp % 8 == 0 &&
                 d.in_channels == in_v.cp && in_v.cp >= 16 && oc % 4 == 0 && oc >= 8 && out_v.cp >= oc && oh * ow <= 4096 && (!res_v || (res_v->cp >= out_v.cp && res_v->cp % 8 == 0)) &&
                 !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_KR16_CONV") && !net->sw.get("FYNHIP_FORCE_P16_CONV") &&
                 // (a test that forces a variant of the general kernel wants the general kernel)

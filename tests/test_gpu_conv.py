@@ -483,6 +483,25 @@ def test_fp16_row_fragment_tiles(k, tile, h, w, residual, monkeypatch):
     assert rel_l2(got, ref) <= TOL[fa.STORAGE_F16], info   # (operands and result rounded to 11 bits, as in the test above)
 
 
+@pytest.mark.parametrize("tuned", [False, True])
+@pytest.mark.parametrize("h,w,residual", [(28, 28, True), (9, 49, False), (64, 64, True), (20, 26, False)])
+def test_fp16_wide_layers_of_few_positions(h, w, residual, tuned, monkeypatch):
+    """Up to 4096 positions the K-resident form is offered against the wide fp16 form too (untimed it is taken); whichever
+    it is, the weights are laid out for it and a second band of rows is not launched beside it."""
+    monkeypatch.setenv("FYNHIP_AUTOTUNE", "1" if tuned else "0")
+    kw = {"bn": True, "residual": (A.RELU, True)} if residual else {"pad_out": 1}
+    b = conv_builder(3, 128, h, w, 128, 1, 1, A.RELU, **kw)
+    wts = conv_block(2500 + h, 128, 3, 128, bn=residual)
+    inputs = [prng.uniform(41 * h + w, (128, h, w), -1, 1)]
+    if residual:
+        inputs.append(prng.uniform(67, (128, h, w), -1, 1))
+    got, info = run_single(b, fa.STORAGE_F16, inputs, wts)
+    ref = oracle_single(b, fa.STORAGE_F16, inputs, wts)
+    print("  ", info, "rel_l2=%.3e" % rel_l2(got, ref), flush=True)
+    assert tuned or "conv_kr16" in info
+    assert rel_l2(got, ref) <= TOL[fa.STORAGE_F16], info   # (as in the test above)
+
+
 KR16_CASES = [
     # (k, cin, cout, h, w, fragments per block, kw)
     (1, 1024, 256, 14, 14, 1, {}),                                              # a ResNet stage-3 reduction layer
