@@ -79,7 +79,7 @@ def main():
         c = _find(os.path.join(a.dir, sub), "copy", "counter_collection")
         if not f or not c:
             continue
-        cal = counter_avg(c, counter, "concat")
+        cal = counter_avg(c, counter, "concat|cat_kernel")
         if not cal:
             continue
         cal_v = list(cal.values())[0][0]
