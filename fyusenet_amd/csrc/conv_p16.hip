@@ -2312,9 +2312,13 @@ static bool p16_uses_fp8(const ConvP16Params& p) {
 bool conv_p16_uses_fp8(const ConvP16Params& p) { return p16_uses_fp8(p); }
 #endif
 
+// (tiles whose fragments are rows reach their weights as a buffer through 32-bit offsets; the other tiles walk them by pointer)
+static bool rows_weights_fit(const ConvP16Params& p) {
+    return (size_t)p.cin_chunks * NT * p.mfrags * NPLW * 1024 < (size_t)1 << 31;
+}
 static const P16Entry* find_entry(const ConvP16Params& p) {
     for (const P16Entry& c : kEntries)
-        if (c.th == p.tile_h && c.tw == p.tile_w && c.stride == p.stride && c.wm == p.wm) return &c;
+        if (c.th == p.tile_h && c.tw == p.tile_w && c.stride == p.stride && c.wm == p.wm) return c.tw != 16 || rows_weights_fit(p) ? &c : nullptr;
     return nullptr;
 }
 size_t P16_NAME(conv_p16_lds_bytes)(const ConvP16Params& p) {

@@ -290,7 +290,7 @@ inline int p16_row_channel(int mf, int row, int fm) { return (mf / fm) * 16 * fm
 bool conv_p16_supported(int k, int stride, int dil, int in_cp, int cout, int out_cp, bool f16);
 int conv_p16_tile_count();
 void conv_p16_tile(int index, int* th, int* tw, int* stride, int* wm);
-size_t conv_p16_lds_bytes(const ConvP16Params& p);   // 0: no such compiled combination
+size_t conv_p16_lds_bytes(const ConvP16Params& p);   // 0: no such compiled combination, or none for weights of this size
 // fp32 tensors: wpack of launch_conv_p16 / launch_tconv_p16 has three planes per fragment (fp16 hi, fp16 lo, and
 // [8 x fp8(hi / 32) | 8 x fp8(64 lo)] per lane); this fills the third from src = [fragment][lane][those sixteen floats]
 int launch_pack_fp8_plane(const float* src, void* wpack, size_t frags, hipStream_t s);
