@@ -346,7 +346,8 @@ const H16Entry H16_TABLE[] = {
 constexpr int H16_COUNT = sizeof(H16_TABLE) / sizeof(H16_TABLE[0]);
 const H16Entry* h16_find(const ConvP16Params& p, int k) {
     for (int i = 0; i < H16_COUNT; i++)
-        if (H16_TABLE[i].k == k && H16_TABLE[i].th == p.tile_h && H16_TABLE[i].tw == p.tile_w) return &H16_TABLE[i];
+        if (H16_TABLE[i].k == k && H16_TABLE[i].th == p.tile_h && H16_TABLE[i].tw == p.tile_w)
+            return (size_t)p.cin_chunks * k * k * p.mfrags * 1024 < (size_t)1 << 31 ? &H16_TABLE[i] : nullptr;   // (offsets into the weights are 32 bits wide)
     return nullptr;
 }
 }  // namespace
@@ -373,8 +374,7 @@ int launch_conv_h16(const ConvP16Params& p, int k, hipStream_t s) {
         (p.res && p.res_cp < p.cout_blocks * 128) || (p.res && p.cin_chunks < 2 && p.pos_groups != p.tiles_x * p.tiles_y) ||
         p.pos_groups < 1 || p.pos_groups > p.tiles_x * p.tiles_y || p.tiles_x < 1 || p.tiles_y < 1 || !p.f16 ||
         p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.tiles_x * p.tiles_y > 4000000 || p.in_cp % 8 != 0 || p.out_cp % 8 != 0 || (p.res && p.res_cp % 8 != 0) ||
-        p.tiles_x * 2 * e->tw < p.npos_x || p.tiles_y * e->th < p.npos_y || !p.in || !p.out || !p.wpack || !p.scale || !p.bias ||
-        (size_t)p.cin_chunks * k * k * p.mfrags * 1024 >= (size_t)1 << 31)   // (offsets into the weights are 32 bits wide)
+        p.tiles_x * 2 * e->tw < p.npos_x || p.tiles_y * e->th < p.npos_y || !p.in || !p.out || !p.wpack || !p.scale || !p.bias)
         return -1;
     const size_t lds = conv_h16_lds_bytes(p, k);
     if (ensure_lds(reinterpret_cast<const void*>(e->fn), lds) != 0) return -2;

@@ -352,7 +352,7 @@ int launch_conv_kr16(const ConvP16Params& p, int k, hipStream_t s);
 bool conv_h16_supported(int k, int stride, int dil, int in_cp, int cout, int out_cp, bool f16);
 int conv_h16_tile_count();
 void conv_h16_tile(int index, int* k, int* th, int* tw);
-size_t conv_h16_lds_bytes(const ConvP16Params& p, int k);
+size_t conv_h16_lds_bytes(const ConvP16Params& p, int k);   // 0: as for conv_p16_lds_bytes
 int launch_conv_h16(const ConvP16Params& p, int k, hipStream_t s);
 
 // ---------------------------------------------------------------------------------------------

@@ -55,7 +55,22 @@ static int p16_rows() {
     return 0;
 }
 
+// conv_h16 (wide fp16 tensors): a layer that it cannot take has no candidates and keeps the forms behind it
+static int h16() {
+    for (int k : {3, 9})
+        for (int rows : {12, 10, 8, 6, 5, 4}) {
+            // 9x9: 3584 -> 3584 channels 2.08e9 bytes, 3712 -> 3712 2.23e9; 3x3: 10752 -> 10752 2.08e9, 11008 -> 11008 2.18e9
+            ConvP16Params p = layer(k == 9 ? 3584 : 10752, k == 9 ? 3584 : 10752, rows, 8, 4, true);
+            CHECK(conv_h16_lds_bytes(p, k) != 0);
+            p = layer(k == 9 ? 3712 : 11008, k == 9 ? 3712 : 11008, rows, 8, 4, true);
+            CHECK(conv_h16_lds_bytes(p, k) == 0);
+            CHECK(launch_conv_h16(p, k, nullptr) == -1);
+        }
+    return 0;
+}
+
 int main(int argc, char** argv) {
+    if (argc == 2 && !strcmp(argv[1], "h16")) return h16();
     if (argc == 2 && !strcmp(argv[1], "p16_rows")) return p16_rows();
     return 2;
 }
