@@ -538,6 +538,13 @@ class ConvLayer : public Layer {
             const bool win = best < t_other;
             if (!want_fm) tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].wm, cands[pick].tile_h * 100 + cands[pick].tile_w);
             if (!win && !always) pick = -1;
+        } else if (h16 && cands[0].pos_groups * cands[0].cout_blocks > 1280) {
+            // (nothing timed: a workgroup per 16 positions and 16 channels against one per tile of 64 and 128.  64 to 1024
+            // channels -> 128 to 512, 8x8 to 64x64 positions, both as they run untimed: up to five workgroups per CU this
+            // form is ahead -- 128 -> 128 at 28x28, 392 of them, 3.7 against 6.2 us; at 48x48, 1152, 6.0 / 6.4 -- but for
+            // 64 -> 128 at 48x48 (5.4 / 4.8); from 1568 on it is behind: 128 -> 128 at 56x56 7.2 / 6.4, 64x64 8.5 / 6.5,
+            // 512 -> 512 at 64x64 72 / 22; but for 512 -> 512 at 28x28, 18.0 / 19.0)
+            pick = -1;
         }
         if (pick >= 0) {
             if (had_p16) net->dev_free(p16_wpack_dev);
