@@ -295,6 +295,11 @@ P16_CASES = [
     (20, 40, 38, 44, 2, "8,6,2", {"bn": True}),                                    # fewer channels than the tensors' pitch (conv3 and conv2 of those nets)
     (12, 20, 50, 36, 2, "4,8,2", {}),
     (44, 48, 23, 19, 1, "8,8,2", {"residual": (A.RELU, False)}),
+    # the residual tile in shares over more chunks than two, workgroups walking tiles
+    (128, 128, 70, 71, 1, "4,4,4", {"bn": True, "residual": (A.RELU, True)}),      # 324 tiles, one share
+    (192, 256, 67, 97, 1, "4,8,4", {"residual": (A.NONE, False)}),                 # 221 on 128 workgroups, six chunks
+    (96, 256, 82, 90, 1, "8,8,4", {"bn": True, "residual": (A.NONE, True)}),       # 132 on 128, three chunks: three passes on fp32 tensors
+    (128, 512, 134, 142, 2, "8,8,4", {"residual": (A.RELU, False)}),               # stride 2, 81 on 64
 ]
 
 
@@ -360,6 +365,15 @@ P16_ROW_CASES = [
     (256, 128, 7, 20, "6,16,4", {"residual": (A.RELU, False)}),                  # eight chunks; every second workgroup begins with the third
     (192, 128, 40, 33, "4,16,4", {"bn": True}),                                  # six
     (128, 256, 3, 15, "4,16,4", {"residual": (A.NONE, True)}),                   # fewer rows and columns than a tile has
+    # workgroups that walk two tiles or three, with a residual tile that arrives in shares over a tile's chunks while the
+    # tile before it is finished, every second of them beginning each tile with its third chunk
+    (128, 128, 67, 261, "4,16,4", {"bn": True, "residual": (A.RELU, True)}),     # 289 tiles on 256 workgroups; two shares, four chunks
+    (192, 256, 59, 181, "5,16,4", {"residual": (A.NONE, False)}),                # 144 on 128; three shares, six chunks
+    (128, 256, 91, 185, "8,16,4", {"bn": True, "residual": (A.NONE, True)}),     # 144 on 128; four shares, four chunks
+    (256, 256, 71, 183, "6,16,4", {"residual": (A.RELU, False)}),                # 144 on 128; three shares, eight chunks
+    (64, 64, 71, 470, "4,16,2", {"residual": (A.RELU, False)}),                  # 270 on 256; two chunks: all shares in the second
+    (128, 64, 101, 500, "6,16,2", {"bn": True, "residual": (A.NONE, True)}),     # 272 on 256; three shares, four chunks
+    (128, 512, 61, 180, "4,16,4", {"residual": (A.RELU, False)}),                # 192 on 64: three tiles each
 ]
 
 
