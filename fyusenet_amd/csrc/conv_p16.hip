@@ -2101,7 +2101,9 @@ constexpr P16Entry entry() {
 const P16Entry kEntries[] = {
     entry<8, 10, 1, 4>(), entry<10, 8, 1, 4>(), entry<8, 8, 1, 4>(), entry<8, 6, 1, 4>(), entry<4, 8, 1, 4>(), entry<4, 4, 1, 4>(),
     entry<8, 8, 1, 2>(), entry<8, 6, 1, 2>(), entry<4, 8, 1, 2>(),
+#if !FYN_P16_HALF   // (rows of sixteen: offered in the fp8 form.  Their three-pass form is what runs where a tensor loses its value-range word behind that choice: Net::assign_range_resets)
     entry<8, 16, 1, 4>(), entry<6, 16, 1, 4>(), entry<5, 16, 1, 4>(), entry<4, 16, 1, 4>(), entry<6, 16, 1, 2>(), entry<4, 16, 1, 2>(),
+#endif
     entry<10, 8, 2, 4>(), entry<8, 10, 2, 4>(), entry<8, 8, 2, 4>(),
     entry<8, 6, 2, 2>(), entry<4, 8, 2, 2>(), entry<8, 4, 2, 2>(),
 };
@@ -2173,7 +2175,7 @@ const KREntry kKRSrcEntries[] = {FYN_KR_SRC(1), FYN_KR_SRC(2), FYN_KR_SRC(3), FY
 }  // namespace
 
 // Host entry points.  The fp32 unit holds the public ones and hands launches on fp16 tensors (p.f16) to the other
-// unit's, which carry the suffix _half; tile tables are the same in both.
+// unit's, which carry the suffix _half; what its tables do not have (an LDS size of 0) is not offered to such tensors.
 #if FYN_P16_HALF
 #define P16_NAME(n) n##_half
 #else

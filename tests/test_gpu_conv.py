@@ -6,7 +6,8 @@ import numpy as np
 import pytest
 
 import fyusenet_amd as fa
-from fyusenet_amd import prng
+from fyusenet_amd import networks, prng
+from oracle import oracle as O
 from util import combos, conv_block, oracle_single, rel_l2, run_single
 
 pytestmark = pytest.mark.gpu
@@ -405,6 +406,43 @@ def test_fp8_form_on_rows_of_sixteen_positions(case, shallow, monkeypatch):
     # (three passes over 22-bit operands; the correction terms, 2^-11 of the result, carry four bits: the bounds of the other tiles)
     assert rel_l2(exact, ref) <= 2e-6
     assert rel_l2(got, exact) <= 3e-5
+
+
+class _TwoLayers(networks._StreamNet):
+    """Two 3x3 layers and nothing behind them: no launch is left to clear the value-range word of the tensor between them."""
+    config_id, input_key, output_layer = 11, (1, 0), 2
+
+    def __init__(self, storage, channels, h, w):
+        super().__init__(storage)
+        self.sizes = channels, h, w
+
+    def define(self):
+        c, h, w = self.sizes
+        self.conv(1, "a", 3, c, c, h, w, None, act=A.RELU, pad_out=1)
+        self.conv(2, "b", 3, c, c, h, w, 1, act=A.RELU)
+
+    def setInput(self, x):
+        self.layers[1].setInput(x, 0)
+
+
+def test_row_tile_whose_input_loses_its_value_range(monkeypatch):
+    """A layer chooses its tile while its input has a value-range word; where the word is given up behind that (nothing to
+    clear it), the chosen row tile runs in three fp16 passes."""
+    monkeypatch.setenv("FYNHIP_AUTOTUNE", "0")
+    x = prng.uniform(97, (128, 128, 256), -1, 1)
+    net = _TwoLayers(fa.STORAGE_F32, 128, 128, 256)   # (256 tiles of eight rows: one for every CU)
+    net.setup()
+    for _ in range(2):
+        net.setInput(x)
+        net.forward()
+        net.finish()
+    got, infos = net.getOutput(2), [net.layers[i].kernelInfo() for i in (1, 2)]
+    net.cleanup()
+    print(infos, flush=True)
+    assert "conv_p16 f16+fp8-split" in infos[0] and "tw=16" in infos[0]
+    assert "conv_p16 f16x2-split" in infos[1] and "tw=16" in infos[1]
+    want = O.run_network(net.describe(), {net.input_key: x})[2]
+    assert rel_l2(got, want) <= 3e-5    # (the first layer's correction terms carry four bits of 2^-11 of the result)
 
 
 H16_CASES = [
