@@ -162,6 +162,26 @@ bool tune_cache_triple(Net* net, const char* key, int (&out)[3]);
 
 void tune_cache_store_triple(Net* net, const char* key, int a, int b, int c);
 
+// The candidate that an earlier setup measured as the best of its own: is(i, b, c) says whether candidate i is the one
+// noted as (1, b, c); *pick = -1 where it was slower than the other form (always: it is taken all the same).  False where
+// nothing is noted, and where what is noted is not offered here -- which candidates there are depends on more than a key
+// names, and a file may come from another build --: the layer is measured again.
+template <class Is>
+bool tune_cache_pick(Net* net, const char* key, size_t n, bool always, Is&& is, int* pick) {
+    int noted[3] = {0, 0, 0};
+    if (!tune_cache_triple(net, key, noted)) return false;
+    if (!noted[0] && !always) {
+        *pick = -1;
+        return true;
+    }
+    for (size_t i = 0; i < n; i++)
+        if (is(i, noted[1], noted[2])) {
+            *pick = (int)i;
+            return true;
+        }
+    return false;
+}
+
 // Picks the tile configuration of one (sub-)convolution: by measurement on the layer's own tensors (default), or by
 // the heuristic score when FYNHIP_AUTOTUNE=0.  Candidates are timed before the weights are packed, i.e. on zero
 // operands; the matrix pipes run about a tenth faster on those than on real data (the part holds a higher clock when

@@ -188,16 +188,9 @@ class ConvLayer : public Layer {
         const bool timing = !(at && at[0] == '0');
         int pick = 0;   // index into cands, -1: the general kernel
         char key[160];
-        snprintf(key, sizeof(key), "p16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
-        int cached[3] = {0, 0, 0};
-        bool have_cached = false;
-        if (!want_h) have_cached = tune_cache_triple(net, key, cached);   // (the cache keeps: chosen?, tile_h*1000 + tile_w, wm)
-        if (have_cached) {
-            pick = -1;
-            if (cached[0] || always)
-                for (size_t i = 0; i < cands.size(); i++)
-                    if (cands[i].q.tile_h * 1000 + cands[i].q.tile_w == cached[1] && cands[i].q.wm == cached[2]) pick = (int)i;
-            if (always && pick < 0) pick = 0;
+        snprintf(key, sizeof(key), "p16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d:q%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift, conv_p16_uses_fp8(q) ? 1 : 0);
+        // (the cache keeps: chosen?, tile_h*1000 + tile_w, wm)
+        if (!want_h && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return cands[i].q.tile_h * 1000 + cands[i].q.tile_w == b && cands[i].q.wm == c; }, &pick)) {
         } else if (timing) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
@@ -272,13 +265,7 @@ class ConvLayer : public Layer {
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "c4p16:k%d:%dx%d:%dx%d:e%d:h%d", k, d.in_channels, oc, oh, ow, clamp ? 1 : 0, q.f16);
-        int cached[3] = {0, 0, 0};
-        if (!want_h && tune_cache_triple(net, key, cached)) {
-            pick = -1;
-            if (cached[0] || always)
-                for (size_t i = 0; i < cands.size(); i++)
-                    if (cands[i].tile_h * 1000 + cands[i].tile_w == cached[1]) pick = (int)i;
-            if (always && pick < 0) pick = 0;
+        if (!want_h && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int) { return cands[i].tile_h * 1000 + cands[i].tile_w == b; }, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
@@ -400,13 +387,7 @@ class ConvLayer : public Layer {
         // (the cache keeps: chosen?, tile_h*1000 + tile_w of the first band, rows*1000 + tile_h of the second or 0)
         auto code1 = [](const Cand& c) { return c.a.tile_h * 1000 + c.a.tile_w; };
         auto code2 = [](const Cand& c) { return c.two ? c.a.npos_y * 1000 + c.b.tile_h : 0; };
-        int cached[3] = {0, 0, 0};
-        if (!forced && tune_cache_triple(net, key, cached)) {
-            pick = -1;
-            if (cached[0] || always)
-                for (size_t i = 0; i < cands.size(); i++)
-                    if (code1(cands[i]) == cached[1] && code2(cands[i]) == cached[2]) pick = (int)i;
-            if (always && pick < 0) pick = 0;
+        if (!forced && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return code1(cands[i]) == b && code2(cands[i]) == c; }, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 2; rep++) {
@@ -507,13 +488,7 @@ class ConvLayer : public Layer {
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "kr16:k%d:%dx%d:%dx%d:s%d:r%d:e%d:h%d:p%d", k, d.in_channels, oc, oh, ow, stride, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, h16 ? 2 : had_p16 ? 1 : 0);
-        int cached[3] = {0, 0, 0};
-        if (!want_fm && tune_cache_triple(net, key, cached)) {
-            pick = -1;
-            if (cached[0] || always)
-                for (size_t i = 0; i < cands.size(); i++)
-                    if (cands[i].wm == cached[1] && cands[i].tile_h * 100 + cands[i].tile_w == cached[2]) pick = (int)i;
-            if (always && pick < 0) pick = 0;
+        if (!want_fm && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return cands[i].wm == b && cands[i].tile_h * 100 + cands[i].tile_w == c; }, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
@@ -751,14 +726,9 @@ class ConvLayer : public Layer {
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "g16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
-        int cached[3] = {0, 0, 0};
         bool timed = false;
         if (always) {
-        } else if (tune_cache_triple(net, key, cached)) {
-            pick = -1;
-            for (size_t i = 0; cached[0] && i < cands.size(); i++)
-                if (cands[i].wm == cached[1]) pick = (int)i;
-        } else {
+        } else if (!tune_cache_pick(net, key, cands.size(), false, [&](size_t i, int b, int) { return cands[i].wm == b; }, &pick)) {
             timed = !(at && at[0] == '0');
             if (!timed) pick = -1;
         }
@@ -826,14 +796,9 @@ class ConvLayer : public Layer {
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "p16n:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
-        int cached[3] = {0, 0, 0};
         bool timed = false;
         if (always) {
-        } else if (tune_cache_triple(net, key, cached)) {
-            pick = -1;
-            for (size_t i = 0; cached[0] && i < cands.size(); i++)
-                if (cands[i].tile_h == cached[1] && cands[i].wm == cached[2]) pick = (int)i;
-        } else {
+        } else if (!tune_cache_pick(net, key, cands.size(), false, [&](size_t i, int b, int c) { return cands[i].tile_h == b && cands[i].wm == c; }, &pick)) {
             timed = !(at && at[0] == '0');
             if (!timed) pick = -1;
         }

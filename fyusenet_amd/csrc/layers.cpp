@@ -118,13 +118,7 @@ class TransConvLayer : public Layer {
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "tp16:%dx%d:%dx%d:cp%d:h%d", d.in_channels, oc, d.height, d.width, in_v.cp, q.f16);
-        int cached[3] = {0, 0, 0};
-        if (!want_h && tune_cache_triple(net, key, cached)) {
-            pick = -1;
-            if (cached[0] || always)
-                for (size_t i = 0; i < cands.size(); i++)
-                    if (cands[i].tile_h * 1000 + cands[i].tile_w == cached[1] && cands[i].wm == cached[2]) pick = (int)i;
-            if (always && pick < 0) pick = 0;
+        if (!want_h && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return cands[i].tile_h * 1000 + cands[i].tile_w == b && cands[i].wm == c; }, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {

@@ -1118,3 +1118,44 @@ def test_tuning_choices_are_remembered_across_processes(tmp_path):
     assert runs[0][1] == runs[1][1]                      # nothing measured again
     lines = runs[0][1].splitlines()
     assert len(lines) >= 4 and all(len(ln.split()) == 8 for ln in lines)
+
+
+_FORMS_CHILD = r"""
+import sys
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests")
+import fyusenet_amd as fa
+from fyusenet_amd import prng
+from util import conv_block, run_single
+from test_gpu_conv import conv_builder
+for k, cin, cout, h, w, storage in ((3, 128, 128, 67, 261, fa.STORAGE_F32), (9, 128, 128, 96, 80, fa.STORAGE_F16), (9, 3, 32, 200, 300, fa.STORAGE_F32)):
+    b = conv_builder(k, cout, h, w, cin, 1, 1, fa.ActType.NONE, pad_out=1)
+    print(run_single(b, storage, [prng.uniform(5, (cin, h, w), -1, 1)], conv_block(900 + k, cout, k, cin))[1].split("tile=")[0])
+"""
+
+
+def _forms(cache, **switches):
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _FORMS_CHILD, root], env=dict(os.environ, FYNHIP_AUTOTUNE="1", FYNHIP_TUNE_CACHE=str(cache), **switches),
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    print(r.stdout, flush=True)
+    return r.stdout.splitlines()
+
+
+def test_noted_choices_that_are_not_offered_are_measured_again(tmp_path):
+    """A noted tile that the layer is not offered (a file of a build with other tiles; a layer of the same geometry that runs
+    in three passes, without the tiles of the fp8 form) does not drop the form: it is measured again."""
+    cache = tmp_path / "tune.txt"
+    first = _forms(cache)
+    assert "conv_p16 f16+fp8-split" in first[0] and "conv_h16" in first[1] and "conv_p16c4" in first[2]
+    noted = cache.read_text()
+    other = ["%s 1 7007 %s" % (ln.split()[0], ln.split(None, 3)[3]) if ln.split(":")[0] in ("p16", "h16", "c4p16") else ln for ln in noted.splitlines()]
+    assert sum(" 1 7007 " in ln for ln in other) == 3
+    cache.write_text("\n".join(other) + "\n")
+    assert _forms(cache) == first
+    cache.write_text(noted)
+    exact = _forms(cache, FYNHIP_EXACT_SPLIT="1")
+    assert "conv_p16 f16x2-split" in exact[0] and exact[1:2] == first[1:2] and "conv_p16c4" in exact[2]
