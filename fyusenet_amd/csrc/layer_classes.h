@@ -795,7 +795,9 @@ class ConvLayer : public Layer {
         const char* at = net->sw.get("FYNHIP_AUTOTUNE");
         int pick = 0;
         char key[160];
-        snprintf(key, sizeof(key), "p16n:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift);
+        // (o: the form chosen so far, against which the note was taken)
+        snprintf(key, sizeof(key), "p16n:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d:o%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift,
+                 g16 ? 4 : kr16 ? 3 : p16 ? (conv_p16_uses_fp8(pp) ? 2 : 1) : 0);
         bool timed = false;
         if (always) {
         } else if (!tune_cache_pick(net, key, cands.size(), false, [&](size_t i, int b, int c) { return cands[i].tile_h == b && cands[i].wm == c; }, &pick)) {

@@ -1127,18 +1127,20 @@ import fyusenet_amd as fa
 from fyusenet_amd import prng
 from util import conv_block, run_single
 from test_gpu_conv import conv_builder
-for k, cin, cout, h, w, storage in ((3, 128, 128, 67, 261, fa.STORAGE_F32), (9, 128, 128, 96, 80, fa.STORAGE_F16), (9, 3, 32, 200, 300, fa.STORAGE_F32)):
+cases = {"forms": ((3, 128, 128, 67, 261, fa.STORAGE_F32), (9, 128, 128, 96, 80, fa.STORAGE_F16), (9, 3, 32, 200, 300, fa.STORAGE_F32)),
+         "few channels": ((3, 40, 40, 156, 128, fa.STORAGE_F32),)}
+for k, cin, cout, h, w, storage in cases[sys.argv[2]]:
     b = conv_builder(k, cout, h, w, cin, 1, 1, fa.ActType.NONE, pad_out=1)
     print(run_single(b, storage, [prng.uniform(5, (cin, h, w), -1, 1)], conv_block(900 + k, cout, k, cin))[1].split("tile=")[0])
 """
 
 
-def _forms(cache, **switches):
+def _forms(cache, which="forms", **switches):
     import os
     import subprocess
     import sys
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    r = subprocess.run([sys.executable, "-c", _FORMS_CHILD, root], env=dict(os.environ, FYNHIP_AUTOTUNE="1", FYNHIP_TUNE_CACHE=str(cache), **switches),
+    r = subprocess.run([sys.executable, "-c", _FORMS_CHILD, root, which], env=dict(os.environ, FYNHIP_AUTOTUNE="1", FYNHIP_TUNE_CACHE=str(cache), **switches),
                        capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-2000:]
     print(r.stdout, flush=True)
@@ -1159,3 +1161,15 @@ def test_noted_choices_that_are_not_offered_are_measured_again(tmp_path):
     cache.write_text(noted)
     exact = _forms(cache, FYNHIP_EXACT_SPLIT="1")
     assert "conv_p16 f16x2-split" in exact[0] and exact[1:2] == first[1:2] and "conv_p16c4" in exact[2]
+
+
+def test_few_channel_choices_are_noted_by_what_they_were_measured_against(tmp_path):
+    """The window form of a layer that conv_p16 has in the fp8 form, then in three passes: two measurements, two notes."""
+    cache = tmp_path / "tune.txt"
+    _forms(cache, "few channels", FYNHIP_FORCE_P16_CONV="1")   # (conv_p16 with its choice noted, the window form not looked at)
+    assert not [ln for ln in cache.read_text().splitlines() if ln.startswith("p16n:")]
+    noted = []
+    for switches in ({}, {"FYNHIP_EXACT_SPLIT": "1"}):
+        _forms(cache, "few channels", **switches)
+        noted.append([ln for ln in cache.read_text().splitlines() if ln.startswith("p16n:")])
+    assert len(noted[0]) == 1 and len(noted[1]) == 2
