@@ -771,13 +771,13 @@ class ConvLayer : public Layer {
         if ((long long)in_v.elems() > (1ll << 30)) return;
         // (64 channels at image size belong to the forms on whole chunks: 23 against 13 us at 256x256, ahead up to 64x64)
         if (in_v.cp > 48 && oh * ow > 8192 && !net->sw.get("FYNHIP_P16N_ROWS") && !net->sw.get("FYNHIP_FORCE_P16N_CONV")) return;
-        int want = 0;   // FYNHIP_P16N_ROWS=rows of a tile (tests)
-        if (const char* e = net->sw.get("FYNHIP_P16N_ROWS")) want = atoi(e);
+        int want = 0, want_fr = 0;   // FYNHIP_P16N_ROWS=rows of a tile[,fragments per workgroup] (tests)
+        if (const char* e = net->sw.get("FYNHIP_P16N_ROWS")) sscanf(e, "%d,%d", &want, &want_fr);
         std::vector<ConvP16Params> cands;
         // as many fragments per workgroup as there are and fit, or fewer where that makes more workgroups than the chip holds otherwise
         for (int fr = std::min(3, q.mfrags); fr >= 1; fr--)
             for (int th : {5, 4, 2}) {
-                if (q.mfrags % fr != 0 || (want && th != want)) continue;
+                if (q.mfrags % fr != 0 || (want && th != want) || (want_fr && fr != want_fr)) continue;
                 ConvP16Params c = q;
                 c.wm = fr;
                 c.cout_blocks = q.mfrags / fr;

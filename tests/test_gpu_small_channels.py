@@ -120,6 +120,37 @@ def test_windows_in_lds(monkeypatch, case, storage):
     assert rel_l2(got, oracle_single(b, storage, inputs, weights)) <= (2e-6 if storage == fa.STORAGE_F32 else TOL[storage])
 
 
+# ... and fewer fragments of output channels in a workgroup than there are: the last element is their number
+WINDOWED_BLOCKS = [
+    (40, 40, 12, 16, 1, False, ActType.RELU, ActType.RELU, 2, 1),    # the samples' layers on small frames: three blocks, the last with eight channels
+    (40, 40, 23, 37, 1, True, ActType.RELU, None, 5, 1),
+    (20, 20, 24, 34, 2, False, ActType.NONE, ActType.NONE, 4, 1),    # two blocks, the last with four
+    (16, 32, 9, 17, 1, True, ActType.LEAKY_RELU, None, 2, 1),
+    (24, 33, 31, 20, 2, True, ActType.CLIP, ActType.RELU, 2, 1),     # three, the last with one channel
+    (48, 44, 18, 33, 1, False, ActType.RELU, ActType.NONE, 5, 1),
+    (40, 96, 11, 18, 2, False, ActType.NONE, None, 4, 2),            # three blocks of two
+    (12, 128, 10, 15, 1, True, ActType.NONE, ActType.RELU, 5, 2),    # four
+    (64, 64, 17, 30, 1, True, ActType.RELU, ActType.RELU, 5, 1),     # four blocks of one
+    (64, 36, 13, 22, 2, False, ActType.RELU, None, 2, 1),
+    (40, 40, 90, 300, 1, False, ActType.NONE, ActType.RELU, 5, 1),   # 342 tiles x 3 blocks: workgroups walk two and three
+]
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("case", WINDOWED_BLOCKS, ids=lambda c: "%dto%d_%dx%d_s%d_%s_th%d_fr%d" % (c[0], c[1], c[2], c[3], c[4], "deep" if c[5] else "shallow", c[8], c[9]))
+def test_windows_in_lds_with_blocks_of_output_channels(monkeypatch, case, storage):
+    cin, cout, h, w, stride, deep, act, residual, rows, frags = case
+    monkeypatch.setenv("FYNHIP_P16N_ROWS", "%d,%d" % (rows, frags))
+    b = _windowed(case[:9])
+    inputs = [prng.normal(151 + cin, (cin, h, w))]
+    if residual is not None:
+        inputs.append(prng.normal(153 + cin, (cout, h // stride, w // stride)))
+    weights = conv_block(157 + cin, cout, 3, cin)
+    got, info = run_single(b, storage, inputs, weights)
+    assert "conv_p16n" in info and "of %dx16" % rows in info and "%d fragment(s)" % frags in info, info
+    assert rel_l2(got, oracle_single(b, storage, inputs, weights)) <= (2e-6 if storage == fa.STORAGE_F32 else TOL[storage])   # (as in the test above)
+
+
 @pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
 @pytest.mark.parametrize("cin,cout,h,w,step,stride", [(40, 20, 13, 16, 0.5, 2), (20, 12, 12, 19, 0.25, 2), (16, 16, 7, 9, 0.5, 1)])
 def test_windows_in_lds_of_repeated_pixels(monkeypatch, storage, cin, cout, h, w, step, stride):
