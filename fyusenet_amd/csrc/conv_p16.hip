@@ -457,13 +457,17 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
             else split_all(std::integral_constant<int, ACT_LEAKY>());
         }
     };
-    // The residual tile of a tile: [position][CPB channels] as stored, in 16-byte pieces.  They are spread over the tile's
-    // chunks but the first (the MFMA waves may still be reading the tile before until that is through), and a chunk's share
-    // is requested before the next stage is converted and written behind it: all of it in the last chunk is a burst that all
-    // workgroups ask for at the same time (3x3 128 -> 128 at 480x270, 8x16 tiles: 69 -> 65 us; 57 without a residual)
-    constexpr int RSH = 4, RSHARES = (G::RNB + RSH - 1) / RSH;   // pieces of a share, shares
+    // The residual tile of a tile: [position][CPB channels] as stored, in 16-byte pieces.  On rows in the fp8 form they are
+    // spread over the tile's chunks but the first (the MFMA waves may still be reading the tile before until that is through),
+    // and a chunk's share is requested before the next stage is converted and written behind it: all of it in the last chunk
+    // is a burst that all workgroups ask for at the same time (3x3 128 -> 128 at 480x270, 8x16 tiles: 69 -> 65 us; 57 without
+    // a residual).  The other tiles take it in the last chunk, ahead of the conversion: in shares fp16 64 -> 128 with step 2 at
+    // 480x270 positions took 40.8-41.9 us instead of 40.4-40.7, and nothing was faster by more than two runs differ (fp32 with
+    // step 2, three fp16 passes, 8x10 and 8x8 tiles of 128 and 64 channels, 156x128 to 480x270 positions)
+    constexpr bool SHARED = C8 && G::ROWS;
+    constexpr int RSH = SHARED ? 4 : G::RNB, RSHARES = (G::RNB + RSH - 1) / RSH;   // pieces of a share, shares
     f32x4_t rv[RSHARES * RSH];
-    auto residual_due = [&](int share, int c) { return nchunks < 2 || share * (nchunks - 1) / RSHARES == c - 1; };
+    auto residual_due = [&](int share, int c) { return SHARED ? nchunks < 2 || share * (nchunks - 1) / RSHARES == c - 1 : c + 1 == nchunks; };
     auto residual_request = [&](int tile, int c) {
         const store_t* res = reinterpret_cast<const store_t*>(p.res);
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
@@ -519,9 +523,14 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
     // One iteration per stage n of the MFMA waves: stage n+1 (fetched an iteration ago) is written to the other
     // buffer, then stage n+2 is fetched into the registers that stage n left.  Unrolled by two: set = parity of the stage.
     auto iteration = [&](auto next_set, auto free_set, unsigned char* next_buf) {
-        if (p.res) residual_request(tile, c);
+        if (p.res) {
+            residual_request(tile, c);
+            if constexpr (!SHARED) residual_store(c);
+        }
         if (have1) store(next_set, next_buf);
-        if (p.res) residual_store(c);
+        if constexpr (SHARED) {
+            if (p.res) residual_store(c);
+        }
         if (have2) fetch(free_set, t2, c2);
         lds_barrier();
         const bool go_on = have1;

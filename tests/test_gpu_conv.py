@@ -296,8 +296,8 @@ P16_CASES = [
     (20, 40, 38, 44, 2, "8,6,2", {"bn": True}),                                    # fewer channels than the tensors' pitch (conv3 and conv2 of those nets)
     (12, 20, 50, 36, 2, "4,8,2", {}),
     (44, 48, 23, 19, 1, "8,8,2", {"residual": (A.RELU, False)}),
-    # the residual tile in shares over more chunks than two, workgroups walking tiles
-    (128, 128, 70, 71, 1, "4,4,4", {"bn": True, "residual": (A.RELU, True)}),      # 324 tiles, one share
+    # a residual tile and more chunks than two, workgroups walking tiles
+    (128, 128, 70, 71, 1, "4,4,4", {"bn": True, "residual": (A.RELU, True)}),      # 324 tiles
     (192, 256, 67, 97, 1, "4,8,4", {"residual": (A.NONE, False)}),                 # 221 on 128 workgroups, six chunks
     (96, 256, 82, 90, 1, "8,8,4", {"bn": True, "residual": (A.NONE, True)}),       # 132 on 128, three chunks: three passes on fp32 tensors
     (128, 512, 134, 142, 2, "8,8,4", {"residual": (A.RELU, False)}),               # stride 2, 81 on 64
