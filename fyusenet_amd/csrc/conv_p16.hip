@@ -7,6 +7,9 @@
 // Why a second MFMA kernel: with 32x32 fragments a workgroup's tile is a multiple of 32 positions, and a layer of
 // 128x156 positions then fills 208 of the 256 CUs for three fragment rounds.  16-position fragments allow tiles of
 // 8x10 positions: 16x16 = 256 workgroups, one per CU, five fragments each (the work of 2.5 of the larger ones).
+// Tiles of rows of sixteen positions (TW = 16, stride 1, fp32 tensors): a fragment is one row, and what output row r takes
+// at tap row ky is what row r + 1 took at ky - 1, so fragments move through registers instead of being read again
+// (p16_rows_c8; the first layer's c4_rows).
 //
 // GEMM view as in conv_mfma.hip: M = output channels (A = weights, packed per lane, streamed through L2 into a register
 // ring), N = positions (B = activations, staged per 32-channel chunk as a halo tile in LDS, fp16 hi and lo planes),
@@ -15,7 +18,7 @@
 // LDS instruction with an immediate offset and the step loop has no address arithmetic.
 //
 // Workgroup = 4 staging waves (next chunk: global loads, activation, hi/lo conversion, LDS writes; scale and bias at
-// the start and, during the last chunk, the residual tile into LDS) + 4 MFMA waves (32 output channels each: 2 channel
+// the start and the residual tile into LDS, during the last chunk or in shares over several) + 4 MFMA waves (32 output channels each: 2 channel
 // fragments x FN position fragments).  A lane's accumulators of one fragment are 4 consecutive fragment rows of one
 // position, so the epilogue needs no transposition: residual and scale/bias from LDS, one 16-byte store per fragment
 // (fp16 tensors: the weights are packed so that row r of fragment fm of a wave's pair is output channel
@@ -1294,7 +1297,7 @@ __device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& rin
             constexpr int m = decltype(index_m)::value, fm = m % 2;
             if constexpr (!(HSTORE && (m == 2 || m == 3))) {
                 if constexpr (m < 2) {
-                    const half8_t b = p < 4 ? b0[r + 2 * p] : p == 4 ? b0[r + 8] : l0[1][r];
+                    const half8_t b = p < 4 ? b0[p < 4 ? r + 2 * p : 0] : p == 4 ? b0[r + 8 < TH + 8 ? r + 8 : 0] : l0[1][r];
                     acc[fm][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[p][0][fm], b, acc[fm][r], 0, 0, 0);
                 } else if constexpr (m < 4) {
                     acc[fm][r] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a2[p][fm], p < 4 ? b8[p < 4 ? r + 2 * p : 0] : u8[p < 4 ? 0 : p - 4][r], acc[fm][r], 0, 0, 0, 0, 0, 0);

@@ -18,7 +18,7 @@
 // 6.4 -> 4.0 (conv_p16); 20 -> 40, step 2, at 12x16 6.0 -> 4.7 (conv_mfma); 40 -> 20 at step 1/2, 156x128 9.1 -> 7.6, 12x16
 // 7.4 -> 5.0; 20 -> 12 at step 1/4, 24x32 5.8 -> 3.8; 40 -> 40 at 156x128 with a residual 8.2 -> 8.0; 64 -> 64 at
 // 56x56 5.7 -> 5.2 (conv_kr16, whose waves split whole chunks of 32 channels: two of four had none).  The samples' 3x3 style
-// net on a 64x48 frame 77.7 -> 69.7 us.  Bound: a launch's start and its memory round trip (a microsecond of matrix
+// net on a 64x48 frame 77-78 -> 70-71 us.  Bound: a launch's start and its memory round trip (a microsecond of matrix
 // instructions in 40 -> 40 at 156x128), on large images the conversion and the partial sums beside them.
 #include <hip/hip_runtime.h>
 
@@ -276,7 +276,11 @@ constexpr P16NEntry p16n_entry() {
     typedef GeoN<HS, G, FR, S, TH> N;
     return P16NEntry{HS, G, FR, S, TH, conv_p16n_kernel<N>, (size_t)N::LDS};
 }
-// (a step of two doubles the window: four rows of it where five fit with a step of one)
+// (a step of two doubles the window: four rows of it where five fit with a step of one; two rows of 64 channels, whose
+// window of four, 88 KB in two planes, is beyond the immediate field.  Not compiled are 32 channels, 56, and 48 with a step of
+// two, although they would gain at some sizes.  This form against the others, us, fp32 and fp16 tensors: 32 -> 32 at 56x56
+// 3.9 / 4.4 and 3.6 / 3.6, at 112x112 4.8 / 4.9 and 4.1 / 4.0, at 256x256 10.1 / 8.7 and 7.4 / 6.6; 48 -> 48, step 2, at 56x56 5.4 / 6.8
+// and 4.5 / 4.6, at 256x256 19.6 / 23.5 and 11.6 / 13.0; 56 -> 56 at 56x56 4.6 / 5.2 and 4.0 / 4.0, at 128x128 7.7 / 6.5 and 5.8 / 4.7)
 #define P16N_ROWS(HS, G, FR, S) p16n_entry<HS, G, FR, S, 2>(), p16n_entry<HS, G, FR, S, S == 1 ? 5 : 4>()
 #define P16N_FRAGS(HS, G, S) P16N_ROWS(HS, G, 1, S), P16N_ROWS(HS, G, 2, S), P16N_ROWS(HS, G, 3, S)
 #define P16N_STEPS(HS, G) P16N_FRAGS(HS, G, 1), P16N_FRAGS(HS, G, 2)

@@ -336,7 +336,7 @@ int conv_g16_steps(int in_cp);                       // matrix steps of the wind
 bool conv_g16_exists(const ConvP16Params& p);        // whether p.wm fragments per wave have been compiled
 size_t conv_g16_lds_bytes(const ConvP16Params& p);   // of a workgroup: its weights
 int launch_conv_g16(const ConvP16Params& p, hipStream_t s);
-// the same layers (up to 48 channels on either side) with a tile's window in LDS, on the same weights (conv_p16n.hip)
+// 3x3 layers of 16 to 64 input and up to 128 output channels with a tile's window in LDS, on the same weights (conv_p16n.hip)
 size_t conv_p16n_lds_bytes(const ConvP16Params& p);   // of a workgroup; 0: no such compiled combination
 int launch_conv_p16n(const ConvP16Params& p, hipStream_t s);
 // a 1x1 layer and the depthwise 3x3 layer behind it as one launch (conv_d16.hip: conv_e16dw_kernel)

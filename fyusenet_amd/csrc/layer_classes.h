@@ -123,7 +123,7 @@ class ConvLayer : public Layer {
         return true;
     }
     // 16-position-fragment form of a 3x3 convolution (conv_p16.hip): the compiled combinations that fit the layer are
-    // timed (the three with the fewest fragment rounds on 256 CUs), and the best is kept if it beats the tuned launch of
+    // timed (the four with the fewest fragment rounds on 256 CUs), and the best is kept if it beats the tuned launch of
     // the general kernel.
     void setup_p16(const TView& in_v, const TView& out_v, const TView* res_v, int res_relu, int res_scale) {
         ConvP16Params q{};
@@ -509,7 +509,7 @@ class ConvLayer : public Layer {
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
                 fprintf(stderr, "[tune] %dx%d on %d channels, %dx%d positions: K-resident form (%d-channel blocks, %dx%d tiles) %.1f us, %s %.1f us\n", k, k,
                         d.in_channels, oh, ow, 16 * cands[pick].wm, cands[pick].tile_h, cands[pick].tile_w, best * 1e3f,
-                        had_p16 ? "16-position 3x3 form" : "general kernel", t_other * 1e3f);
+                        h16 ? "wide fp16 form" : had_p16 ? "16-position 3x3 form" : "general kernel", t_other * 1e3f);
             const bool win = best < t_other;
             if (!want_fm) tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].wm, cands[pick].tile_h * 100 + cands[pick].tile_w);
             if (!win && !always) pick = -1;
@@ -769,7 +769,9 @@ class ConvLayer : public Layer {
         ConvP16Params q = small_channel_params(in_v, out_v, res_v, res_relu, res_scale);
         q.mfrags = (oc + 15) / 16;
         if ((long long)in_v.elems() > (1ll << 30)) return;
-        // (64 channels at image size belong to the forms on whole chunks: 23 against 13 us at 256x256, ahead up to 64x64)
+        // (64 channels at image size belong to the forms on whole chunks.  This form against the one chosen before, us, 64 -> 64 on
+        // fp32 tensors: 5.1 / 5.2 at 64x64 positions, 6.0 / 6.1 at 80x80, 6.8 / 6.1 at 90x91, 8.3 / 6.1 at 112x112, 21.7 / 11.8 at
+        // 256x256; 64 -> 32 4.5 / 4.4, 5.0 / 6.0, 5.8 / 5.9, 6.0 / 6.0, 13.1 / 11.4; with a step of two, and on fp16 tensors, the same line)
         if (in_v.cp > 48 && oh * ow > 8192 && !net->sw.get("FYNHIP_P16N_ROWS") && !net->sw.get("FYNHIP_FORCE_P16N_CONV")) return;
         int want = 0, want_fr = 0;   // FYNHIP_P16N_ROWS=rows of a tile[,fragments per workgroup] (tests)
         if (const char* e = net->sw.get("FYNHIP_P16N_ROWS")) sscanf(e, "%d,%d", &want, &want_fr);
@@ -1215,8 +1217,8 @@ class ConvLayer : public Layer {
             scale_dev = static_cast<float*>(net->dev_alloc(padded * sizeof(float)));
             bias_dev = static_cast<float*>(net->dev_alloc(padded * sizeof(float)));
             launch = tune_mfma(net, sc, in_v, out_v, res_v, d.in_channels, oc, act(), res_relu, res_scale, scale_dev, bias_dev);
-            // the 16-position-fragment forms, each against the tuned launch of the general kernel: for wide fp16 layers the
-            // one with 64-channel wave tiles first, then the 3x3 form, then the small-input form
+            // the 16-position-fragment forms, each against the tuned launch of the general kernel: for fp16 layers of whole
+            // blocks of 128 output channels the wide one first (conv_h16.hip), then the 3x3 form, then the small-input form
             const bool same_storage = in_v.f16 == out_v.f16 && (!res_v || res_v->f16 == out_v.f16);
             // (tests: the K-resident form or nothing; a forced variant of the general kernel means the general kernel)
             const bool only_kr = net->sw.get("FYNHIP_FORCE_KR16_CONV") || net->sw.get("FYNHIP_FORCE_KSPLIT") || net->sw.get("FYNHIP_CONV_TILE") || net->sw.get("FYNHIP_CONV_KC") ||
