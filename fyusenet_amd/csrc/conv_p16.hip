@@ -470,33 +470,25 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
     constexpr bool SHARED = C8 && G::ROWS;
     constexpr int RSH = SHARED ? 4 : G::RNB, RSHARES = (G::RNB + RSH - 1) / RSH;   // pieces of a share, shares
     f32x4_t rv[RSHARES * RSH];
-    auto residual_due = [&](int share, int c) { return SHARED ? nchunks < 2 || share * (nchunks - 1) / RSHARES == c - 1 : c + 1 == nchunks; };
-    auto residual_request = [&](int tile, int c) {
+    auto residual_due = [&](int share, int c) { return nchunks < 2 || share * (nchunks - 1) / RSHARES == c - 1; };
+    auto residual_request = [&](int tile, int share) {
         const store_t* res = reinterpret_cast<const store_t*>(p.res);
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
 #pragma unroll
-        for (int share = 0; share < RSHARES; share++) {
-            if (!residual_due(share, c)) continue;
-#pragma unroll
-            for (int i = share * RSH; i < (share + 1) * RSH; i++) {
-                const int idx = stid + i * 256;
-                const int m = idx / G::RPP, piece = idx % G::RPP;
-                const int ty = m / G::TWG, tx = m - ty * G::TWG;
-                const int py = tyi * G::TH + ty, px = txi * G::TWG + tx;
-                const bool ok = idx < G::RPIECES && py < p.npos_y && px < p.npos_x && cb * CPB + piece * (16 / ESZ) < p.res_cp;
-                rv[i] = *reinterpret_cast<const f32x4_t*>(res + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + cb * CPB + piece * (16 / ESZ) : 0));
-            }
+        for (int i = share * RSH; i < (share + 1) * RSH; i++) {
+            const int idx = stid + i * 256;
+            const int m = idx / G::RPP, piece = idx % G::RPP;
+            const int ty = m / G::TWG, tx = m - ty * G::TWG;
+            const int py = tyi * G::TH + ty, px = txi * G::TWG + tx;
+            const bool ok = idx < G::RPIECES && py < p.npos_y && px < p.npos_x && cb * CPB + piece * (16 / ESZ) < p.res_cp;
+            rv[i] = *reinterpret_cast<const f32x4_t*>(res + (ok ? ((size_t)(p.res_off_y + py) * p.res_wp + p.res_off_x + px) * p.res_cp + cb * CPB + piece * (16 / ESZ) : 0));
         }
     };
-    auto residual_store = [&](int c) {
+    auto residual_store = [&](int share) {
 #pragma unroll
-        for (int share = 0; share < RSHARES; share++) {
-            if (!residual_due(share, c)) continue;
-#pragma unroll
-            for (int i = share * RSH; i < (share + 1) * RSH; i++) {
-                const int idx = stid + i * 256;
-                if (idx < G::RPIECES) *reinterpret_cast<f32x4_t*>(lds + res_off + (idx / G::RPP) * G::RES_PITCH + (idx % G::RPP) * 16) = rv[i];
-            }
+        for (int i = share * RSH; i < (share + 1) * RSH; i++) {
+            const int idx = stid + i * 256;
+            if (idx < G::RPIECES) *reinterpret_cast<f32x4_t*>(lds + res_off + (idx / G::RPP) * G::RES_PITCH + (idx % G::RPP) * 16) = rv[i];
         }
     };
     // the stage after (tile, c); false: there is none
@@ -526,13 +518,23 @@ __device__ __forceinline__ void p16_stager(const ConvP16Params& p, unsigned char
     // One iteration per stage n of the MFMA waves: stage n+1 (fetched an iteration ago) is written to the other
     // buffer, then stage n+2 is fetched into the registers that stage n left.  Unrolled by two: set = parity of the stage.
     auto iteration = [&](auto next_set, auto free_set, unsigned char* next_buf) {
-        if (p.res) {
-            residual_request(tile, c);
-            if constexpr (!SHARED) residual_store(c);
+        if constexpr (SHARED) {
+            if (p.res) {
+#pragma unroll
+                for (int share = 0; share < RSHARES; share++)
+                    if (residual_due(share, c)) residual_request(tile, share);
+            }
+        } else if (c + 1 == nchunks && p.res) {
+            residual_request(tile, 0);
+            residual_store(0);
         }
         if (have1) store(next_set, next_buf);
         if constexpr (SHARED) {
-            if (p.res) residual_store(c);
+            if (p.res) {
+#pragma unroll
+                for (int share = 0; share < RSHARES; share++)
+                    if (residual_due(share, c)) residual_store(share);
+            }
         }
         if (have2) fetch(free_set, t2, c2);
         lds_barrier();
