@@ -181,14 +181,15 @@ class ConvLayer : public Layer {
         std::sort(cands.begin(), cands.end(), [](const Cand& a, const Cand& b) { return a.cost < b.cost; });
         if (cands.size() > 4) cands.resize(4);
         const size_t halves = ((size_t)q.cin_chunks * 9 + 8) * q.mfrags * (q.f16 ? 1 : 3) * 64 * 8;
-        p16_wpack_dev = net->dev_alloc(halves * 2, true);
-        for (Cand& c : cands) c.q.wpack = p16_wpack_dev;
+        void* const wp = net->dev_alloc(halves * 2, true);
+        for (Cand& c : cands) c.q.wpack = wp;
+        const bool had_h16 = h16;   // the wide fp16 form was chosen over the general kernel: this form has to beat it instead
         const bool always = net->sw.get("FYNHIP_FORCE_P16_CONV") != nullptr;
         const char* at = net->sw.get("FYNHIP_AUTOTUNE");
         const bool timing = !(at && at[0] == '0');
-        int pick = 0;   // index into cands, -1: the general kernel
+        int pick = had_h16 ? -1 : 0;   // index into cands, -1: the general kernel or the wide form
         char key[160];
-        snprintf(key, sizeof(key), "p16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d:q%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift, conv_p16_uses_fp8(q) ? 1 : 0);
+        snprintf(key, sizeof(key), "p16:%dx%d:%dx%d:s%d:cp%d:r%d:e%d:h%d:f%d:q%d", d.in_channels, oc, oh, ow, stride, in_v.cp, res_v ? 1 : 0, clamp ? 1 : 0, q.f16, frac_shift, had_h16 ? 2 : conv_p16_uses_fp8(q) ? 1 : 0);
         // (the cache keeps: chosen?, tile_h*1000 + tile_w, wm)
         if (!want_h && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return cands[i].q.tile_h * 1000 + cands[i].q.tile_w == b && cands[i].q.wm == c; }, &pick)) {
         } else if (timing) {
@@ -200,21 +201,23 @@ class ConvLayer : public Layer {
                     }, 10);
                     if (t < best) { best = t; pick = (int)i; }
                 }
-                t_other = std::min(t_other, time_launch(net, launch, 10));
+                t_other = std::min(t_other, had_h16 ? time_calls(net, [&]() { launch_chosen_h16(); }, 10) : time_launch(net, launch, 10));
             }
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
-                fprintf(stderr, "[tune] 3x3: 16-position fragments (%dx%d tiles, %d channel groups) %.1f us, general kernel %.1f us\n",
-                        cands[pick].q.tile_h, cands[pick].q.tile_w, cands[pick].q.wm, best * 1e3f, t_other * 1e3f);
+                fprintf(stderr, "[tune] 3x3: 16-position fragments (%dx%d tiles, %d channel groups) %.1f us, %s %.1f us\n",
+                        cands[pick].q.tile_h, cands[pick].q.tile_w, cands[pick].q.wm, best * 1e3f, had_h16 ? "wide fp16 form" : "general kernel", t_other * 1e3f);
             const bool win = best < t_other;
             if (!want_h) tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].q.tile_h * 1000 + cands[pick].q.tile_w, cands[pick].q.wm);
             if (!win && !always) pick = -1;
         }
         if (pick >= 0) {
+            if (had_h16) net->dev_free(p16_wpack_dev);
+            p16_wpack_dev = wp;
             p16 = true;
+            h16 = h16_two = false;
             pp = cands[pick].q;
         } else {
-            net->dev_free(p16_wpack_dev);
-            p16_wpack_dev = nullptr;
+            net->dev_free(wp);
         }
     }
     // the small-input form (conv_p16.hip, conv_p16c4_kernel): 9x9 on at most four input channels
@@ -291,6 +294,10 @@ class ConvLayer : public Layer {
             net->dev_free(p16_wpack_dev);
             p16_wpack_dev = nullptr;
         }
+    }
+    void launch_chosen_h16() {
+        if (launch_conv_h16(pp, k, net->stream) != 0 || (h16_two && launch_conv_h16(pp2, k, net->stream) != 0))
+            fail(FYN_ERR_DEVICE, "fp16 16-position convolution launch failed while tuning");
     }
     // the fp16-storage form for wide layers (conv_h16.hip): K = 3 or 9, stride 1, blocks of 128 output channels.  A
     // launch takes a whole number of rounds of tiles over the chip's 256 CUs; when the last round of the best single
@@ -500,8 +507,8 @@ class ConvLayer : public Layer {
                 }
                 if (had_p16)
                     t_other = std::min(t_other, time_calls(net, [&]() {
-                        if (h16 ? launch_conv_h16(pp, k, net->stream) != 0 || (h16_two && launch_conv_h16(pp2, k, net->stream) != 0) : launch_conv_p16(pp, net->stream) != 0)
-                            fail(FYN_ERR_DEVICE, "16-position convolution launch failed while tuning");
+                        if (h16) launch_chosen_h16();
+                        else if (launch_conv_p16(pp, net->stream) != 0) fail(FYN_ERR_DEVICE, "16-position convolution launch failed while tuning");
                     }, 10));
                 else
                     t_other = std::min(t_other, time_launch(net, launch, 10));
@@ -1227,7 +1234,14 @@ class ConvLayer : public Layer {
                 (!res_v || res_v->cp >= oc) && !net->sw.get("FYNHIP_NO_P16_CONV") && !net->sw.get("FYNHIP_NO_H16_CONV"))
                 setup_h16(in_v, out_v, res_v, res_relu, res_scale);
             // (channels between a layer's count and the tensor's pitch hold zeros and meet zero weights)
-            if (!only_kr && !p16 && same_storage && !sc.in_sub && conv_p16_supported(k, stride, dil, in_v.cp, oc, out_v.cp, out_v.f16 != 0) &&
+            // (a wide fp16 layer of few tiles: against the wide form, whose workgroups have 64 positions and 128 channels at least.
+            // Timed on 64 to 1024 channels -> 128 to 512, 7x7 to 160x200 positions: up to 128 tiles of that size this form is
+            // ahead, 192 -> 128 at 56x56 6.4 against 7.4 us, 256 -> 256 at 64x64, 128 tiles, 8.6 / 9.1; at 138 they are level
+            // (4.9 / 5.0, 6.7 / 6.5, 7.6 / 7.6), from 168 on the wide one is but for 1024 channels: 128 -> 128 at 96x128 7.4 / 6.7,
+            // 256 -> 256 at 96x128 18.1 / 12.5, 1024 -> 512 at 56x56, 224 tiles, 30.2 / 32.7)
+            const bool few_tiles = h16 && (size_t)((oh + 3) / 4) * ((ow + 15) / 16) * (oc / 128) <= 128 && !net->sw.get("FYNHIP_P16_TILE") && !net->sw.get("FYNHIP_H16_SPLIT") &&
+                                   !net->sw.get("FYNHIP_FORCE_P16_CONV");
+            if (!only_kr && (!p16 || few_tiles) && same_storage && !sc.in_sub && conv_p16_supported(k, stride, dil, in_v.cp, oc, out_v.cp, out_v.f16 != 0) &&
                 d.in_channels <= in_v.cp && (!res_v || (res_v->cp >= oc && res_v->cp % 8 == 0)) && !net->sw.get("FYNHIP_NO_P16_CONV"))
                 setup_p16(in_v, out_v, res_v, res_relu, res_scale);
             if (!only_kr && !p16 && !frac_shift && same_storage && !res_v && conv_p16c4_supported(k, stride, dil, in_v.cp, oc, out_v.cp, out_v.f16 != 0) &&

@@ -1173,3 +1173,36 @@ def test_few_channel_choices_are_noted_by_what_they_were_measured_against(tmp_pa
         _forms(cache, "few channels", **switches)
         noted.append([ln for ln in cache.read_text().splitlines() if ln.startswith("p16n:")])
     assert len(noted[0]) == 1 and len(noted[1]) == 2
+
+
+@pytest.mark.parametrize("cin,cout,h,w,residual,noted", [(192, 128, 56, 56, False, True), (256, 256, 33, 47, True, True), (64, 128, 65, 70, True, True), (128, 128, 96, 128, False, False)])
+def test_wide_fp16_layers_of_few_tiles_are_measured_on_smaller_tiles_too(tmp_path, cin, cout, h, w, residual, noted):
+    """Up to 128 tiles of the wide form conv_p16 is timed against it (what was chosen is right either way: the child compares
+    with the oracle); above, and where nothing is timed, the wide form has the layer."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    cache = tmp_path / "tune.txt"
+    child = r"""
+import sys
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests")
+import fyusenet_amd as fa
+from fyusenet_amd import prng
+from util import conv_block, oracle_single, rel_l2, run_single
+from test_gpu_conv import conv_builder
+cin, cout, h, w, residual = [int(v) for v in sys.argv[2:]]
+b = conv_builder(3, cout, h, w, cin, 1, 1, fa.ActType.RELU, **({"residual": (fa.ActType.RELU, True), "bn": True} if residual else {"pad_out": 1}))
+x = [prng.uniform(61, (cin, h, w), -1, 1)] + ([prng.uniform(62, (cout, h, w), -1, 1)] if residual else [])
+wts = conv_block(63, cout, 3, cin, bn=bool(residual))
+got, info = run_single(b, fa.STORAGE_F16, x, wts)
+print(info, rel_l2(got, oracle_single(b, fa.STORAGE_F16, x, wts)))
+"""
+    for at in ("1", "0"):
+        r = subprocess.run([sys.executable, "-c", child, root] + [str(int(v)) for v in (cin, cout, h, w, residual)], capture_output=True, text=True, timeout=300,
+                           env=dict(os.environ, FYNHIP_AUTOTUNE=at, FYNHIP_NO_KR16_CONV="1", **({"FYNHIP_TUNE_CACHE": str(cache)} if at == "1" else {})))
+        assert r.returncode == 0, r.stderr[-2000:]
+        print(at, r.stdout, flush=True)
+        assert "conv_h16" in r.stdout or (noted and at == "1" and "conv_p16" in r.stdout)
+        assert float(r.stdout.split()[-1]) <= TOL[fa.STORAGE_F16]
+    assert ("p16:%dx%d:%dx%d:" % (cin, cout, h, w) in "".join(ln + "\n" for ln in cache.read_text().splitlines() if ln.startswith("p16:"))) == noted
