@@ -14,7 +14,7 @@
 // positions: no two waves load the same weights, 21 bytes per MFMA cycle and CU through the L1 (which delivers 64) and 23
 // from LDS (128), where two groups of 64 channels x two tiles of positions took 43 and 64.
 // Measured, fp16: 9x9 128 -> 128 at 464x381 positions (469 GFLOP) 290-297 us a layer in a frame = 1.58-1.62 PFLOP/s, what the
-// library reaches on a 16384^3 product here (1.63).  Twenty launches of a layer in a row, one box, before and now: 313-326 and
+// library reaches on a 16384^3 product here (1.63).  Twenty launches of a layer in a row on one card, before and now: 313-326 and
 // 272-286 us; 352x225 167 and 139; 3x3 128 -> 128 at 156x128 (5.9 GFLOP) 11.4 and 8.4.
 // Bound: the matrix pipes at the clock the part holds under them (79 % busy at 1.95-2.0 GHz in the launch of 12-row
 // tiles; without any operand traffic the same loop is 90 % busy at 2.2).  Weights requested 2, 3, 4 or 8 steps ahead,
