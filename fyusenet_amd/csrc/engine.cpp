@@ -414,6 +414,7 @@ void Net::setup() {
         }
     }
     keep_projection_inputs(this);
+    const auto kept = keep_block_inputs(this);
     // 2. device buffers.  Liveness rule of BufferManager::findTexture (base/buffermanager.cpp:512-525)
     //    restated for in-order stream execution: a buffer can take layer N's output when every reader of
     //    its current tenant has a number < N; only buffers of identical geometry are shared so that the
@@ -460,6 +461,7 @@ void Net::setup() {
         t.v.ptr = b.ptr;
         t.written = t.producer;
     }
+    for (auto i = kept.rbegin(); i != kept.rend(); ++i) tensors[i->first].last_reader = i->second;
     // pass-through layers were given the tensor id only; nothing else to do for them
     assign_range_words();
     // 3. per-layer setup (weight packing, kernel selection)
@@ -470,6 +472,7 @@ void Net::setup() {
     fuse_depthwise_layers(this);
     fuse_projection_layers(this);
     fuse_batchnorm_layers(this);
+    fuse_block_layers(this);
     fuse_function_layers(this);
     fuse_concat_layers(this);
     fuse_argmax_layers(this);
@@ -507,6 +510,25 @@ void Net::assign_range_words() {
 // clearing is given to a convolution kernel that runs after the tensor's last reader (kernels of one stream run one
 // after the other, so nothing else touches the word at that time): the first such layer behind the last reader,
 // wrapping around to the layers in front of the producer.  A tensor for which no layer is found loses its word.
+int Net::words_without_reset() const {
+    if (!amax_dev_) return 0;
+    std::map<int, int> room;
+    for (auto& kv : layers) room[kv.first] = kv.second->reset_room();
+    int lost = 0;
+    for (const Tensor& t : tensors) {   // (the order and the rules of assign_range_resets)
+        if (!t.amax || t.producer < 0 || layers.at(t.producer)->d.type == FYN_LAYER_UPLOAD) continue;
+        const int last = std::max(t.last_reader, t.producer);
+        auto at = room.end();
+        for (auto i = room.begin(); i != room.end() && at == room.end(); ++i)
+            if (i->first > last && i->second > 0) at = i;
+        for (auto i = room.begin(); i != room.end() && at == room.end(); ++i)
+            if (i->first < t.written && i->second > 0) at = i;
+        if (at == room.end()) lost++;
+        else at->second--;
+    }
+    return lost;
+}
+
 void Net::assign_range_resets() {
     if (!amax_dev_) return;
     std::vector<int> order;

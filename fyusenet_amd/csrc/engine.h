@@ -96,6 +96,7 @@ class Layer {
     // take on clearing another tensor's word (true: taken)
     virtual bool tracks_range() const { return false; }
     virtual bool add_range_reset(unsigned*) { return false; }
+    virtual int reset_room() const { return 0; }   // how many words it could still take
     virtual void setup_ranges() {}   // (re)reads the words of the layer's tensors into its kernel arguments
     // a sigmoid or tanh layer: its arguments, for the layer in front that computes it as well (computed_by), else null
     virtual const FuncParams* pointwise() const { return nullptr; }
@@ -164,6 +165,9 @@ class Net {
     // than its producer, or to read it later than its last reader; whoever does so enters it in `written` or
     // `last_reader`, which is what the next one to ask finds.
     bool alone(int tensor, int from, int to) const;
+    // Tensors whose value-range word no launch would clear as things stand: they go without one (assign_range_resets).  A
+    // fusion that takes launches away asks before and behind.
+    int words_without_reset() const;
     void read_until(int tensor, int layer_no) { tensors[tensor].last_reader = std::max(tensors[tensor].last_reader, layer_no); }
 
     // device allocations owned by the net
@@ -251,6 +255,8 @@ Layer* create_layer(Net* net, const fyn_layer_desc& d);
 void fuse_batchnorm_layers(Net* net);   // after every layer's setup(): batch-norm layers that their readers (K-resident convolutions) can apply while staging
 void keep_projection_inputs(Net* net);    // before buffers are assigned: inputs of such projections live until the layer that may compute them has run
 void fuse_projection_layers(Net* net);   // after every layer's setup(): 1x1 shortcut projections that the 1x1 layer adding them can compute in its own launch
+std::vector<std::pair<int, int>> keep_block_inputs(Net* net);   // ... and, while they are assigned, inputs of bottlenecks until their last layer, which may compute them, has run; (tensor, its last reader)
+void fuse_block_layers(Net* net);        // after the other passes on convolutions: a 1x1, a 3x3 and a 1x1 layer in one launch
 void fuse_depthwise_layers(Net* net);   // after every layer's setup(): depthwise 3x3 layers that their 1x1 reader can compute itself
 void fuse_function_layers(Net* net);   // after every layer's setup(): sigmoid / tanh layers that the row-rolling convolution in front of them can apply to what it stores
 void fuse_concat_layers(Net* net);   // after every layer's setup(): bilinear scale layers in front of concatenations and batch-norm layers behind them

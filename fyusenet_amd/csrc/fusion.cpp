@@ -337,6 +337,169 @@ void fuse_batchnorm_layers(Net* net) {
     }
 }
 
+// The bottleneck that ends with layer `c`, by the graph alone: a 1x1 layer, a 3x3 layer that alone reads it, and `c`, a 1x1
+// layer that alone reads that one; no step, no dilation, nothing between them.
+static bool block_of(Net* net, ConvLayer* c, ConvLayer*& a, ConvLayer*& b) {
+    auto plain = [](const ConvLayer* l, int k) {
+        return l && l->k == k && l->stride == 1 && l->dil == 1 && !l->clamp && !l->frac_shift && !l->direct && !l->wide;
+    };
+    auto in_front = [&](ConvLayer* l) -> ConvLayer* {
+        if (l->in.empty() || l->in[0] < 0) return nullptr;
+        const Tensor& t = net->tensors[l->in[0]];
+        if (t.producer < 0 || t.locked) return nullptr;
+        int readers = 0;
+        for (auto& kv : net->layers)
+            for (int i : kv.second->in) readers += i == l->in[0];
+        ConvLayer* p = readers == 1 ? dynamic_cast<ConvLayer*>(net->layer(t.producer)) : nullptr;
+        return p && !(p->d.flags & FYN_FLAG_RESIDUAL_INPUT) && p->d.number < l->d.number ? p : nullptr;
+    };
+    if (!plain(c, 1)) return false;
+    b = in_front(c);
+    if (!plain(b, 3)) return false;
+    a = in_front(b);
+    return plain(a, 1) && !a->in.empty() && a->in[0] >= 0 && a->oh == c->oh && a->ow == c->ow && b->oh == c->oh && b->ow == c->ow;
+}
+// While buffers are assigned, the input of such a block is read until its last layer has run, which may compute all of it (the
+// tensors' last readers as they were: whether the block is joined is not known yet).
+std::vector<std::pair<int, int>> keep_block_inputs(Net* net) {
+    std::vector<std::pair<int, int>> were;
+    if (net->sw.get("FYNHIP_NO_BLOCK_FUSION") || !net->reuse_buffers) return were;
+    auto keep = [&](int tensor, int layer_no) {
+        were.push_back({tensor, net->tensors[tensor].last_reader});
+        net->read_until(tensor, layer_no);
+    };
+    for (auto& kv : net->layers) {
+        ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
+        if (!c || !block_of(net, c, a, b)) continue;
+        keep(a->in[0], c->d.number);
+        const Tensor& t = net->tensors[a->in[0]];
+        if (t.producer < 0) continue;
+        BatchNormLayer* bn = dynamic_cast<BatchNormLayer*>(net->layer(t.producer));   // (which the block may apply)
+        if (bn && !bn->in.empty() && bn->in[0] >= 0) keep(bn->in[0], c->d.number);
+    }
+    return were;
+}
+// Bottlenecks (conv_b16.hip) as one launch in the place of their last layer, timed against the launches they run as now:
+// with the batch-norm layer in front that the first layer applies, or the projection that the last one adds.
+void fuse_block_layers(Net* net) {
+    if (net->sw.get("FYNHIP_NO_BLOCK_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV") || !net->reuse_buffers) return;
+    // (tests: whoever forces a form of one of the layers wants to see that form)
+    if (!net->sw.get("FYNHIP_FORCE_BLOCK_FUSION"))
+        for (const char* other : {"FYNHIP_FORCE_PROJECTION_FUSION", "FYNHIP_FORCE_KR16_CONV", "FYNHIP_KR16_FM", "FYNHIP_FORCE_D16_CONV", "FYNHIP_D16_BLOCKS", "FYNHIP_FORCE_P16_CONV", "FYNHIP_P16_TILE",
+                                  "FYNHIP_FORCE_KSPLIT", "FYNHIP_CONV_TILE", "FYNHIP_CONV_KC", "FYNHIP_CONV_KC_MAX", "FYNHIP_CONV_PD"})
+            if (net->sw.get(other)) return;
+    const char* at = net->sw.get("FYNHIP_AUTOTUNE");
+    for (auto& kv : net->layers) {
+        ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
+        if (!c || !block_of(net, c, a, b)) continue;
+        if (a->dw_fused || a->edw_fused || a->pj_fused || a->pj_into >= 0 || b->bn_fused || c->bn_fused || c->dw_fused || c->edw_fused || c->fn_layer_no >= 0 || c->argmax_tail.idx) continue;
+        const TView &iv = a->tin(0).v, &ov = c->tout().v;
+        if (iv.f16 != ov.f16 || a->tout().v.f16 != ov.f16 || b->tout().v.f16 != ov.f16 || iv.cp % 8 != 0 || iv.cp < 8 || ov.cp % 4 != 0 || a->d.in_channels > iv.cp || c->oc > ov.cp ||
+            b->d.in_channels != a->oc || c->d.in_channels != b->oc)
+            continue;
+        // (positions beside the first layer's output are zeros behind the second layer's activation as well)
+        if (b->act().lo > 0.f || b->act().hi < 0.f) continue;
+        ConvLayer* pr = nullptr;
+        ConvB16Params q{};
+        if (c->d.flags & FYN_FLAG_RESIDUAL_INPUT) {
+            if (c->in.size() < 2 || c->in[1] < 0 || c->in[1] == c->in[0]) continue;
+            const TView& rv = c->tin(1).v;
+            if (rv.f16 != ov.f16) continue;
+            pr = projection_of(net, c);
+            const Act x = a->act(), y = pr ? pr->act() : x;
+            if (pr && (pr->stride != 1 || pr->in[0] != a->in[0] || a->bn_fused || pr->bn_fused || x.kind != y.kind || x.lo != y.lo || x.hi != y.hi || x.leak != y.leak || pr->d.in_channels > iv.cp ||
+                       net->tensors[c->in[1]].v.f16 != ov.f16 || net->sw.get("FYNHIP_NO_PROJECTION_FUSION")))
+                pr = nullptr;
+            if (!pr) {
+                if (c->pj_fused || rv.cp < ov.cp || rv.cp % 4 != 0) continue;
+                q.res = rv.ptr; q.res_wp = rv.wp(); q.res_cp = rv.cp; q.res_off = rv.pad;
+                q.res_relu = (c->d.flags & FYN_FLAG_RELU_ON_RESIDUAL) ? 1 : 0;
+            }
+            q.res_scale = ((c->d.flags & FYN_FLAG_BATCHNORM_ON_RESIDUAL) && (c->d.flags & FYN_FLAG_POST_BATCHNORM)) ? 1 : 0;
+        }
+        // (the launch reads the block's input in the last layer's place in the order)
+        int x = a->in[0];
+        if (a->bn_fused) x = net->layer(a->bn_layer_no)->in[0];
+        if (!net->alone(x, a->d.number, c->d.number)) continue;
+        // (the words of value ranges that the launches in front clear: another launch has to be there for them)
+        auto joined = [&](bool yes) {
+            a->blk_into = b->blk_into = yes ? c->d.number : -1;
+            if (pr) pr->blk_into = a->blk_into;
+        };
+        const int reader = net->tensors[x].last_reader, lost = net->words_without_reset();
+        joined(true);
+        net->read_until(x, c->d.number);
+        const int lost_then = net->words_without_reset();
+        joined(false);
+        net->tensors[x].last_reader = reader;
+        if (lost_then > lost) continue;
+        const ConvLayer* L[4] = {a, b, c, pr};
+        for (int i = 0; i < 4; i++) {
+            if (!L[i]) continue;
+            q.scale[i] = L[i]->scale_dev; q.bias[i] = L[i]->bias_dev;
+            q.acc_mul[i] = 1.f;
+        }
+        q.in = a->bn_fused ? a->bn_in : iv.ptr;
+        q.in_mul = a->bn_fused ? a->bn_mul : nullptr; q.in_add = a->bn_fused ? a->bn_add : nullptr;
+        q.out = ov.ptr;
+        q.act[0] = a->act(); q.act[1] = b->act(); q.act[2] = c->act();
+        q.mid = std::max(a->oc, b->oc) <= 64 ? 4 : (std::max(a->oc, b->oc) + 15) / 16;
+        if (q.mid > 4 && q.mid < 8) q.mid = 8;   // (channels behind a layer's count have zero weights, scales and biases)
+        q.proj = pr ? 1 : 0;
+        q.in_hp = iv.hp(); q.in_wp = iv.wp(); q.in_cp = iv.cp; q.in_off = iv.pad;
+        q.h = c->oh; q.w = c->ow;
+        q.out_wp = ov.wp(); q.out_cp = ov.cp; q.out_off = ov.pad;
+        q.tiles_x = (c->ow + 3) / 4; q.tiles_y = (c->oh + 3) / 4;
+        q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
+        q.f16 = ov.f16 ? 1 : 0;
+        // (the next chunk count that a variant is compiled for: the channels behind the tensor read as zero)
+        for (q.chunks = (iv.cp + 31) / 32; q.chunks <= 16 && conv_b16_weight_frags(q) == 0; q.chunks++) {}
+        if (conv_b16_weight_frags(q) == 0 || (long long)q.tiles_x * q.tiles_y > 4096) continue;
+        const size_t halves = conv_b16_weight_frags(q) * (q.f16 ? 1 : 2) * 64 * 8;
+        void* const wp = net->dev_alloc(halves * 2, true);
+        q.wpack = wp;
+        // (untimed: 256 to 64 to 64 to 256, one launch / apart: 9.5 / 15.7 us at 56x56, 17.6 / 21.5 at 80x80, 25.0 / 24.7 at 96x96)
+        bool pick = q.mid == 4 && q.tiles_x * q.tiles_y <= 400;
+        char key[200];
+        snprintf(key, sizeof(key), "blk:%d:%dto%dto%dto%d:%dx%d:r%d:b%d", q.f16, iv.cp, a->oc, b->oc, c->oc, c->oh, c->ow, pr ? 2 : q.res ? 1 : 0, a->bn_fused ? 1 : 0);
+        if (net->sw.get("FYNHIP_FORCE_BLOCK_FUSION")) pick = true;
+        else if (tune_cache_flag(net, key, &pick)) {
+        } else if (!(at && at[0] == '0')) {
+            float t_one = 1e30f, t_apart = 1e30f;
+            for (int rep = 0; rep < 3; rep++) {
+                t_one = std::min(t_one, time_calls(net, [&]() {
+                    if (launch_conv_b16(q, net->stream) != 0) fail(FYN_ERR_DEVICE, "bottleneck launch failed while tuning");
+                }, 10));
+                t_apart = std::min(t_apart, time_calls(net, [&]() {
+                    a->forward_alone(net->stream);
+                    b->forward_alone(net->stream);
+                    if (pr) pr->forward_alone(net->stream);
+                    c->forward_alone(net->stream);
+                }, 10));
+            }
+            if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
+                fprintf(stderr, "[tune] bottleneck %d to %d to %d to %d at %dx%d%s: one launch %.1f us, apart %.1f us\n", iv.cp, a->oc, b->oc, c->oc, c->oh, c->ow, pr ? " with its projection" : "", t_one * 1e3f,
+                        t_apart * 1e3f);
+            // (a near tie goes to the single launch: where networks run side by side, launches are what the chip deals out one
+            // by one.  512 to 128 to 128 to 512 on fp16 tensors at 28x28: 10.9 against 10.5 us, a frame by itself 207 / 206 us, four
+            // instances side by side 100.6 / 103.3)
+            pick = t_one < t_apart * 1.05f;
+            tune_cache_store_flag(net, key, pick);
+        }
+        if (!pick) {
+            net->dev_free(wp);
+            continue;
+        }
+        c->blk = q;
+        c->blk_wpack_dev = wp;
+        c->blk_fused = true;
+        c->blk_layers[0] = a->d.number; c->blk_layers[1] = b->d.number; c->blk_layers[2] = pr ? pr->d.number : -1;
+        joined(true);
+        net->read_until(x, c->d.number);   // (its value-range word is cleared behind its last reader)
+        c->pack_block();
+    }
+}
+
 // A sigmoid or tanh layer whose input comes from a convolution in the row-rolling form and goes nowhere else (the end of
 // the style-net samples): the convolution applies it to what it stores, into the layer's own tensor.  The launch writes
 // that tensor in the convolution's place in the order, earlier than its buffer was handed over for.

@@ -342,6 +342,41 @@ int launch_conv_p16n(const ConvP16Params& p, hipStream_t s);
 // a 1x1 layer and the depthwise 3x3 layer behind it as one launch (conv_d16.hip: conv_e16dw_kernel)
 bool conv_e16dw_supported(int in_cp, int chunks, int dw_stride);
 int launch_conv_e16dw(const ConvP16Params& p, hipStream_t s);
+// A 1x1 layer, the 3x3 layer behind it and the 1x1 layer behind that (a bottleneck) as one launch (conv_b16.hip): h x w
+// positions throughout, 4x4 of them per workgroup.  Index 0, 1, 2: the layers in order; 3: the 1x1 projection of the
+// block's input that the last one adds (proj).
+struct ConvB16Params {
+    // (what a workgroup's first requests depend on stands together: their place in the argument block is one cache line or two)
+    const void* in;
+    const void* wpack;    // [wave 0..7][fragment][plane hi, lo][lane][8 halves]: a wave's in the order it takes them (ConvLayer::pack_block)
+    const unsigned* in_amax;
+    int h, w;
+    int in_wp, in_cp, in_off;   // stored input frame; position (y, x) reads pixel (y + in_off, x + in_off)
+    int tiles_x;
+    float rcp_tiles_x;    // 1.0f / tiles_x
+    int out_cp;
+    const float* in_mul;  // a batch-norm layer in front, as in ConvP16Params
+    const float* in_add;
+    const float* scale[4];
+    const float* bias[4];
+    const void* res;      // what the last layer adds, or nullptr
+    int res_wp, res_cp, res_off, res_relu, res_scale;
+    int out_wp, out_off;
+    void* out;
+    unsigned* out_amax;
+    Act act[3];           // on the fetch of each layer's input
+    float acc_mul[4];
+    unsigned* reset[4];
+    int nreset;
+    int chunks;           // chunks of 32 channels of the input
+    int mid;              // fragments of 16 channels of the two layers in between
+    int proj;
+    int in_hp, tiles_y;
+    int f16;
+};
+size_t conv_b16_weight_frags(const ConvB16Params& p);   // fragments in wpack; 0: no such compiled combination
+size_t conv_b16_lds_bytes(const ConvB16Params& p);
+int launch_conv_b16(const ConvB16Params& p, hipStream_t s);
 int conv_kr16_variant_count();
 void conv_kr16_variant(int index, int* taps, int* chunks, int* fm, int* th, int* tw, int* stride);   // compiled combinations: kernel taps, 32-channel chunks, fragments per block, tile
 size_t conv_kr16_lds_bytes(const ConvP16Params& p, int k);

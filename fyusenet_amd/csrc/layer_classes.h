@@ -115,12 +115,22 @@ class ConvLayer : public Layer {
         pp.in_amax = in_w;
         pp.out_amax = out_w;
     }
+    int reset_room() const override {
+        if (direct || !set_up || pj_into >= 0 || blk_into >= 0) return 0;   // (a layer computed in another one's launch has none to clear words in)
+        return 4 - (rows ? rp.nreset : (p16 ? pp.nreset : launch.p.nreset));
+    }
     bool add_range_reset(unsigned* w) override {
-        if (direct || !set_up || pj_into >= 0) return false;   // (a projection computed by its reader has no launch to clear words in)
+        if (reset_room() <= 0) return false;
         int& n = rows ? rp.nreset : (p16 ? pp.nreset : launch.p.nreset);
-        if (n >= 4) return false;
         (rows ? rp.reset : (p16 ? pp.reset : launch.p.reset))[n++] = w;
         return true;
+    }
+    // the words that the layer's own launch clears, for a launch that takes its place
+    int own_resets(unsigned** to) const {
+        const int n = rows ? rp.nreset : (p16 ? pp.nreset : launch.p.nreset);
+        unsigned* const* r = rows ? rp.reset : (p16 ? pp.reset : launch.p.reset);
+        for (int i = 0; i < n; i++) to[i] = r[i];
+        return n;
     }
     // 16-position-fragment form of a 3x3 convolution (conv_p16.hip): the compiled combinations that fit the layer are
     // timed (the four with the fewest fragment rounds on 256 CUs), and the best is kept if it beats the tuned launch of
@@ -1354,6 +1364,8 @@ class ConvLayer : public Layer {
         have_weights = true;
         if (pj_fused) pack_two_sources();
         if (pj_into >= 0) static_cast<ConvLayer*>(net->layer(pj_into))->pack_two_sources();
+        if (blk_fused) pack_block();
+        if (blk_into >= 0) static_cast<ConvLayer*>(net->layer(blk_into))->pack_block();
     }
     // the weights once more, in the layout of the launch that also runs the depthwise layer behind this one
     void pack_edw() {
@@ -1365,26 +1377,29 @@ class ConvLayer : public Layer {
     }
     void forward(hipStream_t s) override {
         if (!have_weights) fail(FYN_ERR_STATE, "layer %s (%d): forward() without weights", d.name, d.number);
+        if (blk_into >= 0 && net->fusion_on()) return;   // computed in the launch of the block's last layer
+        if (blk_fused && net->fusion_on()) {
+            if (launch_conv_b16(with_block(), s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
+            return;
+        }
+        forward_alone(s);
+    }
+    // (without the layers in front of it that a block's last layer computes as well)
+    void forward_alone(hipStream_t s) {
         if (pj_into >= 0 && net->fusion_on() && static_cast<ConvLayer*>(net->layer(pj_into))->pj_spread_ok) return;   // computed by the layer that adds it
         if (pj_fused && pj_spread_ok && net->fusion_on()) {
             ConvP16Params q = pj;   // (value-range words as the layer's own launch carries them)
             q.in_amax = tin(0).amax;
             q.in2_amax = net->layer(pj_layer_no)->tin(0).amax;
             q.out_amax = tout().amax;
-            const int n = rows ? rp.nreset : (p16 ? pp.nreset : launch.p.nreset);
-            unsigned* const* r = rows ? rp.reset : (p16 ? pp.reset : launch.p.reset);
-            q.nreset = n;
-            for (int i = 0; i < n; i++) q.reset[i] = r[i];
+            q.nreset = own_resets(q.reset);
             if (launch_conv_kr16(q, 1, s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
         }
         if (edw_fused && net->fusion_on()) {
             ConvP16Params q = edw;   // (value-range words as the layer's own launch carries them)
             q.in_amax = tin(0).amax;
-            const int n = rows ? rp.nreset : (p16 ? pp.nreset : launch.p.nreset);
-            unsigned* const* r = rows ? rp.reset : (p16 ? pp.reset : launch.p.reset);
-            q.nreset = n;
-            for (int i = 0; i < n; i++) q.reset[i] = r[i];
+            q.nreset = own_resets(q.reset);
             if (launch_conv_e16dw(q, s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
         }
@@ -1424,6 +1439,14 @@ class ConvLayer : public Layer {
         if (wide && !fused) launch_shift_reduce(sr, s);
     }
     std::string info() const override {
+        if (blk_into >= 0) return "conv " + std::to_string(k) + "x" + std::to_string(k) + " (runs inside the launch of layer " + std::to_string(blk_into) + "; no launch of its own); apart: " + own_info();
+        if (blk_fused) {
+            char buf[300];
+            snprintf(buf, sizeof(buf), "conv_b16 %s a bottleneck in one launch: layers %d (1x1, %d channels in%s), %d (3x3, %d channels) and this one (%d channels out)%s, 4x4 positions per workgroup, blocks=%d lds=%zu; apart: ",
+                     blk.f16 ? "f16" : "f16x2-split", blk_layers[0], blk.in_cp, blk.in_mul ? ", the batch-norm layer in front applied while staging" : "", blk_layers[1], 16 * blk.mid, blk.out_cp,
+                     blk.proj ? (" with the projection " + std::to_string(blk_layers[2])).c_str() : "", blk.tiles_x * blk.tiles_y, conv_b16_lds_bytes(blk));
+            return buf + own_info();
+        }
         if (fn_layer_no >= 0) return own_info() + "; the function layer " + std::to_string(fn_layer_no) + " behind it is applied to what is stored";
         if (pj_into >= 0 && static_cast<ConvLayer*>(net->layer(pj_into))->pj_spread_ok)
             return "conv 1x1 projection (runs inside the launch of layer " + std::to_string(pj_into) + "; no launch of its own); apart: " + own_info();
@@ -1639,6 +1662,64 @@ class ConvLayer : public Layer {
         FYN_HIP(hipStreamSynchronize(net->stream));
         FYN_HIP(hipMemcpyAsync(pj_wpack_dev, pack.data(), pack.size() * 2, hipMemcpyHostToDevice, net->stream));
         FYN_HIP(hipStreamSynchronize(net->stream));
+    }
+    // The 1x1 layer, the 3x3 layer and this 1x1 layer of a bottleneck in one launch of conv_b16_kernel (conv_b16.hip), in this
+    // layer's place (fuse_block_layers below); with the projection this layer adds, where that reads the block's input too.
+    bool blk_fused = false;
+    int blk_into = -1;                    // on the layers in front: the layer whose launch computes them
+    int blk_layers[3] = {-1, -1, -1};     // the 1x1 layer, the 3x3 layer, the projection
+    ConvB16Params blk{};
+    void* blk_wpack_dev = nullptr;
+    ConvB16Params with_block() const {
+        ConvB16Params q = blk;   // (value-range words as the layers' own launches carry them)
+        q.in_amax = q.in_mul ? nullptr : net->layer(blk_layers[0])->tin(0).amax;
+        q.out_amax = tout().amax;
+        q.nreset = own_resets(q.reset);
+        return q;
+    }
+    // weights of that form: [wave][steps of the first layer, of the second, of the last and the projection][plane][lane][8
+    // halves]; the waves that share a fragment of one of the first two layers take its steps in turn
+    void pack_block() {
+        const ConvLayer* L[4] = {static_cast<ConvLayer*>(net->layer(blk_layers[0])), static_cast<ConvLayer*>(net->layer(blk_layers[1])), this,
+                                 blk.proj ? static_cast<ConvLayer*>(net->layer(blk_layers[2])) : nullptr};
+        float wmul[4] = {1.f, 1.f, 1.f, 1.f};
+        for (int i = 0; i < 4; i++) {
+            if (!L[i]) continue;
+            if (L[i]->block.empty()) return;
+            wmul[i] = weight_prescale(L[i]->block.data() + L[i]->oc, (size_t)L[i]->oc * L[i]->k * L[i]->k * L[i]->d.in_channels);
+            blk.acc_mul[i] = 1.0f / wmul[i];
+        }
+        const int npl = blk.f16 ? 1 : 2;
+        std::vector<uint16_t> pack(conv_b16_weight_frags(blk) * npl * 64 * 8, 0);
+        uint16_t* base = pack.data();
+        auto put = [&](int li, int mf, int tap, int chunk, bool there) {   // one fragment of layer li
+            const ConvLayer& l = *L[li];
+            const float* w = l.block.data() + l.oc;
+            const int cin = l.d.in_channels, taps = l.k * l.k;
+            for (int lane = 0; there && lane < 64; lane++) {
+                const int o = mf * 16 + (lane & 15);
+                for (int j = 0; o < l.oc && j < 8; j++) {
+                    const int ci = chunk * 32 + 8 * (lane >> 4) + j;
+                    if (ci >= cin) continue;
+                    const float v = w[((size_t)o * taps + tap) * cin + ci] * wmul[li];
+                    const uint16_t hi = f2h_bits(v);
+                    base[(size_t)lane * 8 + j] = hi;
+                    if (npl == 2) base[(size_t)(64 + lane) * 8 + j] = f2h_bits(v - h2f(hi));
+                }
+            }
+            base += (size_t)npl * 64 * 8;
+        };
+        const int shares = 8 / blk.mid, cm = blk.mid / 2, pairs = ((blk.out_cp + 15) / 16 + 15) / 16;
+        for (int wave = 0; wave < 8; wave++) {
+            for (int li = 0; li < 2; li++) {
+                const int cn = li ? cm : blk.chunks, total = cn * (li ? 9 : 1);
+                for (int step = wave % shares; step - wave % shares < total; step += shares) put(li, wave / shares, step / cn, step % cn, step < total);
+            }
+            for (int pr = 0; pr < pairs; pr++)
+                for (int c = 0; c < cm + (blk.proj ? blk.chunks : 0); c++)
+                    for (int f = 0; f < 2; f++) put(c < cm ? 2 : 3, wave + (2 * pr + f) * 8, 0, c < cm ? c : c - cm, true);
+        }
+        reupload(net, static_cast<uint16_t*>(blk_wpack_dev), pack);
     }
     bool takes_depthwise() const {
         // (not a layer that already runs the depthwise layer behind it: one launch cannot do both)

@@ -186,13 +186,13 @@ class TransConvLayer : public Layer {
         pp.in_amax = tin(0).amax;
         pp.out_amax = tout().amax;
     }
+    int reset_room() const override { return !set_up ? 0 : p16 ? 4 - pp.nreset : group.subs.empty() ? 0 : 4 - group.subs[0].p.nreset; }
     bool add_range_reset(unsigned* w) override {
+        if (reset_room() <= 0) return false;
         if (p16) {
-            if (!set_up || pp.nreset >= 4) return false;
             pp.reset[pp.nreset++] = w;
             return true;
         }
-        if (!set_up || group.subs.empty() || group.subs[0].p.nreset >= 4) return false;
         group.subs[0].p.reset[group.subs[0].p.nreset++] = w;
         group.sync();
         return true;
