@@ -473,6 +473,7 @@ void Net::setup() {
     fuse_projection_layers(this);
     fuse_batchnorm_layers(this);
     fuse_block_layers(this);
+    fuse_pair_layers(this);
     fuse_function_layers(this);
     fuse_concat_layers(this);
     fuse_argmax_layers(this);

@@ -257,6 +257,7 @@ void keep_projection_inputs(Net* net);    // before buffers are assigned: inputs
 void fuse_projection_layers(Net* net);   // after every layer's setup(): 1x1 shortcut projections that the 1x1 layer adding them can compute in its own launch
 std::vector<std::pair<int, int>> keep_block_inputs(Net* net);   // ... and, while they are assigned, inputs of bottlenecks until their last layer, which may compute them, has run; (tensor, its last reader)
 void fuse_block_layers(Net* net);        // after the other passes on convolutions: a 1x1, a 3x3 and a 1x1 layer in one launch
+void fuse_pair_layers(Net* net);         // ... two 3x3 layers between tensors of few channels in one launch
 void fuse_depthwise_layers(Net* net);   // after every layer's setup(): depthwise 3x3 layers that their 1x1 reader can compute itself
 void fuse_function_layers(Net* net);   // after every layer's setup(): sigmoid / tanh layers that the row-rolling convolution in front of them can apply to what it stores
 void fuse_concat_layers(Net* net);   // after every layer's setup(): bilinear scale layers in front of concatenations and batch-norm layers behind them

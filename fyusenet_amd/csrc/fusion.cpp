@@ -337,40 +337,46 @@ void fuse_batchnorm_layers(Net* net) {
     }
 }
 
+// The convolution in front of layer `l` that nothing else reads and that adds nothing itself.
+static ConvLayer* alone_in_front(Net* net, const ConvLayer* l) {
+    if (l->in.empty() || l->in[0] < 0) return nullptr;
+    const Tensor& t = net->tensors[l->in[0]];
+    if (t.producer < 0 || t.locked) return nullptr;
+    int readers = 0;
+    for (auto& kv : net->layers)
+        for (int i : kv.second->in) readers += i == l->in[0];
+    ConvLayer* p = readers == 1 ? dynamic_cast<ConvLayer*>(net->layer(t.producer)) : nullptr;
+    return p && !(p->d.flags & FYN_FLAG_RESIDUAL_INPUT) && p->d.number < l->d.number && !p->in.empty() && p->in[0] >= 0 ? p : nullptr;
+}
+static bool plain_conv(const ConvLayer* l, int k) { return l && l->k == k && l->stride == 1 && l->dil == 1 && !l->frac_shift && !l->direct && !l->wide; }
 // The bottleneck that ends with layer `c`, by the graph alone: a 1x1 layer, a 3x3 layer that alone reads it, and `c`, a 1x1
 // layer that alone reads that one; no step, no dilation, nothing between them.
-static bool block_of(Net* net, ConvLayer* c, ConvLayer*& a, ConvLayer*& b) {
-    auto plain = [](const ConvLayer* l, int k) {
-        return l && l->k == k && l->stride == 1 && l->dil == 1 && !l->clamp && !l->frac_shift && !l->direct && !l->wide;
-    };
-    auto in_front = [&](ConvLayer* l) -> ConvLayer* {
-        if (l->in.empty() || l->in[0] < 0) return nullptr;
-        const Tensor& t = net->tensors[l->in[0]];
-        if (t.producer < 0 || t.locked) return nullptr;
-        int readers = 0;
-        for (auto& kv : net->layers)
-            for (int i : kv.second->in) readers += i == l->in[0];
-        ConvLayer* p = readers == 1 ? dynamic_cast<ConvLayer*>(net->layer(t.producer)) : nullptr;
-        return p && !(p->d.flags & FYN_FLAG_RESIDUAL_INPUT) && p->d.number < l->d.number ? p : nullptr;
-    };
-    if (!plain(c, 1)) return false;
-    b = in_front(c);
-    if (!plain(b, 3)) return false;
-    a = in_front(b);
-    return plain(a, 1) && !a->in.empty() && a->in[0] >= 0 && a->oh == c->oh && a->ow == c->ow && b->oh == c->oh && b->ow == c->ow;
+static bool block_of(Net* net, const ConvLayer* c, ConvLayer*& a, ConvLayer*& b) {
+    if (!plain_conv(c, 1)) return false;
+    b = alone_in_front(net, c);
+    if (!plain_conv(b, 3) || b->clamp) return false;
+    a = alone_in_front(net, b);
+    return plain_conv(a, 1) && a->oh == c->oh && a->ow == c->ow && b->oh == c->oh && b->ow == c->ow;
 }
-// While buffers are assigned, the input of such a block is read until its last layer has run, which may compute all of it (the
-// tensors' last readers as they were: whether the block is joined is not known yet).
+// The 3x3 layer `a` that the 3x3 layer `c` alone reads, both with the same rule at the frame's edge.
+static bool pair_of(Net* net, const ConvLayer* c, ConvLayer*& a) {
+    if (!plain_conv(c, 3)) return false;
+    a = alone_in_front(net, c);
+    return plain_conv(a, 3) && a->clamp == c->clamp && a->oh == c->oh && a->ow == c->ow;
+}
+// While buffers are assigned, the input of such a block or pair is read until its last layer has run, which may compute all of
+// it (the tensors' last readers as they were: whether the layers are joined is not known yet).
 std::vector<std::pair<int, int>> keep_block_inputs(Net* net) {
     std::vector<std::pair<int, int>> were;
-    if (net->sw.get("FYNHIP_NO_BLOCK_FUSION") || !net->reuse_buffers) return were;
+    if (!net->reuse_buffers) return were;
     auto keep = [&](int tensor, int layer_no) {
         were.push_back({tensor, net->tensors[tensor].last_reader});
         net->read_until(tensor, layer_no);
     };
     for (auto& kv : net->layers) {
         ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
-        if (!c || !block_of(net, c, a, b)) continue;
+        if (c && !net->sw.get("FYNHIP_NO_PAIR_FUSION") && pair_of(net, c, a) && a->d.in_channels <= 64) keep(a->in[0], c->d.number);
+        if (!c || net->sw.get("FYNHIP_NO_BLOCK_FUSION") || !block_of(net, c, a, b)) continue;
         keep(a->in[0], c->d.number);
         const Tensor& t = net->tensors[a->in[0]];
         if (t.producer < 0) continue;
@@ -379,15 +385,30 @@ std::vector<std::pair<int, int>> keep_block_inputs(Net* net) {
     }
     return were;
 }
+// (tests: whoever forces a form of a layer wants to see that form)
+static bool single_form_forced(const Net* net) {
+    for (const char* form : {"FYNHIP_FORCE_PROJECTION_FUSION", "FYNHIP_FORCE_KR16_CONV", "FYNHIP_KR16_FM", "FYNHIP_FORCE_D16_CONV", "FYNHIP_D16_BLOCKS", "FYNHIP_FORCE_P16_CONV", "FYNHIP_P16_TILE",
+                             "FYNHIP_FORCE_G16_CONV", "FYNHIP_G16_FRAGS", "FYNHIP_FORCE_P16N_CONV", "FYNHIP_P16N_ROWS", "FYNHIP_FORCE_KSPLIT", "FYNHIP_CONV_TILE", "FYNHIP_CONV_KC",
+                             "FYNHIP_CONV_KC_MAX", "FYNHIP_CONV_PD"})
+        if (net->sw.get(form)) return true;
+    return false;
+}
+// Whether the layers `front` can go into the launch of layer `last`, which then reads tensor x: the words of value ranges
+// that their launches clear need another launch to do so.
+static bool words_survive(Net* net, const std::vector<ConvLayer*>& front, int last, int x) {
+    const int reader = net->tensors[x].last_reader, lost = net->words_without_reset();
+    for (ConvLayer* l : front) l->blk_into = last;
+    net->read_until(x, last);
+    const int then = net->words_without_reset();
+    for (ConvLayer* l : front) l->blk_into = -1;
+    net->tensors[x].last_reader = reader;
+    return then <= lost;
+}
 // Bottlenecks (conv_b16.hip) as one launch in the place of their last layer, timed against the launches they run as now:
 // with the batch-norm layer in front that the first layer applies, or the projection that the last one adds.
 void fuse_block_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_BLOCK_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV") || !net->reuse_buffers) return;
-    // (tests: whoever forces a form of one of the layers wants to see that form)
-    if (!net->sw.get("FYNHIP_FORCE_BLOCK_FUSION"))
-        for (const char* other : {"FYNHIP_FORCE_PROJECTION_FUSION", "FYNHIP_FORCE_KR16_CONV", "FYNHIP_KR16_FM", "FYNHIP_FORCE_D16_CONV", "FYNHIP_D16_BLOCKS", "FYNHIP_FORCE_P16_CONV", "FYNHIP_P16_TILE",
-                                  "FYNHIP_FORCE_KSPLIT", "FYNHIP_CONV_TILE", "FYNHIP_CONV_KC", "FYNHIP_CONV_KC_MAX", "FYNHIP_CONV_PD"})
-            if (net->sw.get(other)) return;
+    if (!net->sw.get("FYNHIP_FORCE_BLOCK_FUSION") && single_form_forced(net)) return;
     const char* at = net->sw.get("FYNHIP_AUTOTUNE");
     for (auto& kv : net->layers) {
         ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
@@ -421,18 +442,9 @@ void fuse_block_layers(Net* net) {
         int x = a->in[0];
         if (a->bn_fused) x = net->layer(a->bn_layer_no)->in[0];
         if (!net->alone(x, a->d.number, c->d.number)) continue;
-        // (the words of value ranges that the launches in front clear: another launch has to be there for them)
-        auto joined = [&](bool yes) {
-            a->blk_into = b->blk_into = yes ? c->d.number : -1;
-            if (pr) pr->blk_into = a->blk_into;
-        };
-        const int reader = net->tensors[x].last_reader, lost = net->words_without_reset();
-        joined(true);
-        net->read_until(x, c->d.number);
-        const int lost_then = net->words_without_reset();
-        joined(false);
-        net->tensors[x].last_reader = reader;
-        if (lost_then > lost) continue;
+        std::vector<ConvLayer*> front = {a, b};
+        if (pr) front.push_back(pr);
+        if (!words_survive(net, front, c->d.number, x)) continue;
         const ConvLayer* L[4] = {a, b, c, pr};
         for (int i = 0; i < 4; i++) {
             if (!L[i]) continue;
@@ -494,9 +506,112 @@ void fuse_block_layers(Net* net) {
         c->blk_wpack_dev = wp;
         c->blk_fused = true;
         c->blk_layers[0] = a->d.number; c->blk_layers[1] = b->d.number; c->blk_layers[2] = pr ? pr->d.number : -1;
-        joined(true);
+        for (ConvLayer* l : front) l->blk_into = c->d.number;
         net->read_until(x, c->d.number);   // (its value-range word is cleared behind its last reader)
         c->pack_block();
+    }
+}
+
+// Pairs of 3x3 layers between tensors of few channels (conv_c16.hip) as one launch in the place of the second.
+void fuse_pair_layers(Net* net) {
+    if (net->sw.get("FYNHIP_NO_PAIR_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV") || !net->reuse_buffers) return;
+    const bool forced = net->sw.get("FYNHIP_FORCE_PAIR_FUSION") != nullptr;
+    if (!forced && single_form_forced(net)) return;
+    const char* at = net->sw.get("FYNHIP_AUTOTUNE");
+    const int want_th = net->sw.get("FYNHIP_PAIR_ROWS") ? atoi(net->sw.get("FYNHIP_PAIR_ROWS")) : 0;   // (tests: that tile height)
+    for (auto& kv : net->layers) {
+        ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr;
+        if (!c || !pair_of(net, c, a) || a->blk_into >= 0 || c->blk_into >= 0 || a->pair_fused || a->fn_layer_no >= 0 || c->fn_layer_no >= 0) continue;
+        const TView &iv = a->tin(0).v, &mv = a->tout().v, &ov = c->tout().v;
+        if (iv.f16 != ov.f16 || mv.f16 != ov.f16 || iv.cp % 8 != 0 || mv.cp != iv.cp || ov.cp % 4 != 0 || a->d.in_channels > iv.cp || c->oc > ov.cp || c->d.in_channels != a->oc) continue;
+        // (positions beside a layer's input are zeros behind its activation as well, or repeat the edge)
+        if (!c->clamp && (a->act().lo > 0.f || a->act().hi < 0.f || c->act().lo > 0.f || c->act().hi < 0.f)) continue;
+        if (c->clamp && (iv.pad != 0 || mv.pad != 0)) continue;
+        ConvC16Params q{};
+        if (c->d.flags & FYN_FLAG_RESIDUAL_INPUT) {
+            if (c->in.size() < 2 || c->in[1] < 0 || c->in[1] == c->in[0]) continue;
+            const TView& rv = c->tin(1).v;
+            if (rv.f16 != ov.f16 || rv.cp < ov.cp || rv.cp % 4 != 0) continue;
+            q.res = rv.ptr; q.res_wp = rv.wp(); q.res_cp = rv.cp; q.res_off = rv.pad;
+            q.res_relu = (c->d.flags & FYN_FLAG_RELU_ON_RESIDUAL) ? 1 : 0;
+            q.res_scale = ((c->d.flags & FYN_FLAG_BATCHNORM_ON_RESIDUAL) && (c->d.flags & FYN_FLAG_POST_BATCHNORM)) ? 1 : 0;
+        }
+        // (the launch reads the pair's input in the second layer's place in the order)
+        const int x = a->in[0];
+        if (!net->alone(x, a->d.number, c->d.number) || !words_survive(net, {a}, c->d.number, x)) continue;
+        const ConvLayer* L[2] = {a, c};
+        for (int i = 0; i < 2; i++) {
+            q.scale[i] = L[i]->scale_dev; q.bias[i] = L[i]->bias_dev;
+            q.acc_mul[i] = 1.f;
+            q.act[i] = L[i]->act();
+        }
+        q.in = iv.ptr; q.in_hp = iv.hp(); q.in_wp = iv.wp(); q.in_cp = iv.cp; q.in_off = iv.pad;
+        q.h = c->oh; q.w = c->ow;
+        q.clamp = c->clamp ? 1 : 0;
+        q.out = ov.ptr; q.out_wp = ov.wp(); q.out_cp = ov.cp; q.out_off = ov.pad;
+        q.groups = iv.cp / 8;
+        q.f16 = ov.f16 ? 1 : 0;
+        q.tiles_x = (q.w + 15) / 16; q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
+        std::vector<ConvC16Params> cands;
+        size_t halves = 0;
+        for (int i = 0; i < conv_c16_count(); i++) {
+            int f16, groups, fr, th;
+            conv_c16_variant(i, &f16, &groups, &fr, &th);
+            if (f16 != q.f16 || groups != q.groups || ov.cp > 16 * fr || (want_th && th != want_th)) continue;
+            ConvC16Params t = q;
+            t.th = th;
+            t.tiles_y = (q.h + th - 1) / th;
+            if ((long long)t.tiles_x * t.tiles_y > (1 << 20)) continue;
+            cands.push_back(t);
+            int shares = 0;
+            const int steps = conv_c16_steps(t, &shares);
+            halves = std::max(halves, (size_t)2 * fr * shares * steps * (q.f16 ? 1 : 2) * 64 * 8);
+        }
+        if (cands.empty()) continue;
+        void* const wp = net->dev_alloc(halves * 2, true);
+        for (ConvC16Params& t : cands) t.wpack = wp;
+        // (untimed: the tallest tiles that give half of the CUs a workgroup, on as many positions as are two rounds of the tallest
+        // at most.  One launch / apart, fp32: 12x16 7.9 / 8.3 us, 156x128 12.0 / 16.3, 256x256 -- 688 tiles of six rows -- 32.0 / 29.2)
+        int pick = 0;
+        for (size_t i = 0; i < cands.size(); i++)
+            if (cands[i].tiles_x * cands[i].tiles_y >= 128) pick = (int)i;
+        if (!forced && (cands.back().tiles_x * cands.back().tiles_y > 512 || cands[0].tiles_x * cands[0].tiles_y < 64)) pick = -1;
+        char key[200];
+        snprintf(key, sizeof(key), "pair:%d:%dto%dto%d:%dx%d:r%d:e%d", q.f16, iv.cp, a->oc, c->oc, c->oh, c->ow, q.res ? 1 : 0, q.clamp);
+        if (want_th || tune_cache_pick(net, key, cands.size(), forced, [&](size_t i, int b, int) { return cands[i].th == b; }, &pick)) {
+        } else if (!(at && at[0] == '0')) {
+            float t_one = 1e30f, t_apart = 1e30f;
+            for (int rep = 0; rep < 3; rep++) {
+                for (size_t i = 0; i < cands.size(); i++) {
+                    const float t = time_calls(net, [&]() {
+                        if (launch_conv_c16(cands[i], net->stream) != 0) fail(FYN_ERR_DEVICE, "launch of two 3x3 layers failed while tuning");
+                    }, 10);
+                    if (t < t_one) { t_one = t; pick = (int)i; }
+                }
+                t_apart = std::min(t_apart, time_calls(net, [&]() {
+                    a->forward_alone(net->stream);
+                    c->forward_alone(net->stream);
+                }, 10));
+            }
+            if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
+                fprintf(stderr, "[tune] 3x3 %d to %d to %d at %dx%d: one launch (%d rows) %.1f us, apart %.1f us\n", iv.cp, a->oc, c->oc, c->oh, c->ow, cands[pick].th, t_one * 1e3f, t_apart * 1e3f);
+            // (a tenth: on a few rows of tiles, where both ways are a chain of latencies, the frame does not show a smaller lead.  40 to 40
+            // to 40 at 33x50 on fp32 tensors 8.1 / 8.9 us here, the sample net's frame 47.5 / 47.4; on fp16 tensors 6.5 / 7.4, 38.2 / 40.1)
+            const bool win = t_one < t_apart * 0.9f;
+            tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].th, 0);
+            if (!win && !forced) pick = -1;
+        }
+        if (pick < 0) {
+            net->dev_free(wp);
+            continue;
+        }
+        c->pair = cands[pick];
+        c->pair_wpack_dev = wp;
+        c->pair_fused = true;
+        c->pair_layer = a->d.number;
+        a->blk_into = c->d.number;
+        net->read_until(x, c->d.number);
+        c->pack_pair();
     }
 }
 

@@ -377,6 +377,38 @@ struct ConvB16Params {
 size_t conv_b16_weight_frags(const ConvB16Params& p);   // fragments in wpack; 0: no such compiled combination
 size_t conv_b16_lds_bytes(const ConvB16Params& p);
 int launch_conv_b16(const ConvB16Params& p, hipStream_t s);
+// Two 3x3 layers between tensors of few channels, one behind the other, as one launch (conv_c16.hip): h x w positions, th rows of
+// sixteen per workgroup.
+struct ConvC16Params {
+    const void* in;
+    const void* wpack;    // [layer][fragment of 16 output channels][share of the steps][step][plane][lane][8 halves] (ConvLayer::pack_pair)
+    const unsigned* in_amax;
+    int h, w;
+    int in_wp, in_cp, in_off;   // stored input frame; position (y, x) is pixel (y + in_off, x + in_off)
+    int tiles_x;
+    float rcp_tiles_x;    // 1.0f / tiles_x
+    int clamp;            // both layers: positions outside the frame repeat its edge instead of reading 0
+    int out_cp;
+    const float* scale[2];
+    const float* bias[2];
+    const void* res;      // what the second layer adds, or nullptr
+    int res_wp, res_cp, res_off, res_relu, res_scale;
+    int out_wp, out_off;
+    void* out;
+    unsigned* out_amax;
+    Act act[2];           // on the fetch of each layer's input
+    float acc_mul[2];
+    unsigned* reset[4];
+    int nreset;
+    int groups, th;       // groups of eight channels of the input and of the tensor in between; rows of a tile
+    int in_hp, tiles_y;
+    int f16;
+};
+int conv_c16_count();     // compiled combinations
+void conv_c16_variant(int index, int* f16, int* groups, int* frags, int* th);
+int conv_c16_steps(const ConvC16Params& p, int* shares);   // of each share of a layer's reduction; 0: no such combination
+size_t conv_c16_lds_bytes(const ConvC16Params& p);
+int launch_conv_c16(const ConvC16Params& p, hipStream_t s);
 int conv_kr16_variant_count();
 void conv_kr16_variant(int index, int* taps, int* chunks, int* fm, int* th, int* tw, int* stride);   // compiled combinations: kernel taps, 32-channel chunks, fragments per block, tile
 size_t conv_kr16_lds_bytes(const ConvP16Params& p, int k);

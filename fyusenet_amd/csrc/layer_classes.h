@@ -1365,7 +1365,12 @@ class ConvLayer : public Layer {
         if (pj_fused) pack_two_sources();
         if (pj_into >= 0) static_cast<ConvLayer*>(net->layer(pj_into))->pack_two_sources();
         if (blk_fused) pack_block();
-        if (blk_into >= 0) static_cast<ConvLayer*>(net->layer(blk_into))->pack_block();
+        if (pair_fused) pack_pair();
+        if (blk_into >= 0) {
+            ConvLayer* c = static_cast<ConvLayer*>(net->layer(blk_into));
+            if (c->blk_fused) c->pack_block();
+            if (c->pair_fused) c->pack_pair();
+        }
     }
     // the weights once more, in the layout of the launch that also runs the depthwise layer behind this one
     void pack_edw() {
@@ -1377,7 +1382,11 @@ class ConvLayer : public Layer {
     }
     void forward(hipStream_t s) override {
         if (!have_weights) fail(FYN_ERR_STATE, "layer %s (%d): forward() without weights", d.name, d.number);
-        if (blk_into >= 0 && net->fusion_on()) return;   // computed in the launch of the block's last layer
+        if (blk_into >= 0 && net->fusion_on()) return;   // computed in the launch of the block's or the pair's last layer
+        if (pair_fused && net->fusion_on()) {
+            if (launch_conv_c16(with_pair(), s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
+            return;
+        }
         if (blk_fused && net->fusion_on()) {
             if (launch_conv_b16(with_block(), s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
@@ -1440,6 +1449,12 @@ class ConvLayer : public Layer {
     }
     std::string info() const override {
         if (blk_into >= 0) return "conv " + std::to_string(k) + "x" + std::to_string(k) + " (runs inside the launch of layer " + std::to_string(blk_into) + "; no launch of its own); apart: " + own_info();
+        if (pair_fused) {
+            char buf[300];
+            snprintf(buf, sizeof(buf), "conv_c16 %s layer %d (3x3) and this one in one launch, %dx16 positions per workgroup, blocks=%d lds=%zu; apart: ", pair.f16 ? "f16" : "f16x2-split", pair_layer, pair.th,
+                     pair.tiles_x * pair.tiles_y, conv_c16_lds_bytes(pair));
+            return buf + own_info();
+        }
         if (blk_fused) {
             char buf[300];
             snprintf(buf, sizeof(buf), "conv_b16 %s a bottleneck in one launch: layers %d (1x1, %d channels in%s), %d (3x3, %d channels) and this one (%d channels out)%s, 4x4 positions per workgroup, blocks=%d lds=%zu; apart: ",
@@ -1662,6 +1677,51 @@ class ConvLayer : public Layer {
         FYN_HIP(hipStreamSynchronize(net->stream));
         FYN_HIP(hipMemcpyAsync(pj_wpack_dev, pack.data(), pack.size() * 2, hipMemcpyHostToDevice, net->stream));
         FYN_HIP(hipStreamSynchronize(net->stream));
+    }
+    // The 3x3 layer in front of this 3x3 layer in the same launch, one of conv_c16_kernel (conv_c16.hip; fuse_pair_layers below)
+    bool pair_fused = false;
+    int pair_layer = -1;
+    ConvC16Params pair{};
+    void* pair_wpack_dev = nullptr;
+    ConvC16Params with_pair() const {
+        ConvC16Params q = pair;   // (value-range words as the layers' own launches carry them)
+        q.in_amax = net->layer(pair_layer)->tin(0).amax;
+        q.out_amax = tout().amax;
+        q.nreset = own_resets(q.reset);
+        return q;
+    }
+    // weights of that form: [layer][cout fragment][share][step][plane][lane][8 halves]; step s of share h of n takes
+    // the groups of eight channels 4 (h + n s) .. of the window, lane / 16 picking one
+    void pack_pair() {
+        const ConvLayer* L[2] = {static_cast<ConvLayer*>(net->layer(pair_layer)), this};
+        const int npl = pair.f16 ? 1 : 2, groups = pair.groups, frags = (8 * groups + 15) / 16;
+        int shares = 0;
+        const int spw = conv_c16_steps(pair, &shares);
+        std::vector<uint16_t> pack((size_t)2 * frags * shares * spw * npl * 64 * 8, 0);
+        uint16_t* base = pack.data();
+        for (int li = 0; li < 2; li++) {
+            if (L[li]->block.empty()) return;
+            const float* w = L[li]->block.data() + L[li]->oc;
+            const int cin = L[li]->d.in_channels;
+            const float wmul = weight_prescale(w, (size_t)L[li]->oc * 9 * cin);
+            pair.acc_mul[li] = 1.0f / wmul;
+            for (int mf = 0; mf < frags; mf++)
+                for (int share = 0; share < shares; share++)
+                    for (int s = 0; s < spw; s++, base += (size_t)npl * 64 * 8)
+                        for (int lane = 0; lane < 64; lane++) {
+                            const int o = mf * 16 + (lane & 15), g = 4 * (share + shares * s) + (lane >> 4), tap = g / groups;
+                            if (o >= L[li]->oc || tap >= 9) continue;
+                            for (int j = 0; j < 8; j++) {
+                                const int ci = (g % groups) * 8 + j;
+                                if (ci >= cin) continue;
+                                const float v = w[((size_t)o * 9 + tap) * cin + ci] * wmul;
+                                const uint16_t hi = f2h_bits(v);
+                                base[(size_t)lane * 8 + j] = hi;
+                                if (npl == 2) base[(size_t)(64 + lane) * 8 + j] = f2h_bits(v - h2f(hi));
+                            }
+                        }
+        }
+        reupload(net, static_cast<uint16_t*>(pair_wpack_dev), pack);
     }
     // The 1x1 layer, the 3x3 layer and this 1x1 layer of a bottleneck in one launch of conv_b16_kernel (conv_b16.hip), in this
     // layer's place (fuse_block_layers below); with the projection this layer adds, where that reads the block's input too.
