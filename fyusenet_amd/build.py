@@ -24,8 +24,9 @@ def build(verbose=True, jobs=8):
     objs = []
     units = [("conv_mfma.hip", "conv_mfma.part%d.o" % i, ["-DFYN_CONV_PARTS=%d" % CONV_PARTS, "-DFYN_CONV_PART=%d" % i])
              for i in range(CONV_PARTS)]
-    # conv_p16.hip once per storage type (fp32 tensors with the host entry points, fp16 tensors)
-    units += [("conv_p16.hip", "conv_p16.f32.o", ["-DFYN_P16_HALF=0"]), ("conv_p16.hip", "conv_p16.f16.o", ["-DFYN_P16_HALF=1"])]
+    # these once per storage type (fp32 tensors with the host entry points, fp16 tensors)
+    for name in ("conv_p16", "conv_a16"):
+        units += [(name + ".hip", name + ".f32.o", ["-DFYN_P16_HALF=0"]), (name + ".hip", name + ".f16.o", ["-DFYN_P16_HALF=1"])]
     units += [(src, src + ".o", []) for src in SOURCES]
     for src, objname, defs in units:
         obj = os.path.join(objdir, objname)

@@ -1,0 +1,395 @@
+// The first two layers of a style-transfer net as one launch: a 9x9 convolution of an image (at most four channels, up to 32
+// out) and the 3x3 convolution with a step of two behind it (up to 64 out), on gfx950 matrix cores.
+//
+// Replaces, for such a pair, two render passes of DeepConvLayerNxN::forward (fyusenet/gpu/deep/deepconvlayerNxN.cpp:129-211).
+//
+// Bound: the matrix pipes.  Apart, the layers meet in the largest tensor of the net -- 265 MB at 1920x1080 on fp32 tensors,
+// written and read again in half of their time --, and in the first one every workgroup multiplies and then stores.  Here it
+// stays in LDS (1920x1080, both layers: 212 us apart, 152 here; fp16 tensors 92 and 72): a workgroup walks tiles of 4 rows x 31 positions of the second layer's output and computes the 9 rows x 63
+// positions of the first layer under them (1.16 times its arithmetic; a tile's columns and rows overlap its neighbours' by
+// one), as hi and lo planes with even and odd columns apart, so that the sixteen positions of a fragment of the second layer
+// are neighbours there whatever the tap and a fragment is one contiguous kilobyte.  Four MFMA waves, four staging waves: a
+// wave computes sixteen columns of the first layer with the schedule of the layer's own kernel (c4_rows, its weights in LDS),
+// then 32 channels x 16 columns x 4 rows of the second one, column of taps by column of taps, where the fragment of row j
+// serves every tap that meets it.  The next tile's window is requested while this one is multiplied and replaces it behind
+// the barrier that hands over the tensor in between.
+#include "c4_common.h"
+
+namespace fynhip {
+namespace {
+// The halves of eight values that carry their scale already, as split_pair gives them: packed conversions and subtractions, 26
+// clocks a pair where the four mixed-precision FMAs of split_pair take 33 (each of them issues for eight).
+__device__ __forceinline__ void split_eight(const float (&x)[8], half8_t& hi, half8_t& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        hi[e] = (_Float16)x[e];
+        lo[e] = (_Float16)(x[e] - (float)hi[e]);
+    }
+}
+
+// The first layer's tile, as GeoC4 describes it for conv_p16c4_kernel (rows without the pad behind them: the LDS is full).
+struct GeoA {
+    static constexpr int K = 9, TH = 9, TWG = 64, FN = TH, NS = 12, PIX = 8;
+    static constexpr int HW = TWG + 9, HH = TH + K - 1;
+    static constexpr int ROW_PITCH = (HW + 1) * PIX;
+    static constexpr int COPY = HH * ROW_PITCH, COPY2 = (COPY + 127) / 128 * 128 + 48, PLANE = COPY2 + COPY + 16, BUF = NPL * PLANE;
+    static constexpr int NITEMS = HH * HW, NB = (NITEMS + 255) / 256;
+    // the second layer's: rows and columns of its tile, the tensor in between [row][even columns, odd columns][32 channels]
+    static constexpr int TH2 = 4, TW2 = 31, MROW = 63 * 64, MPLANE = TH * MROW;
+    static constexpr int NW = HSTORE ? 4 : 8;                       // weight fragments of a pair of steps (c4_rows)
+    static constexpr int WEIGHTS = BUF, MID = WEIGHTS + NS / 2 * NW * 1024, SB = MID + NPL * MPLANE, LDS = SB + (32 + 64) * 2 * 4;
+    static_assert(LDS + 16 <= 160 * 1024 && BUF < 65536 && ROW_PITCH % 16 == 0, "fits a CU; 16-byte reads are aligned");
+};
+
+// (KEEP: the tensor in between is written to memory as well, for a net whose tensors all stay readable)
+template <bool HS, bool KEEP>
+__global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
+    using G = GeoA;
+    constexpr bool C8 = !HS;
+    constexpr int FN = G::FN, NW = G::NW;
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ unsigned range_box[2];
+    if (blockIdx.x == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // (neighbouring tiles, whose windows overlap, meet in one XCD's L2)
+    int group = blockIdx.x;
+    {
+        const int per = (int)gridDim.x >> 3;
+        if (group < (per << 3)) group = (group & 7) * per + (group >> 3);
+    }
+    const int ntiles = p.tiles_x * p.tiles_y, step = (int)gridDim.x;
+    if (tid < 2) range_box[tid] = 0u;
+    const unsigned range_bits = p.in_amax ? range_load(p.in_amax) : 0u;
+    float in_scale = 1.f, inv_in = 1.f;
+    if (wave < 4) {   // ---------------------------------------------------------------- staging waves
+        const store_t* in = reinterpret_cast<const store_t*>(p.in);
+        typedef typename std::conditional<HS, half4_t, float4>::type raw_t;   // a pixel as it comes from memory
+        raw_t raw[G::NB];
+        int yx[G::NB], l_off[G::NB];
+        unsigned inside = 0u;   // one bit an item
+#pragma unroll
+        for (int i = 0; i < G::NB; i++) {
+            const int idx = tid + i * 256, py = idx / G::HW, px = idx - py * G::HW;
+            yx[i] = py << 16 | px;
+            l_off[i] = idx < G::NITEMS ? py * G::ROW_PITCH + px * G::PIX : -1;
+        }
+        auto fetch = [&](int tile) {
+            const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
+            // (row 2 y - 1, column 2 x - 1 of the first layer, four pixels further out)
+            const int y0 = tyi * 2 * G::TH2 - 5, x0 = txi * 2 * G::TW2 - 5;
+            inside = 0u;
+#pragma unroll
+            for (int i = 0; i < G::NB; i++) {
+                const int y = y0 + (yx[i] >> 16), x = x0 + (yx[i] & 0xffff);
+                const bool ok = l_off[i] >= 0 && (unsigned)y < (unsigned)p.h && (unsigned)x < (unsigned)p.w;
+                inside |= ok ? 1u << i : 0u;
+                raw[i] = *reinterpret_cast<const raw_t*>(in + (ok ? ((y + p.in_off) * p.in_wp + x + p.in_off) * 4 : 0));
+            }
+        };
+        const bool plain_act = p.act[0].kind == ACT_NONE;   // (a first layer reads its input as it is)
+        auto store = [&]() {
+#pragma unroll
+            for (int i = 0; i < G::NB; i++) {
+                if (l_off[i] < 0) continue;
+                const bool ok = (inside >> i) & 1u;
+                unsigned char* const at = lds + l_off[i];
+                if constexpr (HS) {
+                    half4_t v;
+                    _Float16 hlo, hhi;
+                    if (act_half_exact(p.act[0], hlo, hhi)) {
+                        v = ok ? act_half4(raw[i], hlo, hhi) : (half4_t)((_Float16)0.f);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[e] = ok ? (_Float16)act_p16((float)raw[i][e], p.act[0]) : (_Float16)0.f;
+                    }
+                    *reinterpret_cast<half4_t*>(at) = v;
+                    *reinterpret_cast<half4_t*>(at + G::COPY2 + 8) = v;
+                } else {
+                    const float r[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+                    float x[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[e] = ok ? (plain_act ? r[e] : act_p16(r[e], p.act[0])) : 0.f;
+                    unsigned h0, l0, h1, l1;
+                    split_pair(x[0], x[1], in_scale, h0, l0);
+                    split_pair(x[2], x[3], in_scale, h1, l1);
+                    const half4_t hi = __builtin_bit_cast(half4_t, uint2{h0, h1}), lo = __builtin_bit_cast(half4_t, uint2{l0, l1});
+                    const int2 c8 = int2{(int)c8_quad(lo[0], lo[1], lo[2], lo[3], 0.03125f), (int)c8_quad(hi[0], hi[1], hi[2], hi[3], 64.f)};
+                    *reinterpret_cast<half4_t*>(at) = hi;
+                    *reinterpret_cast<half4_t*>(at + G::COPY2 + 8) = hi;
+                    *reinterpret_cast<int2*>(at + G::PLANE) = c8;
+                    *reinterpret_cast<int2*>(at + G::PLANE + G::COPY2 + 8) = c8;
+                }
+            }
+        };
+        fetch(group);
+        if (p.in_amax) in_scale = range_scale(range_after_act(range_reduce(range_bits), p.act[0]), &inv_in);
+        float* const sb = reinterpret_cast<float*>(lds + G::SB);
+        if (tid < 32) {
+            sb[tid] = tid < p.mid_cp ? p.scale[0][tid] : 0.f;
+            sb[32 + tid] = tid < p.mid_cp ? p.bias[0][tid] : 0.f;
+        } else if (tid >= 64 && tid < 128) {
+            sb[tid] = tid - 64 < p.out_cp ? p.scale[1][tid - 64] : 0.f;
+            sb[64 + tid] = tid - 64 < p.out_cp ? p.bias[1][tid - 64] : 0.f;
+        }
+        store();
+        for (int tile = group;;) {
+            lds_barrier();   // the window is staged
+            tile += step;
+            if (tile < ntiles) fetch(tile);
+            lds_barrier();   // the first layer is through: the window's place is free
+            if (tile >= ntiles) return;
+            store();
+        }
+    }
+    // ------------------------------------------------------------------------------------ MFMA waves
+    const int mq = lane & 15, kq = lane >> 4, w = wave - 4;
+    const unsigned wlane = lane * 16;
+    __builtin_amdgcn_s_setprio(2);   // (the staging wave on this SIMD has time enough in between)
+    {   // the first layer's weights into LDS, as c4_rows takes them: [pair of steps][fragment][lane]
+        constexpr int SHARE = G::NS / 2 * NW / 4;
+        i32x4_t v[SHARE];
+#pragma unroll
+        for (int i = 0; i < SHARE; i++) {
+            const int c = w * SHARE + i, k = c % NW, st = c / NW * 2 + (k / 2) % 2, fm = k % 2, plane = k < 4 ? 0 : 2;
+            v[i] = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const unsigned char*>(p.wpack[0]) + (size_t)((st * p.mfrags0 + fm) * NPLW + plane) * 1024 + wlane);
+        }
+#pragma unroll
+        for (int i = 0; i < SHARE; i++) *reinterpret_cast<i32x4_t*>(lds + G::WEIGHTS + (w * SHARE + i) * 1024 + wlane) = v[i];
+    }
+    float mid_scale = 1.f, inv_mid = 1.f;
+    if (p.in_amax) {
+        const float r0 = range_after_act(range_reduce(range_bits), p.act[0]);
+        (void)range_scale(r0, &inv_in);
+        // (no value of the first layer is larger than its weights' largest row sum allows: a scale for the tensor in between that
+        // does not wait for it.  Such a bound is some ten times what a frame reaches, 2^4 of the 2^14 that the split has to spare)
+        if constexpr (C8) mid_scale = range_scale(range_after_act(r0 * p.gain + p.base, p.act[1]), &inv_mid);
+    }
+    const float mul1 = p.acc_mul[0] * inv_in, mul2 = p.acc_mul[1] * inv_mid;
+    // this lane's places: in the window, in the tensor in between (as it writes and as it reads)
+    const int x1 = w * 16 + mq;   // column of the first layer's tile
+    const unsigned char* const col = lds + x1 * G::PIX + ((x1 & 1) ? G::COPY2 + 8 : 0);
+    const unsigned char* const rows_at = col + 2 * kq * G::PIX;
+    const unsigned char* const ninth_at = col + kq * G::ROW_PITCH + 8 * G::PIX;
+    const unsigned char* const last_at = col + 8 * G::ROW_PITCH + 8 * G::PIX;
+    unsigned char* const mid_to = lds + G::MID + ((x1 & 1) ? 32 + (x1 >> 1) : x1 >> 1) * 64 + kq * 16;   // (its eight channels side by side; the second layer's weights are laid out for that)
+    const int cpair = w & 1, cfrag = w >> 1;   // of the second layer: 32 channels, 16 columns
+    const unsigned char* const mid_at = lds + G::MID + (cfrag * 16 + mq) * 64 + kq * 16;
+    // (buffer loads: the fragment's place is a scalar operand, where 64-bit addresses of all of them would fill the registers)
+    const __amdgpu_buffer_rsrc_t weights2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.wpack[1]), 0, 36 * NPL * 1024, 0x00020000);   // [kx][32 channels][ky][fragment][plane]
+    const float* const sb = reinterpret_cast<const float*>(lds + G::SB);
+    store_t* const out = reinterpret_cast<store_t*>(p.out);
+    const bool through = store_through_pays(p.out, p.h2, p.w2, p.out_cp * ESZ, !p.plain_stores, hw_block_count());
+    bool drop = through && wave == 4 && hw_block_id() < 8;
+    const float lo1 = p.act[1].kind == ACT_NONE ? -3.0e38f : p.act[1].kind == ACT_RELU ? 0.f : p.act[1].lo * mid_scale;   // (its values carry the scale)
+    const float hi1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 3.0e38f : p.act[1].hi * mid_scale;
+    const float leak1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 0.f : p.act[1].leak;
+    _Float16 hlo1, hhi1;
+    const bool packed1 = act_half_exact(p.act[1], hlo1, hhi1);
+    C4Ring<G> ring;
+    constexpr int LA = C4Ring<G>::LA;
+    lds_barrier();   // the first window is staged, the weights are there
+#pragma unroll
+    for (int d = 0; d < C4Ring<G>::LW; d++)
+#pragma unroll
+        for (int k = 0; k < NW; k++) rows_put_w(ring.a0[d], ring.a2[d], k, *reinterpret_cast<const i32x4_t*>(lds + G::WEIGHTS + (d * NW + k) * 1024 + wlane));
+    float vmax = 0.f;
+    for (int tile = group;;) {
+        const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
+        half8_t wq[2][3][2][NPL];   // the second layer's weights of a column of taps, two columns
+        typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+        auto load_w = [&](int set, int kx) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ky = 0; ky < 3; ky++)
+#pragma unroll
+                for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                    for (int pl = 0; pl < NPL; pl++)
+                        wq[set][ky][fm][pl] = __builtin_bit_cast(half8_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights2, wlane, (unsigned)(((kx * 2 + cpair) * 6 + ky * 2 + fm) * NPL + pl) * 1024u, 0));
+        };
+        {   // ---- first layer ----
+            f32x4_t acc[2][FN];
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                for (int fn = 0; fn < FN; fn++) acc[fm][fn] = (f32x4_t)(0.f);
+#pragma unroll
+            for (int r = 0; r <= LA; r++) ring.b0[r] = *reinterpret_cast<const half8_t*>(rows_at + r * G::ROW_PITCH);
+            if constexpr (C8) {
+#pragma unroll
+                for (int r = 0; r < LA; r++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) rows_load_b8<G>(ring.b8[r], h, rows_at + (r + h) * G::ROW_PITCH + G::PLANE);
+            }
+            c4_rows<G, false>(acc, ring, rows_at, ninth_at, last_at, rows_at, lds + G::WEIGHTS + wlane);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4_t scm[2], bi[2];
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++) {
+                scm[fm] = *reinterpret_cast<const f32x4_t*>(sb + kq * CHK + fm * CHF) * (mul1 * mid_scale);
+                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 32 + kq * CHK + fm * CHF) * mid_scale;
+            }
+            const int px = txi * 2 * G::TW2 - 1 + x1;
+            const bool x_ok = (unsigned)px < (unsigned)p.w;
+            auto leave = [&](auto general_, auto first_, auto end_) __attribute__((always_inline)) {   // (general: an activation other than none, a clamp exact on halves, or a clamp)
+                constexpr bool GENERAL = decltype(general_)::value;
+#pragma unroll
+                for (int r = decltype(first_)::value; r < decltype(end_)::value; r++) {
+                    // (positions outside the layer's output are its zero padding)
+                    const bool ok = x_ok && (unsigned)(tyi * 2 * G::TH2 - 1 + r) < (unsigned)p.h;
+                    unsigned char* const to = mid_to + r * G::MROW;
+                    // (a tile's first row and column are its neighbours' to write)
+                    const bool own = KEEP && ok && r > 0 && x1 > 0;
+                    store_t* const kept = reinterpret_cast<store_t*>(p.mid) + ((size_t)(p.mid_off + tyi * 2 * G::TH2 - 1 + r) * p.mid_wp + p.mid_off + px) * p.mid_cp + kq * CHK;
+                    if constexpr (HS) {
+                        half8_t v;
+#pragma unroll
+                        for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) v[fm * 4 + e] = (_Float16)(acc[fm][r][e] * scm[fm][e] + bi[fm][e]);   // (as the layer would have stored it)
+                        if constexpr (KEEP) {
+                            if (own && kq * CHK < p.mid_cp) *reinterpret_cast<half8_t*>(kept) = v;
+                        }
+                        if constexpr (!GENERAL) {
+                            v = act_half(v, hlo1, hhi1);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 8; e++) v[e] = (_Float16)act_p16((float)v[e], p.act[1]);
+                        }
+                        *reinterpret_cast<half8_t*>(to) = ok ? v : (half8_t)((_Float16)0.f);
+                    } else {
+                        const float lo = ok ? lo1 : 0.f, hi = ok ? hi1 : 0.f, leak = ok ? leak1 : 0.f;
+                        float x[8];
+                        if constexpr (KEEP) {
+#pragma unroll
+                            for (int fm = 0; fm < 2; fm++)
+                                if (own && kq * CHK + fm * CHF < p.mid_cp) *reinterpret_cast<f32x4_t*>(kept + fm * CHF) = (acc[fm][r] * scm[fm] + bi[fm]) * inv_mid;
+                        }
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            const float v = acc[i / 4][r][i % 4] * scm[i / 4][i % 4] + bi[i / 4][i % 4];
+                            x[i] = __builtin_amdgcn_fmed3f(v, lo, hi);
+                            if constexpr (GENERAL) x[i] += leak * fminf(v, 0.f);
+                        }
+                        half8_t H, L;
+                        split_eight(x, H, L);
+                        *reinterpret_cast<half8_t*>(to) = H;
+                        *reinterpret_cast<half8_t*>(to + G::MPLANE) = L;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            auto rows = [&](auto first, auto end) __attribute__((always_inline)) {
+                if (x1 < 63) {   // (the 64th column belongs to nobody)
+                    if (HS ? !packed1 : leak1 != 0.f) leave(std::integral_constant<bool, true>(), first, end);
+                    else leave(std::integral_constant<bool, false>(), first, end);
+                }
+            };
+            constexpr int FIRST = 5;
+            rows(std::integral_constant<int, 0>(), std::integral_constant<int, FIRST>());
+            load_w(0, 0);   // (the second layer's first weights, into registers that the rows so far have left)
+            rows(std::integral_constant<int, FIRST>(), std::integral_constant<int, FN>());
+        }
+        lds_barrier();   // the tensor in between is there
+        {   // ---- second layer: rows 2 r + ky, columns 2 c + kx ----
+            f32x4_t acc[2][G::TH2];
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                for (int r = 0; r < G::TH2; r++) acc[fm][r] = (f32x4_t)(0.f);
+            constexpr int AHEAD = 3, Q = 3 * FN;
+            half8_t b[AHEAD + 1][NPL];
+            auto request = [&](int q) __attribute__((always_inline)) {
+                const int kx = q / FN, j = q % FN;
+#pragma unroll
+                for (int pl = 0; pl < NPL; pl++)
+                    b[q % (AHEAD + 1)][pl] = *reinterpret_cast<const half8_t*>(mid_at + (kx == 1 ? 32 * 64 : kx * 32) + j * G::MROW + pl * G::MPLANE);
+            };
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) request(q);
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                const int kx = q / FN, j = q % FN;
+                if (j == 0 && kx + 1 < 3) load_w((kx + 1) & 1, kx + 1);
+                if (q + AHEAD < Q) request(q + AHEAD);
+#pragma unroll
+                for (int i = 0; i < NPASS; i++)
+#pragma unroll
+                    for (int ky = 0; ky < 3; ky++) {
+                        if (((j - ky) & 1) || j < ky || (j - ky) / 2 >= G::TH2) continue;
+#pragma unroll
+                        for (int fm = 0; fm < 2; fm++)
+                            acc[fm][(j - ky) / 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wq[kx & 1][ky][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][(j - ky) / 2], 0, 0, 0);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (drop) {   // (ahead of this workgroup's first store: what it has read so far may go as well)
+                drop_clean_l2_lines();
+                drop = false;
+            }
+            f32x4_t sc[2], bi[2];
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++) {
+                sc[fm] = *reinterpret_cast<const f32x4_t*>(sb + 64 + cpair * 32 + kq * CHK + fm * CHF) * mul2;
+                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 128 + cpair * 32 + kq * CHK + fm * CHF);
+            }
+            const int c2 = cfrag * 16 + mq, ox = txi * G::TW2 + c2, ch0 = cpair * 32 + kq * CHK;
+#pragma unroll
+            for (int r = 0; r < G::TH2; r++) {
+                const int oy = tyi * G::TH2 + r;
+                const bool inside = c2 < G::TW2 && ox < p.w2 && oy < p.h2;
+                const size_t at = ((size_t)(p.out_off + oy) * p.out_wp + p.out_off + ox) * p.out_cp + ch0;
+                half8_t hv;
+#pragma unroll
+                for (int fm = 0; fm < 2; fm++) {
+                    const bool ok = inside && ch0 + (HS ? 0 : fm * CHF) < p.out_cp;
+                    f32x4_t v;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        v[e] = acc[fm][r][e] * sc[fm][e] + bi[fm][e];
+                        if constexpr (!HS) vmax = fmaxf(vmax, ok ? fabsf(v[e]) : 0.f);
+                        else hv[fm * 4 + e] = (_Float16)v[e];
+                    }
+                    if constexpr (HS) {
+                        if (fm == 1 && ok) store_out(through, reinterpret_cast<half8_t*>(out + at), hv);
+                    } else {
+                        if (ok) store_out(through, reinterpret_cast<f32x4_t*>(out + at + fm * CHF), v);
+                    }
+                }
+            }
+        }
+        tile += step;
+        if (tile >= ntiles) break;
+        lds_barrier();   // the next window is staged, and nobody reads the tensor in between any more
+    }
+    if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 4);
+}
+}  // namespace
+
+#if FYN_P16_HALF
+#define A16_NAME(n) n##_half
+#else
+#define A16_NAME(n) n
+int launch_conv_a16_half(const ConvA16Params& p, hipStream_t s);
+size_t conv_a16_lds_bytes(bool f16) { return (f16 ? 1 : 2) * (size_t)(GeoA::PLANE + GeoA::MPLANE) + (f16 ? 24 : 48) * 1024 + (32 + 64) * 2 * 4; }
+void conv_a16_tile(int* rows, int* cols) { *rows = GeoA::TH2; *cols = GeoA::TW2; }
+#endif
+int A16_NAME(launch_conv_a16)(const ConvA16Params& p, hipStream_t s) {
+#if !FYN_P16_HALF
+    if (p.f16) return launch_conv_a16_half(p, s);
+#endif
+    const long long tiles = (long long)p.tiles_x * p.tiles_y;
+    const int rows = p.mid ? (p.h + 2 * GeoA::TH2 - 1) / (2 * GeoA::TH2) : (p.h2 + GeoA::TH2 - 1) / GeoA::TH2;
+    const int cols = p.mid ? (p.w + 2 * GeoA::TW2 - 1) / (2 * GeoA::TW2) : (p.w2 + GeoA::TW2 - 1) / GeoA::TW2;
+    if ((p.f16 != 0) != HSTORE || !p.in || !p.out || !p.wpack[0] || !p.wpack[1] || (!HSTORE && !p.in_amax) || p.h < 2 || p.w < 2 || p.h2 != p.h / 2 || p.w2 != p.w / 2 || p.in_off < 0 ||
+        p.h + p.in_off > p.in_hp || p.w + p.in_off > p.in_wp || (long long)p.in_hp * p.in_wp * 4 > (1ll << 30) || p.mid_cp < 1 || p.mid_cp > 32 || p.mfrags0 < 2 || p.out_cp < 8 || p.out_cp > 64 ||
+        p.out_cp % 8 != 0 || p.tiles_x != cols || p.tiles_y != rows || tiles > 4000000 || p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.groups < 1 || p.groups > tiles || p.nreset < 0 || p.nreset > 4 ||
+        (p.mid && (p.mid_cp % (HSTORE ? 8 : 4) != 0 || p.mid_off < 0 || p.mid_wp < p.w + p.mid_off)))
+        return -5;
+    const auto kernel = p.mid ? conv_a16_kernel<HSTORE, true> : conv_a16_kernel<HSTORE, false>;
+    if (ensure_lds(reinterpret_cast<const void*>(kernel), GeoA::LDS) != 0) return -2;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)p.groups), dim3(512), GeoA::LDS, s, p);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+}  // namespace fynhip

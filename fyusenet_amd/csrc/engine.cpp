@@ -474,6 +474,7 @@ void Net::setup() {
     fuse_batchnorm_layers(this);
     fuse_block_layers(this);
     fuse_pair_layers(this);
+    fuse_head_layers(this);
     fuse_function_layers(this);
     fuse_concat_layers(this);
     fuse_argmax_layers(this);

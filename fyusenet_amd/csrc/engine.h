@@ -153,6 +153,8 @@ class Net {
     // Layers fused into their neighbour's launch (fuse_depthwise_layers) run that way only in passes that neither time
     // nor dump single layers, and only in networks whose intermediate tensors may share buffers.
     bool fusion_on() const { return reuse_buffers && !timings && dump_dir.empty(); }
+    // ... those that write the tensors in between where buffers aren't shared (the blocks and pairs that don't are not formed there)
+    bool joined_on() const { return !timings && dump_dir.empty(); }
     std::string dump_dir;
     hipStream_t stream = nullptr;
     std::map<int, std::unique_ptr<Layer>> layers;  // ascending number = execution order
@@ -258,6 +260,7 @@ void fuse_projection_layers(Net* net);   // after every layer's setup(): 1x1 sho
 std::vector<std::pair<int, int>> keep_block_inputs(Net* net);   // ... and, while they are assigned, inputs of bottlenecks until their last layer, which may compute them, has run; (tensor, its last reader)
 void fuse_block_layers(Net* net);        // after the other passes on convolutions: a 1x1, a 3x3 and a 1x1 layer in one launch
 void fuse_pair_layers(Net* net);         // ... two 3x3 layers between tensors of few channels in one launch
+void fuse_head_layers(Net* net);         // ... a 9x9 layer on an image and the 3x3 layer with a step of two behind it
 void fuse_depthwise_layers(Net* net);   // after every layer's setup(): depthwise 3x3 layers that their 1x1 reader can compute itself
 void fuse_function_layers(Net* net);   // after every layer's setup(): sigmoid / tanh layers that the row-rolling convolution in front of them can apply to what it stores
 void fuse_concat_layers(Net* net);   // after every layer's setup(): bilinear scale layers in front of concatenations and batch-norm layers behind them

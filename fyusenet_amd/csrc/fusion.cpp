@@ -364,6 +364,14 @@ static bool pair_of(Net* net, const ConvLayer* c, ConvLayer*& a) {
     a = alone_in_front(net, c);
     return plain_conv(a, 3) && a->clamp == c->clamp && a->oh == c->oh && a->ow == c->ow;
 }
+// The 9x9 layer `a` on an image that `c`, a 3x3 layer with a step of two, alone reads.
+static bool head_of(Net* net, const ConvLayer* c, ConvLayer*& a) {
+    if (!c || c->k != 3 || c->stride != 2 || c->dil != 1 || c->clamp || c->frac_shift || c->direct || c->wide || (c->d.flags & FYN_FLAG_RESIDUAL_INPUT)) return false;
+    a = alone_in_front(net, c);
+    if (!plain_conv(a, 9) || a->clamp || a->oc > 32 || c->oc > 64 || a->d.in_channels > 4) return false;
+    const int from = net->tensors[a->in[0]].producer;   // (a frame from the host or the application: its value-range word is never lost)
+    return from < 0 || net->layer(from)->d.type == FYN_LAYER_UPLOAD;
+}
 // While buffers are assigned, the input of such a block or pair is read until its last layer has run, which may compute all of
 // it (the tensors' last readers as they were: whether the layers are joined is not known yet).
 std::vector<std::pair<int, int>> keep_block_inputs(Net* net) {
@@ -375,6 +383,7 @@ std::vector<std::pair<int, int>> keep_block_inputs(Net* net) {
     };
     for (auto& kv : net->layers) {
         ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
+        if (c && !net->sw.get("FYNHIP_NO_HEAD_FUSION") && head_of(net, c, a)) keep(a->in[0], c->d.number);
         if (c && !net->sw.get("FYNHIP_NO_PAIR_FUSION") && pair_of(net, c, a) && a->d.in_channels <= 64) keep(a->in[0], c->d.number);
         if (!c || net->sw.get("FYNHIP_NO_BLOCK_FUSION") || !block_of(net, c, a, b)) continue;
         keep(a->in[0], c->d.number);
@@ -509,6 +518,90 @@ void fuse_block_layers(Net* net) {
         for (ConvLayer* l : front) l->blk_into = c->d.number;
         net->read_until(x, c->d.number);   // (its value-range word is cleared behind its last reader)
         c->pack_block();
+    }
+}
+
+// The first two layers of a style-transfer net (conv_a16.hip) as one launch in the place of the second, timed against their own
+// launches (us, 3 to 32 to 64 channels, one launch / apart): fp32 tensors 384x384 22 / 21, 512x624 32 / 39, 1920x1080 152 / 212;
+// fp16 256x256 7.8 / 9.3, 512x624 16 / 23, 1920x1080 72 / 92.  Untimed it is taken wherever the first layer is in its form on
+// rows of sixteen positions: a tie at the smallest such size, ahead above.
+void fuse_head_layers(Net* net) {
+    if (net->sw.get("FYNHIP_NO_HEAD_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV")) return;
+    const bool forced = net->sw.get("FYNHIP_FORCE_HEAD_FUSION") != nullptr;
+    if (!forced && single_form_forced(net)) return;
+    const char* at = net->sw.get("FYNHIP_AUTOTUNE");
+    for (auto& kv : net->layers) {
+        ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr;
+        if (!head_of(net, c, a) || a->blk_into >= 0 || c->blk_into >= 0 || c->fn_layer_no >= 0) continue;
+        const TView &iv = a->tin(0).v, &mv = a->tout().v, &ov = c->tout().v;
+        if (iv.f16 != ov.f16 || mv.f16 != ov.f16 || iv.cp != 4 || mv.cp > 32 || mv.cp % (mv.f16 ? 8 : 4) != 0 || ov.cp > 64 || ov.cp % 8 != 0 || a->d.in_channels > iv.cp || c->d.in_channels != a->oc || a->oh < 2 || a->ow < 2 || c->oh != a->oh / 2 ||
+            c->ow != a->ow / 2)
+            continue;
+        // (the form whose weights and schedule the launch takes for the first layer; with fp32 tensors its fp8 correction terms too)
+        if (!a->p16 || !a->c4 || a->pp.tile_w != 16 || (!iv.f16 && (!a->tin(0).amax || !conv_p16c4_uses_fp8(a->pp, 9)))) continue;
+        // (positions beside a layer's input are zeros behind its activation as well)
+        if (a->act().lo > 0.f || a->act().hi < 0.f || c->act().lo > 0.f || c->act().hi < 0.f) continue;
+        const int x = a->in[0];
+        if (!net->alone(x, a->d.number, c->d.number) || !words_survive(net, {a}, c->d.number, x)) continue;
+        ConvA16Params q{};
+        q.in = iv.ptr; q.in_hp = iv.hp(); q.in_wp = iv.wp(); q.in_off = iv.pad;
+        q.in_amax = a->tin(0).amax;
+        q.wpack[0] = a->p16_wpack_dev; q.mfrags0 = a->pp.mfrags;
+        q.h = a->oh; q.w = a->ow; q.h2 = c->oh; q.w2 = c->ow;
+        int rows, cols;
+        conv_a16_tile(&rows, &cols);
+        q.tiles_x = (q.w2 + cols - 1) / cols; q.tiles_y = (q.h2 + rows - 1) / rows;
+        q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
+        q.groups = std::min(q.tiles_x * q.tiles_y, 256);   // (one workgroup per CU)
+        const ConvLayer* L[2] = {a, c};
+        for (int i = 0; i < 2; i++) {
+            q.scale[i] = L[i]->scale_dev; q.bias[i] = L[i]->bias_dev;
+            q.acc_mul[i] = 1.f;
+            q.act[i] = L[i]->act();
+        }
+        q.mid_cp = mv.cp;
+        q.out = ov.ptr; q.out_cp = ov.cp; q.out_wp = ov.wp(); q.out_off = ov.pad;
+        q.plain_stores = net->sw.get("FYNHIP_PLAIN_STORES") ? 1 : 0;
+        q.f16 = ov.f16 ? 1 : 0;
+        void* const wp = net->dev_alloc((size_t)36 * (q.f16 ? 1 : 2) * 1024, true);
+        q.wpack[1] = wp;
+        bool pick = true;
+        char key[200];
+        snprintf(key, sizeof(key), "head:%d:%dto%dto%d:%dx%d", q.f16, a->d.in_channels, a->oc, c->oc, a->oh, a->ow);
+        if (forced || tune_cache_flag(net, key, &pick)) {
+        } else if (!(at && at[0] == '0')) {
+            float t_one = 1e30f, t_apart = 1e30f;
+            for (int rep = 0; rep < 3; rep++) {
+                t_one = std::min(t_one, time_calls(net, [&]() {
+                    if (launch_conv_a16(q, net->stream) != 0) fail(FYN_ERR_DEVICE, "launch of a 9x9 and a 3x3 layer failed while tuning");
+                }, 10));
+                t_apart = std::min(t_apart, time_calls(net, [&]() {
+                    a->forward_alone(net->stream);
+                    c->forward_alone(net->stream);
+                }, 10));
+            }
+            if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
+                fprintf(stderr, "[tune] 9x9 %d to %d and 3x3 to %d with a step of two at %dx%d: one launch %.1f us, apart %.1f us\n", a->d.in_channels, a->oc, c->oc, a->oh, a->ow, t_one * 1e3f, t_apart * 1e3f);
+            pick = t_one < t_apart;
+            tune_cache_store_flag(net, key, pick);
+        }
+        if (!pick) {
+            net->dev_free(wp);
+            continue;
+        }
+        if (!net->reuse_buffers) {   // (every tensor stays readable: the launch writes the one in between as well)
+            q.mid = mv.ptr; q.mid_wp = mv.wp(); q.mid_off = mv.pad;
+            q.tiles_x = (q.w + 2 * cols - 1) / (2 * cols); q.tiles_y = (q.h + 2 * rows - 1) / (2 * rows);
+            q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
+            q.groups = std::min(q.tiles_x * q.tiles_y, 256);
+        }
+        c->head = q;
+        c->head_wpack_dev = wp;
+        c->head_fused = true;
+        c->head_layer = a->d.number;
+        a->blk_into = c->d.number;
+        net->read_until(x, c->d.number);
+        c->pack_head();
     }
 }
 

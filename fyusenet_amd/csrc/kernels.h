@@ -377,6 +377,34 @@ struct ConvB16Params {
 size_t conv_b16_weight_frags(const ConvB16Params& p);   // fragments in wpack; 0: no such compiled combination
 size_t conv_b16_lds_bytes(const ConvB16Params& p);
 int launch_conv_b16(const ConvB16Params& p, hipStream_t s);
+// A 9x9 layer on an input of at most four channels (conv_p16c4's weights, tiles of rows) and the 3x3 layer with a step of two
+// behind it as one launch (conv_a16.hip): h x w positions of the first, h2 x w2 of the second.
+struct ConvA16Params {
+    const void* in;
+    const unsigned* in_amax;
+    const void* wpack[2];   // launch_conv_p16c4's; [kx][32 output channels][ky][fragment][plane hi, lo][lane][8 halves] (ConvLayer::pack_head)
+    int mfrags0;            // fragments of a step in wpack[0]
+    int h, w, h2, w2;
+    int in_wp, in_off, in_hp;   // stored input frame, four channels a pixel; position (y, x) is pixel (y + in_off, x + in_off)
+    int tiles_x, tiles_y, groups;   // tiles of conv_a16_tile; workgroups that walk them
+    float rcp_tiles_x;      // 1.0f / tiles_x
+    const float* scale[2];
+    const float* bias[2];
+    int mid_cp, out_cp, out_wp, out_off;
+    float acc_mul[2];
+    float gain, base;       // fp32 tensors: no value of the first layer exceeds gain * (largest input) + base
+    void* mid;              // not null: the tensor in between is written as well (tiles then cover all of it)
+    int mid_wp, mid_off;
+    Act act[2];             // on the fetch of each layer's input
+    void* out;
+    unsigned* out_amax;
+    unsigned* reset[4];
+    int nreset;
+    int plain_stores, f16;
+};
+void conv_a16_tile(int* rows, int* cols);   // of the second layer's output
+size_t conv_a16_lds_bytes(bool f16);
+int launch_conv_a16(const ConvA16Params& p, hipStream_t s);
 // Two 3x3 layers between tensors of few channels, one behind the other, as one launch (conv_c16.hip): h x w positions, th rows of
 // sixteen per workgroup.
 struct ConvC16Params {

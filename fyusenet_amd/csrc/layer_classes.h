@@ -1366,10 +1366,12 @@ class ConvLayer : public Layer {
         if (pj_into >= 0) static_cast<ConvLayer*>(net->layer(pj_into))->pack_two_sources();
         if (blk_fused) pack_block();
         if (pair_fused) pack_pair();
+        if (head_fused) pack_head();
         if (blk_into >= 0) {
             ConvLayer* c = static_cast<ConvLayer*>(net->layer(blk_into));
             if (c->blk_fused) c->pack_block();
             if (c->pair_fused) c->pack_pair();
+            if (c->head_fused) c->pack_head();
         }
     }
     // the weights once more, in the layout of the launch that also runs the depthwise layer behind this one
@@ -1382,7 +1384,11 @@ class ConvLayer : public Layer {
     }
     void forward(hipStream_t s) override {
         if (!have_weights) fail(FYN_ERR_STATE, "layer %s (%d): forward() without weights", d.name, d.number);
-        if (blk_into >= 0 && net->fusion_on()) return;   // computed in the launch of the block's or the pair's last layer
+        if (blk_into >= 0 && net->joined_on()) return;   // computed in the launch of the block's or the pair's last layer
+        if (head_fused && net->joined_on()) {
+            if (launch_conv_a16(with_head(), s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
+            return;
+        }
         if (pair_fused && net->fusion_on()) {
             if (launch_conv_c16(with_pair(), s) != 0) fail(FYN_ERR_DEVICE, "layer %s: convolution launch failed", d.name);
             return;
@@ -1449,6 +1455,15 @@ class ConvLayer : public Layer {
     }
     std::string info() const override {
         if (blk_into >= 0) return "conv " + std::to_string(k) + "x" + std::to_string(k) + " (runs inside the launch of layer " + std::to_string(blk_into) + "; no launch of its own); apart: " + own_info();
+        if (head_fused) {
+            char buf[300];
+            int rows, cols;
+            conv_a16_tile(&rows, &cols);
+            snprintf(buf, sizeof(buf), "conv_a16 %s layer %d (9x9) and this one (3x3, step 2) in one launch, tiles of %dx%d positions, blocks=%d tiles=%d lds=%zu%s; apart: ", head.f16 ? "f16" : "f16+fp8-split, f16x2-split",
+                     head_layer, rows, cols, head.groups, head.tiles_x * head.tiles_y, conv_a16_lds_bytes(head.f16 != 0),
+                     store_through_pays(head.out, head.h2, head.w2, head.out_cp * (head.f16 ? 2 : 4), !head.plain_stores, (size_t)head.groups) ? " stores=through" : "");
+            return buf + own_info();
+        }
         if (pair_fused) {
             char buf[300];
             snprintf(buf, sizeof(buf), "conv_c16 %s layer %d (3x3) and this one in one launch, %dx16 positions per workgroup, blocks=%d lds=%zu; apart: ", pair.f16 ? "f16" : "f16x2-split", pair_layer, pair.th,
@@ -1677,6 +1692,59 @@ class ConvLayer : public Layer {
         FYN_HIP(hipStreamSynchronize(net->stream));
         FYN_HIP(hipMemcpyAsync(pj_wpack_dev, pack.data(), pack.size() * 2, hipMemcpyHostToDevice, net->stream));
         FYN_HIP(hipStreamSynchronize(net->stream));
+    }
+    // The 9x9 layer on an image in front of this 3x3 layer with a step of two in the same launch (conv_a16.hip; fuse_head_layers below)
+    bool head_fused = false;
+    int head_layer = -1;
+    ConvA16Params head{};
+    void* head_wpack_dev = nullptr;
+    ConvA16Params with_head() const {
+        const ConvLayer* a = static_cast<const ConvLayer*>(net->layer(head_layer));
+        ConvA16Params q = head;   // (value-range words as the layers' own launches carry them; the first layer's weights are its own)
+        q.in_amax = a->tin(0).amax;
+        q.acc_mul[0] = a->pp.acc_mul;
+        q.out_amax = tout().amax;
+        q.nreset = own_resets(q.reset);
+        return q;
+    }
+    // weights of that form: [kx][32 output channels][ky][cout fragment][plane][lane][8 halves]; and what the first layer's
+    // values are bounded by: gain * (largest input) + base
+    void pack_head() {
+        const ConvLayer* a = static_cast<const ConvLayer*>(net->layer(head_layer));
+        if (block.empty() || a->block.empty()) return;
+        const float *b1 = a->block.data(), *w1 = b1 + a->oc;
+        const size_t row = (size_t)81 * a->d.in_channels;
+        std::vector<float> sc, bi;
+        fold_bn(b1, w1 + row * a->oc, a->oc, (a->d.flags & FYN_FLAG_POST_BATCHNORM) != 0, a->oc, sc, bi);
+        head.gain = head.base = 0.f;
+        for (int o = 0; o < a->oc; o++) {
+            double sum = 0.;
+            for (size_t i = 0; i < row; i++) sum += std::fabs(w1[o * row + i]);
+            head.gain = std::max(head.gain, (float)(sum * std::fabs(sc[o]) * 1.001));   // (and the sums' own rounding)
+            head.base = std::max(head.base, std::fabs(bi[o]) * 1.001f);
+        }
+        const float* w = block.data() + oc;
+        const int cin = d.in_channels, npl = head.f16 ? 1 : 2;
+        const float wmul = weight_prescale(w, (size_t)oc * 9 * cin);
+        head.acc_mul[1] = 1.0f / wmul;
+        std::vector<uint16_t> pack((size_t)36 * npl * 64 * 8, 0);
+        uint16_t* base = pack.data();
+        for (int kx = 0; kx < 3; kx++)
+            for (int half = 0; half < 2; half++)
+                for (int ky = 0; ky < 3; ky++)
+                    for (int fm = 0; fm < 2; fm++, base += (size_t)npl * 64 * 8)
+                        for (int lane = 0; lane < 64; lane++) {
+                            const int o = p16_row_channel(2 * half + fm, lane & 15, head.f16 ? 2 : 1);
+                            for (int j = 0; o < oc && j < 8; j++) {
+                                const int ci = head.f16 ? 8 * (lane >> 4) + j : 4 * (lane >> 4) + j / 4 * 16 + j % 4;   // (the channels that a lane of the first layer holds, side by side)
+                                if (ci >= cin) continue;
+                                const float v = w[(((size_t)o * 3 + ky) * 3 + kx) * cin + ci] * wmul;
+                                const uint16_t hi = f2h_bits(v);
+                                base[(size_t)lane * 8 + j] = hi;
+                                if (npl == 2) base[(size_t)(64 + lane) * 8 + j] = f2h_bits(v - h2f(hi));
+                            }
+                        }
+        reupload(net, static_cast<uint16_t*>(head_wpack_dev), pack);
     }
     // The 3x3 layer in front of this 3x3 layer in the same launch, one of conv_c16_kernel (conv_c16.hip; fuse_pair_layers below)
     bool pair_fused = false;
