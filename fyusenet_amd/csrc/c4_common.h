@@ -79,7 +79,7 @@ struct GeoC4 {
     static constexpr int NPOS = TH * TW, FN = NPOS / 16;
     static constexpr int NITEMS = HH * HW;                            // staging items: pixels
     static constexpr int NB = (NITEMS + 255) / 256;
-    static constexpr int CPB = 32;
+    static constexpr int CPB = 32, FM = 2;                            // output channels, fragments of them
     // tiles whose fragments are rows of sixteen positions take the tap pairs in another order: c4_rows
     static constexpr bool ROWS = TW == 16;
     static_assert(!ROWS || K == 9, "rows: eight taps of a kernel row and one more");
@@ -206,7 +206,8 @@ __device__ __forceinline__ void c4_stager(const ConvP16Params& p, unsigned char*
 // fp16 78 -> 65 (68).  Bound there: the stores (265 MB in 102 us beside 33 read).
 template <class G>
 struct C4Ring {
-    static constexpr int LA = HSTORE ? 4 : 2;          // slots (64 or 128 matrix-pipe cycles) from an LDS read to its use
+    // slots (64 or 128 matrix-pipe cycles; half of them with one fragment of output channels) from an LDS read to its use
+    static constexpr int LA = (HSTORE ? 4 : 2) * (G::FM == 1 ? 2 : 1);
     static constexpr int LW = 1;                       // pairs of steps from the request of weights to their use
     half8_t a0[LW][2][2];
     i32x8_t a2[LW][2];
@@ -215,7 +216,7 @@ struct C4Ring {
 };
 // (NEXT: false where the next tile is staged only when this one is through: its operands are not requested here)
 template <class G, bool NEXT = true>
-__device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& ring, const unsigned char* at_rows, const unsigned char* at_ninth,
+__device__ __forceinline__ void c4_rows(f32x4_t (&acc)[G::FM][G::FN], C4Ring<G>& ring, const unsigned char* at_rows, const unsigned char* at_ninth,
                                         const unsigned char* at_last, const unsigned char* next_rows, const unsigned char* weights) {
     constexpr int TH = G::FN, LA = C4Ring<G>::LA, LW = C4Ring<G>::LW, NP = 6, RP = G::ROW_PITCH;
     constexpr bool C8 = !HSTORE;
@@ -225,7 +226,7 @@ __device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& rin
 #pragma unroll
     for (int d = 0; d < LW; d++)
 #pragma unroll
-        for (int fm = 0; fm < 2; fm++) {
+        for (int fm = 0; fm < G::FM; fm++) {
             a0[d][0][fm] = ring.a0[d][0][fm]; a0[d][1][fm] = ring.a0[d][1][fm];
             if constexpr (C8) a2[d][fm] = ring.a2[d][fm];
         }
@@ -268,7 +269,8 @@ __device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& rin
         auto issue = [&](auto index_m) __attribute__((always_inline)) {
             constexpr int m = decltype(index_m)::value, fm = m % 2;
             if constexpr (!(HSTORE && (m == 2 || m == 3))) {
-                if constexpr (m < 2) {
+                if constexpr (fm >= G::FM) {   // (a slot keeps its places for the reads)
+                } else if constexpr (m < 2) {
                     const half8_t b = p < 4 ? b0[p < 4 ? r + 2 * p : 0] : p == 4 ? b0[r + 8 < TH + 8 ? r + 8 : 0] : l0[1][r];
                     acc[fm][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[p][0][fm], b, acc[fm][r], 0, 0, 0);
                 } else if constexpr (m < 4) {
@@ -282,7 +284,7 @@ __device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& rin
                 if constexpr (n >= 0 && n < 4) request(std::integral_constant<int, u / TH>(), std::integral_constant<int, u % TH>(), std::integral_constant<int, n>());
                 // a share of the weights of pair p + LW
                 constexpr int NW = HSTORE ? 4 : 8, k = (r * NW + TH - 1) / TH + m - (HSTORE ? 4 : 2);
-                if constexpr (m >= (HSTORE ? 4 : 2) && k < NW && k * TH / NW == r)
+                if constexpr (m >= (HSTORE ? 4 : 2) && k < NW && k * TH / NW == r && k % 2 < G::FM)
                     rows_put_w(a0[p + LW], a2[p + LW], k, *reinterpret_cast<const i32x4_t*>(weights + ((p + LW) % NP * NW + k) * 1024));
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -293,7 +295,7 @@ __device__ __forceinline__ void c4_rows(f32x4_t (&acc)[2][G::FN], C4Ring<G>& rin
 #pragma unroll
     for (int d = 0; d < LW; d++)
 #pragma unroll
-        for (int fm = 0; fm < 2; fm++) {
+        for (int fm = 0; fm < G::FM; fm++) {
             ring.a0[d][0][fm] = a0[NP + d][0][fm]; ring.a0[d][1][fm] = a0[NP + d][1][fm];
             if constexpr (C8) ring.a2[d][fm] = a2[NP + d][fm];
         }

@@ -17,36 +17,42 @@
 
 namespace fynhip {
 namespace {
-// The halves of eight values that carry their scale already, as split_pair gives them: packed conversions and subtractions, 26
+// The halves of values that carry their scale already, as split_pair gives them: packed conversions and subtractions, 26
 // clocks a pair where the four mixed-precision FMAs of split_pair take 33 (each of them issues for eight).
-__device__ __forceinline__ void split_eight(const float (&x)[8], half8_t& hi, half8_t& lo) {
+template <int N, class V>
+__device__ __forceinline__ void split_packed(const float (&x)[N], V& hi, V& lo) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
+    for (int e = 0; e < N; e++) {
         hi[e] = (_Float16)x[e];
         lo[e] = (_Float16)(x[e] - (float)hi[e]);
     }
 }
 
 // The first layer's tile, as GeoC4 describes it for conv_p16c4_kernel (rows without the pad behind them: the LDS is full).
+// SMALL: at most 16 channels in between and 32 behind.
+template <bool SMALL>
 struct GeoA {
-    static constexpr int K = 9, TH = 9, TWG = 64, FN = TH, NS = 12, PIX = 8;
+    static constexpr int K = 9, TH = 9, TWG = 64, FN = TH, FM = SMALL ? 1 : 2, NS = 12, PIX = 8;
     static constexpr int HW = TWG + 9, HH = TH + K - 1;
     static constexpr int ROW_PITCH = (HW + 1) * PIX;
     static constexpr int COPY = HH * ROW_PITCH, COPY2 = (COPY + 127) / 128 * 128 + 48, PLANE = COPY2 + COPY + 16, BUF = NPL * PLANE;
     static constexpr int NITEMS = HH * HW, NB = (NITEMS + 255) / 256;
-    // the second layer's: rows and columns of its tile, the tensor in between [row][even columns, odd columns][32 channels]
-    static constexpr int TH2 = 4, TW2 = 31, MROW = 63 * 64, MPLANE = TH * MROW;
+    // the second layer's: rows and columns of its tile, the tensor in between [row][even columns, odd columns][32 or 16 channels]
+    static constexpr int TH2 = 4, TW2 = 31, SLOT = SMALL ? 32 : 64, MROW = 63 * SLOT, MPLANE = TH * MROW;
+    static constexpr int STEPS2 = 5;                                // SMALL: the second layer's, two taps of 16 channels each; its weights lie in LDS too
     static constexpr int NW = HSTORE ? 4 : 8;                       // weight fragments of a pair of steps (c4_rows)
-    static constexpr int WEIGHTS = BUF, MID = WEIGHTS + NS / 2 * NW * 1024, SB = MID + NPL * MPLANE, LDS = SB + (32 + 64) * 2 * 4;
+    static constexpr int WEIGHTS = BUF, MID = WEIGHTS + NS / 2 * NW * 1024, SB = MID + NPL * MPLANE, W2 = SB + (32 + 64) * 2 * 4, LDS = W2 + (SMALL ? STEPS2 * 2 * NPL * 1024 : 0);
     static_assert(LDS + 16 <= 160 * 1024 && BUF < 65536 && ROW_PITCH % 16 == 0, "fits a CU; 16-byte reads are aligned");
 };
 
 // (KEEP: the tensor in between is written to memory as well, for a net whose tensors all stay readable)
-template <bool HS, bool KEEP>
+template <bool HS, bool KEEP, bool SMALL>
 __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
-    using G = GeoA;
+    using G = GeoA<SMALL>;
     constexpr bool C8 = !HS;
-    constexpr int FN = G::FN, NW = G::NW;
+    constexpr int FN = G::FN, FM = G::FM, NW = G::NW;
+    // a lane's first channel of a fragment, and from one fragment to the next (c4_common.h; one fragment alone is in order)
+    constexpr int CK1 = SMALL ? 4 : CHK;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ unsigned range_box[2];
     if (blockIdx.x == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
@@ -81,7 +87,11 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             inside = 0u;
 #pragma unroll
             for (int i = 0; i < G::NB; i++) {
-                const int y = y0 + (yx[i] >> 16), x = x0 + (yx[i] & 0xffff);
+                int y = y0 + (yx[i] >> 16), x = x0 + (yx[i] & 0xffff);
+                if (p.clamp) {
+                    y = min(max(y, 0), p.h - 1);
+                    x = min(max(x, 0), p.w - 1);
+                }
                 const bool ok = l_off[i] >= 0 && (unsigned)y < (unsigned)p.h && (unsigned)x < (unsigned)p.w;
                 inside |= ok ? 1u << i : 0u;
                 raw[i] = *reinterpret_cast<const raw_t*>(in + (ok ? ((y + p.in_off) * p.in_wp + x + p.in_off) * 4 : 0));
@@ -150,12 +160,12 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
         constexpr int SHARE = G::NS / 2 * NW / 4;
         i32x4_t v[SHARE];
 #pragma unroll
-        for (int i = 0; i < SHARE; i++) {
+        for (int i = 0; i < SHARE; i += SMALL ? 2 : 1) {   // (SMALL: the first fragment's alone)
             const int c = w * SHARE + i, k = c % NW, st = c / NW * 2 + (k / 2) % 2, fm = k % 2, plane = k < 4 ? 0 : 2;
             v[i] = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const unsigned char*>(p.wpack[0]) + (size_t)((st * p.mfrags0 + fm) * NPLW + plane) * 1024 + wlane);
         }
 #pragma unroll
-        for (int i = 0; i < SHARE; i++) *reinterpret_cast<i32x4_t*>(lds + G::WEIGHTS + (w * SHARE + i) * 1024 + wlane) = v[i];
+        for (int i = 0; i < SHARE; i += SMALL ? 2 : 1) *reinterpret_cast<i32x4_t*>(lds + G::WEIGHTS + (w * SHARE + i) * 1024 + wlane) = v[i];
     }
     float mid_scale = 1.f, inv_mid = 1.f;
     if (p.in_amax) {
@@ -172,11 +182,24 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     const unsigned char* const rows_at = col + 2 * kq * G::PIX;
     const unsigned char* const ninth_at = col + kq * G::ROW_PITCH + 8 * G::PIX;
     const unsigned char* const last_at = col + 8 * G::ROW_PITCH + 8 * G::PIX;
-    unsigned char* const mid_to = lds + G::MID + ((x1 & 1) ? 32 + (x1 >> 1) : x1 >> 1) * 64 + kq * 16;   // (its eight channels side by side; the second layer's weights are laid out for that)
-    const int cpair = w & 1, cfrag = w >> 1;   // of the second layer: 32 channels, 16 columns
-    const unsigned char* const mid_at = lds + G::MID + (cfrag * 16 + mq) * 64 + kq * 16;
+    unsigned char* const mid_to = lds + G::MID + ((x1 & 1) ? 32 + (x1 >> 1) : x1 >> 1) * G::SLOT + kq * (G::SLOT / 4);   // (its eight channels side by side; the second layer's weights are laid out for that)
+    const int cpair = SMALL ? 0 : w & 1, cfrag = w >> 1;   // of the second layer: 32 channels, 16 columns
+    constexpr int ROWS2 = SMALL ? G::TH2 / 2 : G::TH2;
+    const int row2 = SMALL ? (w & 1) * ROWS2 : 0;          // rows
+    const unsigned char* const mid_at = lds + G::MID + (cfrag * 16 + mq) * G::SLOT + (SMALL ? (kq & 1) * 16 + row2 * 2 * G::MROW : kq * 16);
     // (buffer loads: the fragment's place is a scalar operand, where 64-bit addresses of all of them would fill the registers)
     const __amdgpu_buffer_rsrc_t weights2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.wpack[1]), 0, 36 * NPL * 1024, 0x00020000);   // [kx][32 channels][ky][fragment][plane]
+    // SMALL: two taps a step, the lanes of either half of the wave one
+    int tap_at[SMALL ? G::STEPS2 : 1];
+    if constexpr (SMALL) {
+#pragma unroll
+        for (int s = 0; s < G::STEPS2; s++) {
+            const int tap = min(2 * s + (kq >> 1), 8), ky = tap / 3, kx = tap - 3 * ky;
+            tap_at[s] = ky * G::MROW + (kx == 1 ? 32 * G::SLOT : kx * (G::SLOT / 2));
+        }
+        for (int i = w; i < G::STEPS2 * 2 * NPL; i += 4)
+            *reinterpret_cast<i32x4_t*>(lds + G::W2 + i * 1024 + wlane) = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const unsigned char*>(p.wpack[1]) + i * 1024 + wlane);
+    }
     const float* const sb = reinterpret_cast<const float*>(lds + G::SB);
     store_t* const out = reinterpret_cast<store_t*>(p.out);
     const bool through = store_through_pays(p.out, p.h2, p.w2, p.out_cp * ESZ, !p.plain_stores, hw_block_count());
@@ -192,11 +215,11 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
 #pragma unroll
     for (int d = 0; d < C4Ring<G>::LW; d++)
 #pragma unroll
-        for (int k = 0; k < NW; k++) rows_put_w(ring.a0[d], ring.a2[d], k, *reinterpret_cast<const i32x4_t*>(lds + G::WEIGHTS + (d * NW + k) * 1024 + wlane));
+        for (int k = 0; k < NW; k += SMALL ? 2 : 1) rows_put_w(ring.a0[d], ring.a2[d], k, *reinterpret_cast<const i32x4_t*>(lds + G::WEIGHTS + (d * NW + k) * 1024 + wlane));
     float vmax = 0.f;
     for (int tile = group;;) {
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
-        half8_t wq[2][3][2][NPL];   // the second layer's weights of a column of taps, two columns
+        half8_t wq[SMALL ? 1 : 2][3][2][NPL];   // the second layer's weights of a column of taps, two columns
         typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
         auto load_w = [&](int set, int kx) __attribute__((always_inline)) {
 #pragma unroll
@@ -208,9 +231,9 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                         wq[set][ky][fm][pl] = __builtin_bit_cast(half8_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights2, wlane, (unsigned)(((kx * 2 + cpair) * 6 + ky * 2 + fm) * NPL + pl) * 1024u, 0));
         };
         {   // ---- first layer ----
-            f32x4_t acc[2][FN];
+            f32x4_t acc[FM][FN];
 #pragma unroll
-            for (int fm = 0; fm < 2; fm++)
+            for (int fm = 0; fm < FM; fm++)
 #pragma unroll
                 for (int fn = 0; fn < FN; fn++) acc[fm][fn] = (f32x4_t)(0.f);
 #pragma unroll
@@ -223,14 +246,15 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             }
             c4_rows<G, false>(acc, ring, rows_at, ninth_at, last_at, rows_at, lds + G::WEIGHTS + wlane);
             __builtin_amdgcn_sched_barrier(0);
-            f32x4_t scm[2], bi[2];
+            f32x4_t scm[FM], bi[FM];
 #pragma unroll
-            for (int fm = 0; fm < 2; fm++) {
-                scm[fm] = *reinterpret_cast<const f32x4_t*>(sb + kq * CHK + fm * CHF) * (mul1 * mid_scale);
-                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 32 + kq * CHK + fm * CHF) * mid_scale;
+            for (int fm = 0; fm < FM; fm++) {
+                scm[fm] = *reinterpret_cast<const f32x4_t*>(sb + kq * CK1 + fm * CHF) * (mul1 * mid_scale);
+                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 32 + kq * CK1 + fm * CHF) * mid_scale;
             }
             const int px = txi * 2 * G::TW2 - 1 + x1;
             const bool x_ok = (unsigned)px < (unsigned)p.w;
+            typedef typename std::conditional<SMALL, half4_t, half8_t>::type piece_t;
             auto leave = [&](auto general_, auto first_, auto end_) __attribute__((always_inline)) {   // (general: an activation other than none, a clamp exact on halves, or a clamp)
                 constexpr bool GENERAL = decltype(general_)::value;
 #pragma unroll
@@ -240,43 +264,45 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                     unsigned char* const to = mid_to + r * G::MROW;
                     // (a tile's first row and column are its neighbours' to write)
                     const bool own = KEEP && ok && r > 0 && x1 > 0;
-                    store_t* const kept = reinterpret_cast<store_t*>(p.mid) + ((size_t)(p.mid_off + tyi * 2 * G::TH2 - 1 + r) * p.mid_wp + p.mid_off + px) * p.mid_cp + kq * CHK;
+                    store_t* const kept = reinterpret_cast<store_t*>(p.mid) + ((size_t)(p.mid_off + tyi * 2 * G::TH2 - 1 + r) * p.mid_wp + p.mid_off + px) * p.mid_cp + kq * CK1;
                     if constexpr (HS) {
-                        half8_t v;
+                        piece_t v;
 #pragma unroll
-                        for (int fm = 0; fm < 2; fm++)
+                        for (int fm = 0; fm < FM; fm++)
 #pragma unroll
                             for (int e = 0; e < 4; e++) v[fm * 4 + e] = (_Float16)(acc[fm][r][e] * scm[fm][e] + bi[fm][e]);   // (as the layer would have stored it)
                         if constexpr (KEEP) {
-                            if (own && kq * CHK < p.mid_cp) *reinterpret_cast<half8_t*>(kept) = v;
+                            if (own && kq * CK1 < p.mid_cp) *reinterpret_cast<piece_t*>(kept) = v;
                         }
-                        if constexpr (!GENERAL) {
-                            v = act_half(v, hlo1, hhi1);
-                        } else {
+                        if constexpr (GENERAL) {
 #pragma unroll
-                            for (int e = 0; e < 8; e++) v[e] = (_Float16)act_p16((float)v[e], p.act[1]);
+                            for (int e = 0; e < 4 * FM; e++) v[e] = (_Float16)act_p16((float)v[e], p.act[1]);
+                        } else if constexpr (SMALL) {
+                            v = act_half4(v, hlo1, hhi1);
+                        } else {
+                            v = act_half(v, hlo1, hhi1);
                         }
-                        *reinterpret_cast<half8_t*>(to) = ok ? v : (half8_t)((_Float16)0.f);
+                        *reinterpret_cast<piece_t*>(to) = ok ? v : (piece_t)((_Float16)0.f);
                     } else {
                         const float lo = ok ? lo1 : 0.f, hi = ok ? hi1 : 0.f, leak = ok ? leak1 : 0.f;
-                        float x[8];
                         if constexpr (KEEP) {
 #pragma unroll
-                            for (int fm = 0; fm < 2; fm++)
-                                if (own && kq * CHK + fm * CHF < p.mid_cp) *reinterpret_cast<f32x4_t*>(kept + fm * CHF) = (acc[fm][r] * scm[fm] + bi[fm]) * inv_mid;
+                            for (int fm = 0; fm < FM; fm++)
+                                if (own && kq * CK1 + fm * CHF < p.mid_cp) *reinterpret_cast<f32x4_t*>(kept + fm * CHF) = (acc[fm][r] * scm[fm] + bi[fm]) * inv_mid;
                         }
+                        float x[4 * FM];
 #pragma unroll
-                        for (int i = 0; i < 8; i++) {
+                        for (int i = 0; i < 4 * FM; i++) {
                             const float v = acc[i / 4][r][i % 4] * scm[i / 4][i % 4] + bi[i / 4][i % 4];
                             x[i] = __builtin_amdgcn_fmed3f(v, lo, hi);
                             if constexpr (GENERAL) x[i] += leak * fminf(v, 0.f);
                         }
-                        half8_t H, L;
-                        split_eight(x, H, L);
-                        *reinterpret_cast<half8_t*>(to) = H;
-                        *reinterpret_cast<half8_t*>(to + G::MPLANE) = L;
+                        piece_t H, L;
+                        split_packed<4 * FM>(x, H, L);
+                        *reinterpret_cast<piece_t*>(to) = H;
+                        *reinterpret_cast<piece_t*>(to + G::MPLANE) = L;
                     }
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (!SMALL || r % 3 == 2) __builtin_amdgcn_sched_barrier(0);   // (four values are too few chains of dependent instructions)
                 }
             };
             auto rows = [&](auto first, auto end) __attribute__((always_inline)) {
@@ -287,40 +313,63 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             };
             constexpr int FIRST = 5;
             rows(std::integral_constant<int, 0>(), std::integral_constant<int, FIRST>());
-            load_w(0, 0);   // (the second layer's first weights, into registers that the rows so far have left)
+            if constexpr (!SMALL) load_w(0, 0);   // (the second layer's first weights, into registers that the rows so far have left)
             rows(std::integral_constant<int, FIRST>(), std::integral_constant<int, FN>());
+            if (p.clamp && (txi == 0 || tyi == 0)) {   // what lies above or to the left of the layer's output repeats its first row and column
+                if (txi == 0 && x1 == 0)
+                    for (int i = 0; i < FN * NPL; i++) {
+                        unsigned char* const to = mid_to + (i % FN) * G::MROW + (i / FN) * G::MPLANE;
+                        *reinterpret_cast<piece_t*>(to) = *reinterpret_cast<const piece_t*>(to + 32 * G::SLOT);
+                    }
+                if (tyi == 0 && x1 < 63)
+                    for (int pl = 0; pl < NPL; pl++) *reinterpret_cast<piece_t*>(mid_to + pl * G::MPLANE) = *reinterpret_cast<const piece_t*>(mid_to + pl * G::MPLANE + G::MROW);
+            }
         }
         lds_barrier();   // the tensor in between is there
         {   // ---- second layer: rows 2 r + ky, columns 2 c + kx ----
-            f32x4_t acc[2][G::TH2];
+            f32x4_t acc[2][ROWS2];
 #pragma unroll
             for (int fm = 0; fm < 2; fm++)
 #pragma unroll
-                for (int r = 0; r < G::TH2; r++) acc[fm][r] = (f32x4_t)(0.f);
-            constexpr int AHEAD = 3, Q = 3 * FN;
-            half8_t b[AHEAD + 1][NPL];
+                for (int r = 0; r < ROWS2; r++) acc[fm][r] = (f32x4_t)(0.f);
+            constexpr int AHEAD = 3, Q = SMALL ? G::STEPS2 * ROWS2 : 3 * FN;
+            half8_t b[AHEAD + 1][NPL], w2[SMALL ? G::STEPS2 : 1][2][NPL];
             auto request = [&](int q) __attribute__((always_inline)) {
                 const int kx = q / FN, j = q % FN;
+                const unsigned char* const at = mid_at + (SMALL ? tap_at[SMALL ? q / ROWS2 : 0] + q % ROWS2 * 2 * G::MROW : (kx == 1 ? 32 * G::SLOT : kx * (G::SLOT / 2)) + j * G::MROW);
 #pragma unroll
-                for (int pl = 0; pl < NPL; pl++)
-                    b[q % (AHEAD + 1)][pl] = *reinterpret_cast<const half8_t*>(mid_at + (kx == 1 ? 32 * 64 : kx * 32) + j * G::MROW + pl * G::MPLANE);
+                for (int pl = 0; pl < NPL; pl++) b[q % (AHEAD + 1)][pl] = *reinterpret_cast<const half8_t*>(at + pl * G::MPLANE);
             };
 #pragma unroll
             for (int q = 0; q < AHEAD; q++) request(q);
+            auto weights2_of = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 2 * NPL; i++) w2[SMALL ? s : 0][i / NPL][i % NPL] = *reinterpret_cast<const half8_t*>(lds + G::W2 + (s * 2 * NPL + i) * 1024 + wlane);
+            };
+            if constexpr (SMALL) weights2_of(0);
 #pragma unroll
             for (int q = 0; q < Q; q++) {
-                const int kx = q / FN, j = q % FN;
-                if (j == 0 && kx + 1 < 3) load_w((kx + 1) & 1, kx + 1);
                 if (q + AHEAD < Q) request(q + AHEAD);
+                if constexpr (SMALL) {
+                    if (q % ROWS2 == 0 && q / ROWS2 + 1 < G::STEPS2) weights2_of(q / ROWS2 + 1);
 #pragma unroll
-                for (int i = 0; i < NPASS; i++)
-#pragma unroll
-                    for (int ky = 0; ky < 3; ky++) {
-                        if (((j - ky) & 1) || j < ky || (j - ky) / 2 >= G::TH2) continue;
+                    for (int i = 0; i < NPASS; i++)
 #pragma unroll
                         for (int fm = 0; fm < 2; fm++)
-                            acc[fm][(j - ky) / 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wq[kx & 1][ky][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][(j - ky) / 2], 0, 0, 0);
-                    }
+                            acc[fm][q % ROWS2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w2[q / ROWS2][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][q % ROWS2], 0, 0, 0);
+                } else {
+                    const int kx = q / FN, j = q % FN;
+                    if (j == 0 && kx + 1 < 3) load_w((kx + 1) & 1, kx + 1);
+#pragma unroll
+                    for (int i = 0; i < NPASS; i++)
+#pragma unroll
+                        for (int ky = 0; ky < 3; ky++) {
+                            if (((j - ky) & 1) || j < ky || (j - ky) / 2 >= G::TH2) continue;
+#pragma unroll
+                            for (int fm = 0; fm < 2; fm++)
+                                acc[fm][(j - ky) / 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wq[kx & 1][ky][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][(j - ky) / 2], 0, 0, 0);
+                        }
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (drop) {   // (ahead of this workgroup's first store: what it has read so far may go as well)
@@ -335,8 +384,8 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             }
             const int c2 = cfrag * 16 + mq, ox = txi * G::TW2 + c2, ch0 = cpair * 32 + kq * CHK;
 #pragma unroll
-            for (int r = 0; r < G::TH2; r++) {
-                const int oy = tyi * G::TH2 + r;
+            for (int r = 0; r < ROWS2; r++) {
+                const int oy = tyi * G::TH2 + row2 + r;
                 const bool inside = c2 < G::TW2 && ox < p.w2 && oy < p.h2;
                 const size_t at = ((size_t)(p.out_off + oy) * p.out_wp + p.out_off + ox) * p.out_cp + ch0;
                 half8_t hv;
@@ -371,24 +420,28 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
 #else
 #define A16_NAME(n) n
 int launch_conv_a16_half(const ConvA16Params& p, hipStream_t s);
-size_t conv_a16_lds_bytes(bool f16) { return (f16 ? 1 : 2) * (size_t)(GeoA::PLANE + GeoA::MPLANE) + (f16 ? 24 : 48) * 1024 + (32 + 64) * 2 * 4; }
-void conv_a16_tile(int* rows, int* cols) { *rows = GeoA::TH2; *cols = GeoA::TW2; }
+size_t conv_a16_lds_bytes(bool f16, bool small) {
+    return (f16 ? 1 : 2) * (size_t)(GeoA<false>::PLANE + (small ? GeoA<true>::MPLANE : GeoA<false>::MPLANE)) + (f16 ? 24 : 48) * 1024 + (32 + 64) * 2 * 4 + (small ? (f16 ? 10 : 20) * 1024 : 0);
+}
+void conv_a16_tile(int* rows, int* cols) { *rows = GeoA<false>::TH2; *cols = GeoA<false>::TW2; }
 #endif
 int A16_NAME(launch_conv_a16)(const ConvA16Params& p, hipStream_t s) {
 #if !FYN_P16_HALF
     if (p.f16) return launch_conv_a16_half(p, s);
 #endif
     const long long tiles = (long long)p.tiles_x * p.tiles_y;
-    const int rows = p.mid ? (p.h + 2 * GeoA::TH2 - 1) / (2 * GeoA::TH2) : (p.h2 + GeoA::TH2 - 1) / GeoA::TH2;
-    const int cols = p.mid ? (p.w + 2 * GeoA::TW2 - 1) / (2 * GeoA::TW2) : (p.w2 + GeoA::TW2 - 1) / GeoA::TW2;
+    const int rows = p.mid ? (p.h + 2 * GeoA<false>::TH2 - 1) / (2 * GeoA<false>::TH2) : (p.h2 + GeoA<false>::TH2 - 1) / GeoA<false>::TH2;
+    const int cols = p.mid ? (p.w + 2 * GeoA<false>::TW2 - 1) / (2 * GeoA<false>::TW2) : (p.w2 + GeoA<false>::TW2 - 1) / GeoA<false>::TW2;
     if ((p.f16 != 0) != HSTORE || !p.in || !p.out || !p.wpack[0] || !p.wpack[1] || (!HSTORE && !p.in_amax) || p.h < 2 || p.w < 2 || p.h2 != p.h / 2 || p.w2 != p.w / 2 || p.in_off < 0 ||
-        p.h + p.in_off > p.in_hp || p.w + p.in_off > p.in_wp || (long long)p.in_hp * p.in_wp * 4 > (1ll << 30) || p.mid_cp < 1 || p.mid_cp > 32 || p.mfrags0 < 2 || p.out_cp < 8 || p.out_cp > 64 ||
-        p.out_cp % 8 != 0 || p.tiles_x != cols || p.tiles_y != rows || tiles > 4000000 || p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.groups < 1 || p.groups > tiles || p.nreset < 0 || p.nreset > 4 ||
-        (p.mid && (p.mid_cp % (HSTORE ? 8 : 4) != 0 || p.mid_off < 0 || p.mid_wp < p.w + p.mid_off)))
+        p.h + p.in_off > p.in_hp || p.w + p.in_off > p.in_wp || (long long)p.in_hp * p.in_wp * 4 > (1ll << 30) || p.mid_cp < 1 || p.mid_cp > 32 || p.mfrags0 < (p.small && HSTORE ? 1 : 2) || p.out_cp < 8 || p.out_cp > 64 ||
+        p.out_cp % 8 != 0 || p.tiles_x != cols || p.tiles_y != rows || tiles > 4000000 || p.rcp_tiles_x != 1.0f / (float)p.tiles_x || p.groups < 1 || p.groups > tiles || p.nreset < 0 || p.nreset > 4 || (p.small && (p.mid_cp > 16 || p.out_cp > 32)) ||
+        (p.mid && (p.mid_cp % (HSTORE && !p.small ? 8 : 4) != 0 || p.mid_off < 0 || p.mid_wp < p.w + p.mid_off)))
         return -5;
-    const auto kernel = p.mid ? conv_a16_kernel<HSTORE, true> : conv_a16_kernel<HSTORE, false>;
-    if (ensure_lds(reinterpret_cast<const void*>(kernel), GeoA::LDS) != 0) return -2;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)p.groups), dim3(512), GeoA::LDS, s, p);
+    const auto kernel = p.small ? (p.mid ? conv_a16_kernel<HSTORE, true, true> : conv_a16_kernel<HSTORE, false, true>)
+                                : (p.mid ? conv_a16_kernel<HSTORE, true, false> : conv_a16_kernel<HSTORE, false, false>);
+    const size_t lds = p.small ? GeoA<true>::LDS : GeoA<false>::LDS;
+    if (ensure_lds(reinterpret_cast<const void*>(kernel), lds) != 0) return -2;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)p.groups), dim3(512), lds, s, p);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -366,9 +366,9 @@ static bool pair_of(Net* net, const ConvLayer* c, ConvLayer*& a) {
 }
 // The 9x9 layer `a` on an image that `c`, a 3x3 layer with a step of two, alone reads.
 static bool head_of(Net* net, const ConvLayer* c, ConvLayer*& a) {
-    if (!c || c->k != 3 || c->stride != 2 || c->dil != 1 || c->clamp || c->frac_shift || c->direct || c->wide || (c->d.flags & FYN_FLAG_RESIDUAL_INPUT)) return false;
+    if (!c || c->k != 3 || c->stride != 2 || c->dil != 1 || c->frac_shift || c->direct || c->wide || (c->d.flags & FYN_FLAG_RESIDUAL_INPUT)) return false;
     a = alone_in_front(net, c);
-    if (!plain_conv(a, 9) || a->clamp || a->oc > 32 || c->oc > 64 || a->d.in_channels > 4) return false;
+    if (!plain_conv(a, 9) || a->clamp != c->clamp || a->oc > 32 || c->oc > 64 || a->d.in_channels > 4) return false;
     const int from = net->tensors[a->in[0]].producer;   // (a frame from the host or the application: its value-range word is never lost)
     return from < 0 || net->layer(from)->d.type == FYN_LAYER_UPLOAD;
 }
@@ -539,6 +539,7 @@ void fuse_head_layers(Net* net) {
             continue;
         // (the form whose weights and schedule the launch takes for the first layer; with fp32 tensors its fp8 correction terms too)
         if (!a->p16 || !a->c4 || a->pp.tile_w != 16 || (!iv.f16 && (!a->tin(0).amax || !conv_p16c4_uses_fp8(a->pp, 9)))) continue;
+        if (c->clamp && (iv.pad || mv.pad)) continue;
         // (positions beside a layer's input are zeros behind its activation as well)
         if (a->act().lo > 0.f || a->act().hi < 0.f || c->act().lo > 0.f || c->act().hi < 0.f) continue;
         const int x = a->in[0];
@@ -560,14 +561,20 @@ void fuse_head_layers(Net* net) {
             q.act[i] = L[i]->act();
         }
         q.mid_cp = mv.cp;
+        q.clamp = c->clamp ? 1 : 0;
+        q.small = mv.cp <= 16 && ov.cp <= 32 ? 1 : 0;
         q.out = ov.ptr; q.out_cp = ov.cp; q.out_wp = ov.wp(); q.out_off = ov.pad;
         q.plain_stores = net->sw.get("FYNHIP_PLAIN_STORES") ? 1 : 0;
         q.f16 = ov.f16 ? 1 : 0;
-        void* const wp = net->dev_alloc((size_t)36 * (q.f16 ? 1 : 2) * 1024, true);
+        void* const wp = net->dev_alloc((size_t)(q.small ? (q.f16 ? 10 + 12 : 20) : 36 * (q.f16 ? 1 : 2)) * 1024, true);
         q.wpack[1] = wp;
+        if (q.small && q.f16) {
+            q.wpack[0] = static_cast<const unsigned char*>(wp) + 10 * 1024;
+            q.mfrags0 = 1;
+        }
         bool pick = true;
         char key[200];
-        snprintf(key, sizeof(key), "head:%d:%dto%dto%d:%dx%d", q.f16, a->d.in_channels, a->oc, c->oc, a->oh, a->ow);
+        snprintf(key, sizeof(key), "head:%d:%dto%dto%d:%dx%d:e%d", q.f16, a->d.in_channels, a->oc, c->oc, a->oh, a->ow, q.clamp);
         if (forced || tune_cache_flag(net, key, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float t_one = 1e30f, t_apart = 1e30f;

@@ -400,10 +400,12 @@ struct ConvA16Params {
     unsigned* out_amax;
     unsigned* reset[4];
     int nreset;
+    int clamp;              // positions outside a layer's input repeat its edge (zeros otherwise)
+    int small;              // at most 16 channels in between and 32 behind: a kernel of its own, with other weights (pack_head)
     int plain_stores, f16;
 };
 void conv_a16_tile(int* rows, int* cols);   // of the second layer's output
-size_t conv_a16_lds_bytes(bool f16);
+size_t conv_a16_lds_bytes(bool f16, bool small);
 int launch_conv_a16(const ConvA16Params& p, hipStream_t s);
 // Two 3x3 layers between tensors of few channels, one behind the other, as one launch (conv_c16.hip): h x w positions, th rows of
 // sixteen per workgroup.

@@ -1460,7 +1460,7 @@ class ConvLayer : public Layer {
             int rows, cols;
             conv_a16_tile(&rows, &cols);
             snprintf(buf, sizeof(buf), "conv_a16 %s layer %d (9x9) and this one (3x3, step 2) in one launch, tiles of %dx%d positions, blocks=%d tiles=%d lds=%zu%s; apart: ", head.f16 ? "f16" : "f16+fp8-split, f16x2-split",
-                     head_layer, rows, cols, head.groups, head.tiles_x * head.tiles_y, conv_a16_lds_bytes(head.f16 != 0),
+                     head_layer, rows, cols, head.groups, head.tiles_x * head.tiles_y, conv_a16_lds_bytes(head.f16 != 0, head.small != 0),
                      store_through_pays(head.out, head.h2, head.w2, head.out_cp * (head.f16 ? 2 : 4), !head.plain_stores, (size_t)head.groups) ? " stores=through" : "");
             return buf + own_info();
         }
@@ -1727,6 +1727,10 @@ class ConvLayer : public Layer {
         const int cin = d.in_channels, npl = head.f16 ? 1 : 2;
         const float wmul = weight_prescale(w, (size_t)oc * 9 * cin);
         head.acc_mul[1] = 1.0f / wmul;
+        if (head.small) {
+            pack_small_head(a, w, wmul);
+            return;
+        }
         std::vector<uint16_t> pack((size_t)36 * npl * 64 * 8, 0);
         uint16_t* base = pack.data();
         for (int kx = 0; kx < 3; kx++)
@@ -1744,6 +1748,40 @@ class ConvLayer : public Layer {
                                 if (npl == 2) base[(size_t)(64 + lane) * 8 + j] = f2h_bits(v - h2f(hi));
                             }
                         }
+        reupload(net, static_cast<uint16_t*>(head_wpack_dev), pack);
+    }
+    // with at most 16 channels in between: [pair of taps][cout fragment][plane][lane][8 halves], and on fp16 tensors, whose
+    // first layer's own weights have its channels dealt to two fragments, behind them those of one: [step][lane][8 halves]
+    void pack_small_head(const ConvLayer* a, const float* w, float wmul) {
+        const int cin = d.in_channels, npl = head.f16 ? 1 : 2;
+        std::vector<uint16_t> pack((size_t)(5 * 2 * npl + (head.f16 ? 12 : 0)) * 64 * 8, 0);
+        uint16_t* base = pack.data();
+        for (int s = 0; s < 5; s++)
+            for (int fm = 0; fm < 2; fm++, base += (size_t)npl * 64 * 8)
+                for (int lane = 0; lane < 64; lane++) {
+                    const int o = p16_row_channel(fm, lane & 15, head.f16 ? 2 : 1), tap = 2 * s + (lane >> 5);
+                    for (int j = 0; o < oc && tap < 9 && j < 8; j++) {
+                        const int ci = 8 * ((lane >> 4) & 1) + j;
+                        if (ci >= cin) continue;
+                        const float v = w[((size_t)o * 9 + tap) * cin + ci] * wmul;
+                        const uint16_t hi = f2h_bits(v);
+                        base[(size_t)lane * 8 + j] = hi;
+                        if (npl == 2) base[(size_t)(64 + lane) * 8 + j] = f2h_bits(v - h2f(hi));
+                    }
+                }
+        if (head.f16) {   // (as pack_c4 does for rows of sixteen positions)
+            const int c1 = a->d.in_channels;
+            const float* w1 = a->block.data() + a->oc;
+            const float mul1 = 1.0f / a->pp.acc_mul;
+            for (int st = 0; st < 12; st++, base += 64 * 8)
+                for (int lane = 0; lane < 64; lane++) {
+                    const int o = lane & 15, ky = st < 9 ? st : 4 * (st - 9) + (lane >> 4), kx0 = st < 9 ? 2 * (lane >> 4) : 8;
+                    for (int j = 0; o < a->oc && ky < 9 && j < 8; j++) {
+                        const int kx = kx0 + j / 4, ci = j % 4;
+                        if (kx < 9 && ci < c1) base[(size_t)lane * 8 + j] = f2h_bits(w1[(((size_t)o * 9 + ky) * 9 + kx) * c1 + ci] * mul1);
+                    }
+                }
+        }
         reupload(net, static_cast<uint16_t*>(head_wpack_dev), pack);
     }
     // The 3x3 layer in front of this 3x3 layer in the same launch, one of conv_c16_kernel (conv_c16.hip; fuse_pair_layers below)
