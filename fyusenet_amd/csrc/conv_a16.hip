@@ -13,6 +13,10 @@
 // then 32 channels x 16 columns x 4 rows of the second one, column of taps by column of taps, where the fragment of row j
 // serves every tap that meets it.  The next tile's window is requested while this one is multiplied and replaces it behind
 // the barrier that hands over the tensor in between.
+//
+// At most 16 channels in between and 32 behind (SMALL): one fragment of channels in the first layer, two taps of 16 channels a
+// step in the second, whose weights lie in LDS; bound by the fragment reads of the first layer (134 KB a wave and tile at 128
+// bytes a clock: 4.2k of a tile's 10k clocks).  3 -> 12 -> 20 channels at 512x624: 30.8 us apart, 20 here (fp16 19.8 and 11.5).
 #include "c4_common.h"
 
 namespace fynhip {

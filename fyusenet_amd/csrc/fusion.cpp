@@ -523,8 +523,9 @@ void fuse_block_layers(Net* net) {
 
 // The first two layers of a style-transfer net (conv_a16.hip) as one launch in the place of the second, timed against their own
 // launches (us, 3 to 32 to 64 channels, one launch / apart): fp32 tensors 384x384 22 / 21, 512x624 32 / 39, 1920x1080 152 / 212;
-// fp16 256x256 7.8 / 9.3, 512x624 16 / 23, 1920x1080 72 / 92.  Untimed it is taken wherever the first layer is in its form on
-// rows of sixteen positions: a tie at the smallest such size, ahead above.
+// fp16 256x256 7.8 / 9.3, 512x624 16 / 23, 1920x1080 72 / 92; 3 to 12 to 20 channels, fp32, 512x624 20 / 31, 1024x1024 49 / 71.
+// Untimed it is taken wherever the first layer is in its form on rows of sixteen positions: a tie at the smallest such size,
+// ahead above.
 void fuse_head_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_HEAD_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV")) return;
     const bool forced = net->sw.get("FYNHIP_FORCE_HEAD_FUSION") != nullptr;
