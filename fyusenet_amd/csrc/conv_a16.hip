@@ -5,18 +5,22 @@
 //
 // Bound: the matrix pipes.  Apart, the layers meet in the largest tensor of the net -- 265 MB at 1920x1080 on fp32 tensors,
 // written and read again in half of their time --, and in the first one every workgroup multiplies and then stores.  Here it
-// stays in LDS (1920x1080, both layers: 212 us apart, 152 here; fp16 tensors 92 and 72): a workgroup walks tiles of 4 rows x 31 positions of the second layer's output and computes the 9 rows x 63
+// stays in LDS: a workgroup walks tiles of 4 rows x 31 positions of the second layer's output and computes the 9 rows x 63
 // positions of the first layer under them (1.16 times its arithmetic; a tile's columns and rows overlap its neighbours' by
 // one), as hi and lo planes with even and odd columns apart, so that the sixteen positions of a fragment of the second layer
-// are neighbours there whatever the tap and a fragment is one contiguous kilobyte.  Four MFMA waves, four staging waves: a
-// wave computes sixteen columns of the first layer with the schedule of the layer's own kernel (c4_rows, its weights in LDS),
-// then 32 channels x 16 columns x 4 rows of the second one, column of taps by column of taps, where the fragment of row j
-// serves every tap that meets it.  The next tile's window is requested while this one is multiplied and replaces it behind
-// the barrier that hands over the tensor in between.
+// are neighbours there whatever the tap and a fragment is one contiguous kilobyte.  Four waves compute the first layer, sixteen
+// columns each, with the schedule of the layer's own kernel (c4_rows, its weights in LDS).  Four others compute the second one
+// of the tile before at the same time, 32 channels x 16 columns x 4 rows each, column of taps by column of taps, where the
+// fragment of row j serves every tap that meets it, and make the operands of the tile behind in registers.  Behind a barrier the
+// first ones split their result into the tensor in between while the others put the window in place and store theirs: the
+// vector work of either half of the waves lies beside the matrix work of the other, or beside its vector work.  With one
+// group of waves for all matrix work and one that staged a tile of fp32 tensors took 18.7k clocks, now 15.0k (fp16 9.1k and
+// 7.8k); 10.4k of them are matrix instructions, of either group in one pipe.  1920x1080, both layers: 212 us apart, 131 here
+// (142 before); fp16 tensors 92 and 66 (72).
 //
 // At most 16 channels in between and 32 behind (SMALL): one fragment of channels in the first layer, two taps of 16 channels a
 // step in the second, whose weights lie in LDS; bound by the fragment reads of the first layer (134 KB a wave and tile at 128
-// bytes a clock: 4.2k of a tile's 10k clocks).  3 -> 12 -> 20 channels at 512x624: 30.8 us apart, 20 here (fp16 19.8 and 11.5).
+// bytes a clock: 4.2k of a tile's 8.6k clocks).  3 -> 12 -> 20 channels at 512x624: 30.8 us apart, 19 here (fp16 19.8 and 11).
 #include "c4_common.h"
 
 namespace fynhip {
@@ -72,7 +76,19 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     if (tid < 2) range_box[tid] = 0u;
     const unsigned range_bits = p.in_amax ? range_load(p.in_amax) : 0u;
     float in_scale = 1.f, inv_in = 1.f;
-    if (wave < 4) {   // ---------------------------------------------------------------- staging waves
+    float mid_scale = 1.f, inv_mid = 1.f;
+    auto scales = [&]() __attribute__((always_inline)) {
+        if (!p.in_amax) return;
+        const float r0 = range_after_act(range_reduce(range_bits), p.act[0]);
+        in_scale = range_scale(r0, &inv_in);
+        // (no value of the first layer is larger than its weights' largest row sum allows: a scale for the tensor in between that
+        // does not wait for it.  Such a bound is some ten times what a frame reaches, 2^4 of the 2^14 that the split has to spare)
+        if constexpr (C8) mid_scale = range_scale(range_after_act(r0 * p.gain + p.base, p.act[1]), &inv_mid);
+    };
+    const int mq = lane & 15, kq = lane >> 4, w = wave & 3;
+    const unsigned wlane = lane * 16;
+    const float* const sb = reinterpret_cast<const float*>(lds + G::SB);
+    if (wave < 4) {   // ------------------------------------------- the waves that stage and compute the second layer
         const store_t* in = reinterpret_cast<const store_t*>(p.in);
         typedef typename std::conditional<HS, half4_t, float4>::type raw_t;   // a pixel as it comes from memory
         raw_t raw[G::NB];
@@ -102,12 +118,13 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             }
         };
         const bool plain_act = p.act[0].kind == ACT_NONE;   // (a first layer reads its input as it is)
-        auto store = [&]() {
+        // (the operands of an item take the registers that its pixel came in: they are made while the matrix pipes are busy and
+        // wait there for the window's place)
+        typedef typename std::conditional<HS, half4_t, int4>::type staged_t;
+        auto convert = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < G::NB; i++) {
-                if (l_off[i] < 0) continue;
                 const bool ok = (inside >> i) & 1u;
-                unsigned char* const at = lds + l_off[i];
                 if constexpr (HS) {
                     half4_t v;
                     _Float16 hlo, hhi;
@@ -117,8 +134,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
 #pragma unroll
                         for (int e = 0; e < 4; e++) v[e] = ok ? (_Float16)act_p16((float)raw[i][e], p.act[0]) : (_Float16)0.f;
                     }
-                    *reinterpret_cast<half4_t*>(at) = v;
-                    *reinterpret_cast<half4_t*>(at + G::COPY2 + 8) = v;
+                    raw[i] = v;
                 } else {
                     const float r[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
                     float x[4];
@@ -128,38 +144,174 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                     split_pair(x[0], x[1], in_scale, h0, l0);
                     split_pair(x[2], x[3], in_scale, h1, l1);
                     const half4_t hi = __builtin_bit_cast(half4_t, uint2{h0, h1}), lo = __builtin_bit_cast(half4_t, uint2{l0, l1});
-                    const int2 c8 = int2{(int)c8_quad(lo[0], lo[1], lo[2], lo[3], 0.03125f), (int)c8_quad(hi[0], hi[1], hi[2], hi[3], 64.f)};
-                    *reinterpret_cast<half4_t*>(at) = hi;
-                    *reinterpret_cast<half4_t*>(at + G::COPY2 + 8) = hi;
-                    *reinterpret_cast<int2*>(at + G::PLANE) = c8;
-                    *reinterpret_cast<int2*>(at + G::PLANE + G::COPY2 + 8) = c8;
+                    raw[i] = __builtin_bit_cast(float4, int4{(int)h0, (int)h1, (int)c8_quad(lo[0], lo[1], lo[2], lo[3], 0.03125f), (int)c8_quad(hi[0], hi[1], hi[2], hi[3], 64.f)});
+                }
+            }
+        };
+        auto put = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < G::NB; i++) {
+                if (l_off[i] < 0) continue;
+                unsigned char* const at = lds + l_off[i];
+                const staged_t v = __builtin_bit_cast(staged_t, raw[i]);
+                if constexpr (HS) {
+                    *reinterpret_cast<half4_t*>(at) = v;
+                    *reinterpret_cast<half4_t*>(at + G::COPY2 + 8) = v;
+                } else {
+                    *reinterpret_cast<int2*>(at) = int2{v.x, v.y};
+                    *reinterpret_cast<int2*>(at + G::COPY2 + 8) = int2{v.x, v.y};
+                    *reinterpret_cast<int2*>(at + G::PLANE) = int2{v.z, v.w};
+                    *reinterpret_cast<int2*>(at + G::PLANE + G::COPY2 + 8) = int2{v.z, v.w};
                 }
             }
         };
         fetch(group);
-        if (p.in_amax) in_scale = range_scale(range_after_act(range_reduce(range_bits), p.act[0]), &inv_in);
-        float* const sb = reinterpret_cast<float*>(lds + G::SB);
-        if (tid < 32) {
-            sb[tid] = tid < p.mid_cp ? p.scale[0][tid] : 0.f;
-            sb[32 + tid] = tid < p.mid_cp ? p.bias[0][tid] : 0.f;
-        } else if (tid >= 64 && tid < 128) {
-            sb[tid] = tid - 64 < p.out_cp ? p.scale[1][tid - 64] : 0.f;
-            sb[64 + tid] = tid - 64 < p.out_cp ? p.bias[1][tid - 64] : 0.f;
+        scales();
+        {
+            float* const to = reinterpret_cast<float*>(lds + G::SB);
+            if (tid < 32) {
+                to[tid] = tid < p.mid_cp ? p.scale[0][tid] : 0.f;
+                to[32 + tid] = tid < p.mid_cp ? p.bias[0][tid] : 0.f;
+            } else if (tid >= 64 && tid < 128) {
+                to[tid] = tid - 64 < p.out_cp ? p.scale[1][tid - 64] : 0.f;
+                to[64 + tid] = tid - 64 < p.out_cp ? p.bias[1][tid - 64] : 0.f;
+            }
         }
-        store();
-        for (int tile = group;;) {
-            lds_barrier();   // the window is staged
-            tile += step;
-            if (tile < ntiles) fetch(tile);
-            lds_barrier();   // the first layer is through: the window's place is free
-            if (tile >= ntiles) return;
-            store();
+        convert();
+        put();
+        const int cpair = SMALL ? 0 : w & 1, cfrag = w >> 1;   // of the second layer: 32 channels, 16 columns
+        constexpr int ROWS2 = SMALL ? G::TH2 / 2 : G::TH2;
+        const int row2 = SMALL ? (w & 1) * ROWS2 : 0;          // rows
+        const unsigned char* const mid_at = lds + G::MID + (cfrag * 16 + mq) * G::SLOT + (SMALL ? (kq & 1) * 16 + row2 * 2 * G::MROW : kq * 16);
+        // (buffer loads: the fragment's place is a scalar operand, where 64-bit addresses of all of them would fill the registers)
+        const __amdgpu_buffer_rsrc_t weights2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.wpack[1]), 0, 36 * NPL * 1024, 0x00020000);   // [kx][32 channels][ky][fragment][plane]
+        // SMALL: two taps a step, the lanes of either half of the wave one
+        int tap_at[SMALL ? G::STEPS2 : 1];
+        if constexpr (SMALL) {
+#pragma unroll
+            for (int s = 0; s < G::STEPS2; s++) {
+                const int tap = min(2 * s + (kq >> 1), 8), ky = tap / 3, kx = tap - 3 * ky;
+                tap_at[s] = ky * G::MROW + (kx == 1 ? 32 * G::SLOT : kx * (G::SLOT / 2));
+            }
+            for (int i = w; i < G::STEPS2 * 2 * NPL; i += 4)
+                *reinterpret_cast<i32x4_t*>(lds + G::W2 + i * 1024 + wlane) = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const unsigned char*>(p.wpack[1]) + i * 1024 + wlane);
         }
+        const float mul2 = p.acc_mul[1] * inv_mid;
+        store_t* const out = reinterpret_cast<store_t*>(p.out);
+        const bool through = store_through_pays(p.out, p.h2, p.w2, p.out_cp * ESZ, !p.plain_stores, hw_block_count());
+        bool drop = through && wave == 0 && hw_block_id() < 8;
+        float vmax = 0.f;
+        f32x4_t acc[2][ROWS2];
+        auto multiply = [&]() __attribute__((always_inline)) {   // rows 2 r + ky, columns 2 c + kx of the tensor in between
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                for (int r = 0; r < ROWS2; r++) acc[fm][r] = (f32x4_t)(0.f);
+            constexpr int AHEAD = 3, Q = SMALL ? G::STEPS2 * ROWS2 : 3 * FN;
+            half8_t wq[SMALL ? 1 : 2][3][2][NPL], b[AHEAD + 1][NPL], w2[SMALL ? G::STEPS2 : 1][2][NPL];
+            typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+            auto load_w = [&](int set, int kx) __attribute__((always_inline)) {
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++)
+#pragma unroll
+                    for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                        for (int pl = 0; pl < NPL; pl++)
+                            wq[set][ky][fm][pl] = __builtin_bit_cast(half8_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights2, wlane, (unsigned)(((kx * 2 + cpair) * 6 + ky * 2 + fm) * NPL + pl) * 1024u, 0));
+            };
+            if constexpr (!SMALL) load_w(0, 0);   // (a column of taps, two columns in flight)
+            auto request = [&](int q) __attribute__((always_inline)) {
+                const int kx = q / FN, j = q % FN;
+                const unsigned char* const at = mid_at + (SMALL ? tap_at[SMALL ? q / ROWS2 : 0] + q % ROWS2 * 2 * G::MROW : (kx == 1 ? 32 * G::SLOT : kx * (G::SLOT / 2)) + j * G::MROW);
+#pragma unroll
+                for (int pl = 0; pl < NPL; pl++) b[q % (AHEAD + 1)][pl] = *reinterpret_cast<const half8_t*>(at + pl * G::MPLANE);
+            };
+#pragma unroll
+            for (int q = 0; q < AHEAD; q++) request(q);
+            auto weights2_of = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 2 * NPL; i++) w2[SMALL ? s : 0][i / NPL][i % NPL] = *reinterpret_cast<const half8_t*>(lds + G::W2 + (s * 2 * NPL + i) * 1024 + wlane);
+            };
+            if constexpr (SMALL) weights2_of(0);
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                if (q + AHEAD < Q) request(q + AHEAD);
+                if constexpr (SMALL) {
+                    if (q % ROWS2 == 0 && q / ROWS2 + 1 < G::STEPS2) weights2_of(q / ROWS2 + 1);
+#pragma unroll
+                    for (int i = 0; i < NPASS; i++)
+#pragma unroll
+                        for (int fm = 0; fm < 2; fm++)
+                            acc[fm][q % ROWS2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w2[q / ROWS2][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][q % ROWS2], 0, 0, 0);
+                } else {
+                    const int kx = q / FN, j = q % FN;
+                    if (j == 0 && kx + 1 < 3) load_w((kx + 1) & 1, kx + 1);
+#pragma unroll
+                    for (int i = 0; i < NPASS; i++)
+#pragma unroll
+                        for (int ky = 0; ky < 3; ky++) {
+                            if (((j - ky) & 1) || j < ky || (j - ky) / 2 >= G::TH2) continue;
+#pragma unroll
+                            for (int fm = 0; fm < 2; fm++)
+                                acc[fm][(j - ky) / 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wq[kx & 1][ky][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][(j - ky) / 2], 0, 0, 0);
+                        }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        auto finish = [&](int tile) __attribute__((always_inline)) {
+            const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
+            if (drop) {   // (ahead of this workgroup's first store: what it has read so far may go as well)
+                drop_clean_l2_lines();
+                drop = false;
+            }
+            f32x4_t sc[2], bi[2];
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++) {
+                sc[fm] = *reinterpret_cast<const f32x4_t*>(sb + 64 + cpair * 32 + kq * CHK + fm * CHF) * mul2;
+                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 128 + cpair * 32 + kq * CHK + fm * CHF);
+            }
+            const int c2 = cfrag * 16 + mq, ox = txi * G::TW2 + c2, ch0 = cpair * 32 + kq * CHK;
+#pragma unroll
+            for (int r = 0; r < ROWS2; r++) {
+                const int oy = tyi * G::TH2 + row2 + r;
+                const bool inside = c2 < G::TW2 && ox < p.w2 && oy < p.h2;
+                const size_t at = ((size_t)(p.out_off + oy) * p.out_wp + p.out_off + ox) * p.out_cp + ch0;
+                half8_t hv;
+#pragma unroll
+                for (int fm = 0; fm < 2; fm++) {
+                    const bool ok = inside && ch0 + (HS ? 0 : fm * CHF) < p.out_cp;
+                    f32x4_t v;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        v[e] = acc[fm][r][e] * sc[fm][e] + bi[fm][e];
+                        if constexpr (!HS) vmax = fmaxf(vmax, ok ? fabsf(v[e]) : 0.f);
+                        else hv[fm * 4 + e] = (_Float16)v[e];
+                    }
+                    if constexpr (HS) {
+                        if (fm == 1 && ok) store_out(through, reinterpret_cast<half8_t*>(out + at), hv);
+                    } else {
+                        if (ok) store_out(through, reinterpret_cast<f32x4_t*>(out + at + fm * CHF), v);
+                    }
+                }
+            }
+        };
+        lds_barrier();   // the first window is staged
+        for (int tile = group, before = -1;; before = tile, tile += step) {   // (the tile that the other waves are on, the one before it)
+            const bool more = tile < ntiles, next = tile + step < ntiles;
+            if (next) fetch(tile + step);
+            if (before >= 0) multiply();
+            if (next) convert();
+            if (more) lds_barrier();   // the first layer is through: the window's place is free
+            if (next) put();
+            if (before >= 0) finish(before);
+            if (!more) break;
+            lds_barrier();   // the window is staged, the tensor in between is there
+        }
+        if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 4);
+        return;
     }
-    // ------------------------------------------------------------------------------------ MFMA waves
-    const int mq = lane & 15, kq = lane >> 4, w = wave - 4;
-    const unsigned wlane = lane * 16;
-    __builtin_amdgcn_s_setprio(2);   // (the staging wave on this SIMD has time enough in between)
+    // ------------------------------------------------------------- the waves that compute the first layer
     {   // the first layer's weights into LDS, as c4_rows takes them: [pair of steps][fragment][lane]
         constexpr int SHARE = G::NS / 2 * NW / 4;
         i32x4_t v[SHARE];
@@ -171,15 +323,6 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
 #pragma unroll
         for (int i = 0; i < SHARE; i += SMALL ? 2 : 1) *reinterpret_cast<i32x4_t*>(lds + G::WEIGHTS + (w * SHARE + i) * 1024 + wlane) = v[i];
     }
-    float mid_scale = 1.f, inv_mid = 1.f;
-    if (p.in_amax) {
-        const float r0 = range_after_act(range_reduce(range_bits), p.act[0]);
-        (void)range_scale(r0, &inv_in);
-        // (no value of the first layer is larger than its weights' largest row sum allows: a scale for the tensor in between that
-        // does not wait for it.  Such a bound is some ten times what a frame reaches, 2^4 of the 2^14 that the split has to spare)
-        if constexpr (C8) mid_scale = range_scale(range_after_act(r0 * p.gain + p.base, p.act[1]), &inv_mid);
-    }
-    const float mul1 = p.acc_mul[0] * inv_in, mul2 = p.acc_mul[1] * inv_mid;
     // this lane's places: in the window, in the tensor in between (as it writes and as it reads)
     const int x1 = w * 16 + mq;   // column of the first layer's tile
     const unsigned char* const col = lds + x1 * G::PIX + ((x1 & 1) ? G::COPY2 + 8 : 0);
@@ -187,27 +330,8 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     const unsigned char* const ninth_at = col + kq * G::ROW_PITCH + 8 * G::PIX;
     const unsigned char* const last_at = col + 8 * G::ROW_PITCH + 8 * G::PIX;
     unsigned char* const mid_to = lds + G::MID + ((x1 & 1) ? 32 + (x1 >> 1) : x1 >> 1) * G::SLOT + kq * (G::SLOT / 4);   // (its eight channels side by side; the second layer's weights are laid out for that)
-    const int cpair = SMALL ? 0 : w & 1, cfrag = w >> 1;   // of the second layer: 32 channels, 16 columns
-    constexpr int ROWS2 = SMALL ? G::TH2 / 2 : G::TH2;
-    const int row2 = SMALL ? (w & 1) * ROWS2 : 0;          // rows
-    const unsigned char* const mid_at = lds + G::MID + (cfrag * 16 + mq) * G::SLOT + (SMALL ? (kq & 1) * 16 + row2 * 2 * G::MROW : kq * 16);
-    // (buffer loads: the fragment's place is a scalar operand, where 64-bit addresses of all of them would fill the registers)
-    const __amdgpu_buffer_rsrc_t weights2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.wpack[1]), 0, 36 * NPL * 1024, 0x00020000);   // [kx][32 channels][ky][fragment][plane]
-    // SMALL: two taps a step, the lanes of either half of the wave one
-    int tap_at[SMALL ? G::STEPS2 : 1];
-    if constexpr (SMALL) {
-#pragma unroll
-        for (int s = 0; s < G::STEPS2; s++) {
-            const int tap = min(2 * s + (kq >> 1), 8), ky = tap / 3, kx = tap - 3 * ky;
-            tap_at[s] = ky * G::MROW + (kx == 1 ? 32 * G::SLOT : kx * (G::SLOT / 2));
-        }
-        for (int i = w; i < G::STEPS2 * 2 * NPL; i += 4)
-            *reinterpret_cast<i32x4_t*>(lds + G::W2 + i * 1024 + wlane) = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const unsigned char*>(p.wpack[1]) + i * 1024 + wlane);
-    }
-    const float* const sb = reinterpret_cast<const float*>(lds + G::SB);
-    store_t* const out = reinterpret_cast<store_t*>(p.out);
-    const bool through = store_through_pays(p.out, p.h2, p.w2, p.out_cp * ESZ, !p.plain_stores, hw_block_count());
-    bool drop = through && wave == 4 && hw_block_id() < 8;
+    scales();
+    const float mul1 = p.acc_mul[0] * inv_in;
     const float lo1 = p.act[1].kind == ACT_NONE ? -3.0e38f : p.act[1].kind == ACT_RELU ? 0.f : p.act[1].lo * mid_scale;   // (its values carry the scale)
     const float hi1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 3.0e38f : p.act[1].hi * mid_scale;
     const float leak1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 0.f : p.act[1].leak;
@@ -220,20 +344,8 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     for (int d = 0; d < C4Ring<G>::LW; d++)
 #pragma unroll
         for (int k = 0; k < NW; k += SMALL ? 2 : 1) rows_put_w(ring.a0[d], ring.a2[d], k, *reinterpret_cast<const i32x4_t*>(lds + G::WEIGHTS + (d * NW + k) * 1024 + wlane));
-    float vmax = 0.f;
     for (int tile = group;;) {
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
-        half8_t wq[SMALL ? 1 : 2][3][2][NPL];   // the second layer's weights of a column of taps, two columns
-        typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-        auto load_w = [&](int set, int kx) __attribute__((always_inline)) {
-#pragma unroll
-            for (int ky = 0; ky < 3; ky++)
-#pragma unroll
-                for (int fm = 0; fm < 2; fm++)
-#pragma unroll
-                    for (int pl = 0; pl < NPL; pl++)
-                        wq[set][ky][fm][pl] = __builtin_bit_cast(half8_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(weights2, wlane, (unsigned)(((kx * 2 + cpair) * 6 + ky * 2 + fm) * NPL + pl) * 1024u, 0));
-        };
         {   // ---- first layer ----
             f32x4_t acc[FM][FN];
 #pragma unroll
@@ -250,6 +362,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             }
             c4_rows<G, false>(acc, ring, rows_at, ninth_at, last_at, rows_at, lds + G::WEIGHTS + wlane);
             __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();   // the window's place is free, and nobody reads the tensor in between any more
             f32x4_t scm[FM], bi[FM];
 #pragma unroll
             for (int fm = 0; fm < FM; fm++) {
@@ -259,10 +372,10 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             const int px = txi * 2 * G::TW2 - 1 + x1;
             const bool x_ok = (unsigned)px < (unsigned)p.w;
             typedef typename std::conditional<SMALL, half4_t, half8_t>::type piece_t;
-            auto leave = [&](auto general_, auto first_, auto end_) __attribute__((always_inline)) {   // (general: an activation other than none, a clamp exact on halves, or a clamp)
+            auto leave = [&](auto general_) __attribute__((always_inline)) {   // (general: an activation other than none, a clamp exact on halves, or a clamp)
                 constexpr bool GENERAL = decltype(general_)::value;
 #pragma unroll
-                for (int r = decltype(first_)::value; r < decltype(end_)::value; r++) {
+                for (int r = 0; r < FN; r++) {
                     // (positions outside the layer's output are its zero padding)
                     const bool ok = x_ok && (unsigned)(tyi * 2 * G::TH2 - 1 + r) < (unsigned)p.h;
                     unsigned char* const to = mid_to + r * G::MROW;
@@ -309,16 +422,10 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                     if (!SMALL || r % 3 == 2) __builtin_amdgcn_sched_barrier(0);   // (four values are too few chains of dependent instructions)
                 }
             };
-            auto rows = [&](auto first, auto end) __attribute__((always_inline)) {
-                if (x1 < 63) {   // (the 64th column belongs to nobody)
-                    if (HS ? !packed1 : leak1 != 0.f) leave(std::integral_constant<bool, true>(), first, end);
-                    else leave(std::integral_constant<bool, false>(), first, end);
-                }
-            };
-            constexpr int FIRST = 5;
-            rows(std::integral_constant<int, 0>(), std::integral_constant<int, FIRST>());
-            if constexpr (!SMALL) load_w(0, 0);   // (the second layer's first weights, into registers that the rows so far have left)
-            rows(std::integral_constant<int, FIRST>(), std::integral_constant<int, FN>());
+            if (x1 < 63) {   // (the 64th column belongs to nobody)
+                if (HS ? !packed1 : leak1 != 0.f) leave(std::integral_constant<bool, true>());
+                else leave(std::integral_constant<bool, false>());
+            }
             if (p.clamp && (txi == 0 || tyi == 0)) {   // what lies above or to the left of the layer's output repeats its first row and column
                 if (txi == 0 && x1 == 0)
                     for (int i = 0; i < FN * NPL; i++) {
@@ -329,93 +436,10 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                     for (int pl = 0; pl < NPL; pl++) *reinterpret_cast<piece_t*>(mid_to + pl * G::MPLANE) = *reinterpret_cast<const piece_t*>(mid_to + pl * G::MPLANE + G::MROW);
             }
         }
-        lds_barrier();   // the tensor in between is there
-        {   // ---- second layer: rows 2 r + ky, columns 2 c + kx ----
-            f32x4_t acc[2][ROWS2];
-#pragma unroll
-            for (int fm = 0; fm < 2; fm++)
-#pragma unroll
-                for (int r = 0; r < ROWS2; r++) acc[fm][r] = (f32x4_t)(0.f);
-            constexpr int AHEAD = 3, Q = SMALL ? G::STEPS2 * ROWS2 : 3 * FN;
-            half8_t b[AHEAD + 1][NPL], w2[SMALL ? G::STEPS2 : 1][2][NPL];
-            auto request = [&](int q) __attribute__((always_inline)) {
-                const int kx = q / FN, j = q % FN;
-                const unsigned char* const at = mid_at + (SMALL ? tap_at[SMALL ? q / ROWS2 : 0] + q % ROWS2 * 2 * G::MROW : (kx == 1 ? 32 * G::SLOT : kx * (G::SLOT / 2)) + j * G::MROW);
-#pragma unroll
-                for (int pl = 0; pl < NPL; pl++) b[q % (AHEAD + 1)][pl] = *reinterpret_cast<const half8_t*>(at + pl * G::MPLANE);
-            };
-#pragma unroll
-            for (int q = 0; q < AHEAD; q++) request(q);
-            auto weights2_of = [&](int s) __attribute__((always_inline)) {
-#pragma unroll
-                for (int i = 0; i < 2 * NPL; i++) w2[SMALL ? s : 0][i / NPL][i % NPL] = *reinterpret_cast<const half8_t*>(lds + G::W2 + (s * 2 * NPL + i) * 1024 + wlane);
-            };
-            if constexpr (SMALL) weights2_of(0);
-#pragma unroll
-            for (int q = 0; q < Q; q++) {
-                if (q + AHEAD < Q) request(q + AHEAD);
-                if constexpr (SMALL) {
-                    if (q % ROWS2 == 0 && q / ROWS2 + 1 < G::STEPS2) weights2_of(q / ROWS2 + 1);
-#pragma unroll
-                    for (int i = 0; i < NPASS; i++)
-#pragma unroll
-                        for (int fm = 0; fm < 2; fm++)
-                            acc[fm][q % ROWS2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w2[q / ROWS2][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][q % ROWS2], 0, 0, 0);
-                } else {
-                    const int kx = q / FN, j = q % FN;
-                    if (j == 0 && kx + 1 < 3) load_w((kx + 1) & 1, kx + 1);
-#pragma unroll
-                    for (int i = 0; i < NPASS; i++)
-#pragma unroll
-                        for (int ky = 0; ky < 3; ky++) {
-                            if (((j - ky) & 1) || j < ky || (j - ky) / 2 >= G::TH2) continue;
-#pragma unroll
-                            for (int fm = 0; fm < 2; fm++)
-                                acc[fm][(j - ky) / 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wq[kx & 1][ky][fm][i == 1 ? NPL - 1 : 0], b[q % (AHEAD + 1)][i == 2 ? NPL - 1 : 0], acc[fm][(j - ky) / 2], 0, 0, 0);
-                        }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (drop) {   // (ahead of this workgroup's first store: what it has read so far may go as well)
-                drop_clean_l2_lines();
-                drop = false;
-            }
-            f32x4_t sc[2], bi[2];
-#pragma unroll
-            for (int fm = 0; fm < 2; fm++) {
-                sc[fm] = *reinterpret_cast<const f32x4_t*>(sb + 64 + cpair * 32 + kq * CHK + fm * CHF) * mul2;
-                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 128 + cpair * 32 + kq * CHK + fm * CHF);
-            }
-            const int c2 = cfrag * 16 + mq, ox = txi * G::TW2 + c2, ch0 = cpair * 32 + kq * CHK;
-#pragma unroll
-            for (int r = 0; r < ROWS2; r++) {
-                const int oy = tyi * G::TH2 + row2 + r;
-                const bool inside = c2 < G::TW2 && ox < p.w2 && oy < p.h2;
-                const size_t at = ((size_t)(p.out_off + oy) * p.out_wp + p.out_off + ox) * p.out_cp + ch0;
-                half8_t hv;
-#pragma unroll
-                for (int fm = 0; fm < 2; fm++) {
-                    const bool ok = inside && ch0 + (HS ? 0 : fm * CHF) < p.out_cp;
-                    f32x4_t v;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        v[e] = acc[fm][r][e] * sc[fm][e] + bi[fm][e];
-                        if constexpr (!HS) vmax = fmaxf(vmax, ok ? fabsf(v[e]) : 0.f);
-                        else hv[fm * 4 + e] = (_Float16)v[e];
-                    }
-                    if constexpr (HS) {
-                        if (fm == 1 && ok) store_out(through, reinterpret_cast<half8_t*>(out + at), hv);
-                    } else {
-                        if (ok) store_out(through, reinterpret_cast<f32x4_t*>(out + at + fm * CHF), v);
-                    }
-                }
-            }
-        }
+        lds_barrier();   // the tensor in between is there, and the next window
         tile += step;
-        if (tile >= ntiles) break;
-        lds_barrier();   // the next window is staged, and nobody reads the tensor in between any more
+        if (tile >= ntiles) return;
     }
-    if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 4);
 }
 }  // namespace
 
