@@ -23,6 +23,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <type_traits>
 
 #include "kernels.h"
@@ -36,6 +37,7 @@ namespace {
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 
 constexpr int RING = 16;   // input rows resident per strip: K + 3 in use by a round, 4 being staged (K <= 9)
@@ -54,15 +56,16 @@ struct Raw8;
 template <>
 struct Raw8<float> {
     float4 a, b;
-    __device__ __forceinline__ void zero() { a = b = float4{0.f, 0.f, 0.f, 0.f}; }
-    __device__ __forceinline__ void load(const float* src) { a = *reinterpret_cast<const float4*>(src); b = *reinterpret_cast<const float4*>(src + 4); }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t row, int at) {
+        a = __builtin_bit_cast(float4, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(row, at, 0, 0));
+        b = __builtin_bit_cast(float4, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(row, at, 16, 0));
+    }
     __device__ __forceinline__ void get(float* v) const { v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w; }
 };
 template <>
 struct Raw8<_Float16> {
     half8_t h;
-    __device__ __forceinline__ void zero() { h = (half8_t)((_Float16)0.f); }
-    __device__ __forceinline__ void load(const _Float16* src) { h = *reinterpret_cast<const half8_t*>(src); }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t row, int at) { h = __builtin_bit_cast(half8_t, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128(row, at, 0, 0)); }
     __device__ __forceinline__ void get(float* v) const {
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = (float)h[i];
@@ -133,33 +136,36 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
 
     // ---- staging: q row j (relative to y_begin) is stored input row in_y0 + y_begin + j ----
     const TIn* in = reinterpret_cast<const TIn*>(p.in);
-    const int stid = tid & 255;
     // Four rows at a time: ITEMS items per row dealt to the 256 staging threads.  fetch() issues the loads of a batch
     // into registers, store() converts and writes them into the ring; a batch is fetched one round before it is stored.
     // (The rows of the first round are dealt to all 512 threads: the MFMA waves have nothing else to do until they are in.)
+    // A thread has the same column and channels in every batch, and a wave's items lie in one row: what depends on the row is
+    // scalar, a buffer's limits stand for the frame's (what lies outside reads as zeros), and an item is its loads and nothing
+    // else.  With an address and a condition per item a batch took 1.2 to 1.7k clocks of a staging wave, 4.9k a round.
+    static_assert(ITEMS % 64 == 0 && 256 % ITEMS == 0, "a wave's items lie in one row");
     constexpr int PER = (4 * ITEMS + 255) / 256;   // items per thread and batch
-    auto fetch = [&](auto& bt, int j_first, int nrows, int t, int nthreads) {
-        constexpr int N = sizeof(bt.dst) / sizeof(int);
+    const int s_col = (tid % ITEMS) / NCH, s_chunk = tid % NCH;
+    const int s_ring = ring_off<CS>(s_col, s_chunk);
+    int s_at;   // byte of the row
+    {
+        // (coordinates in the frame of repeated pixels, which is the stored frame unless the step is fractional)
+        const int vwp = p.in_wp << p.in_shift;
+        int gx = p.in_x0 + x0 + s_col;
+        if (p.in_clamp) gx = min(max(gx, 0), vwp - 1);
+        s_at = (unsigned)gx < (unsigned)vwp && s_chunk * 8 < p.in_cp ? ((gx >> p.in_shift) * p.in_cp + s_chunk * 8) * (int)sizeof(TIn) : INT_MIN;
+    }
+    const int row_bytes = p.in_wp * p.in_cp * (int)sizeof(TIn);
+    auto fetch = [&](auto& bt, int j_first, int nrows, auto nwaves_, int w) {   // (wave w of the nwaves that the batch is dealt to)
+        constexpr int N = sizeof(bt.dst) / sizeof(int), NWAVES = decltype(nwaves_)::value;
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            const int idx = i * nthreads + t;
-            bt.dst[i] = -1;
-            bt.v[i].zero();
-            if (idx < nrows * ITEMS) {
-                const int jr = idx / ITEMS, it = idx - jr * ITEMS;
-                const int col = it / NCH, chunk = it - col * NCH;
-                const int j = j_first + jr;
-                // (coordinates in the frame of repeated pixels, which is the stored frame unless the step is fractional)
-                int gy = p.in_y0 + y_begin + j, gx = p.in_x0 + x0 + col;
-                const int vhp = p.in_hp << p.in_shift, vwp = p.in_wp << p.in_shift;
-                if (p.in_clamp) {
-                    gy = min(max(gy, 0), vhp - 1);
-                    gx = min(max(gx, 0), vwp - 1);
-                }
-                bt.dst[i] = (j & (RING - 1)) * ROWB + ring_off<CS>(col, chunk);
-                if ((unsigned)gy < (unsigned)vhp && (unsigned)gx < (unsigned)vwp && chunk * 8 < p.in_cp)
-                    bt.v[i].load(in + ((size_t)(gy >> p.in_shift) * p.in_wp + (gx >> p.in_shift)) * p.in_cp + chunk * 8);
-            }
+            const int jr = (i * NWAVES + w) * 64 / ITEMS, j = j_first + jr, vhp = p.in_hp << p.in_shift;
+            int gy = p.in_y0 + y_begin + j;
+            if (p.in_clamp) gy = min(max(gy, 0), vhp - 1);
+            const bool ok = jr < nrows && (unsigned)gy < (unsigned)vhp;
+            const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(const_cast<TIn*>(in) + (size_t)(ok ? gy >> p.in_shift : 0) * p.in_wp * p.in_cp, 0, ok ? row_bytes : 0, 0x00020000);
+            bt.dst[i] = jr < nrows ? (j & (RING - 1)) * ROWB : -1;
+            bt.v[i].load(row, s_at);
         }
     };
     // (fp32 tensors: the activation's kind chosen once per call and the hi/lo split in four instructions per pair of values,
@@ -177,8 +183,8 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
                     bt.v[i].get(r);
                     half8_t hi, lo;
                     split8<KIND>(r, true, p.act, in_scale, hi, lo);
-                    *reinterpret_cast<half8_t*>(ring + bt.dst[i]) = hi;
-                    *reinterpret_cast<half8_t*>(ring + bt.dst[i] + PLANE) = C8 ? c8_plane(hi, lo) : lo;
+                    *reinterpret_cast<half8_t*>(ring + bt.dst[i] + s_ring) = hi;
+                    *reinterpret_cast<half8_t*>(ring + bt.dst[i] + s_ring + PLANE) = C8 ? c8_plane(hi, lo) : lo;
                 }
             };
             if (act_kind_ == ACT_RELU) split_all(std::integral_constant<int, ACT_RELU>());
@@ -199,7 +205,7 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
 #pragma unroll
                     for (int e = 0; e < 8; e++) v[e] = (_Float16)act1r(r[e], p.act);
                 }
-                *reinterpret_cast<half8_t*>(ring + bt.dst[i]) = v;
+                *reinterpret_cast<half8_t*>(ring + bt.dst[i] + s_ring) = v;
             }
         }
     };
@@ -214,12 +220,12 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
         // the first round's rows, all threads: every load is issued before the first conversion
         constexpr int PER0 = (NB0 * 4 * ITEMS + 511) / 512;
         RowBatch<TIn, PER0> first;
-        fetch(first, 0, min(4 * NB0, rows_total), tid, 512);
+        fetch(first, 0, min(4 * NB0, rows_total), std::integral_constant<int, 8>(), wave);
         store(first);
     }
     // (the batch of the second round is requested once the first round's rows are in: every workgroup of the
     // launch is in this phase at the same time, and it is bound by memory bandwidth)
-    if (!mfma_wave) fetch(nxt, 4 * NB0, NB0 < nbatches ? rows_of(NB0) : 0, stid, 256);
+    if (!mfma_wave) fetch(nxt, 4 * NB0, NB0 < nbatches ? rows_of(NB0) : 0, std::integral_constant<int, 4>(), wave & 3);
     // ---- weights: one fragment per step and plane, in registers from here on (placed behind the staging code so that
     //      the two never hold registers at the same point) ----
     // (fp8 form: the fp16 hi fragment of every step, and per input row the fp8 operands of channels 16g .. 16g + 15 for
@@ -275,18 +281,85 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
             // write batch NB0 + g (fetched a round ago; no round up to g reads its ring slots), fetch the next one
             store(nxt);
             const int b = NB0 + g + 1;
-            fetch(nxt, 4 * b, b < nbatches ? rows_of(b) : 0, stid, 256);
+            fetch(nxt, 4 * b, b < nbatches ? rows_of(b) : 0, std::integral_constant<int, 4>(), wave & 3);
             lds_barrier();
         }
         return;
     }
     float vmax = 0.f;   // largest magnitude this lane wrote
+    // out[y][x][o] = sum_kx q[x + kx][o*K + kx]: one output column per lane, from the wave's area, while the matrix pipe is on
+    // the next round's row: one kx per input row, its four values added a row behind their request (channels beyond cout read
+    // some row of the column and are discarded below).  Summed behind the row's own matrix instructions it took 0.7k of a
+    // round's 4.2k clocks.
+    static_assert(OW <= 64, "a lane holds one output column");
+    const float* const column = scratch + min(lane, OW - 1) * sp;
+    float a[4], qv[2][4];
+    auto request = [&](int kx) __attribute__((always_inline)) {
+#pragma unroll
+        for (int o = 0; o < 4; o++) qv[kx & 1][o] = column[kx * sp + ((o * K + kx < 28) ? o * K + kx : 27)];
+    };
+    auto add = [&](int kx) __attribute__((always_inline)) {
+#pragma unroll
+        for (int o = 0; o < 4; o++) a[o] = kx == 0 ? qv[0][o] : a[o] + qv[kx & 1][o];
+    };
+    auto sum_step = [&](int kx) __attribute__((always_inline)) {
+        request(kx);
+        if (kx > 0) add(kx - 1);
+    };
+    auto finish = [&](int y) __attribute__((always_inline)) {
+        add(K - 1);
+        const int x = lane, gx = x0 + x;
+        if (x >= OW || gx >= p.out_w) return;
+        float rv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (res) {
+            const TOut* rp = res + ((size_t)(p.res_off_y + y) * p.res_wp + p.res_off_x + gx) * p.res_cp;
+            if (sizeof(TOut) == 4) {
+                const float4 r4 = *reinterpret_cast<const float4*>(rp);
+                rv[0] = r4.x; rv[1] = r4.y; rv[2] = r4.z; rv[3] = r4.w;
+            } else {
+                const half4_t r4 = *reinterpret_cast<const half4_t*>(rp);
+#pragma unroll
+                for (int o = 0; o < 4; o++) rv[o] = (float)r4[o];
+            }
+            // (all of it in here: where the paths meet again nothing waits for memory, or every row would wait for the stores of
+            // the row before it)
+#pragma unroll
+            for (int o = 0; o < 4; o++) {
+                if (p.res_relu) rv[o] = fmaxf(rv[o], 0.f);
+                if (p.res_scale) rv[o] *= sc4[o];
+            }
+        }
+        f32x4_t v;
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+            v[o] = o < p.cout ? ((a[o] * acc_mul) * sc4[o] + bi4[o]) + rv[o] : 0.f;
+            vmax = fmaxf(vmax, fabsf(v[o]));
+        }
+        if (p.post_fn != FFN_COPY) {   // (what the layer behind would have read, and its own arithmetic)
+#pragma unroll
+            for (int o = 0; o < 4; o++) {
+                float x = sizeof(TOut) == 4 ? v[o] : (float)(_Float16)v[o];
+                if (p.post_act.kind != ACT_NONE) x = fminf(p.post_act.hi, fmaxf(p.post_act.lo, x)) + p.post_act.leak * fminf(x, 0.f);
+                x = p.post_fn == FFN_SIGMOID ? sigmoid1(x) : tanh1(x);
+                v[o] = o < p.cout ? x : 0.f;
+            }
+        }
+        const size_t oidx = ((size_t)(p.out_off_y + y) * p.out_wp + p.out_off_x + gx) * p.out_cp;
+        if (sizeof(TOut) == 4) {
+            *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + oidx) = v;
+        } else {
+            half4_t hv;
+#pragma unroll
+            for (int o = 0; o < 4; o++) hv[o] = (_Float16)v[o];
+            *reinterpret_cast<half4_t*>(reinterpret_cast<_Float16*>(out) + oidx) = hv;
+        }
+    };
     for (int g = 0; g < nrounds; g++) {
         {
             const int yl = 4 * g + wave;          // output row relative to y_begin
-            const int y = y_begin + yl;
-            if (y < y_end) {
-                float16_t acc[FN];
+            const bool here = y_begin + yl < y_end;
+            float16_t acc[FN];
+            if (here) {
 #pragma unroll
                 for (int fn = 0; fn < FN; fn++)
 #pragma unroll
@@ -312,6 +385,7 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
                     }
 #pragma unroll
                     for (int ky = 0; ky < K; ky++) {
+                        sum_step(ky);
 #pragma unroll
                         for (int sub = 0; sub < CS; sub++)
 #pragma unroll
@@ -343,6 +417,7 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
                 constexpr int NMF = FN * (SPLIT ? 3 : 1), NDS = FN * NPL;
 #pragma unroll
                 for (int t = 0; t < NSTEPS; t++) {
+                    if (t % CS == 0) sum_step(t / CS);
                     const int kyn = (t + 1) / CS, subn = (t + 1) % CS;
                     const unsigned char* rown = ring + ((yl + kyn) & (RING - 1)) * ROWB;
 #pragma unroll
@@ -359,6 +434,12 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
                     }
                 }
                 }
+            } else {
+#pragma unroll
+                for (int kx = 0; kx < K; kx++) sum_step(kx);
+            }
+            if (g > 0) finish(y_begin + yl - 4);   // (the rounds before the last one have all their rows)
+            if (here) {
                 // accumulators -> this wave's area [column][virtual channel]: a lane holds column lane%32 of each
                 // fragment and rows 8*(r/4) + 4*(lane/32) + r%4
 #pragma unroll
@@ -372,67 +453,14 @@ __global__ __launch_bounds__(512) void conv_rows_kernel(const ConvRowsParams p) 
                             for (int e = 0; e < 4; e++) dstp[e] = acc[fn][q * 4 + e];
                         }
                     }
-                // out[y][x][o] = sum_kx q[x + kx][o*K + kx]: one output column per lane
-                for (int x = lane; x < OW; x += 64) {
-                    const int gx = x0 + x;
-                    if (gx >= p.out_w) break;
-                    // all K*4 reads are issued before the first sum (a read under a condition would cost one LDS round
-                    // trip each); channels beyond cout read some row of the column and are discarded below
-                    float qv[K][4];
-#pragma unroll
-                    for (int kx = 0; kx < K; kx++) {
-                        const float* qp = scratch + (x + kx) * sp;
-#pragma unroll
-                        for (int o = 0; o < 4; o++) qv[kx][o] = qp[(o * K + kx < 28) ? o * K + kx : 27];
-                    }
-                    float a[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int kx = 0; kx < K; kx++)
-#pragma unroll
-                        for (int o = 0; o < 4; o++) a[o] += qv[kx][o];
-                    float rv[4] = {0.f, 0.f, 0.f, 0.f};
-                    if (res) {
-                        const TOut* rp = res + ((size_t)(p.res_off_y + y) * p.res_wp + p.res_off_x + gx) * p.res_cp;
-                        if (sizeof(TOut) == 4) {
-                            const float4 r4 = *reinterpret_cast<const float4*>(rp);
-                            rv[0] = r4.x; rv[1] = r4.y; rv[2] = r4.z; rv[3] = r4.w;
-                        } else {
-                            const half4_t r4 = *reinterpret_cast<const half4_t*>(rp);
-#pragma unroll
-                            for (int o = 0; o < 4; o++) rv[o] = (float)r4[o];
-                        }
-                    }
-                    f32x4_t v;
-#pragma unroll
-                    for (int o = 0; o < 4; o++) {
-                        float r = rv[o];
-                        if (p.res_relu) r = fmaxf(r, 0.f);
-                        if (p.res_scale) r *= sc4[o];
-                        v[o] = o < p.cout ? ((a[o] * acc_mul) * sc4[o] + bi4[o]) + r : 0.f;
-                        vmax = fmaxf(vmax, fabsf(v[o]));
-                    }
-                    if (p.post_fn != FFN_COPY) {   // (what the layer behind would have read, and its own arithmetic)
-#pragma unroll
-                        for (int o = 0; o < 4; o++) {
-                            float x = sizeof(TOut) == 4 ? v[o] : (float)(_Float16)v[o];
-                            if (p.post_act.kind != ACT_NONE) x = fminf(p.post_act.hi, fmaxf(p.post_act.lo, x)) + p.post_act.leak * fminf(x, 0.f);
-                            x = p.post_fn == FFN_SIGMOID ? sigmoid1(x) : tanh1(x);
-                            v[o] = o < p.cout ? x : 0.f;
-                        }
-                    }
-                    const size_t oidx = ((size_t)(p.out_off_y + y) * p.out_wp + p.out_off_x + gx) * p.out_cp;
-                    if (sizeof(TOut) == 4) {
-                        *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + oidx) = v;
-                    } else {
-                        half4_t hv;
-#pragma unroll
-                        for (int o = 0; o < 4; o++) hv[o] = (_Float16)v[o];
-                        *reinterpret_cast<half4_t*>(reinterpret_cast<_Float16*>(out) + oidx) = hv;
-                    }
-                }
             }
         }
         lds_barrier();   // the round's rows are consumed, the next round's rows are in the ring
+    }
+    if (y_begin + 4 * (nrounds - 1) + wave < y_end && nrounds > 0) {
+#pragma unroll
+        for (int kx = 0; kx < K; kx++) sum_step(kx);
+        finish(y_begin + 4 * (nrounds - 1) + wave);
     }
     if (SPLIT && p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 4);
 }
