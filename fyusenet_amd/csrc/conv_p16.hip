@@ -941,6 +941,256 @@ __global__ __launch_bounds__(512) void tconv_p16_kernel(const ConvP16Params p) {
     if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 4);
 }
 
+// The same layer with two groups of four waves that take tiles in turn: while one group computes a tile the other one stores
+// the tile before and brings the window of the tile behind into its own half of the LDS (all NCH chunks of it).  In the form
+// above the waves that compute also store, one after the other, and nothing is on its way to memory while they compute: of 113
+// us for 64 -> 32 channels at 960x540 (fp32 tensors) 57 go when the stores go, and 50 are left when the loads go too, where 400 MB
+// take 78 us.  The weights lie in LDS: a wave that loads them waits behind the stores of the other group, which leave through
+// the same path (6x8 tiles on fp32 tensors, which leave no room for them: 110 us).  Bound: memory.  64 -> 32 channels, us, the
+// other form and this one: fp32 960x540 116 and 100, 256x312 18.5 and 16 (2x8 tiles); fp16 762x928 71 and 61.5 (6x8 tiles).
+// 32 channels gain nothing (fp16 322x242 10.4 and 10.5), 128 leave no room for their weights (tiles of 4x8 and 8x4: slower).
+template <class G, int NCH, int PDT>
+__device__ __forceinline__ void tp16_tile(f32x4_t (&acc)[4][2][G::FN], half8_t (&a_q)[PDT][2][NPL], const int (&bbase)[G::FN], const unsigned char* lds,
+                                          const unsigned char* weights) {
+    constexpr int FN = G::FN, STEPS = NT * NCH;
+    half8_t b[2][FN][NPL];
+#pragma unroll
+    for (int fn = 0; fn < FN; fn++)
+#pragma unroll
+        for (int pl = 0; pl < NPL; pl++) b[0][fn][pl] = *reinterpret_cast<const half8_t*>(lds + bbase[fn] + G::ROW_PITCH + PITCH + pl * G::PLANE);
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const int t = s % NT, d = s % PDT, dprev = (d + PDT - 1) % PDT;
+        const int sh = tt_shift(t), set = sh & 1, par = tt_parity(t), nsh = (sh + 1) & 3;
+        const int noff = ((t == NT - 1) ? s / NT + 1 : s / NT) * G::BUF + (1 - (nsh >> 1)) * G::ROW_PITCH + (1 - (nsh & 1)) * PITCH;
+        constexpr int SL = 2 * NPASS, NS = SL * FN, NW = 2 * NPL;
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            const int fn = i / SL, r = i % SL, kind = r / 2, fm = r % 2;
+            const int apl = (kind == 1) ? 1 : 0, bpl = (kind == 2) ? 1 : 0;
+            acc[par][fm][fn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_q[d][fm][apl], b[set][fn][bpl], acc[par][fm][fn], 0, 0, 0);
+            if (tt_last_of_shift(t) && s + 1 < STEPS && i < NPL * FN)
+                b[1 - set][i / NPL][i % NPL] = *reinterpret_cast<const half8_t*>(lds + bbase[i / NPL] + noff + (i % NPL) * G::PLANE);
+#pragma unroll
+            for (int j = 0; j < NW; j++)   // the weight fragments of a step, spread over its slots
+                if (s + PDT - 1 < STEPS && i == ((j * NS) / NW + 1 < NS ? (j * NS) / NW + 1 : NS - 1))
+                    a_q[dprev][j % 2][j / 2] = *reinterpret_cast<const half8_t*>(weights + ((s + PDT - 1) * 2 * NPL + (j % 2) * NPL + j / 2) * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+template <int TH, int TW, int NCH>
+__global__ __launch_bounds__(512) void tconv_p16x2_kernel(const ConvP16Params p) {
+    using G = Geo<TH, TW, 1, 1, 1>;
+    constexpr int FN = G::FN, CPB = G::CPB, NB = G::NB, PDT = 3;
+    extern __shared__ __align__(16) unsigned char lds_all[];
+    __shared__ unsigned range_box[2];
+    if (blockIdx.x == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
+    const int tid = threadIdx.x, lane = tid & 63, stid = tid & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2;
+    int bid = blockIdx.x;
+    {
+        const int nblk = p.pos_groups * p.cout_blocks;
+        const int per = nblk >> 3;
+        if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+    }
+    const int cb = bid % p.cout_blocks;
+    const int group = bid / p.cout_blocks;
+    const int ntiles = p.tiles_x * p.tiles_y;
+    if (tid < 2) range_box[tid] = 0u;
+    const unsigned range_bits = p.in_amax ? range_load(p.in_amax) : 0u;
+    unsigned char* const lds = lds_all + half * NCH * G::BUF;
+    float* const sb = reinterpret_cast<float*>(lds_all + 2 * NCH * G::BUF);
+    // ---- staging: item i of a thread is eight channels of a pixel of the window, the same of every chunk ----
+    const store_t* const in = reinterpret_cast<const store_t*>(p.in);
+    const int g8 = (stid & 3) * 8;
+    struct RawF { float4 a, b; };
+    typedef typename std::conditional<HSTORE, half8_t, RawF>::type raw_t;
+    struct Window {   // (lives where it is fetched and staged, not through the matrix work)
+        raw_t raw[NCH][NB];
+        unsigned inside;
+    };
+    auto fetch = [&](Window& win, int tile) __attribute__((always_inline)) {
+        const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
+        const int y0 = tyi * TH + p.in_y0, x0 = txi * G::TWG + p.in_x0;
+        win.inside = 0u;
+        int sid = stid;
+        asm volatile("" : "+v"(sid));   // (places are worked out here, not kept in registers through the matrix work; below too)
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const int idx = sid + i * 256, pix = idx >> 2, py = pix / G::HW, px = pix - py * G::HW;
+            int gy = y0 + py, gx = x0 + px;
+            if (p.in_clamp) {
+                gy = min(max(gy, 0), p.in_hp - 1);
+                gx = min(max(gx, 0), p.in_wp - 1);
+            }
+            const bool ok = idx < G::NITEMS && (unsigned)gy < (unsigned)p.in_hp && (unsigned)gx < (unsigned)p.in_wp;
+            win.inside |= ok ? 1u << i : 0u;
+            const store_t* const src = in + (ok ? (gy * p.in_wp + gx) * p.in_cp + g8 : 0);
+#pragma unroll
+            for (int c = 0; c < NCH; c++) {
+                if constexpr (HSTORE) {
+                    win.raw[c][i] = *reinterpret_cast<const half8_t*>(src + c * KC);
+                } else {
+                    win.raw[c][i].a = *reinterpret_cast<const float4*>(src + c * KC);
+                    win.raw[c][i].b = *reinterpret_cast<const float4*>(src + c * KC + 4);
+                }
+            }
+        }
+    };
+    float in_scale = 1.f, inv_in_scale = 1.f;
+    auto stage = [&](const Window& win) __attribute__((always_inline)) {
+        auto convert = [&](auto kind_) __attribute__((always_inline)) {
+            constexpr int KIND = decltype(kind_)::value;
+            _Float16 hlo, hhi;
+            const bool half_act = act_half_exact(p.act, hlo, hhi);
+            int sid = stid;
+            asm volatile("" : "+v"(sid));
+#pragma unroll
+            for (int c = 0; c < NCH; c++)
+#pragma unroll
+                for (int i = 0; i < NB; i++) {
+                    const int idx = sid + i * 256, pix = idx >> 2, py = pix / G::HW, px = pix - py * G::HW;
+                    const bool ok = (win.inside >> i) & 1u;
+                    unsigned char* const to = lds + c * G::BUF + py * G::ROW_PITCH + px * PITCH + (idx & 3) * 16;
+                    if constexpr (HSTORE) {
+                        half8_t v;
+                        if (half_act) {
+                            v = ok ? act_half(win.raw[c][i], hlo, hhi) : (half8_t)((_Float16)0.f);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 8; e++) v[e] = ok ? (_Float16)act_p16((float)win.raw[c][i][e], p.act) : (_Float16)0.f;
+                        }
+                        if (idx < G::NITEMS) *reinterpret_cast<half8_t*>(to) = v;
+                    } else {
+                        const float4 r0 = win.raw[c][i].a, r1 = win.raw[c][i].b;
+                        const float r[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+                        half8_t hi, lo;
+                        split8<KIND>(r, ok, p.act, in_scale, hi, lo);
+                        if (idx < G::NITEMS) {
+                            *reinterpret_cast<half8_t*>(to) = hi;
+                            *reinterpret_cast<half8_t*>(to + G::PLANE) = lo;
+                        }
+                    }
+                }
+        };
+        if (HSTORE || p.act.kind == ACT_LEAKY || p.act.kind == ACT_CLIP) convert(std::integral_constant<int, ACT_LEAKY>());
+        else if (p.act.kind == ACT_RELU) convert(std::integral_constant<int, ACT_RELU>());
+        else convert(std::integral_constant<int, ACT_NONE>());
+    };
+    // ---- this wave's part of a tile ----
+    const int mq = lane & 15, kq = lane >> 4;
+    const int wn = wave & 3;
+    int bbase[FN];
+#pragma unroll
+    for (int fn = 0; fn < FN; fn++) {
+        const int m = fn * 16 + mq;
+        const int ty = m / TW, tx = m - ty * TW;
+        bbase[fn] = ty * G::ROW_PITCH + (wn * TW + tx) * PITCH + kq * 16;
+    }
+    unsigned char* const weights = lds_all + 2 * NCH * G::BUF + 2 * CPB * 4 + lane * 16;   // [step][fragment][plane]
+    for (int i = wave; i < NT * NCH * 2 * NPL; i += 8)
+        *reinterpret_cast<half8_t*>(weights + i * 1024) =
+            *reinterpret_cast<const half8_t*>(reinterpret_cast<const unsigned char*>(p.wpack) + ((size_t)(i / (2 * NPL)) * p.mfrags * NPLW + (cb * 2 + i / NPL % 2) * NPLW + i % NPL) * 1024 + lane * 16);
+    half8_t a_q[PDT][2][NPL];
+    store_t* const out = reinterpret_cast<store_t*>(p.out);
+    const bool through = store_through_pays(p.out, 2 * p.npos_y, 2 * p.npos_x, p.out_cp * ESZ, (p.cout_blocks == 1 || (CPB * ESZ) % 128 == 0) && !p.plain_stores, hw_block_count());
+    bool drop = through && wave == 0 && hw_block_id() < 8;
+    float acc_mul = p.acc_mul, vmax = 0.f;
+    f32x4_t acc[4][2][FN];
+    auto finish_tile = [&](int tile) __attribute__((always_inline)) {
+        if (drop) {   // (ahead of this workgroup's first store: what it has read so far may go as well)
+            drop_clean_l2_lines();
+            drop = false;
+        }
+        const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
+        f32x4_t bi[2], scm[2];
+        int q = mq;
+        asm volatile("" : "+v"(q));
+#pragma unroll
+        for (int fm = 0; fm < 2; fm++) {
+            scm[fm] = *reinterpret_cast<const f32x4_t*>(sb + kq * CHK + fm * CHF) * acc_mul;
+            bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + CPB + kq * CHK + fm * CHF);
+        }
+#pragma unroll
+        for (int fn = 0; fn < FN; fn++) {
+            const int m = fn * 16 + q;
+            const int ty = m / TW, tx = wn * TW + (m - ty * TW);
+            const int a = tyi * TH + ty, bx = txi * G::TWG + tx;
+            const bool ok = a < p.npos_y && bx < p.npos_x;
+            const size_t obase = ((size_t)(p.out_off_y + 2 * a) * p.out_wp + p.out_off_x + 2 * bx) * p.out_cp + cb * CPB + kq * CHK;
+            float fmax_ = 0.f;
+#pragma unroll
+            for (int par = 0; par < 4; par++) {
+                const size_t o = obase + ((size_t)(par >> 1) * p.out_wp + (par & 1)) * p.out_cp;
+                half8_t hv;
+#pragma unroll
+                for (int fm = 0; fm < 2; fm++) {
+                    f32x4_t v;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        v[e] = acc[par][fm][fn][e] * scm[fm][e] + bi[fm][e];
+                        if constexpr (!HSTORE) fmax_ = fmaxf(fmax_, fabsf(v[e]));
+                    }
+                    if constexpr (HSTORE) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) hv[fm * 4 + e] = (_Float16)v[e];
+                        if (fm == 1 && ok) store_out(through, reinterpret_cast<half8_t*>(out + o), hv);
+                    } else {
+                        if (ok) store_out(through, reinterpret_cast<f32x4_t*>(out + o + fm * CHF), v);
+                    }
+                }
+            }
+            vmax = fmaxf(vmax, ok ? fmax_ : 0.f);
+        }
+    };
+    int tile = group + half * p.pos_groups;
+    const int step = 2 * p.pos_groups;
+    if (p.in_amax) in_scale = range_scale(range_after_act(range_reduce(range_bits), p.act), &inv_in_scale);
+    acc_mul *= inv_in_scale;
+    if (tid < CPB) {
+        sb[tid] = cb * CPB + tid < p.out_cp ? p.scale[cb * CPB + tid] : 0.f;
+        sb[CPB + tid] = cb * CPB + tid < p.out_cp ? p.bias[cb * CPB + tid] : 0.f;
+    }
+    if (half == 0) {
+        Window win;
+        fetch(win, tile);
+        stage(win);
+    }
+    lds_barrier();   // the first group's first window is staged
+    if (half == 1) {
+        if (tile < ntiles) {
+            Window win;
+            fetch(win, tile);
+            stage(win);
+        }
+        lds_barrier();   // the second group's
+    }
+    // (either group passes two barriers a tile; a group without another tile ends, and the other one goes on by itself)
+    for (; tile < ntiles; tile += step) {
+#pragma unroll
+        for (int par = 0; par < 4; par++)
+#pragma unroll
+            for (int fm = 0; fm < 2; fm++)
+#pragma unroll
+                for (int fn = 0; fn < FN; fn++) acc[par][fm][fn] = (f32x4_t)(0.f);
+#pragma unroll
+        for (int i = 0; i < (PDT - 1) * 2 * NPL; i++) a_q[i / (2 * NPL)][i / NPL % 2][i % NPL] = *reinterpret_cast<const half8_t*>(weights + i * 1024);
+        tp16_tile<G, NCH, PDT>(acc, a_q, bbase, lds, weights);
+        lds_barrier();   // this group's tile is through, the other group's window is staged
+        {
+            const bool next = tile + step < ntiles;
+            Window win;
+            if (next) fetch(win, tile + step);
+            finish_tile(tile);
+            if (next) stage(win);
+        }
+        lds_barrier();   // this group's next window is staged, the other group's tile is through
+    }
+    if (p.out_amax) range_publish_waves(p.out_amax, vmax, range_box, 8);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // K x K convolution (K = 9) on an input of at most four channels (the first layer of a style-transfer net; replaces the
 // render passes of DeepConvLayerNxN::forward, gpu/deep/deepconvlayerNxN.cpp:129-211, for such layers).  A staged pixel
@@ -1837,17 +2087,27 @@ size_t entry_lds(const P16Entry& e, bool residual) {   // (e.buf and e.res_bytes
     return 2 * e.buf + 2 * (size_t)(32 * e.wm) * 4 + (residual ? e.res_bytes : 0);
 }
 struct TP16Entry {
-    int th, tw, wm;
+    int th, tw, wm, two;   // (two: chunks of a form with two groups of waves, 0 for the others)
     p16_fn fn;
-    size_t buf;
+    size_t lds;
 };
 template <int TH, int TW, int WM>
 constexpr TP16Entry tentry() {
-    return TP16Entry{TH, TW, WM, tconv_p16_kernel<TH, TW, WM>, (size_t)Geo<TH, TW, 1, WM, 1>::BUF};
+    return TP16Entry{TH, TW, WM, 0, tconv_p16_kernel<TH, TW, WM>, 2 * (size_t)Geo<TH, TW, 1, WM, 1>::BUF + 2 * 32 * WM * 4};
+}
+// (USED: on tensors of this type; the list is the same for both)
+template <int TH, int TW, int NCH, bool USED>
+constexpr TP16Entry tentry2() {
+    if constexpr (USED) {
+        constexpr size_t lds = 2 * (size_t)NCH * Geo<TH, TW, 1, 1, 1>::BUF + 2 * 32 * 4 + NT * NCH * 2 * NPL * 1024;
+        static_assert(lds <= 160 * 1024 - 64, "fits a CU");
+        return TP16Entry{TH, TW, 1, NCH, tconv_p16x2_kernel<TH, TW, NCH>, lds};
+    } else return TP16Entry{TH, TW, 1, NCH, nullptr, 0};
 }
 const TP16Entry kTEntries[] = {
     tentry<4, 8, 1>(), tentry<8, 4, 1>(), tentry<2, 8, 1>(), tentry<6, 8, 1>(),
     tentry<4, 8, 2>(), tentry<8, 4, 2>(), tentry<2, 8, 2>(), tentry<6, 8, 2>(), tentry<8, 6, 2>(),
+    tentry2<2, 8, 2, !HSTORE>(), tentry2<6, 8, 2, HSTORE>(),
 };
 struct C4Entry {
     int k, th, tw;
@@ -1926,8 +2186,8 @@ bool conv_p16_supported(int k, int stride, int dil, int in_cp, int cout, int out
     return k == 3 && (stride == 1 || stride == 2) && dil == 1 && in_cp % 8 == 0 && in_cp >= 16 && cout >= 8 && out_cp % og == 0 && out_cp >= cout;
 }
 int tconv_p16_tile_count() { return (int)(sizeof(kTEntries) / sizeof(kTEntries[0])); }
-void tconv_p16_tile(int index, int* th, int* tw, int* wm) {
-    *th = kTEntries[index].th; *tw = kTEntries[index].tw; *wm = kTEntries[index].wm;
+void tconv_p16_tile(int index, int* th, int* tw, int* wm, int* two) {
+    *th = kTEntries[index].th; *tw = kTEntries[index].tw; *wm = kTEntries[index].wm; *two = kTEntries[index].two;
 }
 void tconv_p16_tap(int t, int* ky, int* kx) { *ky = TT_KY[t]; *kx = TT_KX[t]; }
 bool tconv_p16_supported(int k, int crop, int in_cp, int in_pad, int cout, int out_cp, bool f16) {
@@ -2083,7 +2343,7 @@ int P16_NAME(launch_conv_p16)(const ConvP16Params& p, hipStream_t s) {
 
 static const TP16Entry* find_tentry(const ConvP16Params& p) {
     for (const TP16Entry& c : kTEntries)
-        if (c.th == p.tile_h && c.tw == p.tile_w && c.wm == p.wm) return &c;
+        if (c.th == p.tile_h && c.tw == p.tile_w && c.wm == p.wm && c.two == (p.two_groups ? p.cin_chunks : 0)) return &c;
     return nullptr;
 }
 size_t P16_NAME(tconv_p16_lds_bytes)(const ConvP16Params& p) {
@@ -2091,7 +2351,7 @@ size_t P16_NAME(tconv_p16_lds_bytes)(const ConvP16Params& p) {
     if (p.f16) return tconv_p16_lds_bytes_half(p);
 #endif
     const TP16Entry* e = find_tentry(p);
-    return e ? 2 * e->buf + 2 * (size_t)(32 * e->wm) * 4 : 0;
+    return e ? e->lds : 0;
 }
 
 // npos_y x npos_x: the input size (positions are input pixels); out_off_*: stored coordinate of output pixel (0, 0)
@@ -2100,7 +2360,7 @@ int P16_NAME(launch_tconv_p16)(const ConvP16Params& p, hipStream_t s) {
     if (p.f16) return launch_tconv_p16_half(p, s);
 #endif
     const TP16Entry* e = find_tentry(p);
-    if (!e) return -1;
+    if (!e || !e->fn) return -1;
     const int cpb = 32 * e->wm, twg = (4 / e->wm) * e->tw;
     if (p.cin_chunks < 1 || p.in_cp != p.cin_chunks * KC || p.cout_blocks < 1 || p.mfrags < p.cout_blocks * 2 * e->wm ||
         p.tiles_x * twg < p.npos_x || p.tiles_y * p.tile_h < p.npos_y || p.out_cp < p.cout_blocks * cpb || (p.out_cp * ESZ) % 16 != 0 || p.res || p.stride != 1 || p.in_shift != 0 ||

@@ -244,6 +244,7 @@ struct ConvP16Params {
     int pos_groups;       // workgroups per block of output channels; workgroup g walks tiles g, g + pos_groups, ...
     int cin_chunks;
     int exact_split;      // launch_conv_p16 on fp32 tensors: three fp16 passes even where the fp8 form of the correction terms would run
+    int two_groups;       // launch_tconv_p16: the form with two groups of waves
     int plain_stores;     // launch_conv_p16, launch_tconv_p16, launch_conv_p16c4: never write the output through (store_through_pays)
     int mfrags;           // cout fragments (16 each) in wpack
     int cout_blocks;      // workgroups along cout (32*wm channels each)
@@ -302,7 +303,7 @@ bool conv_p16c4_uses_fp8(const ConvP16Params& p, int k);   // the same for launc
 // in the order of their input shift (conv_p16.hip: TT_KY / TT_KX)
 bool tconv_p16_supported(int k, int crop, int in_cp, int in_pad, int cout, int out_cp, bool f16);
 int tconv_p16_tile_count();
-void tconv_p16_tile(int index, int* th, int* tw, int* wm);
+void tconv_p16_tile(int index, int* th, int* tw, int* wm, int* two);   // two: chunks of a form with two groups of waves, or 0
 void tconv_p16_tap(int t, int* ky, int* kx);   // kernel tap of step t of a chunk
 size_t tconv_p16_lds_bytes(const ConvP16Params& p);
 int launch_tconv_p16(const ConvP16Params& p, hipStream_t s);

@@ -90,16 +90,16 @@ class TransConvLayer : public Layer {
         q.act = act();
         q.in_amax = tin(0).amax;   // (timed in the form the frame will run)
         q.plain_stores = net->sw.get("FYNHIP_PLAIN_STORES") ? 1 : 0;
-        int want_h = 0, want_w = 0, want_wm = 0;   // FYNHIP_P16_TILE=h,w[,wm] (tests): that combination
-        if (const char* e = net->sw.get("FYNHIP_P16_TILE")) sscanf(e, "%d,%d,%d", &want_h, &want_w, &want_wm);
+        int want_h = 0, want_w = 0, want_wm = 0, want_two = 0;   // FYNHIP_P16_TILE=h,w[,wm[,1: two groups of waves]] (tests): that combination
+        if (const char* e = net->sw.get("FYNHIP_P16_TILE")) sscanf(e, "%d,%d,%d,%d", &want_h, &want_w, &want_wm, &want_two);
         std::vector<ConvP16Params> cands;
         for (int i = 0; i < tconv_p16_tile_count(); i++) {
-            int th, tw, wm;
-            tconv_p16_tile(i, &th, &tw, &wm);
-            if (oc % (32 * wm) != 0) continue;
-            if (want_h && (th != want_h || tw != want_w || (want_wm && wm != want_wm))) continue;
+            int th, tw, wm, two;
+            tconv_p16_tile(i, &th, &tw, &wm, &two);
+            if (oc % (32 * wm) != 0 || (two && two != q.cin_chunks)) continue;
+            if (want_h && (th != want_h || tw != want_w || (want_wm && wm != want_wm) || (two != 0) != (want_two != 0))) continue;
             ConvP16Params c = q;
-            c.tile_h = th; c.tile_w = tw; c.wm = wm;
+            c.tile_h = th; c.tile_w = tw; c.wm = wm; c.two_groups = two ? 1 : 0;
             const int twg = (4 / wm) * tw;
             c.tiles_x = (d.width + twg - 1) / twg; c.tiles_y = (d.height + th - 1) / th;
             c.rcp_tiles_x = 1.0f / (float)c.tiles_x;
@@ -118,7 +118,7 @@ class TransConvLayer : public Layer {
         int pick = 0;
         char key[160];
         snprintf(key, sizeof(key), "tp16:%dx%d:%dx%d:cp%d:h%d", d.in_channels, oc, d.height, d.width, in_v.cp, q.f16);
-        if (!want_h && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return cands[i].tile_h * 1000 + cands[i].tile_w == b && cands[i].wm == c; }, &pick)) {
+        if (!want_h && tune_cache_pick(net, key, cands.size(), always, [&](size_t i, int b, int c) { return cands[i].tile_h * 1000 + cands[i].tile_w == b && cands[i].wm + 10 * cands[i].two_groups == c; }, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float best = 1e30f, t_other = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
@@ -131,10 +131,10 @@ class TransConvLayer : public Layer {
                 t_other = std::min(t_other, time_group(net, group, 10));
             }
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
-                fprintf(stderr, "[tune] transposed 3x3: 16-position fragments (%dx%d tiles, %d channel groups) %.1f us, general kernel %.1f us\n",
-                        cands[pick].tile_h, cands[pick].tile_w, cands[pick].wm, best * 1e3f, t_other * 1e3f);
+                fprintf(stderr, "[tune] transposed 3x3: 16-position fragments (%dx%d tiles, %d channel groups%s) %.1f us, general kernel %.1f us\n",
+                        cands[pick].tile_h, cands[pick].tile_w, cands[pick].wm, cands[pick].two_groups ? ", two groups of waves" : "", best * 1e3f, t_other * 1e3f);
             const bool win = best < t_other;
-            if (!want_h) tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].tile_h * 1000 + cands[pick].tile_w, cands[pick].wm);
+            if (!want_h) tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].tile_h * 1000 + cands[pick].tile_w, cands[pick].wm + 10 * cands[pick].two_groups);
             if (!win && !always) pick = -1;
         }
         if (pick >= 0) {
@@ -229,10 +229,10 @@ class TransConvLayer : public Layer {
     }
     std::string info() const override {
         if (p16) {
-            char buf[220];
-            snprintf(buf, sizeof(buf), "transconv, tconv_p16 %s 4 parities per tile, tile=%dx%d(cout x input pos) waves=%dx%d th=%d tw=%d blocks=%d tiles=%d lds=%zu steps=9 chunks=%d", pp.f16 ? "f16" : "f16x2-split",
+            char buf[260];
+            snprintf(buf, sizeof(buf), "transconv, tconv_p16 %s 4 parities per tile, tile=%dx%d(cout x input pos) waves=%dx%d th=%d tw=%d blocks=%d tiles=%d lds=%zu steps=9 chunks=%d%s", pp.f16 ? "f16" : "f16x2-split",
                      32 * pp.wm, pp.tile_h * pp.tile_w * (4 / pp.wm), pp.wm, 4 / pp.wm, pp.tile_h, pp.tile_w, pp.pos_groups * pp.cout_blocks,
-                     pp.tiles_x * pp.tiles_y * pp.cout_blocks, tconv_p16_lds_bytes(pp), pp.cin_chunks);
+                     pp.tiles_x * pp.tiles_y * pp.cout_blocks, tconv_p16_lds_bytes(pp), pp.cin_chunks, pp.two_groups ? ", two groups of waves" : "");
             return std::string(buf) + (conv_p16_stores_through(pp, 2) ? " stores=through" : "");
         }
         return group.subs.empty() ? "transconv" : "transconv, " + std::to_string(group.subs.size()) + " parities in one launch: " + mfma_info(group.subs[0]);

@@ -973,6 +973,41 @@ def test_transconv_sixteen_position_fragment_form(case, act, storage, monkeypatc
     assert err <= TOL[storage], info
 
 
+TP16_TWO_CASES = [
+    # cin, cout, h, w: two groups of waves with tiles in turn, of 2x32 positions (fp32 tensors) or 6x32 (fp16)
+    (64, 32, 1, 3),           # one tile: the second group has none
+    (64, 32, 6, 33),          # two, or six: an odd row and column in the last
+    (64, 64, 13, 95),         # two blocks of output channels
+    (64, 96, 21, 130),
+    (64, 32, 100, 700),       # 1100 and 374 tiles: workgroups walk four or five, one or two
+    (64, 64, 150, 330),       # 825 and 275 for 128 workgroups a block
+]
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("case", TP16_TWO_CASES, ids=lambda c: "%dx%dx%d_to%d" % (c[0], c[2], c[3], c[1]))
+def test_transconv_with_two_groups_of_waves(case, storage, monkeypatch):
+    """The same layer where one group of waves computes while the other stores and stages: against the oracle, and the same
+    bits as the form with one group (the sums are added in the same order)."""
+    cin, cout, h, w = case
+    tile = "2,8,1" if storage == fa.STORAGE_F32 else "6,8,1"
+    wts = conv_block(1300 + cin + h, cout, 3, cin, bn=True)
+    x = prng.uniform(61 * cin + w, (cin, h, w), -1, 1)
+    outs = []
+    for two in ("", ",1"):
+        b = fa.ConvLayerBuilder(3, "tconv").type(fa.LayerType.TRANSCONVOLUTION2D).number(1).shape(cout, h, w, cin)
+        b.upsample(2).inputPadding(1).outputPadding(2).prefixAct(A.RELU).deep().crop(1).postfixNorm(fa.NormType.BATCHNORM)
+        monkeypatch.setenv("FYNHIP_FORCE_P16_CONV", "1")
+        monkeypatch.setenv("FYNHIP_P16_TILE", tile + two)
+        got, info = run_single(b, storage, [x], wts)
+        assert ("two groups of waves" in info) == (two != "") and "tconv_p16 " in info and "th=%s tw=%s" % tuple(tile.split(",")[:2]) in info, info
+        outs.append(got)
+    ref = oracle_single(b, storage, [x], wts)
+    print("  ", info, "rel_l2=%.3e" % rel_l2(outs[1], ref), flush=True)
+    assert np.array_equal(*outs)
+    assert rel_l2(outs[1], ref) <= TOL[storage], info
+
+
 FRAC_CASES = [
     # k, cin, cout, h, w, step, stride, pad_in, act, kwargs
     (3, 40, 20, 12, 16, 0.5, 2, 0, A.NONE, {}),                   # deconv1 of the reference's style nets (stylenet3x3.cpp:163)
