@@ -278,7 +278,7 @@ __global__ __launch_bounds__(512, HS && M == 4 && SRC == 0 ? 4 : 2) void conv_b1
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     acc0[j][e] = inside ? act(v[e]) : 0.f;
-                    top = fmaxf(top, fabsf(acc0[j][e]));
+                    top = fmaxf(top, inside ? fabsf(v[e]) : 0.f);   // (in front of the activation, whose clamp makes a number of a NaN)
                 }
             }
         }
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(512, HS && M == 4 && SRC == 0 ? 4 : 2) void conv_b1
             if (lane == 0) atomicMax(&box[0], __float_as_uint(top));
             lds_barrier();
             float unused;
-            s = range_scale(__uint_as_float(box[0]), &unused);
+            s = range_scale(range_after_act(__uint_as_float(box[0]), p.act[1]), &unused);
         }
 #pragma unroll
         for (int j = 0; j < OWN; j++) {
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(512, HS && M == 4 && SRC == 0 ? 4 : 2) void conv_b1
     float inv_mid = 1.f, inv_mid2 = 1.f;
     {
         const MidAct act(p.act[2]);
-        if constexpr (!HS) (void)range_scale(__uint_as_float(box[0]), &inv_mid);
+        if constexpr (!HS) (void)range_scale(range_after_act(__uint_as_float(box[0]), p.act[1]), &inv_mid);
         const float mul = p.acc_mul[1] * inv_mid;
         f32x4_t v;
         half4_t hv;
@@ -360,13 +360,13 @@ __global__ __launch_bounds__(512, HS && M == 4 && SRC == 0 ? 4 : 2) void conv_b1
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
+                top = fmaxf(top, pos_ok ? fabsf(v[e]) : 0.f);
                 v[e] = pos_ok ? act(v[e]) : 0.f;
-                top = fmaxf(top, fabsf(v[e]));
             }
             top = range_wave_max(top);
             if (lane == 0) atomicMax(&box[1], __float_as_uint(top));
             lds_barrier();
-            s = range_scale(__uint_as_float(box[1]), &inv_mid2);
+            s = range_scale(range_after_act(__uint_as_float(box[1]), p.act[2]), &inv_mid2);
         }
         if (share == 0) {   // (every wave of a fragment has the sum)
             unsigned char* const to = lds + MID2 + mq * MID_PIT + (mf * 16 + kq * 4) * 2;

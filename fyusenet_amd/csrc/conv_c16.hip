@@ -256,7 +256,7 @@ __global__ __launch_bounds__(N::NT) void conv_c16_kernel(const ConvC16Params p) 
                     float x = __builtin_amdgcn_fmed3f(v, lo, hi);
                     if (leak != 0.f) x += leak * fminf(v, 0.f);
                     sum1[j][e] = ok ? x : 0.f;
-                    top = fmaxf(top, fabsf(sum1[j][e]));
+                    top = fmaxf(top, ok ? fabsf(v) : 0.f);   // (in front of the activation, whose clamp makes a number of a NaN)
                 }
             }
             if constexpr (HS) {
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(N::NT) void conv_c16_kernel(const ConvC16Params p) 
             top = range_wave_max(top);
             if (lane == 0) atomicMax(&box[0], __float_as_uint(top));
             lds_barrier();
-            s = range_scale(__uint_as_float(box[0]), &inv_mid);
+            s = range_scale(range_after_act(__uint_as_float(box[0]), p.act[1]), &inv_mid);
         }
 #pragma unroll
         for (int j = 0; j < N::OWN1; j++) {

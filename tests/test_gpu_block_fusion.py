@@ -194,3 +194,25 @@ def test_bottleneck_weights_loaded_again_and_timed_apart(monkeypatch):
     apart = net.getOutput(net.output_layer)
     net.cleanup()
     assert rel_l2(apart, ref) <= AGREE[fa.STORAGE_F32]
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("kind", ["identity", "projection"])
+def test_nan_stays_in_its_window(kind, storage, monkeypatch):
+    """What a NaN does not reach (one position around it, by the 3x3 layer) is as it is without it, also where no activation
+    drops it in between."""
+    monkeypatch.setenv("FYNHIP_FORCE_BLOCK_FUSION", "1")
+    cin = 256 if kind == "identity" else 64
+    net = Block(storage, cin, 64, 256, 14, 11, kind=kind, act=ActType.NONE, mid_act=ActType.NONE)
+    x, want, infos = run(net)
+    assert together(infos)
+    y = x.copy()
+    y[0, 6, 5] = np.nan
+    net.setInput(y)
+    net.forward()
+    net.finish()
+    got = net.getOutput(net.output_layer)
+    net.cleanup()
+    mask = np.ones(got.shape[1:], bool)
+    mask[5:8, 4:7] = False
+    assert not np.array_equal(got, want) and rel_l2(got[:, mask], want[:, mask]) <= TOL[storage]

@@ -166,3 +166,25 @@ def test_pair_weights_loaded_again_and_timed_apart(monkeypatch):
     apart = net.getOutput(net.output_layer)
     net.cleanup()
     assert rel_l2(apart, ref) <= AGREE[fa.STORAGE_F32]
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows", [2, 4, 6])
+def test_nan_stays_in_its_window(rows, storage, monkeypatch):
+    """What a NaN does not reach (two positions around it) is as it is without it, also where no activation drops it in
+    between."""
+    monkeypatch.setenv("FYNHIP_FORCE_PAIR_FUSION", "1")
+    monkeypatch.setenv("FYNHIP_PAIR_ROWS", str(rows))
+    net = Pair(storage, 40, 40, 24, 33, False, act=ActType.NONE, mid_act=ActType.NONE)
+    x, want, infos = run(net)
+    assert together(infos)
+    y = x.copy()
+    y[0, 12, 16] = np.nan
+    net.setInput(y)
+    net.forward()
+    net.finish()
+    got = net.getOutput(net.output_layer)
+    net.cleanup()
+    mask = np.ones(got.shape[1:], bool)
+    mask[10:15, 14:19] = False
+    assert not np.array_equal(got, want) and rel_l2(got[:, mask], want[:, mask]) <= TOL[storage]
