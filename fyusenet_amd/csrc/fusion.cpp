@@ -541,6 +541,7 @@ void fuse_head_layers(Net* net) {
         // (the form whose weights and schedule the launch takes for the first layer; with fp32 tensors its fp8 correction terms too)
         if (!a->p16 || !a->c4 || a->pp.tile_w != 16 || (!iv.f16 && (!a->tin(0).amax || !conv_p16c4_uses_fp8(a->pp, 9)))) continue;
         if (c->clamp && (iv.pad || mv.pad)) continue;
+        if ((long long)iv.hp() * iv.wp() * iv.cp > (1ll << 30)) continue;   // (32-bit offsets)
         // (positions beside a layer's input are zeros behind its activation as well)
         if (a->act().lo > 0.f || a->act().hi < 0.f || c->act().lo > 0.f || c->act().hi < 0.f) continue;
         const int x = a->in[0];
@@ -628,6 +629,7 @@ void fuse_pair_layers(Net* net) {
         // (positions beside a layer's input are zeros behind its activation as well, or repeat the edge)
         if (!c->clamp && (a->act().lo > 0.f || a->act().hi < 0.f || c->act().lo > 0.f || c->act().hi < 0.f)) continue;
         if (c->clamp && (iv.pad != 0 || mv.pad != 0)) continue;
+        if ((long long)iv.hp() * iv.wp() * iv.cp > (1ll << 30)) continue;   // (32-bit offsets)
         ConvC16Params q{};
         if (c->d.flags & FYN_FLAG_RESIDUAL_INPUT) {
             if (c->in.size() < 2 || c->in[1] < 0 || c->in[1] == c->in[0]) continue;
