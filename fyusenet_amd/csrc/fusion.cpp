@@ -422,6 +422,7 @@ void fuse_block_layers(Net* net) {
     for (auto& kv : net->layers) {
         ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
         if (!c || !block_of(net, c, a, b)) continue;
+        if (a->blk_fused) continue;   // (the last layer of a block in front: its launch writes what this one's first layer would have to compute)
         if (a->dw_fused || a->edw_fused || a->pj_fused || a->pj_into >= 0 || b->bn_fused || c->bn_fused || c->dw_fused || c->edw_fused || c->fn_layer_no >= 0 || c->argmax_tail.idx) continue;
         const TView &iv = a->tin(0).v, &ov = c->tout().v;
         if (iv.f16 != ov.f16 || a->tout().v.f16 != ov.f16 || b->tout().v.f16 != ov.f16 || iv.cp % 8 != 0 || iv.cp < 8 || ov.cp % 4 != 0 || a->d.in_channels > iv.cp || c->oc > ov.cp ||

@@ -216,3 +216,47 @@ def test_nan_stays_in_its_window(kind, storage, monkeypatch):
     mask = np.ones(got.shape[1:], bool)
     mask[5:8, 4:7] = False
     assert not np.array_equal(got, want) and rel_l2(got[:, mask], want[:, mask]) <= TOL[storage]
+
+
+class Chain(Block):
+    """upload -> 1x1 -> 3x3 -> 1x1 -> 3x3 -> 1x1 [-> 3x3 -> 1x1 ...] -> tail -> download: every 1x1 layer in the middle could end a
+    block and begin one."""
+
+    def __init__(self, storage, channels, h, w, blocks):
+        super().__init__(storage, channels, channels, channels, h, w)
+        self.blocks = blocks
+
+    def define(self):
+        h, w, c = self.h, self.w, self.cin
+        self._add(UpDownLayerBuilder(UpDownLayerBuilder.UPLOAD, "upload").number(0).shape(c, h, w, c))
+        self.conv(1, "front", 1, c, c, h, w, 0)
+        self.conv(2, "p0", 1, c, c, h, w, 1, act=ActType.RELU, pad_out=1)
+        last = 2
+        for i in range(1, self.blocks + 1):
+            self.conv(last + 1, "s%d" % i, 3, c, c, h, w, last, act=ActType.RELU)
+            self.conv(last + 2, "p%d" % i, 1, c, c, h, w, last + 1, act=ActType.RELU, pad_out=1 if i < self.blocks else 0)
+            last += 2
+        self.conv(last + 1, "tail", 1, c, c, h, w, last)
+        self.conv(last + 2, "tail2", 1, c, c, h, w, last + 1)
+        self._add(UpDownLayerBuilder(UpDownLayerBuilder.DOWNLOAD, "download").number(last + 3).shape(c, h, w, c).deep())
+        self._edges.append((last + 2, last + 3, 0))
+        self.output_layer = last + 3
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("channels,h,w", [(64, 9, 14), (32, 12, 12)])
+@pytest.mark.parametrize("blocks", [2, 3])
+def test_blocks_that_share_a_layer(blocks, channels, h, w, storage, monkeypatch):
+    """A 1x1 layer that ends one block does not begin the next one: its launch is what writes the tensor between them."""
+    monkeypatch.setenv("FYNHIP_FORCE_BLOCK_FUSION", "1")
+    net = Chain(storage, channels, h, w, blocks)
+    x, got, infos = run(net, passes=2)
+    desc = net.describe()
+    net.cleanup()
+    joined = [n for n in infos if infos[n].startswith("conv_b16")]
+    inside = [n for n in infos if "no launch of its own" in infos[n]]
+    print("  ", joined, inside, flush=True)
+    assert (joined, inside) == ((["p1"], ["p0", "s1"]) if blocks == 2 else (["p1", "p3"], ["p0", "s1", "p2", "s3"]))
+    err = rel_l2(got, O.run_network(desc, {net.input_key: x})[net.output_layer])
+    print("   rel_l2=%.3e" % err, flush=True)
+    assert err <= AGREE[storage]   # (a 3x3 layer runs by itself; nine roundings to 11 bits, 3e-4 each, add up to 1e-3)
