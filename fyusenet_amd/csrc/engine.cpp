@@ -472,12 +472,13 @@ void Net::setup() {
     fuse_depthwise_layers(this);
     fuse_projection_layers(this);
     fuse_batchnorm_layers(this);
-    fuse_block_layers(this);
-    fuse_pair_layers(this);
-    fuse_head_layers(this);
+    // (a layer that computes what stands behind it keeps its own launch, which the last three ask for)
     fuse_function_layers(this);
     fuse_concat_layers(this);
     fuse_argmax_layers(this);
+    fuse_block_layers(this);
+    fuse_pair_layers(this);
+    fuse_head_layers(this);
     assign_range_resets();
     poison_lds_ = sw.get("FYNHIP_POISON_LDS") != nullptr;
     FYN_HIP(hipStreamSynchronize(stream));

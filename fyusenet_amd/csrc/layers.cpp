@@ -803,7 +803,7 @@ void fuse_argmax_layers(Net* net) {
         const Tensor& t = net->tensors[am->in[0]];
         const Tensor& o = net->tensors[am->out];
         ConvLayer* c = t.producer >= 0 ? dynamic_cast<ConvLayer*>(net->layer(t.producer)) : nullptr;
-        if (!c || !c->s16 || c->argmax_tail.idx || o.v.f16 != t.v.f16 || o.v.cp != 4 || o.v.h != t.v.h || o.v.w != t.v.w || t.v.c > 16 * c->pp.mfrags) continue;
+        if (!c || !c->s16 || c->pj_fused || c->argmax_tail.idx || o.v.f16 != t.v.f16 || o.v.cp != 4 || o.v.h != t.v.h || o.v.w != t.v.w || t.v.c > 16 * c->pp.mfrags) continue;
         if (!net->alone(am->out, c->d.number, am->d.number)) continue;
         c->argmax_tail = ArgMaxTail{o.v, am->idx_dev, t.v.c, am->act()};
         am->fused_into = c->d.number;

@@ -260,3 +260,47 @@ def test_blocks_that_share_a_layer(blocks, channels, h, w, storage, monkeypatch)
     err = rel_l2(got, O.run_network(desc, {net.input_key: x})[net.output_layer])
     print("   rel_l2=%.3e" % err, flush=True)
     assert err <= AGREE[storage]   # (a 3x3 layer runs by itself; nine roundings to 11 bits, 3e-4 each, add up to 1e-3)
+
+
+class Scores(Block):
+    """upload -> two 1x1 layers -> 1x1 -> 3x3 -> 1x1 scores -> arg-max: a segmentation head that ends as a block does."""
+
+    def __init__(self, storage, channels, classes, h, w):
+        super().__init__(storage, channels, channels, classes, h, w)
+        self.output_layer, self.argmax_layer = 5, 6
+
+    def define(self):
+        h, w, c = self.h, self.w, self.cin
+        self._add(UpDownLayerBuilder(UpDownLayerBuilder.UPLOAD, "upload").number(0).shape(c, h, w, c))
+        self.conv(1, "first", 1, c, c, h, w, 0)
+        self.conv(2, "front", 1, c, c, h, w, 1)
+        self.conv(3, "reduce", 1, c, c, h, w, 2, act=ActType.RELU, pad_out=1)
+        self.conv(4, "spatial", 3, c, c, h, w, 3, act=ActType.RELU)
+        self.conv(5, "scores", 1, c, self.cout, h, w, 4, act=ActType.RELU)
+        self._add(fa.ArgMaxLayerBuilder("labels").number(6).shape(2, h, w, self.cout).deep())
+        self._edges.append((5, 6, 0))
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("forced", [True, False], ids=["streaming", "general"])
+@pytest.mark.parametrize("channels,classes,h,w", [(64, 21, 128, 128), (32, 21, 18, 13)])
+def test_argmax_behind_a_block(channels, classes, h, w, forced, storage, monkeypatch):
+    """Where the last layer also computes the arg-max layer behind it, it keeps its launch; elsewhere the arg-max layer runs behind
+    the block.  Labels and best values are those of this frame's scores."""
+    monkeypatch.setenv("FYNHIP_FORCE_BLOCK_FUSION", "1")
+    monkeypatch.setenv("FYNHIP_FORCE_S16_CONV" if forced else "FYNHIP_NO_S16_CONV", "1")
+    net = Scores(storage, channels, classes, h, w)
+    net.setup()
+    infos = {lyr.name: lyr.kernelInfo() for lyr in net.layers}
+    assert ("conv_s16" if forced else "conv_b16") in infos["scores"].split("; apart")[0], infos["scores"]
+    assert ("no launch of its own" in infos["labels"]) == forced
+    for gain in (1.0, -1.0):   # (another frame, another answer)
+        x = net.makeInput() * np.float32(gain)
+        net.setInput(x)
+        net.forward()
+        labels, best = net.getArgMax(net.argmax_layer)
+        scores = net.getOutput(net.output_layer)
+        ref = O.run_network(net.describe(), {net.input_key: x})
+        assert rel_l2(scores, ref[net.output_layer]) <= AGREE[storage]
+        assert np.array_equal(labels, scores.argmax(axis=0)) and np.array_equal(best, scores.max(axis=0))
+    net.cleanup()
