@@ -427,6 +427,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                 else leave(std::integral_constant<bool, false>());
             }
             if (p.clamp && (txi == 0 || tyi == 0)) {   // what lies above or to the left of the layer's output repeats its first row and column
+                asm volatile("" ::: "memory");   // (the first column reads what another lane of its wave stored: in this order)
                 if (txi == 0 && x1 == 0)
                     for (int i = 0; i < FN * NPL; i++) {
                         unsigned char* const to = mid_to + (i % FN) * G::MROW + (i / FN) * G::MPLANE;
