@@ -14,13 +14,15 @@
 // fragment of row j serves every tap that meets it, and make the operands of the tile behind in registers.  Behind a barrier the
 // first ones split their result into the tensor in between while the others put the window in place and store theirs: the
 // vector work of either half of the waves lies beside the matrix work of the other, or beside its vector work.  With one
-// group of waves for all matrix work and one that staged a tile of fp32 tensors took 18.7k clocks, now 15.0k (fp16 9.1k and
-// 7.8k); 10.4k of them are matrix instructions, of either group in one pipe.  1920x1080, both layers: 212 us apart, 131 here
-// (142 before); fp16 tensors 92 and 66 (72).
+// group of waves for all matrix work and one that staged a tile of fp32 tensors took 18.7k clocks, now 15.6k (fp16 9.1k and
+// 7.8k); 10.4k of them are matrix instructions, of either group in one pipe.  0.6k are the tile's own scale for the tensor in
+// between, which has to be known in front of the split: with one from a bound on the weights the launch at 1920x1080 took
+// 118 us, and values far below that bound lost bits (1.2e-5 of error where 2.6e-7 are left now).  1920x1080, both layers
+// timed back to back: 209 us apart, 123 here; fp16 tensors 88 and 60.
 //
 // At most 16 channels in between and 32 behind (SMALL): one fragment of channels in the first layer, two taps of 16 channels a
 // step in the second, whose weights lie in LDS; bound by the fragment reads of the first layer (134 KB a wave and tile at 128
-// bytes a clock: 4.2k of a tile's 8.6k clocks).  3 -> 12 -> 20 channels at 512x624: 30.8 us apart, 19 here (fp16 19.8 and 11).
+// bytes a clock: 4.2k of a tile's 9.1k clocks).  3 -> 12 -> 20 channels at 512x624: 35.7 us apart, 19 here (fp16 24 and 11).
 #include "c4_common.h"
 
 namespace fynhip {
@@ -50,7 +52,7 @@ struct GeoA {
     static constexpr int STEPS2 = 5;                                // SMALL: the second layer's, two taps of 16 channels each; its weights lie in LDS too
     static constexpr int NW = HSTORE ? 4 : 8;                       // weight fragments of a pair of steps (c4_rows)
     static constexpr int WEIGHTS = BUF, MID = WEIGHTS + NS / 2 * NW * 1024, SB = MID + NPL * MPLANE, W2 = SB + (32 + 64) * 2 * 4, LDS = W2 + (SMALL ? STEPS2 * 2 * NPL * 1024 : 0);
-    static_assert(LDS + 16 <= 160 * 1024 && BUF < 65536 && ROW_PITCH % 16 == 0, "fits a CU; 16-byte reads are aligned");
+    static_assert(LDS + 48 <= 160 * 1024 && BUF < 65536 && ROW_PITCH % 16 == 0, "fits a CU; 16-byte reads are aligned");
 };
 
 // (KEEP: the tensor in between is written to memory as well, for a net whose tensors all stay readable)
@@ -63,6 +65,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     constexpr int CK1 = SMALL ? 4 : CHK;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ unsigned range_box[2];
+    __shared__ __align__(16) float mid_top[2][4];   // fp32 tensors: what the first layer's waves found, in this tile and the one before
     if (blockIdx.x == 0) range_clear(p.reset[0], p.reset[1], p.reset[2], p.reset[3], p.nreset);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -76,14 +79,15 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     if (tid < 2) range_box[tid] = 0u;
     const unsigned range_bits = p.in_amax ? range_load(p.in_amax) : 0u;
     float in_scale = 1.f, inv_in = 1.f;
-    float mid_scale = 1.f, inv_mid = 1.f;
     auto scales = [&]() __attribute__((always_inline)) {
-        if (!p.in_amax) return;
-        const float r0 = range_after_act(range_reduce(range_bits), p.act[0]);
-        in_scale = range_scale(r0, &inv_in);
-        // (no value of the first layer is larger than its weights' largest row sum allows: a scale for the tensor in between that
-        // does not wait for it.  Such a bound is some ten times what a frame reaches, 2^4 of the 2^14 that the split has to spare)
-        if constexpr (C8) mid_scale = range_scale(range_after_act(r0 * p.gain + p.base, p.act[1]), &inv_mid);
+        if (p.in_amax) in_scale = range_scale(range_after_act(range_reduce(range_bits), p.act[0]), &inv_in);
+    };
+    // The tensor in between takes its scale from the tile: no value is larger than its channel's largest sum of products there
+    // allows, with the bias.  (Where a bias cancels such a sum, the sum's own 22 bits are what is left; a bound from the
+    // weights alone can lie any number of bits above what a frame reaches, and values then lose theirs.)
+    auto mid_scale = [&](int turn, float* inv) __attribute__((always_inline)) {
+        const f32x4_t t = *reinterpret_cast<const f32x4_t*>(mid_top[turn]);
+        return range_scale(range_after_act(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])), p.act[1]), inv);
     };
     const int mq = lane & 15, kq = lane >> 4, w = wave & 3;
     const unsigned wlane = lane * 16;
@@ -196,7 +200,6 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             for (int i = w; i < G::STEPS2 * 2 * NPL; i += 4)
                 *reinterpret_cast<i32x4_t*>(lds + G::W2 + i * 1024 + wlane) = *reinterpret_cast<const i32x4_t*>(reinterpret_cast<const unsigned char*>(p.wpack[1]) + i * 1024 + wlane);
         }
-        const float mul2 = p.acc_mul[1] * inv_mid;
         store_t* const out = reinterpret_cast<store_t*>(p.out);
         const bool through = store_through_pays(p.out, p.h2, p.w2, p.out_cp * ESZ, !p.plain_stores, hw_block_count());
         bool drop = through && wave == 0 && hw_block_id() < 8;
@@ -259,7 +262,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        auto finish = [&](int tile) __attribute__((always_inline)) {
+        auto finish = [&](int tile, float mul2) __attribute__((always_inline)) {
             const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
             if (drop) {   // (ahead of this workgroup's first store: what it has read so far may go as well)
                 drop_clean_l2_lines();
@@ -297,14 +300,18 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             }
         };
         lds_barrier();   // the first window is staged
-        for (int tile = group, before = -1;; before = tile, tile += step) {   // (the tile that the other waves are on, the one before it)
+        for (int tile = group, before = -1, turn = 0;; before = tile, tile += step, turn ^= 1) {   // (the tile that the other waves are on, the one before it)
             const bool more = tile < ntiles, next = tile + step < ntiles;
             if (next) fetch(tile + step);
+            float inv_mid = 1.f;
+            if constexpr (C8) {
+                if (before >= 0) (void)mid_scale(turn ^ 1, &inv_mid);
+            }
             if (before >= 0) multiply();
             if (next) convert();
             if (more) lds_barrier();   // the first layer is through: the window's place is free
             if (next) put();
-            if (before >= 0) finish(before);
+            if (before >= 0) finish(before, p.acc_mul[1] * inv_mid);
             if (!more) break;
             lds_barrier();   // the window is staged, the tensor in between is there
         }
@@ -332,8 +339,8 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     unsigned char* const mid_to = lds + G::MID + ((x1 & 1) ? 32 + (x1 >> 1) : x1 >> 1) * G::SLOT + kq * (G::SLOT / 4);   // (its eight channels side by side; the second layer's weights are laid out for that)
     scales();
     const float mul1 = p.acc_mul[0] * inv_in;
-    const float lo1 = p.act[1].kind == ACT_NONE ? -3.0e38f : p.act[1].kind == ACT_RELU ? 0.f : p.act[1].lo * mid_scale;   // (its values carry the scale)
-    const float hi1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 3.0e38f : p.act[1].hi * mid_scale;
+    const float lo1 = p.act[1].kind == ACT_NONE ? -3.0e38f : p.act[1].kind == ACT_RELU ? 0.f : p.act[1].lo;
+    const float hi1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 3.0e38f : p.act[1].hi;
     const float leak1 = p.act[1].kind == ACT_NONE || p.act[1].kind == ACT_RELU ? 0.f : p.act[1].leak;
     _Float16 hlo1, hhi1;
     const bool packed1 = act_half_exact(p.act[1], hlo1, hhi1);
@@ -344,7 +351,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
     for (int d = 0; d < C4Ring<G>::LW; d++)
 #pragma unroll
         for (int k = 0; k < NW; k += SMALL ? 2 : 1) rows_put_w(ring.a0[d], ring.a2[d], k, *reinterpret_cast<const i32x4_t*>(lds + G::WEIGHTS + (d * NW + k) * 1024 + wlane));
-    for (int tile = group;;) {
+    for (int tile = group, turn = 0;; turn ^= 1) {
         const int tyi = (int)(((float)tile + 0.5f) * p.rcp_tiles_x), txi = tile - tyi * p.tiles_x;
         {   // ---- first layer ----
             f32x4_t acc[FM][FN];
@@ -362,26 +369,64 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
             }
             c4_rows<G, false>(acc, ring, rows_at, ninth_at, last_at, rows_at, lds + G::WEIGHTS + wlane);
             __builtin_amdgcn_sched_barrier(0);
-            lds_barrier();   // the window's place is free, and nobody reads the tensor in between any more
-            f32x4_t scm[FM], bi[FM];
-#pragma unroll
-            for (int fm = 0; fm < FM; fm++) {
-                scm[fm] = *reinterpret_cast<const f32x4_t*>(sb + kq * CK1 + fm * CHF) * (mul1 * mid_scale);
-                bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 32 + kq * CK1 + fm * CHF) * mid_scale;
-            }
-            const int px = txi * 2 * G::TW2 - 1 + x1;
+            const int px = txi * 2 * G::TW2 - 1 + x1, py = tyi * 2 * G::TH2 - 1;
             const bool x_ok = (unsigned)px < (unsigned)p.w;
+            f32x4_t scm[FM], bi[FM];
+            auto scale_and_bias = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int fm = 0; fm < FM; fm++) {
+                    scm[fm] = *reinterpret_cast<const f32x4_t*>(sb + kq * CK1 + fm * CHF) * mul1;
+                    bi[fm] = *reinterpret_cast<const f32x4_t*>(sb + 32 + kq * CK1 + fm * CHF);
+                }
+            };
+            float mid = 1.f, inv_mid = 1.f;
+            if constexpr (C8) {
+                scale_and_bias();
+                f32x4_t m[FM];
+                auto larger = [](f32x4_t& m, const f32x4_t v) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) m[e] = fmaxf(m[e], fabsf(v[e]));
+                };
+#pragma unroll
+                for (int fm = 0; fm < FM; fm++) m[fm] = (f32x4_t)(0.f);
+                if (py >= 0 && py + FN <= p.h) {
+#pragma unroll
+                    for (int r = 0; r < FN; r++)
+#pragma unroll
+                        for (int fm = 0; fm < FM; fm++) larger(m[fm], acc[fm][r]);
+                } else {   // (positions outside the layer's output don't count)
+#pragma unroll
+                    for (int r = 0; r < FN; r++)
+                        if ((unsigned)(py + r) < (unsigned)p.h)
+#pragma unroll
+                            for (int fm = 0; fm < FM; fm++) larger(m[fm], acc[fm][r]);
+                }
+                float top = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4 * FM; i++) top = fmaxf(top, m[i / 4][i % 4] * fabsf(scm[i / 4][i % 4]) + fabsf(bi[i / 4][i % 4]));
+                top = range_wave_max(x_ok && x1 < 63 ? top : 0.f);
+                if (lane == 0) mid_top[turn][w] = top;
+            }
+            lds_barrier();   // the window's place is free, and nobody reads the tensor in between any more
+            if constexpr (C8) {
+                mid = mid_scale(turn, &inv_mid);
+#pragma unroll
+                for (int fm = 0; fm < FM; fm++) { scm[fm] *= mid; bi[fm] *= mid; }
+            } else {
+                scale_and_bias();
+            }
+            const float lo_mid = lo1 * mid, hi_mid = hi1 * mid;   // (its values carry the scale)
             typedef typename std::conditional<SMALL, half4_t, half8_t>::type piece_t;
             auto leave = [&](auto general_) __attribute__((always_inline)) {   // (general: an activation other than none, a clamp exact on halves, or a clamp)
                 constexpr bool GENERAL = decltype(general_)::value;
 #pragma unroll
                 for (int r = 0; r < FN; r++) {
                     // (positions outside the layer's output are its zero padding)
-                    const bool ok = x_ok && (unsigned)(tyi * 2 * G::TH2 - 1 + r) < (unsigned)p.h;
+                    const bool ok = x_ok && (unsigned)(py + r) < (unsigned)p.h;
                     unsigned char* const to = mid_to + r * G::MROW;
                     // (a tile's first row and column are its neighbours' to write)
                     const bool own = KEEP && ok && r > 0 && x1 > 0;
-                    store_t* const kept = reinterpret_cast<store_t*>(p.mid) + ((size_t)(p.mid_off + tyi * 2 * G::TH2 - 1 + r) * p.mid_wp + p.mid_off + px) * p.mid_cp + kq * CK1;
+                    store_t* const kept = reinterpret_cast<store_t*>(p.mid) + ((size_t)(p.mid_off + py + r) * p.mid_wp + p.mid_off + px) * p.mid_cp + kq * CK1;
                     if constexpr (HS) {
                         piece_t v;
 #pragma unroll
@@ -401,7 +446,7 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
                         }
                         *reinterpret_cast<piece_t*>(to) = ok ? v : (piece_t)((_Float16)0.f);
                     } else {
-                        const float lo = ok ? lo1 : 0.f, hi = ok ? hi1 : 0.f, leak = ok ? leak1 : 0.f;
+                        const float lo = ok ? lo_mid : 0.f, hi = ok ? hi_mid : 0.f, leak = ok ? leak1 : 0.f;
                         if constexpr (KEEP) {
 #pragma unroll
                             for (int fm = 0; fm < FM; fm++)

@@ -523,10 +523,10 @@ void fuse_block_layers(Net* net) {
 }
 
 // The first two layers of a style-transfer net (conv_a16.hip) as one launch in the place of the second, timed against their own
-// launches (us, 3 to 32 to 64 channels, one launch / apart): fp32 tensors 384x384 22 / 21, 512x624 28 / 39, 1920x1080 131 / 212;
-// fp16 256x256 7.8 / 9.3, 512x624 15 / 23, 1920x1080 66 / 92; 3 to 12 to 20 channels, fp32, 512x624 19 / 31, 1024x1024 43 / 71.
-// Untimed it is taken wherever the first layer is in its form on rows of sixteen positions: a tie at the smallest such size,
-// ahead above.
+// launches (us, 3 to 32 to 64 channels, one launch / apart): fp32 tensors 384x384 19 / 25, 512x624 26 / 39, 1920x1080 123 / 209;
+// fp16 256x256 7.7 / 9.7, 512x624 14 / 29, 1920x1080 60 / 88; 3 to 12 to 20 channels, fp32, 256x256 9.8 / 12, 512x624 19 / 36,
+// 1024x1024 43 / 67.  Untimed it is taken wherever the first layer is in its form on rows of sixteen positions: ahead at all of
+// these.
 void fuse_head_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_HEAD_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV")) return;
     const bool forced = net->sw.get("FYNHIP_FORCE_HEAD_FUSION") != nullptr;

@@ -393,7 +393,6 @@ struct ConvA16Params {
     const float* bias[2];
     int mid_cp, out_cp, out_wp, out_off;
     float acc_mul[2];
-    float gain, base;       // fp32 tensors: no value of the first layer exceeds gain * (largest input) + base
     void* mid;              // not null: the tensor in between is written as well (tiles then cover all of it)
     int mid_wp, mid_off;
     Act act[2];             // on the fetch of each layer's input

@@ -1707,22 +1707,10 @@ class ConvLayer : public Layer {
         q.nreset = own_resets(q.reset);
         return q;
     }
-    // weights of that form: [kx][32 output channels][ky][cout fragment][plane][lane][8 halves]; and what the first layer's
-    // values are bounded by: gain * (largest input) + base
+    // weights of that form: [kx][32 output channels][ky][cout fragment][plane][lane][8 halves]
     void pack_head() {
         const ConvLayer* a = static_cast<const ConvLayer*>(net->layer(head_layer));
         if (block.empty() || a->block.empty()) return;
-        const float *b1 = a->block.data(), *w1 = b1 + a->oc;
-        const size_t row = (size_t)81 * a->d.in_channels;
-        std::vector<float> sc, bi;
-        fold_bn(b1, w1 + row * a->oc, a->oc, (a->d.flags & FYN_FLAG_POST_BATCHNORM) != 0, a->oc, sc, bi);
-        head.gain = head.base = 0.f;
-        for (int o = 0; o < a->oc; o++) {
-            double sum = 0.;
-            for (size_t i = 0; i < row; i++) sum += std::fabs(w1[o * row + i]);
-            head.gain = std::max(head.gain, (float)(sum * std::fabs(sc[o]) * 1.001));   // (and the sums' own rounding)
-            head.base = std::max(head.base, std::fabs(bi[o]) * 1.001f);
-        }
         const float* w = block.data() + oc;
         const int cin = d.in_channels, npl = head.f16 ? 1 : 2;
         const float wmul = weight_prescale(w, (size_t)oc * 9 * cin);

@@ -116,8 +116,8 @@ def test_head_in_one_launch(size, channels, edge, storage, forced):
 @pytest.mark.parametrize("storage", STORAGE[0], ids=STORAGE[1])
 @pytest.mark.parametrize("what", ["leaky", "none", "prefix", "large", "small", "rounds", "few", "few_leaky"])
 def test_head_variants(what, storage, forced):
-    """Activations on either input, magnitudes far from 1 (the tensor in between has a scale of its own, from a bound on its
-    values), and several tiles a workgroup."""
+    """Activations on either input, magnitudes far from 1 (the tensor in between has a scale of its own, tile by tile), and several
+    tiles a workgroup."""
     gain = {"large": 3e6, "small": 3e-8}.get(what, 1.0) if storage == fa.STORAGE_F32 else {"large": 64.0, "small": 1.0 / 64}.get(what, 1.0)
     mid_act = {"leaky": ActType.LEAKY_RELU, "few_leaky": ActType.LEAKY_RELU, "none": ActType.NONE}.get(what, ActType.RELU)
     net = Head(storage, (260, 700) if what in ("rounds", "few") else (21, 140), mid=12 if "few" in what else 32, cout=20 if "few" in what else 64, edge="few" in what, mid_act=mid_act, act=ActType.LEAKY_RELU if what == "prefix" else ActType.NONE, gain=gain, bn=what != "small")
@@ -190,3 +190,33 @@ def test_head_weights_loaded_again_and_timed_apart(forced):
     apart = net.getOutput(net.output_layer)
     net.cleanup()
     assert rel_l2(apart, ref) <= TOL[fa.STORAGE_F32]
+
+
+@pytest.mark.parametrize("reuse", [True, False], ids=["reuse", "keep"])
+@pytest.mark.parametrize("channels", [(4, 32, 64), (4, 12, 20)], ids=["32_64", "12_20"])
+def test_head_keeps_the_bits_of_small_values_under_large_weights(channels, reuse, forced):
+    """A colour channel that is dark in the frame, under weights 2^24 times the others': the tensor in between is far smaller than
+    its weights would allow and is split by what it holds.  Weights are powers of two and pixels multiples of 1/64, so that
+    the first layer's products are exact; what is left are 22-bit operands and fp32 sums, 3e-7 a layer."""
+    net = Head(fa.STORAGE_F32, (30, 140), *channels)
+    net.setup(reuseBuffers=reuse)
+    lyr = net.layers["first"]
+    cin, mid, _ = channels
+    blk = np.array(lyr.weights, np.float32)
+    w = blk[mid:mid + mid * 81 * cin].reshape(mid, 9, 9, cin)
+    w[...] = np.sign(w) * np.exp2(np.clip(np.round(np.log2(np.abs(w) + 1e-9)), -6, -2))
+    w[..., cin - 1] = 0.0
+    w[:, 4, 4, cin - 1] = 2.0 ** 22
+    lyr.loadWeightsAndBiases(blk)
+    x = np.round(net.makeInput() * 64) / np.float32(64)
+    x[cin - 1] = 0.0
+    net.setInput(x)
+    net.forward()
+    got = net.getOutput(net.output_layer)
+    infos = {layer.name: layer.kernelInfo() for layer in net.layers}
+    desc = net.describe()
+    net.cleanup()
+    assert together(infos), infos
+    err = rel_l2(got, O.run_network(desc, {net.input_key: x})[net.output_layer])
+    print("   rel_l2=%.3e" % err, flush=True)
+    assert err <= 3e-6
