@@ -525,8 +525,8 @@ void fuse_block_layers(Net* net) {
 // The first two layers of a style-transfer net (conv_a16.hip) as one launch in the place of the second, timed against their own
 // launches (us, 3 to 32 to 64 channels, one launch / apart): fp32 tensors 384x384 19 / 25, 512x624 26 / 39, 1920x1080 123 / 209;
 // fp16 256x256 7.7 / 9.7, 512x624 14 / 29, 1920x1080 60 / 88; 3 to 12 to 20 channels, fp32, 256x256 9.8 / 12, 512x624 19 / 36,
-// 1024x1024 43 / 67.  Untimed it is taken wherever the first layer is in its form on rows of sixteen positions: ahead at all of
-// these.
+// 1024x1024 43 / 67.  Where the tensor in between is written as well, 512x624 32 / 39, 1920x1080 145 / 211, fp16 71 / 90.  Untimed it
+// is taken wherever the first layer is in its form on rows of sixteen positions: ahead at all of these.
 void fuse_head_layers(Net* net) {
     if (net->sw.get("FYNHIP_NO_HEAD_FUSION") || net->sw.get("FYNHIP_NO_P16_CONV")) return;
     const bool forced = net->sw.get("FYNHIP_FORCE_HEAD_FUSION") != nullptr;
@@ -555,6 +555,10 @@ void fuse_head_layers(Net* net) {
         int rows, cols;
         conv_a16_tile(&rows, &cols);
         q.tiles_x = (q.w2 + cols - 1) / cols; q.tiles_y = (q.h2 + rows - 1) / rows;
+        if (!net->reuse_buffers) {   // (every tensor stays readable: the launch writes the one in between as well)
+            q.mid = mv.ptr; q.mid_wp = mv.wp(); q.mid_off = mv.pad;
+            q.tiles_x = (q.w + 2 * cols - 1) / (2 * cols); q.tiles_y = (q.h + 2 * rows - 1) / (2 * rows);
+        }
         q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
         q.groups = std::min(q.tiles_x * q.tiles_y, 256);   // (one workgroup per CU)
         const ConvLayer* L[2] = {a, c};
@@ -577,7 +581,7 @@ void fuse_head_layers(Net* net) {
         }
         bool pick = true;
         char key[200];
-        snprintf(key, sizeof(key), "head:%d:%dto%dto%d:%dx%d:e%d", q.f16, a->d.in_channels, a->oc, c->oc, a->oh, a->ow, q.clamp);
+        snprintf(key, sizeof(key), "head:%d:%dto%dto%d:%dx%d:e%d:k%d", q.f16, a->d.in_channels, a->oc, c->oc, a->oh, a->ow, q.clamp, q.mid ? 1 : 0);
         if (forced || tune_cache_flag(net, key, &pick)) {
         } else if (!(at && at[0] == '0')) {
             float t_one = 1e30f, t_apart = 1e30f;
@@ -591,19 +595,14 @@ void fuse_head_layers(Net* net) {
                 }, 10));
             }
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
-                fprintf(stderr, "[tune] 9x9 %d to %d and 3x3 to %d with a step of two at %dx%d: one launch %.1f us, apart %.1f us\n", a->d.in_channels, a->oc, c->oc, a->oh, a->ow, t_one * 1e3f, t_apart * 1e3f);
+                fprintf(stderr, "[tune] 9x9 %d to %d and 3x3 to %d with a step of two at %dx%d%s: one launch %.1f us, apart %.1f us\n", a->d.in_channels, a->oc, c->oc, a->oh, a->ow,
+                        q.mid ? ", the tensor in between written" : "", t_one * 1e3f, t_apart * 1e3f);
             pick = t_one < t_apart;
             tune_cache_store_flag(net, key, pick);
         }
         if (!pick) {
             net->dev_free(wp);
             continue;
-        }
-        if (!net->reuse_buffers) {   // (every tensor stays readable: the launch writes the one in between as well)
-            q.mid = mv.ptr; q.mid_wp = mv.wp(); q.mid_off = mv.pad;
-            q.tiles_x = (q.w + 2 * cols - 1) / (2 * cols); q.tiles_y = (q.h + 2 * rows - 1) / (2 * rows);
-            q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
-            q.groups = std::min(q.tiles_x * q.tiles_y, 256);
         }
         c->head = q;
         c->head_wpack_dev = wp;

@@ -220,3 +220,19 @@ def test_head_keeps_the_bits_of_small_values_under_large_weights(channels, reuse
     err = rel_l2(got, O.run_network(desc, {net.input_key: x})[net.output_layer])
     print("   rel_l2=%.3e" % err, flush=True)
     assert err <= 3e-6
+
+
+def test_head_is_timed_in_the_form_that_will_run(monkeypatch, tmp_path):
+    """Without buffer reuse the launch writes the tensor in between too: that form is measured, and its choice noted, by itself."""
+    notes = tmp_path / "choices"
+    monkeypatch.setenv("FYNHIP_AUTOTUNE", "1")
+    monkeypatch.setenv("FYNHIP_TUNE_CACHE", str(notes))
+    found = []
+    for reuse in (True, False):
+        net = Head(fa.STORAGE_F32, (618, 516))
+        net.setup(reuseBuffers=reuse)
+        info = net.layers["first"].kernelInfo()
+        net.cleanup()
+        assert "tw=16" in info, info   # (the form that the launch is made for)
+        found.append({line.split()[0] for line in notes.read_text().splitlines() if line.startswith("head:")})
+    assert found[0] == {"head:0:3to32to64:618x516:e0:k0"} and found[1] - found[0] == {"head:0:3to32to64:618x516:e0:k1"}
