@@ -512,50 +512,41 @@ void Net::assign_range_words() {
 // A word raised during a forward pass must read 0 again before the tensor's producer runs in the next pass.  The
 // clearing is given to a convolution kernel that runs after the tensor's last reader (kernels of one stream run one
 // after the other, so nothing else touches the word at that time): the first such layer behind the last reader,
-// wrapping around to the layers in front of the producer.  A tensor for which no layer is found loses its word.
-int Net::words_without_reset() const {
-    if (!amax_dev_) return 0;
-    std::map<int, int> room;
-    for (auto& kv : layers) room[kv.first] = kv.second->reset_room();
-    int lost = 0;
-    for (const Tensor& t : tensors) {   // (the order and the rules of assign_range_resets)
-        if (!t.amax || t.producer < 0 || layers.at(t.producer)->d.type == FYN_LAYER_UPLOAD) continue;
+// wrapping around to the layers in front of the producer.  take(layer, word) says whether the layer's launch has room for
+// the word; the result are the tensors for which none has.
+template <class Take>
+std::vector<int> Net::place_range_resets(Take&& take) const {
+    std::vector<int> lost;
+    for (size_t i = 0; i < tensors.size(); i++) {
+        const Tensor& t = tensors[i];
+        if (!t.amax || t.producer < 0 || layers.at(t.producer)->d.type == FYN_LAYER_UPLOAD) continue;   // (an upload's: cleared where it is written from the host)
         const int last = std::max(t.last_reader, t.producer);
-        auto at = room.end();
-        for (auto i = room.begin(); i != room.end() && at == room.end(); ++i)
-            if (i->first > last && i->second > 0) at = i;
-        for (auto i = room.begin(); i != room.end() && at == room.end(); ++i)
-            if (i->first < t.written && i->second > 0) at = i;
-        if (at == room.end()) lost++;
-        else at->second--;
+        bool done = false;
+        // layers behind the last reader, in execution order ...
+        for (auto& kv : layers)
+            if (kv.first > last && take(kv.second.get(), t.amax)) { done = true; break; }
+        // ... then the layers in front of the launch that writes it (they run in the next pass, before it)
+        if (!done)
+            for (auto& kv : layers)
+                if (kv.first < t.written && take(kv.second.get(), t.amax)) { done = true; break; }
+        if (!done) lost.push_back((int)i);
     }
     return lost;
 }
 
+int Net::words_without_reset() const {
+    if (!amax_dev_) return 0;
+    std::map<const Layer*, int> room;
+    for (auto& kv : layers) room[kv.second.get()] = kv.second->reset_room();
+    return (int)place_range_resets([&](Layer* l, unsigned*) { return room[l]-- > 0; }).size();
+}
+
+// A tensor for which no layer is found loses its word.
 void Net::assign_range_resets() {
     if (!amax_dev_) return;
-    std::vector<int> order;
-    for (auto& kv : layers) order.push_back(kv.first);
-    bool lost = false;
-    for (Tensor& t : tensors) {
-        if (!t.amax || t.producer < 0) continue;
-        Layer* pl = layer(t.producer);
-        if (pl->d.type == FYN_LAYER_UPLOAD) continue;   // cleared where it is written from the host
-        const int last = std::max(t.last_reader, t.producer);
-        bool done = false;
-        // layers behind the last reader, in execution order ...
-        for (int no : order)
-            if (no > last && layer(no)->add_range_reset(t.amax)) { done = true; break; }
-        // ... then the layers in front of the launch that writes it (they run in the next pass, before it)
-        if (!done)
-            for (int no : order)
-                if (no < t.written && layer(no)->add_range_reset(t.amax)) { done = true; break; }
-        if (!done) {
-            t.amax = nullptr;
-            lost = true;
-        }
-    }
-    if (lost) {
+    const std::vector<int> lost = place_range_resets([](Layer* l, unsigned* word) { return l->add_range_reset(word); });
+    for (int i : lost) tensors[i].amax = nullptr;
+    if (!lost.empty()) {
         // layers copied the word addresses into their kernel arguments during setup: let them look again
         for (auto& kv : layers) kv.second->setup_ranges();
     }

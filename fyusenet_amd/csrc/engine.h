@@ -245,6 +245,8 @@ class Net {
     float* static_scratch_ = nullptr;   // this device's address of the fixed staging area
     unsigned* amax_dev_ = nullptr;      // one value-range word per tensor
     void assign_range_words();
+    template <class Take>
+    std::vector<int> place_range_resets(Take&& take) const;   // (which launch clears which word: engine.cpp)
     void assign_range_resets();
     hipGraph_t graph_ = nullptr;
     hipGraphExec_t graph_exec_ = nullptr;
