@@ -372,25 +372,52 @@ static bool head_of(Net* net, const ConvLayer* c, ConvLayer*& a) {
     const int from = net->tensors[a->in[0]].producer;   // (a frame from the host or the application: its value-range word is never lost)
     return from < 0 || net->layer(from)->d.type == FYN_LAYER_UPLOAD;
 }
-// While buffers are assigned, the input of such a block or pair is read until its last layer has run, which may compute all of
-// it (the tensors' last readers as they were: whether the layers are joined is not known yet).
+// What says which compiled variant computes a bottleneck: the next chunk count that there is one for (the channels behind the
+// tensor read as zero).  False: none does.
+static bool block_variant(const ConvLayer* a, const ConvLayer* b, const ConvLayer* c, bool bn, bool proj, ConvB16Params& q) {
+    static const float some = 0.f;   // (whether the batch-norm layer is there is all that counts)
+    const TView &iv = a->tin(0).v, &ov = c->tout().v;
+    q.in_mul = q.in_add = bn ? &some : nullptr;
+    q.proj = proj ? 1 : 0;
+    q.f16 = ov.f16 ? 1 : 0;
+    q.in_cp = iv.cp; q.out_cp = ov.cp;
+    q.mid = std::max(a->oc, b->oc) <= 64 ? 4 : (std::max(a->oc, b->oc) + 15) / 16;
+    if (q.mid > 4 && q.mid < 8) q.mid = 8;   // (channels behind a layer's count have zero weights, scales and biases)
+    q.tiles_x = (c->ow + 3) / 4; q.tiles_y = (c->oh + 3) / 4;
+    for (q.chunks = (iv.cp + 31) / 32; q.chunks <= 16 && conv_b16_weight_frags(q) == 0; q.chunks++) {}
+    return conv_b16_weight_frags(q) != 0 && (long long)q.tiles_x * q.tiles_y <= 4096;
+}
+// ... and a pair: the compiled tile heights (indices of conv_c16_variant).
+static std::vector<int> pair_variants(const ConvLayer* a, const ConvLayer* c) {
+    std::vector<int> out;
+    const TView &iv = a->tin(0).v, &mv = a->tout().v, &ov = c->tout().v;
+    for (int i = 0; i < conv_c16_count(); i++) {
+        int f16, groups, fr, th;
+        conv_c16_variant(i, &f16, &groups, &fr, &th);
+        if (f16 == (ov.f16 ? 1 : 0) && iv.cp == 8 * groups && mv.cp == iv.cp && ov.cp <= 16 * fr && (long long)((c->ow + 15) / 16) * ((c->oh + th - 1) / th) <= (1 << 20)) out.push_back(i);
+    }
+    return out;
+}
+// While buffers are assigned, the input of a block or pair that a variant is compiled for is read until its last layer has run,
+// which may compute all of it (the tensors' last readers as they were: whether the layers are joined is not known yet).  A
+// head's input is the frame, whose buffer nobody shares.
 std::vector<std::pair<int, int>> keep_block_inputs(Net* net) {
     std::vector<std::pair<int, int>> were;
-    if (!net->reuse_buffers) return were;
+    if (!net->reuse_buffers || net->sw.get("FYNHIP_NO_P16_CONV")) return were;
     auto keep = [&](int tensor, int layer_no) {
         were.push_back({tensor, net->tensors[tensor].last_reader});
         net->read_until(tensor, layer_no);
     };
     for (auto& kv : net->layers) {
         ConvLayer *c = dynamic_cast<ConvLayer*>(kv.second.get()), *a = nullptr, *b = nullptr;
-        if (c && !net->sw.get("FYNHIP_NO_HEAD_FUSION") && head_of(net, c, a)) keep(a->in[0], c->d.number);
-        if (c && !net->sw.get("FYNHIP_NO_PAIR_FUSION") && pair_of(net, c, a) && a->d.in_channels <= 64) keep(a->in[0], c->d.number);
-        if (!c || net->sw.get("FYNHIP_NO_BLOCK_FUSION") || !block_of(net, c, a, b)) continue;
-        keep(a->in[0], c->d.number);
-        const Tensor& t = net->tensors[a->in[0]];
-        if (t.producer < 0) continue;
-        BatchNormLayer* bn = dynamic_cast<BatchNormLayer*>(net->layer(t.producer));   // (which the block may apply)
-        if (bn && !bn->in.empty() && bn->in[0] >= 0) keep(bn->in[0], c->d.number);
+        if (!c) continue;
+        if (!net->sw.get("FYNHIP_NO_PAIR_FUSION") && pair_of(net, c, a) && !pair_variants(a, c).empty()) keep(a->in[0], c->d.number);
+        if (net->sw.get("FYNHIP_NO_BLOCK_FUSION") || !block_of(net, c, a, b)) continue;
+        const int x = a->in[0], from = net->tensors[x].producer;
+        const BatchNormLayer* bn = from < 0 ? nullptr : dynamic_cast<BatchNormLayer*>(net->layer(from));   // (which the block may apply)
+        ConvB16Params q{};
+        if (block_variant(a, b, c, false, false, q) || (projection_of(net, c) && block_variant(a, b, c, false, true, q))) keep(x, c->d.number);
+        if (bn && !bn->in.empty() && bn->in[0] >= 0 && block_variant(a, b, c, true, false, q)) keep(bn->in[0], c->d.number);
     }
     return were;
 }
@@ -461,22 +488,15 @@ void fuse_block_layers(Net* net) {
             q.scale[i] = L[i]->scale_dev; q.bias[i] = L[i]->bias_dev;
             q.acc_mul[i] = 1.f;
         }
+        if (!block_variant(a, b, c, a->bn_fused, pr != nullptr, q)) continue;
         q.in = a->bn_fused ? a->bn_in : iv.ptr;
         q.in_mul = a->bn_fused ? a->bn_mul : nullptr; q.in_add = a->bn_fused ? a->bn_add : nullptr;
         q.out = ov.ptr;
         q.act[0] = a->act(); q.act[1] = b->act(); q.act[2] = c->act();
-        q.mid = std::max(a->oc, b->oc) <= 64 ? 4 : (std::max(a->oc, b->oc) + 15) / 16;
-        if (q.mid > 4 && q.mid < 8) q.mid = 8;   // (channels behind a layer's count have zero weights, scales and biases)
-        q.proj = pr ? 1 : 0;
-        q.in_hp = iv.hp(); q.in_wp = iv.wp(); q.in_cp = iv.cp; q.in_off = iv.pad;
+        q.in_hp = iv.hp(); q.in_wp = iv.wp(); q.in_off = iv.pad;
         q.h = c->oh; q.w = c->ow;
-        q.out_wp = ov.wp(); q.out_cp = ov.cp; q.out_off = ov.pad;
-        q.tiles_x = (c->ow + 3) / 4; q.tiles_y = (c->oh + 3) / 4;
+        q.out_wp = ov.wp(); q.out_off = ov.pad;
         q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
-        q.f16 = ov.f16 ? 1 : 0;
-        // (the next chunk count that a variant is compiled for: the channels behind the tensor read as zero)
-        for (q.chunks = (iv.cp + 31) / 32; q.chunks <= 16 && conv_b16_weight_frags(q) == 0; q.chunks++) {}
-        if (conv_b16_weight_frags(q) == 0 || (long long)q.tiles_x * q.tiles_y > 4096) continue;
         const size_t halves = conv_b16_weight_frags(q) * (q.f16 ? 1 : 2) * 64 * 8;
         void* const wp = net->dev_alloc(halves * 2, true);
         q.wpack = wp;
@@ -657,14 +677,13 @@ void fuse_pair_layers(Net* net) {
         q.tiles_x = (q.w + 15) / 16; q.rcp_tiles_x = 1.0f / (float)q.tiles_x;
         std::vector<ConvC16Params> cands;
         size_t halves = 0;
-        for (int i = 0; i < conv_c16_count(); i++) {
+        for (int i : pair_variants(a, c)) {
             int f16, groups, fr, th;
             conv_c16_variant(i, &f16, &groups, &fr, &th);
-            if (f16 != q.f16 || groups != q.groups || ov.cp > 16 * fr || (want_th && th != want_th)) continue;
+            if (want_th && th != want_th) continue;
             ConvC16Params t = q;
             t.th = th;
             t.tiles_y = (q.h + th - 1) / th;
-            if ((long long)t.tiles_x * t.tiles_y > (1 << 20)) continue;
             cands.push_back(t);
             int shares = 0;
             const int steps = conv_c16_steps(t, &shares);

@@ -9,7 +9,7 @@ import fyusenet_amd as fa
 from fyusenet_amd import networks, prng
 from fyusenet_amd.builders import ActType, UpDownLayerBuilder
 from oracle import oracle as O
-from util import combos, rel_l2
+from util import combos, device_bytes, rel_l2
 
 pytestmark = pytest.mark.gpu
 TOL = {fa.STORAGE_F32: 3e-6, fa.STORAGE_F16: 2e-3}
@@ -304,3 +304,13 @@ def test_argmax_behind_a_block(channels, classes, h, w, forced, storage, monkeyp
         assert rel_l2(scores, ref[net.output_layer]) <= AGREE[storage]
         assert np.array_equal(labels, scores.argmax(axis=0)) and np.array_equal(best, scores.max(axis=0))
     net.cleanup()
+
+
+@pytest.mark.parametrize("channels,mid,more", [(512, 128, False), (256, 64, True)])
+def test_no_memory_for_blocks_that_no_variant_computes(channels, mid, more, monkeypatch):
+    """The block's input keeps its buffer until the last layer has run only where that layer's launch may read it."""
+    monkeypatch.setenv("FYNHIP_AUTOTUNE", "0")
+    with_blocks = device_bytes(Block(fa.STORAGE_F32, channels, mid, channels, 24, 24, kind="none"))
+    monkeypatch.setenv("FYNHIP_NO_BLOCK_FUSION", "1")
+    without = device_bytes(Block(fa.STORAGE_F32, channels, mid, channels, 24, 24, kind="none"))
+    assert with_blocks > without if more else with_blocks == without

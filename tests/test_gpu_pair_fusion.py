@@ -9,7 +9,7 @@ import fyusenet_amd as fa
 from fyusenet_amd import networks, prng
 from fyusenet_amd.builders import ActType, ConvLayerBuilder, LayerType, UpDownLayerBuilder
 from oracle import oracle as O
-from util import combos, rel_l2
+from util import combos, device_bytes, rel_l2
 
 pytestmark = pytest.mark.gpu
 TOL = {fa.STORAGE_F32: 3e-6, fa.STORAGE_F16: 2e-3}
@@ -188,3 +188,13 @@ def test_nan_stays_in_its_window(rows, storage, monkeypatch):
     mask = np.ones(got.shape[1:], bool)
     mask[10:15, 14:19] = False
     assert not np.array_equal(got, want) and rel_l2(got[:, mask], want[:, mask]) <= TOL[storage]
+
+
+@pytest.mark.parametrize("channels,more", [(24, False), (40, True)])
+def test_no_memory_for_pairs_that_no_variant_computes(channels, more, monkeypatch):
+    """The pair's input keeps its buffer until the second layer has run only where that layer's launch may read it."""
+    monkeypatch.setenv("FYNHIP_AUTOTUNE", "0")
+    with_pairs = device_bytes(Pair(fa.STORAGE_F32, channels, channels, 96, 96, True, residual=False))
+    monkeypatch.setenv("FYNHIP_NO_PAIR_FUSION", "1")
+    without = device_bytes(Pair(fa.STORAGE_F32, channels, channels, 96, 96, True, residual=False))
+    assert with_pairs > without if more else with_pairs == without

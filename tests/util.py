@@ -1,4 +1,5 @@
 """Shared helpers of the test-suite."""
+import ctypes
 import itertools
 
 import numpy as np
@@ -84,3 +85,13 @@ def oracle_single(builder, storage, inputs, weights=None):
     desc = {"layers": [{"builder": builder, "number": builder.number_, "weights": weights}], "connections": [], "storage": storage}
     feeds = {(builder.number_, p): x for p, x in enumerate(inputs)}
     return O.run_network(desc, feeds)[builder.number_]
+
+
+def device_bytes(net):
+    """What setting up a network allocates (fyn_net_device_allocations)."""
+    from fyusenet_amd import capi
+    calls, nbytes = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    net.setup()
+    capi.check(capi.lib().fyn_net_device_allocations(net._h, ctypes.byref(calls), ctypes.byref(nbytes)))
+    net.cleanup()
+    return nbytes.value
