@@ -385,7 +385,8 @@ static bool block_variant(const ConvLayer* a, const ConvLayer* b, const ConvLaye
     if (q.mid > 4 && q.mid < 8) q.mid = 8;   // (channels behind a layer's count have zero weights, scales and biases)
     q.tiles_x = (c->ow + 3) / 4; q.tiles_y = (c->oh + 3) / 4;
     for (q.chunks = (iv.cp + 31) / 32; q.chunks <= 16 && conv_b16_weight_frags(q) == 0; q.chunks++) {}
-    return conv_b16_weight_frags(q) != 0 && (long long)q.tiles_x * q.tiles_y <= 4096;
+    // (32-bit offsets)
+    return conv_b16_weight_frags(q) != 0 && (long long)q.tiles_x * q.tiles_y <= 4096 && (long long)iv.hp() * iv.wp() * iv.cp <= (1ll << 30);
 }
 // ... and a pair: the compiled tile heights (indices of conv_c16_variant).
 static std::vector<int> pair_variants(const ConvLayer* a, const ConvLayer* c) {

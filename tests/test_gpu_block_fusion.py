@@ -314,3 +314,17 @@ def test_no_memory_for_blocks_that_no_variant_computes(channels, mid, more, monk
     monkeypatch.setenv("FYNHIP_NO_BLOCK_FUSION", "1")
     without = device_bytes(Block(fa.STORAGE_F32, channels, mid, channels, 24, 24, kind="none"))
     assert with_blocks > without if more else with_blocks == without
+
+
+def test_block_on_an_input_beyond_32_bit_offsets(monkeypatch):
+    """A few positions in a halo so wide that the tensor has more than 2^30 values: the layers run by themselves."""
+    outs = []
+    for switch in ("FYNHIP_FORCE_BLOCK_FUSION", "FYNHIP_NO_BLOCK_FUSION"):
+        monkeypatch.setenv(switch, "1")
+        net = Block(fa.STORAGE_F16, 256, 64, 256, 4, 4, kind="none", halo=1024)
+        _, got, infos = run(net)
+        net.cleanup()
+        assert "conv_b16" not in infos["expand"]
+        outs.append(got)
+        monkeypatch.delenv(switch)
+    assert np.any(outs[0]) and rel_l2(*outs) <= TOL[fa.STORAGE_F16]
