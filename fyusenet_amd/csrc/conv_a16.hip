@@ -491,12 +491,12 @@ __global__ __launch_bounds__(512) void conv_a16_kernel(const ConvA16Params p) {
 
 #if FYN_P16_HALF
 #define A16_NAME(n) n##_half
+size_t conv_a16_lds_half(bool small) { return small ? (size_t)GeoA<true>::LDS : (size_t)GeoA<false>::LDS; }
 #else
 #define A16_NAME(n) n
 int launch_conv_a16_half(const ConvA16Params& p, hipStream_t s);
-size_t conv_a16_lds_bytes(bool f16, bool small) {
-    return (f16 ? 1 : 2) * (size_t)(GeoA<false>::PLANE + (small ? GeoA<true>::MPLANE : GeoA<false>::MPLANE)) + (f16 ? 24 : 48) * 1024 + (32 + 64) * 2 * 4 + (small ? (f16 ? 10 : 20) * 1024 : 0);
-}
+size_t conv_a16_lds_half(bool small);
+size_t conv_a16_lds_bytes(bool f16, bool small) { return f16 ? conv_a16_lds_half(small) : small ? (size_t)GeoA<true>::LDS : (size_t)GeoA<false>::LDS; }
 void conv_a16_tile(int* rows, int* cols) { *rows = GeoA<false>::TH2; *cols = GeoA<false>::TW2; }
 #endif
 int A16_NAME(launch_conv_a16)(const ConvA16Params& p, hipStream_t s) {
