@@ -523,9 +523,11 @@ void fuse_block_layers(Net* net) {
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
                 fprintf(stderr, "[tune] bottleneck %d to %d to %d to %d at %dx%d%s: one launch %.1f us, apart %.1f us\n", iv.cp, a->oc, b->oc, c->oc, c->oh, c->ow, pr ? " with its projection" : "", t_one * 1e3f,
                         t_apart * 1e3f);
-            // (a near tie goes to the single launch: where networks run side by side, launches are what the chip deals out one
-            // by one.  512 to 128 to 128 to 512 on fp16 tensors at 28x28: 10.9 against 10.5 us, a frame by itself 207 / 206 us, four
-            // instances side by side 100.6 / 103.3)
+            // (a near tie goes to the single launch.  512 to 128 to 128 to 512 on fp16 tensors, one launch / apart: 10.9 / 10.4 us at 24x24,
+            // 10.9 / 10.5 at 28x28, 11.0 / 10.7 at 32x32.  A ResNet-50's frame with its three such blocks joined / apart, images of
+            // 192, 224 and 256: four instances side by side 88 / 91, 99 / 102, 109 / 113 us, passes queued launch by launch 231 / 238, 237 / 243,
+            // 236 / 249, a host frame by itself 272 / 277, 278 / 281, 285 / 289; on the other side a captured graph 215 / 212, 220 / 217,
+            // 222 / 218, two instances 131 / 129, 138 / 136, 146 / 143, one stream of frames 223 / 221, 230 / 228, 238 / 236)
             pick = t_one < t_apart * 1.05f;
             tune_cache_store_flag(net, key, pick);
         }
@@ -719,7 +721,10 @@ void fuse_pair_layers(Net* net) {
             if (net->sw.get("FYNHIP_TUNE_VERBOSE"))
                 fprintf(stderr, "[tune] 3x3 %d to %d to %d at %dx%d: one launch (%d rows) %.1f us, apart %.1f us\n", iv.cp, a->oc, c->oc, c->oh, c->ow, cands[pick].th, t_one * 1e3f, t_apart * 1e3f);
             // (a tenth: on a few rows of tiles, where both ways are a chain of latencies, the frame does not show a smaller lead.  40 to 40
-            // to 40 at 33x50 on fp32 tensors 8.1 / 8.9 us here, the sample net's frame 47.5 / 47.4; on fp16 tensors 6.5 / 7.4, 38.2 / 40.1)
+            // to 40, one launch / apart, and the frame of the sample net with its pairs joined / apart, us: fp32 12x16 7.9 / 8.3, 43.9 / 42.8;
+            // 24x32 8.1 / 8.6, 44.1 / 43.1; 33x50 8.1 / 8.8, 45.5 / 45.0; 48x64 8.2 / 9.3, 47.0 / 47.3; 80x80 8.2 / 11.4, 55.9 / 61.0; fp16 24x32
+            // 6.4 / 6.5, 35.0 / 34.8; 33x50 6.5 / 7.4, 35.6 / 37.0; 48x64 6.5 / 7.6, 36.7 / 39.3.  At 192x256, where the tiles take more than a
+            // round, the timings tie, 22.5 / 22.3, and the frame with them within 1 %, 153.6 / 155.4; fp16 15.9 / 16.5, 104.8 / 105.8)
             const bool win = t_one < t_apart * 0.9f;
             tune_cache_store_triple(net, key, win ? 1 : 0, cands[pick].th, 0);
             if (!win && !forced) pick = -1;
