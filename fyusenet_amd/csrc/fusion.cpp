@@ -501,8 +501,12 @@ void fuse_block_layers(Net* net) {
         const size_t halves = conv_b16_weight_frags(q) * (q.f16 ? 1 : 2) * 64 * 8;
         void* const wp = net->dev_alloc(halves * 2, true);
         q.wpack = wp;
-        // (untimed: 256 to 64 to 64 to 256, one launch / apart: 9.5 / 15.7 us at 56x56, 17.6 / 21.5 at 80x80, 25.0 / 24.7 at 96x96)
-        bool pick = q.mid == 4 && q.tiles_x * q.tiles_y <= 400;
+        // (untimed, us, one launch / apart.  In one round of workgroups it is ahead whatever the channels: fp32 56x56 256 to 64 to 64 to
+        // 256 9.8 / 15.9, 64 to 32 to 32 to 64 9.1 / 13.2, 16 to 8 9.1 / 13.3, 7x7 9.0 / 10.7, 8.6 / 10.5, 8.7 / 13.3.  A second one costs
+        // a launch of narrow fp32 layers more than the three: 72x72 64 to 32 16.5 / 13.8, 128 to 32 16.8 / 14.9, but 128 to 64 16.8 / 18.1,
+        // 256 to 64 17.9 / 21.7; fp16 64 to 32 8.4 / 10.1.  256 to 64 at 96x96 25.0 / 24.7)
+        const int tiles = q.tiles_x * q.tiles_y;
+        bool pick = q.mid == 4 && (tiles <= 256 || (tiles <= 400 && (q.f16 || std::max(a->oc, b->oc) > 32)));
         char key[200];
         snprintf(key, sizeof(key), "blk:%d:%dto%dto%dto%d:%dx%d:r%d:b%d", q.f16, iv.cp, a->oc, b->oc, c->oc, c->oh, c->ow, pr ? 2 : q.res ? 1 : 0, a->bn_fused ? 1 : 0);
         if (net->sw.get("FYNHIP_FORCE_BLOCK_FUSION")) pick = true;

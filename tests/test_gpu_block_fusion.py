@@ -328,3 +328,16 @@ def test_block_on_an_input_beyond_32_bit_offsets(monkeypatch):
         outs.append(got)
         monkeypatch.delenv(switch)
     assert np.any(outs[0]) and rel_l2(*outs) <= TOL[fa.STORAGE_F16]
+
+
+@pytest.mark.parametrize("storage,channels,mid,side,one", [
+    (fa.STORAGE_F32, 64, 32, 64, True), (fa.STORAGE_F32, 64, 32, 68, False), (fa.STORAGE_F32, 128, 64, 68, True), (fa.STORAGE_F32, 128, 64, 84, False), (fa.STORAGE_F16, 64, 32, 68, True),
+    (fa.STORAGE_F16, 64, 32, 84, False)])
+def test_blocks_that_nothing_is_timed_for(storage, channels, mid, side, one, monkeypatch):
+    """One launch in a single round of 256 workgroups, and in up to 400 where the layers are wide enough or the tensors fp16."""
+    monkeypatch.setenv("FYNHIP_AUTOTUNE", "0")
+    net = Block(storage, channels, mid, channels, side, side)
+    net.setup()
+    infos = {lyr.name: lyr.kernelInfo() for lyr in net.layers}
+    net.cleanup()
+    assert together(infos) == one, infos["expand"]
