@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import fyusenet_amd as fa
-from fyusenet_amd import prng
+from fyusenet_amd import networks, prng
 from oracle import oracle as O
 from util import conv_block, rel_l2
 
@@ -339,3 +339,160 @@ def test_random_shallow_chain(seed, storage):
         assert got[lyr.number].shape == tuple(specs[lyr.number - 1]["out"])
         assert e <= TOL[storage], (seed, lyr.name, e)
     net.cleanup()
+
+
+class Motifs(networks._StreamNet):
+    """Random rows of what the engine joins into one launch, with what may stand around it: heads, bottlenecks with every kind of
+    shortcut, chains of them that share layers, pairs of 3x3 layers, batch-norm, scale and concatenation layers in between, and
+    an arg-max, a sigmoid or nothing at the end."""
+    config_id = 8
+    input_key = (0, 0)
+
+    def __init__(self, storage, seed):
+        super().__init__(storage)
+        self.seed = seed
+        rng = self.rng = np.random.RandomState(20_000 + seed)
+        self.head = seed % 3 == 0
+        self.h, self.w = [int(rng.randint(10, 40)) for _ in range(2)] if self.head else [int(rng.randint(5, 26)) for _ in range(2)]
+        self.parts = [str(rng.choice(["block", "block", "chain", "pair", "pair", "cat", "bn", "up"])) for _ in range(int(rng.randint(2, 5)))]
+        if not self.head and not set(self.parts) & {"block", "chain", "pair"}:
+            self.parts.insert(1, ["block", "chain", "pair"][seed % 3])
+        self.tail = ["argmax", "sigmoid", "plain"][int(rng.randint(0, 3))]
+
+    def _act(self):
+        return [A.RELU, A.RELU, A.NONE, A.LEAKY_RELU][int(self.rng.randint(0, 4))]
+
+    def _one(self, src, k, cin, cout, **kw):
+        """A convolution behind the layers so far, which a launch may have taken in."""
+        self.no += 1
+        self.conv(self.no, "c%d" % self.no, k, cin, cout, self.y, self.x, src, act=kw.pop("act", A.RELU), bn=bool(self.rng.randint(0, 2)), **kw)
+        return self.no
+
+    def define(self):
+        rng = self.rng = np.random.RandomState(30_000 + self.seed)
+        self.y, self.x, self.no = self.h, self.w, 0
+        self._add(fa.UpDownLayerBuilder(fa.UpDownLayerBuilder.UPLOAD, "upload").number(0).shape(3, self.h, self.w, 3).outputPadding(4 if self.head else 0))
+        if self.head:
+            few = bool(rng.randint(0, 2))
+            self._one(0, 9, 3, 12 if few else 32, act=A.NONE, pad_out=1)
+            c = 20 if few else 64
+            last = self._one(1, 3, 12 if few else 32, c, stride=2, act=self._act())
+            self.y, self.x = self.y // 2, self.x // 2
+        else:
+            c = int(rng.choice([32, 48, 64, 200]))
+            last = self._one(0, 1, 3, c, act=A.NONE)
+        for part in self.parts:
+            if part in ("block", "chain"):
+                mid, act = int(rng.choice([16, 24, 64])), self._act()
+                out, short = c, None
+                kind = "none" if part == "chain" else str(rng.choice(["none", "identity", "projection"]))
+                if kind == "projection":
+                    c, was = int(rng.choice([32, 64])), c
+                    last = self._one(last, 1, was, c, act=A.RELU)
+                    out = int(rng.choice([64, 72, 256]))
+                    short = self._one(last, 1, c, out, act=act)
+                elif kind == "identity":
+                    short = last
+                a = self._one(last, 1, c, mid, act=act, pad_out=1)
+                b = self._one(a, 3, mid, mid, act=self._act())
+                if part == "chain":
+                    p = self._one(b, 1, mid, mid, act=self._act(), pad_out=1)
+                    b = self._one(p, 3, mid, mid, act=self._act())
+                res = {} if short is None else {"residual": short, "res_act": [A.NONE, A.RELU][int(rng.randint(0, 2))] if kind == "identity" else A.NONE}
+                last, c = self._one(b, 1, mid, out, act=self._act(), **res), out
+            elif part == "pair":
+                ch = int(rng.choice([40, 48]))
+                x = self._one(last, 1, c, ch, pad_out=1)
+                a = self._one(x, 3, ch, ch, act=self._act(), pad_out=1)
+                res = {"residual": x, "res_pad": 1} if rng.randint(0, 2) else {}
+                last, c = self._one(a, 3, ch, ch, act=self._act(), **res), ch
+            elif part == "bn":
+                self.no += 1
+                seed = self._next_seed()
+                self._add(fa.GPULayerBuilder("c%d" % self.no).type(T.BATCHNORM).number(self.no).shape(c, self.y, self.x, c).deep(),
+                          lambda c=c, seed=seed: np.concatenate([prng.uniform(seed, (c,), 0.5, 1.5), prng.normal(seed + 1, (c,), 0.0, 0.2)]))
+                self._edges.append((last, self.no, 0))
+                last = self.no
+            elif part == "up" and self.y * self.x <= 300:
+                self.no += 1
+                self._add(fa.ScaleLayerBuilder("c%d" % self.no).number(self.no).shape(c, self.y, self.x, c).scale(2.0).scaleType(fa.ScalingType.LINEAR).deep())
+                self._edges.append((last, self.no, 0))
+                last, self.y, self.x = self.no, 2 * self.y, 2 * self.x
+            elif part == "cat":
+                a, b = self._one(last, 1, c, 32), self._one(last, 1, c, 16)
+                self.no += 1
+                cat = fa.ConcatLayerBuilder("c%d" % self.no).number(self.no).deep().input(32, 0).input(16, 0)
+                cat.size(self.x, self.y)
+                cat.outputChannels_ = 48
+                self._add(cat)
+                self._edges += [(a, self.no, 0), (b, self.no, 1)]
+                last, c = self.no, 48
+        self.argmax_layer = None
+        if self.tail == "sigmoid":
+            last = self._one(last, 1, c, 24, pad_out=1)
+            last = self._one(last, 3, 24, 3)
+            self.no += 1
+            self._add(fa.GPULayerBuilder("c%d" % self.no).type(T.SIGMOID).number(self.no).shape(3, self.y, self.x, 3).deep())
+            self._edges.append((last, self.no, 0))
+            last, c = self.no, 3
+        elif self.tail == "argmax":   # (the scores end a bottleneck)
+            a = self._one(last, 1, c, 32, pad_out=1)
+            b = self._one(a, 3, 32, 32)
+            last, c = self._one(b, 1, 32, 21), 21
+            self.no += 1
+            self._add(fa.ArgMaxLayerBuilder("c%d" % self.no).number(self.no).shape(2, self.y, self.x, 21).deep())
+            self._edges.append((last, self.no, 0))
+            self.argmax_layer = self.no
+        if self.argmax_layer is None:   # (launches behind everything that clear the words of the tensors' value ranges)
+            for _ in range(2):
+                last = self._one(last, 1, c, c)
+            self.no += 1
+            self._add(fa.UpDownLayerBuilder(fa.UpDownLayerBuilder.DOWNLOAD, "download").number(self.no).shape(c, self.y, self.x, c).deep())
+            self._edges.append((last, self.no, 0))
+            last = self.no
+        self.output_layer = last
+
+    def setInput(self, x):
+        self.layers[0].setInput(x, 0)
+
+
+@pytest.mark.parametrize("storage", [fa.STORAGE_F32, fa.STORAGE_F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("seed", range(48))
+def test_random_rows_of_joined_launches(seed, storage, monkeypatch):
+    """Whatever is joined, the result is the oracle's and that of the layers apart, for one frame behind another.  fp16 storage: up
+    to 25 layers round to 11 bits, 2.8e-4 each, 1.4e-3 together and twice that at most between two orders of summation."""
+    frames = [prng.uniform(9000 + seed + i, (3, *(lambda n: (n.h, n.w))(Motifs(storage, seed))), -1.0, 1.0) for i in range(2)]
+    outs, infos = {}, {}
+    for mode in ("FORCE", "NO"):
+        for what in ("BLOCK", "PAIR", "HEAD"):
+            monkeypatch.delenv("FYNHIP_FORCE_%s_FUSION" % what, raising=False)
+            monkeypatch.setenv("FYNHIP_%s_%s_FUSION" % (mode, what), "1")
+        if seed % 3 == 0:
+            monkeypatch.setenv("FYNHIP_FORCE_P16_CONV", "1")
+            monkeypatch.setenv("FYNHIP_P16_TILE", "4,16")
+        elif seed % 3 == 1:
+            monkeypatch.setenv("FYNHIP_FORCE_S16_CONV", "1")
+        net = Motifs(storage, seed)
+        net.setup()
+        infos[mode] = [lyr.kernelInfo().split("; apart")[0] for lyr in net.layers]
+        if mode == "FORCE":
+            print("seed", seed, net.head, net.parts, net.tail, (net.h, net.w), flush=True)
+        for x in frames:
+            net.setInput(x)
+            net.forward()
+            net.finish()
+            got = net.getOutput(net.output_layer)
+            outs.setdefault(mode, []).append(got)
+            if net.argmax_layer is not None:
+                labels, best = net.getArgMax(net.argmax_layer)
+                assert np.array_equal(labels, got.argmax(axis=0)) and np.array_equal(best, got.max(axis=0)), (seed, mode)
+        desc = net.describe()
+        net.cleanup()
+    joined = [i for i in infos["FORCE"] if i.startswith(("conv_a16", "conv_b16", "conv_c16"))]
+    print("   ", [i[:8] for i in joined], flush=True)
+    assert not any(i.startswith(("conv_a16", "conv_b16", "conv_c16")) for i in infos["NO"])
+    tol = {fa.STORAGE_F32: 1e-4, fa.STORAGE_F16: 3e-3}[storage]
+    for x, one, apart in zip(frames, outs["FORCE"], outs["NO"]):
+        e = rel_l2(one, O.run_network(desc, {net.input_key: x})[net.output_layer]), rel_l2(one, apart)
+        print("    rel_l2 %.2e, against the layers apart %.2e" % e, flush=True)
+        assert max(e) <= tol, (seed, e)
